@@ -99,7 +99,8 @@ long long onhip_split_tail_launches(void);
 long long onhip_direct_lds_launches(void);
 /* Diagnostic, no counterpart in the reference: how the calling thread's last dense convolution / MatMul launch ran:
  * out = {tile rows, tile columns, K slices of every tile (1 = none), K slices of the leftover tiles only (0 = none),
- * 1 if the fp32 kernel that reads B straight from memory ran, 1 if the slices were added up inside the launch,
+ * 1 if the fp32 kernel that reads B straight from memory ran, 2 if the fp32 kernel on the 16-bit matrix cores did (its
+ * rows are then the columns of a MatMul), 1 if the slices were added up inside the launch,
  * 1 / 2 if the kernel that loads operand tiles straight into LDS ran (short / long ring)}; zeros before the first such
  * launch; launches of the other kernel families (depthwise, first-layer, few-channel int8) leave it as it is. */
 void onhip_last_launch_choice(int32_t out[7]);
@@ -555,6 +556,11 @@ int onhip_plugin_set_stream(void *stream);
  * [base, base + bytes), so that other data at the same address later is packed afresh.  The device-resident runtime calls it when a net is freed.  No counterpart in the
  * reference (its weights live in host vectors for the life of the process). */
 int onhip_plugin_forget(const void *base, size_t bytes);
+/* Weights of a loaded model: device memory [base, base + bytes) whose contents stay as they are until onhip_plugin_forget
+ * is called for it.  The library may keep re-laid-out copies of any weight tensor in such a range (1x1 convolutions and
+ * products included, which it otherwise reads as they are on every call).  The device-resident runtime calls it when a net's
+ * initialisers are in place.  No counterpart in the reference. */
+int onhip_plugin_hold(const void *base, size_t bytes);
 /* `eval` keeps a device copy of every weight and table it was handed in host memory and, on each call, hashes the host
  * buffer to see whether the copy is still current: all of it by default (about 0.05 ms per MiB), so weights updated in
  * place are picked up.  on != 0: only 4096 sampled words are hashed, for a caller whose weights never change while the

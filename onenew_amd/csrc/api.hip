@@ -131,6 +131,22 @@ static int get_scratch(size_t bytes, void **out) {
     return ONHIP_OK;
 }
 
+// Split weights of a call whose caller has none (launch_choice): one block per process, allocated at first use and never
+// outgrown (weights whose split form is larger run the other fp32 kernels); the entry point that allocates nothing has its own.
+static const long long kSplitWsBytes = 16LL << 20;
+static __device__ __align__(256) unsigned char split_scratch[kSplitWsBytes];
+static void *g_split_ws = nullptr;
+static int get_split_ws(void **out) {
+    if (tl_noalloc) {
+        ONHIP_CHECK_HIP(hipGetSymbolAddress(out, HIP_SYMBOL(split_scratch)));
+        return ONHIP_OK;
+    }
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    if (!g_split_ws) ONHIP_CHECK_HIP(hipMalloc(&g_split_ws, kSplitWsBytes));
+    *out = g_split_ws;
+    return ONHIP_OK;
+}
+
 // Workspace of the split-K reduction that runs inside the launch: partial sums and one arrival counter per tile in
 // uncached device memory, so that what one XCD wrote is what another reads without flushing anybody's L2.  Allocated
 // once at first use and kept for the life of the process.
@@ -170,7 +186,8 @@ static const int kSplits[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16, 24, 32};
 static const int kNumSplits = 13;
 
 // tail > 1: the tiles left over after whole rounds of 256 are cut `tail` ways along K (launch_choice)
-// rowb != 0: the kernel that feeds B from global memory straight into the MFMAs (igemm_rowb.hip), tile bm x bn
+// rowb == 1: the kernel that feeds B from global memory straight into the MFMAs (igemm_rowb.hip), tile bm x bn; rowb == 2: the
+// fp32 kernel on the 16-bit matrix cores (igemm_f3.hip), tile bm x bn
 // fin != 0 (with split > 1 or tail > 1): the slices of a tile are added up by the last of them to arrive, inside the
 // launch, instead of by a finishing launch (igemm_kernel, `arrive`)
 // dma != 0: the kernel that loads its operand tiles straight into LDS (igemm_dma_kernel.hpp), tile bm x bn, never split;
@@ -296,15 +313,26 @@ static bool tail_geometry(const IgemmLaunch &cfg, const IgemmParams &p, int bm, 
 
 static const int kRowbTiles[][2] = {{64, 128}, {128, 128}, {64, 256}, {96, 128}, {32, 256}, {32, 512}};
 static const int kNumRowbTiles = 6;
+static const int kF3Tiles[][2] = {{256, 128}, {256, 64}, {128, 128}, {128, 64}, {64, 64}};
+static const int kNumF3Tiles = 5;
 
 // (bm, bn) is a tile this build has a kernel for
 static bool tile_exists(const Choice &c) {
     if (c.dma) return c.dma <= 2 && dma_tile_ok(c.bm, c.bn);
-    const int (*list)[2] = c.rowb ? kRowbTiles : kTiles;
-    const int n = c.rowb ? kNumRowbTiles : kNumTiles;
+    const int (*list)[2] = c.rowb == 2 ? kF3Tiles : c.rowb ? kRowbTiles : kTiles;
+    const int n = c.rowb == 2 ? kNumF3Tiles : c.rowb ? kNumRowbTiles : kNumTiles;
     for (int t = 0; t < n; ++t)
         if (list[t][0] == c.bm && list[t][1] == c.bn) return true;
     return false;
+}
+
+// the fp32 kernel on the 16-bit matrix cores: a weight matrix for A, split already or small enough to be split on the call
+static bool f3_ok(const IgemmLaunch &cfg, const IgemmParams &p) {
+    static const bool off = getenv("ONHIP_NO_F3") != nullptr;   // tuning hook: fp32 matrix instructions only
+    if (off || cfg.dtype != DT_F32 || cfg.batch != 1 || (!p.a_split && !p.w_src)) return false;
+    if (cfg.bl != BL_PLAIN && cfg.bl != BL_TAPC && cfg.bl != BL_GATHER && cfg.bl != BL_ROWS) return false;
+    const long long bytes = split_weights_bytes(p.M, p.K);
+    return bytes < (1LL << 31) && (p.a_split || bytes <= kSplitWsBytes);
 }
 
 static bool candidate_ok(const IgemmLaunch &cfg, const IgemmParams &p, const Choice &c) {
@@ -318,12 +346,13 @@ static bool candidate_ok(const IgemmLaunch &cfg, const IgemmParams &p, const Cho
         return (!off || h16) && c.split == 1 && c.tail <= 1 && !c.rowb && !c.fin && dma_ok(cfg, p);
     }
     if (h16) return false;
-    if (c.rowb && (c.split != 1 || !rowb_f32_ok(cfg, p))) return false;
+    if (c.rowb == 2 && !f3_ok(cfg, p)) return false;
+    if (c.rowb == 1 && (c.split != 1 || !rowb_f32_ok(cfg, p))) return false;
     if (c.fin) {
         static const bool off = getenv("ONHIP_NO_FIN") != nullptr;   // tuning hook: finishing launches only
         if (off) return false;
         const long long tiles = (long long) ((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn) * cfg.batch;
-        if (cfg.dtype == DT_I8 || c.rowb || (c.split <= 1 && c.tail <= 1) || tiles > (1 << 20)) return false;
+        if (cfg.dtype == DT_I8 || c.rowb == 1 || (c.split <= 1 && c.tail <= 1) || tiles > (1 << 20)) return false;
     }
     if (c.tail > 1) {
         int dpc, left;
@@ -397,6 +426,33 @@ static bool dma_model_choice(const IgemmLaunch &cfg, const IgemmParams &p, Choic
     return true;
 }
 
+// Best tile and K split of the fp32 kernel on the 16-bit matrix cores and what the launch takes, in microseconds.  Fitted to
+// 1100 timed launches over the layers of ResNet-50 (batch 1, 8, 32) and MobileNetV2 (batch 8, 64), median error 10 %, the
+// choices within 2 % of the fastest: a compute unit works through its workgroups at a rate that depends on the tile alone
+// (larger tiles stage less per multiply-add), whether one or several are resident.
+static bool f3_choice(const IgemmLaunch &cfg, const IgemmParams &p, Choice *out, double *us) {
+    static const double per_k_tile[kNumF3Tiles] = {0.82, 0.50, 0.50, 0.29, 0.215};   // per K tile of 16 and workgroup
+    static const double per_tile[kNumF3Tiles] = {3.8, 1.8, 1.25, 0.70, 0.37};        // first loads and store of a workgroup
+    *us = 1e300;
+    for (int t = 0; t < kNumF3Tiles; ++t)
+        for (int s = 0; s < kNumSplits; ++s) {
+            const Choice c = {kF3Tiles[t][0], kF3Tiles[t][1], kSplits[s], 0, 2, 0, 0};
+            if (c.bm > 64 && p.M <= c.bm / 2) continue;
+            if (c.split > 1 && cfg.bl == BL_ROWS) continue;
+            if (!candidate_ok(cfg, p, c)) continue;
+            const int k_tiles = (p.k_units + 3) / 4, per = (k_tiles + c.split - 1) / c.split;
+            const double tiles = (double) ((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn);
+            double t_us = 4.2 + ceil(tiles * c.split / 256.0) * (per * per_k_tile[t] + per_tile[t]);
+            if (c.split > 1) t_us += 3.4 + 0.33e-6 * c.split * 4.0 * p.M * p.N;   // partial sums, and the launch that adds them up
+            if (t_us < *us) { *us = t_us; *out = c; }
+        }
+    if (*us > 1e299) return false;
+    if (!p.a_split) *us += 2.5 + 10.0 / 3e6 * p.M * p.K;   // the pass that splits the weights: 4 bytes read, 6 written
+    return true;
+}
+// the same for the fp32 matrix instructions' kernels (2250 cycles of model_cost take a microsecond; same launches, error 10 %)
+static double f32_us(double cycles) { return 3.75 + cycles / 2250.0; }
+
 static Choice model_choice(const IgemmLaunch &cfg, const IgemmParams &p) {
     Choice best = {64, 64, 1, 0, 0, 0};
     const bool vec = cfg.bl == BL_KVEC || cfg.bl == BL_KVEC_TAP;
@@ -426,6 +482,14 @@ static Choice model_choice(const IgemmLaunch &cfg, const IgemmParams &p) {
                 if (cost < best_cost) { best_cost = cost; best = c; }
             }
         if (best_cost < 1e300) break;
+    }
+    // fp32 with a weight matrix for A: the 16-bit matrix cores where that is expected to be faster.  Not for up to 32 rows
+    // (the smallest of those tiles has 64: 0.74-0.98 of these kernels' speed on MobileNetV2's projections) nor for reductions
+    // below 48 (bound by memory: 0.69 on its 16 -> 96 expansion, where the kernel that reads B straight from memory runs).
+    if (cfg.dtype == DT_F32 && !tl_hint_bm && p.M > 32 && p.K >= 48) {
+        Choice c;
+        double us;
+        if (f3_choice(cfg, p, &c, &us) && us < f32_us(model_cost(cfg, p, best))) return c;
     }
     // What measuring the candidates keeps finding on top of the tile and split above (fp32, one batch slice):
     //  * no split, and a few tiles left over after whole rounds of 256: those tiles alone cut along K so that the leftover,
@@ -485,8 +549,16 @@ static int launch_choice(IgemmLaunch cfg, IgemmParams p, const Choice &c, hipStr
         g_dma_launches.fetch_add(1, std::memory_order_relaxed);
         return dma_launch(cfg, p, st);
     }
+    if (c.rowb == 2 && !p.a_split) {
+        void *ws = nullptr;
+        int rc = get_split_ws(&ws);
+        if (!rc) rc = split_weights_launch(p.w_src, p.M, p.K, p.w_row, p.w_k, ws, st);
+        if (rc) return rc;
+        p.a_split = ws;
+        p.a_split_bytes = split_weights_bytes(p.M, p.K);
+    }
     auto launch = [&]() {
-        const int rc = c.rowb ? rowb_f32_launch(cfg, p, st) : igemm_launch(cfg, p, st);
+        const int rc = c.rowb == 2 ? f3_launch(cfg, p, st) : c.rowb ? rowb_f32_launch(cfg, p, st) : igemm_launch(cfg, p, st);
         if (rc && p.arrive) {   // whatever part of the launch ran may have left arrival counters above zero
             std::lock_guard<std::mutex> lock(g_scratch_mu);
             g_arrive_dirty = true;
@@ -494,14 +566,14 @@ static int launch_choice(IgemmLaunch cfg, IgemmParams p, const Choice &c, hipStr
         return rc;
     };
     if (c.tail <= 1 || !tail_geometry(cfg, p, c.bm, c.bn, &dpc, &left)) {
-        const Choice plain = {c.bm, c.bn, c.rowb ? 1 : c.split, 0, 0, c.rowb ? 0 : c.fin};
+        const Choice plain = {c.bm, c.bn, c.rowb == 1 ? 1 : c.split, 0, 0, c.rowb == 1 ? 0 : c.fin};
         int rc = apply_choice(cfg, p, plain);
         return rc ? rc : launch();
     }
     // one launch: dpc column blocks as whole tiles, the rest in c.tail K slices each; partial sums and the
     // finishing pass cover the columns from dpc * bn on only
     p.part_begin = dpc * c.bn;
-    const Choice tail = {c.bm, c.bn, c.tail, 0, 0, c.rowb ? 0 : c.fin};
+    const Choice tail = {c.bm, c.bn, c.tail, 0, 0, c.rowb == 1 ? 0 : c.fin};
     int rc = apply_choice(cfg, p, tail);
     if (rc) return rc;
     if (cfg.split <= 1) {
@@ -552,6 +624,7 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmParams &p, hipStre
                 if (c.bm == 128 && c.bn == 64) c.bm = 64;
             }
             if (c.fin && !candidate_ok(cfg, p, c)) c.fin = 0;
+            if (c.rowb == 2 && !candidate_ok(cfg, p, c)) { c = {64, 64, 1, 0, 0, 0, 0}; }
             if (c.rowb && !candidate_ok(cfg, p, c)) {   // not a problem for that kernel: the tiled one, same tile if it has it
                 c.rowb = 0;
                 if (c.bn > 128) c.bn = 128;
@@ -643,6 +716,16 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmParams &p, hipStre
             }
         }
     }
+    // the fp32 kernel on the 16-bit matrix cores: every tile, with the model's K split and without
+    Choice f3;
+    double f3_us;
+    if (!rc && f3_ok(cfg, p) && f3_choice(cfg, p, &f3, &f3_us))
+        for (int t = 0; t < kNumF3Tiles && !rc; ++t) {
+            const Choice c = {kF3Tiles[t][0], kF3Tiles[t][1], f3.split, 0, 2, 0, 0};
+            if (candidate_ok(cfg, p, c)) try_choice(c);
+            const Choice whole = {c.bm, c.bn, 1, 0, 2, 0, 0};
+            if (!rc && f3.split > 1 && candidate_ok(cfg, p, whole)) try_choice(whole);
+        }
     // the int8 kernel that loads its tiles straight into LDS
     static const int kDmaTiles[][2] = {{128, 128}, {128, 64}, {64, 128}, {64, 64}};
     for (int t = 0; t < 8 && !rc; ++t) {
@@ -786,8 +869,10 @@ static int add_relu_in_place(const onhip_conv_desc_t *d, int OH, int OW, const f
     return rc;
 }
 
+// split, when not null: the same weights (as w has them) in split_weights_launch's form
 static int conv2d_f32_impl(const onhip_conv_desc_t *d, const float *x, const float *w, int packed, const float *bias,
-                           const float *silu_lut, float *y, void *stream, const float *addend = nullptr, int relu_after = 0) {
+                           const float *silu_lut, float *y, void *stream, const float *addend = nullptr, int relu_after = 0,
+                           const void *split = nullptr) {
     int32_t OH, OW;
     int rc = check_conv(d, &OH, &OW);
     if (rc) return rc;
@@ -846,6 +931,11 @@ static int conv2d_f32_impl(const onhip_conv_desc_t *d, const float *x, const flo
     p.k_units = (p.K + kpu - 1) / kpu;
     p.A = w;
     p.lda = p.K;
+    p.w_src = w;
+    p.w_row = p.K;
+    p.w_k = 1;
+    p.a_split = split;
+    p.a_split_bytes = split ? split_weights_bytes(p.M, p.K) : 0;
     p.B = x;
     p.b_img_stride = (long long) d->cin * d->h * d->w;
     p.b_shift_bytes = ((long long) d->pad_t * d->w + d->pad_l) * 4;
@@ -1278,8 +1368,39 @@ int onhip_conv2d_w8_link(const onhip_conv_desc_t *d, const float *x, const int8_
                              d->out_s8 ? 1 : 0, stream, addend, relu_after, y_twin);
 }
 
+// A product with a shared right operand (a weight matrix) as the fp32 kernel on the 16-bit matrix cores takes it: transposed,
+// the columns of `b` the rows of its A operand, the rows of `a` (K contiguous) its B, `out` [rows][n] written four columns at
+// a time
+static void matmul_rows_problem(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias, const float *gelu_lut,
+                                const float *addend, float *out, const void *split, IgemmLaunch *cfg, IgemmParams *p) {
+    memset(cfg, 0, sizeof(*cfg));
+    cfg->dtype = DT_F32;
+    cfg->bl = BL_ROWS;
+    cfg->batch = 1;
+    memset(p, 0, sizeof(*p));
+    const long long rows = (long long) d->batch * d->m;
+    p->M = d->n; p->N = (int) rows; p->K = d->k;
+    p->k_units = (p->K + 3) / 4;
+    p->w_src = b; p->w_row = 1; p->w_k = d->n;
+    p->a_split = split;
+    p->a_split_bytes = split ? split_weights_bytes(p->M, p->K) : 0;
+    p->B = a;
+    p->ldb = d->k;
+    p->b_slice_bytes = rows * d->k * 4;
+    p->c_slice_bytes = rows * d->n * 4;
+    p->C = out;
+    p->out_mode = OUT_PLAIN;
+    p->c_stride_m = 1;
+    p->c_stride_n = d->n;
+    p->bias = bias;
+    p->bias_mode = bias ? BIAS_M : BIAS_NONE;
+    p->ep.act = gelu_lut ? ONHIP_ACT_GELU_LUT : NOT_ACT;
+    p->ep.lut = gelu_lut;
+    p->res = addend;
+}
+
 static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias,
-                       const float *gelu_lut, const float *addend, float *out, void *stream) {
+                       const float *gelu_lut, const float *addend, float *out, void *stream, const void *split = nullptr) {
     if (!d || d->batch < 1 || d->m < 1 || d->k < 1 || d->n < 1) return set_error(ONHIP_ERR_ARG, "matmul: bad shape");
     if (!a || !b || !out) return set_error(ONHIP_ERR_ARG, "matmul: null tensor pointer");
     int batch = d->batch, M = d->m;
@@ -1335,6 +1456,21 @@ static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float
         return onhip_add_f32(&ad, out, addend, out, stream);
     }
     p.res = addend;   // laid out like the result; added after the bias, as the Add operator after it would
+    if (cfg.dtype == DT_F32 && batch == 1 && !getenv("ONHIP_TILE")) {
+        IgemmLaunch rcfg;
+        IgemmParams rp;
+        matmul_rows_problem(d, a, b, bias, gelu_lut, addend, out, split, &rcfg, &rp);
+        Choice c;
+        double us;
+        // rule as in model_choice; the pass that splits the weights is priced in even where the caller has them split, so that
+        // a product runs the same way, with the same bits, whether its right operand is a model's weight or not
+        if (split) { rp.a_split = nullptr; }
+        if (rp.M > 32 && rp.K >= 48 && p.b_slice_bytes < (1LL << 31) && rp.b_slice_bytes < (1LL << 31) && rp.c_slice_bytes < (1LL << 31) &&
+            f3_choice(rcfg, rp, &c, &us) && us < f32_us(model_cost(cfg, p, model_choice(cfg, p)))) {
+            rp.a_split = split;
+            return launch_choice(rcfg, rp, c, st);
+        }
+    }
     return plan_and_launch(cfg, p, st);
 }
 
@@ -1705,3 +1841,42 @@ int onhip_gemm_f32(int32_t m, int32_t k, int32_t n, const float *a, const float 
 }
 
 }  // extern "C"
+
+// The plugins keep weights that belong to a loaded model split.  *_split_source: how (the caller's weights as M rows of K
+// elements), where a call with them would run the kernel that reads that form; M = 0 otherwise.
+namespace onhip {
+int conv2d_f32_split(const onhip_conv_desc_t *d, const float *x, const float *w, int packed, const float *bias, const float *silu_lut,
+                     const float *addend, int relu_after, float *y, const void *split, void *stream) {
+    return conv2d_f32_impl(d, x, w, packed, bias, silu_lut, y, stream, addend, relu_after, split);
+}
+SplitSource conv2d_f32_split_source(const onhip_conv_desc_t *d, int packed) {
+    SplitSource src = {0, 0, 0, 0};
+    int32_t OH, OW;
+    if (check_conv(d, &OH, &OW) || d->group != 1 || d->compute != ONHIP_COMPUTE_F32 || getenv("ONHIP_TILE")) return src;
+    if (stem_f32_ok(*d, OH, OW) && (packed || OW >= 96)) return src;
+    IgemmLaunch cfg;
+    memset(&cfg, 0, sizeof(cfg));
+    cfg.dtype = DT_F32;
+    cfg.batch = 1;
+    cfg.bl = packed ? BL_TAPC : plain_pointwise(d) ? BL_PLAIN : BL_GATHER;
+    IgemmParams p;
+    memset(&p, 0, sizeof(p));
+    p.M = d->cout;
+    p.N = d->n * OH * OW;
+    p.K = d->kh * d->kw * (packed ? packed_cp(d) : d->cin);
+    p.k_units = (p.K + 3) / 4;
+    p.a_split = &src;   // as if there were one
+    if (model_choice(cfg, p).rowb == 2) src = {p.M, p.K, p.K, 1};
+    return src;
+}
+int matmul_f32_split(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias, const float *gelu_lut, const float *addend,
+                     float *out, const void *split, void *stream) {
+    return matmul_impl(d, a, b, bias, gelu_lut, addend, out, stream, split);
+}
+SplitSource matmul_f32_split_source(const onhip_matmul_desc_t *d) {
+    SplitSource src = {0, 0, 0, 0};
+    if ((!d->b_shared && d->batch != 1) || d->compute != ONHIP_COMPUTE_F32 || d->n <= 32 || d->k < 48 || getenv("ONHIP_TILE")) return src;
+    src = {d->n, d->k, 1, d->n};   // made whenever a call might use it: the call decides by the number of rows
+    return src;
+}
+}  // namespace onhip

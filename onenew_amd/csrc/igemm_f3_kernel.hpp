@@ -1,0 +1,420 @@
+// fp32 implicit GEMM on the 16-bit matrix cores (gfx950): C[M, N] = A[M, K] * B[K, N], operands and result fp32.
+//
+// Arithmetic.  Every fp32 operand is written as the sum of three bf16 numbers, x = h + m + l: h = bf16(x), m = bf16(x - h),
+// l = x - h - m, each rounded to nearest.  The two differences are exact, and so is the sum: 24 significant bits are three
+// times eight (|m| <= 2^-8 |h|, |l| <= 2^-8 |m|).  bf16 has fp32's exponent range, so no operand needs scaling.  Of the nine
+// partial products six are formed, each exact in the matrix core and added to the fp32 accumulator: l h, m m, m h, h l, h m,
+// h h.  The three left out, m l, l m and l l, are at most 2^-23 and typically 2^-26 of |a b|, below the rounding that a chain
+// of fp32 multiply-adds makes at every step.  Measured against 64-bit sums over K = 16 ... 4608: relative error 0.46 ... 0.87
+// of v_mfma_f32_32x32x2_f32's on normal operands and on all-positive ones, and on operands spread over 2^+-24 a largest
+// error over sum |a b| within 15 % of it either way; the nine products give the same errors as the six.
+// What differs from an fp32 multiply: magnitudes below 2^-111 lose low bits (their l falls below bf16's subnormals), and an
+// infinity or a NaN, or an activation that rounds to a bf16 infinity, has no finite parts and makes the sum NaN.  A wavefront
+// that holds a non-finite sum when its K loop is over computes those elements again with fp32 multiply-adds (fix_nonfinite),
+// so infinities and overflow come out as they do in fp32 arithmetic.
+//
+// Why: v_mfma_f32_32x32x16_bf16 does the multiply-adds of eight v_mfma_f32_32x32x2_f32 in a sixteenth of their time.  On
+// random operands the card holds its power limit by its clock (1.2 to 1.7 GHz in these loops), so what counts is energy: six
+// products reach 200-210 TFLOP/s of fp32 multiply-adds on 1024 x 32768 x 1024 and on a 3x3 convolution over 256 channels,
+// where fp32 matrix instructions reach 146-155 on their own and 116 in igemm_kernel.
+//
+// Work decomposition: as igemm_kernel.hpp, whose column state, scalar load descriptions, store and split-K pieces this
+// kernel uses; K in tiles of 4 units of 4 floats = one 16-deep MFMA step.  What differs:
+//   * A, the weights, is split ahead of time (split_weights_launch) into the order the matrix instructions read it, and goes
+//     from memory straight into operand registers, one contiguous KiB per load: no LDS, no vector instruction.  The
+//     wavefronts of a tile lie along M (the 64 x 64 and 128 x 128 tiles apart), so no two of them load the same rows;
+//   * B is split on its way into LDS, [part][k / 8][column][8 bf16], a unit per thread and K tile, in four phases of four to
+//     six vector instructions each behind an MFMA of its own: 22 vector instructions per 12 to 24 MFMAs and wavefront.
+// Per K tile of the 128 x 64 tile a wavefront issues 12 MFMAs, 3 A loads, 4 B loads, 3 LDS stores and 6 LDS reads.
+//
+// Replaces, for the dense fp32 cases with enough work (f3_plan in api.hip): device/x86/Conv/conv.c im2col (:168,:260) +
+// opt_gemm.h SGEMM (:17) + bias sweep (:405) + do_act (:1216); device/x86/MatMul/mat_mul.c:10.
+#pragma once
+#include "igemm_kernel.hpp"
+
+namespace onhip {
+
+// f(integral_constant<int, 0>), ..., f(integral_constant<int, N - 1>): indices the front end knows, so that every register
+// array of the kernel is taken apart before anything else happens to it
+template <int N, class F> __device__ __forceinline__ void static_for(F &&f) {
+    [&]<int... I>(std::integer_sequence<int, I...>) __attribute__((always_inline)) { (f(std::integral_constant<int, I>{}), ...); }(std::make_integer_sequence<int, N>{});
+}
+
+// two floats -> their three bf16 parts, packed in pairs
+__device__ __forceinline__ unsigned cvt_pk_bf16(float a, float b) {
+    unsigned d;   // the conversion of a pair; from C the compiler converts some of the values twice
+    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
+    return d;
+}
+__device__ __forceinline__ void split_pair(float x0, float x1, unsigned &h, unsigned &m, unsigned &l) {
+    h = cvt_pk_bf16(x0, x1);
+    const float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xffff0000u);
+    m = cvt_pk_bf16(r0, r1);
+    l = cvt_pk_bf16(r0 - __uint_as_float(m << 16), r1 - __uint_as_float(m & 0xffff0000u));
+}
+// A unit of four floats on its way to three parts, in four phases of four to six vector instructions: few enough to issue
+// behind one MFMA while it runs.
+struct SplitUnit {
+    float r0, r1, r2, r3, u0, u1, u2, u3;
+    unsigned h0, h1, m0, m1, l0, l1;   // the parts, packed in pairs
+    __device__ __forceinline__ void unpack(unsigned a, unsigned b) {
+        u0 = __uint_as_float(a << 16); u1 = __uint_as_float(a & 0xffff0000u);
+        u2 = __uint_as_float(b << 16); u3 = __uint_as_float(b & 0xffff0000u);
+    }
+    template <int Q> __device__ __forceinline__ void phase(float x0, float x1, float x2, float x3) {
+        if constexpr (Q == 0) {
+            h0 = cvt_pk_bf16(x0, x1); h1 = cvt_pk_bf16(x2, x3);
+            unpack(h0, h1);
+        } else if constexpr (Q == 1) {
+            r0 = x0 - u0; r1 = x1 - u1; r2 = x2 - u2; r3 = x3 - u3;
+            m0 = cvt_pk_bf16(r0, r1); m1 = cvt_pk_bf16(r2, r3);
+        } else if constexpr (Q == 2) {
+            unpack(m0, m1);
+        } else {
+            l0 = cvt_pk_bf16(r0 - u0, r1 - u1); l1 = cvt_pk_bf16(r2 - u2, r3 - u3);
+        }
+    }
+};
+__device__ __forceinline__ void mma_bf16(f32x16 &c, const uint4 &a, const uint4 &b) {
+    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+// the six partial products, (part of a, part of b) with 0 = h, 1 = m, 2 = l, smallest first
+constexpr int F3_PRODUCTS = 6;
+__device__ constexpr int f3_pa(int i) { constexpr int t[F3_PRODUCTS] = {2, 1, 1, 0, 0, 0}; return t[i]; }
+__device__ constexpr int f3_pb(int i) { constexpr int t[F3_PRODUCTS] = {0, 1, 0, 2, 1, 0}; return t[i]; }
+
+// column n's share of the B addresses
+template <int BL>
+__device__ __forceinline__ ColState f3_col(const IgemmParams &p, int n) {
+    if constexpr (BL == BL_ROWS) return {n < p.N ? (unsigned) (n * p.ldb) * 4u : OOB, 0, 0, 0u, 0u};
+    else return make_col<BL>(p, n);
+}
+
+// Sums that are not finite, computed again in fp32: see the head of the file.  scratch: 32 x 33 floats of LDS private to the
+// wavefront.  Units u_begin .. of the reduction up to klim elements; operands through the K loop's own loads.
+template <int BL, int TM, int TN>
+__device__ __forceinline__ void fix_nonfinite(const IgemmParams &p, f32x16 (&acc)[TM][TN], float *scratch, rsrc_t ra, rsrc_t rb, int m_wave,
+                                              int n_wave, int lane, int u_begin, int klim) {
+    float probe = 0.0f;   // stays zero while every sum is finite: 0 * inf and 0 * NaN are NaN
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) probe = __builtin_fmaf(acc[a][b][r], 0.0f, probe);
+    if (__builtin_amdgcn_ballot_w64(probe != probe) == 0ull) return;
+    const int li = lane & 31, lh = lane >> 5;
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) scratch[(8 * (r / 4) + 4 * lh + r % 4) * 33 + li] = acc[a][b][r];
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+            for (int e = 0; e < 16; ++e) {   // two rows of the block at a time: lane -> row 2 e + lh, column li
+                float *cell = scratch + (2 * e + lh) * 33 + li;
+                const int m = m_wave + a * 32 + 2 * e + lh, n = n_wave + b * 32 + li;
+                const float v = *cell;
+                const bool bad = v * 0.0f != 0.0f && m < p.M && n < p.N;
+                if (__builtin_amdgcn_ballot_w64(bad) == 0ull) continue;
+                const ColState col = f3_col<BL>(p, n);
+                float s = 0.0f;
+#pragma unroll 1
+                for (int u = u_begin; u * 4 < klim; ++u)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int k = u * 4 + j;
+                        float bv;
+                        if constexpr (BL == BL_ROWS) {
+                            bv = buf_load_f32(rb, (unsigned) (n * p.ldb) * 4u, (unsigned) k * 4u);
+                        } else {
+                            const BPrep q = prep_b<DT_F32, BL>(p, u, BL == BL_TAPC ? 0 : j, klim);
+                            const unsigned voff = b_voff<BL>(p, col, q, BL == BL_GATHER ? k : u);
+                            bv = buf_load_f32(rb, voff, q.soff + (BL == BL_TAPC ? (unsigned) j * (unsigned) p.HW * 4u : 0u));
+                        }
+                        const unsigned row = bad ? (unsigned) (m / 32) * (unsigned) ((p.K + 15) / 16) * 3072u + (unsigned) (m % 32) * 16u : OOB;
+                        const unsigned at = (unsigned) (k / 16) * 3072u + (unsigned) (k % 16 / 8) * 512u + (unsigned) (k % 8) * 2u;
+                        auto part = [&](unsigned z) __attribute__((always_inline)) {
+                            return __uint_as_float((unsigned) (unsigned short) __builtin_amdgcn_raw_buffer_load_b16(ra, row, at + z * 1024u, 0) << 16);
+                        };
+                        const float av = (part(0) + part(1)) + part(2);   // the parts add up to the weight exactly
+                        const float t = __builtin_fmaf(av, bv, s);
+                        s = k < klim ? t : s;
+                    }
+                if (bad) *cell = s;
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[a][b][r] = scratch[(8 * (r / 4) + 4 * lh + r % 4) * 33 + li];
+            __builtin_amdgcn_wave_barrier();
+        }
+}
+
+// The store for B given as rows (a product's left operand): C is row-major with the tile's columns as its rows, so the four
+// consecutive rows of the tile that a lane holds in registers 4 q .. 4 q + 3 are 16 contiguous bytes of C.  Residual and bias
+// as in write_tile.
+template <int EPI, int TM, int TN, bool RES>
+__device__ __forceinline__ void write_tile_rows(const IgemmParams &p, f32x16 (&acc)[TM][TN], int m_wave, int n_wave, int li, int lh,
+                                                const float *sbias) {
+    const rsrc_t rc = make_rsrc(p.C, (unsigned) p.c_slice_bytes), rr = make_rsrc(RES ? p.res : nullptr, RES ? (unsigned) p.c_slice_bytes : 0u);
+#pragma unroll
+    for (int b = 0; b < TN; ++b) {
+        const int n = n_wave + b * 32 + li;
+#pragma unroll
+        for (int a = 0; a < TM; ++a) {
+            const int m4 = m_wave + a * 32 + 4 * lh;
+            const unsigned base = n < p.N ? (unsigned) (n * (int) p.c_stride_n + m4) * 4u : OOB;
+            u32x4 rv[4];
+            if constexpr (RES)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) rv[q] = __builtin_amdgcn_raw_buffer_load_b128(rr, base, 32u * q, 0);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 bias = *reinterpret_cast<const float4 *>(sbias + a * 32 + 8 * q + 4 * lh);
+                const float bv[4] = {bias.x, bias.y, bias.z, bias.w};
+                u32x4 o;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    float v = act_fast<EPI>(__fadd_rn(acc[a][b][4 * q + j], bv[j]), p.ep);
+                    if constexpr (RES) v = __fadd_rn(v, __uint_as_float(rv[q][j]));
+                    o[j] = __float_as_uint(v);
+                }
+                const int left = p.M - (m4 + 8 * q);   // columns of C from this group on
+                if (left >= 4) {
+                    __builtin_amdgcn_raw_buffer_store_b128(o, rc, base, 32u * q, 0);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 3; ++j)
+                        if (j < left) __builtin_amdgcn_raw_buffer_store_b32(o[j], rc, base + 4u * j, 32u * q, 0);
+                }
+            }
+        }
+    }
+}
+
+template <int BL, int BM, int BN, int WM, int WN, bool RES>
+__global__ __launch_bounds__(64 * WM * WN, (BM / WM) * (BN / WN) >= 32 * 128 ? 2 : (BM / WM) * (BN / WN) >= 32 * 64 ? 3 : 4)
+void igemm_f3_kernel(const IgemmParams p) {
+    static_assert(BM % (WM * 32) == 0 && BN % (WN * 32) == 0, "wavefronts of 32 x 32 blocks");
+    constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
+    constexpr int UPT = 4, NT = 64 * WM * WN;
+    static_assert(BN * UPT == NT, "a thread stages one unit of B per K tile");
+    constexpr int LD = BL == BL_ROWS ? BN + 1 : BN;   // 16-byte slots per 8 elements of K; rows arrive from neighbouring lanes
+    constexpr int PLANE = 2 * LD, SLOTS = 3 * PLANE, FIX_SLOTS = (WM * WN * 32 * 33 * 4 + 15) / 16;   // fix_nonfinite's scratch fits as well
+    __shared__ uint4 lds[2 * SLOTS > FIX_SLOTS ? 2 * SLOTS : FIX_SLOTS];   // two K tiles
+    __shared__ __attribute__((aligned(16))) float s_bias[BM];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 31, lh = lane >> 5;
+    const int wm = wave / WN, wn = wave % WN;
+
+    const TilePlace tp = place_tile<BM, BN>(p);
+    const int m0 = tp.m0, n0 = tp.n0, slice = tp.slice, lid = tp.lid;
+    const bool whole_k = tp.whole_k;
+    const int batch = blockIdx.z;
+    const int u_begin = whole_k ? 0 : slice * p.k_split_units;
+    const int u_end = whole_k ? p.k_units : min(p.k_units, u_begin + p.k_split_units);
+    const int k_tiles = (u_end - u_begin + UPT - 1) / UPT;
+    const int klim = min(p.K, u_end * 4);
+
+    const char *b_base = reinterpret_cast<const char *>(p.B) + (size_t) batch * p.b_batch_stride * 4 - (size_t) p.b_shift_bytes;
+    const unsigned b_bytes = (unsigned) (p.b_slice_bytes + p.b_shift_bytes);
+
+    // A: [32 rows][16 of K][part][lane][16 bytes], row block, K tile and part in the scalar offset
+    const rsrc_t ra = make_rsrc(p.a_split, (unsigned) p.a_split_bytes);
+    const unsigned a_pitch = (unsigned) ((p.K + 15) / 16) * 3072u;
+    const unsigned a_block0 = (unsigned) ((m0 + wm * (BM / WM)) / 32) * a_pitch + (unsigned) (u_begin / UPT) * 3072u;
+    const unsigned lane16 = (unsigned) lane * 16u;
+
+    // B: this thread's column and its unit of every K tile.  From NCHW activations lanes run along the columns and the unit
+    // is the wavefront's; from rows four neighbouring lanes hold the four units of a row (64 contiguous bytes)
+    const int bcol = BL == BL_ROWS ? tid / UPT : tid % BN;
+    const int bunit = BL == BL_ROWS ? tid % UPT : __builtin_amdgcn_readfirstlane(tid / BN);
+    const ColState col = f3_col<BL>(p, n0 + bcol);
+
+    f32x16 acc[TM][TN];
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.0f;
+
+    constexpr int BE = BL == BL_GATHER ? 4 : 1;         // scalar descriptions per B unit
+    constexpr int STEPS = F3_PRODUCTS * TM * TN;        // MFMAs per K tile and wavefront
+    constexpr int BAR = STEPS / 2 + 1;                  // the barrier stands before this step
+    constexpr int READS = 3 * TN;
+    struct Operands { uint4 a[3][TM], b[3][TN]; };
+    RawUnit<DT_F32> qb[2];                              // two K tiles in flight between memory and LDS
+    BPrep bp[BE];
+    const unsigned hw4 = (unsigned) p.HW * 4u;
+
+    auto prep_unit = [&](int kt) __attribute__((always_inline)) {
+        if constexpr (BL != BL_ROWS)
+#pragma unroll
+            for (int e = 0; e < BE; ++e) bp[e] = prep_b<DT_F32, BL>(p, u_begin + kt * UPT + bunit, e, klim);
+    };
+    // the loads of B for K tile kt; a tile past the end reads through an empty descriptor (zeros, no traffic)
+    auto issue_b = [&](int kt, auto slot) __attribute__((always_inline)) {
+        RawUnit<DT_F32> &q = qb[decltype(slot)::value];
+        const rsrc_t rb = make_rsrc(b_base, kt < k_tiles ? b_bytes : 0u);
+        const int u = u_begin + kt * UPT + bunit;
+        if constexpr (BL == BL_ROWS) {
+            const uint4 t = buf_load_b128(rb, col.pixoff + (unsigned) bunit * 16u, (unsigned) (u_begin + kt * UPT) * 16u);
+            q.v[0] = __uint_as_float(t.x); q.v[1] = __uint_as_float(t.y); q.v[2] = __uint_as_float(t.z); q.v[3] = __uint_as_float(t.w);
+        } else if constexpr (BL == BL_TAPC) {
+            const unsigned voff = b_voff<BL>(p, col, bp[0], u);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) q.v[e] = buf_load_f32(rb, voff, bp[0].soff + (unsigned) e * hw4);
+        } else if constexpr (BL == BL_PLAIN) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) q.v[e] = buf_load_f32(rb, col.pixoff, bp[0].soff + (unsigned) e * hw4);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) q.v[e] = buf_load_f32(rb, b_voff<BL>(p, col, bp[e], u * 4 + e), bp[e].soff);
+        }
+    };
+    auto load_a = [&](Operands &o, int kt, int part) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < TM; ++t) o.a[part][t] = buf_load_b128(ra, lane16, a_block0 + (unsigned) t * a_pitch + (unsigned) kt * 3072u + part * 1024u);
+    };
+    SplitUnit work;   // the unit being split
+    auto stage_b = [&](int buf, auto phase, auto slot) __attribute__((always_inline)) {
+        constexpr int Q = decltype(phase)::value;
+        const RawUnit<DT_F32> &q = qb[decltype(slot)::value];
+        work.phase<Q>(q.v[0], q.v[1], q.v[2], q.v[3]);
+        if constexpr (Q == 3) {
+            uint2 *base = reinterpret_cast<uint2 *>(&lds[buf + bunit / 2 * LD + bcol]) + bunit % 2;
+            base[0] = make_uint2(work.h0, work.h1);
+            base[2 * PLANE] = make_uint2(work.m0, work.m1);
+            base[4 * PLANE] = make_uint2(work.l0, work.l1);
+        }
+    };
+    // LDS reads in the order the products need them
+    auto read_operand = [&](Operands &o, int buf, auto idx) __attribute__((always_inline)) {
+        constexpr int pb = decltype(idx)::value / TN, t = decltype(idx)::value % TN;
+        o.b[pb][t] = lds[buf + pb * PLANE + lh * LD + wn * (BN / WN) + t * 32 + li];
+    };
+
+    Operands op0, op1;
+    constexpr std::integral_constant<int, 0> S0{};
+    constexpr std::integral_constant<int, 1> S1{};
+    prep_unit(0);
+    issue_b(0, S0);
+#pragma unroll
+    for (int z = 2; z >= 0; --z) load_a(op0, 0, z);
+    prep_unit(1);
+    issue_b(1, S1);
+#pragma unroll
+    for (int z = 2; z >= 0; --z) load_a(op1, 1, z);
+    float bias_row[(BM + NT - 1) / NT];   // the tile's rows of the bias, for LDS when the K loop is over; -0.0f changes nothing
+#pragma unroll
+    for (int i = 0; i < (BM + NT - 1) / NT; ++i) {
+        const bool on = p.bias_mode == BIAS_M;
+        const int row = tid + i * NT;
+        const float bv = buf_load_f32(make_rsrc(p.bias, on ? (unsigned) (p.M * 4) : 0u), row < BM ? (unsigned) (m0 + row) * 4u : OOB, 0);
+        bias_row[i] = on ? bv : -0.0f;
+    }
+    static_for<4>([&](auto ph) __attribute__((always_inline)) { stage_b(0, ph, S0); });
+    prep_unit(2);
+    issue_b(2, S0);
+    prep_unit(3);
+    __syncthreads();
+    static_for<READS>([&](auto i) __attribute__((always_inline)) { read_operand(op0, 0, i); });
+
+    // Body kt: the MFMAs of tile kt, whose operands are in registers.  Behind them, a phase at a time over the steps before the
+    // barrier, B of tile kt + 1 goes through the split to LDS, with the loads of tile kt + 3 into the registers that frees;
+    // after the barrier the LDS reads of tile kt + 1.  A of tile kt + 2 is loaded into the operand registers of tile kt as
+    // its products retire them (l first, h last).
+    auto body = [&](Operands &cur, Operands &nxt, int kt, auto wr) __attribute__((always_inline)) {
+        constexpr int WR = decltype(wr)::value * SLOTS;
+        __builtin_amdgcn_sched_barrier(0);
+        static_for<STEPS>([&](auto step) __attribute__((always_inline)) {
+            constexpr int st = decltype(step)::value, pr = st / (TM * TN), a = (st / TN) % TM, b = st % TN;
+            mma_bf16(acc[a][b], cur.a[f3_pa(pr)][a], cur.b[f3_pb(pr)][b]);
+            static_for<4>([&](auto phase) __attribute__((always_inline)) {
+                constexpr int ph = decltype(phase)::value;
+                if constexpr (ph * (BAR - 1) / 4 == st) {
+                    stage_b(WR, phase, wr);
+                    if constexpr (ph == 1) {   // the unit's floats are used up
+                        issue_b(kt + 3, wr);
+                        prep_unit(kt + 4);
+                    }
+                }
+            });
+            if constexpr (st == 1 * TM * TN - 1) load_a(cur, kt + 2, 2);
+            if constexpr (st == 3 * TM * TN - 1) load_a(cur, kt + 2, 1);
+            if constexpr (st == 6 * TM * TN - 1) load_a(cur, kt + 2, 0);
+            static_for<READS>([&](auto i) __attribute__((always_inline)) {
+                if constexpr (st >= BAR && BAR + decltype(i)::value * (STEPS - BAR) / READS == st) read_operand(nxt, WR, i);
+            });
+            if constexpr (st == BAR - 1) __syncthreads();
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    // Two tiles a trip; behind an odd last tile runs one more, whose B is zero.  No test of reduction indices anywhere: beyond
+    // K the split weights are zero, and what B brings in there (the next row or image, zeros behind the tensor) is multiplied
+    // by that; should it not be finite, fix_nonfinite sums the elements over K alone.
+    for (int kt = 0; kt < k_tiles; kt += 2) {
+        body(op0, op1, kt, S1);
+        body(op1, op0, kt + 1, S0);
+    }
+#pragma unroll
+    for (int i = 0; i < (BM + NT - 1) / NT; ++i)
+        if (tid + i * NT < BM) s_bias[tid + i * NT] = bias_row[i];
+    __syncthreads();
+
+    const int m_wave = m0 + wm * (BM / WM), n_wave = n0 + wn * (BN / WN);
+    fix_nonfinite<BL, TM, TN>(p, acc, reinterpret_cast<float *>(lds) + wave * (32 * 33), ra, make_rsrc(b_base, b_bytes), m_wave, n_wave, lane, u_begin,
+                              klim);
+    if (p.partial && !whole_k) {
+        if (!p.arrive) {   // a finishing launch adds the slices up
+            write_partial<TM, TN, false>(p, acc, slice * gridDim.z + batch, m_wave, n_wave, li, lh);
+            return;
+        }
+        if (!reduce_in_launch<TM, TN>(p, acc, slice, batch, lid, m_wave, n_wave, li, lh, tid)) return;
+    }
+    const float *sb = s_bias + wm * (BM / WM);
+    auto store = [&](auto epi) __attribute__((always_inline)) {
+        constexpr int EPI = decltype(epi)::value;
+        if constexpr (BL == BL_ROWS) write_tile_rows<EPI, TM, TN, RES>(p, acc, m_wave, n_wave, li, lh, sb);
+        else write_tile<DT_F32, EPI, TM, TN, RES, true>(p, acc, batch, m_wave, n_wave, li, lh, sb);
+    };
+    switch (p.ep.act) {
+        case NOT_ACT:
+        case RELU6: store(std::integral_constant<int, EPI_NONE>{}); break;
+        case RELU: store(std::integral_constant<int, EPI_RELU>{}); break;
+        case CLIP: store(std::integral_constant<int, EPI_CLIP>{}); break;
+        case SILU:
+        case ONHIP_ACT_GELU_LUT: store(std::integral_constant<int, EPI_LUT>{}); break;
+        default: store(std::integral_constant<int, EPI_GENERIC>{}); break;
+    }
+}
+
+template <int BL, int BM, int BN, int WM, int WN, bool RES>
+static int f3_launch_one(const IgemmLaunch &cfg, const IgemmParams &p_in, hipStream_t stream) {
+    IgemmParams p = p_in;
+    dim3 grid;
+    const int rc = tile_grid<BM, BN>(cfg, p, &grid);
+    if (rc) return rc;
+    if (RES != (p.res != nullptr)) return set_error(ONHIP_ERR_ARG, "igemm: residual operand and kernel variant do not match");
+    hipLaunchKernelGGL((igemm_f3_kernel<BL, BM, BN, WM, WN, RES>), grid, dim3(64 * WM * WN), 0, stream, p);
+    ONHIP_CHECK_HIP(hipGetLastError());
+    return finish_launch<false>(cfg, p, stream);
+}
+
+template <int BL, bool RES>
+int f3_launch_tile(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t stream) {
+    switch (cfg.bm * 1000 + cfg.bn) {
+        case 256128: return f3_launch_one<BL, 256, 128, 8, 1, RES>(cfg, p, stream);
+        case 256064: return f3_launch_one<BL, 256, 64, 4, 1, RES>(cfg, p, stream);
+        case 128128: return f3_launch_one<BL, 128, 128, 4, 2, RES>(cfg, p, stream);
+        case 128064: return f3_launch_one<BL, 128, 64, 4, 1, RES>(cfg, p, stream);
+        case 64064: return f3_launch_one<BL, 64, 64, 2, 2, RES>(cfg, p, stream);
+        default: return set_error(ONHIP_ERR_ARG, "igemm f32: no kernel for tile %dx%d", cfg.bm, cfg.bn);
+    }
+}
+
+}  // namespace onhip

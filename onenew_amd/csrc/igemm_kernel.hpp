@@ -956,6 +956,107 @@ __device__ __forceinline__ void pw2_stage(const IgemmParams &p, const f32x16 &ac
     }
 }
 
+// which tile, and which slice of K, this workgroup computes
+struct TilePlace {
+    int m0, n0;      // first row and column
+    int lid, slice;
+    bool whole_k;    // a whole tile of a launch whose leftover tiles alone are cut along K
+};
+template <int BM, int BN>
+__device__ __forceinline__ TilePlace place_tile(const IgemmParams &p) {
+    // XCD-aware tile order: consecutive workgroup ids go round-robin over the 8 XCDs (each with its
+    // own L2); give every XCD a contiguous run of tiles so neighbours in (m, n) share an L2.
+    const int tiles_m = (p.M + BM - 1) / BM;
+    // A launch with dp_tiles > 0 has two kinds of workgroups: the first dp_tiles take one whole tile each (all of K,
+    // result written directly), the others take one of `split` K slices of one of the tail_tiles tiles left over and
+    // write partial sums.  Slices of one tile are tail_tiles workgroup ids apart, so they land on different CUs.
+    int lid, slice = blockIdx.y;
+    bool whole_k = false;
+    {
+        const int bid = blockIdx.x;
+        if (p.dp_tiles > 0 && bid >= p.dp_tiles) {
+            const int r = bid - p.dp_tiles;
+            slice = r / p.tail_tiles;
+            lid = p.dp_tiles + (r - slice * p.tail_tiles);
+        } else {
+            const int nb = p.dp_tiles > 0 ? p.dp_tiles : (int) gridDim.x;
+            const int q = nb >> 3, rmd = nb & 7, xcd = bid & 7, idx = bid >> 3;
+            lid = xcd * q + (xcd < rmd ? xcd : rmd) + idx;
+            whole_k = p.dp_tiles > 0;
+        }
+    }
+    int tile_n = (int) div31((unsigned) lid, p.div_tiles_m), tile_m = lid - tile_n * tiles_m;
+    if (p.n_fast && p.dp_tiles == 0) {   // uniform: rows of A stay in the XCD's L2 while it sweeps the column blocks
+        const int tiles_n = (p.N + BN - 1) / BN;
+        tile_m = (int) div31((unsigned) lid, p.div_tiles_n);
+        tile_n = lid - tile_m * tiles_n;
+    }
+    return {tile_m * BM, tile_n * BN, lid, slice, whole_k};
+}
+
+// Publishes this slice's partial sums and counts it in; true in the last of the tile's slices to arrive, whose accumulators
+// then hold the whole sum.
+template <int TM, int TN>
+__device__ __forceinline__ bool reduce_in_launch(const IgemmParams &p, f32x16 (&acc)[TM][TN], int slice, int batch, int lid, int m_wave,
+                                                 int n_wave, int li, int lh, int tid) {
+            write_partial<TM, TN, true>(p, acc, slice * gridDim.z + batch, m_wave, n_wave, li, lh);
+            // The reduction inside the launch.  Partial sums and counters live in uncached memory and are stored and
+            // loaded with system scope (AUX_SYSTEM_SCOPE): once this workgroup's stores are acknowledged (written
+            // through, vmcnt(0)) it counts itself in with a device-scope atomic, and the last of a tile's slices to arrive
+            // adds all of them up in slice order (the order of the finishing kernel: the same bits) with loads that
+            // bypass the caches, and goes on to the epilogue as if it had computed the whole tile.  Nobody waits for
+            // anybody, so the launch cannot hang; the counter is back at zero for the next launch.
+            __shared__ int s_last;
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            if (tid == 0) {
+                int *ctr = p.arrive + lid + batch * (int) gridDim.x;
+                const int old = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const int last = old == p.n_slices - 1;
+                if (last) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                s_last = last;
+            }
+            __syncthreads();
+            if (!s_last) return false;
+                        const int width = p.N - p.part_begin;
+                const bool m_edge = m_wave + TM * 32 > p.M;
+#pragma unroll
+                for (int a = 0; a < TM; ++a)
+#pragma unroll
+                    for (int b = 0; b < TN; ++b)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) acc[a][b][r] = 0;
+                for (int s = 0; s < p.n_slices; ++s) {
+                    const rsrc_t rp = make_rsrc(reinterpret_cast<const char *>(p.partial) +
+                                                (size_t) (s * gridDim.z + batch) * p.M * width * 4, RSRC_RANGE);
+                    // half a 32x32 block at a time: eight loads in flight, not sixteen per block of the tile, which would
+                    // cost the kernels registers and with them occupancy
+#pragma unroll
+                    for (int a = 0; a < TM; ++a)
+#pragma unroll
+                        for (int b = 0; b < TN; ++b) {
+                            const int n = n_wave + b * 32 + li;
+                            const unsigned cv = n < p.N ? (unsigned) (n - p.part_begin + 4 * lh * width) * 4u : OOB;
+#pragma unroll
+                            for (int h = 0; h < 2; ++h) {
+                                float v[8];
+#pragma unroll
+                                for (int q = 0; q < 8; ++q) {
+                                    const int r = 8 * h + q;
+                                    const int m_uni = m_wave + a * 32 + 8 * (r / 4) + (r % 4);
+                                    const bool row_ok = !m_edge || m_uni + 4 * lh < p.M;
+                                    v[q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                                        rp, row_ok ? cv : OOB, (unsigned) m_uni * (unsigned) width * 4u, AUX_SYSTEM_SCOPE));
+                                }
+#pragma unroll
+                                for (int q = 0; q < 8; ++q) acc[a][b][8 * h + q] = __fadd_rn(acc[a][b][8 * h + q], v[q]);
+                                __builtin_amdgcn_sched_barrier(0);
+                            }
+                        }
+                }
+    return true;
+}
+
 // ---- the kernel --------------------------------------------------------------------------------
 template <int DT, int BL, int BM, int BN, int WM, int WN, int PF = 1, bool RES = false, bool PW2 = false>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(PW2 ? 4 : 1))) void igemm_kernel(const IgemmParams p) {
@@ -995,34 +1096,9 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(PW2 ? 4
     const int li = lane & 31, lh = lane >> 5;
     const int wm = wave / WN, wn = wave % WN;
 
-    // XCD-aware tile order: consecutive workgroup ids go round-robin over the 8 XCDs (each with its
-    // own L2); give every XCD a contiguous run of tiles so neighbours in (m, n) share an L2.
-    const int tiles_m = (p.M + BM - 1) / BM;
-    // A launch with dp_tiles > 0 has two kinds of workgroups: the first dp_tiles take one whole tile each (all of K,
-    // result written directly), the others take one of `split` K slices of one of the tail_tiles tiles left over and
-    // write partial sums.  Slices of one tile are tail_tiles workgroup ids apart, so they land on different CUs.
-    int lid, slice = blockIdx.y;
-    bool whole_k = false;
-    {
-        const int bid = blockIdx.x;
-        if (p.dp_tiles > 0 && bid >= p.dp_tiles) {
-            const int r = bid - p.dp_tiles;
-            slice = r / p.tail_tiles;
-            lid = p.dp_tiles + (r - slice * p.tail_tiles);
-        } else {
-            const int nb = p.dp_tiles > 0 ? p.dp_tiles : (int) gridDim.x;
-            const int q = nb >> 3, rmd = nb & 7, xcd = bid & 7, idx = bid >> 3;
-            lid = xcd * q + (xcd < rmd ? xcd : rmd) + idx;
-            whole_k = p.dp_tiles > 0;
-        }
-    }
-    int tile_n = (int) div31((unsigned) lid, p.div_tiles_m), tile_m = lid - tile_n * tiles_m;
-    if (p.n_fast && p.dp_tiles == 0) {   // uniform: rows of A stay in the XCD's L2 while it sweeps the column blocks
-        const int tiles_n = (p.N + BN - 1) / BN;
-        tile_m = (int) div31((unsigned) lid, p.div_tiles_n);
-        tile_n = lid - tile_m * tiles_n;
-    }
-    const int m0 = tile_m * BM, n0 = tile_n * BN;
+    const TilePlace tp = place_tile<BM, BN>(p);
+    const int m0 = tp.m0, n0 = tp.n0, slice = tp.slice, lid = tp.lid;
+    const bool whole_k = tp.whole_k;
     const int batch = blockIdx.z;
     const int u_begin = whole_k ? 0 : slice * p.k_split_units;
     const int u_end = whole_k ? p.k_units : min(p.k_units, u_begin + p.k_split_units);
@@ -1307,63 +1383,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(PW2 ? 4
             write_partial<TM, TN, false>(p, acc, slice * gridDim.z + batch, m_wave, n_wave, li, lh);
             return;
         }
-        write_partial<TM, TN, true>(p, acc, slice * gridDim.z + batch, m_wave, n_wave, li, lh);
-        // The reduction inside the launch.  Partial sums and counters live in uncached memory and are stored and
-        // loaded with system scope (AUX_SYSTEM_SCOPE): once this workgroup's stores are acknowledged (written
-        // through, vmcnt(0)) it counts itself in with a device-scope atomic, and the last of a tile's slices to arrive
-        // adds all of them up in slice order (the order of the finishing kernel: the same bits) with loads that
-        // bypass the caches, and goes on to the epilogue as if it had computed the whole tile.  Nobody waits for
-        // anybody, so the launch cannot hang; the counter is back at zero for the next launch.
-        __shared__ int s_last;
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (tid == 0) {
-            int *ctr = p.arrive + lid + batch * (int) gridDim.x;
-            const int old = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const int last = old == p.n_slices - 1;
-            if (last) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            s_last = last;
-        }
-        __syncthreads();
-        if (!s_last) return;
-        if constexpr (DT != DT_I8) {
-            const int width = p.N - p.part_begin;
-            const bool m_edge = m_wave + TM * 32 > p.M;
-#pragma unroll
-            for (int a = 0; a < TM; ++a)
-#pragma unroll
-                for (int b = 0; b < TN; ++b)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[a][b][r] = 0;
-            for (int s = 0; s < p.n_slices; ++s) {
-                const rsrc_t rp = make_rsrc(reinterpret_cast<const char *>(p.partial) +
-                                            (size_t) (s * gridDim.z + batch) * p.M * width * 4, RSRC_RANGE);
-                // half a 32x32 block at a time: eight loads in flight, not sixteen per block of the tile, which would
-                // cost the kernels registers and with them occupancy
-#pragma unroll
-                for (int a = 0; a < TM; ++a)
-#pragma unroll
-                    for (int b = 0; b < TN; ++b) {
-                        const int n = n_wave + b * 32 + li;
-                        const unsigned cv = n < p.N ? (unsigned) (n - p.part_begin + 4 * lh * width) * 4u : OOB;
-#pragma unroll
-                        for (int h = 0; h < 2; ++h) {
-                            float v[8];
-#pragma unroll
-                            for (int q = 0; q < 8; ++q) {
-                                const int r = 8 * h + q;
-                                const int m_uni = m_wave + a * 32 + 8 * (r / 4) + (r % 4);
-                                const bool row_ok = !m_edge || m_uni + 4 * lh < p.M;
-                                v[q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                                    rp, row_ok ? cv : OOB, (unsigned) m_uni * (unsigned) width * 4u, AUX_SYSTEM_SCOPE));
-                            }
-#pragma unroll
-                            for (int q = 0; q < 8; ++q) acc[a][b][8 * h + q] = __fadd_rn(acc[a][b][8 * h + q], v[q]);
-                            __builtin_amdgcn_sched_barrier(0);
-                        }
-                    }
-            }
-        }
+        if constexpr (DT != DT_I8)
+            if (!reduce_in_launch<TM, TN>(p, acc, slice, batch, lid, m_wave, n_wave, li, lh, tid)) return;
     }
     if constexpr (DT == DT_I8) {
         // int8 NHWC output without the raw-accumulator copy: 128-bit stores through LDS (batch is 1 on this path)
@@ -1469,35 +1490,46 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(const IgemmParams p,
 }
 
 // ---- launch ------------------------------------------------------------------------------------------
-template <int DT, int BL, int BM, int BN, int WM, int WN, int PF = 1, bool RES = false>
-static int launch_one(const IgemmLaunch &cfg, const IgemmParams &p_in, hipStream_t stream) {
-    IgemmParams p = p_in;
+// the launch's grid, and the divisions of its kernel parameters
+template <int BM, int BN>
+static int tile_grid(const IgemmLaunch &cfg, IgemmParams &p, dim3 *grid) {
     const int tiles_m = (p.M + BM - 1) / BM;
     const int tiles = tiles_m * ((p.N + BN - 1) / BN);
     p.div_ohw = make_div31((unsigned) (p.OHW > 0 ? p.OHW : 1));
     p.div_ow = make_div31((unsigned) (p.OW > 0 ? p.OW : 1));
     p.div_tiles_m = make_div31((unsigned) tiles_m);
     p.div_tiles_n = make_div31((unsigned) ((p.N + BN - 1) / BN));
-    dim3 grid(tiles, cfg.split, cfg.batch);
+    *grid = dim3(tiles, cfg.split, cfg.batch);
     if (p.dp_tiles > 0) {   // whole tiles first, then the K slices of the leftover tiles (igemm_kernel)
         if (cfg.batch != 1 || p.dp_tiles + p.tail_tiles != tiles || !p.partial || p.part_begin != p.dp_tiles / tiles_m * BN)
             return set_error(ONHIP_ERR_ARG, "igemm: inconsistent leftover-tile launch");
-        grid = dim3(p.dp_tiles + p.tail_tiles * cfg.split, 1, 1);
+        *grid = dim3(p.dp_tiles + p.tail_tiles * cfg.split, 1, 1);
     }
-    if (RES != (p.res != nullptr)) return set_error(ONHIP_ERR_ARG, "igemm: residual operand and kernel variant do not match");
-    hipLaunchKernelGGL((igemm_kernel<DT, BL, BM, BN, WM, WN, PF, RES>), grid, dim3(THREADS), 0, stream, p);
-    ONHIP_CHECK_HIP(hipGetLastError());
+    return ONHIP_OK;
+}
+// the pass that adds up the K slices of a launch that does not do so itself
+template <bool IS_INT>
+static int finish_launch(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t stream) {
     if (p.partial && !p.arrive) {
         if (p.M > 4 * 65535 || cfg.batch > 65535)
             return set_error(ONHIP_ERR_ARG, "igemm: split-K with %d rows, %d batches", p.M, cfg.batch);
         const dim3 fgrid((p.N - p.part_begin + 63) / 64, (p.M + 3) / 4, cfg.batch);
-        if (DT == DT_I8)
-            hipLaunchKernelGGL((splitk_finish_kernel<true>), fgrid, dim3(64, 4), 0, stream, p, cfg.split, cfg.batch);
-        else
-            hipLaunchKernelGGL((splitk_finish_kernel<false>), fgrid, dim3(64, 4), 0, stream, p, cfg.split, cfg.batch);
+        hipLaunchKernelGGL((splitk_finish_kernel<IS_INT>), fgrid, dim3(64, 4), 0, stream, p, cfg.split, cfg.batch);
         ONHIP_CHECK_HIP(hipGetLastError());
     }
     return ONHIP_OK;
+}
+
+template <int DT, int BL, int BM, int BN, int WM, int WN, int PF = 1, bool RES = false>
+static int launch_one(const IgemmLaunch &cfg, const IgemmParams &p_in, hipStream_t stream) {
+    IgemmParams p = p_in;
+    dim3 grid;
+    const int rc = tile_grid<BM, BN>(cfg, p, &grid);
+    if (rc) return rc;
+    if (RES != (p.res != nullptr)) return set_error(ONHIP_ERR_ARG, "igemm: residual operand and kernel variant do not match");
+    hipLaunchKernelGGL((igemm_kernel<DT, BL, BM, BN, WM, WN, PF, RES>), grid, dim3(THREADS), 0, stream, p);
+    ONHIP_CHECK_HIP(hipGetLastError());
+    return finish_launch<DT == DT_I8>(cfg, p, stream);
 }
 
 template <int DT, int BL, int PF = 1, bool RES = false>

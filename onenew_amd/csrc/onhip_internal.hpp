@@ -124,6 +124,7 @@ enum { BL_GATHER = 0,  // element gather from NCHW activations (implicit im2col)
        BL_KVEC = 1,    // 16-byte vectors along K from NHWC int8 activations
        BL_PLAIN = 2,   // 1x1 filter without padding, or a row-major [K, N] matrix: no tap arithmetic
        BL_TAPC = 3,    // NCHW activations against tap-major packed weights: K = (tap, channel), one tap per unit
+       BL_ROWS = 5,     // igemm_f3_kernel.hpp only: rows of K contiguous floats (a product's left operand), ldb apart
        BL_KVEC_TAP = 4 };  // BL_KVEC whose K tiles never straddle a filter tap (units per tap a multiple of the
                            // tile, at most 64 taps): tap arithmetic is scalar and the K loop has no branches
 
@@ -159,7 +160,16 @@ struct IgemmParams {
     const void *A;
     long long a_batch_stride;  // elements; 0 = shared
     int lda;                   // elements between rows
+    // fp32: the same operand (a weight matrix shared by all batches) split into bf16 parts ahead of time, in the order the
+    // matrix instructions read it (igemm_f3_kernel.hpp), or nullptr
+    const void *a_split;
+    long long a_split_bytes;
+    // where that form can be made from on each call when the caller has none: element (row, k) at w_src[row * w_row + k * w_k]
+    // (nullptr: A is not a weight matrix)
+    const float *w_src;
+    long long w_row, w_k;
     // B
+    int ldb;                   // elements between rows (BL_ROWS)
     const void *B;
     long long b_batch_stride;  // elements
     // gather geometry (BL_GATHER)
@@ -251,6 +261,18 @@ int igemm_launch_f32_pw(const IgemmParams &p, hipStream_t stream);
 // fp32 kernel for plain problems with B rows contiguous along N (igemm_rowb.hip): tiles 64x128, 128x128, 64x256
 bool rowb_f32_ok(const IgemmLaunch &cfg, const IgemmParams &p);
 int rowb_f32_launch(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t stream);
+// fp32 kernel on the 16-bit matrix cores (igemm_f3.hip): p.a_split holds the weights in split_weights_launch's form
+int f3_launch(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t stream);
+inline long long split_weights_bytes(long long M, long long K) { return (M + 31) / 32 * ((K + 15) / 16) * 3072; }
+// api.hip: fp32 convolution and product on weights that are split already (the plugins'), and how to split them
+struct SplitSource { int M, K; long long s_row, s_k; };
+SplitSource conv2d_f32_split_source(const onhip_conv_desc_t *d, int packed);
+int conv2d_f32_split(const onhip_conv_desc_t *d, const float *x, const float *w, int packed, const float *bias, const float *silu_lut,
+                     const float *addend, int relu_after, float *y, const void *split, void *stream);
+SplitSource matmul_f32_split_source(const onhip_matmul_desc_t *d);
+int matmul_f32_split(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias, const float *gelu_lut, const float *addend,
+                     float *out, const void *split, void *stream);
+int split_weights_launch(const float *w, int M, int K, long long s_row, long long s_k, void *out, hipStream_t stream);
 // int8 kernel with operand tiles loaded from global memory straight into LDS (igemm_dma.hip): NHWC int8 activations whose
 // padded channel count is a multiple of 64, tiles 128x128, 128x64, 64x128, 64x64, no split-K
 bool dma_ok(const IgemmLaunch &cfg, const IgemmParams &p);

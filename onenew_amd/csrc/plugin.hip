@@ -11,9 +11,12 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
+#include <iterator>
 #include <map>
 #include <mutex>
 #include <utility>
+#include <vector>
 
 #include "onhip_internal.hpp"
 
@@ -103,7 +106,69 @@ struct PackedEntry {
 };
 static std::map<const void *, PackedEntry> g_packed;
 
+// Weights in the form of the fp32 kernel on the 16-bit matrix cores (igemm_f3.hip), keyed by the device address of the
+// original: those of a loaded model (onhip_plugin_hold), and those uploaded here from host memory.  They live in blocks of
+// at least 32 MiB that are given back when the last of their tensors is dropped.
+struct SplitBlock { char *base; size_t size, used; int live; };
+struct SplitEntry { void *dev; SplitSource src; SplitBlock *block; };
+static std::map<const void *, SplitEntry> g_split;
+static std::vector<SplitBlock *> g_split_blocks;
+static std::vector<std::pair<const char *, const char *>> g_held;   // address ranges of loaded models' weights
+
+static bool is_held(const void *p) {
+    for (const auto &r : g_held)
+        if (static_cast<const char *>(p) >= r.first && static_cast<const char *>(p) < r.second) return true;
+    return false;
+}
+static void drop_split(std::map<const void *, SplitEntry>::iterator it) {
+    SplitBlock *b = it->second.block;
+    g_split.erase(it);
+    if (--b->live) return;
+    (void) hipFree(b->base);
+    g_split_blocks.erase(std::find(g_split_blocks.begin(), g_split_blocks.end(), b));
+    delete b;
+}
+// *out = the split form of the weights `key` (laid out as `from` and ss say), made when first asked for; nullptr where there
+// is none (ss.M == 0)
+static int split_of(const void *key, const float *from, const SplitSource &ss, const void **out) {
+    *out = nullptr;
+    if (!ss.M) return ONHIP_OK;
+    auto it = g_split.find(key);
+    if (it != g_split.end()) {
+        const SplitSource &h = it->second.src;
+        if (h.M == ss.M && h.K == ss.K && h.s_row == ss.s_row && h.s_k == ss.s_k) { *out = it->second.dev; return ONHIP_OK; }
+        ONHIP_CHECK_HIP(hipDeviceSynchronize());
+        drop_split(it);
+    }
+    const size_t bytes = ((size_t) split_weights_bytes(ss.M, ss.K) + 255) / 256 * 256;
+    SplitBlock *block = nullptr;
+    for (SplitBlock *b : g_split_blocks)
+        if (b->size - b->used >= bytes) block = b;
+    if (!block) {
+        block = new SplitBlock{nullptr, bytes > (32u << 20) ? bytes : (32u << 20), 0, 0};
+        const hipError_t e = hipMalloc(reinterpret_cast<void **>(&block->base), block->size);
+        if (e != hipSuccess) {
+            delete block;
+            return set_error(ONHIP_ERR_RUNTIME, "split weights: hipMalloc failed: %s", hipGetErrorString(e));
+        }
+        g_split_blocks.push_back(block);
+    }
+    void *dev = block->base + block->used;
+    block->used += bytes;
+    ++block->live;
+    it = g_split.emplace(key, SplitEntry{dev, ss, block}).first;
+    const int rc = split_weights_launch(from, ss.M, ss.K, ss.s_row, ss.s_k, dev, g_stream);
+    if (rc) { drop_split(it); return rc; }
+    *out = dev;
+    return ONHIP_OK;
+}
+
 static void drop_packed(const void *w_dev) {
+    auto sp = g_split.find(w_dev);
+    if (sp != g_split.end()) {
+        (void) hipDeviceSynchronize();   // a kernel may still be reading it, and its block need not be freed now
+        drop_split(sp);
+    }
     auto it = g_packed.find(w_dev);
     if (it != g_packed.end()) {
         (void) hipFree(it->second.dev);
@@ -322,6 +387,8 @@ static int conv_eval_fused(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_
     if (rc) return rc;
     // int8 weights sit at the front of the fp32-sized buffer, the int32 bias in the fp32 bias buffer
     rc = const_on_device(reinterpret_cast<const void *>(inputs[1].addr), int8 ? w_elems : w_elems * 4, &w);
+    // weights that stay as they are: a loaded model's, or uploaded from host memory (compared on every call)
+    const bool keep_split = w != reinterpret_cast<const void *>(inputs[1].addr) || is_held(w);
     if (rc) return rc;
     if (d.has_bias) {
         rc = const_on_device(reinterpret_cast<const void *>(inputs[2].addr), (size_t) d.cout * 4, &b);
@@ -399,20 +466,20 @@ static int conv_eval_fused(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_
     } else if (fuse) {
         const float *wp = nullptr;
         rc = packed_weights(&d, (const float *) w, &wp);
+        const void *split = nullptr;
+        if (!rc && keep_split) rc = split_of(w, wp ? wp : (const float *) w, conv2d_f32_split_source(&d, wp != nullptr), &split);
         if (rc) return rc;
-        rc = onhip_conv2d_f32_add(&d, (const float *) x, wp ? wp : (const float *) w, wp ? 1 : 0, (const float *) b,
-                                  (const float *) lut, (const float *) addend, fuse == 2, (float *) y, g_stream);
+        rc = conv2d_f32_split(&d, (const float *) x, wp ? wp : (const float *) w, wp ? 1 : 0, (const float *) b, (const float *) lut,
+                              (const float *) addend, fuse == 2, (float *) y, split, g_stream);
     } else {
         // k x k dense weights are re-laid out tap-major once, next to their device copy
         const float *wp = nullptr;
         rc = packed_weights(&d, (const float *) w, &wp);
+        const void *split = nullptr;
+        if (!rc && keep_split) rc = split_of(w, wp ? wp : (const float *) w, conv2d_f32_split_source(&d, wp != nullptr), &split);
         if (rc) return rc;
-        if (wp)
-            rc = onhip_conv2d_f32_packed(&d, (const float *) x, wp, (const float *) b, (const float *) lut, (float *) y,
-                                         g_stream);
-        else
-            rc = onhip_conv2d_f32(&d, (const float *) x, (const float *) w, (const float *) b, (const float *) lut,
-                                  (float *) y, g_stream);
+        rc = conv2d_f32_split(&d, (const float *) x, wp ? wp : (const float *) w, wp ? 1 : 0, (const float *) b, (const float *) lut, nullptr, 0,
+                              (float *) y, split, g_stream);
     }
     if (rc) return rc;
     if (!out_on_dev) return copy_out(host_out, y, out_bytes);
@@ -629,6 +696,11 @@ static int matmul_eval_mode(int mode, BUFFER_INFO_S *params, BUFFER_INFO_S *inpu
     if (b_t->is_fixed_val) rc = const_on_device(b_host, b_bytes, &b);
     else rc = input_on_device(1, b_host, b_bytes, &b);
     if (rc) return rc;
+    const void *split = nullptr;
+    if (b_t->is_fixed_val && (b != b_host || is_held(b))) {
+        rc = split_of(b, (const float *) b, matmul_f32_split_source(&d), &split);
+        if (rc) return rc;
+    }
     void *host_out = reinterpret_cast<void *>(outputs[0].addr);
     void *y = host_out;
     const bool out_on_dev = is_device_ptr(host_out);
@@ -652,9 +724,9 @@ static int matmul_eval_mode(int mode, BUFFER_INFO_S *params, BUFFER_INFO_S *inpu
         const void *addend;
         rc = input_on_device(5, reinterpret_cast<const void *>(inputs[3].addr), o_bytes, &addend);
         if (rc) return rc;
-        rc = onhip_matmul_add(&d, (const float *) a, (const float *) b, (const float *) bias, (const float *) addend, (float *) y, g_stream);
+        rc = matmul_f32_split(&d, (const float *) a, (const float *) b, (const float *) bias, nullptr, (const float *) addend, (float *) y, split, g_stream);
     } else {
-        rc = onhip_matmul(&d, (const float *) a, (const float *) b, (const float *) bias, (const float *) lut, (float *) y, g_stream);
+        rc = matmul_f32_split(&d, (const float *) a, (const float *) b, (const float *) bias, (const float *) lut, nullptr, (float *) y, split, g_stream);
     }
     if (rc) return rc;
     if (!out_on_dev) return copy_out(host_out, y, o_bytes);
@@ -1185,7 +1257,26 @@ int onhip_plugin_forget(const void *base, size_t bytes) {
             ++it;
         }
     }
+    for (auto it = g_split.begin(); it != g_split.end();) {
+        const char *k = static_cast<const char *>(it->first);
+        auto next = std::next(it);
+        if (k >= lo && k < hi) {
+            if (!any) ONHIP_CHECK_HIP(hipDeviceSynchronize());
+            any = true;
+            drop_split(it);
+        }
+        it = next;
+    }
+    for (size_t i = g_held.size(); i-- > 0;)
+        if (g_held[i].first >= lo && g_held[i].second <= hi) g_held.erase(g_held.begin() + i);
     return forget_quantised_tables(base, bytes);
+}
+
+int onhip_plugin_hold(const void *base, size_t bytes) {
+    if (!base || !bytes) return set_error(ONHIP_ERR_ARG, "onhip_plugin_hold: empty range");
+    std::lock_guard<std::mutex> lock(g_mu);
+    g_held.emplace_back(static_cast<const char *>(base), static_cast<const char *>(base) + bytes);
+    return ONHIP_OK;
 }
 
 int onhip_plugin_trust_weights(int on) {
@@ -1199,6 +1290,7 @@ int onhip_plugin_release(void) {
     ONHIP_CHECK_HIP(hipDeviceSynchronize());
     for (auto &kv : g_packed) (void) hipFree(kv.second.dev);
     g_packed.clear();
+    while (!g_split.empty()) drop_split(g_split.begin());
     for (auto &kv : g_const) (void) hipFree(kv.second.dev);
     g_const.clear();
     for (auto &b : g_stage) {

@@ -159,6 +159,7 @@ struct onrt_net {
     std::string lib_dir;
     std::map<std::string, void *> handles;
     std::vector<set_async_fn> async_switches;
+    std::set<forget_fn> holders;      // plugins to tell where this net's weights lie
     std::set<forget_fn> forgetters;   // plugins that keep re-laid-out copies of device-resident weights
     std::set<set_stream_fn> stream_setters;
     size_t plugin_libs = 0;           // libraries bound; a graph needs every one of them to follow set_stream
@@ -431,6 +432,9 @@ int allocate(onrt_net &net) {
             t.desc.p_data = 0;
             off += (t.bytes + 255) & ~(size_t) 255;
         }
+        // they stay as they are until the net is freed (and the plugins told to forget them)
+        for (forget_fn f : net.holders)
+            if (f(net.init_arena, init_total)) return fail(ONRT_ERR_PLUGIN, "onhip_plugin_hold failed");
     }
     // operands: fp32 elements (elem_size * sizeof(float) in the reference), views excepted
     for (auto &kv : net.tensors) {
@@ -529,7 +533,10 @@ int bind_plugins(onrt_net &net) {
             it = net.handles.emplace(type, h).first;
             // our plugins can leave a device-resident output to stream order instead of waiting for it
             if (set_async_fn f = reinterpret_cast<set_async_fn>(dlsym(h, "onhip_plugin_set_async"))) net.async_switches.push_back(f);
-            if (forget_fn f = reinterpret_cast<forget_fn>(dlsym(h, "onhip_plugin_forget"))) net.forgetters.insert(f);
+            if (forget_fn f = reinterpret_cast<forget_fn>(dlsym(h, "onhip_plugin_forget"))) {
+                net.forgetters.insert(f);
+                if (forget_fn hold = reinterpret_cast<forget_fn>(dlsym(h, "onhip_plugin_hold"))) net.holders.insert(hold);
+            }
             ++net.plugin_libs;
             if (set_stream_fn f = reinterpret_cast<set_stream_fn>(dlsym(h, "onhip_plugin_set_stream"))) net.stream_setters.insert(f);
             else net.graph_refused = true;   // a plugin that launches where it likes cannot be recorded

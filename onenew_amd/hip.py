@@ -46,7 +46,7 @@ EXPORTS = ["onhip_init", "onhip_last_error", "onhip_set_tuning", "onhip_split_ta
            "onhip_gelu_lut_f32", "onhip_layernorm_f32", "onhip_softmax_f32", "onhip_transpose_f32",
            "onhip_conv_eval", "onhip_matmul_eval", "onhip_matmul_attention_eval", "onhip_matmul_bias_eval", "onhip_matmul_bias_gelu_eval", "onhip_matmul_bias_add_eval", "onhip_gemm_eval", "onhip_add_eval", "onhip_relu_eval",
            "onhip_maxpool_eval", "onhip_global_avgpool_eval", "onhip_gelu_eval", "onhip_layernorm_eval",
-           "onhip_softmax_eval", "onhip_transpose_eval", "onhip_plugin_set_async", "onhip_plugin_set_stream", "onhip_plugin_forget", "onhip_plugin_trust_weights", "onhip_plugin_release"]
+           "onhip_softmax_eval", "onhip_transpose_eval", "onhip_plugin_set_async", "onhip_plugin_set_stream", "onhip_plugin_forget", "onhip_plugin_hold", "onhip_plugin_trust_weights", "onhip_plugin_release"]
 
 
 def load():
@@ -103,6 +103,7 @@ def load():
     L.onhip_gemm_f32.argtypes = [C.c_int32, C.c_int32, C.c_int32, vp, vp, vp, vp, vp]
     L.onhip_copy_f32.argtypes = [vp, vp, C.c_longlong, vp]
     L.onhip_plugin_forget.argtypes = [vp, C.c_size_t]
+    L.onhip_plugin_hold.argtypes = [vp, C.c_size_t]
     i32 = C.c_int32
     L.onhip_h16_pitch.argtypes = [i32]
     L.onhip_h16_packed_weight_bytes.argtypes = [i32, i32, i32]
