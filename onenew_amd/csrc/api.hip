@@ -11,6 +11,8 @@
 #include <atomic>
 #include <map>
 #include <mutex>
+#include <thread>
+#include <utility>
 #include <vector>
 
 #include "onhip_internal.hpp"
@@ -131,19 +133,38 @@ static int get_scratch(size_t bytes, void **out) {
     return ONHIP_OK;
 }
 
-// Split weights of a call whose caller has none (launch_choice): one block per process, allocated at first use and never
-// outgrown (weights whose split form is larger run the other fp32 kernels); the entry point that allocates nothing has its own.
+// Split weights of a call whose caller has none (launch_choice).  A stream keeps the slot that its first such call took and
+// allocated, since launches on two streams may overlap; the per-thread default stream is one for each thread.  Slots are kept
+// until the process ends, as recorded graphs hold their addresses, eight at most.  A stream that finds all slots taken or that
+// is being captured before it has one, and weights whose split form is larger than a slot, run the other fp32 kernels.  The
+// pass that splits and the launch that reads follow each other on the stream while g_split_mu is held: another thread's calls
+// on the same stream go before both or behind both.  The entry point that allocates nothing takes part of its own array.
 static const long long kSplitWsBytes = 16LL << 20;
-static __device__ __align__(256) unsigned char split_scratch[kSplitWsBytes];
-static void *g_split_ws = nullptr;
-static int get_split_ws(void **out) {
-    if (tl_noalloc) {
-        ONHIP_CHECK_HIP(hipGetSymbolAddress(out, HIP_SYMBOL(split_scratch)));
+static const size_t kSplitSlots = 8;
+static std::mutex g_split_mu;
+struct SplitSlot { int dev; hipStream_t stream; std::thread::id thread; void *mem; };
+static std::vector<SplitSlot> g_split_slots;
+// *out = the slot of stream st on the current device, nullptr if there is none; g_split_mu held
+static int split_slot(hipStream_t st, long long bytes, void **out) {
+    if (tl_noalloc) {   // the last part of its array: f3_choice leaves the partial sums the rest
+        *out = static_cast<char *>(tl_noalloc) + kNoAllocScratchBytes - bytes;
         return ONHIP_OK;
     }
-    std::lock_guard<std::mutex> lock(g_scratch_mu);
-    if (!g_split_ws) ONHIP_CHECK_HIP(hipMalloc(&g_split_ws, kSplitWsBytes));
-    *out = g_split_ws;
+    int dev = -1;
+    ONHIP_CHECK_HIP(hipGetDevice(&dev));
+    const std::thread::id me = st == hipStreamPerThread ? std::this_thread::get_id() : std::thread::id();
+    *out = nullptr;
+    for (const SplitSlot &s : g_split_slots)
+        if (s.dev == dev && s.stream == st && s.thread == me) *out = s.mem;
+    if (*out || g_split_slots.size() == kSplitSlots) return ONHIP_OK;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return ONHIP_OK;
+    if (hipMalloc(out, kSplitWsBytes) != hipSuccess) {
+        (void) hipGetLastError();   // no memory for it: as without a slot
+        *out = nullptr;
+        return ONHIP_OK;
+    }
+    g_split_slots.push_back({dev, st, me, *out});
     return ONHIP_OK;
 }
 
@@ -257,7 +278,7 @@ static double tile_mfma_cycles(int dt, int bm, int bn) {
     return flops / per_clk;
 }
 
-static int apply_choice(IgemmLaunch &cfg, IgemmParams &p, const Choice &c) {
+static int apply_choice(IgemmLaunch &cfg, IgemmProblem &p, const Choice &c) {
     cfg.bm = c.bm; cfg.bn = c.bn; cfg.split = 1;
     p.k_split_units = p.k_units;
     p.partial = nullptr;
@@ -296,7 +317,7 @@ static int apply_choice(IgemmLaunch &cfg, IgemmParams &p, const Choice &c) {
 // rounds) are whole tiles, each of the remaining tiles is cut along K into slices so that the leftover, too, puts about
 // one small workgroup on every CU.  (Running the leftover as a second launch on another stream was tried first: the
 // cross-queue event waits cost more than the balance gained.)
-static bool tail_geometry(const IgemmLaunch &cfg, const IgemmParams &p, int bm, int bn, int *dp_cols, int *tail_tiles) {
+static bool tail_geometry(const IgemmLaunch &cfg, const IgemmProblem &p, int bm, int bn, int *dp_cols, int *tail_tiles) {
     if (cfg.batch != 1 || cfg.dtype == DT_I8) return false;
     const int tiles_m = (p.M + bm - 1) / bm, cols = (p.N + bn - 1) / bn;
     const long long tiles = (long long) tiles_m * cols;
@@ -327,7 +348,7 @@ static bool tile_exists(const Choice &c) {
 }
 
 // the fp32 kernel on the 16-bit matrix cores: a weight matrix for A, split already or small enough to be split on the call
-static bool f3_ok(const IgemmLaunch &cfg, const IgemmParams &p) {
+static bool f3_ok(const IgemmLaunch &cfg, const IgemmProblem &p) {
     static const bool off = getenv("ONHIP_NO_F3") != nullptr;   // tuning hook: fp32 matrix instructions only
     if (off || cfg.dtype != DT_F32 || cfg.batch != 1 || (!p.a_split && !p.w_src)) return false;
     if (cfg.bl != BL_PLAIN && cfg.bl != BL_TAPC && cfg.bl != BL_GATHER && cfg.bl != BL_ROWS) return false;
@@ -335,7 +356,7 @@ static bool f3_ok(const IgemmLaunch &cfg, const IgemmParams &p) {
     return bytes < (1LL << 31) && (p.a_split || bytes <= kSplitWsBytes);
 }
 
-static bool candidate_ok(const IgemmLaunch &cfg, const IgemmParams &p, const Choice &c) {
+static bool candidate_ok(const IgemmLaunch &cfg, const IgemmProblem &p, const Choice &c) {
     if (!tile_exists(c)) return false;   // e.g. a line of the cache file written by another build or by hand
     const int k_tiles = (p.k_units + k_tile_units(cfg.dtype) - 1) / k_tile_units(cfg.dtype);
     const bool h16 = cfg.dtype != DT_I8 && (cfg.bl == BL_KVEC || cfg.bl == BL_KVEC_TAP);   // 16-bit storage: that kernel only
@@ -366,7 +387,7 @@ static bool candidate_ok(const IgemmLaunch &cfg, const IgemmParams &p, const Cho
 // Cost model (cycles).  A CU works through its share of the workgroups; co-resident workgroups share
 // the MFMA pipes, so the MFMA time adds up while the per-workgroup fill/drain latency overlaps when
 // several are resident.  Split-K adds the partial-sum traffic and a second launch.
-static double model_cost(const IgemmLaunch &cfg, const IgemmParams &p, const Choice &c) {
+static double model_cost(const IgemmLaunch &cfg, const IgemmProblem &p, const Choice &c) {
     const long long tiles = (long long) ((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn) * cfg.batch;
     const int k_tiles = (p.k_units + 3) / 4;
     const int per = (k_tiles + c.split - 1) / c.split;
@@ -398,7 +419,7 @@ static thread_local int tl_hint_bm = 0, tl_hint_bn = 0;
 // register-staged kernel wherever it has work for most of the CUs): the largest tile that still gives every CU a
 // workgroup and then some.  Problems with so few tiles that only a split along K reaches all CUs stay with the
 // register-staged kernel, which has one.
-static bool dma_model_choice(const IgemmLaunch &cfg, const IgemmParams &p, Choice *out) {
+static bool dma_model_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out) {
     static const int order[4][2] = {{128, 128}, {128, 64}, {64, 128}, {64, 64}};
     // what a tile's steady state costs per output against the largest one's (measured on the YOLOv8s layers)
     static const double eff[4] = {1.0, 1.08, 1.10, 1.20};
@@ -430,7 +451,7 @@ static bool dma_model_choice(const IgemmLaunch &cfg, const IgemmParams &p, Choic
 // 1100 timed launches over the layers of ResNet-50 (batch 1, 8, 32) and MobileNetV2 (batch 8, 64), median error 10 %, the
 // choices within 2 % of the fastest: a compute unit works through its workgroups at a rate that depends on the tile alone
 // (larger tiles stage less per multiply-add), whether one or several are resident.
-static bool f3_choice(const IgemmLaunch &cfg, const IgemmParams &p, Choice *out, double *us) {
+static bool f3_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out, double *us) {
     static const double per_k_tile[kNumF3Tiles] = {0.82, 0.50, 0.50, 0.29, 0.215};   // per K tile of 16 and workgroup
     static const double per_tile[kNumF3Tiles] = {3.8, 1.8, 1.25, 0.70, 0.37};        // first loads and store of a workgroup
     *us = 1e300;
@@ -440,6 +461,7 @@ static bool f3_choice(const IgemmLaunch &cfg, const IgemmParams &p, Choice *out,
             if (c.bm > 64 && p.M <= c.bm / 2) continue;
             if (c.split > 1 && cfg.bl == BL_ROWS) continue;
             if (!candidate_ok(cfg, p, c)) continue;
+            if (tl_noalloc && c.split > 1 && 4LL * c.split * p.M * p.N + split_weights_bytes(p.M, p.K) > (long long) kNoAllocScratchBytes) continue;
             const int k_tiles = (p.k_units + 3) / 4, per = (k_tiles + c.split - 1) / c.split;
             const double tiles = (double) ((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn);
             double t_us = 4.2 + ceil(tiles * c.split / 256.0) * (per * per_k_tile[t] + per_tile[t]);
@@ -453,7 +475,7 @@ static bool f3_choice(const IgemmLaunch &cfg, const IgemmParams &p, Choice *out,
 // the same for the fp32 matrix instructions' kernels (2250 cycles of model_cost take a microsecond; same launches, error 10 %)
 static double f32_us(double cycles) { return 3.75 + cycles / 2250.0; }
 
-static Choice model_choice(const IgemmLaunch &cfg, const IgemmParams &p) {
+static Choice model_choice(const IgemmLaunch &cfg, const IgemmProblem &p) {
     Choice best = {64, 64, 1, 0, 0, 0};
     const bool vec = cfg.bl == BL_KVEC || cfg.bl == BL_KVEC_TAP;
     if (vec && (cfg.dtype != DT_I8 || !tl_hint_bm) && dma_model_choice(cfg, p, &best)) return best;
@@ -528,12 +550,33 @@ static std::atomic<long long> g_dma_launches{0};
 // slices of the leftover tiles, and which kernel
 static thread_local int tl_last_choice[7] = {0, 0, 0, 0, 0, 0, 0};
 
+// launch_choice of a problem in the form that only the fp32 kernel on the 16-bit matrix cores reads (matmul_rows_problem):
+// this stream has no slot for the split weights, nothing was launched
+static const int kNoSplitSlot = 1;
+
 // Runs the problem the way the choice says.
-static int launch_choice(IgemmLaunch cfg, IgemmParams p, const Choice &c, hipStream_t st) {
+static int launch_choice(IgemmLaunch cfg, IgemmProblem p, const Choice &c, hipStream_t st) {
+    std::unique_lock<std::mutex> split_lock(g_split_mu, std::defer_lock);
+    if (c.rowb == 2 && !p.a_split) {
+        split_lock.lock();
+        void *ws = nullptr;
+        int rc = split_slot(st, split_weights_bytes(p.M, p.K), &ws);
+        if (rc) return rc;
+        if (!ws) {
+            if (!p.A) return kNoSplitSlot;   // only this kernel reads the problem in this form
+            split_lock.unlock();
+            p.w_src = nullptr;               // as a call whose weights are too large to be split
+            return launch_choice(cfg, p, model_choice(cfg, p), st);
+        }
+        rc = split_weights_launch(p.w_src, p.M, p.K, p.w_row, p.w_k, ws, st);
+        if (rc) return rc;
+        p.a_split = ws;
+        p.a_split_bytes = split_weights_bytes(p.M, p.K);
+    }
     int dpc = 0, left = 0;
     p.part_begin = p.dp_tiles = p.tail_tiles = 0;
     struct Note {   // filled in on every way out of this function
-        const IgemmLaunch &cfg; const IgemmParams &p; const Choice &c;
+        const IgemmLaunch &cfg; const IgemmProblem &p; const Choice &c;
         ~Note() {
             const bool tail = p.tail_tiles > 0;
             const int v[7] = {c.bm, c.bn, c.dma || tail ? 1 : cfg.split, tail ? cfg.split : 0, c.dma ? 0 : c.rowb, p.arrive ? 1 : 0, c.dma};
@@ -548,14 +591,6 @@ static int launch_choice(IgemmLaunch cfg, IgemmParams p, const Choice &c, hipStr
         p.arrive = nullptr;
         g_dma_launches.fetch_add(1, std::memory_order_relaxed);
         return dma_launch(cfg, p, st);
-    }
-    if (c.rowb == 2 && !p.a_split) {
-        void *ws = nullptr;
-        int rc = get_split_ws(&ws);
-        if (!rc) rc = split_weights_launch(p.w_src, p.M, p.K, p.w_row, p.w_k, ws, st);
-        if (rc) return rc;
-        p.a_split = ws;
-        p.a_split_bytes = split_weights_bytes(p.M, p.K);
     }
     auto launch = [&]() {
         const int rc = c.rowb == 2 ? f3_launch(cfg, p, st) : c.rowb ? rowb_f32_launch(cfg, p, st) : igemm_launch(cfg, p, st);
@@ -586,7 +621,7 @@ static int launch_choice(IgemmLaunch cfg, IgemmParams p, const Choice &c, hipStr
     return launch();
 }
 
-static int time_choice(IgemmLaunch cfg, IgemmParams p, const Choice &c, hipStream_t st, hipEvent_t e0, hipEvent_t e1,
+static int time_choice(IgemmLaunch cfg, IgemmProblem p, const Choice &c, hipStream_t st, hipEvent_t e0, hipEvent_t e1,
                        float *best_ms) {
     int rc = launch_choice(cfg, p, c, st);   // warm-up
     if (rc) return rc;
@@ -608,7 +643,7 @@ static int time_choice(IgemmLaunch cfg, IgemmParams p, const Choice &c, hipStrea
 }
 
 // Chooses tile, split and tail handling for the problem and launches it.
-static int plan_and_launch(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t st) {
+static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t st) {
     // the entry point that allocates nothing: the cost model's choice (never the in-launch reduction, whose uncached
     // workspace is allocated on first use; no measuring, which creates events and may grow buffers)
     if (tl_noalloc) return launch_choice(cfg, p, model_choice(cfg, p), st);
@@ -904,7 +939,7 @@ static int conv2d_f32_impl(const onhip_conv_desc_t *d, const float *x, const flo
     rc = dtype_of_compute(d->compute, &cfg.dtype);
     if (rc) return rc;
     cfg.batch = 1;
-    IgemmParams p;
+    IgemmProblem p;
     memset(&p, 0, sizeof(p));
     const int kpu = kpu_of(cfg.dtype);
     p.M = d->cout;
@@ -1043,7 +1078,7 @@ int onhip_conv2d_pw_f32(const onhip_conv_desc_t *a, const onhip_conv_desc_t *b, 
     if (!x || !wa_packed || !wb_packed || !y || (a->has_bias && !bias_a) || (b->has_bias && !bias_b))
         return set_error(ONHIP_ERR_ARG, "conv + 1x1: null tensor pointer");
     if (addend == y) return set_error(ONHIP_ERR_ARG, "conv + 1x1: the addend may not be the output buffer");
-    IgemmParams p;
+    IgemmProblem p;
     memset(&p, 0, sizeof(p));
     const int cp = packed_cp(a);
     p.M = a->cout;
@@ -1260,7 +1295,7 @@ static int conv2d_w8a32_impl(const onhip_conv_desc_t *d, const float *x, const i
     cfg.dtype = DT_I8;
     cfg.bl = BL_KVEC;
     cfg.batch = 1;
-    IgemmParams p;
+    IgemmProblem p;
     memset(&p, 0, sizeof(p));
     p.M = d->cout;
     p.N = d->n * OH * OW;
@@ -1372,7 +1407,7 @@ int onhip_conv2d_w8_link(const onhip_conv_desc_t *d, const float *x, const int8_
 // the columns of `b` the rows of its A operand, the rows of `a` (K contiguous) its B, `out` [rows][n] written four columns at
 // a time
 static void matmul_rows_problem(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias, const float *gelu_lut,
-                                const float *addend, float *out, const void *split, IgemmLaunch *cfg, IgemmParams *p) {
+                                const float *addend, float *out, const void *split, IgemmLaunch *cfg, IgemmProblem *p) {
     memset(cfg, 0, sizeof(*cfg));
     cfg->dtype = DT_F32;
     cfg->bl = BL_ROWS;
@@ -1415,7 +1450,7 @@ static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float
     if (rc) return rc;
     cfg.bl = BL_PLAIN;
     cfg.batch = batch;
-    IgemmParams p;
+    IgemmProblem p;
     memset(&p, 0, sizeof(p));
     p.M = M; p.N = d->n; p.K = d->k;
     const int kpu = kpu_of(cfg.dtype);
@@ -1458,7 +1493,7 @@ static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float
     p.res = addend;   // laid out like the result; added after the bias, as the Add operator after it would
     if (cfg.dtype == DT_F32 && batch == 1 && !getenv("ONHIP_TILE")) {
         IgemmLaunch rcfg;
-        IgemmParams rp;
+        IgemmProblem rp;
         matmul_rows_problem(d, a, b, bias, gelu_lut, addend, out, split, &rcfg, &rp);
         Choice c;
         double us;
@@ -1468,7 +1503,8 @@ static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float
         if (rp.M > 32 && rp.K >= 48 && p.b_slice_bytes < (1LL << 31) && rp.b_slice_bytes < (1LL << 31) && rp.c_slice_bytes < (1LL << 31) &&
             f3_choice(rcfg, rp, &c, &us) && us < f32_us(model_cost(cfg, p, model_choice(cfg, p)))) {
             rp.a_split = split;
-            return launch_choice(rcfg, rp, c, st);
+            const int rc = launch_choice(rcfg, rp, c, st);
+            if (rc != kNoSplitSlot) return rc;
         }
     }
     return plan_and_launch(cfg, p, st);
@@ -1590,7 +1626,7 @@ static int conv2d_h16_impl(const onhip_conv_desc_t *d, const void *x, const void
         return set_error(ONHIP_ERR_ARG, "conv 16-bit: tensors of 2 GiB or more are not supported");
     cfg.bl = BL_KVEC;
     cfg.batch = 1;
-    IgemmParams p;
+    IgemmProblem p;
     memset(&p, 0, sizeof(p));
     p.M = d->cout;
     p.N = d->n * OH * OW;
@@ -1859,7 +1895,7 @@ SplitSource conv2d_f32_split_source(const onhip_conv_desc_t *d, int packed) {
     cfg.dtype = DT_F32;
     cfg.batch = 1;
     cfg.bl = packed ? BL_TAPC : plain_pointwise(d) ? BL_PLAIN : BL_GATHER;
-    IgemmParams p;
+    IgemmProblem p;
     memset(&p, 0, sizeof(p));
     p.M = d->cout;
     p.N = d->n * OH * OW;

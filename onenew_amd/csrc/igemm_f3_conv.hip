@@ -3,10 +3,10 @@
 
 namespace onhip {
 
-int f3_launch_tapc(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t stream) {
+int f3_launch_tapc(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t stream) {
     return p.res ? f3_launch_tile<BL_TAPC, true>(cfg, p, stream) : f3_launch_tile<BL_TAPC, false>(cfg, p, stream);
 }
-int f3_launch_gather(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t stream) {
+int f3_launch_gather(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t stream) {
     return p.res ? f3_launch_tile<BL_GATHER, true>(cfg, p, stream) : f3_launch_tile<BL_GATHER, false>(cfg, p, stream);
 }
 

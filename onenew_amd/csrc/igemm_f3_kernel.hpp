@@ -27,7 +27,7 @@
 //     six vector instructions each behind an MFMA of its own: 22 vector instructions per 12 to 24 MFMAs and wavefront.
 // Per K tile of the 128 x 64 tile a wavefront issues 12 MFMAs, 3 A loads, 4 B loads, 3 LDS stores and 6 LDS reads.
 //
-// Replaces, for the dense fp32 cases with enough work (f3_plan in api.hip): device/x86/Conv/conv.c im2col (:168,:260) +
+// Replaces, for the dense fp32 cases with enough work (f3_choice in api.hip): device/x86/Conv/conv.c im2col (:168,:260) +
 // opt_gemm.h SGEMM (:17) + bias sweep (:405) + do_act (:1216); device/x86/MatMul/mat_mul.c:10.
 #pragma once
 #include "igemm_kernel.hpp"
@@ -85,7 +85,7 @@ __device__ constexpr int f3_pb(int i) { constexpr int t[F3_PRODUCTS] = {0, 1, 0,
 
 // column n's share of the B addresses
 template <int BL>
-__device__ __forceinline__ ColState f3_col(const IgemmParams &p, int n) {
+__device__ __forceinline__ ColState f3_col(const IgemmProblem &p, int n) {
     if constexpr (BL == BL_ROWS) return {n < p.N ? (unsigned) (n * p.ldb) * 4u : OOB, 0, 0, 0u, 0u};
     else return make_col<BL>(p, n);
 }
@@ -93,7 +93,7 @@ __device__ __forceinline__ ColState f3_col(const IgemmParams &p, int n) {
 // Sums that are not finite, computed again in fp32: see the head of the file.  scratch: 32 x 33 floats of LDS private to the
 // wavefront.  Units u_begin .. of the reduction up to klim elements; operands through the K loop's own loads.
 template <int BL, int TM, int TN>
-__device__ __forceinline__ void fix_nonfinite(const IgemmParams &p, f32x16 (&acc)[TM][TN], float *scratch, rsrc_t ra, rsrc_t rb, int m_wave,
+__device__ __forceinline__ void fix_nonfinite(const IgemmProblem &p, f32x16 (&acc)[TM][TN], float *scratch, rsrc_t ra, rsrc_t rb, int m_wave,
                                               int n_wave, int lane, int u_begin, int klim) {
     float probe = 0.0f;   // stays zero while every sum is finite: 0 * inf and 0 * NaN are NaN
 #pragma unroll
@@ -155,7 +155,7 @@ __device__ __forceinline__ void fix_nonfinite(const IgemmParams &p, f32x16 (&acc
 // consecutive rows of the tile that a lane holds in registers 4 q .. 4 q + 3 are 16 contiguous bytes of C.  Residual and bias
 // as in write_tile.
 template <int EPI, int TM, int TN, bool RES>
-__device__ __forceinline__ void write_tile_rows(const IgemmParams &p, f32x16 (&acc)[TM][TN], int m_wave, int n_wave, int li, int lh,
+__device__ __forceinline__ void write_tile_rows(const IgemmProblem &p, f32x16 (&acc)[TM][TN], int m_wave, int n_wave, int li, int lh,
                                                 const float *sbias) {
     const rsrc_t rc = make_rsrc(p.C, (unsigned) p.c_slice_bytes), rr = make_rsrc(RES ? p.res : nullptr, RES ? (unsigned) p.c_slice_bytes : 0u);
 #pragma unroll
@@ -168,7 +168,7 @@ __device__ __forceinline__ void write_tile_rows(const IgemmParams &p, f32x16 (&a
             u32x4 rv[4];
             if constexpr (RES)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) rv[q] = __builtin_amdgcn_raw_buffer_load_b128(rr, base, 32u * q, 0);
+                for (int q = 0; q < 4; ++q) rv[q] = __builtin_amdgcn_raw_buffer_load_b128(rr, base + 32u * q, 0, 0);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const float4 bias = *reinterpret_cast<const float4 *>(sbias + a * 32 + 8 * q + 4 * lh);
@@ -182,11 +182,11 @@ __device__ __forceinline__ void write_tile_rows(const IgemmParams &p, f32x16 (&a
                 }
                 const int left = p.M - (m4 + 8 * q);   // columns of C from this group on
                 if (left >= 4) {
-                    __builtin_amdgcn_raw_buffer_store_b128(o, rc, base, 32u * q, 0);
+                    __builtin_amdgcn_raw_buffer_store_b128(o, rc, base + 32u * q, 0, 0);
                 } else {
 #pragma unroll
                     for (int j = 0; j < 3; ++j)
-                        if (j < left) __builtin_amdgcn_raw_buffer_store_b32(o[j], rc, base + 4u * j, 32u * q, 0);
+                        if (j < left) __builtin_amdgcn_raw_buffer_store_b32(o[j], rc, base + 32u * q + 4u * j, 0, 0);
                 }
             }
         }
@@ -195,7 +195,7 @@ __device__ __forceinline__ void write_tile_rows(const IgemmParams &p, f32x16 (&a
 
 template <int BL, int BM, int BN, int WM, int WN, bool RES>
 __global__ __launch_bounds__(64 * WM * WN, (BM / WM) * (BN / WN) >= 32 * 128 ? 2 : (BM / WM) * (BN / WN) >= 32 * 64 ? 3 : 4)
-void igemm_f3_kernel(const IgemmParams p) {
+void igemm_f3_kernel(const IgemmProblem p) {
     static_assert(BM % (WM * 32) == 0 && BN % (WN * 32) == 0, "wavefronts of 32 x 32 blocks");
     constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
     constexpr int UPT = 4, NT = 64 * WM * WN;
@@ -394,8 +394,8 @@ void igemm_f3_kernel(const IgemmParams p) {
 }
 
 template <int BL, int BM, int BN, int WM, int WN, bool RES>
-static int f3_launch_one(const IgemmLaunch &cfg, const IgemmParams &p_in, hipStream_t stream) {
-    IgemmParams p = p_in;
+static int f3_launch_one(const IgemmLaunch &cfg, const IgemmProblem &p_in, hipStream_t stream) {
+    IgemmProblem p = p_in;
     dim3 grid;
     const int rc = tile_grid<BM, BN>(cfg, p, &grid);
     if (rc) return rc;
@@ -406,7 +406,7 @@ static int f3_launch_one(const IgemmLaunch &cfg, const IgemmParams &p_in, hipStr
 }
 
 template <int BL, bool RES>
-int f3_launch_tile(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t stream) {
+int f3_launch_tile(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t stream) {
     switch (cfg.bm * 1000 + cfg.bn) {
         case 256128: return f3_launch_one<BL, 256, 128, 8, 1, RES>(cfg, p, stream);
         case 256064: return f3_launch_one<BL, 256, 64, 4, 1, RES>(cfg, p, stream);

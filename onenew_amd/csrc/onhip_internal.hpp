@@ -160,16 +160,7 @@ struct IgemmParams {
     const void *A;
     long long a_batch_stride;  // elements; 0 = shared
     int lda;                   // elements between rows
-    // fp32: the same operand (a weight matrix shared by all batches) split into bf16 parts ahead of time, in the order the
-    // matrix instructions read it (igemm_f3_kernel.hpp), or nullptr
-    const void *a_split;
-    long long a_split_bytes;
-    // where that form can be made from on each call when the caller has none: element (row, k) at w_src[row * w_row + k * w_k]
-    // (nullptr: A is not a weight matrix)
-    const float *w_src;
-    long long w_row, w_k;
     // B
-    int ldb;                   // elements between rows (BL_ROWS)
     const void *B;
     long long b_batch_stride;  // elements
     // gather geometry (BL_GATHER)
@@ -243,6 +234,20 @@ struct IgemmParams {
     Epilogue ep2;
 };
 
+// A problem as the host plans it: with what only the fp32 kernel on the 16-bit matrix cores (igemm_f3_kernel.hpp) takes as
+// well, so that the other kernels' parameters are no longer for it.
+struct IgemmProblem : IgemmParams {
+    // the operand A (a weight matrix shared by all batches) split into bf16 parts ahead of time, in the order the matrix
+    // instructions read it, or nullptr
+    const void *a_split;
+    long long a_split_bytes;
+    // where that form can be made from on each call when the caller has none: element (row, k) at w_src[row * w_row + k * w_k]
+    // (nullptr: A is not a weight matrix)
+    const float *w_src;
+    long long w_row, w_k;
+    int ldb;                   // B given as rows (BL_ROWS): elements between them
+};
+
 enum { DT_F32 = 0, DT_BF16 = 1, DT_F16 = 2, DT_I8 = 3 };
 
 struct IgemmLaunch {
@@ -262,7 +267,7 @@ int igemm_launch_f32_pw(const IgemmParams &p, hipStream_t stream);
 bool rowb_f32_ok(const IgemmLaunch &cfg, const IgemmParams &p);
 int rowb_f32_launch(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t stream);
 // fp32 kernel on the 16-bit matrix cores (igemm_f3.hip): p.a_split holds the weights in split_weights_launch's form
-int f3_launch(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t stream);
+int f3_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t stream);
 inline long long split_weights_bytes(long long M, long long K) { return (M + 31) / 32 * ((K + 15) / 16) * 3072; }
 // api.hip: fp32 convolution and product on weights that are split already (the plugins'), and how to split them
 struct SplitSource { int M, K; long long s_row, s_k; };

@@ -1,0 +1,128 @@
+"""fp32 convolutions and products on the 16-bit matrix cores (operands as three bf16 parts): every tile and loader at ragged
+sizes against 64-bit sums.  The bound is that of a chain of fp32 multiply-adds, K 2^-24 sum |a b|, plus what the three left-out
+partial products can reach, 2^-23 sum |a b|, and the roundings of the bias and the result."""
+import threading
+
+import numpy as np
+import pytest
+
+from onenew_amd import abi, hip
+from onenew_amd.abi import ConvDesc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch_dev():
+    import torch
+    hip.init(0)
+    return torch
+
+
+def conv_desc(n, cin, h, w, cout, k, stride, pad):
+    return ConvDesc(n=n, cin=cin, h=h, w=w, cout=cout, kh=k, kw=k, stride_h=stride, stride_w=stride, pad_t=pad, pad_l=pad, pad_b=pad, pad_r=pad,
+                    group=1, has_bias=1, act_type=abi.NOT_ACT, compute=abi.COMPUTE_F32)
+
+
+def check(got, ref, magnitude, k):
+    """got within the bound of ref (fp64), non-finite where ref is; magnitude: sum |a b| + |bias| in fp64"""
+    got = got.double().cpu()
+    bad = ~ref.isfinite()
+    assert bool((got.isnan() == ref.isnan()).all()) and bool((got[bad & ~ref.isnan()] == ref[bad & ~ref.isnan()]).all())
+    err = (got - ref).abs()[~bad]
+    bound = (magnitude * ((k + 4) * 2.0 ** -24 + 2.0 ** -23))[~bad]
+    assert bool((err <= bound + 1e-38).all()), float((err / bound).max())
+
+
+def conv_ref(torch, d, x, w, b):
+    conv = lambda x, w, b: torch.nn.functional.conv2d(x.double().cpu(), w.double().cpu(), b.double().cpu(), stride=d.stride_h, padding=d.pad_t)  # noqa: E731
+    return conv(x, w, b), conv(x.abs(), w.abs(), b.abs())
+
+
+TILES = [(256, 128), (256, 64), (128, 128), (128, 64), (64, 64)]
+# loader, (n, cin, h, w, cout, filter, stride, pad): rows and columns off every tile, reductions off a K tile of 16 and off a unit of 4
+SHAPES = [("plain", (2, 109, 9, 23, 67, 1, 1, 0)), ("plain", (1, 130, 16, 17, 259, 1, 1, 0)), ("tapc", (2, 13, 11, 9, 97, 3, 1, 1)),
+          ("tapc", (1, 33, 15, 12, 260, 3, 2, 1)), ("gather", (1, 13, 13, 21, 65, 3, 1, 1)), ("gather", (2, 117, 14, 9, 40, 1, 2, 0))]
+
+
+@pytest.mark.parametrize("special", [False, True], ids=["finite", "special"])
+@pytest.mark.parametrize("split", [1, 3])
+@pytest.mark.parametrize("bm,bn", TILES)
+@pytest.mark.parametrize("loader,shape", SHAPES, ids=[f"{s[0]}{i}" for i, s in enumerate(SHAPES)])
+def test_convolution(loader, shape, bm, bn, split, special, torch_dev, monkeypatch):
+    torch = torch_dev
+    print(f"f3 {loader} {shape} tile {bm}x{bn} split {split} special {special}", flush=True)
+    monkeypatch.setenv("ONHIP_TILE", f"{bm}x{bn}x{split}x0x2")
+    d = conv_desc(*shape)
+    if special and loader == "tapc":
+        d.cin += -d.cin % 4   # packed weights round the channels up to four; what lies there (the next image) meets zero weights
+    g = torch.Generator().manual_seed(hash((shape, bm)) % 1000)
+    x = torch.randn(d.n, d.cin, d.h, d.w, generator=g)
+    w, b = torch.randn(d.cout, d.cin, d.kh, d.kw, generator=g) / (d.cin * d.kh * d.kw) ** 0.5, torch.randn(d.cout, generator=g)
+    if special:   # an infinity, a NaN, values that round to bf16 infinities (products with them stay finite)
+        x[0, 0, 1, 2], x[-1, 1, 3, 4], x[0, 2, 5, 5], w[5, 3] = float("inf"), float("nan"), 3.4e38, -3.4e38
+        x[:, 3] *= 1e-3
+    x, w, b = x.cuda(), w.cuda(), b.cuda()
+    wk = hip.pack_conv_weights(d, w) if loader == "tapc" else w
+    y = hip.conv2d_f32(d, x, wk, b, packed=loader == "tapc")
+    assert hip.last_launch_choice()[4] == 2
+    torch.cuda.synchronize()
+    ref, magnitude = conv_ref(torch, d, x, w, b)
+    if special:
+        ok = magnitude < 1e38   # sums that may overflow on the way are left to the infinities' and NaNs' own check
+        ref, got, magnitude = ref[ok | ~magnitude.isfinite()], y.cpu()[ok | ~magnitude.isfinite()], magnitude[ok | ~magnitude.isfinite()]
+        return check(got, ref, magnitude, d.cin * d.kh * d.kw)
+    check(y, ref, magnitude, d.cin * d.kh * d.kw)
+
+
+@pytest.mark.parametrize("m,k,n", [(4099, 1031, 2053), (8195, 773, 1030), (8190, 1029, 1027), (12545, 193, 768)])
+@pytest.mark.parametrize("special", [False, True], ids=["finite", "special"])
+def test_product(m, k, n, special, torch_dev):
+    torch = torch_dev
+    print(f"f3 product {m} x {k} x {n} special {special}", flush=True)
+    g = torch.Generator().manual_seed(m + k)
+    a, b, bias = torch.randn(m, k, generator=g), torch.randn(k, n, generator=g) / k ** 0.5, torch.randn(n, generator=g)
+    if special:
+        a[3, 5], a[m - 1, k - 1], b[7, n - 1] = float("inf"), float("nan"), -float("inf")
+    a, b, bias = a.cuda(), b.cuda(), bias.cuda()
+    y = hip.matmul(a, b, bias)
+    assert hip.last_launch_choice()[4] == 2
+    torch.cuda.synchronize()
+    check(y, (a.double() @ b.double() + bias.double()).cpu(), (a.double().abs() @ b.double().abs() + bias.double().abs()).cpu(), k)
+
+
+def test_streams_and_threads(torch_dev):
+    """weights split on the call: more streams than there are slots for them, one after another, and two threads on one stream"""
+    torch = torch_dev
+    print("f3 streams and threads", flush=True)
+    m, k, n = 8195, 773, 1030
+    g = torch.Generator(device="cuda").manual_seed(3)
+    jobs = []
+    for _ in range(10):
+        a, b = torch.randn(m, k, generator=g, device="cuda"), torch.randn(k, n, generator=g, device="cuda")
+        jobs.append((a, b, torch.empty(m, n, device="cuda"), (a.double() @ b.double()).cpu(), (a.double().abs() @ b.double().abs()).cpu()))
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in jobs]
+    for s, (a, b, y, _, _) in zip(streams, jobs):   # no cut along K: nothing but the split weights could be shared
+        with torch.cuda.stream(s):
+            hip.matmul(a, b, out=y)
+    torch.cuda.synchronize()
+
+    def verify():
+        for _, _, y, ref, magnitude in jobs:
+            check(y, ref, magnitude, k)
+            y.zero_()
+        torch.cuda.synchronize()
+    verify()
+
+    def work(mine):
+        for _ in range(8):
+            for a, b, y, _, _ in mine:
+                hip.matmul(a, b, out=y)
+    threads = [threading.Thread(target=work, args=(jobs[i::2],)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    verify()
