@@ -351,7 +351,7 @@ static bool tile_exists(const Choice &c) {
 static bool f3_ok(const IgemmLaunch &cfg, const IgemmProblem &p) {
     static const bool off = getenv("ONHIP_NO_F3") != nullptr;   // tuning hook: fp32 matrix instructions only
     if (off || cfg.dtype != DT_F32 || cfg.batch != 1 || (!p.a_split && !p.w_src)) return false;
-    if (cfg.bl != BL_PLAIN && cfg.bl != BL_TAPC && cfg.bl != BL_GATHER && cfg.bl != BL_ROWS) return false;
+    if (cfg.bl != BL_PLAIN && cfg.bl != BL_ROWS && !((cfg.bl == BL_TAPC || cfg.bl == BL_GATHER) && p.use_tapmask)) return false;
     const long long bytes = split_weights_bytes(p.M, p.K);
     return bytes < (1LL << 31) && (p.a_split || bytes <= kSplitWsBytes);
 }
@@ -406,7 +406,13 @@ static double model_cost(const IgemmLaunch &cfg, const IgemmProblem &p, const Ch
     // the fixed part of co-resident workgroups overlaps; a last, partly filled group of them pays its share of it, not
     // all of it (with all of it the 64 x 128 tile won over 64 x 64 on short-K layers, where it measures 15 % slower)
     double cycles = per_cu * mfma + per_cu / resident * fixed;
-    if (c.split > 1) cycles += 9000.0 + (double) (c.split + 1) * p.M * p.N * cfg.batch * 4.0 / 1500.0;
+    // int8 with up to two workgroups per CU: a K tile takes about 500 cycles (0.23 us) whatever its MFMAs, a workgroup's loads,
+    // LDS and barrier one after the other; the launch that adds slices up costs 2.8 us.  YOLOv8s at batch 1, the layers with
+    // a few tiles and a K of 2304 / 4608: 17.3-19.0 / 25.7 us in one piece, 13.7 / 14.5 us in four slices
+    // (int8 results stay whole: a launch in slices leaves the padding of their channels unwritten)
+    const bool few_int8 = cfg.dtype == DT_I8 && !p.out_s8 && wgs <= 512.0;
+    if (few_int8) cycles = fmax(cycles, ceil(per_cu / resident) * (per * 500.0 + fixed));
+    if (c.split > 1) cycles += (few_int8 ? 6300.0 : 9000.0) + (double) (c.split + 1) * p.M * p.N * cfg.batch * 4.0 / 1500.0;
     return cycles;
 }
 
@@ -1901,6 +1907,7 @@ SplitSource conv2d_f32_split_source(const onhip_conv_desc_t *d, int packed) {
     p.N = d->n * OH * OW;
     p.K = d->kh * d->kw * (packed ? packed_cp(d) : d->cin);
     p.k_units = (p.K + 3) / 4;
+    p.use_tapmask = d->kh * d->kw <= 64;
     p.a_split = &src;   // as if there were one
     if (model_choice(cfg, p).rowb == 2) src = {p.M, p.K, p.K, 1};
     return src;

@@ -90,6 +90,32 @@ __device__ __forceinline__ ColState f3_col(const IgemmProblem &p, int n) {
     else return make_col<BL>(p, n);
 }
 
+// prep_b and b_voff for the K loop: filters of at most 64 taps (f3_ok) and no test of the reduction index, so nothing that a
+// branch could come of (those stood between the MFMAs of every K tile).  Beyond K the tap's bit is clear, or another tap's:
+// what is read there meets zero weights.
+struct F3Prep { unsigned soff, tap; };
+template <int BL>
+__device__ __forceinline__ F3Prep f3_prep(const IgemmProblem &p, int u, int e) {
+    if constexpr (BL == BL_PLAIN) {
+        return {(unsigned) (u * 4 + e) * (unsigned) p.HW * 4u, 0u};
+    } else if constexpr (BL == BL_GATHER) {
+        const unsigned k = (unsigned) (u * 4 + e), ch = fast_div(k, p.magic_khkw, p.pass_khkw), tap = k - ch * (unsigned) p.khkw;
+        const unsigned i = fast_div(tap, p.magic_kw, p.pass_kw), j = tap - i * (unsigned) p.kw;
+        return {(ch * (unsigned) p.HW + i * (unsigned) p.W + j) * 4u, tap};
+    } else {
+        const unsigned tap = fast_div((unsigned) u, p.magic_upt, p.pass_upt), cb = (unsigned) u - tap * (unsigned) p.units_per_tap;
+        const unsigned i = fast_div(tap, p.magic_kw, p.pass_kw), j = tap - i * (unsigned) p.kw;
+        return {(cb * 4u * (unsigned) p.HW + i * (unsigned) p.W + j) * 4u, tap};
+    }
+}
+template <int BL>
+__device__ __forceinline__ unsigned f3_voff(const ColState &c, unsigned tap) {
+    if constexpr (BL == BL_PLAIN) return c.pixoff;
+    const unsigned long long taps = (unsigned long long) c.mask_hi << 32 | c.mask_lo;
+    const unsigned keep = 0u - ((unsigned) (taps >> (tap & 63u)) & 1u);
+    return (c.pixoff & keep) | (OOB & ~keep);
+}
+
 // Sums that are not finite, computed again in fp32: see the head of the file.  scratch: 32 x 33 floats of LDS private to the
 // wavefront.  Units u_begin .. of the reduction up to klim elements; operands through the K loop's own loads.
 template <int BL, int TM, int TN>
@@ -248,24 +274,23 @@ void igemm_f3_kernel(const IgemmProblem p) {
     constexpr int READS = 3 * TN;
     struct Operands { uint4 a[3][TM], b[3][TN]; };
     RawUnit<DT_F32> qb[2];                              // two K tiles in flight between memory and LDS
-    BPrep bp[BE];
+    F3Prep bp[BE];
     const unsigned hw4 = (unsigned) p.HW * 4u;
 
     auto prep_unit = [&](int kt) __attribute__((always_inline)) {
         if constexpr (BL != BL_ROWS)
 #pragma unroll
-            for (int e = 0; e < BE; ++e) bp[e] = prep_b<DT_F32, BL>(p, u_begin + kt * UPT + bunit, e, klim);
+            for (int e = 0; e < BE; ++e) bp[e] = f3_prep<BL>(p, u_begin + kt * UPT + bunit, e);
     };
     // the loads of B for K tile kt; a tile past the end reads through an empty descriptor (zeros, no traffic)
     auto issue_b = [&](int kt, auto slot) __attribute__((always_inline)) {
         RawUnit<DT_F32> &q = qb[decltype(slot)::value];
         const rsrc_t rb = make_rsrc(b_base, kt < k_tiles ? b_bytes : 0u);
-        const int u = u_begin + kt * UPT + bunit;
         if constexpr (BL == BL_ROWS) {
             const uint4 t = buf_load_b128(rb, col.pixoff + (unsigned) bunit * 16u, (unsigned) (u_begin + kt * UPT) * 16u);
             q.v[0] = __uint_as_float(t.x); q.v[1] = __uint_as_float(t.y); q.v[2] = __uint_as_float(t.z); q.v[3] = __uint_as_float(t.w);
         } else if constexpr (BL == BL_TAPC) {
-            const unsigned voff = b_voff<BL>(p, col, bp[0], u);
+            const unsigned voff = f3_voff<BL>(col, bp[0].tap);
 #pragma unroll
             for (int e = 0; e < 4; ++e) q.v[e] = buf_load_f32(rb, voff, bp[0].soff + (unsigned) e * hw4);
         } else if constexpr (BL == BL_PLAIN) {
@@ -273,7 +298,7 @@ void igemm_f3_kernel(const IgemmProblem p) {
             for (int e = 0; e < 4; ++e) q.v[e] = buf_load_f32(rb, col.pixoff, bp[0].soff + (unsigned) e * hw4);
         } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) q.v[e] = buf_load_f32(rb, b_voff<BL>(p, col, bp[e], u * 4 + e), bp[e].soff);
+            for (int e = 0; e < 4; ++e) q.v[e] = buf_load_f32(rb, f3_voff<BL>(col, bp[e].tap), bp[e].soff);
         }
     };
     auto load_a = [&](Operands &o, int kt, int part) __attribute__((always_inline)) {

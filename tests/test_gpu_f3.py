@@ -20,7 +20,8 @@ def torch_dev():
 
 
 def conv_desc(n, cin, h, w, cout, k, stride, pad):
-    return ConvDesc(n=n, cin=cin, h=h, w=w, cout=cout, kh=k, kw=k, stride_h=stride, stride_w=stride, pad_t=pad, pad_l=pad, pad_b=pad, pad_r=pad,
+    kh, kw = k if isinstance(k, tuple) else (k, k)
+    return ConvDesc(n=n, cin=cin, h=h, w=w, cout=cout, kh=kh, kw=kw, stride_h=stride, stride_w=stride, pad_t=pad, pad_l=pad, pad_b=pad, pad_r=pad,
                     group=1, has_bias=1, act_type=abi.NOT_ACT, compute=abi.COMPUTE_F32)
 
 
@@ -42,7 +43,7 @@ def conv_ref(torch, d, x, w, b):
 TILES = [(256, 128), (256, 64), (128, 128), (128, 64), (64, 64)]
 # loader, (n, cin, h, w, cout, filter, stride, pad): rows and columns off every tile, reductions off a K tile of 16 and off a unit of 4
 SHAPES = [("plain", (2, 109, 9, 23, 67, 1, 1, 0)), ("plain", (1, 130, 16, 17, 259, 1, 1, 0)), ("tapc", (2, 13, 11, 9, 97, 3, 1, 1)),
-          ("tapc", (1, 33, 15, 12, 260, 3, 2, 1)), ("gather", (1, 13, 13, 21, 65, 3, 1, 1)), ("gather", (2, 117, 14, 9, 40, 1, 2, 0))]
+          ("tapc", (1, 33, 15, 12, 260, 3, 2, 1)), ("gather", (1, 13, 13, 21, 65, 3, 1, 1)), ("tapc", (1, 20, 12, 13, 70, 7, 1, 3)), ("gather", (1, 6, 9, 14, 66, (5, 11), 2, 2)), ("gather", (2, 117, 14, 9, 40, 1, 2, 0))]
 
 
 @pytest.mark.parametrize("special", [False, True], ids=["finite", "special"])
