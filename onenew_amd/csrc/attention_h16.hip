@@ -21,11 +21,15 @@ struct AttnH16Params {
     float scale;
 };
 
-template <int DT, int NKT>
-__global__ __launch_bounds__(256, 2) void attention_h16_kernel(const AttnH16Params p) {
-    constexpr int HD = 64, KEYS = NKT * 32;
+// NW wavefronts of 32 queries each share one copy of k and v in LDS
+template <int DT, int NKT, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void attention_h16_kernel(const AttnH16Params p) {
+    constexpr int HD = 64, KEYS = NKT * 32, NT = 64 * NW;
     constexpr int LDK = HD + 8;       // 16-bit elements per key row of k (144 bytes: 16-byte reads of neighbouring rows spread over the banks)
-    constexpr int LDVT = KEYS + 8;    // 16-bit elements per channel row of v^T
+    // 16-bit elements per channel row of v^T.  KEYS is a multiple of 32, so rows are 2 (mod 16) dwords apart (the 8-byte reads of
+    // 32 rows touch every bank once) and 8 rows 16 (mod 64): the 16 key pairs of 4 channel groups that a wavefront writes together
+    // do as well
+    constexpr int LDVT = KEYS + 4;
     __shared__ __attribute__((aligned(16))) unsigned short Ks[KEYS * LDK];
     __shared__ __attribute__((aligned(16))) unsigned short Vt[HD * LDVT];
 
@@ -36,21 +40,32 @@ __global__ __launch_bounds__(256, 2) void attention_h16_kernel(const AttnH16Para
     const unsigned short *kb = p.k + b * p.ks[0] + h * p.ks[1];
     const unsigned short *vb = p.v + b * p.vs[0] + h * p.vs[1];
 
-    // k rows as they are, v transposed; rows / columns past the last key as zeros.  All loads first.
-    constexpr int PARTS = HD / 8, NV = (KEYS * PARTS + 255) / 256;
-    uint4 kq[NV], vq[NV];
+    // k rows as they are, v transposed; rows / columns past the last key as zeros.  All loads first.  Of v a lane takes 8
+    // channels of two neighbouring keys, 4 channel groups of 16 key pairs a wavefront, and stores each channel's pair as one
+    // dword: no two lanes on one bank.  (One key a lane, 8 keys of 8 channel groups a wavefront, was 8 stores of 2 bytes per
+    // 16 bytes with 8 lanes on one bank each.)
+    constexpr int PARTS = HD / 8, NK = (KEYS * PARTS + NT - 1) / NT, NV = (2 * NKT + NW - 1) / NW;
+    uint4 kq[NK], vq[NV][2];
+#pragma unroll
+    for (int i = 0; i < NK; ++i) {
+        const int f = tid + i * NT;
+        const int key = f / PARTS, part = f % PARTS;
+        kq[i] = make_uint4(0u, 0u, 0u, 0u);
+        if (key < T) kq[i] = *reinterpret_cast<const uint4 *>(kb + key * p.ks[2] + part * 8);
+    }
+    const int vpart = lane / 16, vpair = lane % 16;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-        const int f = tid + i * 256;
-        const int key = f / PARTS, part = f % PARTS;
-        kq[i] = vq[i] = make_uint4(0u, 0u, 0u, 0u);
-        if (key < T) {
-            kq[i] = *reinterpret_cast<const uint4 *>(kb + key * p.ks[2] + part * 8);
-            vq[i] = *reinterpret_cast<const uint4 *>(vb + key * p.vs[2] + part * 8);
+        const int u = wave + i * NW;   // half of the channels of 32 keys
+#pragma unroll
+        for (int z = 0; z < 2; ++z) {
+            const int key = u / 2 * 32 + 2 * vpair + z;
+            vq[i][z] = make_uint4(0u, 0u, 0u, 0u);
+            if (u < 2 * NKT && key < T) vq[i][z] = *reinterpret_cast<const uint4 *>(vb + key * p.vs[2] + (u % 2 * 4 + vpart) * 8);
         }
     }
     // this lane's query row: the channels 16 s + 8 (lane / 32) .. + 7 of MFMA step s
-    const int q0 = (blockIdx.x * 4 + wave) * 32;
+    const int q0 = (blockIdx.x * NW + wave) * 32;
     const int query = q0 + li;
     uint4 qf[HD / 16];
     {
@@ -60,14 +75,19 @@ __global__ __launch_bounds__(256, 2) void attention_h16_kernel(const AttnH16Para
             qf[s] = query < T ? *reinterpret_cast<const uint4 *>(qb + 16 * s + 8 * lh) : make_uint4(0u, 0u, 0u, 0u);
     }
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        const int f = tid + i * 256;
-        const int key = f / PARTS, part = f % PARTS;
-        if (f < KEYS * PARTS) {
-            *reinterpret_cast<uint4 *>(Ks + key * LDK + part * 8) = kq[i];
-            const unsigned w[4] = {vq[i].x, vq[i].y, vq[i].z, vq[i].w};
+    for (int i = 0; i < NK; ++i) {
+        const int f = tid + i * NT;
+        if (f < KEYS * PARTS) *reinterpret_cast<uint4 *>(Ks + f / PARTS * LDK + f % PARTS * 8) = kq[i];
+    }
 #pragma unroll
-            for (int e = 0; e < 8; ++e) Vt[(part * 8 + e) * LDVT + key] = (unsigned short) (w[e / 2] >> (16 * (e & 1)));
+    for (int i = 0; i < NV; ++i) {
+        const int u = wave + i * NW;
+        if (u < 2 * NKT) {   // uniform
+            const unsigned lo[4] = {vq[i][0].x, vq[i][0].y, vq[i][0].z, vq[i][0].w}, hi[4] = {vq[i][1].x, vq[i][1].y, vq[i][1].z, vq[i][1].w};
+            unsigned *dst = reinterpret_cast<unsigned *>(Vt + (u % 2 * 4 + vpart) * 8 * LDVT) + u / 2 * 16 + vpair;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)   // the low or the high halves of the two keys' words
+                dst[e * (LDVT / 2)] = __builtin_amdgcn_perm(hi[e / 2], lo[e / 2], e % 2 ? 0x07060302u : 0x05040100u);
         }
     }
     __syncthreads();
@@ -98,14 +118,20 @@ __global__ __launch_bounds__(256, 2) void attention_h16_kernel(const AttnH16Para
     // Softmax over the keys in fp32 (softmax.c:26-59); keys past the last count as minus infinity
     float mx = -INFINITY;
 #pragma unroll
-    for (int t = 0; t < NKT; ++t)
+    for (int t = 0; t < NKT; ++t) {
+        if (32 * t + 32 <= T) {   // uniform: every key of the tile exists
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int key = 32 * t + 8 * (r / 4) + 4 * lh + (r % 4);
-            const float val = key < T ? __fmul_rn(s[t][r], p.scale) : -INFINITY;
-            s[t][r] = val;
-            mx = fmaxf(mx, val);
+            for (int r = 0; r < 16; ++r) s[t][r] = __fmul_rn(s[t][r], p.scale);
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int key = 32 * t + 8 * (r / 4) + 4 * lh + (r % 4);
+                s[t][r] = key < T ? __fmul_rn(s[t][r], p.scale) : -INFINITY;
+            }
         }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[t][r]);
+    }
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     float sum = 0.0f;
 #pragma unroll
@@ -157,12 +183,19 @@ __global__ __launch_bounds__(256, 2) void attention_h16_kernel(const AttnH16Para
 
 template <int DT>
 static int attention_h16_launch_dt(const AttnH16Params &p, int batch, hipStream_t stream) {
-    const dim3 grid((unsigned) ((p.tokens + 127) / 128), (unsigned) (batch * p.heads));
     const int nkt = (p.tokens + 31) / 32;
-    if (nkt <= 2) hipLaunchKernelGGL((attention_h16_kernel<DT, 2>), grid, dim3(256), 0, stream, p);
-    else if (nkt <= 4) hipLaunchKernelGGL((attention_h16_kernel<DT, 4>), grid, dim3(256), 0, stream, p);
-    else if (nkt <= 7) hipLaunchKernelGGL((attention_h16_kernel<DT, 7>), grid, dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL((attention_h16_kernel<DT, 8>), grid, dim3(256), 0, stream, p);
+    const unsigned heads = (unsigned) (batch * p.heads);
+    // Eight wavefronts share a copy of k and v where four would make a second copy for the same head, and the heads alone give
+    // half of the CUs a workgroup (fewer heads: two workgroups on two CUs do the staging side by side).  64 x 3 heads of 197
+    // tokens 16.9 us a launch with two copies and v stored by halves of a word, 11.4 now.
+    const bool wide = nkt > 4 && heads >= 128;
+    const dim3 grid(wide ? 1u : (unsigned) ((p.tokens + 127) / 128), heads);
+    if (nkt <= 2) hipLaunchKernelGGL((attention_h16_kernel<DT, 2, 4>), grid, dim3(256), 0, stream, p);
+    else if (nkt <= 4) hipLaunchKernelGGL((attention_h16_kernel<DT, 4, 4>), grid, dim3(256), 0, stream, p);
+    else if (nkt <= 7 && wide) hipLaunchKernelGGL((attention_h16_kernel<DT, 7, 8>), grid, dim3(512), 0, stream, p);
+    else if (nkt <= 7) hipLaunchKernelGGL((attention_h16_kernel<DT, 7, 4>), grid, dim3(256), 0, stream, p);
+    else if (wide) hipLaunchKernelGGL((attention_h16_kernel<DT, 8, 8>), grid, dim3(512), 0, stream, p);
+    else hipLaunchKernelGGL((attention_h16_kernel<DT, 8, 4>), grid, dim3(256), 0, stream, p);
     ONHIP_CHECK_HIP(hipGetLastError());
     return ONHIP_OK;
 }
