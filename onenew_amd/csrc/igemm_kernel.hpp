@@ -322,9 +322,12 @@ __device__ __forceinline__ int requant_s8(float y, float inv_scale) {
 // over, so that the store does not begin with a trip to memory: sbias the per-row bias (-0.0f for a launch without
 // one); for int8 operands the de-quantisation factors weight_aux / 127, divided once per row and not by every lane,
 // and srow2 the int32 biases as floats.
+// twin_at (int8 with a residual operand): LDS for the tile's int8 form, [column of the tile][twin_ld bytes], at this wavefront's
+// first column and row; store_twin writes it out.
 template <int DT, int EPI, int TM, int TN, bool RES, bool BIAS_LDS = false, class ACC>
 __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][TN], int batch, int m_wave, int n_wave,
-                                           int li, int lh, const float *sbias = nullptr, const float *srow2 = nullptr) {
+                                           int li, int lh, const float *sbias = nullptr, const float *srow2 = nullptr,
+                                           unsigned char *twin_at = nullptr, int twin_ld = 0) {
     const int esz = (DT == DT_I8 && p.out_s8) ? 1 : 4;
     const rsrc_t rc = make_rsrc(reinterpret_cast<const char *>(p.C) + (size_t) batch * p.c_batch_stride * esz,
                                 RSRC_RANGE);
@@ -386,7 +389,6 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
         // RES: the residual operand of a folded Add (fp32 results): a row tile's addends are requested together
         const rsrc_t rres = make_rsrc(RES ? reinterpret_cast<const char *>(p.res) + (size_t) batch * p.c_batch_stride * 4 : nullptr,
                                       RES ? RSRC_RANGE : 0u);
-        const rsrc_t rtwin = make_rsrc(RES ? p.twin : nullptr, RES && p.twin ? RSRC_RANGE : 0u);
         unsigned tq[TN][4];
 #pragma unroll
         for (int b = 0; b < TN; ++b)
@@ -431,12 +433,10 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
                             tq[b][r % 4] = (unsigned) round_half_away_small(
                                 __builtin_amdgcn_fmed3f(__fmul_rn(y, p.twin_inv_scale), -128.0f, 127.0f));
                             if (r % 4 == 3) {
-                                const int n = n_wave + b * 32 + li, m4 = m_wave + a * 32 + 8 * (r / 4) + 4 * lh;
-                                const bool ok = n < p.N && m4 < p.M;
                                 const unsigned p01 = __builtin_amdgcn_perm(tq[b][1], tq[b][0], 0x0c0c0400u);
                                 const unsigned p23 = __builtin_amdgcn_perm(tq[b][3], tq[b][2], 0x0c0c0400u);
-                                __builtin_amdgcn_raw_buffer_store_b32(__builtin_amdgcn_perm(p23, p01, 0x05040100u), rtwin,
-                                                                      ok ? (unsigned) (n * p.twin_pitch + m4) : OOB, 0, 0);
+                                *reinterpret_cast<unsigned *>(twin_at + (b * 32 + li) * twin_ld + a * 32 + 8 * (r / 4) + 4 * lh) =
+                                    __builtin_amdgcn_perm(p23, p01, 0x05040100u);
                             }
                         }
                     }
@@ -507,6 +507,24 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
         };
         if (m_edge) store_rows(std::true_type{});
         else store_rows(std::false_type{});
+    }
+}
+
+// The int8 form of a finished tile (p.twin) from LDS, 16 channels of a pixel per thread: a 64 x 64 tile is one store per
+// thread to 64 contiguous bytes per pixel.  (Four channels per lane straight from the registers were 64 separate cache lines
+// an instruction, 64 cycles of the CU's address path each, more than the tile's fp32 result and residual together: ResNet-50
+// W8A32 batch 32, the 1x1 layers with an Add, 507 us of a pass before.)
+template <int BM, int BN>
+__device__ __forceinline__ void store_twin(const IgemmParams &p, const unsigned char *stage, int m0, int n0, int tid) {
+    constexpr int GROUPS = BM / 16;
+    const rsrc_t rt = make_rsrc(p.twin, RSRC_RANGE);
+#pragma unroll
+    for (int f0 = 0; f0 < BN * GROUPS; f0 += THREADS) {
+        const int f = f0 + tid, nl = f / GROUPS, g = f % GROUPS;
+        const uint4 v = *reinterpret_cast<const uint4 *>(stage + nl * (BM + 16) + g * 16);
+        const int n = n0 + nl, m = m0 + g * 16;
+        const bool ok = n < p.N && m < p.M;   // M is a multiple of 16
+        __builtin_amdgcn_raw_buffer_store_b128(u32x4{v.x, v.y, v.z, v.w}, rt, ok ? (unsigned) (n * p.twin_pitch + m) : OOB, 0, 0);
     }
 }
 
@@ -1409,15 +1427,25 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(PW2 ? 4
             return;
         }
     }
+    unsigned char *twin_at = nullptr;
+    if constexpr (DT == DT_I8 && RES) {
+        static_assert(BN * (BM / 16) % THREADS == 0 && sizeof(lds) >= (size_t) BN * (BM + 16), "the int8 form of the tile fits the operand buffers");
+        twin_at = reinterpret_cast<unsigned char *>(&lds[0][0]) + wn * (BN / WN) * (BM + 16) + wm * (BM / WM);
+        if (p.twin) __syncthreads();   // every wavefront is done with the operand buffers
+    }
     switch (p.ep.act) {
         case NOT_ACT:
-        case RELU6: write_tile<DT, EPI_NONE, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM)); break;
-        case RELU: write_tile<DT, EPI_RELU, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM)); break;
-        case CLIP: write_tile<DT, EPI_CLIP, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM)); break;
+        case RELU6: write_tile<DT, EPI_NONE, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM), twin_at, BM + 16); break;
+        case RELU: write_tile<DT, EPI_RELU, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM), twin_at, BM + 16); break;
+        case CLIP: write_tile<DT, EPI_CLIP, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM), twin_at, BM + 16); break;
         case SILU:
-        case ONHIP_ACT_GELU_LUT: write_tile<DT, EPI_LUT, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM)); break;
-        default: write_tile<DT, EPI_GENERIC, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM)); break;
-    }
+        case ONHIP_ACT_GELU_LUT: write_tile<DT, EPI_LUT, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM), twin_at, BM + 16); break;
+        default: write_tile<DT, EPI_GENERIC, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM), twin_at, BM + 16); break;
+    }    if constexpr (DT == DT_I8 && RES)
+        if (p.twin) {
+            __syncthreads();
+            store_twin<BM, BN>(p, reinterpret_cast<const unsigned char *>(&lds[0][0]), m0, n0, tid);
+        }
 }
 
 // sums the split-K partials in slice order and applies the epilogue: one thread per output element; a
