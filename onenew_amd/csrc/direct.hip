@@ -11,7 +11,8 @@ namespace onhip {
 // wavefront covers CBW neighbouring channel blocks of 64 / CBW consecutive pixels, so its stores are runs of
 // CBW * 16 contiguous bytes per pixel (whole pixels when cp <= 64) and each of its 16 loads reads runs of
 // 64 / CBW consecutive pixels of a channel plane.  Grid: (pixel blocks, channel block groups, images).
-template <int CBW>
+// FULL: c is a multiple of 16, so the 16 loads of a lane stand without a test (a test is a branch around each of them).
+template <int CBW, bool FULL>
 __global__ __launch_bounds__(256) void quantize_nhwc_kernel(const float *x, int c, int hw, int cp, float inv_scale,
                                                             int8_t *q) {
     constexpr int PIXW = 64 / CBW;
@@ -23,7 +24,7 @@ __global__ __launch_bounds__(256) void quantize_nhwc_kernel(const float *x, int 
     const float *src = x + (img * c + (long long) cb * 16) * hw + pix;
     float v[16];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) v[e] = cb * 16 + e < c ? src[(long long) e * hw] : 0.0f;
+    for (int e = 0; e < 16; ++e) v[e] = FULL || cb * 16 + e < c ? src[(long long) e * hw] : 0.0f;
     unsigned out[4];
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
@@ -41,9 +42,10 @@ int quantize_nhwc_launch(const float *x, int n, int c, int h, int w, int cp, flo
     if (n > 65535) return set_error(ONHIP_ERR_ARG, "quantize: batch of %d", n);
     const int cbw = cblocks >= 4 ? 4 : cblocks >= 2 ? 2 : 1;
     const dim3 grid((hw + 4 * (64 / cbw) - 1) / (4 * (64 / cbw)), (cblocks + cbw - 1) / cbw, n);
-    if (cbw == 4) hipLaunchKernelGGL(quantize_nhwc_kernel<4>, grid, dim3(256), 0, stream, x, c, hw, cp, inv_scale, q);
-    else if (cbw == 2) hipLaunchKernelGGL(quantize_nhwc_kernel<2>, grid, dim3(256), 0, stream, x, c, hw, cp, inv_scale, q);
-    else hipLaunchKernelGGL(quantize_nhwc_kernel<1>, grid, dim3(256), 0, stream, x, c, hw, cp, inv_scale, q);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, x, c, hw, cp, inv_scale, q); };
+    if (cbw == 4) c % 16 == 0 ? go(quantize_nhwc_kernel<4, true>) : go(quantize_nhwc_kernel<4, false>);
+    else if (cbw == 2) c % 16 == 0 ? go(quantize_nhwc_kernel<2, true>) : go(quantize_nhwc_kernel<2, false>);
+    else c % 16 == 0 ? go(quantize_nhwc_kernel<1, true>) : go(quantize_nhwc_kernel<1, false>);
     ONHIP_CHECK_HIP(hipGetLastError());
     return ONHIP_OK;
 }
