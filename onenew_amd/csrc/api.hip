@@ -1,6 +1,6 @@
 // Kernel-level C ABI (include/onenew_hip.h): argument checks, geometry set-up and kernel choice.
 // Device pointers in, asynchronous launches on the caller's stream, no allocation except the
-// lazily grown split-K scratch.
+// lazily grown split-K scratch and the slots for weights split on the call.
 #include <stdarg.h>
 #include <stdio.h>
 #include <string.h>
@@ -334,8 +334,8 @@ static bool tail_geometry(const IgemmLaunch &cfg, const IgemmProblem &p, int bm,
 
 static const int kRowbTiles[][2] = {{64, 128}, {128, 128}, {64, 256}, {96, 128}, {32, 256}, {32, 512}};
 static const int kNumRowbTiles = 6;
-static const int kF3Tiles[][2] = {{256, 128}, {256, 64}, {128, 128}, {128, 64}, {64, 64}};
-static const int kNumF3Tiles = 5;
+static const int kF3Tiles[][2] = {{256, 128}, {256, 64}, {192, 64}, {128, 128}, {128, 64}, {64, 64}};
+static const int kNumF3Tiles = 6;
 
 // (bm, bn) is a tile this build has a kernel for
 static bool tile_exists(const Choice &c) {
@@ -457,9 +457,14 @@ static bool dma_model_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choi
 // 1100 timed launches over the layers of ResNet-50 (batch 1, 8, 32) and MobileNetV2 (batch 8, 64), median error 10 %, the
 // choices within 2 % of the fastest: a compute unit works through its workgroups at a rate that depends on the tile alone
 // (larger tiles stage less per multiply-add), whether one or several are resident.
+// 192 x 64 is for row counts that 128 does not divide (192, 576, 960 of transformers and expansions, 2053): 192 x 12544 x 768
+// 30.4 us, 128 x 128 32.5 and 64 x 64 34.1.
 static bool f3_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out, double *us) {
-    static const double per_k_tile[kNumF3Tiles] = {0.82, 0.50, 0.50, 0.29, 0.215};   // per K tile of 16 and workgroup
-    static const double per_tile[kNumF3Tiles] = {3.8, 1.8, 1.25, 0.70, 0.37};        // first loads and store of a workgroup
+    // below 0.6 GFLOP (6 us of fp32 matrix instructions) the pass alone costs more than there is to gain: not worth the host's
+    // time either (0.7 us of a call that takes 8)
+    if (!p.a_split && 2.0 * p.M * p.N * p.K < 6e8) return false;
+    static const double per_k_tile[kNumF3Tiles] = {0.82, 0.50, 0.46, 0.50, 0.29, 0.215};   // per K tile of 16 and workgroup
+    static const double per_tile[kNumF3Tiles] = {3.8, 1.8, 1.7, 1.25, 0.70, 0.37};        // first loads and store of a workgroup
     *us = 1e300;
     for (int t = 0; t < kNumF3Tiles; ++t)
         for (int s = 0; s < kNumSplits; ++s) {
@@ -475,7 +480,13 @@ static bool f3_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out
             if (t_us < *us) { *us = t_us; *out = c; }
         }
     if (*us > 1e299) return false;
-    if (!p.a_split) *us += 2.5 + 10.0 / 3e6 * p.M * p.K;   // the pass that splits the weights: 4 bytes read, 6 written
+    // The pass that splits the weights is a launch of its own: 4 bytes read, 6 written.  Against convolutions, and products with
+    // fewer columns than a tile has rows, count the 10 % that both estimates are off by as well: 43 x 4536 x 383 and 42 x 8488 x
+    // 903, where the estimates are level, take 10.7 and 19.4 us with fp32 matrix instructions, 12.3 and 21.1 with the pass.
+    if (!p.a_split) {
+        const bool level = cfg.bl != BL_ROWS || p.M < 64;
+        *us = (level ? 1.1 : 1.0) * (*us + (level ? 3.5 : 2.5) + 10.0 / 3e6 * p.M * p.K);
+    }
     return true;
 }
 // the same for the fp32 matrix instructions' kernels (2250 cycles of model_cost take a microsecond; same launches, error 10 %)

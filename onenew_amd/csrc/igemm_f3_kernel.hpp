@@ -22,7 +22,7 @@
 // kernel uses; K in tiles of 4 units of 4 floats = one 16-deep MFMA step.  What differs:
 //   * A, the weights, is split ahead of time (split_weights_launch) into the order the matrix instructions read it, and goes
 //     from memory straight into operand registers, one contiguous KiB per load: no LDS, no vector instruction.  The
-//     wavefronts of a tile lie along M (the 64 x 64 and 128 x 128 tiles apart), so no two of them load the same rows;
+//     wavefronts of a tile lie along M (the 64 x 64, 192 x 64 and 128 x 128 tiles apart), so no two of them load the same rows;
 //   * B is split on its way into LDS, [part][k / 8][column][8 bf16], a unit per thread and K tile, in four phases of four to
 //     six vector instructions each behind an MFMA of its own: 22 vector instructions per 12 to 24 MFMAs and wavefront.
 // Per K tile of the 128 x 64 tile a wavefront issues 12 MFMAs, 3 A loads, 4 B loads, 3 LDS stores and 6 LDS reads.
@@ -435,6 +435,7 @@ int f3_launch_tile(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t st
     switch (cfg.bm * 1000 + cfg.bn) {
         case 256128: return f3_launch_one<BL, 256, 128, 8, 1, RES>(cfg, p, stream);
         case 256064: return f3_launch_one<BL, 256, 64, 4, 1, RES>(cfg, p, stream);
+        case 192064: return f3_launch_one<BL, 192, 64, 2, 2, RES>(cfg, p, stream);
         case 128128: return f3_launch_one<BL, 128, 128, 4, 2, RES>(cfg, p, stream);
         case 128064: return f3_launch_one<BL, 128, 64, 4, 1, RES>(cfg, p, stream);
         case 64064: return f3_launch_one<BL, 64, 64, 2, 2, RES>(cfg, p, stream);

@@ -209,7 +209,9 @@ __device__ __forceinline__ ColState make_col(const IgemmParams &p, int n) {
     c.pixoff = valid ? off : OOB;
     c.mask_lo = c.mask_hi = 0;
     if constexpr (BL != BL_PLAIN) {
-        if (p.use_tapmask) {
+        if (p.use_tapmask && p.khkw == 1) {
+            c.mask_lo = (unsigned) c.ih0 < (unsigned) p.H && (unsigned) c.iw0 < (unsigned) p.W ? 1u : 0u;
+        } else if (p.use_tapmask) {
             // The taps of a filter row that lie inside the image are a run of bits, the same for every filter row: one 64-bit
             // shift per row instead of a test of every tap (9 tests per column, and up to four columns per lane, stood before
             // the first load of every launch).

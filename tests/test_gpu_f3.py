@@ -40,7 +40,7 @@ def conv_ref(torch, d, x, w, b):
     return conv(x, w, b), conv(x.abs(), w.abs(), b.abs())
 
 
-TILES = [(256, 128), (256, 64), (128, 128), (128, 64), (64, 64)]
+TILES = [(256, 128), (256, 64), (192, 64), (128, 128), (128, 64), (64, 64)]
 # loader, (n, cin, h, w, cout, filter, stride, pad): rows and columns off every tile, reductions off a K tile of 16 and off a unit of 4
 SHAPES = [("plain", (2, 109, 9, 23, 67, 1, 1, 0)), ("plain", (1, 130, 16, 17, 259, 1, 1, 0)), ("tapc", (2, 13, 11, 9, 97, 3, 1, 1)),
           ("tapc", (1, 33, 15, 12, 260, 3, 2, 1)), ("gather", (1, 13, 13, 21, 65, 3, 1, 1)), ("tapc", (1, 20, 12, 13, 70, 7, 1, 3)), ("gather", (1, 6, 9, 14, 66, (5, 11), 2, 2)), ("gather", (2, 117, 14, 9, 40, 1, 2, 0))]
