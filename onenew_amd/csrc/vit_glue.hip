@@ -98,6 +98,8 @@ __global__ __launch_bounds__(256) void layernorm_rows_kernel(const float *__rest
 // The same for rows of a multiple of four floats, 16-byte aligned: a thread's share of the workgroup's rows (up to
 // LN_VEC 16-byte pieces) is requested in one go and held in registers, so the staging costs one memory round trip instead of
 // one per loop iteration; sums in memory order by one thread per row as above; the normalised rows leave as 16-byte stores.
+// Weight and bias are requested with the rows, and rows and columns of the pieces follow from the first one's without a
+// division each (sixteen per thread were as long as the sums): 12544 rows of 192 8.5 -> 7.5 us.
 constexpr int LN_VEC = 8;
 
 __global__ __launch_bounds__(256) void layernorm_rows4_kernel(const float *__restrict__ x, const float *__restrict__ w,
@@ -110,17 +112,22 @@ __global__ __launch_bounds__(256) void layernorm_rows4_kernel(const float *__res
     const int pitch = reduce + 1, groups = reduce / 4;
     const int total = nr * groups;
     const float4 *src = reinterpret_cast<const float4 *>(x + (long long) row0 * reduce);
-    float4 v[LN_VEC];
-    int at[LN_VEC], col[LN_VEC];
+    float4 v[LN_VEC], wv[LN_VEC], bv[LN_VEC];
+    int at[LN_VEC], row[LN_VEC];
+    const int dr = 256 / groups, dc = 256 - dr * groups;   // 256 pieces further on: dr rows, dc pieces
+    int r = (int) threadIdx.x / groups, c = (int) threadIdx.x - r * groups;
 #pragma unroll
     for (int i = 0; i < LN_VEC; ++i) {
         const int f = threadIdx.x + i * 256;
         const bool live = f < total;
-        const int ff = live ? f : 0;
-        const int r = ff / groups;
-        col[i] = (ff - r * groups) * 4;
-        at[i] = live ? r * pitch + col[i] : -1;
-        v[i] = live ? src[ff] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        row[i] = live ? r : 0;
+        at[i] = live ? r * pitch + 4 * c : -1;
+        v[i] = live ? src[f] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        wv[i] = *reinterpret_cast<const float4 *>(w + 4 * c);
+        bv[i] = *reinterpret_cast<const float4 *>(b + 4 * c);
+        r += dr;
+        c += dc;
+        if (c >= groups) { c -= groups; ++r; }
     }
 #pragma unroll
     for (int i = 0; i < LN_VEC; ++i)
@@ -139,17 +146,10 @@ __global__ __launch_bounds__(256) void layernorm_rows4_kernel(const float *__res
     }
     __syncthreads();
     float4 *dst = reinterpret_cast<float4 *>(y + (long long) row0 * reduce);
-    float4 wv[LN_VEC], bv[LN_VEC];
-#pragma unroll
-    for (int i = 0; i < LN_VEC; ++i) {
-        wv[i] = *reinterpret_cast<const float4 *>(w + col[i]);
-        bv[i] = *reinterpret_cast<const float4 *>(b + col[i]);
-    }
 #pragma unroll
     for (int i = 0; i < LN_VEC; ++i) {
         if (at[i] < 0) continue;
-        const int r = at[i] / pitch;
-        const float m = s_mean[r], s = s_inv[r];
+        const float m = s_mean[row[i]], s = s_inv[row[i]];
         float4 o;
         o.x = __fadd_rn(__fmul_rn(__fmul_rn(__fsub_rn(v[i].x, m), s), wv[i].x), bv[i].x);
         o.y = __fadd_rn(__fmul_rn(__fmul_rn(__fsub_rn(v[i].y, m), s), wv[i].y), bv[i].y);
