@@ -151,8 +151,8 @@ int onhip_conv2d_f32_packed(const onhip_conv_desc_t *d, const float *x, const fl
 /* onhip_conv2d_f32 (packed == 0) or onhip_conv2d_f32_packed (packed != 0) for callers that cannot allocate device
  * memory: code under HIP graph capture, serving loops, harnesses that forbid it.  No counterpart in the reference.
  * It calls no allocating routine: the partial sums of a split-K launch go to a 32 MiB array built into the library's
- * code object (one copy per GPU, held until the process ends), tile and split come from the cost model only, and the
- * slices are added up by a finishing launch.  A problem whose chosen split needs more than 32 MiB of partial sums
+ * code object (one copy per GPU, held until the process ends), as do weights that the launch wants split into bf16
+ * parts, tile and split come from the cost model only, and the slices are added up by a finishing launch.  A problem whose chosen split needs more than 32 MiB of partial sums
  * (split x output bytes) is refused with ONHIP_ERR_WORKSPACE.  The array keeps the last call's contents; every
  * element read is written first by the same call, so nothing needs clearing.  All calls on one GPU share the array:
  * calls that may overlap there (different streams without an ordering between them) race.  Same results as the entry

@@ -134,16 +134,28 @@ static int get_scratch(size_t bytes, void **out) {
 }
 
 // Split weights of a call whose caller has none (launch_choice).  A stream keeps the slot that its first such call took and
-// allocated, since launches on two streams may overlap; the per-thread default stream is one for each thread.  Slots are kept
-// until the process ends, as recorded graphs hold their addresses, eight at most.  A stream that finds all slots taken or that
-// is being captured before it has one, and weights whose split form is larger than a slot, run the other fp32 kernels.  The
+// allocated, since launches on two streams may overlap; the per-thread default stream is one for each thread.  A recorded graph
+// may be replayed on any stream, also while the one it was recorded on goes on using its slot: each capture has slots of its
+// own.  Slots are kept until the process ends, as graphs hold their addresses, eight for streams and 32 for captures at most.
+// A call that finds all of them taken, and weights whose split form is larger than a slot, run the other fp32 kernels.  The
 // pass that splits and the launch that reads follow each other on the stream while g_split_mu is held: another thread's calls
 // on the same stream go before both or behind both.  The entry point that allocates nothing takes part of its own array.
 static const long long kSplitWsBytes = 16LL << 20;
-static const size_t kSplitSlots = 8;
+static const int kSplitSlots = 8, kSplitCaptureSlots = 32;
 static std::mutex g_split_mu;
-struct SplitSlot { int dev; hipStream_t stream; std::thread::id thread; void *mem; };
+struct SplitSlot { int dev; hipStream_t stream; std::thread::id thread; bool captured; unsigned long long capture; void *mem; };
 static std::vector<SplitSlot> g_split_slots;
+// st is being captured (or may be: *known false); *id = which capture, 0 for none
+static bool under_capture(hipStream_t st, unsigned long long *id = nullptr, bool *known = nullptr) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    unsigned long long which = 0;
+    const bool ok = hipStreamGetCaptureInfo(st, &cap, &which) == hipSuccess;
+    if (!ok) (void) hipGetLastError();   // the legacy stream while another one is captured
+    const bool on = !ok || cap != hipStreamCaptureStatusNone;
+    if (id) *id = on ? which : 0;
+    if (known) *known = ok && (cap == hipStreamCaptureStatusNone || cap == hipStreamCaptureStatusActive);
+    return on;
+}
 // *out = the slot of stream st on the current device, nullptr if there is none; g_split_mu held
 static int split_slot(hipStream_t st, long long bytes, void **out) {
     if (tl_noalloc) {   // the last part of its array: f3_choice leaves the partial sums the rest
@@ -154,17 +166,27 @@ static int split_slot(hipStream_t st, long long bytes, void **out) {
     ONHIP_CHECK_HIP(hipGetDevice(&dev));
     const std::thread::id me = st == hipStreamPerThread ? std::this_thread::get_id() : std::thread::id();
     *out = nullptr;
-    for (const SplitSlot &s : g_split_slots)
-        if (s.dev == dev && s.stream == st && s.thread == me) *out = s.mem;
-    if (*out || g_split_slots.size() == kSplitSlots) return ONHIP_OK;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return ONHIP_OK;
-    if (hipMalloc(out, kSplitWsBytes) != hipSuccess) {
+    unsigned long long capture;
+    bool known;
+    const bool captured = under_capture(st, &capture, &known);
+    if (!known) return ONHIP_OK;
+    int taken = 0;
+    for (const SplitSlot &s : g_split_slots) {
+        taken += s.captured == captured;
+        if (s.dev == dev && s.stream == st && s.thread == me && s.captured == captured && s.capture == capture) *out = s.mem;
+    }
+    if (*out || taken == (captured ? kSplitCaptureSlots : kSplitSlots)) return ONHIP_OK;
+    // an allocation of its own, not part of what is captured (here or by another thread)
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    ONHIP_CHECK_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+    const hipError_t e = hipMalloc(out, kSplitWsBytes);
+    ONHIP_CHECK_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+    if (e != hipSuccess) {
         (void) hipGetLastError();   // no memory for it: as without a slot
         *out = nullptr;
         return ONHIP_OK;
     }
-    g_split_slots.push_back({dev, st, me, *out});
+    g_split_slots.push_back({dev, st, me, captured, capture, *out});
     return ONHIP_OK;
 }
 
@@ -571,6 +593,14 @@ static thread_local int tl_last_choice[7] = {0, 0, 0, 0, 0, 0, 0};
 // this stream has no slot for the split weights, nothing was launched
 static const int kNoSplitSlot = 1;
 
+// What a problem without a slot runs instead.  Under capture nothing is cut along K: the calls before the capture ran with
+// their weights split, so none of them need have allocated the partial sums' scratch, and a capture may not.
+static Choice slotless_choice(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t st) {
+    Choice c = model_choice(cfg, p);
+    if (under_capture(st)) { c.split = 1; c.tail = c.fin = 0; }
+    return c;
+}
+
 // Runs the problem the way the choice says.
 static int launch_choice(IgemmLaunch cfg, IgemmProblem p, const Choice &c, hipStream_t st) {
     std::unique_lock<std::mutex> split_lock(g_split_mu, std::defer_lock);
@@ -583,7 +613,7 @@ static int launch_choice(IgemmLaunch cfg, IgemmProblem p, const Choice &c, hipSt
             if (!p.A) return kNoSplitSlot;   // only this kernel reads the problem in this form
             split_lock.unlock();
             p.w_src = nullptr;               // as a call whose weights are too large to be split
-            return launch_choice(cfg, p, model_choice(cfg, p), st);
+            return launch_choice(cfg, p, slotless_choice(cfg, p, st), st);
         }
         rc = split_weights_launch(p.w_src, p.M, p.K, p.w_row, p.w_k, ws, st);
         if (rc) return rc;
@@ -1522,6 +1552,7 @@ static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float
             rp.a_split = split;
             const int rc = launch_choice(rcfg, rp, c, st);
             if (rc != kNoSplitSlot) return rc;
+            if (under_capture(st)) return launch_choice(cfg, p, slotless_choice(cfg, p, st), st);
         }
     }
     return plan_and_launch(cfg, p, st);

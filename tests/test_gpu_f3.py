@@ -127,3 +127,64 @@ def test_streams_and_threads(torch_dev):
         t.join()
     torch.cuda.synchronize()
     verify()
+
+
+def test_capture(torch_dev, monkeypatch):
+    """Split weights under capture: graphs recorded on one stream and replayed on two at once each have a slot of their own.
+    33 captures are one more than there are slots for: the last ones run other kernels, cut nowhere, as nothing else may be
+    allocated there."""
+    torch = torch_dev
+    print("f3 capture", flush=True)
+    m, k, n = 8195, 773, 1030
+    d = conv_desc(3, 300, 20, 19, 259, 1, 1, 0)
+    g = torch.Generator(device="cuda").manual_seed(4)
+    rand = lambda *shape: torch.randn(shape, generator=g, device="cuda")  # noqa: E731
+    jobs = []
+    for _ in range(2):
+        a, b, x, w, bias = rand(m, k), rand(k, n), rand(d.n, d.cin, d.h, d.w), rand(d.cout, d.cin, 1, 1), rand(d.cout)
+        jobs.append((a, b, x, w, bias, torch.empty(m, n, device="cuda"), torch.empty(d.n, d.cout, d.h, d.w, device="cuda"),
+                     ((a.double() @ b.double()).cpu(), (a.double().abs() @ b.double().abs()).cpu()), conv_ref(torch, d, x, w, bias)))
+    choices = []
+
+    def work(job):
+        a, b, x, w, bias, y, z = job[:7]
+        choices.clear()
+        hip.matmul(a, b, out=y)
+        choices.append(hip.last_launch_choice())
+        monkeypatch.setenv("ONHIP_TILE", "128x64x1x0x2")
+        hip.conv2d_f32(d, x, w, bias, out=z)
+        monkeypatch.delenv("ONHIP_TILE")
+        choices.append(hip.last_launch_choice())
+
+    stream, others = torch.cuda.Stream(), [torch.cuda.Stream() for _ in jobs]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        work(jobs[0])
+    torch.cuda.synchronize()
+
+    def record(job):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            work(job)
+        return graph
+
+    def replay(graphs):
+        for _ in range(3):
+            for job in jobs:
+                job[5].zero_()
+                job[6].zero_()
+            torch.cuda.synchronize()
+            for graph, s in zip(graphs, others):
+                with torch.cuda.stream(s):
+                    graph.replay()
+            with torch.cuda.stream(stream):   # the recording stream goes on with weights of its own
+                hip.matmul(jobs[0][0], jobs[1][1])
+            torch.cuda.synchronize()
+            for job in jobs:
+                check(job[5], *job[7], k)
+                check(job[6], *job[8], d.cin)
+
+    replay([record(job) for job in jobs])
+    graphs = [record(jobs[i % 2]) for i in range(33)]
+    assert all(c[4] != 2 and c[2] == 1 and c[3] == 0 for c in choices), choices
+    replay(graphs[-2:])
