@@ -1023,61 +1023,61 @@ __device__ __forceinline__ TilePlace place_tile(const IgemmParams &p) {
 template <int TM, int TN>
 __device__ __forceinline__ bool reduce_in_launch(const IgemmParams &p, f32x16 (&acc)[TM][TN], int slice, int batch, int lid, int m_wave,
                                                  int n_wave, int li, int lh, int tid) {
-            write_partial<TM, TN, true>(p, acc, slice * gridDim.z + batch, m_wave, n_wave, li, lh);
-            // The reduction inside the launch.  Partial sums and counters live in uncached memory and are stored and
-            // loaded with system scope (AUX_SYSTEM_SCOPE): once this workgroup's stores are acknowledged (written
-            // through, vmcnt(0)) it counts itself in with a device-scope atomic, and the last of a tile's slices to arrive
-            // adds all of them up in slice order (the order of the finishing kernel: the same bits) with loads that
-            // bypass the caches, and goes on to the epilogue as if it had computed the whole tile.  Nobody waits for
-            // anybody, so the launch cannot hang; the counter is back at zero for the next launch.
-            __shared__ int s_last;
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __syncthreads();
-            if (tid == 0) {
-                int *ctr = p.arrive + lid + batch * (int) gridDim.x;
-                const int old = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const int last = old == p.n_slices - 1;
-                if (last) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                s_last = last;
-            }
-            __syncthreads();
-            if (!s_last) return false;
-                        const int width = p.N - p.part_begin;
-                const bool m_edge = m_wave + TM * 32 > p.M;
+    write_partial<TM, TN, true>(p, acc, slice * gridDim.z + batch, m_wave, n_wave, li, lh);
+    // The reduction inside the launch.  Partial sums and counters live in uncached memory and are stored and
+    // loaded with system scope (AUX_SYSTEM_SCOPE): once this workgroup's stores are acknowledged (written
+    // through, vmcnt(0)) it counts itself in with a device-scope atomic, and the last of a tile's slices to arrive
+    // adds all of them up in slice order (the order of the finishing kernel: the same bits) with loads that
+    // bypass the caches, and goes on to the epilogue as if it had computed the whole tile.  Nobody waits for
+    // anybody, so the launch cannot hang; the counter is back at zero for the next launch.
+    __shared__ int s_last;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+        int *ctr = p.arrive + lid + batch * (int) gridDim.x;
+        const int old = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int last = old == p.n_slices - 1;
+        if (last) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = last;
+    }
+    __syncthreads();
+    if (!s_last) return false;
+    const int width = p.N - p.part_begin;
+    const bool m_edge = m_wave + TM * 32 > p.M;
 #pragma unroll
-                for (int a = 0; a < TM; ++a)
+    for (int a = 0; a < TM; ++a)
 #pragma unroll
-                    for (int b = 0; b < TN; ++b)
+        for (int b = 0; b < TN; ++b)
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) acc[a][b][r] = 0;
-                for (int s = 0; s < p.n_slices; ++s) {
-                    const rsrc_t rp = make_rsrc(reinterpret_cast<const char *>(p.partial) +
-                                                (size_t) (s * gridDim.z + batch) * p.M * width * 4, RSRC_RANGE);
-                    // half a 32x32 block at a time: eight loads in flight, not sixteen per block of the tile, which would
-                    // cost the kernels registers and with them occupancy
+            for (int r = 0; r < 16; ++r) acc[a][b][r] = 0;
+    for (int s = 0; s < p.n_slices; ++s) {
+        const rsrc_t rp = make_rsrc(reinterpret_cast<const char *>(p.partial) +
+                                    (size_t) (s * gridDim.z + batch) * p.M * width * 4, RSRC_RANGE);
+        // half a 32x32 block at a time: eight loads in flight, not sixteen per block of the tile, which would
+        // cost the kernels registers and with them occupancy
 #pragma unroll
-                    for (int a = 0; a < TM; ++a)
+        for (int a = 0; a < TM; ++a)
 #pragma unroll
-                        for (int b = 0; b < TN; ++b) {
-                            const int n = n_wave + b * 32 + li;
-                            const unsigned cv = n < p.N ? (unsigned) (n - p.part_begin + 4 * lh * width) * 4u : OOB;
+            for (int b = 0; b < TN; ++b) {
+                const int n = n_wave + b * 32 + li;
+                const unsigned cv = n < p.N ? (unsigned) (n - p.part_begin + 4 * lh * width) * 4u : OOB;
 #pragma unroll
-                            for (int h = 0; h < 2; ++h) {
-                                float v[8];
+                for (int h = 0; h < 2; ++h) {
+                    float v[8];
 #pragma unroll
-                                for (int q = 0; q < 8; ++q) {
-                                    const int r = 8 * h + q;
-                                    const int m_uni = m_wave + a * 32 + 8 * (r / 4) + (r % 4);
-                                    const bool row_ok = !m_edge || m_uni + 4 * lh < p.M;
-                                    v[q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                                        rp, row_ok ? cv : OOB, (unsigned) m_uni * (unsigned) width * 4u, AUX_SYSTEM_SCOPE));
-                                }
+                    for (int q = 0; q < 8; ++q) {
+                        const int r = 8 * h + q;
+                        const int m_uni = m_wave + a * 32 + 8 * (r / 4) + (r % 4);
+                        const bool row_ok = !m_edge || m_uni + 4 * lh < p.M;
+                        v[q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                            rp, row_ok ? cv : OOB, (unsigned) m_uni * (unsigned) width * 4u, AUX_SYSTEM_SCOPE));
+                    }
 #pragma unroll
-                                for (int q = 0; q < 8; ++q) acc[a][b][8 * h + q] = __fadd_rn(acc[a][b][8 * h + q], v[q]);
-                                __builtin_amdgcn_sched_barrier(0);
-                            }
-                        }
+                    for (int q = 0; q < 8; ++q) acc[a][b][8 * h + q] = __fadd_rn(acc[a][b][8 * h + q], v[q]);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
+            }
+    }
     return true;
 }
 
@@ -1443,7 +1443,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(PW2 ? 4
         case SILU:
         case ONHIP_ACT_GELU_LUT: write_tile<DT, EPI_LUT, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM), twin_at, BM + 16); break;
         default: write_tile<DT, EPI_GENERIC, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM), twin_at, BM + 16); break;
-    }    if constexpr (DT == DT_I8 && RES)
+    }
+    if constexpr (DT == DT_I8 && RES)
         if (p.twin) {
             __syncthreads();
             store_twin<BM, BN>(p, reinterpret_cast<const unsigned char *>(&lds[0][0]), m0, n0, tid);
