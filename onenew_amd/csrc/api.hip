@@ -146,15 +146,28 @@ static std::mutex g_split_mu;
 struct SplitSlot { int dev; hipStream_t stream; std::thread::id thread; bool captured; unsigned long long capture; void *mem; };
 static std::vector<SplitSlot> g_split_slots;
 // st is being captured (or may be: *known false); *id = which capture, 0 for none
-static bool under_capture(hipStream_t st, unsigned long long *id = nullptr, bool *known = nullptr) {
+static bool capture_info(hipStream_t st, unsigned long long *id, bool *known) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     unsigned long long which = 0;
     const bool ok = hipStreamGetCaptureInfo(st, &cap, &which) == hipSuccess;
     if (!ok) (void) hipGetLastError();   // the legacy stream while another one is captured
     const bool on = !ok || cap != hipStreamCaptureStatusNone;
-    if (id) *id = on ? which : 0;
-    if (known) *known = ok && (cap == hipStreamCaptureStatusNone || cap == hipStreamCaptureStatusActive);
+    *id = on ? which : 0;
+    *known = ok && (cap == hipStreamCaptureStatusNone || cap == hipStreamCaptureStatusActive);
     return on;
+}
+bool under_capture(hipStream_t st) {
+    unsigned long long id;
+    bool known;
+    return capture_info(st, &id, &known);
+}
+hipError_t malloc_outside_capture(void **out, size_t bytes) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) return e;
+    e = hipMalloc(out, bytes);
+    const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
+    return e != hipSuccess ? e : back;
 }
 // *out = the slot of stream st on the current device, nullptr if there is none; g_split_mu held
 static int split_slot(hipStream_t st, long long bytes, void **out) {
@@ -168,7 +181,7 @@ static int split_slot(hipStream_t st, long long bytes, void **out) {
     *out = nullptr;
     unsigned long long capture;
     bool known;
-    const bool captured = under_capture(st, &capture, &known);
+    const bool captured = capture_info(st, &capture, &known);
     if (!known) return ONHIP_OK;
     int taken = 0;
     for (const SplitSlot &s : g_split_slots) {
@@ -176,12 +189,7 @@ static int split_slot(hipStream_t st, long long bytes, void **out) {
         if (s.dev == dev && s.stream == st && s.thread == me && s.captured == captured && s.capture == capture) *out = s.mem;
     }
     if (*out || taken == (captured ? kSplitCaptureSlots : kSplitSlots)) return ONHIP_OK;
-    // an allocation of its own, not part of what is captured (here or by another thread)
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    ONHIP_CHECK_HIP(hipThreadExchangeStreamCaptureMode(&mode));
-    const hipError_t e = hipMalloc(out, kSplitWsBytes);
-    ONHIP_CHECK_HIP(hipThreadExchangeStreamCaptureMode(&mode));
-    if (e != hipSuccess) {
+    if (malloc_outside_capture(out, kSplitWsBytes) != hipSuccess) {
         (void) hipGetLastError();   // no memory for it: as without a slot
         *out = nullptr;
         return ONHIP_OK;
@@ -369,13 +377,13 @@ static bool tile_exists(const Choice &c) {
     return false;
 }
 
-// the fp32 kernel on the 16-bit matrix cores: a weight matrix for A, split already or small enough to be split on the call
+// the fp32 kernel on the 16-bit matrix cores: a weight matrix for A, kept split or small enough to be split on the call
 static bool f3_ok(const IgemmLaunch &cfg, const IgemmProblem &p) {
     static const bool off = getenv("ONHIP_NO_F3") != nullptr;   // tuning hook: fp32 matrix instructions only
-    if (off || cfg.dtype != DT_F32 || cfg.batch != 1 || (!p.a_split && !p.w_src)) return false;
+    if (off || cfg.dtype != DT_F32 || cfg.batch != 1 || !p.w_src) return false;
     if (cfg.bl != BL_PLAIN && cfg.bl != BL_ROWS && !((cfg.bl == BL_TAPC || cfg.bl == BL_GATHER) && p.use_tapmask)) return false;
     const long long bytes = split_weights_bytes(p.M, p.K);
-    return bytes < (1LL << 31) && (p.a_split || bytes <= kSplitWsBytes);
+    return bytes < (1LL << 31) && (p.keeper || bytes <= kSplitWsBytes);
 }
 
 static bool candidate_ok(const IgemmLaunch &cfg, const IgemmProblem &p, const Choice &c) {
@@ -484,7 +492,7 @@ static bool dma_model_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choi
 static bool f3_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out, double *us) {
     // below 0.6 GFLOP (6 us of fp32 matrix instructions) the pass alone costs more than there is to gain: not worth the host's
     // time either (0.7 us of a call that takes 8)
-    if (!p.a_split && 2.0 * p.M * p.N * p.K < 6e8) return false;
+    if (!p.keeper && 2.0 * p.M * p.N * p.K < 6e8) return false;
     static const double per_k_tile[kNumF3Tiles] = {0.82, 0.50, 0.46, 0.50, 0.29, 0.215};   // per K tile of 16 and workgroup
     static const double per_tile[kNumF3Tiles] = {3.8, 1.8, 1.7, 1.25, 0.70, 0.37};        // first loads and store of a workgroup
     *us = 1e300;
@@ -505,7 +513,7 @@ static bool f3_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out
     // The pass that splits the weights is a launch of its own: 4 bytes read, 6 written.  Against convolutions, and products with
     // fewer columns than a tile has rows, count the 10 % that both estimates are off by as well: 43 x 4536 x 383 and 42 x 8488 x
     // 903, where the estimates are level, take 10.7 and 19.4 us with fp32 matrix instructions, 12.3 and 21.1 with the pass.
-    if (!p.a_split) {
+    if (!p.keeper) {
         const bool level = cfg.bl != BL_ROWS || p.M < 64;
         *us = (level ? 1.1 : 1.0) * (*us + (level ? 3.5 : 2.5) + 10.0 / 3e6 * p.M * p.K);
     }
@@ -604,21 +612,31 @@ static Choice slotless_choice(const IgemmLaunch &cfg, const IgemmProblem &p, hip
 // Runs the problem the way the choice says.
 static int launch_choice(IgemmLaunch cfg, IgemmProblem p, const Choice &c, hipStream_t st) {
     std::unique_lock<std::mutex> split_lock(g_split_mu, std::defer_lock);
-    if (c.rowb == 2 && !p.a_split) {
-        split_lock.lock();
-        void *ws = nullptr;
-        int rc = split_slot(st, split_weights_bytes(p.M, p.K), &ws);
-        if (rc) return rc;
-        if (!ws) {
-            if (!p.A) return kNoSplitSlot;   // only this kernel reads the problem in this form
-            split_lock.unlock();
-            p.w_src = nullptr;               // as a call whose weights are too large to be split
-            return launch_choice(cfg, p, slotless_choice(cfg, p, st), st);
-        }
-        rc = split_weights_launch(p.w_src, p.M, p.K, p.w_row, p.w_k, ws, st);
-        if (rc) return rc;
-        p.a_split = ws;
+    if (c.rowb == 2) {
+        const void *kept = nullptr;
         p.a_split_bytes = split_weights_bytes(p.M, p.K);
+        if (p.keeper) {
+            const int rc = p.keeper->get(p.keeper->key, p.w_src, {p.M, p.K, p.w_row, p.w_k}, &kept);
+            if (rc) return rc;
+        }
+        if (!kept) {
+            void *ws = nullptr;
+            split_lock.lock();
+            if (p.a_split_bytes <= kSplitWsBytes) {
+                const int rc = split_slot(st, p.a_split_bytes, &ws);
+                if (rc) return rc;
+            }
+            if (!ws) {
+                if (!p.A) return kNoSplitSlot;   // only this kernel reads the problem in this form
+                split_lock.unlock();
+                p.w_src = nullptr;               // as a call whose weights are too large to be split
+                return launch_choice(cfg, p, slotless_choice(cfg, p, st), st);
+            }
+            const int rc = split_weights_launch(p.w_src, p.M, p.K, p.w_row, p.w_k, ws, st);
+            if (rc) return rc;
+            kept = ws;
+        }
+        p.a_split = kept;
     }
     int dpc = 0, left = 0;
     p.part_begin = p.dp_tiles = p.tail_tiles = 0;
@@ -951,10 +969,9 @@ static int add_relu_in_place(const onhip_conv_desc_t *d, int OH, int OW, const f
     return rc;
 }
 
-// split, when not null: the same weights (as w has them) in split_weights_launch's form
 static int conv2d_f32_impl(const onhip_conv_desc_t *d, const float *x, const float *w, int packed, const float *bias,
                            const float *silu_lut, float *y, void *stream, const float *addend = nullptr, int relu_after = 0,
-                           const void *split = nullptr) {
+                           const SplitKeeper *keeper = nullptr) {
     int32_t OH, OW;
     int rc = check_conv(d, &OH, &OW);
     if (rc) return rc;
@@ -1016,8 +1033,7 @@ static int conv2d_f32_impl(const onhip_conv_desc_t *d, const float *x, const flo
     p.w_src = w;
     p.w_row = p.K;
     p.w_k = 1;
-    p.a_split = split;
-    p.a_split_bytes = split ? split_weights_bytes(p.M, p.K) : 0;
+    p.keeper = keeper;
     p.B = x;
     p.b_img_stride = (long long) d->cin * d->h * d->w;
     p.b_shift_bytes = ((long long) d->pad_t * d->w + d->pad_l) * 4;
@@ -1454,7 +1470,7 @@ int onhip_conv2d_w8_link(const onhip_conv_desc_t *d, const float *x, const int8_
 // the columns of `b` the rows of its A operand, the rows of `a` (K contiguous) its B, `out` [rows][n] written four columns at
 // a time
 static void matmul_rows_problem(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias, const float *gelu_lut,
-                                const float *addend, float *out, const void *split, IgemmLaunch *cfg, IgemmProblem *p) {
+                                const float *addend, float *out, IgemmLaunch *cfg, IgemmProblem *p) {
     memset(cfg, 0, sizeof(*cfg));
     cfg->dtype = DT_F32;
     cfg->bl = BL_ROWS;
@@ -1464,8 +1480,6 @@ static void matmul_rows_problem(const onhip_matmul_desc_t *d, const float *a, co
     p->M = d->n; p->N = (int) rows; p->K = d->k;
     p->k_units = (p->K + 3) / 4;
     p->w_src = b; p->w_row = 1; p->w_k = d->n;
-    p->a_split = split;
-    p->a_split_bytes = split ? split_weights_bytes(p->M, p->K) : 0;
     p->B = a;
     p->ldb = d->k;
     p->b_slice_bytes = rows * d->k * 4;
@@ -1482,7 +1496,7 @@ static void matmul_rows_problem(const onhip_matmul_desc_t *d, const float *a, co
 }
 
 static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias,
-                       const float *gelu_lut, const float *addend, float *out, void *stream, const void *split = nullptr) {
+                       const float *gelu_lut, const float *addend, float *out, void *stream, const SplitKeeper *keeper = nullptr) {
     if (!d || d->batch < 1 || d->m < 1 || d->k < 1 || d->n < 1) return set_error(ONHIP_ERR_ARG, "matmul: bad shape");
     if (!a || !b || !out) return set_error(ONHIP_ERR_ARG, "matmul: null tensor pointer");
     int batch = d->batch, M = d->m;
@@ -1541,15 +1555,14 @@ static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float
     if (cfg.dtype == DT_F32 && batch == 1 && !getenv("ONHIP_TILE")) {
         IgemmLaunch rcfg;
         IgemmProblem rp;
-        matmul_rows_problem(d, a, b, bias, gelu_lut, addend, out, split, &rcfg, &rp);
+        matmul_rows_problem(d, a, b, bias, gelu_lut, addend, out, &rcfg, &rp);
         Choice c;
         double us;
-        // rule as in model_choice; the pass that splits the weights is priced in even where the caller has them split, so that
+        // rule as in model_choice; the pass that splits the weights is priced in even where the caller keeps them split, so that
         // a product runs the same way, with the same bits, whether its right operand is a model's weight or not
-        if (split) { rp.a_split = nullptr; }
         if (rp.M > 32 && rp.K >= 48 && p.b_slice_bytes < (1LL << 31) && rp.b_slice_bytes < (1LL << 31) && rp.c_slice_bytes < (1LL << 31) &&
             f3_choice(rcfg, rp, &c, &us) && us < f32_us(model_cost(cfg, p, model_choice(cfg, p)))) {
-            rp.a_split = split;
+            rp.keeper = keeper;
             const int rc = launch_choice(rcfg, rp, c, st);
             if (rc != kNoSplitSlot) return rc;
             if (under_capture(st)) return launch_choice(cfg, p, slotless_choice(cfg, p, st), st);
@@ -1926,42 +1939,14 @@ int onhip_gemm_f32(int32_t m, int32_t k, int32_t n, const float *a, const float 
 
 }  // extern "C"
 
-// The plugins keep weights that belong to a loaded model split.  *_split_source: how (the caller's weights as M rows of K
-// elements), where a call with them would run the kernel that reads that form; M = 0 otherwise.
+// The plugins' calls, on weights that they may keep split.
 namespace onhip {
-int conv2d_f32_split(const onhip_conv_desc_t *d, const float *x, const float *w, int packed, const float *bias, const float *silu_lut,
-                     const float *addend, int relu_after, float *y, const void *split, void *stream) {
-    return conv2d_f32_impl(d, x, w, packed, bias, silu_lut, y, stream, addend, relu_after, split);
+int conv2d_f32_kept(const onhip_conv_desc_t *d, const float *x, const float *w, int packed, const float *bias, const float *silu_lut,
+                    const float *addend, int relu_after, float *y, const SplitKeeper *keeper, void *stream) {
+    return conv2d_f32_impl(d, x, w, packed, bias, silu_lut, y, stream, addend, relu_after, keeper);
 }
-SplitSource conv2d_f32_split_source(const onhip_conv_desc_t *d, int packed) {
-    SplitSource src = {0, 0, 0, 0};
-    int32_t OH, OW;
-    if (check_conv(d, &OH, &OW) || d->group != 1 || d->compute != ONHIP_COMPUTE_F32 || getenv("ONHIP_TILE")) return src;
-    if (stem_f32_ok(*d, OH, OW) && (packed || OW >= 96)) return src;
-    IgemmLaunch cfg;
-    memset(&cfg, 0, sizeof(cfg));
-    cfg.dtype = DT_F32;
-    cfg.batch = 1;
-    cfg.bl = packed ? BL_TAPC : plain_pointwise(d) ? BL_PLAIN : BL_GATHER;
-    IgemmProblem p;
-    memset(&p, 0, sizeof(p));
-    p.M = d->cout;
-    p.N = d->n * OH * OW;
-    p.K = d->kh * d->kw * (packed ? packed_cp(d) : d->cin);
-    p.k_units = (p.K + 3) / 4;
-    p.use_tapmask = d->kh * d->kw <= 64;
-    p.a_split = &src;   // as if there were one
-    if (model_choice(cfg, p).rowb == 2) src = {p.M, p.K, p.K, 1};
-    return src;
-}
-int matmul_f32_split(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias, const float *gelu_lut, const float *addend,
-                     float *out, const void *split, void *stream) {
-    return matmul_impl(d, a, b, bias, gelu_lut, addend, out, stream, split);
-}
-SplitSource matmul_f32_split_source(const onhip_matmul_desc_t *d) {
-    SplitSource src = {0, 0, 0, 0};
-    if ((!d->b_shared && d->batch != 1) || d->compute != ONHIP_COMPUTE_F32 || d->n <= 32 || d->k < 48 || getenv("ONHIP_TILE")) return src;
-    src = {d->n, d->k, 1, d->n};   // made whenever a call might use it: the call decides by the number of rows
-    return src;
+int matmul_f32_kept(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias, const float *gelu_lut, const float *addend,
+                    float *out, const SplitKeeper *keeper, void *stream) {
+    return matmul_impl(d, a, b, bias, gelu_lut, addend, out, stream, keeper);
 }
 }  // namespace onhip

@@ -237,14 +237,14 @@ struct IgemmParams {
 // A problem as the host plans it: with what only the fp32 kernel on the 16-bit matrix cores (igemm_f3_kernel.hpp) takes as
 // well, so that the other kernels' parameters are no longer for it.
 struct IgemmProblem : IgemmParams {
-    // the operand A (a weight matrix shared by all batches) split into bf16 parts ahead of time, in the order the matrix
-    // instructions read it, or nullptr
+    // the operand A (a weight matrix shared by all batches) split into bf16 parts, in the order the matrix instructions read
+    // it: set by launch_choice
     const void *a_split;
     long long a_split_bytes;
-    // where that form can be made from on each call when the caller has none: element (row, k) at w_src[row * w_row + k * w_k]
-    // (nullptr: A is not a weight matrix)
+    // where that form is made from: element (row, k) at w_src[row * w_row + k * w_k] (nullptr: A is not a weight matrix)
     const float *w_src;
     long long w_row, w_k;
+    const struct SplitKeeper *keeper;   // who keeps it from call to call, or nullptr: made on each call
     int ldb;                   // B given as rows (BL_ROWS): elements between them
 };
 
@@ -269,14 +269,24 @@ int rowb_f32_launch(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t st
 // fp32 kernel on the 16-bit matrix cores (igemm_f3.hip): p.a_split holds the weights in split_weights_launch's form
 int f3_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t stream);
 inline long long split_weights_bytes(long long M, long long K) { return (M + 31) / 32 * ((K + 15) / 16) * 3072; }
-// api.hip: fp32 convolution and product on weights that are split already (the plugins'), and how to split them
+// Weights as M rows of K elements, element (row, k) at row * s_row + k * s_k.
 struct SplitSource { int M, K; long long s_row, s_k; };
-SplitSource conv2d_f32_split_source(const onhip_conv_desc_t *d, int packed);
-int conv2d_f32_split(const onhip_conv_desc_t *d, const float *x, const float *w, int packed, const float *bias, const float *silu_lut,
-                     const float *addend, int relu_after, float *y, const void *split, void *stream);
-SplitSource matmul_f32_split_source(const onhip_matmul_desc_t *d);
-int matmul_f32_split(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias, const float *gelu_lut, const float *addend,
-                     float *out, const void *split, void *stream);
+// A caller that keeps weights split (the plugins): the launch that reads the split form asks for it.  get: *out = the split form of
+// the weights `from`, laid out as src says and known to the caller as `key`; nullptr where it has none and can make none now, and
+// the launch then splits them on the call.
+struct SplitKeeper {
+    const void *key;
+    int (*get)(const void *key, const float *from, const SplitSource &src, const void **out);
+};
+// api.hip: fp32 convolution and product whose caller keeps the weights split
+int conv2d_f32_kept(const onhip_conv_desc_t *d, const float *x, const float *w, int packed, const float *bias, const float *silu_lut,
+                    const float *addend, int relu_after, float *y, const SplitKeeper *keeper, void *stream);
+int matmul_f32_kept(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias, const float *gelu_lut, const float *addend,
+                    float *out, const SplitKeeper *keeper, void *stream);
+// st is being captured; true as well for the legacy stream while another thread's capture keeps it from being asked
+bool under_capture(hipStream_t st);
+// hipMalloc that is no part of what is captured, by this thread or by another
+hipError_t malloc_outside_capture(void **out, size_t bytes);
 int split_weights_launch(const float *w, int M, int K, long long s_row, long long s_k, void *out, hipStream_t stream);
 // int8 kernel with operand tiles loaded from global memory straight into LDS (igemm_dma.hip): NHWC int8 activations whose
 // padded channel count is a multiple of 64, tiles 128x128, 128x64, 64x128, 64x64, no split-K

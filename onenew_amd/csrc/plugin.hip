@@ -128,15 +128,17 @@ static void drop_split(std::map<const void *, SplitEntry>::iterator it) {
     g_split_blocks.erase(std::find(g_split_blocks.begin(), g_split_blocks.end(), b));
     delete b;
 }
-// *out = the split form of the weights `key` (laid out as `from` and ss say), made when first asked for; nullptr where there
-// is none (ss.M == 0)
+// SplitKeeper::get: made when a launch first asks for it.  Not under capture: the pass would be recorded and not run, and an eval
+// before the first replay would read what nothing has written; the captured call splits for itself.
 static int split_of(const void *key, const float *from, const SplitSource &ss, const void **out) {
     *out = nullptr;
-    if (!ss.M) return ONHIP_OK;
     auto it = g_split.find(key);
     if (it != g_split.end()) {
         const SplitSource &h = it->second.src;
         if (h.M == ss.M && h.K == ss.K && h.s_row == ss.s_row && h.s_k == ss.s_k) { *out = it->second.dev; return ONHIP_OK; }
+    }
+    if (under_capture(g_stream)) return ONHIP_OK;
+    if (it != g_split.end()) {
         ONHIP_CHECK_HIP(hipDeviceSynchronize());
         drop_split(it);
     }
@@ -146,10 +148,10 @@ static int split_of(const void *key, const float *from, const SplitSource &ss, c
         if (b->size - b->used >= bytes) block = b;
     if (!block) {
         block = new SplitBlock{nullptr, bytes > (32u << 20) ? bytes : (32u << 20), 0, 0};
-        const hipError_t e = hipMalloc(reinterpret_cast<void **>(&block->base), block->size);
-        if (e != hipSuccess) {
+        if (malloc_outside_capture(reinterpret_cast<void **>(&block->base), block->size) != hipSuccess) {
+            (void) hipGetLastError();   // no memory to keep it in: the call splits for itself
             delete block;
-            return set_error(ONHIP_ERR_RUNTIME, "split weights: hipMalloc failed: %s", hipGetErrorString(e));
+            return ONHIP_OK;
         }
         g_split_blocks.push_back(block);
     }
@@ -463,23 +465,14 @@ static int conv_eval_fused(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_
             ad.relu = fuse == 2 ? 2 : 0;   // the Relu operator's rules by element index, in the same pass
             rc = onhip_add_f32(&ad, (const float *) y, (const float *) addend, (float *) y, g_stream);
         }
-    } else if (fuse) {
-        const float *wp = nullptr;
-        rc = packed_weights(&d, (const float *) w, &wp);
-        const void *split = nullptr;
-        if (!rc && keep_split) rc = split_of(w, wp ? wp : (const float *) w, conv2d_f32_split_source(&d, wp != nullptr), &split);
-        if (rc) return rc;
-        rc = conv2d_f32_split(&d, (const float *) x, wp ? wp : (const float *) w, wp ? 1 : 0, (const float *) b, (const float *) lut,
-                              (const float *) addend, fuse == 2, (float *) y, split, g_stream);
     } else {
         // k x k dense weights are re-laid out tap-major once, next to their device copy
         const float *wp = nullptr;
         rc = packed_weights(&d, (const float *) w, &wp);
-        const void *split = nullptr;
-        if (!rc && keep_split) rc = split_of(w, wp ? wp : (const float *) w, conv2d_f32_split_source(&d, wp != nullptr), &split);
         if (rc) return rc;
-        rc = conv2d_f32_split(&d, (const float *) x, wp ? wp : (const float *) w, wp ? 1 : 0, (const float *) b, (const float *) lut, nullptr, 0,
-                              (float *) y, split, g_stream);
+        const SplitKeeper keeper = {w, split_of};
+        rc = conv2d_f32_kept(&d, (const float *) x, wp ? wp : (const float *) w, wp ? 1 : 0, (const float *) b, (const float *) lut,
+                             (const float *) addend, fuse == 2, (float *) y, keep_split ? &keeper : nullptr, g_stream);
     }
     if (rc) return rc;
     if (!out_on_dev) return copy_out(host_out, y, out_bytes);
@@ -696,11 +689,7 @@ static int matmul_eval_mode(int mode, BUFFER_INFO_S *params, BUFFER_INFO_S *inpu
     if (b_t->is_fixed_val) rc = const_on_device(b_host, b_bytes, &b);
     else rc = input_on_device(1, b_host, b_bytes, &b);
     if (rc) return rc;
-    const void *split = nullptr;
-    if (b_t->is_fixed_val && (b != b_host || is_held(b))) {
-        rc = split_of(b, (const float *) b, matmul_f32_split_source(&d), &split);
-        if (rc) return rc;
-    }
+    const SplitKeeper kept = {b, split_of}, *keeper = b_t->is_fixed_val && (b != b_host || is_held(b)) ? &kept : nullptr;
     void *host_out = reinterpret_cast<void *>(outputs[0].addr);
     void *y = host_out;
     const bool out_on_dev = is_device_ptr(host_out);
@@ -724,9 +713,9 @@ static int matmul_eval_mode(int mode, BUFFER_INFO_S *params, BUFFER_INFO_S *inpu
         const void *addend;
         rc = input_on_device(5, reinterpret_cast<const void *>(inputs[3].addr), o_bytes, &addend);
         if (rc) return rc;
-        rc = matmul_f32_split(&d, (const float *) a, (const float *) b, (const float *) bias, nullptr, (const float *) addend, (float *) y, split, g_stream);
+        rc = matmul_f32_kept(&d, (const float *) a, (const float *) b, (const float *) bias, nullptr, (const float *) addend, (float *) y, keeper, g_stream);
     } else {
-        rc = matmul_f32_split(&d, (const float *) a, (const float *) b, (const float *) bias, (const float *) lut, nullptr, (float *) y, split, g_stream);
+        rc = matmul_f32_kept(&d, (const float *) a, (const float *) b, (const float *) bias, (const float *) lut, nullptr, (float *) y, keeper, g_stream);
     }
     if (rc) return rc;
     if (!out_on_dev) return copy_out(host_out, y, o_bytes);
