@@ -12,6 +12,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <compare>
 #include <iterator>
 #include <map>
 #include <mutex>
@@ -106,12 +107,20 @@ struct PackedEntry {
 };
 static std::map<const void *, PackedEntry> g_packed;
 
-// Weights in the form of the fp32 kernel on the 16-bit matrix cores (igemm_f3.hip), keyed by the device address of the
-// original: those of a loaded model (onhip_plugin_hold), and those uploaded here from host memory.  They live in blocks of
-// at least 32 MiB that are given back when the last of their tensors is dropped.
+// Weights in the form of the fp32 kernel on the 16-bit matrix cores (igemm_f3.hip): those of a loaded model (onhip_plugin_hold),
+// and those uploaded here from host memory.  A recorded graph holds their addresses, so a copy stays where it is until its weights
+// are forgotten: one whose weights change is made again in place.  They live in blocks of at least 32 MiB that are given back
+// when the last of their tensors is dropped.
 struct SplitBlock { char *base; size_t size, used; int live; };
-struct SplitEntry { void *dev; SplitSource src; SplitBlock *block; };
-static std::map<const void *, SplitEntry> g_split;
+struct SplitKey {
+    const void *w;     // device address of the original weights
+    bool from_copy;    // made from their tap-major copy, not from the original
+    int M, K;
+    long long s_row, s_k;
+    auto operator<=>(const SplitKey &) const = default;
+};
+struct SplitEntry { void *dev; SplitBlock *block; bool stale; };   // stale: the weights changed after it was made
+static std::map<SplitKey, SplitEntry> g_split;
 static std::vector<SplitBlock *> g_split_blocks;
 static std::vector<std::pair<const char *, const char *>> g_held;   // address ranges of loaded models' weights
 
@@ -120,7 +129,7 @@ static bool is_held(const void *p) {
         if (static_cast<const char *>(p) >= r.first && static_cast<const char *>(p) < r.second) return true;
     return false;
 }
-static void drop_split(std::map<const void *, SplitEntry>::iterator it) {
+static void drop_split(std::map<SplitKey, SplitEntry>::iterator it) {
     SplitBlock *b = it->second.block;
     g_split.erase(it);
     if (--b->live) return;
@@ -132,45 +141,52 @@ static void drop_split(std::map<const void *, SplitEntry>::iterator it) {
 // before the first replay would read what nothing has written; the captured call splits for itself.
 static int split_of(const void *key, const float *from, const SplitSource &ss, const void **out) {
     *out = nullptr;
-    auto it = g_split.find(key);
-    if (it != g_split.end()) {
-        const SplitSource &h = it->second.src;
-        if (h.M == ss.M && h.K == ss.K && h.s_row == ss.s_row && h.s_k == ss.s_k) { *out = it->second.dev; return ONHIP_OK; }
-    }
+    const SplitKey k = {key, from != key, ss.M, ss.K, ss.s_row, ss.s_k};
+    auto it = g_split.find(k);
+    if (it != g_split.end() && !it->second.stale) { *out = it->second.dev; return ONHIP_OK; }
     if (under_capture(g_stream)) return ONHIP_OK;
-    if (it != g_split.end()) {
-        ONHIP_CHECK_HIP(hipDeviceSynchronize());
-        drop_split(it);
-    }
-    const size_t bytes = ((size_t) split_weights_bytes(ss.M, ss.K) + 255) / 256 * 256;
-    SplitBlock *block = nullptr;
-    for (SplitBlock *b : g_split_blocks)
-        if (b->size - b->used >= bytes) block = b;
-    if (!block) {
-        block = new SplitBlock{nullptr, bytes > (32u << 20) ? bytes : (32u << 20), 0, 0};
-        if (malloc_outside_capture(reinterpret_cast<void **>(&block->base), block->size) != hipSuccess) {
-            (void) hipGetLastError();   // no memory to keep it in: the call splits for itself
-            delete block;
-            return ONHIP_OK;
+    if (it == g_split.end()) {
+        const size_t bytes = ((size_t) split_weights_bytes(ss.M, ss.K) + 255) / 256 * 256;
+        SplitBlock *block = nullptr;
+        for (SplitBlock *b : g_split_blocks)
+            if (b->size - b->used >= bytes) block = b;
+        if (!block) {
+            block = new SplitBlock{nullptr, bytes > (32u << 20) ? bytes : (32u << 20), 0, 0};
+            if (malloc_outside_capture(reinterpret_cast<void **>(&block->base), block->size) != hipSuccess) {
+                (void) hipGetLastError();   // no memory to keep it in: the call splits for itself
+                delete block;
+                return ONHIP_OK;
+            }
+            g_split_blocks.push_back(block);
         }
-        g_split_blocks.push_back(block);
+        it = g_split.emplace(k, SplitEntry{block->base + block->used, block, true}).first;
+        block->used += bytes;
+        ++block->live;
     }
-    void *dev = block->base + block->used;
-    block->used += bytes;
-    ++block->live;
-    it = g_split.emplace(key, SplitEntry{dev, ss, block}).first;
-    const int rc = split_weights_launch(from, ss.M, ss.K, ss.s_row, ss.s_k, dev, g_stream);
-    if (rc) { drop_split(it); return rc; }
-    *out = dev;
+    const int rc = split_weights_launch(from, ss.M, ss.K, ss.s_row, ss.s_k, it->second.dev, g_stream);
+    if (rc) return rc;
+    it->second.stale = false;
+    *out = it->second.dev;
+    return ONHIP_OK;
+}
+// The weights at w_dev have just been uploaded again (default stream, complete): their split forms follow at once, so that a replay of a
+// graph sees them as it sees the upload itself; one made from a tap-major copy follows when that copy has been made again.
+static int refresh_split(const void *w_dev) {
+    bool any = false;
+    for (auto it = g_split.lower_bound(SplitKey{w_dev, false, 0, 0, 0, 0}); it != g_split.end() && it->first.w == w_dev; ++it) {
+        const SplitKey &k = it->first;
+        it->second.stale = true;
+        if (k.from_copy) continue;
+        const int rc = split_weights_launch(static_cast<const float *>(w_dev), k.M, k.K, k.s_row, k.s_k, it->second.dev, nullptr);
+        if (rc) return rc;
+        it->second.stale = false;
+        any = true;
+    }
+    if (any) ONHIP_CHECK_HIP(hipStreamSynchronize(nullptr));
     return ONHIP_OK;
 }
 
 static void drop_packed(const void *w_dev) {
-    auto sp = g_split.find(w_dev);
-    if (sp != g_split.end()) {
-        (void) hipDeviceSynchronize();   // a kernel may still be reading it, and its block need not be freed now
-        drop_split(sp);
-    }
     auto it = g_packed.find(w_dev);
     if (it != g_packed.end()) {
         (void) hipFree(it->second.dev);
@@ -302,6 +318,8 @@ static int const_on_device(const void *host, size_t bytes, const void **dev) {
             ONHIP_CHECK_HIP(hipMemcpy(it->second.dev, host, bytes, hipMemcpyHostToDevice));
             it->second.fingerprint = fp;
             drop_packed(it->second.dev);   // a packed copy of the old content is stale
+            const int rc = refresh_split(it->second.dev);
+            if (rc) return rc;
         }
         *dev = it->second.dev;
         return ONHIP_OK;
@@ -1247,7 +1265,7 @@ int onhip_plugin_forget(const void *base, size_t bytes) {
         }
     }
     for (auto it = g_split.begin(); it != g_split.end();) {
-        const char *k = static_cast<const char *>(it->first);
+        const char *k = static_cast<const char *>(it->first.w);
         auto next = std::next(it);
         if (k >= lo && k < hi) {
             if (!any) ONHIP_CHECK_HIP(hipDeviceSynchronize());

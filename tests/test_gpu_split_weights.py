@@ -130,3 +130,25 @@ def test_first_needed_under_capture(kind, torch_dev):
         assert torch.equal(recorded, y)
         layer(x, y)
         layer.check(x, y)
+
+
+@pytest.mark.parametrize("kind", ["conv", "linear"])
+def test_weights_changed_under_a_recorded_graph(kind, torch_dev):
+    """host weights updated in place: the graph recorded before goes on reading its copy of them, which holds the new ones"""
+    torch = torch_dev
+    print(f"split weights changed under a graph: {kind}", flush=True)
+    layer = Layer(torch, kind, 12)
+    x, y = layer.input(16384)
+    layer(x, y)
+    layer.check(x, y)
+    recorded = torch.zeros_like(y)
+    graph = record(torch, layer, x, recorded, torch.cuda.Stream())
+    for _ in range(3):
+        layer.set_weights(torch.randn(layer.M, layer.K, generator=layer.g) / 16)
+        layer(x, y)
+        layer.check(x, y)
+        recorded.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(recorded, y)
