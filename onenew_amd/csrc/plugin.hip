@@ -32,8 +32,11 @@ static bool g_async = false;
 // (onhip_plugin_set_stream)
 static hipStream_t g_stream = nullptr;
 
+static void settle_split(hipStream_t done);
 static int wait_for_output() {
-    if (!g_async) ONHIP_CHECK_HIP(hipStreamSynchronize(g_stream));
+    if (g_async) return ONHIP_OK;
+    ONHIP_CHECK_HIP(hipStreamSynchronize(g_stream));
+    settle_split(g_stream);
     return ONHIP_OK;
 }
 
@@ -119,8 +122,23 @@ struct SplitKey {
     long long s_row, s_k;
     auto operator<=>(const SplitKey &) const = default;
 };
-struct SplitEntry { void *dev; SplitBlock *block; bool stale; };   // stale: the weights changed after it was made
+struct SplitEntry {
+    void *dev;
+    SplitBlock *block;
+    bool stale;            // the weights changed after it was made
+    bool settled;          // the pass that made it is known to be over: any stream may read it
+    hipStream_t made_on;   // until then this one only
+};
 static std::map<SplitKey, SplitEntry> g_split;
+static bool g_split_unsettled = false;   // some entry is not settled
+static void settle_split(hipStream_t done) {   // `done` has been waited for
+    if (!g_split_unsettled) return;
+    g_split_unsettled = false;
+    for (auto &kv : g_split) {
+        if (kv.second.made_on == done) kv.second.settled = true;
+        if (!kv.second.settled) g_split_unsettled = true;
+    }
+}
 static std::vector<SplitBlock *> g_split_blocks;
 static std::vector<std::pair<const char *, const char *>> g_held;   // address ranges of loaded models' weights
 
@@ -143,8 +161,18 @@ static int split_of(const void *key, const float *from, const SplitSource &ss, c
     *out = nullptr;
     const SplitKey k = {key, from != key, ss.M, ss.K, ss.s_row, ss.s_k};
     auto it = g_split.find(k);
-    if (it != g_split.end() && !it->second.stale) { *out = it->second.dev; return ONHIP_OK; }
+    const bool made = it != g_split.end() && !it->second.stale;
+    if (made && (it->second.settled || it->second.made_on == g_stream)) { *out = it->second.dev; return ONHIP_OK; }
     if (under_capture(g_stream)) return ONHIP_OK;
+    if (made) {   // by a pass on another stream, which may not have run yet
+        if (hipStreamSynchronize(it->second.made_on) != hipSuccess) {   // destroyed since
+            (void) hipGetLastError();
+            ONHIP_CHECK_HIP(hipDeviceSynchronize());
+        }
+        settle_split(it->second.made_on);
+        *out = it->second.dev;
+        return ONHIP_OK;
+    }
     if (it == g_split.end()) {
         const size_t bytes = ((size_t) split_weights_bytes(ss.M, ss.K) + 255) / 256 * 256;
         SplitBlock *block = nullptr;
@@ -159,13 +187,17 @@ static int split_of(const void *key, const float *from, const SplitSource &ss, c
             }
             g_split_blocks.push_back(block);
         }
-        it = g_split.emplace(k, SplitEntry{block->base + block->used, block, true}).first;
+        it = g_split.emplace(k, SplitEntry{block->base + block->used, block, true, false, nullptr}).first;
         block->used += bytes;
         ++block->live;
     }
     const int rc = split_weights_launch(from, ss.M, ss.K, ss.s_row, ss.s_k, it->second.dev, g_stream);
     if (rc) return rc;
     it->second.stale = false;
+    it->second.made_on = g_stream;
+    it->second.settled = g_stream == hipStreamPerThread;   // one handle, a stream for each thread
+    if (it->second.settled) ONHIP_CHECK_HIP(hipStreamSynchronize(g_stream));
+    else g_split_unsettled = true;
     *out = it->second.dev;
     return ONHIP_OK;
 }
@@ -180,7 +212,7 @@ static int refresh_split(const void *w_dev) {
         const int rc = split_weights_launch(static_cast<const float *>(w_dev), k.M, k.K, k.s_row, k.s_k, it->second.dev, nullptr);
         if (rc) return rc;
         it->second.stale = false;
-        any = true;
+        it->second.settled = any = true;
     }
     if (any) ONHIP_CHECK_HIP(hipStreamSynchronize(nullptr));
     return ONHIP_OK;

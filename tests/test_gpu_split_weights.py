@@ -152,3 +152,28 @@ def test_weights_changed_under_a_recorded_graph(kind, torch_dev):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(recorded, y)
+
+
+@pytest.mark.parametrize("kind", ["conv", "linear"])
+def test_next_eval_on_another_stream(kind, torch_dev):
+    """the split form is made behind other work of one stream; the next eval, on a second stream, does not run ahead of it"""
+    torch = torch_dev
+    print(f"split weights and a second stream: {kind}", flush=True)
+    layer = Layer(torch, kind, 13)
+    x, y = layer.input(16)
+    layer.hint(64)
+    layer(x, y)                       # weights on the device, no split form
+    layer.hint(16)
+    x, y = layer.input(16384)
+    z = torch.zeros_like(y)
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(first):
+        torch.cuda._sleep(20_000_000)   # about 10 ms
+    for stream, out in ((first, y), (second, z)):
+        with evals_on(stream):
+            layer(x, out)
+            assert hip.last_launch_choice()[4] == 2
+    torch.cuda.synchronize()
+    layer.check(x, z)
+    assert torch.equal(y, z)
