@@ -164,12 +164,13 @@ static int split_of(const void *key, const float *from, const SplitSource &ss, c
     const bool made = it != g_split.end() && !it->second.stale;
     if (made && (it->second.settled || it->second.made_on == g_stream)) { *out = it->second.dev; return ONHIP_OK; }
     if (under_capture(g_stream)) return ONHIP_OK;
-    if (made) {   // by a pass on another stream, which may not have run yet
-        if (hipStreamSynchronize(it->second.made_on) != hipSuccess) {   // destroyed since
+    if (made) {   // by a pass on another stream, which may not have run yet; that stream may be gone
+        if (hipDeviceSynchronize() != hipSuccess) {   // another thread's capture forbids it
             (void) hipGetLastError();
-            ONHIP_CHECK_HIP(hipDeviceSynchronize());
+            return ONHIP_OK;
         }
-        settle_split(it->second.made_on);
+        for (auto &kv : g_split) kv.second.settled = !kv.second.stale;
+        g_split_unsettled = false;
         *out = it->second.dev;
         return ONHIP_OK;
     }
