@@ -567,7 +567,8 @@ int onhip_plugin_hold(const void *base, size_t bytes);
  * library is loaded (the reference keeps them in vectors filled once at load, host/op.h).  No counterpart in the
  * reference. */
 int onhip_plugin_trust_weights(int on);
-/* Drops the device copies of weights the plugin level keeps between calls. */
+/* Drops the device copies of weights the plugin level keeps between calls, and the kernel level's memory for weights that are split
+ * on the call, but for what recorded graphs hold. */
 int onhip_plugin_release(void);
 
 #ifdef __cplusplus

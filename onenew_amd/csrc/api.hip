@@ -133,69 +133,159 @@ static int get_scratch(size_t bytes, void **out) {
     return ONHIP_OK;
 }
 
-// Split weights of a call whose caller has none (launch_choice).  A stream keeps the slot that its first such call took and
-// allocated, since launches on two streams may overlap; the per-thread default stream is one for each thread.  A recorded graph
-// may be replayed on any stream, also while the one it was recorded on goes on using its slot: each capture has slots of its
-// own.  Slots are kept until the process ends, as graphs hold their addresses, eight for streams and 32 for captures at most.
-// A call that finds all of them taken, and weights whose split form is larger than a slot, run the other fp32 kernels.  The
-// pass that splits and the launch that reads follow each other on the stream while g_split_mu is held: another thread's calls
-// on the same stream go before both or behind both.  The entry point that allocates nothing takes part of its own array.
+// Split weights of a call whose caller keeps none (launch_choice): 16 MiB slots.  Launches on two streams may overlap, so each
+// stream has a slot (the per-thread default stream one for each thread), eight streams of a device at a time: one more takes over
+// the slot used least recently that is free of work, or runs behind its work.  Another stream's handle says nothing about
+// that, as the stream may have been destroyed: from the first such take-over on, which waits for the device, an event follows every
+// use (1 us of the GPU's time and 3 of the host's, 3 of the GPU's if the event fences the host's memory as well).
+// A recorded graph may be replayed on any stream, also while the one it was recorded on goes on using its slot: each capture has
+// slots of its own, which the graph holds as user objects, so that they are free again when it and what was instantiated
+// from it are gone.  32 of a device at most: one more capture while all their graphs live, a device without memory for another slot,
+// and weights whose split form is larger than a slot run the other fp32 kernels.  onhip_plugin_release gives the memory of the
+// slots back that no graph holds.
+// The pass that splits and the launch that reads follow each other on the stream while g_split_mu is held: another thread's
+// calls on the same stream go before both or behind both.  The entry point that allocates nothing takes part of its own array.
 static const long long kSplitWsBytes = 16LL << 20;
 static const int kSplitSlots = 8, kSplitCaptureSlots = 32;
+struct SplitSlot {
+    int dev;
+    void *mem;
+    std::atomic<bool> idle{true};   // nobody's: not a stream's, and no graph holds it
+    // whose it is otherwise
+    hipStream_t stream;
+    std::thread::id thread;
+    bool captured;
+    unsigned long long capture, used;
+    hipEvent_t over = nullptr;      // behind its last use, where recorded
+    bool recorded = false;
+};
 static std::mutex g_split_mu;
-struct SplitSlot { int dev; hipStream_t stream; std::thread::id thread; bool captured; unsigned long long capture; void *mem; };
-static std::vector<SplitSlot> g_split_slots;
-// st is being captured (or may be: *known false); *id = which capture, 0 for none
-static bool capture_info(hipStream_t st, unsigned long long *id, bool *known) {
+static std::vector<SplitSlot *> &g_split_slots = *new std::vector<SplitSlot *>;   // graphs may outlive the static objects
+static unsigned long long g_split_uses = 0;
+static bool g_split_crowded = false;   // a slot has been taken over
+// what this thread calls meanwhile is no part of a capture, its own or another thread's
+struct OutsideCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    OutsideCapture() { (void) hipThreadExchangeStreamCaptureMode(&mode); }
+    ~OutsideCapture() { (void) hipThreadExchangeStreamCaptureMode(&mode); }
+};
+hipError_t malloc_outside_capture(void **out, size_t bytes) {
+    OutsideCapture scope;
+    return hipMalloc(out, bytes);
+}
+// st is being captured (or may be: *known false); *id = which capture, 0 for none, and *graph = what it records into
+static bool capture_info(hipStream_t st, unsigned long long *id, bool *known, hipGraph_t *graph) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    unsigned long long which = 0;
-    const bool ok = hipStreamGetCaptureInfo(st, &cap, &which) == hipSuccess;
+    *id = 0;
+    const bool ok = hipStreamGetCaptureInfo_v2(st, &cap, id, graph, nullptr, nullptr) == hipSuccess;
     if (!ok) (void) hipGetLastError();   // the legacy stream while another one is captured
     const bool on = !ok || cap != hipStreamCaptureStatusNone;
-    *id = on ? which : 0;
+    if (!on) *id = 0;
     *known = ok && (cap == hipStreamCaptureStatusNone || cap == hipStreamCaptureStatusActive);
     return on;
 }
 bool under_capture(hipStream_t st) {
-    unsigned long long id;
-    bool known;
-    return capture_info(st, &id, &known);
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
+    (void) hipGetLastError();
+    return true;
 }
-hipError_t malloc_outside_capture(void **out, size_t bytes) {
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
-    if (e != hipSuccess) return e;
-    e = hipMalloc(out, bytes);
-    const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
-    return e != hipSuccess ? e : back;
+static void slot_given_back(void *slot) { static_cast<SplitSlot *>(slot)->idle.store(true); }   // HIP's, when the last graph is gone
+// A slot of another stream for st, whose work from here on does not meet that stream's; nullptr if there is none.
+static SplitSlot *take_over(int dev, hipStream_t st) {
+    OutsideCapture scope;
+    SplitSlot *oldest = nullptr, *done = nullptr;
+    for (SplitSlot *s : g_split_slots) {
+        if (s->dev != dev || s->idle.load() || s->captured) continue;
+        if (!oldest || s->used < oldest->used) oldest = s;
+        if ((!done || s->used < done->used) && s->recorded && hipEventQuery(s->over) == hipSuccess) done = s;
+    }
+    (void) hipGetLastError();   // an event that is not ready
+    g_split_crowded = true;
+    if (done || !oldest) return done;
+    const bool ordered = oldest->recorded ? hipStreamWaitEvent(st, oldest->over, 0) == hipSuccess : hipDeviceSynchronize() == hipSuccess;
+    if (!ordered) (void) hipGetLastError();
+    return ordered ? oldest : nullptr;
+}
+// behind the launch that has read the slot's weights; g_split_mu held
+static void slot_used(SplitSlot *s, hipStream_t st) {
+    s->recorded = false;
+    if (s->captured || !g_split_crowded) return;
+    OutsideCapture scope;
+    if (!s->over && hipEventCreateWithFlags(&s->over, hipEventDisableTiming | hipEventDisableSystemFence) != hipSuccess) s->over = nullptr;
+    s->recorded = s->over && hipEventRecord(s->over, st) == hipSuccess;
+    if (!s->recorded) (void) hipGetLastError();
 }
 // *out = the slot of stream st on the current device, nullptr if there is none; g_split_mu held
-static int split_slot(hipStream_t st, long long bytes, void **out) {
-    if (tl_noalloc) {   // the last part of its array: f3_choice leaves the partial sums the rest
-        *out = static_cast<char *>(tl_noalloc) + kNoAllocScratchBytes - bytes;
-        return ONHIP_OK;
-    }
+static int split_slot(hipStream_t st, SplitSlot **out) {
+    *out = nullptr;
     int dev = -1;
     ONHIP_CHECK_HIP(hipGetDevice(&dev));
     const std::thread::id me = st == hipStreamPerThread ? std::this_thread::get_id() : std::thread::id();
-    *out = nullptr;
     unsigned long long capture;
     bool known;
-    const bool captured = capture_info(st, &capture, &known);
+    hipGraph_t graph = nullptr;
+    const bool captured = capture_info(st, &capture, &known, &graph);
     if (!known) return ONHIP_OK;
+    SplitSlot *slot = nullptr, *idle = nullptr;
     int taken = 0;
-    for (const SplitSlot &s : g_split_slots) {
-        taken += s.captured == captured;
-        if (s.dev == dev && s.stream == st && s.thread == me && s.captured == captured && s.capture == capture) *out = s.mem;
+    for (SplitSlot *s : g_split_slots) {
+        if (s->dev != dev) continue;
+        if (s->idle.load()) { idle = s; continue; }
+        if (s->captured != captured) continue;
+        ++taken;
+        if (s->stream == st && s->thread == me && s->capture == capture) slot = s;
     }
-    if (*out || taken == (captured ? kSplitCaptureSlots : kSplitSlots)) return ONHIP_OK;
-    if (malloc_outside_capture(out, kSplitWsBytes) != hipSuccess) {
-        (void) hipGetLastError();   // no memory for it: as without a slot
-        *out = nullptr;
-        return ONHIP_OK;
+    if (!slot) {
+        if (taken < (captured ? kSplitCaptureSlots : kSplitSlots)) {
+            slot = idle;
+            void *mem = nullptr;
+            if (!slot && malloc_outside_capture(&mem, kSplitWsBytes) == hipSuccess) {
+                slot = new SplitSlot;
+                slot->dev = dev;
+                slot->mem = mem;
+                g_split_slots.push_back(slot);
+            }
+            if (!slot) (void) hipGetLastError();
+        }
+        if (!slot && !captured) slot = take_over(dev, st);
+        if (!slot) return ONHIP_OK;
+        if (captured) {   // the graph's from here on
+            hipUserObject_t owner;
+            if (hipUserObjectCreate(&owner, slot, slot_given_back, 1, hipUserObjectNoDestructorSync) != hipSuccess) {
+                (void) hipGetLastError();
+                return ONHIP_OK;
+            }
+            slot->idle.store(false);
+            if (hipGraphRetainUserObject(graph, owner, 1, hipGraphUserObjectMove) != hipSuccess) {
+                (void) hipGetLastError();
+                (void) hipUserObjectRelease(owner, 1);   // gives the slot back
+                return ONHIP_OK;
+            }
+        }
+        slot->idle.store(false);
+        slot->stream = st;
+        slot->thread = me;
+        slot->captured = captured;
+        slot->capture = capture;
+        slot->recorded = false;
     }
-    g_split_slots.push_back({dev, st, me, captured, capture, *out});
+    slot->used = ++g_split_uses;
+    *out = slot;
     return ONHIP_OK;
+}
+// the memory of every slot that no graph holds; the device is idle
+void release_split_slots() {
+    std::lock_guard<std::mutex> lock(g_split_mu);
+    (void) hipDeviceSynchronize();   // and stays so: a launch that uses a slot holds the lock
+    for (size_t i = g_split_slots.size(); i-- > 0;) {
+        SplitSlot *s = g_split_slots[i];
+        if (!s->idle.load() && s->captured) continue;
+        (void) hipFree(s->mem);
+        if (s->over) (void) hipEventDestroy(s->over);
+        delete s;
+        g_split_slots.erase(g_split_slots.begin() + i);
+    }
 }
 
 // Workspace of the split-K reduction that runs inside the launch: partial sums and one arrival counter per tile in
@@ -612,6 +702,10 @@ static Choice slotless_choice(const IgemmLaunch &cfg, const IgemmProblem &p, hip
 // Runs the problem the way the choice says.
 static int launch_choice(IgemmLaunch cfg, IgemmProblem p, const Choice &c, hipStream_t st) {
     std::unique_lock<std::mutex> split_lock(g_split_mu, std::defer_lock);
+    struct Use {   // of a slot, on every way out, before the lock is given up
+        SplitSlot *slot; hipStream_t st;
+        ~Use() { if (slot) slot_used(slot, st); }
+    } use{nullptr, st};
     if (c.rowb == 2) {
         const void *kept = nullptr;
         p.a_split_bytes = split_weights_bytes(p.M, p.K);
@@ -621,14 +715,17 @@ static int launch_choice(IgemmLaunch cfg, IgemmProblem p, const Choice &c, hipSt
         }
         if (!kept) {
             void *ws = nullptr;
-            split_lock.lock();
-            if (p.a_split_bytes <= kSplitWsBytes) {
-                const int rc = split_slot(st, p.a_split_bytes, &ws);
+            if (tl_noalloc) {   // the last part of its array: f3_choice leaves the partial sums the rest
+                ws = static_cast<char *>(tl_noalloc) + kNoAllocScratchBytes - p.a_split_bytes;
+            } else if (p.a_split_bytes <= kSplitWsBytes) {
+                split_lock.lock();
+                const int rc = split_slot(st, &use.slot);
                 if (rc) return rc;
+                if (use.slot) ws = use.slot->mem;
             }
             if (!ws) {
                 if (!p.A) return kNoSplitSlot;   // only this kernel reads the problem in this form
-                split_lock.unlock();
+                if (split_lock.owns_lock()) split_lock.unlock();
                 p.w_src = nullptr;               // as a call whose weights are too large to be split
                 return launch_choice(cfg, p, slotless_choice(cfg, p, st), st);
             }

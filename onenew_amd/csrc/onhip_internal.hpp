@@ -287,6 +287,7 @@ int matmul_f32_kept(const onhip_matmul_desc_t *d, const float *a, const float *b
 bool under_capture(hipStream_t st);
 // hipMalloc that is no part of what is captured, by this thread or by another
 hipError_t malloc_outside_capture(void **out, size_t bytes);
+void release_split_slots();   // api.hip: memory of weights split on the call
 int split_weights_launch(const float *w, int M, int K, long long s_row, long long s_k, void *out, hipStream_t stream);
 // int8 kernel with operand tiles loaded from global memory straight into LDS (igemm_dma.hip): NHWC int8 activations whose
 // padded channel count is a multiple of 64, tiles 128x128, 128x64, 64x128, 64x64, no split-K

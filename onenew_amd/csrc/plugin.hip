@@ -1331,6 +1331,7 @@ int onhip_plugin_release(void) {
     for (auto &kv : g_packed) (void) hipFree(kv.second.dev);
     g_packed.clear();
     while (!g_split.empty()) drop_split(g_split.begin());
+    release_split_slots();
     for (auto &kv : g_const) (void) hipFree(kv.second.dev);
     g_const.clear();
     for (auto &b : g_stage) {

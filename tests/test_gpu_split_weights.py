@@ -177,3 +177,91 @@ def test_next_eval_on_another_stream(kind, torch_dev):
     torch.cuda.synchronize()
     layer.check(x, z)
     assert torch.equal(y, z)
+
+
+@pytest.fixture(scope="module")
+def products(torch_dev):
+    """products with enough work for weights split on the call, on operands of their own, and what they come to"""
+    torch = torch_dev
+    m, k, n = 8195, 773, 1030
+    g = torch.Generator(device="cuda").manual_seed(5)
+    jobs = []
+    for _ in range(12):
+        a, b = torch.randn(m, k, generator=g, device="cuda"), torch.randn(k, n, generator=g, device="cuda")
+        bound = (a.double().abs() @ b.double().abs()) * ((k + 4) * 2.0 ** -24 + 2.0 ** -23)
+        jobs.append((a, b, torch.zeros(m, n, device="cuda"), a.double() @ b.double(), bound))
+    return jobs
+
+
+def multiply(job):
+    hip.matmul(job[0], job[1], out=job[2])
+    assert hip.last_launch_choice()[4] == 2
+
+
+def right(job):
+    err = (job[2].double() - job[3]).abs()
+    assert bool((err <= job[4]).all()), float((err / job[4]).max())
+    job[2].zero_()
+
+
+def test_more_streams_than_slots(products, torch_dev):
+    """twelve streams at once, a second round in another order, and streams that come and go: every one splits on the call"""
+    torch = torch_dev
+    print("split weights: streams", flush=True)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in products]
+    for order in (range(12), range(11, -1, -1)):
+        for i in order:
+            with torch.cuda.stream(streams[i]):
+                multiply(products[i])
+        torch.cuda.synchronize()
+        for job in products:
+            right(job)
+    hiprt, old = C.CDLL(None), []
+    for _ in range(3):   # nine new streams while the nine before are still there, which are destroyed then
+        new = [C.c_void_p() for _ in range(9)]
+        for handle in new:
+            assert hiprt.hipStreamCreate(C.byref(handle)) == 0
+        for handle in old:
+            assert hiprt.hipStreamDestroy(handle) == 0
+        for handle, job in zip(new, products):
+            with torch.cuda.stream(torch.cuda.ExternalStream(handle.value)):
+                multiply(job)
+        torch.cuda.synchronize()
+        for job in products[:9]:
+            right(job)
+        old = new
+    for handle in old:
+        assert hiprt.hipStreamDestroy(handle) == 0
+
+
+def test_captures_that_come_and_go(products, torch_dev):
+    """graphs recorded and dropped, more of them than there are slots: each has a slot, and the one that lives keeps its own"""
+    torch = torch_dev
+    print("split weights: captures", flush=True)
+    stream = torch.cuda.Stream()
+
+    def graph_of(job):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            multiply(job)
+        return graph
+
+    torch.cuda.synchronize()
+    kept = graph_of(products[0])
+    for i in range(70):
+        job = products[1 + i % 11]
+        graph = graph_of(job)
+        graph.replay()
+        kept.replay()
+        torch.cuda.synchronize()
+        if i % 10 == 9:
+            right(job)
+            right(products[0])
+        del graph
+    assert hip.load().onhip_plugin_release() == 0   # slots that no graph holds are given back, not this one's
+    kept.replay()
+    multiply(products[1])
+    torch.cuda.synchronize()
+    right(products[0])
+    right(products[1])
