@@ -171,8 +171,10 @@ int onhip_conv2d_f32_noalloc(const onhip_conv_desc_t *d, const float *x, const f
 int onhip_conv2d_f32_add(const onhip_conv_desc_t *d, const float *x, const float *w, int32_t packed, const float *bias,
                          const float *silu_lut, const float *addend, int32_t relu_after, float *y, void *stream);
 
-/* Bytes of device scratch onhip_conv2d_w8a32 (and onhip_conv2d_w8_link on fp32 activations) needs for `d`: the int8
- * copy of the activations.  A depthwise convolution uses it only in onhip_conv2d_w8_link with fp32 in and int8 out. */
+/* Bytes of device scratch onhip_conv2d_w8a32 (and onhip_conv2d_w8_link on fp32 activations) takes for `d`: the re-laid-out
+ * weights, the int8 copy of the activations and, for layers with few output tiles and a long reduction, up to 8 MiB for partial
+ * sums.  A call that is given less, but enough for the weights (unless packed) and the activations, runs in one piece, with the
+ * same results.  A depthwise convolution uses it only in onhip_conv2d_w8_link with fp32 in and int8 out. */
 size_t onhip_conv2d_w8a32_workspace(const onhip_conv_desc_t *d);
 
 /* W8A32 convolution: fp32 activations quantised with d->input_scale, int8 weights
@@ -190,7 +192,7 @@ int onhip_conv2d_w8a32(const onhip_conv_desc_t *d, const float *x, const int8_t 
  * blocks, zero padded), so that a call does not repeat it: same role as the weight buffer the
  * reference keeps for the lifetime of the net (host/ops/conv.h:148-154).  Bytes needed (0 for
  * depthwise, which reads the reference layout), the packing, and the convolution on packed weights
- * (w8_packed 16-byte aligned; the workspace then only holds the int8 activations, the size
+ * (w8_packed 16-byte aligned; the workspace then holds the int8 activations and partial sums, the size
  * onhip_conv2d_w8a32_workspace reports is enough).  Results are identical to onhip_conv2d_w8a32. */
 size_t onhip_conv2d_w8a32_packed_weight_bytes(const onhip_conv_desc_t *d);
 int onhip_conv2d_w8a32_pack_weights(const onhip_conv_desc_t *d, const int8_t *w8, int8_t *packed,

@@ -413,7 +413,9 @@ static int apply_choice(IgemmLaunch &cfg, IgemmProblem &p, const Choice &c) {
             cfg.split = split;
             p.k_split_units = tiles_per * upt;
             p.arrive = nullptr;
-            if (c.fin && cfg.dtype != DT_I8 && bytes <= kUcBytes && !tl_noalloc) {
+            if ((long long) bytes <= p.slices_bytes) {
+                p.partial = p.slices;
+            } else if (c.fin && cfg.dtype != DT_I8 && bytes <= kUcBytes && !tl_noalloc) {
                 void *uc; int *arr;
                 rc = get_uc(&uc, &arr);
                 if (rc) return rc;
@@ -504,6 +506,11 @@ static bool candidate_ok(const IgemmLaunch &cfg, const IgemmProblem &p, const Ch
     return true;
 }
 
+// K slices that an int8 launch with an fp32 result may be cut into on the caller's workspace (0 or 1: none)
+static long long int8_slices(const IgemmLaunch &cfg, const IgemmProblem &p) {
+    return cfg.dtype == DT_I8 && !p.out_s8 ? p.slices_bytes / (4LL * p.M * p.N) : 0;
+}
+
 // Cost model (cycles).  A CU works through its share of the workgroups; co-resident workgroups share
 // the MFMA pipes, so the MFMA time adds up while the per-workgroup fill/drain latency overlaps when
 // several are resident.  Split-K adds the partial-sum traffic and a second launch.
@@ -529,8 +536,10 @@ static double model_cost(const IgemmLaunch &cfg, const IgemmProblem &p, const Ch
     // int8 with up to two workgroups per CU: a K tile takes about 500 cycles (0.23 us) whatever its MFMAs, a workgroup's loads,
     // LDS and barrier one after the other; the launch that adds slices up costs 2.8 us.  YOLOv8s at batch 1, the layers with
     // a few tiles and a K of 2304 / 4608: 17.3-19.0 / 25.7 us in one piece, 13.7 / 14.5 us in four slices
-    // (int8 results stay whole: a launch in slices leaves the padding of their channels unwritten)
-    const bool few_int8 = cfg.dtype == DT_I8 && !p.out_s8 && wgs <= 512.0;
+    // (int8 results stay whole: a launch in slices leaves the padding of their channels unwritten).  Only where the caller's
+    // workspace has room for the partial sums: the shared block for them allocates and is not for overlapping launches, which
+    // such layers did without before
+    const bool few_int8 = int8_slices(cfg, p) > 1 && wgs <= 512.0;
     if (few_int8) cycles = fmax(cycles, ceil(per_cu / resident) * (per * 500.0 + fixed));
     if (c.split > 1) cycles += (few_int8 ? 6300.0 : 9000.0) + (double) (c.split + 1) * p.M * p.N * cfg.batch * 4.0 / 1500.0;
     return cycles;
@@ -630,12 +639,14 @@ static Choice model_choice(const IgemmLaunch &cfg, const IgemmProblem &p) {
         const long long tiles = (long long) ((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn);
         if (tiles >= 512 && candidate_ok(cfg, p, c)) return c;   // measured at batch 64 only: at least two workgroups per CU
     }
+    const long long slices = int8_slices(cfg, p) > 1 ? int8_slices(cfg, p) : 1 << 20;
     for (int pass = tl_hint_bm ? 0 : 1; pass < 2; ++pass) {   // pass 0: the hinted tile; pass 1: every tile
         double best_cost = 1e300;
         for (int t = 0; t < kNumTiles; ++t)
             for (int s = 0; s < kNumSplits; ++s) {
                 const Choice c = {kTiles[t][0], kTiles[t][1], kSplits[s], 0, 0, 0};
                 if (pass == 0 && (c.bm != tl_hint_bm || c.bn != tl_hint_bn)) continue;
+                if (c.split > slices) continue;
                 if (!candidate_ok(cfg, p, c)) continue;
                 const double cost = model_cost(cfg, p, c);
                 if (cost < best_cost) { best_cost = cost; best = c; }
@@ -1288,13 +1299,22 @@ static void w8a32_layout(const onhip_conv_desc_t *d, int *cp, int *k_units, size
     *q_bytes = ((size_t) d->n * d->h * d->w * *cp + 255) / 256 * 256;
 }
 
+// Partial sums of the layers with few tiles and a K that can be cut (model_cost): up to 512 workgroups of 64 x 64, so at most 8 MiB.
+static size_t w8a32_slices_bytes(const onhip_conv_desc_t *d, int k_units) {
+    int32_t OH, OW;
+    if (d->out_s8 || check_conv(d, &OH, &OW)) return 0;
+    const long long n = (long long) d->n * OH * OW, tiles = (d->cout + 63LL) / 64 * ((n + 63) / 64);
+    const long long slices = std::min(std::min(512 / tiles, 16LL), (long long) (k_units + 3) / 4 / 2);
+    return slices > 1 ? (size_t) (slices * d->cout * n * 4) : 0;
+}
+
 size_t onhip_conv2d_w8a32_workspace(const onhip_conv_desc_t *d) {
     if (!d) return 0;
     int cp, ku;
     size_t pb, qb;
     w8a32_layout(d, &cp, &ku, &pb, &qb);
     // depthwise: only the form with fp32 activations in and an int8 NHWC result out stages anything (the quantised input)
-    return d->group != 1 ? qb : pb + qb;
+    return d->group != 1 ? qb : pb + qb + w8a32_slices_bytes(d, ku);
 }
 
 size_t onhip_conv2d_w8a32_packed_weight_bytes(const onhip_conv_desc_t *d) {
@@ -1496,6 +1516,10 @@ static int conv2d_w8a32_impl(const onhip_conv_desc_t *d, const float *x, const i
     p.acc_out = acc32;
     p.out_s8 = d->out_s8;
     p.out_inv_scale = d->out_s8 ? 1.0f / d->output_scale : 0.0f;
+    if (packed_bytes + q_bytes > 0) {   // a call that takes its workspace has what is left of it as well
+        p.slices = reinterpret_cast<float *>(reinterpret_cast<char *>(workspace) + packed_bytes + q_bytes);
+        p.slices_bytes = (long long) (workspace_bytes - packed_bytes - q_bytes);
+    }
     if (nhwc_out && ep.act == SILU && ep.lut && !acc32) {   // the staged int8 store: gather quantised table entries
         rc = quantised_table(ep.lut, p.out_inv_scale, st, &p.ep.qlut);
         if (rc) return rc;

@@ -245,6 +245,9 @@ struct IgemmProblem : IgemmParams {
     const float *w_src;
     long long w_row, w_k;
     const struct SplitKeeper *keeper;   // who keeps it from call to call, or nullptr: made on each call
+    // room for partial sums of K slices in the caller's own workspace, or none
+    float *slices;
+    long long slices_bytes;
     int ldb;                   // B given as rows (BL_ROWS): elements between them
 };
 
