@@ -794,15 +794,15 @@ static int launch_choice(IgemmLaunch cfg, IgemmProblem p, const Choice &c, hipSt
     return launch();
 }
 
-static int time_choice(IgemmLaunch cfg, IgemmProblem p, const Choice &c, hipStream_t st, hipEvent_t e0, hipEvent_t e1,
-                       float *best_ms) {
-    int rc = launch_choice(cfg, p, c, st);   // warm-up
+template <class F>
+static int time_choice(const F &launch, const Choice &c, hipStream_t st, hipEvent_t e0, hipEvent_t e1, float *best_ms) {
+    int rc = launch(c);   // warm-up
     if (rc) return rc;
     float best = 1e30f;
     for (int rep = 0; rep < 2; ++rep) {
         ONHIP_CHECK_HIP(hipEventRecord(e0, st));
         for (int i = 0; i < 3; ++i) {
-            rc = launch_choice(cfg, p, c, st);
+            rc = launch(c);
             if (rc) return rc;
         }
         ONHIP_CHECK_HIP(hipEventRecord(e1, st));
@@ -815,8 +815,23 @@ static int time_choice(IgemmLaunch cfg, IgemmProblem p, const Choice &c, hipStre
     return ONHIP_OK;
 }
 
+// A product's other form, for the fp32 kernel on the 16-bit matrix cores (rowb == 2 in a choice), and what the cost model says of both.
+struct RowsForm {
+    IgemmLaunch cfg;
+    IgemmProblem p;
+    Choice rows, plain;
+    bool faster;   // rows expected to be
+};
+
 // Chooses tile, split and tail handling for the problem and launches it.
-static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t st) {
+static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t st, const RowsForm *other = nullptr) {
+    auto launch = [&](const Choice &c) {
+        if (!other || c.rowb != 2) return launch_choice(cfg, p, c, st);
+        const int rc = launch_choice(other->cfg, other->p, c, st);
+        return rc == kNoSplitSlot ? launch_choice(cfg, p, slotless_choice(cfg, p, st), st) : rc;
+    };
+    auto ok = [&](const Choice &c) { return other && c.rowb == 2 ? candidate_ok(other->cfg, other->p, c) : candidate_ok(cfg, p, c); };
+    auto by_model = [&]() { return !other ? model_choice(cfg, p) : other->faster ? other->rows : other->plain; };
     // the entry point that allocates nothing: the cost model's choice (never the in-launch reduction, whose uncached
     // workspace is allocated on first use; no measuring, which creates events and may grow buffers)
     if (tl_noalloc) return launch_choice(cfg, p, model_choice(cfg, p), st);
@@ -842,7 +857,7 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
             return launch_choice(cfg, p, c, st);
         }
     }
-    if (!tune_mode()) return launch_choice(cfg, p, model_choice(cfg, p), st);
+    if (!tune_mode()) return launch(by_model());
     std::vector<long long> key = {cfg.dtype, cfg.bl, cfg.batch, p.M, p.N, p.K, p.k_units, p.khkw, p.sh, p.sw,
                                   p.H, p.W, p.out_mode + (p.res ? 16 : 0), p.lda};   // a residual operand narrows the kernels
     {
@@ -851,9 +866,9 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
         auto it = g_tuned.find(key);
         if (it != g_tuned.end()) {
             const Choice c = it->second;
-            if (candidate_ok(cfg, p, c)) {
+            if (ok(c)) {
                 lock.unlock();
-                return launch_choice(cfg, p, c, st);
+                return launch(c);
             }
             g_tuned.erase(it);   // a line of the cache file that this build would not have written: measure again
         }
@@ -861,9 +876,9 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
     // measure: the candidates the model ranks within 2.5x of its best, on the caller's stream
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
-        return launch_choice(cfg, p, model_choice(cfg, p), st);
-    const Choice guess = model_choice(cfg, p);
-    const double guess_cost = model_cost(cfg, p, guess);
+        return launch(by_model());
+    const Choice guess = by_model();
+    const double guess_cost = model_cost(cfg, p, other ? other->plain : guess);
     hipEvent_t e0, e1;
     ONHIP_CHECK_HIP(hipEventCreate(&e0));
     ONHIP_CHECK_HIP(hipEventCreate(&e1));
@@ -873,7 +888,7 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
     // The model's own choice is measured first (it need not be among the candidates below), and another one takes its
     // place only by beating it by 2 %: the measurements repeat within about 3 %, and without the margin a launch that is
     // no faster replaces the model's on a coin toss (seen as a tuned stack slower than the untuned one).
-    rc = time_choice(cfg, p, guess, st, e0, e1, &guess_ms);
+    rc = time_choice(launch, guess, st, e0, e1, &guess_ms);
     best_ms = guess_ms;
     auto same = [](const Choice &a, const Choice &b) {
         return a.bm == b.bm && a.bn == b.bn && a.split == b.split && a.tail == b.tail && a.rowb == b.rowb && a.fin == b.fin && a.dma == b.dma;
@@ -881,7 +896,7 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
     auto try_choice = [&](const Choice &c) {
         if (same(c, guess)) return;
         float ms = 0.f;
-        rc = time_choice(cfg, p, c, st, e0, e1, &ms);
+        rc = time_choice(launch, c, st, e0, e1, &ms);
         if (!rc && ms < best_ms && ms < 0.98f * guess_ms) { best_ms = ms; best = c; }
     };
     for (int t = 0; t < kNumTiles && !rc; ++t) {
@@ -927,7 +942,12 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
     // the fp32 kernel on the 16-bit matrix cores: every tile, with the model's K split and without
     Choice f3;
     double f3_us;
-    if (!rc && f3_ok(cfg, p) && f3_choice(cfg, p, &f3, &f3_us))
+    if (other) {
+        for (int t = 0; t < kNumF3Tiles && !rc; ++t) {
+            const Choice c = {kF3Tiles[t][0], kF3Tiles[t][1], 1, 0, 2, 0, 0};
+            if (ok(c)) try_choice(c);
+        }
+    } else if (!rc && f3_ok(cfg, p) && f3_choice(cfg, p, &f3, &f3_us))
         for (int t = 0; t < kNumF3Tiles && !rc; ++t) {
             const Choice c = {kF3Tiles[t][0], kF3Tiles[t][1], f3.split, 0, 2, 0, 0};
             if (candidate_ok(cfg, p, c)) try_choice(c);
@@ -952,7 +972,7 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
         g_tuned[key] = best;
         append_tune_cache_locked(key, best);
     }
-    return launch_choice(cfg, p, best, st);
+    return launch(best);
 }
 
 static int dtype_of_compute(int compute, int *dt) {
@@ -1674,19 +1694,17 @@ static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float
     }
     p.res = addend;   // laid out like the result; added after the bias, as the Add operator after it would
     if (cfg.dtype == DT_F32 && batch == 1 && !getenv("ONHIP_TILE")) {
-        IgemmLaunch rcfg;
-        IgemmProblem rp;
-        matmul_rows_problem(d, a, b, bias, gelu_lut, addend, out, &rcfg, &rp);
-        Choice c;
+        RowsForm form;
+        matmul_rows_problem(d, a, b, bias, gelu_lut, addend, out, &form.cfg, &form.p);
         double us;
         // rule as in model_choice; the pass that splits the weights is priced in even where the caller keeps them split, so that
         // a product runs the same way, with the same bits, whether its right operand is a model's weight or not
-        if (rp.M > 32 && rp.K >= 48 && p.b_slice_bytes < (1LL << 31) && rp.b_slice_bytes < (1LL << 31) && rp.c_slice_bytes < (1LL << 31) &&
-            f3_choice(rcfg, rp, &c, &us) && us < f32_us(model_cost(cfg, p, model_choice(cfg, p)))) {
-            rp.keeper = keeper;
-            const int rc = launch_choice(rcfg, rp, c, st);
-            if (rc != kNoSplitSlot) return rc;
-            if (under_capture(st)) return launch_choice(cfg, p, slotless_choice(cfg, p, st), st);
+        if (form.p.M > 32 && form.p.K >= 48 && p.b_slice_bytes < (1LL << 31) && form.p.b_slice_bytes < (1LL << 31) &&
+            form.p.c_slice_bytes < (1LL << 31) && f3_choice(form.cfg, form.p, &form.rows, &us)) {
+            form.plain = model_choice(cfg, p);
+            form.faster = !tl_hint_bm && us < f32_us(model_cost(cfg, p, form.plain));   // a hint is for the plain form's tile
+            form.p.keeper = keeper;
+            return plan_and_launch(cfg, p, st, &form);
         }
     }
     return plan_and_launch(cfg, p, st);

@@ -92,6 +92,62 @@ def test_product(m, k, n, special, torch_dev):
     check(y, (a.double() @ b.double() + bias.double()).cpu(), (a.double().abs() @ b.double().abs() + bias.double().abs()).cpu(), k)
 
 
+def test_product_under_a_tile_hint(torch_dev):
+    """a hint restricts the choice to its tile, which this kernel's choice is not"""
+    torch = torch_dev
+    print("f3 product under a tile hint", flush=True)
+    a, b = torch.randn(8195, 773, device="cuda"), torch.randn(773, 1030, device="cuda")
+    lib = hip.load()
+    assert lib.onhip_set_tile_hint(64, 128) == 1
+    try:
+        y = hip.matmul(a, b)
+        assert hip.last_launch_choice()[:2] == (64, 128) and hip.last_launch_choice()[4] != 2
+    finally:
+        assert lib.onhip_set_tile_hint(0, 0) == 0
+    hip.matmul(a, b)
+    assert hip.last_launch_choice()[4] == 2
+    check(y, (a.double() @ b.double()).cpu(), (a.double().abs() @ b.double().abs()).cpu(), 773)
+
+
+MEASURED = """
+import sys, torch
+sys.path.insert(0, sys.argv[1])
+from onenew_amd import hip
+hip.init(0)
+a, b = torch.randn(8195, 773, device="cuda"), torch.randn(773, 1030, device="cuda")
+y = hip.matmul(a, b)
+ref, scale = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+print("RAN", *hip.last_launch_choice(), float(((y.double() - ref).abs() / scale).max()))
+"""
+
+
+def test_product_measured(tmp_path):
+    """with measured choices the product's launches of both forms are timed, the winner is kept, and a kept choice is obeyed"""
+    import os
+    import subprocess
+    import sys
+    root, cache = os.path.dirname(os.path.dirname(os.path.abspath(__file__))), tmp_path / "tune.txt"
+    env = {k: v for k, v in os.environ.items() if k != "ONHIP_TILE"}
+    env.update(ONHIP_TUNE="1", ONHIP_TUNE_CACHE=str(cache))
+
+    def ran():
+        print("f3 product measured", flush=True)
+        out = subprocess.run([sys.executable, "-c", MEASURED, root], env=env, capture_output=True, text=True, timeout=100)
+        assert out.returncode == 0, out.stderr[-2000:]
+        *choice, err = [line for line in out.stdout.splitlines() if line.startswith("RAN")][0].split()[1:]
+        assert float(err) <= (773 + 4) * 2.0 ** -24 + 2.0 ** -23
+        return [int(v) for v in choice]
+
+    ran()
+    lines = cache.read_text().splitlines()
+    assert len(lines) == 1
+    for choice in ("128 128 1 0 0 0 0", "192 64 1 0 2 0 0"):
+        cache.write_text(lines[0].split(":")[0] + ": " + choice + "\n")
+        got = ran()
+        assert [got[0], got[1], got[4]] == [int(v) for v in (choice.split()[0], choice.split()[1], choice.split()[4])]
+        assert len(cache.read_text().splitlines()) == 1
+
+
 def test_streams_and_threads(torch_dev):
     """weights split on the call: more streams than there are slots for them, one after another, and two threads on one stream"""
     torch = torch_dev
