@@ -859,7 +859,9 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
     }
     if (!tune_mode()) return launch(by_model());
     std::vector<long long> key = {cfg.dtype, cfg.bl, cfg.batch, p.M, p.N, p.K, p.k_units, p.khkw, p.sh, p.sw,
-                                  p.H, p.W, p.out_mode + (p.res ? 16 : 0), p.lda};   // a residual operand narrows the kernels
+                                  p.H, p.W, p.out_mode, p.lda};
+    if (p.res) key[12] += 16;   // a residual operand narrows the kernels
+    if (other ? other->p.keeper : p.keeper) key[12] += 32;   // weights kept split: no pass to pay for, and none too large
     {
         std::unique_lock<std::mutex> lock(g_tune_mu);
         load_tune_cache_locked();

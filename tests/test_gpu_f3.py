@@ -121,19 +121,26 @@ print("RAN", *hip.last_launch_choice(), float(((y.double() - ref).abs() / scale)
 """
 
 
-def test_product_measured(tmp_path):
-    """with measured choices the product's launches of both forms are timed, the winner is kept, and a kept choice is obeyed"""
+def measuring(program, cache):
+    """a process of its own, as measured choices are kept for the life of one"""
     import os
     import subprocess
     import sys
-    root, cache = os.path.dirname(os.path.dirname(os.path.abspath(__file__))), tmp_path / "tune.txt"
+    print("f3 measured choices", flush=True)
     env = {k: v for k, v in os.environ.items() if k != "ONHIP_TILE"}
     env.update(ONHIP_TUNE="1", ONHIP_TUNE_CACHE=str(cache))
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-c", program, root], env=env, capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0, out.stderr[-2000:]
+    return out
+
+
+def test_product_measured(tmp_path):
+    """with measured choices the product's launches of both forms are timed, the winner is kept, and a kept choice is obeyed"""
+    cache = tmp_path / "tune.txt"
 
     def ran():
-        print("f3 product measured", flush=True)
-        out = subprocess.run([sys.executable, "-c", MEASURED, root], env=env, capture_output=True, text=True, timeout=100)
-        assert out.returncode == 0, out.stderr[-2000:]
+        out = measuring(MEASURED, cache)
         *choice, err = [line for line in out.stdout.splitlines() if line.startswith("RAN")][0].split()[1:]
         assert float(err) <= (773 + 4) * 2.0 ** -24 + 2.0 ** -23
         return [int(v) for v in choice]
@@ -146,6 +153,25 @@ def test_product_measured(tmp_path):
         got = ran()
         assert [got[0], got[1], got[4]] == [int(v) for v in (choice.split()[0], choice.split()[1], choice.split()[4])]
         assert len(cache.read_text().splitlines()) == 1
+
+
+KEPT = """
+import sys, numpy as np, torch
+sys.path.insert(0, sys.argv[1])
+from onenew_amd import hip, ops
+hip.init(0)
+d = ops.ConvDesc(n=4, cin=256, h=20, w=20, cout=128, kh=1, kw=1, stride_h=1, stride_w=1, group=1, has_bias=1)
+x, w, b = (np.random.default_rng(0).standard_normal(s, dtype=np.float32) for s in ((4, 256, 20, 20), (128, 256, 1, 1), (128,)))
+hip.conv2d_f32(d, *(torch.from_numpy(t).cuda() for t in (x, w, b)))
+ops.Conv(ops.Plugin(hip.plugin_path("Conv")).eval, d, w, b)(x)
+"""
+
+
+def test_kept_weights_are_measured_apart(tmp_path):
+    """a layer whose weights are kept split and one that splits them on the call do not share a measured choice"""
+    measuring(KEPT, tmp_path / "tune.txt")
+    keys = {line.split(":")[0] for line in (tmp_path / "tune.txt").read_text().splitlines()}
+    assert len(keys) == 2, keys
 
 
 def test_streams_and_threads(torch_dev):
