@@ -601,7 +601,9 @@ static bool f3_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out
             if (c.bm > 64 && p.M <= c.bm / 2) continue;
             if (c.split > 1 && cfg.bl == BL_ROWS) continue;
             if (!candidate_ok(cfg, p, c)) continue;
-            if (tl_noalloc && c.split > 1 && 4LL * c.split * p.M * p.N + split_weights_bytes(p.M, p.K) > (long long) kNoAllocScratchBytes) continue;
+            // (with the weights split on the call: cut no finer than the entry point that allocates nothing has room for, an image
+            // at a time, so that it runs what this one does)
+            if (!p.keeper && c.split > 1 && 4LL * c.split * p.M * p.OHW + split_weights_bytes(p.M, p.K) > (long long) kNoAllocScratchBytes) continue;
             const int k_tiles = (p.k_units + 3) / 4, per = (k_tiles + c.split - 1) / c.split;
             const double tiles = (double) ((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn);
             double t_us = 4.2 + ceil(tiles * c.split / 256.0) * (per * per_k_tile[t] + per_tile[t]);
@@ -717,7 +719,7 @@ static int launch_choice(IgemmLaunch cfg, IgemmProblem p, const Choice &c, hipSt
         SplitSlot *slot; hipStream_t st;
         ~Use() { if (slot) slot_used(slot, st); }
     } use{nullptr, st};
-    if (c.rowb == 2) {
+    if (c.rowb == 2 && !p.a_split) {
         const void *kept = nullptr;
         p.a_split_bytes = split_weights_bytes(p.M, p.K);
         if (p.keeper) {
@@ -745,6 +747,23 @@ static int launch_choice(IgemmLaunch cfg, IgemmProblem p, const Choice &c, hipSt
             kept = ws;
         }
         p.a_split = kept;
+        // partial sums that do not fit next to the weights: some images at a time (f3_choice: at least one), the same sums
+        const long long room = (long long) kNoAllocScratchBytes - p.a_split_bytes, image = 4LL * c.split * p.M * p.OHW;
+        if (tl_noalloc && c.split > 1 && image * (p.N / p.OHW) > room) {
+            const int images = p.N / p.OHW, step = (int) (room / image);
+            for (int i = 0; i < images; i += step) {
+                IgemmProblem part = p;
+                const int count = images - i < step ? images - i : step;
+                part.N = count * p.OHW;
+                part.B = static_cast<const float *>(p.B) + i * p.b_img_stride;
+                part.C = static_cast<float *>(p.C) + i * p.c_img_stride;
+                part.b_slice_bytes = count * p.b_img_stride * 4;
+                part.c_slice_bytes = count * p.c_img_stride * 4;
+                const int rc = launch_choice(cfg, part, c, st);
+                if (rc) return rc;
+            }
+            return ONHIP_OK;
+        }
     }
     int dpc = 0, left = 0;
     p.part_begin = p.dp_tiles = p.tail_tiles = 0;

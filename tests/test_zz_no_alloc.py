@@ -69,3 +69,27 @@ def test_no_alloc_entry_point_matches_the_allocating_one():
         assert float(out.abs().max()) == 0.0
     finally:
         hip.set_tuning(prev)
+
+
+def test_partial_sums_next_to_split_weights():
+    """weights split on the call leave less of the built-in array than the partial sums of all images take (5 x 6.4 MB beside 14 MB):
+    the call makes them some images at a time, with the bits of the entry point it mirrors"""
+    import torch
+    hip.init(0)
+    prev = hip.set_tuning(0)
+    try:
+        d = _desc(16, 512, 14, 512, 3, 1)
+        print("no-alloc case next to split weights", flush=True)
+        x, w, b = _inputs(torch, "next_to_weights", d)
+        wp = hip.pack_conv_weights(d, w)
+        ref = hip.conv2d_f32(d, x, wp, b, packed=True)
+        choice = hip.last_launch_choice()
+        assert choice[4] == 2 and choice[2] * ref.numel() * 4 + 512 * 9 * 512 * 6 > 32 << 20
+        out = torch.full_like(ref, float("nan"))
+        used = hip.load().onhip_noalloc_scratch_launches()
+        hip.conv2d_f32_noalloc(d, x, wp, out, b, packed=True)
+        torch.cuda.synchronize()
+        assert hip.last_launch_choice() == choice and hip.load().onhip_noalloc_scratch_launches() > used + 1
+        assert torch.equal(out, ref)
+    finally:
+        hip.set_tuning(prev)
