@@ -10,7 +10,7 @@
 // error over sum |a b| within 15 % of it either way; the nine products give the same errors as the six.
 // What differs from an fp32 multiply: magnitudes below 2^-111 lose low bits (their l falls below bf16's subnormals), and an
 // infinity or a NaN, or an activation that rounds to a bf16 infinity, has no finite parts and makes the sum NaN.  A wavefront
-// that holds a non-finite sum when its K loop is over computes those elements again with fp32 multiply-adds (fix_nonfinite),
+// that holds a non-finite sum when its K loop is over computes its tile again with fp32 matrix instructions (fix_nonfinite),
 // so infinities and overflow come out as they do in fp32 arithmetic.
 //
 // Why: v_mfma_f32_32x32x16_bf16 does the multiply-adds of eight v_mfma_f32_32x32x2_f32 in a sixteenth of their time.  On
@@ -116,11 +116,25 @@ __device__ __forceinline__ unsigned f3_voff(const ColState &c, unsigned tap) {
     return (c.pixoff & keep) | (OOB & ~keep);
 }
 
-// Sums that are not finite, computed again in fp32: see the head of the file.  scratch: 32 x 33 floats of LDS private to the
-// wavefront.  Units u_begin .. of the reduction up to klim elements; operands through the K loop's own loads.
+// Byte offset of element (k, column) of B for fix_nonfinite, where k differs between lanes; OOB beyond the column's taps.
+template <int BL>
+__device__ __forceinline__ unsigned f3_element(const IgemmProblem &p, const ColState &c, unsigned k) {
+    if constexpr (BL == BL_ROWS) return c.pixoff == OOB ? OOB : c.pixoff + k * 4u;
+    if constexpr (BL == BL_PLAIN) return c.pixoff == OOB ? OOB : c.pixoff + k * (unsigned) p.HW * 4u;
+    const F3Prep q = BL == BL_GATHER ? f3_prep<BL_GATHER>(p, (int) (k / 4), (int) (k % 4)) : f3_prep<BL_TAPC>(p, (int) (k / 4), 0);
+    const unsigned at = f3_voff<BL>(c, q.tap);
+    return at == OOB ? OOB : at + q.soff + (BL == BL_TAPC ? (k % 4) * (unsigned) p.HW * 4u : 0u);
+}
+
+// Sums that are not finite, computed again in fp32 (see the head of the file): a wavefront that holds one multiplies its whole tile
+// again with v_mfma_f32_32x32x2_f32, operands straight from memory, and takes the elements that were not finite from there.
+// Sixteen of K a step, 8 (lane / 32) + j in MFMA j.  Units u_begin .. of the reduction up to klim elements.
+// A product of 4099 x 1031 x 2053 takes 0.127 ms, with a NaN in one row of the left operand 0.23, all of it NaN 0.54; a 3x3 convolution
+// 256 -> 256 over 32 x 14 x 14 0.075, and 0.22 with a NaN in one plane of each image.  (One element a lane and multiply-add: 4.6 and
+// 15 ms, 2.7 ms.)
 template <int BL, int TM, int TN>
-__device__ __forceinline__ void fix_nonfinite(const IgemmProblem &p, f32x16 (&acc)[TM][TN], float *scratch, rsrc_t ra, rsrc_t rb, int m_wave,
-                                              int n_wave, int lane, int u_begin, int klim) {
+__device__ __forceinline__ void fix_nonfinite(const IgemmProblem &p, f32x16 (&acc)[TM][TN], rsrc_t ra, rsrc_t rb, int m_wave, int n_wave, int lane,
+                                              int u_begin, int klim) {
     float probe = 0.0f;   // stays zero while every sum is finite: 0 * inf and 0 * NaN are NaN
 #pragma unroll
     for (int a = 0; a < TM; ++a)
@@ -130,51 +144,47 @@ __device__ __forceinline__ void fix_nonfinite(const IgemmProblem &p, f32x16 (&ac
             for (int r = 0; r < 16; ++r) probe = __builtin_fmaf(acc[a][b][r], 0.0f, probe);
     if (__builtin_amdgcn_ballot_w64(probe != probe) == 0ull) return;
     const int li = lane & 31, lh = lane >> 5;
+    ColState col[TN];
 #pragma unroll
-    for (int a = 0; a < TM; ++a)
+    for (int b = 0; b < TN; ++b) col[b] = f3_col<BL>(p, n_wave + b * 32 + li);
+    // a row block at a time: no more registers than the K loop has given up
 #pragma unroll
-        for (int b = 0; b < TN; ++b) {
+    for (int a = 0; a < TM; ++a) {
+        f32x16 s[TN];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) scratch[(8 * (r / 4) + 4 * lh + r % 4) * 33 + li] = acc[a][b][r];
-            __builtin_amdgcn_wave_barrier();
+        for (int b = 0; b < TN; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[b][r] = 0.0f;
+        const unsigned a_row = (unsigned) (m_wave / 32 + a) * (unsigned) ((p.K + 15) / 16) * 3072u;
 #pragma unroll 1
-            for (int e = 0; e < 16; ++e) {   // two rows of the block at a time: lane -> row 2 e + lh, column li
-                float *cell = scratch + (2 * e + lh) * 33 + li;
-                const int m = m_wave + a * 32 + 2 * e + lh, n = n_wave + b * 32 + li;
-                const float v = *cell;
-                const bool bad = v * 0.0f != 0.0f && m < p.M && n < p.N;
-                if (__builtin_amdgcn_ballot_w64(bad) == 0ull) continue;
-                const ColState col = f3_col<BL>(p, n);
-                float s = 0.0f;
-#pragma unroll 1
-                for (int u = u_begin; u * 4 < klim; ++u)
+        for (int k0 = u_begin * 4; k0 < klim; k0 += 16) {
+            uint4 part[3];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int k = u * 4 + j;
-                        float bv;
-                        if constexpr (BL == BL_ROWS) {
-                            bv = buf_load_f32(rb, (unsigned) (n * p.ldb) * 4u, (unsigned) k * 4u);
-                        } else {
-                            const BPrep q = prep_b<DT_F32, BL>(p, u, BL == BL_TAPC ? 0 : j, klim);
-                            const unsigned voff = b_voff<BL>(p, col, q, BL == BL_GATHER ? k : u);
-                            bv = buf_load_f32(rb, voff, q.soff + (BL == BL_TAPC ? (unsigned) j * (unsigned) p.HW * 4u : 0u));
-                        }
-                        const unsigned row = bad ? (unsigned) (m / 32) * (unsigned) ((p.K + 15) / 16) * 3072u + (unsigned) (m % 32) * 16u : OOB;
-                        const unsigned at = (unsigned) (k / 16) * 3072u + (unsigned) (k % 16 / 8) * 512u + (unsigned) (k % 8) * 2u;
-                        auto part = [&](unsigned z) __attribute__((always_inline)) {
-                            return __uint_as_float((unsigned) (unsigned short) __builtin_amdgcn_raw_buffer_load_b16(ra, row, at + z * 1024u, 0) << 16);
-                        };
-                        const float av = (part(0) + part(1)) + part(2);   // the parts add up to the weight exactly
-                        const float t = __builtin_fmaf(av, bv, s);
-                        s = k < klim ? t : s;
-                    }
-                if (bad) *cell = s;
+            for (int z = 0; z < 3; ++z) part[z] = buf_load_b128(ra, (unsigned) lane * 16u, a_row + (unsigned) (k0 / 16) * 3072u + z * 1024u);
+            float bv[TN][8];
+#pragma unroll
+            for (int b = 0; b < TN; ++b)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int k = k0 + 8 * lh + j;
+                    bv[b][j] = buf_load_f32(rb, k < klim ? f3_element<BL>(p, col[b], (unsigned) k) : OOB, 0);
+                }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                auto up = [&](const uint4 &q) __attribute__((always_inline)) {
+                    const unsigned w = j / 2 == 0 ? q.x : j / 2 == 1 ? q.y : j / 2 == 2 ? q.z : q.w;
+                    return __uint_as_float(j % 2 ? w & 0xffff0000u : w << 16);
+                };
+                const float av = (up(part[0]) + up(part[1])) + up(part[2]);   // the parts add up to the weight exactly
+#pragma unroll
+                for (int b = 0; b < TN; ++b) s[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv[b][j], s[b], 0, 0, 0);
             }
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[a][b][r] = scratch[(8 * (r / 4) + 4 * lh + r % 4) * 33 + li];
-            __builtin_amdgcn_wave_barrier();
         }
+#pragma unroll
+        for (int b = 0; b < TN; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[a][b][r] = acc[a][b][r] * 0.0f != 0.0f ? s[b][r] : acc[a][b][r];
+    }
 }
 
 // The store for B given as rows (a product's left operand): C is row-major with the tile's columns as its rows, so the four
@@ -227,8 +237,8 @@ void igemm_f3_kernel(const IgemmProblem p) {
     constexpr int UPT = 4, NT = 64 * WM * WN;
     static_assert(BN * UPT == NT, "a thread stages one unit of B per K tile");
     constexpr int LD = BL == BL_ROWS ? BN + 1 : BN;   // 16-byte slots per 8 elements of K; rows arrive from neighbouring lanes
-    constexpr int PLANE = 2 * LD, SLOTS = 3 * PLANE, FIX_SLOTS = (WM * WN * 32 * 33 * 4 + 15) / 16;   // fix_nonfinite's scratch fits as well
-    __shared__ uint4 lds[2 * SLOTS > FIX_SLOTS ? 2 * SLOTS : FIX_SLOTS];   // two K tiles
+    constexpr int PLANE = 2 * LD, SLOTS = 3 * PLANE;
+    __shared__ uint4 lds[2 * SLOTS];   // two K tiles
     __shared__ __attribute__((aligned(16))) float s_bias[BM];
 
     const int tid = threadIdx.x;
@@ -392,8 +402,7 @@ void igemm_f3_kernel(const IgemmProblem p) {
     __syncthreads();
 
     const int m_wave = m0 + wm * (BM / WM), n_wave = n0 + wn * (BN / WN);
-    fix_nonfinite<BL, TM, TN>(p, acc, reinterpret_cast<float *>(lds) + wave * (32 * 33), ra, make_rsrc(b_base, b_bytes), m_wave, n_wave, lane, u_begin,
-                              klim);
+    fix_nonfinite<BL, TM, TN>(p, acc, ra, make_rsrc(b_base, b_bytes), m_wave, n_wave, lane, u_begin, klim);
     if (p.partial && !whole_k) {
         if (!p.arrive) {   // a finishing launch adds the slices up
             write_partial<TM, TN, false>(p, acc, slice * gridDim.z + batch, m_wave, n_wave, li, lh);
