@@ -489,7 +489,7 @@ static bool candidate_ok(const IgemmLaunch &cfg, const IgemmProblem &p, const Ch
         return (!off || h16) && c.split == 1 && c.tail <= 1 && !c.rowb && !c.fin && dma_ok(cfg, p);
     }
     if (h16) return false;
-    if (c.rowb == 2 && !f3_ok(cfg, p)) return false;
+    if (c.rowb == 2 && (c.tail > 1 || c.fin || (c.split > 1 && cfg.bl == BL_ROWS) || !f3_ok(cfg, p))) return false;   // whole tiles, or slices and a finishing launch
     if (c.rowb == 1 && (c.split != 1 || !rowb_f32_ok(cfg, p))) return false;
     if (c.fin) {
         static const bool off = getenv("ONHIP_NO_FIN") != nullptr;   // tuning hook: finishing launches only
@@ -599,7 +599,6 @@ static bool f3_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out
         for (int s = 0; s < kNumSplits; ++s) {
             const Choice c = {kF3Tiles[t][0], kF3Tiles[t][1], kSplits[s], 0, 2, 0, 0};
             if (c.bm > 64 && p.M <= c.bm / 2) continue;
-            if (c.split > 1 && cfg.bl == BL_ROWS) continue;
             if (!candidate_ok(cfg, p, c)) continue;
             // (with the weights split on the call: cut no finer than the entry point that allocates nothing has room for, an image
             // at a time, so that it runs what this one does)
@@ -866,6 +865,7 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
                 if (c.bm == 128 && c.bn == 64) c.bm = 64;
             }
             if (c.fin && !candidate_ok(cfg, p, c)) c.fin = 0;
+            if (c.rowb == 2 && c.tail > 1) c.tail = 0;
             if (c.rowb == 2 && !candidate_ok(cfg, p, c)) { c = {64, 64, 1, 0, 0, 0, 0}; }
             if (c.rowb && !candidate_ok(cfg, p, c)) {   // not a problem for that kernel: the tiled one, same tile if it has it
                 c.rowb = 0;

@@ -7,7 +7,7 @@ int f3_launch_tapc(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t st
 int f3_launch_gather(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t stream);
 
 int f3_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t stream) {
-    if (p.M < 1 || p.N < 1 || p.K < 1 || cfg.batch != 1 || cfg.split < 1 || !p.a_split || p.a_split_bytes >= (1LL << 31) ||
+    if (p.M < 1 || p.N < 1 || p.K < 1 || cfg.batch != 1 || cfg.split < 1 || p.dp_tiles || p.arrive || !p.a_split || p.a_split_bytes >= (1LL << 31) ||
         p.b_slice_bytes + 2 * p.b_shift_bytes >= (1LL << 31) || p.c_slice_bytes >= (1LL << 31))
         return set_error(ONHIP_ERR_ARG, "igemm f3: not a problem of this kernel");
     switch (cfg.bl) {

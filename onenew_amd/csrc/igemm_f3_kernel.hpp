@@ -247,15 +247,12 @@ void igemm_f3_kernel(const IgemmProblem p) {
     const int wm = wave / WN, wn = wave % WN;
 
     const TilePlace tp = place_tile<BM, BN>(p);
-    const int m0 = tp.m0, n0 = tp.n0, slice = tp.slice, lid = tp.lid;
-    const bool whole_k = tp.whole_k;
-    const int batch = blockIdx.z;
-    const int u_begin = whole_k ? 0 : slice * p.k_split_units;
-    const int u_end = whole_k ? p.k_units : min(p.k_units, u_begin + p.k_split_units);
+    const int m0 = tp.m0, n0 = tp.n0, slice = tp.slice;
+    const int u_begin = slice * p.k_split_units, u_end = min(p.k_units, u_begin + p.k_split_units);
     const int k_tiles = (u_end - u_begin + UPT - 1) / UPT;
     const int klim = min(p.K, u_end * 4);
 
-    const char *b_base = reinterpret_cast<const char *>(p.B) + (size_t) batch * p.b_batch_stride * 4 - (size_t) p.b_shift_bytes;
+    const char *b_base = reinterpret_cast<const char *>(p.B) - (size_t) p.b_shift_bytes;
     const unsigned b_bytes = (unsigned) (p.b_slice_bytes + p.b_shift_bytes);
 
     // A: [32 rows][16 of K][part][lane][16 bytes], row block, K tile and part in the scalar offset
@@ -403,18 +400,15 @@ void igemm_f3_kernel(const IgemmProblem p) {
 
     const int m_wave = m0 + wm * (BM / WM), n_wave = n0 + wn * (BN / WN);
     fix_nonfinite<BL, TM, TN>(p, acc, ra, make_rsrc(b_base, b_bytes), m_wave, n_wave, lane, u_begin, klim);
-    if (p.partial && !whole_k) {
-        if (!p.arrive) {   // a finishing launch adds the slices up
-            write_partial<TM, TN, false>(p, acc, slice * gridDim.z + batch, m_wave, n_wave, li, lh);
-            return;
-        }
-        if (!reduce_in_launch<TM, TN>(p, acc, slice, batch, lid, m_wave, n_wave, li, lh, tid)) return;
+    if (p.partial) {   // a finishing launch adds the slices up
+        write_partial<TM, TN, false>(p, acc, slice, m_wave, n_wave, li, lh);
+        return;
     }
     const float *sb = s_bias + wm * (BM / WM);
     auto store = [&](auto epi) __attribute__((always_inline)) {
         constexpr int EPI = decltype(epi)::value;
         if constexpr (BL == BL_ROWS) write_tile_rows<EPI, TM, TN, RES>(p, acc, m_wave, n_wave, li, lh, sb);
-        else write_tile<DT_F32, EPI, TM, TN, RES, true>(p, acc, batch, m_wave, n_wave, li, lh, sb);
+        else write_tile<DT_F32, EPI, TM, TN, RES, true>(p, acc, 0, m_wave, n_wave, li, lh, sb);
     };
     switch (p.ep.act) {
         case NOT_ACT:
