@@ -23,8 +23,8 @@ int f3_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t stream)
 
 // ---- weights -> the split form ---------------------------------------------------------------------------------------
 // element (row, k) of the weights at w[row * s_row + k * s_k]; out [32 rows][16 of K][part][lane (row, half of 8)][8 bf16], zeros beyond
-// M rows and K.  A weight that rounds to a bf16 infinity keeps its upper half instead (the rest still fits the other two
-// parts); one that is not finite has no other parts.
+// M rows and K.  A weight that is not finite when scaled has an infinity for its first part, which makes every sum it takes part in
+// infinite or NaN, and its own upper and lower half for the others, from which those sums are computed again.
 __global__ __launch_bounds__(256) void split_weights_kernel(const float *w, int M, int K, long long s_row, long long s_k, int ksteps, uint4 *out,
                                                             long long total) {
     const long long i = (long long) blockIdx.x * blockDim.x + threadIdx.x;
@@ -39,12 +39,11 @@ __global__ __launch_bounds__(256) void split_weights_kernel(const float *w, int 
     unsigned part[3][4];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-        const bool finite = x[j] - x[j] == 0.0f;
-        float h = (float) (__bf16) x[j];
-        if (finite && h - h != 0.0f) h = __uint_as_float(__float_as_uint(x[j]) & 0xffff0000u);
-        const float r = finite ? x[j] - h : 0.0f;
-        const float m = (float) (__bf16) r;
-        const unsigned hml[3] = {__float_as_uint(h) >> 16, __float_as_uint(m) >> 16, __float_as_uint((float) (__bf16) (r - m)) >> 16};
+        const float v = x[j] * F3_SCALE, h = (float) (__bf16) v, r = v - h, m = (float) (__bf16) r;
+        const bool finite = h - h == 0.0f;
+        const unsigned raw = __float_as_uint(x[j]);
+        const unsigned hml[3] = {finite ? __float_as_uint(h) >> 16 : 0x7f80u, finite ? __float_as_uint(m) >> 16 : raw >> 16,
+                                 finite ? __float_as_uint((float) (__bf16) (r - m)) >> 16 : raw & 0xffffu};
 #pragma unroll
         for (int z = 0; z < 3; ++z) part[z][j / 2] = j % 2 ? part[z][j / 2] | hml[z] << 16 : hml[z];
     }

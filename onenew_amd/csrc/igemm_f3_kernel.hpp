@@ -2,16 +2,19 @@
 //
 // Arithmetic.  Every fp32 operand is written as the sum of three bf16 numbers, x = h + m + l: h = bf16(x), m = bf16(x - h),
 // l = x - h - m, each rounded to nearest.  The two differences are exact, and so is the sum: 24 significant bits are three
-// times eight (|m| <= 2^-8 |h|, |l| <= 2^-8 |m|).  bf16 has fp32's exponent range, so no operand needs scaling.  Of the nine
+// times eight (|m| <= 2^-8 |h|, |l| <= 2^-8 |m|).  Of the nine
 // partial products six are formed, each exact in the matrix core and added to the fp32 accumulator: l h, m m, m h, h l, h m,
 // h h.  The three left out, m l, l m and l l, are at most 2^-23 and typically 2^-26 of |a b|, below the rounding that a chain
-// of fp32 multiply-adds makes at every step.  Measured against 64-bit sums over K = 16 ... 4608: relative error 0.46 ... 0.87
-// of v_mfma_f32_32x32x2_f32's on normal operands and on all-positive ones, and on operands spread over 2^+-24 a largest
-// error over sum |a b| within 15 % of it either way; the nine products give the same errors as the six.
-// What differs from an fp32 multiply: magnitudes below 2^-111 lose low bits (their l falls below bf16's subnormals), and an
-// infinity or a NaN, or an activation that rounds to a bf16 infinity, has no finite parts and makes the sum NaN.  A wavefront
-// that holds a non-finite sum when its K loop is over computes its tile again with fp32 matrix instructions (fix_nonfinite),
-// so infinities and overflow come out as they do in fp32 arithmetic.
+// of fp32 multiply-adds makes at every step.  Measured against 64-bit sums over K = 48 ... 4608,
+// root mean square of the error as a share of sum |a b|: 0.73 ... 0.88 of v_mfma_f32_32x32x2_f32's on normal operands, 0.63 ... 0.82 on
+// all-positive ones, 0.77 ... 0.82 on operands spread over 2^+-4; 1.10 ... 1.19 where they spread over 2^+-24 and one term decides a sum.
+// The nine products give the same errors as the six.
+// The parts are those of x 2^24 (F3_SCALE): every fp32 number, subnormals included, is a multiple of 2^-149, so the parts are
+// multiples of 2^-125 and none falls below bf16's smallest normal number (unscaled, an operand below 2^-110 lost low bits: a relative
+// 2^-14 of it at 2^-120, all of it at 2^-134).  The sum is of a 2^24 times b 2^24 and loses 2^48 again when the K loop is over.
+// What differs from an fp32 multiply: an infinity, a NaN and an operand of 2^104 or more have no finite parts, and sums of 2^80
+// or more may overflow on the way; either leaves a sum that is not finite.  A wavefront that holds one when its K loop is over
+// computes its tile again with fp32 matrix instructions (unscale_fix_nonfinite), so all of these come out as they do in fp32 arithmetic.
 //
 // Why: v_mfma_f32_32x32x16_bf16 does the multiply-adds of eight v_mfma_f32_32x32x2_f32 in a sixteenth of their time.  On
 // random operands the card holds its power limit by its clock (1.2 to 1.7 GHz in these loops), so what counts is energy: six
@@ -24,7 +27,7 @@
 //     from memory straight into operand registers, one contiguous KiB per load: no LDS, no vector instruction.  The
 //     wavefronts of a tile lie along M (the 64 x 64, 192 x 64 and 128 x 128 tiles apart), so no two of them load the same rows;
 //   * B is split on its way into LDS, [part][k / 8][column][8 bf16], a unit per thread and K tile, in four phases of four to
-//     six vector instructions each behind an MFMA of its own: 22 vector instructions per 12 to 24 MFMAs and wavefront.
+//     ten vector instructions each behind an MFMA of its own: 26 vector instructions per 12 to 24 MFMAs and wavefront.
 // Per K tile of the 128 x 64 tile a wavefront issues 12 MFMAs, 3 A loads, 4 B loads, 3 LDS stores and 6 LDS reads.
 //
 // Replaces, for the dense fp32 cases with enough work (f3_choice in api.hip): device/x86/Conv/conv.c im2col (:168,:260) +
@@ -40,22 +43,18 @@ template <int N, class F> __device__ __forceinline__ void static_for(F &&f) {
     [&]<int... I>(std::integer_sequence<int, I...>) __attribute__((always_inline)) { (f(std::integral_constant<int, I>{}), ...); }(std::make_integer_sequence<int, N>{});
 }
 
-// two floats -> their three bf16 parts, packed in pairs
+constexpr float F3_SCALE = 0x1p24f, F3_UNSCALE = 0x1p-48f;   // of each operand, and of a sum of their products
+
+// two floats, each rounded to bf16, packed
 __device__ __forceinline__ unsigned cvt_pk_bf16(float a, float b) {
     unsigned d;   // the conversion of a pair; from C the compiler converts some of the values twice
     asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
     return d;
 }
-__device__ __forceinline__ void split_pair(float x0, float x1, unsigned &h, unsigned &m, unsigned &l) {
-    h = cvt_pk_bf16(x0, x1);
-    const float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xffff0000u);
-    m = cvt_pk_bf16(r0, r1);
-    l = cvt_pk_bf16(r0 - __uint_as_float(m << 16), r1 - __uint_as_float(m & 0xffff0000u));
-}
-// A unit of four floats on its way to three parts, in four phases of four to six vector instructions: few enough to issue
-// behind one MFMA while it runs.
+// A unit of four floats on its way to three parts, in four phases of four to ten vector instructions, each behind an MFMA while it
+// runs.
 struct SplitUnit {
-    float r0, r1, r2, r3, u0, u1, u2, u3;
+    float r0, r1, r2, r3, u0, u1, u2, u3;   // what is left to split; the part taken last
     unsigned h0, h1, m0, m1, l0, l1;   // the parts, packed in pairs
     __device__ __forceinline__ void unpack(unsigned a, unsigned b) {
         u0 = __uint_as_float(a << 16); u1 = __uint_as_float(a & 0xffff0000u);
@@ -63,10 +62,11 @@ struct SplitUnit {
     }
     template <int Q> __device__ __forceinline__ void phase(float x0, float x1, float x2, float x3) {
         if constexpr (Q == 0) {
-            h0 = cvt_pk_bf16(x0, x1); h1 = cvt_pk_bf16(x2, x3);
+            r0 = x0 * F3_SCALE; r1 = x1 * F3_SCALE; r2 = x2 * F3_SCALE; r3 = x3 * F3_SCALE;
+            h0 = cvt_pk_bf16(r0, r1); h1 = cvt_pk_bf16(r2, r3);
             unpack(h0, h1);
         } else if constexpr (Q == 1) {
-            r0 = x0 - u0; r1 = x1 - u1; r2 = x2 - u2; r3 = x3 - u3;
+            r0 -= u0; r1 -= u1; r2 -= u2; r3 -= u3;
             m0 = cvt_pk_bf16(r0, r1); m1 = cvt_pk_bf16(r2, r3);
         } else if constexpr (Q == 2) {
             unpack(m0, m1);
@@ -116,7 +116,7 @@ __device__ __forceinline__ unsigned f3_voff(const ColState &c, unsigned tap) {
     return (c.pixoff & keep) | (OOB & ~keep);
 }
 
-// Byte offset of element (k, column) of B for fix_nonfinite, where k differs between lanes; OOB beyond the column's taps.
+// Byte offset of element (k, column) of B for unscale_fix_nonfinite, where k differs between lanes; OOB beyond the column's taps.
 template <int BL>
 __device__ __forceinline__ unsigned f3_element(const IgemmProblem &p, const ColState &c, unsigned k) {
     if constexpr (BL == BL_ROWS) return c.pixoff == OOB ? OOB : c.pixoff + k * 4u;
@@ -126,14 +126,14 @@ __device__ __forceinline__ unsigned f3_element(const IgemmProblem &p, const ColS
     return at == OOB ? OOB : at + q.soff + (BL == BL_TAPC ? (k % 4) * (unsigned) p.HW * 4u : 0u);
 }
 
-// Sums that are not finite, computed again in fp32 (see the head of the file): a wavefront that holds one multiplies its whole tile
+// Sums with the operands' scale taken out, and those that are not finite computed again in fp32 (see the head of the file): a wavefront that holds one multiplies its whole tile
 // again with v_mfma_f32_32x32x2_f32, operands straight from memory, and takes the elements that were not finite from there.
 // Sixteen of K a step, 8 (lane / 32) + j in MFMA j.  Units u_begin .. of the reduction up to klim elements.
 // A product of 4099 x 1031 x 2053 takes 0.127 ms, with a NaN in one row of the left operand 0.23, all of it NaN 0.54; a 3x3 convolution
 // 256 -> 256 over 32 x 14 x 14 0.075, and 0.22 with a NaN in one plane of each image.  (One element a lane and multiply-add: 4.6 and
 // 15 ms, 2.7 ms.)
 template <int BL, int TM, int TN>
-__device__ __forceinline__ void fix_nonfinite(const IgemmProblem &p, f32x16 (&acc)[TM][TN], rsrc_t ra, rsrc_t rb, int m_wave, int n_wave, int lane,
+__device__ __forceinline__ void unscale_fix_nonfinite(const IgemmProblem &p, f32x16 (&acc)[TM][TN], rsrc_t ra, rsrc_t rb, int m_wave, int n_wave, int lane,
                                               int u_begin, int klim) {
     float probe = 0.0f;   // stays zero while every sum is finite: 0 * inf and 0 * NaN are NaN
 #pragma unroll
@@ -142,7 +142,15 @@ __device__ __forceinline__ void fix_nonfinite(const IgemmProblem &p, f32x16 (&ac
         for (int b = 0; b < TN; ++b)
 #pragma unroll
             for (int r = 0; r < 16; ++r) probe = __builtin_fmaf(acc[a][b][r], 0.0f, probe);
-    if (__builtin_amdgcn_ballot_w64(probe != probe) == 0ull) return;
+    if (__builtin_amdgcn_ballot_w64(probe != probe) == 0ull) {
+#pragma unroll
+        for (int a = 0; a < TM; ++a)
+#pragma unroll
+            for (int b = 0; b < TN; ++b)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[a][b][r] *= F3_UNSCALE;
+        return;
+    }
     const int li = lane & 31, lh = lane >> 5;
     ColState col[TN];
 #pragma unroll
@@ -175,7 +183,10 @@ __device__ __forceinline__ void fix_nonfinite(const IgemmProblem &p, f32x16 (&ac
                     const unsigned w = j / 2 == 0 ? q.x : j / 2 == 1 ? q.y : j / 2 == 2 ? q.z : q.w;
                     return __uint_as_float(j % 2 ? w & 0xffff0000u : w << 16);
                 };
-                const float av = (up(part[0]) + up(part[1])) + up(part[2]);   // the parts add up to the weight exactly
+                // the parts add up to the scaled weight exactly, or are a marker and the weight's two halves (split_weights_kernel)
+                const float hi = up(part[0]), mid = up(part[1]), low = up(part[2]);
+                const float whole = __uint_as_float(__float_as_uint(mid) | __float_as_uint(low) >> 16);
+                const float av = hi - hi == 0.0f ? ((hi + mid) + low) * (1.0f / F3_SCALE) : whole;
 #pragma unroll
                 for (int b = 0; b < TN; ++b) s[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv[b][j], s[b], 0, 0, 0);
             }
@@ -183,7 +194,7 @@ __device__ __forceinline__ void fix_nonfinite(const IgemmProblem &p, f32x16 (&ac
 #pragma unroll
         for (int b = 0; b < TN; ++b)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[a][b][r] = acc[a][b][r] * 0.0f != 0.0f ? s[b][r] : acc[a][b][r];
+            for (int r = 0; r < 16; ++r) acc[a][b][r] = acc[a][b][r] * 0.0f != 0.0f ? s[b][r] : acc[a][b][r] * F3_UNSCALE;
     }
 }
 
@@ -388,7 +399,7 @@ void igemm_f3_kernel(const IgemmProblem p) {
     };
     // Two tiles a trip; behind an odd last tile runs one more, whose B is zero.  No test of reduction indices anywhere: beyond
     // K the split weights are zero, and what B brings in there (the next row or image, zeros behind the tensor) is multiplied
-    // by that; should it not be finite, fix_nonfinite sums the elements over K alone.
+    // by that; should it not be finite, unscale_fix_nonfinite sums the elements over K alone.
     for (int kt = 0; kt < k_tiles; kt += 2) {
         body(op0, op1, kt, S1);
         body(op1, op0, kt + 1, S0);
@@ -399,7 +410,7 @@ void igemm_f3_kernel(const IgemmProblem p) {
     __syncthreads();
 
     const int m_wave = m0 + wm * (BM / WM), n_wave = n0 + wn * (BN / WN);
-    fix_nonfinite<BL, TM, TN>(p, acc, ra, make_rsrc(b_base, b_bytes), m_wave, n_wave, lane, u_begin, klim);
+    unscale_fix_nonfinite<BL, TM, TN>(p, acc, ra, make_rsrc(b_base, b_bytes), m_wave, n_wave, lane, u_begin, klim);
     if (p.partial) {   // a finishing launch adds the slices up
         write_partial<TM, TN, false>(p, acc, slice, m_wave, n_wave, li, lh);
         return;

@@ -296,3 +296,66 @@ def test_capture(torch_dev, monkeypatch):
     graphs = [record(jobs[i % 2]) for i in range(33)]
     assert all(c[4] != 2 and c[2] == 1 and c[3] == 0 for c in choices), choices
     replay(graphs[-2:])
+
+
+# exponents of the left and the right operand: low bits below bf16's subnormals, subnormal fp32 numbers, operands and sums that
+# overflow with the operands' scale on them
+RANGES = [(-120, 0), (0, -120), (-66, -58), (-140, 20), (20, -140), (108, -20), (-20, 108), (50, 40)]
+
+
+@pytest.mark.parametrize("form", ["plain", "tapc", "gather", "rows"])
+@pytest.mark.parametrize("ea,eb", RANGES)
+def test_ends_of_the_range(ea, eb, form, torch_dev, monkeypatch):
+    """no operand that fp32 holds loses bits: the bound of a chain of fp32 multiply-adds, each of which may round at 2^-149"""
+    torch = torch_dev
+    print(f"f3 operands of 2^{ea} and 2^{eb}, {form}", flush=True)
+    g = torch.Generator().manual_seed(5)
+    scaled = lambda e, *shape: (torch.randn(shape, generator=g).double() * 2.0 ** e).float().cuda()  # noqa: E731
+    if form == "rows":
+        k = 773
+        a, b = scaled(ea, 8195, k), scaled(eb, k, 1030)
+        y, chosen = hip.matmul(a, b), hip.last_launch_choice()[4]
+        ref, magnitude = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    else:
+        d = conv_desc(2, 36, 13, 11, 70, 1 if form == "plain" else 3, 1, 0)
+        d.has_bias = 0
+        k = d.cin * d.kh * d.kw
+        x, w = scaled(ea, d.n, d.cin, d.h, d.w), scaled(eb, d.cout, d.cin, d.kh, d.kw)
+        monkeypatch.setenv("ONHIP_TILE", "64x64x1x0x2")
+        y = hip.conv2d_f32(d, x, hip.pack_conv_weights(d, w) if form == "tapc" else w, None, packed=form == "tapc")
+        chosen = hip.last_launch_choice()[4]
+        zero = torch.zeros(d.cout)
+        ref, magnitude = conv_ref(torch, d, x, w, zero)
+    assert chosen == 2
+    err, bound = (y.double().cpu() - ref.cpu()).abs(), magnitude.cpu() * ((k + 4) * 2.0 ** -24 + 2.0 ** -23) + k * 2.0 ** -149
+    assert bool((err <= bound).all()), float((err / bound).max())
+
+
+@pytest.mark.parametrize("values", ["normal", "positive", "uneven", "spread"])
+@pytest.mark.parametrize("cin,filt", [(48, 1), (192, 1), (768, 1), (128, 3), (512, 3)])
+def test_error_no_larger_than_of_fp32_matrix_instructions(cin, filt, values, torch_dev, monkeypatch):
+    """both kernels of a layer against 64-bit sums, errors as a share of sum |a b|: the root mean square over the outputs.  0.63-0.88 on values
+    as layers hold them (spread over 2^+-4 among them).  Where operands spread over 2^+-24 a single term decides the sum and its own
+    rounding the error: 1.10-1.19, asked to stay below 1.25."""
+    torch = torch_dev
+    d = conv_desc(2, cin, 24, 24, 192, filt, 1, filt // 2)
+    d.has_bias = 0
+    g = torch.Generator().manual_seed(cin)
+    x, w = torch.randn(d.n, cin, d.h, d.w, generator=g), torch.randn(d.cout, cin, filt, filt, generator=g)
+    if values == "positive":
+        x, w = x.abs(), w.abs()
+    if values in ("uneven", "spread"):
+        e = 4 if values == "uneven" else 24
+        x, w = (t * 2.0 ** (2 * e * torch.rand(t.shape, generator=g) - e) for t in (x, w))
+    ref, magnitude = conv_ref(torch, d, x, w, torch.zeros(d.cout))
+    x, w = x.cuda(), w.cuda()
+    wk = hip.pack_conv_weights(d, w) if filt > 1 else w
+
+    def error(tile):
+        monkeypatch.setenv("ONHIP_TILE", tile)
+        y = hip.conv2d_f32(d, x, wk, None, packed=filt > 1).double().cpu()
+        return float(((y - ref) / magnitude).square().mean().sqrt())
+
+    ours, theirs = error("64x64x1x0x2"), error("64x64x1")
+    print(f"f3 error K {cin * filt * filt} {values}: {ours:.3e}, of fp32 matrix instructions {theirs:.3e}, ratio {ours / theirs:.3f}", flush=True)
+    assert ours <= (1.25 if values == "spread" else 1.0) * theirs
