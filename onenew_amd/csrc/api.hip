@@ -595,20 +595,27 @@ static bool f3_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out
     static const double per_k_tile[kNumF3Tiles] = {0.82, 0.50, 0.46, 0.50, 0.29, 0.215};   // per K tile of 16 and workgroup
     static const double per_tile[kNumF3Tiles] = {3.8, 1.8, 1.7, 1.25, 0.70, 0.37};        // first loads and store of a workgroup
     *us = 1e300;
-    for (int t = 0; t < kNumF3Tiles; ++t)
-        for (int s = 0; s < kNumSplits; ++s) {
-            const Choice c = {kF3Tiles[t][0], kF3Tiles[t][1], kSplits[s], 0, 2, 0, 0};
-            if (c.bm > 64 && p.M <= c.bm / 2) continue;
-            if (!candidate_ok(cfg, p, c)) continue;
-            // (with the weights split on the call: cut no finer than the entry point that allocates nothing has room for, an image
-            // at a time, so that it runs what this one does)
-            if (!p.keeper && c.split > 1 && 4LL * c.split * p.M * p.OHW + split_weights_bytes(p.M, p.K) > (long long) kNoAllocScratchBytes) continue;
-            const int k_tiles = (p.k_units + 3) / 4, per = (k_tiles + c.split - 1) / c.split;
-            const double tiles = (double) ((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn);
-            double t_us = 4.2 + ceil(tiles * c.split / 256.0) * (per * per_k_tile[t] + per_tile[t]);
-            if (c.split > 1) t_us += 3.4 + 0.33e-6 * c.split * 4.0 * p.M * p.N;   // partial sums, and the launch that adds them up
-            if (t_us < *us) { *us = t_us; *out = c; }
+    if (!f3_ok(cfg, p)) return false;
+    // what candidate_ok asks of each choice, asked once where it is the same for all: 78 of them for each launch of a pass
+    const long long outputs = (long long) p.M * p.N;
+    const int k_tiles = (p.k_units + 3) / 4;
+    long long most = cfg.bl == BL_ROWS ? 1 : std::min(k_tiles / 2LL, (256LL << 20) / (4 * outputs));
+    // (with the weights split on the call: cut no finer than the entry point that allocates nothing has room for, an image at a
+    // time, so that it runs what this one does)
+    if (!p.keeper && cfg.bl != BL_ROWS) most = std::min(most, ((long long) kNoAllocScratchBytes - split_weights_bytes(p.M, p.K)) / (4LL * p.M * p.OHW));
+    int per_slice[kNumSplits], cuts = 0;
+    for (; cuts < kNumSplits && (cuts == 0 || kSplits[cuts] <= most); ++cuts) per_slice[cuts] = (k_tiles + kSplits[cuts] - 1) / kSplits[cuts];
+    for (int t = 0; t < kNumF3Tiles; ++t) {
+        const int bm = kF3Tiles[t][0], bn = kF3Tiles[t][1];
+        if (bm > 64 && p.M <= bm / 2) continue;
+        const long long tiles = (long long) ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
+        for (int s = 0; s < cuts; ++s) {
+            const int cut = kSplits[s], per = per_slice[s], rounds = (int) ((tiles * cut + 255) >> 8);
+            double t_us = 4.2 + rounds * (per * per_k_tile[t] + per_tile[t]);
+            if (cut > 1) t_us += 3.4 + 0.33e-6 * cut * 4.0 * outputs;   // partial sums, and the launch that adds them up
+            if (t_us < *us) { *us = t_us; *out = Choice{bm, bn, cut, 0, 2, 0, 0}; }
         }
+    }
     if (*us > 1e299) return false;
     // The pass that splits the weights is a launch of its own: 4 bytes read, 6 written.  Against convolutions, and products with
     // fewer columns than a tile has rows, count the 10 % that both estimates are off by as well: 43 x 4536 x 383 and 42 x 8488 x
