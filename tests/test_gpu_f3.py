@@ -200,6 +200,22 @@ def test_kept_weights_are_measured_apart(tmp_path):
     assert len(keys) == 2, keys
 
 
+@pytest.mark.parametrize("n,cin,hw,cout,ours", [(64, 384, 14, 64, False), (64, 96, 14, 576, True), (64, 320, 7, 1280, True)])
+def test_layers_bound_by_their_activations(n, cin, hw, cout, ours, torch_dev):
+    """1x1 layers of MobileNetV2 on kept weights: a lone workgroup per compute unit that waits for its activations gains too little from the
+    16-bit matrix cores (16.8 -> 16.0 us for the first layer) for what they draw; the others gain a quarter"""
+    from onenew_amd import ops
+    torch = torch_dev
+    print(f"f3 choice {n} x {cin} x {hw} -> {cout}", flush=True)
+    d = conv_desc(n, cin, hw, hw, cout, 1, 1, 0)
+    rng = np.random.default_rng(cin)
+    x, w, b = (rng.standard_normal(s, dtype=np.float32) for s in ((n, cin, hw, hw), (cout, cin, 1, 1), (cout,)))
+    y = torch.from_numpy(ops.Conv(ops.Plugin(hip.plugin_path("Conv")).eval, d, w, b)(x)).double()
+    assert (hip.last_launch_choice()[4] == 2) == ours
+    x, w, b = (torch.from_numpy(t) for t in (x, w, b))
+    check(y, *conv_ref(torch, d, x, w, b), cin)
+
+
 def test_streams_and_threads(torch_dev):
     """weights split on the call: more streams than there are slots for them, one after another, and two threads on one stream"""
     torch = torch_dev
