@@ -514,7 +514,7 @@ static long long int8_slices(const IgemmLaunch &cfg, const IgemmProblem &p) {
 // Cost model (cycles).  A CU works through its share of the workgroups; co-resident workgroups share
 // the MFMA pipes, so the MFMA time adds up while the per-workgroup fill/drain latency overlaps when
 // several are resident.  Split-K adds the partial-sum traffic and a second launch.
-static double model_cost(const IgemmLaunch &cfg, const IgemmProblem &p, const Choice &c) {
+static double model_cost(const IgemmLaunch &cfg, const IgemmProblem &p, const Choice &c, bool whole = false) {
     const long long tiles = (long long) ((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn) * cfg.batch;
     const int k_tiles = (p.k_units + 3) / 4;
     const int per = (k_tiles + c.split - 1) / c.split;
@@ -538,8 +538,8 @@ static double model_cost(const IgemmLaunch &cfg, const IgemmProblem &p, const Ch
     // a few tiles and a K of 2304 / 4608: 17.3-19.0 / 25.7 us in one piece, 13.7 / 14.5 us in four slices
     // (int8 results stay whole: a launch in slices leaves the padding of their channels unwritten).  Only where the caller's
     // workspace has room for the partial sums: the shared block for them allocates and is not for overlapping launches, which
-    // such layers did without before
-    const bool few_int8 = int8_slices(cfg, p) > 1 && wgs <= 512.0;
+    // such layers did without before.  whole: among launches in one piece
+    const bool few_int8 = cfg.dtype == DT_I8 && !p.out_s8 && wgs <= 512.0 && (whole || p.slices_bytes >= 8LL * p.M * p.N);
     if (few_int8) cycles = fmax(cycles, ceil(per_cu / resident) * (per * 500.0 + fixed));
     if (c.split > 1) cycles += (few_int8 ? 6300.0 : 9000.0) + (double) (c.split + 1) * p.M * p.N * cfg.batch * 4.0 / 1500.0;
     return cycles;
@@ -665,20 +665,26 @@ static Choice model_choice(const IgemmLaunch &cfg, const IgemmProblem &p) {
         const long long tiles = (long long) ((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn);
         if (tiles >= 512 && candidate_ok(cfg, p, c)) return c;   // measured at batch 64 only: at least two workgroups per CU
     }
-    const long long slices = int8_slices(cfg, p) > 1 ? int8_slices(cfg, p) : 1 << 20;
-    for (int pass = tl_hint_bm ? 0 : 1; pass < 2; ++pass) {   // pass 0: the hinted tile; pass 1: every tile
-        double best_cost = 1e300;
-        for (int t = 0; t < kNumTiles; ++t)
-            for (int s = 0; s < kNumSplits; ++s) {
-                const Choice c = {kTiles[t][0], kTiles[t][1], kSplits[s], 0, 0, 0};
-                if (pass == 0 && (c.bm != tl_hint_bm || c.bn != tl_hint_bn)) continue;
-                if (c.split > slices) continue;
-                if (!candidate_ok(cfg, p, c)) continue;
-                const double cost = model_cost(cfg, p, c);
-                if (cost < best_cost) { best_cost = cost; best = c; }
-            }
-        if (best_cost < 1e300) break;
-    }
+    auto cheapest = [&](long long slices, bool whole) {
+        for (int pass = tl_hint_bm ? 0 : 1; pass < 2; ++pass) {   // pass 0: the hinted tile; pass 1: every tile
+            double best_cost = 1e300;
+            for (int t = 0; t < kNumTiles; ++t)
+                for (int s = 0; s < kNumSplits; ++s) {
+                    const Choice c = {kTiles[t][0], kTiles[t][1], kSplits[s], 0, 0, 0};
+                    if (pass == 0 && (c.bm != tl_hint_bm || c.bn != tl_hint_bn)) continue;
+                    if (c.split > slices) break;
+                    if (!candidate_ok(cfg, p, c)) continue;
+                    const double cost = model_cost(cfg, p, c, whole);
+                    if (cost < best_cost) { best_cost = cost; best = c; }
+                }
+            if (best_cost < 1e300) break;
+        }
+    };
+    const long long room = int8_slices(cfg, p);
+    cheapest(room > 1 ? room : 1 << 20, false);
+    // int8 in one piece for want of room or of K tiles to cut: the tile by what a K tile takes (MobileNetV2 W8A32 at batch 8, 25088 pixels:
+    // 96 -> 24 channels 6.4 us with 64 x 64 tiles, 7.3 with 32 x 128; 144 -> 24 and an Add 8.9 and 10.7)
+    if (cfg.dtype == DT_I8 && !p.out_s8 && room <= 1 && best.split == 1) cheapest(1, true);
     // fp32 with a weight matrix for A: the 16-bit matrix cores where that is expected to be faster.  Not for up to 32 rows
     // (the smallest of those tiles has 64: 0.74-0.98 of these kernels' speed on MobileNetV2's projections) nor for reductions
     // below 48 (bound by memory: 0.69 on its 16 -> 96 expansion, where the kernel that reads B straight from memory runs).

@@ -33,6 +33,29 @@ def test_few_tiles_long_reduction(cin, hw, cout, monkeypatch):
     assert torch.equal(y, whole) and bool((y > 0).any())
 
 
+def test_tile_of_a_short_reduction(monkeypatch):
+    """a layer whose K has nothing to cut: the tile is chosen by the time of its K tiles all the same"""
+    import torch
+    hip.init(0)
+    print("int8 96 -> 24 56x56 batch 8", flush=True)
+    d = ConvDesc(n=8, cin=96, h=56, w=56, cout=24, kh=1, kw=1, stride_h=1, stride_w=1, group=1, has_bias=1, act_type=abi.NOT_ACT, compute=abi.COMPUTE_F32)
+    d.input_scale = 1.0 / 127
+    g = torch.Generator(device="cuda").manual_seed(96)
+    w8 = torch.randint(-127, 128, (24, 96, 1, 1), generator=g, device="cuda", dtype=torch.int8)
+    x = torch.rand((8, 96, 56, 56), generator=g, device="cuda") * 2 - 1
+    b32, aux = torch.randint(-9999, 9999, (24,), generator=g, device="cuda", dtype=torch.int32), torch.rand((24,), generator=g, device="cuda")
+    wp, before = hip.pack_conv_weights_w8(d, w8), hip.set_tuning(0)
+    try:
+        y = hip.conv2d_w8a32(d, x, wp, b32, aux, packed=True)
+        assert hip.last_launch_choice()[:3] == (64, 64, 1)
+        monkeypatch.setenv("ONHIP_TILE", "32x128x1")
+        other = hip.conv2d_w8a32(d, x, wp, b32, aux, packed=True)
+        assert hip.last_launch_choice()[:2] == (32, 128)
+    finally:
+        hip.set_tuning(before)
+    assert torch.equal(y, other) and bool((y > 0).any())
+
+
 def test_slices_stay_in_the_callers_workspace():
     """Layers that run in K slices on two streams at once, each with a workspace of its own: nothing of the process is shared or
     allocated.  With a workspace that holds the int8 activations alone they run in one piece."""
