@@ -92,6 +92,53 @@ def test_product(m, k, n, special, torch_dev):
     check(y, (a.double() @ b.double() + bias.double()).cpu(), (a.double().abs() @ b.double().abs() + bias.double().abs()).cpu(), k)
 
 
+@pytest.mark.parametrize("bm,bn", TILES)
+@pytest.mark.parametrize("loader,shape", [SHAPES[i] for i in (0, 1, 3, 4, 7)], ids=["plain0", "plain1", "tapc3", "gather4", "gather7"])
+def test_stores(loader, shape, bm, bn, torch_dev, monkeypatch):
+    """the residual operand's kernels and the activations of a store, bit for bit what the operators do to the plain store's result"""
+    torch = torch_dev
+    print(f"f3 stores {loader} {shape} tile {bm}x{bn}", flush=True)
+    monkeypatch.setenv("ONHIP_TILE", f"{bm}x{bn}x1x0x2")
+    d = conv_desc(*shape)
+    g = torch.Generator(device="cuda").manual_seed(bm + bn)
+    rand = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    x, w, b = rand(d.n, d.cin, d.h, d.w), rand(d.cout, d.cin, d.kh, d.kw) / (d.cin * d.kh * d.kw) ** 0.5, rand(d.cout)
+    wk = hip.pack_conv_weights(d, w) if loader == "tapc" else w
+    packed = loader == "tapc"
+    y = hip.conv2d_f32(d, x, wk, b, packed=packed)
+    r = rand(*y.shape)
+    for relu in (False, True):
+        z = hip.conv2d_f32_add(d, x, wk, r, b, relu=relu, packed=packed)
+        assert hip.last_launch_choice()[4] == 2 and hip.last_launch_choice()[:2] == (bm, bn)
+        assert torch.equal(z, (y + r).clamp(min=0) if relu else y + r)
+    d.act_type = abi.RELU
+    assert torch.equal(hip.conv2d_f32(d, x, wk, b, packed=packed), y.clamp(min=0))
+    d.act_type, d.clip_min, d.clip_max = abi.CLIP, -0.5, 0.75
+    assert torch.equal(hip.conv2d_f32(d, x, wk, b, packed=packed), y.clamp(-0.5, 0.75))
+    assert hip.last_launch_choice()[4] == 2
+
+
+@pytest.mark.parametrize("m,k,n", [(8195, 773, 1030), (12545, 193, 768), (8190, 1029, 193)])
+def test_product_stores(m, k, n, torch_dev, oracle):
+    """an addend with and without a bias, and the table GELU, bit for bit what the operators do to the plain store's result"""
+    torch = torch_dev
+    print(f"f3 product stores {m} x {k} x {n}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m)
+    rand = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    a, b, bias, r = rand(m, k), rand(k, n) / k ** 0.5, rand(n), rand(m, n)
+    lut = torch.from_numpy(np.ascontiguousarray(oracle.gelu_lut())).cuda()
+    for v in (None, bias):
+        y = hip.matmul(a, b, v)
+        assert hip.last_launch_choice()[4] == 2
+        plain = hip.last_launch_choice()
+        z = hip.matmul(a, b, v, addend=r)
+        assert hip.last_launch_choice() == plain
+        assert torch.equal(z, y + r)
+        z = hip.matmul(a, b, v, gelu_lut=lut)
+        assert hip.last_launch_choice() == plain
+        assert torch.equal(z, hip.gelu_lut_f32(y, lut))
+
+
 def test_time_on_nonfinite_data(torch_dev):
     """sums that are not finite are computed again at the rate of matrix instructions: 4.3 times the time where all of them are, 118 times
     with one multiply-add a lane and element"""
@@ -284,6 +331,7 @@ def test_capture(torch_dev, monkeypatch):
     torch.cuda.synchronize()
     with torch.cuda.stream(stream):
         work(jobs[0])
+    assert all(c[4] == 2 for c in choices), choices
     torch.cuda.synchronize()
 
     def record(job):
@@ -303,12 +351,17 @@ def test_capture(torch_dev, monkeypatch):
                     graph.replay()
             with torch.cuda.stream(stream):   # the recording stream goes on with weights of its own
                 hip.matmul(jobs[0][0], jobs[1][1])
+                assert hip.last_launch_choice()[4] == 2
             torch.cuda.synchronize()
             for job in jobs:
                 check(job[5], *job[7], k)
                 check(job[6], *job[8], d.cin)
 
-    replay([record(job) for job in jobs])
+    first = []
+    for job in jobs:
+        first.append(record(job))
+        assert all(c[4] == 2 for c in choices), choices
+    replay(first)
     graphs = [record(jobs[i % 2]) for i in range(33)]
     assert all(c[4] != 2 and c[2] == 1 and c[3] == 0 for c in choices), choices
     replay(graphs[-2:])
