@@ -583,7 +583,7 @@ static bool dma_model_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choi
 }
 
 // a 1x1 convolution whose activations come from beyond the L2s
-static bool f3_streams(const IgemmLaunch &cfg, const IgemmProblem &p) { return cfg.bl == BL_PLAIN && p.b_slice_bytes > (8LL << 20); }
+static bool f3_streams(const IgemmLaunch &cfg, const IgemmProblem &p) { return cfg.bl == BL_PLAIN && p.w_src && p.b_slice_bytes > (8LL << 20); }
 
 // Best tile and K split of the fp32 kernel on the 16-bit matrix cores and what the launch takes, in microseconds.  Fitted to
 // 1100 timed launches over the layers of ResNet-50 (batch 1, 8, 32) and MobileNetV2 (batch 8, 64), median error 10 %, the
@@ -591,12 +591,12 @@ static bool f3_streams(const IgemmLaunch &cfg, const IgemmProblem &p) { return c
 // (larger tiles stage less per multiply-add), whether one or several are resident.
 // 192 x 64 is for row counts that 128 does not divide (192, 576, 960 of transformers and expansions, 2053): 192 x 12544 x 768
 // 30.4 us, 128 x 128 32.5 and 64 x 64 34.1.
-// Those launches ran on their own.  Two things that they do not show, from traces of whole passes (90 layers of ResNet-50 at batch 1, 8
-// and 32, MobileNetV2 at 8, 24 and 64, ViT-Tiny at 64):
-//  * A lone workgroup per compute unit that streams a 1x1 convolution's activations from beyond the L2 waits for its loads, three K tiles of
-//    which are in flight: 0.35-0.54 us a K tile of the tiles with 64 columns, whatever it multiplies with (160 x 3136 x 960 in 64 x 64 tiles
-//    25.9 us, 24.3 with fp32 matrix instructions in four slices and 20.8 in five of 128 x 128; 96 x 12544 x 576 in 128 x 64 tiles
-//    24.4, 23.8 and 22.6 in 64 x 64).
+// Those launches ran on their own.  What they do not show, from traces of whole passes (90 layers of ResNet-50 at batch 1, 8 and 32,
+// MobileNetV2 at 8, 24 and 64, ViT-Tiny at 64):
+//  * One or two workgroups per compute unit that stream a 1x1 convolution's activations from beyond the L2 wait for their loads, three K
+//    tiles of which are in flight, whatever they multiply with: 0.35-0.48 us a K tile of 64 x 64, 0.41-0.54 of 128 x 64, 0.35-0.49 of
+//    the fp32 kernels (f32_us).  Slices written there cost half as much again (256 x 6272 x 1024 in two of 128 x 128 36 us, in one piece of
+//    128 x 64 31).
 //  * A residual operand is read when all workgroups store: 0.18 us a MB (1024 x 6272 x 256 23.3 us, 26.4 with one; 512 x 25088 x 128 29.3
 //    and 34.2), 0.066 for the fp32 kernels, more of whose workgroups are resident.
 static bool f3_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out, double *us) {
@@ -623,8 +623,9 @@ static bool f3_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out
         const long long tiles = (long long) ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
         for (int s = 0; s < cuts; ++s) {
             const int cut = kSplits[s], per = per_slice[s], rounds = (int) ((tiles * cut + 255) >> 8);
-            double t_us = 4.2 + rounds * (per * per_k_tile[t] * (streams && rounds == 1 && bn == 64 ? 1.7 : 1.0) + per_tile[t]);
-            if (cut > 1) t_us += 3.4 + 0.33e-6 * cut * 4.0 * outputs;   // partial sums, and the launch that adds them up
+            const double waits = !streams || rounds > 1 ? 1.0 : bm == 64 ? 1.7 : bm == 128 && bn == 64 ? 1.4 : 1.0;
+            double t_us = 4.2 + rounds * (per * per_k_tile[t] * waits + per_tile[t]);
+            if (cut > 1) t_us += 3.4 + (streams ? 0.5e-6 : 0.33e-6) * cut * 4.0 * outputs;   // partial sums, and the launch that adds them up
             if (t_us < *us) { *us = t_us; *out = Choice{bm, bn, cut, 0, 2, 0, 0}; }
         }
     }
@@ -640,11 +641,14 @@ static bool f3_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out
     return true;
 }
 // the same for the fp32 matrix instructions' kernels (2250 cycles of model_cost take a microsecond; same launches, error 10 %)
-static double f32_us(const IgemmProblem &p, double cycles) { return 3.75 + cycles / 2250.0 + (p.res ? 0.066e-6 * 4.0 * p.M * p.N : 0.0); }
+static double f32_us(const IgemmLaunch &cfg, const IgemmProblem &p, const Choice &c) {
+    const long long wgs = (long long) ((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn) * c.split;
+    return 3.75 + model_cost(cfg, p, c) / (f3_streams(cfg, p) && wgs <= 512 ? 2250.0 / 1.2 : 2250.0) + (p.res ? 0.066e-6 * 4.0 * p.M * p.N : 0.0);
+}
 // Where the activations are streamed, a gain below 8 % is left alone.  The kernel draws so much power that the card lowers its clock, for
 // the launches around it as well: MobileNetV2 at batch 64 runs at 2.4 GHz without it and at 2.3 with it in twenty launches, where the one-launch
-// blocks then take 98 -> 102 us.  With every layer that was expected to be faster at all, the pass took 1037, 1046, 1056, 1070 and 1090 us
-// on five cards, without the kernel 1065, 1065, 1062, 1066 and 1067; on the second of them it takes 1041 now.
+// blocks then take 98 -> 102 us.  With every layer that was expected to be faster at all, the pass took 1036, 1046, 1056, 1070, 1078 and
+// 1090 us on six cards, without the kernel 1062-1067; now 1029, 1041, -, -, 1072 and -.
 static bool f3_wins(const IgemmLaunch &cfg, const IgemmProblem &p, double f3, double f32) { return f3 < (f3_streams(cfg, p) ? 0.92 : 1.0) * f32; }
 
 static Choice model_choice(const IgemmLaunch &cfg, const IgemmProblem &p) {
@@ -691,7 +695,7 @@ static Choice model_choice(const IgemmLaunch &cfg, const IgemmProblem &p) {
     if (cfg.dtype == DT_F32 && !tl_hint_bm && p.M > 32 && p.K >= 48) {
         Choice c;
         double us;
-        if (f3_choice(cfg, p, &c, &us) && f3_wins(cfg, p, us, f32_us(p, model_cost(cfg, p, best)))) return c;
+        if (f3_choice(cfg, p, &c, &us) && f3_wins(cfg, p, us, f32_us(cfg, p, best))) return c;
     }
     // What measuring the candidates keeps finding on top of the tile and split above (fp32, one batch slice):
     //  * no split, and a few tiles left over after whole rounds of 256: those tiles alone cut along K so that the leftover,
@@ -1754,7 +1758,7 @@ static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float
         if (form.p.M > 32 && form.p.K >= 48 && p.b_slice_bytes < (1LL << 31) && form.p.b_slice_bytes < (1LL << 31) &&
             form.p.c_slice_bytes < (1LL << 31) && f3_choice(form.cfg, form.p, &form.rows, &us)) {
             form.plain = model_choice(cfg, p);
-            form.faster = !tl_hint_bm && us < f32_us(p, model_cost(cfg, p, form.plain));   // a hint is for the plain form's tile
+            form.faster = !tl_hint_bm && us < f32_us(cfg, p, form.plain);   // a hint is for the plain form's tile
             form.p.keeper = keeper;
             return plan_and_launch(cfg, p, st, &form);
         }
