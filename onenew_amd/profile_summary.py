@@ -38,11 +38,19 @@ LEGEND = ("Kernel names: `onhip::igemm_kernel<dtype, loader, BM, BN, WM, WN, PF,
           "RES the variant whose store adds a residual operand; PW2 the variant that multiplies its finished tile by a second, 1x1 weight "
           "matrix before storing: a convolution and the 1x1 convolution after it in one launch), `onhip::igemm_dma_kernel<dtype, BM, BN, WM, WN, KS, NST>` (int8 and "
           "16-bit storage: operand tiles loaded straight into LDS, KS bytes of K per stage, ring of NST stages), `onhip::rowb_f32_kernel<WM, WN>` (fp32, B "
-          "straight from memory, tile 32 WM x 128 WN), `onhip::splitk_finish_kernel`, `onhip::depthwise_tiled_kernel<int8, stride, "
+          "straight from memory, tile 32 WM x 128 WN), `onhip::igemm_f3_kernel<loader, BM, BN, WM, WN, RES>` (fp32 on the 16-bit matrix cores; loader 5 "
+          "the rows of a product) and `onhip::split_weights_kernel` in front of it where the weights are split on the call, `onhip::splitk_finish_kernel`, `onhip::depthwise_tiled_kernel<int8, stride, "
           "act>`, `onhip::quantize_nhwc_kernel<CBW>`, `onhip::stem_f32_kernel<filter size, act, two row tiles>` (first-layer "
           "convolutions from an LDS patch), `onhip::i8patch_kernel<bytes per pixel, WM, pixel tiles>` and `onhip::i8direct_kernel<bytes per pixel, taps, WM, TM, pixel "
           "tiles, workgroups per CU>` (int8 chain form, 3x3 with few channels: input rows in LDS / windows loaded per tap), `onhip::attention_f32_kernel<16-key tiles, head dim>`, `onhip::dw_s8_nhwc_kernel<3x3 stride, epilogue, fp32 out>` (depthwise on int8 NHWC), `onhip::irblock_f32_kernel<act, input channels / 4, row tiles, "
           "patches>` (1x1 expansion + depthwise 3x3 + 1x1 projection in one launch), and the element-wise kernels.")
+
+
+HELPERS = ("splitk_finish", "split_weights")   # launches that belong to a layer's own
+
+
+def helper(name):
+    return any(h in name for h in HELPERS)
 
 
 def short(name):
@@ -54,7 +62,7 @@ def short(name):
 def family(name):
     if "_pack_kernel" in name:   # weight re-layouts: once per model, not part of a pass
         return None
-    if "igemm" in name or "splitk_finish" in name or "rowb_f32" in name or "attention" in name or "stem_f32" in name or "i8patch" in name or "i8direct" in name:
+    if "igemm" in name or helper(name) or "rowb_f32" in name or "attention" in name or "stem_f32" in name or "i8patch" in name or "i8direct" in name:
         return "igemm"
     if "depthwise" in name or "irblock" in name or "dw_s8" in name:
         return "depthwise"
@@ -113,7 +121,7 @@ def summarise(workload, raw, out_dir):
     if whole_model:
         # the operator that runs once per inference has the fewest calls: that count is the number of inferences traced
         # (warm-up, timed steps, and the runs bench.py makes before them to fill the tile cache and check the outputs)
-        passes = min([int(r["Calls"]) for rs in groups.values() for r in rs if "splitk_finish" not in r["Name"]] or [passes])
+        passes = min([int(r["Calls"]) for rs in groups.values() for r in rs if not helper(r["Name"])] or [passes])
         L.append(f"The traced run makes {passes} inferences of the {nl} operators ({bench['warmup']} warm-up + {bench['steps']} timed, the rest "
                  f"before them: tile choices, output checks).")
     else:
@@ -122,8 +130,8 @@ def summarise(workload, raw, out_dir):
                  f"where the cache did not have them.")
     for g, rs in groups.items():
         ns = sum(float(r["TotalDurationNs"]) for r in rs)
-        main = sum(int(r["Calls"]) for r in rs if "splitk_finish" not in r["Name"])
-        L.append(f"- {g}: {main} layer launches, {ns / 1e6:.3f} ms in total (split-K reduction included) = "
+        main = sum(int(r["Calls"]) for r in rs if not helper(r["Name"]))
+        L.append(f"- {g}: {main} layer launches, {ns / 1e6:.3f} ms in total (split-K reduction and weight split included) = "
                  f"**{ns / main / 1e3:.2f} us per layer launch**, {ns / passes / 1e6:.4f} ms per pass.")
     rf = bench["roofline"]
     if whole_model:
@@ -149,7 +157,7 @@ def summarise(workload, raw, out_dir):
             fv, wv = fetch[k]["FETCH_SIZE"], write[k]["WRITE_SIZE"]
             L.append(f"| `{k}` | {len(fv)} | {mean(fv):.1f} | {mean(wv):.1f} | {mean(fv) * ff / 1024:.2f} | {mean(wv) * wf / 1024:.2f} |")
             traffic[g] += (sum(fv) * ff + sum(wv) * wf) * 1024
-            if "splitk_finish" not in k:
+            if not helper(k):
                 launches[g] += len(fv)
         L.append("")
         for g in traffic:
