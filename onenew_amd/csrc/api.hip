@@ -328,7 +328,8 @@ static const int kNumSplits = 13;
 
 // tail > 1: the tiles left over after whole rounds of 256 are cut `tail` ways along K (launch_choice)
 // rowb == 1: the kernel that feeds B from global memory straight into the MFMAs (igemm_rowb.hip), tile bm x bn; rowb == 2: the
-// fp32 kernel on the 16-bit matrix cores (igemm_f3.hip), tile bm x bn
+// fp32 kernel on the 16-bit matrix cores (igemm_f3.hip), tile bm x bn; rowb == 3: the fp32 kernel whose wavefronts share K
+// (igemm_kw.hip), tile bm x bn, `split` wavefronts a workgroup
 // fin != 0 (with split > 1 or tail > 1): the slices of a tile are added up by the last of them to arrive, inside the
 // launch, instead of by a finishing launch (igemm_kernel, `arrive`)
 // dma != 0: the kernel that loads its operand tiles straight into LDS (igemm_dma_kernel.hpp), tile bm x bn, never split;
@@ -458,10 +459,16 @@ static const int kRowbTiles[][2] = {{64, 128}, {128, 128}, {64, 256}, {96, 128},
 static const int kNumRowbTiles = 6;
 static const int kF3Tiles[][2] = {{256, 128}, {256, 64}, {192, 64}, {128, 128}, {128, 64}, {64, 64}};
 static const int kNumF3Tiles = 6;
+static const int kKwShapes[][3] = {{16, 16, 4}, {32, 32, 4}, {32, 32, 8}, {64, 32, 4}};   // tile, wavefronts
 
 // (bm, bn) is a tile this build has a kernel for
 static bool tile_exists(const Choice &c) {
     if (c.dma) return c.dma <= 2 && dma_tile_ok(c.bm, c.bn);
+    if (c.rowb == 3) {
+        for (const auto &k : kKwShapes)
+            if (k[0] == c.bm && k[1] == c.bn && k[2] == c.split) return true;
+        return false;
+    }
     const int (*list)[2] = c.rowb == 2 ? kF3Tiles : c.rowb ? kRowbTiles : kTiles;
     const int n = c.rowb == 2 ? kNumF3Tiles : c.rowb ? kNumRowbTiles : kNumTiles;
     for (int t = 0; t < n; ++t)
@@ -478,6 +485,9 @@ static bool f3_ok(const IgemmLaunch &cfg, const IgemmProblem &p) {
     return bytes < (1LL << 31) && (p.keeper || bytes <= kSplitWsBytes);
 }
 
+// the kernel whose wavefronts share K takes split weights where the caller keeps them, and never makes them on the call
+static bool kw_split(const IgemmLaunch &cfg, const IgemmProblem &p) { return p.keeper && f3_ok(cfg, p); }
+
 static bool candidate_ok(const IgemmLaunch &cfg, const IgemmProblem &p, const Choice &c) {
     if (!tile_exists(c)) return false;   // e.g. a line of the cache file written by another build or by hand
     const int k_tiles = (p.k_units + k_tile_units(cfg.dtype) - 1) / k_tile_units(cfg.dtype);
@@ -489,6 +499,7 @@ static bool candidate_ok(const IgemmLaunch &cfg, const IgemmProblem &p, const Ch
         return (!off || h16) && c.split == 1 && c.tail <= 1 && !c.rowb && !c.fin && dma_ok(cfg, p);
     }
     if (h16) return false;
+    if (c.rowb == 3) return c.tail <= 1 && !c.fin && kw_ok(cfg, p, c.bm, kw_split(cfg, p));
     if (c.rowb == 2 && (c.tail > 1 || c.fin || (c.split > 1 && cfg.bl == BL_ROWS) || !f3_ok(cfg, p))) return false;   // whole tiles, or slices and a finishing launch
     if (c.rowb == 1 && (c.split != 1 || !rowb_f32_ok(cfg, p))) return false;
     if (c.fin) {
@@ -640,8 +651,34 @@ static bool f3_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out
     }
     return true;
 }
+// Best shape of the kernel whose wavefronts share K, and its microseconds.  From the layers of ResNet-50 at batch 1 (80 layers, 4
+// shapes and both forms of the weights, weights beyond the L2; error 10 %): a compute unit does its workgroups' steps one after the
+// other, whoever's they are, and a workgroup costs its start.  A stride along the columns takes twice the cache lines.  Two wavefronts per
+// SIMD pay from 32 steps a tile on where a workgroup has its unit to itself (128 x 784 x 1152 12.0 -> 9.7 us).  Only for operands that
+// fit the L2s: with more the other kernels, which load a tile once, are ahead anyway.
+static bool kw_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out, double *us) {
+    static const double step[2][3] = {{0.122, 0.105, 0.21}, {0.087, 0.086, 0.13}};   // fp32 / split weights; tiles of 16, 32, 64 rows
+    static const double base[2][3] = {{2.8, 3.6, 4.0}, {3.4, 3.6, 3.9}}, start[3] = {0.0016, 0.003, 0.003};
+    *us = 1e300;
+    if (cfg.dtype != DT_F32 || p.b_slice_bytes > (8LL << 20)) return false;
+    const int split = kw_split(cfg, p);
+    for (int t = 0; t < 3; ++t) {
+        const int bm = 16 << t, bn = t ? 32 : 16, ks = t ? 16 : 32;
+        const long long tiles = (long long) ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
+        if (tiles > 2048 || (bm > p.M + 15) || !kw_ok(cfg, p, bm, split != 0)) continue;
+        const int steps = (p.K + ks - 1) / ks;
+        const double t_us = base[split][t] + ((tiles + 255) / 256) * steps * step[split][t] * (p.sw > 1 ? 1.4 : 1.0) + tiles * start[t];
+        if (t_us < *us) { *us = t_us; *out = Choice{bm, bn, t == 1 && tiles <= 256 && steps >= 32 ? 8 : 4, 0, 3, 0, 0}; }
+    }
+    return *us < 1e299;
+}
 // the same for the fp32 matrix instructions' kernels (2250 cycles of model_cost take a microsecond; same launches, error 10 %)
 static double f32_us(const IgemmLaunch &cfg, const IgemmProblem &p, const Choice &c) {
+    if (c.rowb == 3) {
+        Choice same;
+        double us;
+        return kw_choice(cfg, p, &same, &us) ? us : 1e300;
+    }
     const long long wgs = (long long) ((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn) * c.split;
     return 3.75 + model_cost(cfg, p, c) / (f3_streams(cfg, p) && wgs <= 512 ? 2250.0 / 1.2 : 2250.0) + (p.res ? 0.066e-6 * 4.0 * p.M * p.N : 0.0);
 }
@@ -689,14 +726,18 @@ static Choice model_choice(const IgemmLaunch &cfg, const IgemmProblem &p) {
     // int8 in one piece for want of room or of K tiles to cut: the tile by what a K tile takes (MobileNetV2 W8A32 at batch 8, 25088 pixels:
     // 96 -> 24 channels 6.4 us with 64 x 64 tiles, 7.3 with 32 x 128; 144 -> 24 and an Add 8.9 and 10.7)
     if (cfg.dtype == DT_I8 && !p.out_s8 && room <= 1 && best.split == 1) cheapest(1, true);
+    double kw_us = 1e300;
+    Choice kw;
+    if (cfg.dtype == DT_F32 && !tl_hint_bm && kw_choice(cfg, p, &kw, &kw_us) && kw_us > 0.95 * f32_us(cfg, p, best)) kw_us = 1e300;
     // fp32 with a weight matrix for A: the 16-bit matrix cores where that is expected to be faster.  Not for up to 32 rows
     // (the smallest of those tiles has 64: 0.74-0.98 of these kernels' speed on MobileNetV2's projections) nor for reductions
     // below 48 (bound by memory: 0.69 on its 16 -> 96 expansion, where the kernel that reads B straight from memory runs).
     if (cfg.dtype == DT_F32 && !tl_hint_bm && p.M > 32 && p.K >= 48) {
         Choice c;
         double us;
-        if (f3_choice(cfg, p, &c, &us) && f3_wins(cfg, p, us, f32_us(cfg, p, best))) return c;
+        if (f3_choice(cfg, p, &c, &us) && us < 1.05 * kw_us && f3_wins(cfg, p, us, f32_us(cfg, p, best))) return c;
     }
+    if (kw_us < 1e299) return kw;
     // What measuring the candidates keeps finding on top of the tile and split above (fp32, one batch slice):
     //  * no split, and a few tiles left over after whole rounds of 256: those tiles alone cut along K so that the leftover,
     //    too, puts about a workgroup on every compute unit (launch_choice);
@@ -742,7 +783,7 @@ static const int kNoSplitSlot = 1;
 // their weights split, so none of them need have allocated the partial sums' scratch, and a capture may not.
 static Choice slotless_choice(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t st) {
     Choice c = model_choice(cfg, p);
-    if (under_capture(st)) { c.split = 1; c.tail = c.fin = 0; }
+    if (under_capture(st) && c.rowb != 3) { c.split = 1; c.tail = c.fin = 0; }
     return c;
 }
 
@@ -753,12 +794,16 @@ static int launch_choice(IgemmLaunch cfg, IgemmProblem p, const Choice &c, hipSt
         SplitSlot *slot; hipStream_t st;
         ~Use() { if (slot) slot_used(slot, st); }
     } use{nullptr, st};
-    if (c.rowb == 2 && !p.a_split) {
+    if ((c.rowb == 2 || (c.rowb == 3 && p.keeper && f3_ok(cfg, p))) && !p.a_split) {
         const void *kept = nullptr;
         p.a_split_bytes = split_weights_bytes(p.M, p.K);
         if (p.keeper) {
             const int rc = p.keeper->get(p.keeper->key, p.w_src, {p.M, p.K, p.w_row, p.w_k}, &kept);
             if (rc) return rc;
+        }
+        if (!kept && c.rowb == 3) {   // none can be made now: the weights as they are, here or in another kernel
+            p.keeper = nullptr;
+            return launch_choice(cfg, p, kw_ok(cfg, p, c.bm, false) ? c : slotless_choice(cfg, p, st), st);
         }
         if (!kept) {
             void *ws = nullptr;
@@ -805,7 +850,7 @@ static int launch_choice(IgemmLaunch cfg, IgemmProblem p, const Choice &c, hipSt
         const IgemmLaunch &cfg; const IgemmProblem &p; const Choice &c;
         ~Note() {
             const bool tail = p.tail_tiles > 0;
-            const int v[7] = {c.bm, c.bn, c.dma || tail ? 1 : cfg.split, tail ? cfg.split : 0, c.dma ? 0 : c.rowb, p.arrive ? 1 : 0, c.dma};
+            const int v[7] = {c.bm, c.bn, c.rowb == 3 ? c.split : c.dma || tail ? 1 : cfg.split, tail ? cfg.split : 0, c.dma ? 0 : c.rowb, p.arrive ? 1 : 0, c.dma};
             for (int i = 0; i < 7; ++i) tl_last_choice[i] = v[i];
         }
     } note{cfg, p, c};
@@ -817,6 +862,13 @@ static int launch_choice(IgemmLaunch cfg, IgemmProblem p, const Choice &c, hipSt
         p.arrive = nullptr;
         g_dma_launches.fetch_add(1, std::memory_order_relaxed);
         return dma_launch(cfg, p, st);
+    }
+    if (c.rowb == 3) {
+        cfg.bm = c.bm; cfg.bn = c.bn; cfg.split = 1;
+        p.k_split_units = p.k_units;
+        p.partial = nullptr;
+        p.arrive = nullptr;
+        return kw_launch(cfg, p, c.split, st);
     }
     auto launch = [&]() {
         const int rc = c.rowb == 2 ? f3_launch(cfg, p, st) : c.rowb ? rowb_f32_launch(cfg, p, st) : igemm_launch(cfg, p, st);
@@ -901,6 +953,7 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
             }
             if (c.fin && !candidate_ok(cfg, p, c)) c.fin = 0;
             if (c.rowb == 2 && c.tail > 1) c.tail = 0;
+            if (c.rowb == 3 && !candidate_ok(cfg, p, c)) c = model_choice(cfg, p);
             if (c.rowb == 2 && !candidate_ok(cfg, p, c)) { c = {64, 64, 1, 0, 0, 0, 0}; }
             if (c.rowb && !candidate_ok(cfg, p, c)) {   // not a problem for that kernel: the tiled one, same tile if it has it
                 c.rowb = 0;
@@ -934,7 +987,8 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
     if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
         return launch(by_model());
     const Choice guess = by_model();
-    const double guess_cost = model_cost(cfg, p, other ? other->plain : guess);
+    const Choice &tiled = other ? other->plain : guess;
+    const double guess_cost = model_cost(cfg, p, tiled.rowb == 3 ? Choice{64, 64, 1, 0, 0, 0, 0} : tiled);
     hipEvent_t e0, e1;
     ONHIP_CHECK_HIP(hipEventCreate(&e0));
     ONHIP_CHECK_HIP(hipEventCreate(&e1));
@@ -995,6 +1049,11 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
             }
         }
     }
+    // the fp32 kernel whose wavefronts share K, where the cost model would look at it
+    double kw_us;
+    if (Choice kw; !rc && kw_choice(cfg, p, &kw, &kw_us))
+        for (const auto &k : kKwShapes)
+            if (const Choice c = {k[0], k[1], k[2], 0, 3, 0, 0}; !rc && candidate_ok(cfg, p, c)) try_choice(c);
     // the fp32 kernel on the 16-bit matrix cores: every tile, with the model's K split and without
     Choice f3;
     double f3_us;

@@ -271,6 +271,9 @@ bool rowb_f32_ok(const IgemmLaunch &cfg, const IgemmParams &p);
 int rowb_f32_launch(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t stream);
 // fp32 kernel on the 16-bit matrix cores (igemm_f3.hip): p.a_split holds the weights in split_weights_launch's form
 int f3_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t stream);
+// fp32 kernel whose wavefronts share K (igemm_kw.hip), tile 16 x 16, 32 x 32 or 64 x 32 of bm rows; weights split (p.a_split) or as given
+bool kw_ok(const IgemmLaunch &cfg, const IgemmProblem &p, int bm, bool split);
+int kw_launch(const IgemmLaunch &cfg, const IgemmProblem &p, int waves, hipStream_t stream);
 inline long long split_weights_bytes(long long M, long long K) { return (M + 31) / 32 * ((K + 15) / 16) * 3072; }
 // Weights as M rows of K elements, element (row, k) at row * s_row + k * s_k.
 struct SplitSource { int M, K; long long s_row, s_k; };
