@@ -752,6 +752,24 @@ __device__ __forceinline__ void write_tile_nhwc_h16(const IgemmParams &p, f32x16
                                                     const float *rows) {
     static_assert(DT == DT_BF16 || DT == DT_F16, "16-bit floating-point outputs");
     constexpr int PITCH = 2 * BM + 16;
+    constexpr int GROUPS = BM / 8, NV = (BN * GROUPS + THREADS - 1) / THREADS;   // 16-byte vectors of a pixel, and of this thread
+    const int pitch = (int) p.c_stride_n;
+    const bool with_res = p.res16 != nullptr, relu = p.res_relu != 0;
+    const rsrc_t rr = make_rsrc(p.res16, p.res16 ? RSRC_RANGE : 0u);
+    // The addends of all of the thread's vectors are requested here, on their way while the tile goes through LDS: one memory
+    // round trip.  (Requested where each is added, behind a branch, they were as many trips as vectors, up to eight.)
+    unsigned at[NV];
+    u32x4 addend[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int f = i * THREADS + tid, nl = f / GROUPS, g = f % GROUPS, n = n0 + nl, m = m0 + g * 8;
+        const bool ok = ((BN * GROUPS) % THREADS == 0 || f < BN * GROUPS) && n < p.N && m < pitch;
+        at[i] = ok ? (unsigned) (n * pitch + m) * 2u : OOB;
+        addend[i] = u32x4{0, 0, 0, 0};
+    }
+    if (with_res)   // uniform
+#pragma unroll
+        for (int i = 0; i < NV; ++i) addend[i] = __builtin_amdgcn_raw_buffer_load_b128(rr, at[i], 0, 0);
     // Table activations: the 8192 fp32 entries rounded to the output type, 16 KiB of LDS behind the staging area (the
     // caller leaves them free).  The value stored is round(table[i]) either way; the gathers then hit LDS instead of
     // sending 64 addresses per instruction to memory.
@@ -814,31 +832,22 @@ __device__ __forceinline__ void write_tile_nhwc_h16(const IgemmParams &p, f32x16
             }
         }
     __syncthreads();
-    constexpr int GROUPS = BM / 8;
     const rsrc_t rc = make_rsrc(p.C, RSRC_RANGE);
-    const rsrc_t rr = make_rsrc(p.res16, p.res16 ? RSRC_RANGE : 0u);
-    const int pitch = (int) p.c_stride_n;
-    const bool with_res = p.res16 != nullptr, relu = p.res_relu != 0;
 #pragma unroll
-    for (int f0 = 0; f0 < BN * GROUPS; f0 += THREADS) {
-        const int f = f0 + tid;
-        const int nl = f / GROUPS, g = f % GROUPS;
-        uint4 v = *reinterpret_cast<const uint4 *>(stage + nl * PITCH + g * 16);
-        const int n = n0 + nl, m = m0 + g * 8;
-        const bool ok = ((BN * GROUPS) % THREADS == 0 || f < BN * GROUPS) && n < p.N && m < pitch;
-        const unsigned off = ok ? (unsigned) (n * pitch + m) * 2u : OOB;
+    for (int i = 0; i < NV; ++i) {
+        const int f = i * THREADS + tid;
+        uint4 v = *reinterpret_cast<const uint4 *>(stage + f / GROUPS * PITCH + f % GROUPS * 16);
         if (with_res) {   // uniform
-            const u32x4 r = __builtin_amdgcn_raw_buffer_load_b128(rr, off, 0, 0);
             unsigned *w = reinterpret_cast<unsigned *>(&v);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float lo = __fadd_rn(unpack_h16<DT>(w[i], 0), unpack_h16<DT>(r[i], 0));
-                float hi = __fadd_rn(unpack_h16<DT>(w[i], 1), unpack_h16<DT>(r[i], 1));
+            for (int j = 0; j < 4; ++j) {
+                float lo = __fadd_rn(unpack_h16<DT>(w[j], 0), unpack_h16<DT>(addend[i][j], 0));
+                float hi = __fadd_rn(unpack_h16<DT>(w[j], 1), unpack_h16<DT>(addend[i][j], 1));
                 if (relu) { lo = lo > 0.0f ? lo : 0.0f; hi = hi > 0.0f ? hi : 0.0f; }
-                w[i] = pack_h16<DT>(lo, hi);
+                w[j] = pack_h16<DT>(lo, hi);
             }
         }
-        __builtin_amdgcn_raw_buffer_store_b128(u32x4{v.x, v.y, v.z, v.w}, rc, off, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(u32x4{v.x, v.y, v.z, v.w}, rc, at[i], 0, 0);
     }
 }
 
