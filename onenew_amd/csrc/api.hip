@@ -333,7 +333,7 @@ static const int kNumSplits = 13;
 // fin != 0 (with split > 1 or tail > 1): the slices of a tile are added up by the last of them to arrive, inside the
 // launch, instead of by a finishing launch (igemm_kernel, `arrive`)
 // dma != 0: the kernel that loads its operand tiles straight into LDS (igemm_dma_kernel.hpp), tile bm x bn, never split;
-// 1 = ring of stages within 64 KiB of LDS, 2 = the long ring
+// 1 = ring of stages within 64 KiB of LDS, 2 = the long ring, 3 = the one in between
 struct Choice { int bm, bn, split, tail, rowb, fin, dma; };
 
 static std::mutex g_tune_mu;
@@ -463,7 +463,7 @@ static const int kKwShapes[][3] = {{16, 16, 4}, {32, 32, 4}, {32, 32, 8}, {64, 3
 
 // (bm, bn) is a tile this build has a kernel for
 static bool tile_exists(const Choice &c) {
-    if (c.dma) return c.dma <= 2 && dma_tile_ok(c.bm, c.bn);
+    if (c.dma) return c.dma <= 3 && dma_tile_ok(c.bm, c.bn);
     if (c.rowb == 3) {
         for (const auto &k : kKwShapes)
             if (k[0] == c.bm && k[1] == c.bn && k[2] == c.split) return true;
@@ -496,7 +496,7 @@ static bool candidate_ok(const IgemmLaunch &cfg, const IgemmProblem &p, const Ch
     if (p.res && cfg.dtype == DT_I8 && (c.dma || c.split > 1 || c.tail > 1 || c.fin || c.rowb)) return false;
     if (c.dma) {
         static const bool off = getenv("ONHIP_NO_DMA") != nullptr;   // tuning hook: the register-staged kernel only
-        return (!off || h16) && c.split == 1 && c.tail <= 1 && !c.rowb && !c.fin && dma_ok(cfg, p);
+        return (!off || h16) && c.split == 1 && c.tail <= 1 && !c.rowb && !c.fin && dma_ok(cfg, p) && dma_ring_ok(cfg, p, c.bm, c.bn, c.dma - 1);
     }
     if (h16) return false;
     if (c.rowb == 3) return c.tail <= 1 && !c.fin && kw_ok(cfg, p, c.bm, kw_split(cfg, p));
@@ -567,8 +567,10 @@ static thread_local int tl_hint_bm = 0, tl_hint_bn = 0;
 // register-staged kernel, which has one.
 static bool dma_model_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out) {
     static const int order[4][2] = {{128, 128}, {128, 64}, {64, 128}, {64, 64}};
-    // what a tile's steady state costs per output against the largest one's (measured on the YOLOv8s layers)
-    static const double eff[4] = {1.0, 1.08, 1.10, 1.20};
+    // what a tile's steady state costs per output against the largest one's (measured on the YOLOv8s and, in bf16, the ResNet-50
+    // layers); up to two stages of K are mostly the tile's store, which takes as long per output in 64 x 128 (256 x 100352 x 64 in bf16
+    // with an Add 25.0 -> 23.2 us, 512 x 25088 x 128 17.8 -> 16.0, 17.0 in 128 x 64)
+    const double eff[4] = {1.0, 1.10, p.k_units <= 16 ? 1.0 : 1.08, 1.20};
     const bool only = cfg.dtype != DT_I8;   // the 16-bit types have no other kernel for these operands
     // int8 with a large fp32 result (the reference's W8A32 form on big planes): the register-staged kernel's store of
     // fp32 rows is the faster one from about 6.5 million outputs up (every such YOLOv8s layer at batch 16, 5-35 %)
@@ -589,7 +591,16 @@ static bool dma_model_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choi
         if (cost < best_cost) { best_cost = cost; best = t; }
     }
     if (best < 0) return false;
-    *out = Choice{order[best][0], order[best][1], 1, 0, 0, 0, 1};
+    // The ring by how many workgroups a compute unit gets.  Up to two wait for their loads (an L2 trip a stage with the short ring,
+    // which leaves room for three): in bf16 128 x 25088 x 1152 19.4 -> 16.0 us, 256 x 6272 x 2304 17.8 -> 16.4, in int8 128 x 25600 x
+    // 1152 13.7 -> 12.8.  A lone one takes all the LDS: 512 x 1568 x 4608 in bf16 27.0 -> 19.8 (21.3 with the ring in between), in int8
+    // 16.0 -> 12.3.  With more workgroups than that the third resident one is worth more (100352 columns: 20.1 against 22.8), and so it is
+    // with stages of 64 bytes.
+    const int bm = order[best][0], bn = order[best][1];
+    const long long tiles = (long long) ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
+    int dma = 1;
+    if (tiles <= 512 && dma_ring_ok(cfg, p, bm, bn, 2)) dma = tiles <= 256 && best == 3 ? 2 : 3;
+    *out = Choice{bm, bn, 1, 0, 0, 0, dma};
     return true;
 }
 
@@ -856,7 +867,7 @@ static int launch_choice(IgemmLaunch cfg, IgemmProblem p, const Choice &c, hipSt
     } note{cfg, p, c};
     if (c.dma) {
         cfg.bm = c.bm; cfg.bn = c.bn; cfg.split = 1;
-        cfg.ring = c.dma > 1;
+        cfg.ring = c.dma - 1;
         p.k_split_units = p.k_units;
         p.partial = nullptr;
         p.arrive = nullptr;
@@ -944,7 +955,7 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
         Choice c = {0, 0, 1, 0, 0, 0, 0};
         if (sscanf(env, "%dx%dx%dx%dx%dx%dx%d", &c.bm, &c.bn, &c.split, &c.tail, &c.rowb, &c.fin, &c.dma) >= 2) {
             if (cfg.dtype != DT_I8 && (cfg.bl == BL_KVEC || cfg.bl == BL_KVEC_TAP)) {   // 16-bit storage: one kernel, its tiles
-                c = {c.bm, c.bn, 1, 0, 0, 0, c.dma > 1 ? 2 : 1};
+                c = {c.bm, c.bn, 1, 0, 0, 0, c.dma > 1 ? c.dma : 1};
                 if (!candidate_ok(cfg, p, c)) c = model_choice(cfg, p);
             }
             if (c.dma && !candidate_ok(cfg, p, c)) {   // not a problem (or a tile) for that kernel: the register-staged one
@@ -1071,8 +1082,8 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
         }
     // the int8 kernel that loads its tiles straight into LDS
     static const int kDmaTiles[][2] = {{128, 128}, {128, 64}, {64, 128}, {64, 64}};
-    for (int t = 0; t < 8 && !rc; ++t) {
-        const Choice c = {kDmaTiles[t % 4][0], kDmaTiles[t % 4][1], 1, 0, 0, 0, 1 + t / 4};   // both ring lengths
+    for (int t = 0; t < 12 && !rc; ++t) {
+        const Choice c = {kDmaTiles[t % 4][0], kDmaTiles[t % 4][1], 1, 0, 0, 0, 1 + t / 4};   // every ring length
         if (candidate_ok(cfg, p, c)) try_choice(c);
     }
     (void) hipEventDestroy(e0);

@@ -13,6 +13,10 @@ bool dma_ok(const IgemmLaunch &cfg, const IgemmParams &p) {
     return dma_stage_bytes(p) != 0 || dma_multi_tap(cfg.dtype, p);
 }
 
+bool dma_ring_ok(const IgemmLaunch &cfg, const IgemmParams &p, int bm, int bn, int ring) {
+    return ring <= 1 || (ring == 2 && dma_stage_bytes(p) == 128 && !dma_multi_tap(cfg.dtype, p) && bm * bn < 128 * 128);
+}
+
 bool dma_tile_ok(int bm, int bn) {
     return (bm == 128 && bn == 128) || (bm == 128 && bn == 64) || (bm == 64 && bn == 128) || (bm == 64 && bn == 64);
 }

@@ -384,10 +384,14 @@ int dma_launch_dt(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t stre
         }
     }
     const int ks = dma_stage_bytes(p);
-    // cfg.ring != 0: the long rings, more than 64 KiB of LDS for one workgroup (one or two workgroups per compute unit,
-    // three to seven stages of loads in flight each); otherwise rings of at most 64 KiB
+    // cfg.ring == 1: the long rings, more than 64 KiB of LDS for one workgroup (one or two workgroups per compute unit,
+    // three to seven stages of loads in flight each); 2: rings of 64 to 72 KiB, two workgroups per compute unit with two or three
+    // stages in flight each, 128-byte stages only; otherwise rings of at most 64 KiB
     if (ks == 128) {
-        switch (key + (cfg.ring ? 1000000 : 0)) {
+        switch (key + cfg.ring * 1000000) {
+            case 2128064: return dma_launch_one<DT, 128, 64, 128, 3>(p, stream);
+            case 2064128: return dma_launch_one<DT, 64, 128, 128, 3>(p, stream);
+            case 2064064: return dma_launch_one<DT, 64, 64, 128, 4>(p, stream);
             case 128128: return dma_launch_one<DT, 128, 128, 128, 2>(p, stream);
             case 128064: return dma_launch_one<DT, 128, 64, 128, 2>(p, stream);
             case 64128: return dma_launch_one<DT, 64, 128, 128, 2>(p, stream);

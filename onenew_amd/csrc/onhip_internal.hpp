@@ -259,7 +259,7 @@ struct IgemmLaunch {
     int bm, bn;     // tile
     int batch;      // grid.z
     int split;      // grid.y
-    int ring;       // direct-to-LDS kernel: 0 = ring of stage buffers within 64 KiB of LDS, 1 = the long ring
+    int ring;       // direct-to-LDS kernel: 0 = ring of stage buffers within 64 KiB of LDS, 1 = the long ring, 2 = the one in between
 };
 
 int igemm_launch(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t stream);
@@ -299,6 +299,7 @@ int split_weights_launch(const float *w, int M, int K, long long s_row, long lon
 // padded channel count is a multiple of 64, tiles 128x128, 128x64, 64x128, 64x64, no split-K
 bool dma_ok(const IgemmLaunch &cfg, const IgemmParams &p);
 bool dma_tile_ok(int bm, int bn);
+bool dma_ring_ok(const IgemmLaunch &cfg, const IgemmParams &p, int bm, int bn, int ring);   // IgemmLaunch::ring of a problem dma_ok takes
 int dma_launch(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t stream);
 
 // ---- other kernels -------------------------------------------------------------------------------------
