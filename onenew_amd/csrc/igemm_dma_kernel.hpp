@@ -49,6 +49,8 @@ __device__ __forceinline__ void wait_operands(i32x4 (&av)[TM], i32x4 (&bv)[TN]) 
 }
 #endif
 
+__host__ __device__ inline bool dma_lone(unsigned workgroups) { return workgroups <= 256u; }   // one a compute unit at most
+
 template <int KS> __device__ __forceinline__ int dma_swz(int row) { return KS == 128 ? ((row >> 1) & 7) : ((row >> 2) & 3); }
 
 template <int DT, int BM, int BN, int WM, int WN, int KS, int NST, bool MULTI = false>
@@ -74,9 +76,15 @@ __global__ __launch_bounds__(THREADS) void igemm_dma_kernel(const IgemmParams p)
     // after the K loop the same memory holds the store's staging area, the quantised activation table and the per-row constants
     constexpr int OUT_STAGE = DT == DT_I8 ? BN * (BM + 16) : BN * (2 * BM + 16), ROWS_AT = OUT_STAGE + (DT == DT_I8 ? 8192 : 16384), OUT_BYTES = ROWS_AT + 2 * BM * 4;
     static_assert(ROWS_AT % 16 == 0, "the per-row constants are read 16 bytes at a time");
-    constexpr int LDS_BYTES = NST * STAGE > OUT_BYTES ? NST * STAGE : OUT_BYTES;
+    // stores of fp32 results through an activation table: the table, and the per-row constants behind it (not for the kernels of
+    // short taps, which would lose a resident workgroup to it)
+    constexpr bool TABLE = !MULTI;
+    constexpr int TABLE_ROWS = TABLE_BYTES + 2 * BM * 4;
+    constexpr int STORE_BYTES = TABLE && TABLE_ROWS > OUT_BYTES ? TABLE_ROWS : OUT_BYTES;
+    constexpr int LDS_BYTES = NST * STAGE > STORE_BYTES ? NST * STAGE : STORE_BYTES;
     __shared__ __attribute__((aligned(1024))) unsigned char lds[LDS_BYTES];
 
+    warm_params<IgemmParams>();
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 31, lh = lane >> 5;
@@ -91,40 +99,6 @@ __global__ __launch_bounds__(THREADS) void igemm_dma_kernel(const IgemmParams p)
     }
     const int tile_n = (int) div31((unsigned) lid, p.div_tiles_m), tile_m = lid - tile_n * tiles_m;
     const int m0 = tile_m * BM, n0 = tile_n * BN;
-
-    // the per-row constants of the epilogue, one row per thread, fetched while the first stages are on their way: the
-    // de-quantisation factor weight_aux / 127 (conv.c:1049-1056) and the int32 bias as a float
-    // (the 16-bit types have the fp32 bias alone)
-    float row_coeff = 0.0f, row_bias = 0.0f;
-    if (tid < BM) {
-        const int m = m0 + tid;
-        if constexpr (DT == DT_I8) {
-            const rsrc_t raux = make_rsrc(p.weight_aux, (unsigned) (p.M * 4));
-            const rsrc_t rb32 = make_rsrc(p.bias32, p.bias32 ? (unsigned) (p.M * 4) : 0u);
-            row_coeff = buf_load_f32(raux, (unsigned) m * 4u, 0);          // rows beyond M read as zero
-            row_bias = (float) (int) __builtin_amdgcn_raw_buffer_load_b32(rb32, (unsigned) m * 4u, 0, 0);
-        } else {
-            const rsrc_t rb = make_rsrc(p.bias, p.bias_mode == BIAS_M ? (unsigned) (p.M * 4) : 0u);
-            row_bias = buf_load_f32(rb, (unsigned) m * 4u, 0);
-        }
-    }
-
-    // the quantised activation table that the int8 NHWC store gathers from (8 KiB, 32 bytes per thread): requested here,
-    // before any operand load (being the oldest loads in flight, the K loop's counted waits cover them), and written
-    // to LDS behind the staging area once the K loop has left it, instead of a memory round trip plus a barrier of its own
-    // at the head of every tile's store
-    uint4 table_q[2] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
-    bool table_pre = false;
-    if constexpr (DT == DT_I8) {
-        table_pre = p.out_s8 && p.out_mode == OUT_PLAIN && p.c_stride_m == 1 && !p.acc_out && p.ep.qlut != nullptr &&
-                    (p.ep.act == SILU || p.ep.act == ONHIP_ACT_GELU_LUT);   // uniform
-        if (table_pre) {
-            const rsrc_t rq = make_rsrc(p.ep.qlut, 8192u);
-            table_q[0] = buf_load_b128(rq, (unsigned) tid * 16u, 0);
-            table_q[1] = buf_load_b128(rq, (unsigned) (tid + THREADS) * 16u, 0);
-        }
-    }
-    asm volatile("" ::: "memory");   // these loads stay ahead of the operand loads: the stage waits count loads in issue order
 
     const char *a_base = reinterpret_cast<const char *>(p.A);
     const char *b_base = reinterpret_cast<const char *>(p.B) - (size_t) p.b_shift_bytes;
@@ -213,6 +187,43 @@ __global__ __launch_bounds__(THREADS) void igemm_dma_kernel(const IgemmParams p)
 
 #pragma unroll
     for (int s = 0; s < NST - 1; ++s) issue(s, s);
+    // Behind the first stages (whose counted waits then cover these loads as well): the per-row constants of the epilogue, one row per
+    // thread, the de-quantisation factor weight_aux / 127 (conv.c:1049-1056) and the int32 bias as loaded, converted when the K loop
+    // is over; the 16-bit types have the fp32 bias alone.  Ahead of the first stages, and converted there, they were a trip to memory
+    // of their own at the start of every workgroup.
+    float row_coeff = 0.0f, row_bias = 0.0f;
+    int row_bias_int = 0;
+    if (tid < BM) {
+        const int m = m0 + tid;
+        if constexpr (DT == DT_I8) {
+            const rsrc_t raux = make_rsrc(p.weight_aux, (unsigned) (p.M * 4));
+            const rsrc_t rb32 = make_rsrc(p.bias32, p.bias32 ? (unsigned) (p.M * 4) : 0u);
+            row_coeff = buf_load_f32(raux, (unsigned) m * 4u, 0);          // rows beyond M read as zero
+            row_bias_int = (int) __builtin_amdgcn_raw_buffer_load_b32(rb32, (unsigned) m * 4u, 0, 0);
+        } else {
+            const rsrc_t rb = make_rsrc(p.bias, p.bias_mode == BIAS_M ? (unsigned) (p.M * 4) : 0u);
+            row_bias = buf_load_f32(rb, (unsigned) m * 4u, 0);
+        }
+    }
+    // the quantised activation table that the int8 NHWC store gathers from (8 KiB, 32 bytes per thread), written to LDS behind the
+    // staging area once the K loop has left it, instead of a memory round trip plus a barrier of its own at the head of every
+    // tile's store
+    uint4 table_q[2] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
+    bool table_pre = false;
+    if constexpr (DT == DT_I8) {
+        table_pre = p.out_s8 && p.out_mode == OUT_PLAIN && p.c_stride_m == 1 && !p.acc_out && p.ep.qlut != nullptr &&
+                    (p.ep.act == SILU || p.ep.act == ONHIP_ACT_GELU_LUT);   // uniform
+        if (table_pre) {
+            const rsrc_t rq = make_rsrc(p.ep.qlut, 8192u);
+            table_q[0] = buf_load_b128(rq, (unsigned) tid * 16u, 0);
+            table_q[1] = buf_load_b128(rq, (unsigned) (tid + THREADS) * 16u, 0);
+        }
+    }
+    // the table of a store of fp32 results: here where every workgroup has
+    // its compute unit's LDS to itself; behind the K loop, in the ring's memory, otherwise
+    extern __shared__ __attribute__((aligned(1024))) float s_table[];
+    const bool table = TABLE && table_in_lds(p), table_first = table && dma_lone(gridDim.x);   // uniform
+    if (table_first) request_table(p.ep.lut, s_table, wave, lane, THREADS);
 
     const unsigned lds0 = (unsigned) (size_t) (__attribute__((address_space(3))) unsigned char *) lds;
     unsigned a_addr[NSETS][TM][KSTEPS], b_addr[NSETS][TN][KSTEPS];
@@ -286,11 +297,13 @@ __global__ __launch_bounds__(THREADS) void igemm_dma_kernel(const IgemmParams p)
     // every wavefront done with the operand buffers, before the store reuses that memory
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    float *rows = reinterpret_cast<float *>(lds + ROWS_AT);
+    float *rows = reinterpret_cast<float *>(lds + (table ? TABLE_BYTES : ROWS_AT));
+    if (table && !table_first) request_table(p.ep.lut, reinterpret_cast<float *>(lds), wave, lane, THREADS);
     if (tid < BM) {
         if constexpr (DT == DT_I8) {
             rows[tid] = __fdiv_rn(row_coeff, 127.0f);
-            rows[BM + tid] = row_bias;
+            asm volatile("" : "+v"(row_bias_int));   // not converted any earlier, where it would be waited for
+            rows[BM + tid] = p.bias32 ? (float) row_bias_int : -0.0f;   // the addend that changes nothing
         } else {
             rows[tid] = row_bias;
         }
@@ -303,6 +316,7 @@ __global__ __launch_bounds__(THREADS) void igemm_dma_kernel(const IgemmParams p)
             if (tid == 0) ql[-1] = 0;                   // its "below the table" entry
         }
     }
+    if (table) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
 
     const int m_wave = m0 + wm * (BM / WM), n_wave = n0 + wn * (BN / WN);
@@ -339,7 +353,7 @@ __global__ __launch_bounds__(THREADS) void igemm_dma_kernel(const IgemmParams p)
         case RELU: write_tile<DT, EPI_RELU, TM, TN, false, DT == DT_I8>(p, acc, 0, m_wave, n_wave, li, lh, rows + (m_wave - m0), rows + BM + (m_wave - m0)); break;
         case CLIP: write_tile<DT, EPI_CLIP, TM, TN, false, DT == DT_I8>(p, acc, 0, m_wave, n_wave, li, lh, rows + (m_wave - m0), rows + BM + (m_wave - m0)); break;
         case SILU:
-        case ONHIP_ACT_GELU_LUT: write_tile<DT, EPI_LUT, TM, TN, false, DT == DT_I8>(p, acc, 0, m_wave, n_wave, li, lh, rows + (m_wave - m0), rows + BM + (m_wave - m0)); break;
+        case ONHIP_ACT_GELU_LUT: write_tile<DT, EPI_LUT, TM, TN, false, DT == DT_I8, TABLE>(p, acc, 0, m_wave, n_wave, li, lh, rows + (m_wave - m0), rows + BM + (m_wave - m0), nullptr, 0, table_first ? (lds_f32_t) s_table : (lds_f32_t) reinterpret_cast<float *>(lds)); break;
         default: write_tile<DT, EPI_GENERIC, TM, TN, false, DT == DT_I8>(p, acc, 0, m_wave, n_wave, li, lh, rows + (m_wave - m0), rows + BM + (m_wave - m0)); break;
     }
 #endif
@@ -364,7 +378,8 @@ int dma_launch_one(const IgemmParams &p_in, hipStream_t stream) {
     p.div_ohw = make_div31((unsigned) (p.OHW > 0 ? p.OHW : 1));
     p.div_ow = make_div31((unsigned) (p.OW > 0 ? p.OW : 1));
     p.div_tiles_m = make_div31((unsigned) tiles_m);
-    hipLaunchKernelGGL((igemm_dma_kernel<DT, BM, BN, 2, 2, KS, NST, MULTI>), dim3((unsigned) tiles), dim3(THREADS), 0, stream, p);
+    hipLaunchKernelGGL((igemm_dma_kernel<DT, BM, BN, 2, 2, KS, NST, MULTI>), dim3((unsigned) tiles), dim3(THREADS),
+                       !MULTI && dma_lone((unsigned) tiles) ? table_lds_bytes(p) : 0u, stream, p);
     ONHIP_CHECK_HIP(hipGetLastError());
     return ONHIP_OK;
 }

@@ -203,7 +203,7 @@ __device__ __forceinline__ void unscale_fix_nonfinite(const IgemmProblem &p, f32
 // as in write_tile.
 template <int EPI, int TM, int TN, bool RES>
 __device__ __forceinline__ void write_tile_rows(const IgemmProblem &p, f32x16 (&acc)[TM][TN], int m_wave, int n_wave, int li, int lh,
-                                                const float *sbias) {
+                                                const float *sbias, lds_f32_t table) {
     const rsrc_t rc = make_rsrc(p.C, (unsigned) p.c_slice_bytes), rr = make_rsrc(RES ? p.res : nullptr, RES ? (unsigned) p.c_slice_bytes : 0u);
 #pragma unroll
     for (int b = 0; b < TN; ++b) {
@@ -220,12 +220,15 @@ __device__ __forceinline__ void write_tile_rows(const IgemmProblem &p, f32x16 (&
             for (int q = 0; q < 4; ++q) {
                 const float4 bias = *reinterpret_cast<const float4 *>(sbias + a * 32 + 8 * q + 4 * lh);
                 const float bv[4] = {bias.x, bias.y, bias.z, bias.w};
+                float v[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[j] = __fadd_rn(acc[a][b][4 * q + j], bv[j]);
+                act_store<EPI, true>(v, p.ep, table);
                 u32x4 o;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    float v = act_fast<EPI>(__fadd_rn(acc[a][b][4 * q + j], bv[j]), p.ep);
-                    if constexpr (RES) v = __fadd_rn(v, __uint_as_float(rv[q][j]));
-                    o[j] = __float_as_uint(v);
+                    if constexpr (RES) v[j] = __fadd_rn(v[j], __uint_as_float(rv[q][j]));
+                    o[j] = __float_as_uint(v[j]);
                 }
                 const int left = p.M - (m4 + 8 * q);   // columns of C from this group on
                 if (left >= 4) {
@@ -252,10 +255,14 @@ void igemm_f3_kernel(const IgemmProblem p) {
     __shared__ uint4 lds[2 * SLOTS];   // two K tiles
     __shared__ __attribute__((aligned(16))) float s_bias[BM];
 
+    warm_params<IgemmProblem>();
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 31, lh = lane >> 5;
     const int wm = wave / WN, wn = wave % WN;
+
+    extern __shared__ __attribute__((aligned(1024))) float s_table[];   // TABLE_BYTES where table_in_lds says so
+    if (table_in_lds(p)) request_table(p.ep.lut, s_table, wave, lane, NT);
 
     const TilePlace tp = place_tile<BM, BN>(p);
     const int m0 = tp.m0, n0 = tp.n0, slice = tp.slice;
@@ -418,8 +425,8 @@ void igemm_f3_kernel(const IgemmProblem p) {
     const float *sb = s_bias + wm * (BM / WM);
     auto store = [&](auto epi) __attribute__((always_inline)) {
         constexpr int EPI = decltype(epi)::value;
-        if constexpr (BL == BL_ROWS) write_tile_rows<EPI, TM, TN, RES>(p, acc, m_wave, n_wave, li, lh, sb);
-        else write_tile<DT_F32, EPI, TM, TN, RES, true>(p, acc, 0, m_wave, n_wave, li, lh, sb);
+        if constexpr (BL == BL_ROWS) write_tile_rows<EPI, TM, TN, RES>(p, acc, m_wave, n_wave, li, lh, sb, (lds_f32_t) s_table);
+        else write_tile<DT_F32, EPI, TM, TN, RES, true, true>(p, acc, 0, m_wave, n_wave, li, lh, sb, nullptr, nullptr, 0, (lds_f32_t) s_table);
     };
     switch (p.ep.act) {
         case NOT_ACT:
@@ -439,7 +446,7 @@ static int f3_launch_one(const IgemmLaunch &cfg, const IgemmProblem &p_in, hipSt
     const int rc = tile_grid<BM, BN>(cfg, p, &grid);
     if (rc) return rc;
     if (RES != (p.res != nullptr)) return set_error(ONHIP_ERR_ARG, "igemm: residual operand and kernel variant do not match");
-    hipLaunchKernelGGL((igemm_f3_kernel<BL, BM, BN, WM, WN, RES>), grid, dim3(64 * WM * WN), 0, stream, p);
+    hipLaunchKernelGGL((igemm_f3_kernel<BL, BM, BN, WM, WN, RES>), grid, dim3(64 * WM * WN), table_lds_bytes(p), stream, p);
     ONHIP_CHECK_HIP(hipGetLastError());
     return finish_launch<false>(cfg, p, stream);
 }

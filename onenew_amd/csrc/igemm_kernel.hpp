@@ -67,6 +67,21 @@ __device__ __forceinline__ uint4 buf_load_b128(rsrc_t r, unsigned voff, unsigned
     return make_uint4(q.x, q.y, q.z, q.w);
 }
 
+// The kernel's parameters into the scalar cache, all of their lines at once.  A kernel reads its few hundred bytes of parameters where
+// it needs them, a scalar load and a wait at a time, and each first touch of a 64-byte line is a trip to memory: six to nine of
+// them one after the other stood in front of the first operand load.
+template <class P>
+__device__ __forceinline__ void warm_params() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const auto *k = (const __attribute__((address_space(4))) unsigned *) __builtin_amdgcn_kernarg_segment_ptr();
+    constexpr int LAST = (int) (sizeof(P) / 4) - 1;
+    auto at = [](int line) { return 16 * line < LAST ? 16 * line : LAST; };
+    static_assert(sizeof(P) <= 10 * 64, "ten lines");
+    asm volatile("" :: "s"(k[at(0)]), "s"(k[at(1)]), "s"(k[at(2)]), "s"(k[at(3)]), "s"(k[at(4)]), "s"(k[at(5)]), "s"(k[at(6)]), "s"(k[at(7)]),
+                 "s"(k[at(8)]), "s"(k[at(9)]));
+#endif
+}
+
 template <int DT> struct Traits;
 // mma_part: one MFMA instruction of the PARTS that consume a pair of 16-byte units
 template <> struct Traits<DT_F32> {
@@ -295,6 +310,47 @@ __device__ __forceinline__ unsigned b_voff(const IgemmParams &p, const ColState 
 }
 
 // ---- epilogue ----------------------------------------------------------------------------------------
+// The 8192-entry table of a table activation in LDS, for stores of fp32 results: a gather from memory takes the compute unit a
+// cycle per cache line, about 45 of a wavefront's 64 addresses, one from LDS about eight; a 128 x 64 tile makes 128 of them.  The
+// launcher gives the kernel the memory (table_lds_bytes) where its workgroups store such results; the kernel requests the table
+// ahead of everything else, so its operand loads cover the trip.
+constexpr int TABLE_BYTES = 8192 * 4;
+typedef const __attribute__((address_space(3))) float *lds_f32_t;
+__host__ __device__ inline bool table_in_lds(const IgemmParams &p) {
+    const bool int8_rows = p.out_s8 && p.out_mode == OUT_PLAIN && p.c_stride_m == 1 && !p.acc_out;   // has the quantised table
+    const bool slices_only = p.partial && !p.arrive && p.dp_tiles == 0;
+    return (p.ep.act == SILU || p.ep.act == ONHIP_ACT_GELU_LUT) && !int8_rows && !p.out_h16 && !slices_only;
+}
+inline unsigned table_lds_bytes(const IgemmParams &p) { return table_in_lds(p) ? TABLE_BYTES : 0u; }
+// every wavefront of the workgroup (nt threads) takes its share; complete once its loads are (vmcnt) and a barrier has passed
+__device__ __forceinline__ void request_table(const float *lut, float *table, int wave, int lane, int nt) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const rsrc_t rt = make_rsrc(lut, TABLE_BYTES);
+    for (int c = wave; c < TABLE_BYTES / 1024; c += nt / 64)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rt, (__attribute__((address_space(3))) void *) (table + c * 256), 16, (unsigned) lane * 16u,
+                                                 (unsigned) c * 1024u, 0, 0);
+#endif
+}
+// act_fast of N values, with the table there: the reads of all of them are on their way before the first is used.  (volatile: left
+// alone, the compiler makes each read a branch of its own for values below the table, with a wait behind it.)
+template <int EPI, bool TABLE, int N>
+__device__ __forceinline__ void act_store(float (&v)[N], const Epilogue &e, lds_f32_t table) {
+    if constexpr (EPI == EPI_LUT && TABLE) {
+        float l[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            int idx = (int) __fmul_rn(__fadd_rn(v[i], 8.0f), 512.0f);
+            idx = idx < 0 ? 0 : idx > 8191 ? 8191 : idx;
+            l[i] = *(const volatile __attribute__((address_space(3))) float *) (table + idx);
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = v[i] < -8.0f ? 0.0f : v[i] >= 8.0f ? v[i] : l[i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = act_fast<EPI>(v[i], e);
+    }
+}
+
 // byte offset of column n inside one batch slice of C (rows are added through the scalar offset)
 __device__ __forceinline__ unsigned out_col_offset(const IgemmParams &p, int n, int esz) {
     if (p.out_mode == OUT_CONV) {
@@ -326,10 +382,11 @@ __device__ __forceinline__ int requant_s8(float y, float inv_scale) {
 // and srow2 the int32 biases as floats.
 // twin_at (int8 with a residual operand): LDS for the tile's int8 form, [column of the tile][twin_ld bytes], at this wavefront's
 // first column and row; store_twin writes it out.
-template <int DT, int EPI, int TM, int TN, bool RES, bool BIAS_LDS = false, class ACC>
+// TABLE: the table of a table activation waits in LDS.
+template <int DT, int EPI, int TM, int TN, bool RES, bool BIAS_LDS = false, bool TABLE = false, class ACC>
 __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][TN], int batch, int m_wave, int n_wave,
                                            int li, int lh, const float *sbias = nullptr, const float *srow2 = nullptr,
-                                           unsigned char *twin_at = nullptr, int twin_ld = 0) {
+                                           unsigned char *twin_at = nullptr, int twin_ld = 0, lds_f32_t table = nullptr) {
     const int esz = (DT == DT_I8 && p.out_s8) ? 1 : 4;
     const rsrc_t rc = make_rsrc(reinterpret_cast<const char *>(p.C) + (size_t) batch * p.c_batch_stride * esz,
                                 RSRC_RANGE);
@@ -375,7 +432,8 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
                 for (int r = 0; r < 16; ++r) {
                     const unsigned soff = (unsigned) (m_wave + a * 32 + 8 * (r / 4) + (r % 4)) * 4u;
                     aux[a][r] = buf_load_f32(raux, lh16, soff);
-                    fb32[a][r] = (float) (int) __builtin_amdgcn_raw_buffer_load_b32(rb32, lh16, soff, 0);
+                    const float fb = (float) (int) __builtin_amdgcn_raw_buffer_load_b32(rb32, lh16, soff, 0);
+                    fb32[a][r] = p.bias32 ? fb : -0.0f;   // the addend that changes nothing
                 }
 #pragma unroll
             for (int a = 0; a < TM; ++a)
@@ -391,66 +449,82 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
         // RES: the residual operand of a folded Add (fp32 results): a row tile's addends are requested together
         const rsrc_t rres = make_rsrc(RES ? reinterpret_cast<const char *>(p.res) + (size_t) batch * p.c_batch_stride * 4 : nullptr,
                                       RES ? RSRC_RANGE : 0u);
-        unsigned tq[TN][4];
+        // What is the same for all values of a launch is decided once, out here: the tile at the edge of M (rows are tested), whether
+        // the result is fp32 and nothing else (no raw accumulators, no int8), whether the int8 twin is wanted.  Asked per value they
+        // were three branches and some forty instructions each, 16 values a lane.
+        auto store = [&](auto edge, auto fp32_only, auto twin) __attribute__((always_inline)) {
+            constexpr bool EDGE = decltype(edge)::value, FP32 = decltype(fp32_only)::value, TWIN = decltype(twin)::value;
+            unsigned tq[TN][4];
 #pragma unroll
-        for (int b = 0; b < TN; ++b)
+            for (int a = 0; a < TM; ++a) {
+                float rv[RES ? 16 : 1][RES ? TN : 1];
+                if constexpr (RES) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) tq[b][j] = 0;
+                    for (int r = 0; r < 16; ++r) {
+                        const int m_uni = m_wave + a * 32 + 8 * (r / 4) + (r % 4);
+                        const bool row_ok = !EDGE || m_uni + 4 * lh < p.M;
 #pragma unroll
-        for (int a = 0; a < TM; ++a) {
-            float rv[RES ? 16 : 1][RES ? TN : 1];
-            if constexpr (RES) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m_uni = m_wave + a * 32 + 8 * (r / 4) + (r % 4);
-                    const bool row_ok = !m_edge || m_uni + 4 * lh < p.M;
-#pragma unroll
-                    for (int b = 0; b < TN; ++b) rv[r][b] = buf_load_f32(rres, row_ok ? col_voff[b] : OOB, (unsigned) m_uni * row_bytes);
+                        for (int b = 0; b < TN; ++b) rv[r][b] = buf_load_f32(rres, row_ok ? col_voff[b] : OOB, (unsigned) m_uni * row_bytes);
+                    }
                 }
-            }
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m_uni = m_wave + a * 32 + 8 * (r / 4) + (r % 4);
-                const bool row_ok = !m_edge || m_uni + 4 * lh < p.M;
-                // conv.c:1041-1056: acc * s, + bias, * (aux / 127): three separately rounded operations
-                const float coeff = aux[a][r];
-                const float fb = fb32[a][r];
+                for (int q = 0; q < 4; ++q) {
+                    const int m_uni = m_wave + a * 32 + 8 * q;   // first of the group of four rows, of lanes with lh == 0
+                    float y[4 * TN];
 #pragma unroll
-                for (int b = 0; b < TN; ++b) {
-                    const int av = acc[a][b][r];
-                    if (p.acc_out)
-                        __builtin_amdgcn_raw_buffer_store_b32((unsigned) av, racc, row_ok ? col_voff4[b] : OOB,
-                                                              (unsigned) m_uni * row_bytes4, 0);
-                    float f = __fmul_rn((float) av, p.in_scale);
-                    const float fbias = __fadd_rn(f, fb);
-                    f = p.bias32 ? fbias : f;
-                    float y = act_fast<EPI>(__fmul_rn(f, coeff), p.ep);
-                    if constexpr (RES) {
-                        y = add_res(y, rv[r][b], p.res_relu, (col_voff[b] + (unsigned) m_uni * row_bytes) >> 2, p.res_body);
-                        // the int8 twin: registers 4 q .. 4 q + 3 are four consecutive channels of the lane's pixel.  The
-                        // quantiser's product and clamp as a multiply and a median of three (a NaN comes out as -128 here
-                        // and as 0 from the comparisons of requant_s8; no finite operand produces one), the four low
-                        // bytes packed with three byte permutes
-                        if (p.twin) {   // uniform
-                            tq[b][r % 4] = (unsigned) round_half_away_small(
-                                __builtin_amdgcn_fmed3f(__fmul_rn(y, p.twin_inv_scale), -128.0f, 127.0f));
-                            if (r % 4 == 3) {
-                                const unsigned p01 = __builtin_amdgcn_perm(tq[b][1], tq[b][0], 0x0c0c0400u);
-                                const unsigned p23 = __builtin_amdgcn_perm(tq[b][3], tq[b][2], 0x0c0c0400u);
-                                *reinterpret_cast<unsigned *>(twin_at + (b * 32 + li) * twin_ld + a * 32 + 8 * (r / 4) + 4 * lh) =
-                                    __builtin_amdgcn_perm(p23, p01, 0x05040100u);
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int b = 0; b < TN; ++b) {
+                            // conv.c:1041-1056: acc * s, + bias, * (aux / 127): three separately rounded operations
+                            const float f = __fadd_rn(__fmul_rn((float) acc[a][b][4 * q + j], p.in_scale), fb32[a][4 * q + j]);
+                            y[j * TN + b] = __fmul_rn(f, aux[a][4 * q + j]);
+                        }
+                    act_store<EPI, TABLE>(y, p.ep, table);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const bool row_ok = !EDGE || m_uni + j + 4 * lh < p.M;
+#pragma unroll
+                        for (int b = 0; b < TN; ++b) {
+                            if constexpr (!FP32)
+                                if (p.acc_out)
+                                    __builtin_amdgcn_raw_buffer_store_b32((unsigned) acc[a][b][4 * q + j], racc, row_ok ? col_voff4[b] : OOB,
+                                                                          (unsigned) (m_uni + j) * row_bytes4, 0);
+                            float v = y[j * TN + b];
+                            if constexpr (RES) {
+                                v = add_res(v, rv[4 * q + j][b], p.res_relu, (col_voff[b] + (unsigned) (m_uni + j) * row_bytes) >> 2, p.res_body);
+                                // the int8 twin: registers 4 q .. 4 q + 3 are four consecutive channels of the lane's pixel.  The
+                                // quantiser's product and clamp as a multiply and a median of three (a NaN comes out as -128 here
+                                // and as 0 from the comparisons of requant_s8; no finite operand produces one), the four low
+                                // bytes packed with three byte permutes
+                                if constexpr (TWIN) {
+                                    tq[b][j] = (unsigned) round_half_away_small(
+                                        __builtin_amdgcn_fmed3f(__fmul_rn(v, p.twin_inv_scale), -128.0f, 127.0f));
+                                    if (j == 3) {
+                                        const unsigned p01 = __builtin_amdgcn_perm(tq[b][1], tq[b][0], 0x0c0c0400u);
+                                        const unsigned p23 = __builtin_amdgcn_perm(tq[b][3], tq[b][2], 0x0c0c0400u);
+                                        *reinterpret_cast<unsigned *>(twin_at + (b * 32 + li) * twin_ld + a * 32 + 8 * q + 4 * lh) =
+                                            __builtin_amdgcn_perm(p23, p01, 0x05040100u);
+                                    }
+                                }
                             }
+                            const unsigned voff = row_ok ? col_voff[b] : OOB;
+                            if (!FP32 && p.out_s8)
+                                __builtin_amdgcn_raw_buffer_store_b8((unsigned char) requant_s8(v, p.out_inv_scale), rc, voff,
+                                                                     (unsigned) (m_uni + j) * row_bytes, 0);
+                            else
+                                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rc, voff, (unsigned) (m_uni + j) * row_bytes, 0);
                         }
                     }
-                    const unsigned voff = row_ok ? col_voff[b] : OOB;
-                    if (p.out_s8)
-                        __builtin_amdgcn_raw_buffer_store_b8((unsigned char) requant_s8(y, p.out_inv_scale), rc, voff,
-                                                             (unsigned) m_uni * row_bytes, 0);
-                    else
-                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), rc, voff, (unsigned) m_uni * row_bytes, 0);
                 }
             }
-        }
+        };
+        auto kind = [&](auto twin) __attribute__((always_inline)) {
+            if (p.acc_out || p.out_s8) store(std::true_type{}, std::false_type{}, twin);
+            else if (m_edge) store(std::true_type{}, std::true_type{}, twin);
+            else store(std::false_type{}, std::true_type{}, twin);
+        };
+        if (RES && p.twin) kind(std::bool_constant<RES>{});
+        else kind(std::false_type{});
     } else {
         float rv[RES ? TM : 1][RES ? 16 : 1][RES ? TN : 1];
         if constexpr (RES) {
@@ -492,18 +566,26 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
 #pragma unroll
             for (int a = 0; a < TM; ++a)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m_uni = m_wave + a * 32 + 8 * (r / 4) + (r % 4);   // row of lanes with lh == 0
-                    const bool row_ok = !EDGE || m_uni + 4 * lh < p.M;
+                for (int q = 0; q < 4; ++q) {
+                    float y[4 * TN];
 #pragma unroll
-                    for (int b = 0; b < TN; ++b) {
-                        // bias after the full sum
-                        float v = __fadd_rn(acc[a][b][r], (BIAS_LDS ? !bias_n_on : bias_m_on) ? bias_m[a][r] : bias_sel[b]);
-                        v = act_fast<EPI>(v, p.ep);
-                        if constexpr (RES)
-                            v = add_res(v, rv[a][r][b], p.res_relu, (col_voff[b] + (unsigned) m_uni * row_bytes) >> 2, p.res_body);
-                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rc, row_ok ? col_voff[b] : OOB,
-                                                              (unsigned) m_uni * row_bytes, 0);
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int b = 0; b < TN; ++b)   // bias after the full sum
+                            y[j * TN + b] = __fadd_rn(acc[a][b][4 * q + j], (BIAS_LDS ? !bias_n_on : bias_m_on) ? bias_m[a][4 * q + j] : bias_sel[b]);
+                    act_store<EPI, TABLE>(y, p.ep, table);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int r = 4 * q + j, m_uni = m_wave + a * 32 + 8 * q + j;   // row of lanes with lh == 0
+                        const bool row_ok = !EDGE || m_uni + 4 * lh < p.M;
+#pragma unroll
+                        for (int b = 0; b < TN; ++b) {
+                            float v = y[j * TN + b];
+                            if constexpr (RES)
+                                v = add_res(v, rv[a][r][b], p.res_relu, (col_voff[b] + (unsigned) m_uni * row_bytes) >> 2, p.res_body);
+                            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rc, row_ok ? col_voff[b] : OOB,
+                                                                  (unsigned) m_uni * row_bytes, 0);
+                        }
                     }
                 }
         };
@@ -1123,11 +1205,15 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(PW2 ? 4
     constexpr bool BIAS_LDS = true;
     __shared__ __attribute__((aligned(16))) float s_bias[DT == DT_I8 ? 2 * BM : BM];
 
+    warm_params<IgemmParams>();
     const int tid = threadIdx.x;
     // the wavefront index is uniform; saying so keeps everything derived from it in scalar registers
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 31, lh = lane >> 5;
     const int wm = wave / WN, wn = wave % WN;
+
+    extern __shared__ __attribute__((aligned(1024))) float s_table[];   // TABLE_BYTES where table_in_lds says so
+    if (!PW2 && table_in_lds(p)) request_table(p.ep.lut, s_table, wave, lane, THREADS);
 
     const TilePlace tp = place_tile<BM, BN>(p);
     const int m0 = tp.m0, n0 = tp.n0, slice = tp.slice, lid = tp.lid;
@@ -1326,12 +1412,13 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(PW2 ? 4
     }(std::make_integer_sequence<int, PF>{});
     // the tile's bias rows, behind the first operand loads (nothing waits for them before the K loop is over)
     float bias_row = -0.0f;   // the addend that changes nothing
+    int bias_int = 0;         // int8: as loaded; the conversion would wait for it here
     float aux_row = 0.0f;
     {
         const unsigned row_off = tid < BM ? (unsigned) (m0 + tid) * 4u : OOB;   // rows beyond M read as zero
         if constexpr (DT == DT_I8) {
             aux_row = buf_load_f32(make_rsrc(p.weight_aux, p.weight_aux ? (unsigned) (p.M * 4) : 0u), row_off, 0);
-            bias_row = (float) (int) __builtin_amdgcn_raw_buffer_load_b32(make_rsrc(p.bias32, p.bias32 ? (unsigned) (p.M * 4) : 0u), row_off, 0, 0);
+            bias_int = (int) __builtin_amdgcn_raw_buffer_load_b32(make_rsrc(p.bias32, p.bias32 ? (unsigned) (p.M * 4) : 0u), row_off, 0, 0);
         } else {
             const bool on = p.bias_mode == BIAS_M;
             const float bv = buf_load_f32(make_rsrc(p.bias, on ? (unsigned) (p.M * 4) : 0u), row_off, 0);
@@ -1389,7 +1476,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(PW2 ? 4
     if (tid < BM) {
         if constexpr (DT == DT_I8) {
             s_bias[tid] = __fdiv_rn(aux_row, 127.0f);   // conv.c:1049-1056: the factor is weight_aux / 127, rounded once
-            s_bias[BM + tid] = bias_row;
+            asm volatile("" : "+v"(bias_int));   // not converted any earlier, where it would be waited for
+            s_bias[BM + tid] = p.bias32 ? (float) bias_int : -0.0f;   // the addend that changes nothing
         } else {
             s_bias[tid] = bias_row;
         }
@@ -1450,7 +1538,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(PW2 ? 4
         case RELU: write_tile<DT, EPI_RELU, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM), twin_at, BM + 16); break;
         case CLIP: write_tile<DT, EPI_CLIP, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM), twin_at, BM + 16); break;
         case SILU:
-        case ONHIP_ACT_GELU_LUT: write_tile<DT, EPI_LUT, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM), twin_at, BM + 16); break;
+        case ONHIP_ACT_GELU_LUT: write_tile<DT, EPI_LUT, TM, TN, RES, BIAS_LDS, true>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM), twin_at, BM + 16, (lds_f32_t) s_table); break;
         default: write_tile<DT, EPI_GENERIC, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM), twin_at, BM + 16); break;
     }
     if constexpr (DT == DT_I8 && RES)
@@ -1571,7 +1659,7 @@ static int launch_one(const IgemmLaunch &cfg, const IgemmParams &p_in, hipStream
     const int rc = tile_grid<BM, BN>(cfg, p, &grid);
     if (rc) return rc;
     if (RES != (p.res != nullptr)) return set_error(ONHIP_ERR_ARG, "igemm: residual operand and kernel variant do not match");
-    hipLaunchKernelGGL((igemm_kernel<DT, BL, BM, BN, WM, WN, PF, RES>), grid, dim3(THREADS), 0, stream, p);
+    hipLaunchKernelGGL((igemm_kernel<DT, BL, BM, BN, WM, WN, PF, RES>), grid, dim3(THREADS), table_lds_bytes(p), stream, p);
     ONHIP_CHECK_HIP(hipGetLastError());
     return finish_launch<DT == DT_I8>(cfg, p, stream);
 }
