@@ -84,7 +84,7 @@ __global__ __launch_bounds__(THREADS) void igemm_dma_kernel(const IgemmParams p)
     constexpr int LDS_BYTES = NST * STAGE > STORE_BYTES ? NST * STAGE : STORE_BYTES;
     __shared__ __attribute__((aligned(1024))) unsigned char lds[LDS_BYTES];
 
-    warm_params<IgemmParams>();
+    warm_params<sizeof(IgemmParams)>();
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 31, lh = lane >> 5;

@@ -255,7 +255,7 @@ void igemm_f3_kernel(const IgemmProblem p) {
     __shared__ uint4 lds[2 * SLOTS];   // two K tiles
     __shared__ __attribute__((aligned(16))) float s_bias[BM];
 
-    warm_params<IgemmProblem>();
+    warm_params<sizeof(IgemmProblem)>();
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 31, lh = lane >> 5;

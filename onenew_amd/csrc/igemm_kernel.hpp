@@ -67,21 +67,6 @@ __device__ __forceinline__ uint4 buf_load_b128(rsrc_t r, unsigned voff, unsigned
     return make_uint4(q.x, q.y, q.z, q.w);
 }
 
-// The kernel's parameters into the scalar cache, all of their lines at once.  A kernel reads its few hundred bytes of parameters where
-// it needs them, a scalar load and a wait at a time, and each first touch of a 64-byte line is a trip to memory: six to nine of
-// them one after the other stood in front of the first operand load.
-template <class P>
-__device__ __forceinline__ void warm_params() {
-#if defined(__HIP_DEVICE_COMPILE__)
-    const auto *k = (const __attribute__((address_space(4))) unsigned *) __builtin_amdgcn_kernarg_segment_ptr();
-    constexpr int LAST = (int) (sizeof(P) / 4) - 1;
-    auto at = [](int line) { return 16 * line < LAST ? 16 * line : LAST; };
-    static_assert(sizeof(P) <= 10 * 64, "ten lines");
-    asm volatile("" :: "s"(k[at(0)]), "s"(k[at(1)]), "s"(k[at(2)]), "s"(k[at(3)]), "s"(k[at(4)]), "s"(k[at(5)]), "s"(k[at(6)]), "s"(k[at(7)]),
-                 "s"(k[at(8)]), "s"(k[at(9)]));
-#endif
-}
-
 template <int DT> struct Traits;
 // mma_part: one MFMA instruction of the PARTS that consume a pair of 16-byte units
 template <> struct Traits<DT_F32> {
@@ -1205,7 +1190,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(PW2 ? 4
     constexpr bool BIAS_LDS = true;
     __shared__ __attribute__((aligned(16))) float s_bias[DT == DT_I8 ? 2 * BM : BM];
 
-    warm_params<IgemmParams>();
+    warm_params<sizeof(IgemmParams)>();
     const int tid = threadIdx.x;
     // the wavefront index is uniform; saying so keeps everything derived from it in scalar registers
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);

@@ -51,7 +51,7 @@ __global__ __launch_bounds__(64 * NW) void igemm_kw_kernel(const IgemmProblem p)
     __shared__ float s_sum[NW * VALS];            // [wavefront][row block][register][lane]
     __shared__ int s_again;
 
-    warm_params<IgemmProblem>();
+    warm_params<sizeof(IgemmProblem)>();
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lc = lane % T, lg = lane / T;

@@ -163,8 +163,10 @@ def _ptr(t):
 
 
 def _stream():
+    """handle of the calling thread's current stream on its current device; without the Stream object that torch.cuda.current_stream()
+    makes around it, 2.9 us of a call that takes 8"""
     import torch
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def init(device=0):
