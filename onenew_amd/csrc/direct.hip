@@ -1,6 +1,5 @@
 // Bandwidth-bound kernels where MFMA does not pay: depthwise convolution (fp32 and W8A32), the
-// activation quantiser that stages NCHW fp32 as NHWC int8 for the int8 MFMA path, the int8 weight
-// re-layout, and the skinny Gemm  out = A * W^T + bias  with a wavefront-shuffle reduction.
+// activation quantiser that stages NCHW fp32 as NHWC int8 for the int8 MFMA path and the int8 weight re-layout.
 #include "onhip_internal.hpp"
 
 namespace onhip {
@@ -127,57 +126,6 @@ __global__ __launch_bounds__(256) void build_qlut_kernel(const float *__restrict
 
 int build_qlut_launch(const float *lut, float out_inv_scale, signed char *qlut, hipStream_t stream) {
     hipLaunchKernelGGL(build_qlut_kernel, dim3(32), dim3(256), 0, stream, lut, out_inv_scale, qlut);
-    ONHIP_CHECK_HIP(hipGetLastError());
-    return ONHIP_OK;
-}
-
-// ---- skinny Gemm: out[m][n] = sum_k a[m][k] * w[n][k] + bias[n]  (device/x86/Gemm/gemm.c:9-79) ---------
-// One wavefront per output column n; lanes stride over k, eight rows of A at a time share each
-// weight load; butterfly reduction over the 64 lanes; the bias is added last.
-constexpr int GEMM_ROWS = 8;
-__global__ __launch_bounds__(256) void gemm_nt_kernel(int M, int K, int N, const float *a, const float *w,
-                                                      const float *bias, float *out, int vec) {
-    const int lane = threadIdx.x & 63;
-    const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (n >= N) return;
-    const float *wr = w + (long long) n * K;
-    for (int m0 = 0; m0 < M; m0 += GEMM_ROWS) {
-        float acc[GEMM_ROWS];
-#pragma unroll
-        for (int r = 0; r < GEMM_ROWS; ++r) acc[r] = 0.0f;
-        if (vec) {
-            for (int k = lane * 4; k < K; k += 256) {
-                const float4 wv = *reinterpret_cast<const float4 *>(wr + k);
-#pragma unroll
-                for (int r = 0; r < GEMM_ROWS; ++r) {
-                    if (m0 + r < M) {
-                        const float4 av = *reinterpret_cast<const float4 *>(a + (long long) (m0 + r) * K + k);
-                        acc[r] = fmaf(av.x, wv.x, fmaf(av.y, wv.y, fmaf(av.z, wv.z, fmaf(av.w, wv.w, acc[r]))));
-                    }
-                }
-            }
-        } else {
-            for (int k = lane; k < K; k += 64) {
-                const float wv = wr[k];
-#pragma unroll
-                for (int r = 0; r < GEMM_ROWS; ++r)
-                    if (m0 + r < M) acc[r] = fmaf(a[(long long) (m0 + r) * K + k], wv, acc[r]);
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < GEMM_ROWS; ++r) {
-            float v = acc[r];
-#pragma unroll
-            for (int s = 32; s >= 1; s >>= 1) v += __shfl_xor(v, s, 64);
-            if (lane == 0 && m0 + r < M) out[(long long) (m0 + r) * N + n] = __fadd_rn(v, bias[n]);
-        }
-    }
-}
-
-int gemm_nt_launch(int m, int k, int n, const float *a, const float *w, const float *bias, float *out,
-                   hipStream_t stream) {
-    const int vec = (k % 4 == 0) && ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w)) % 16 == 0);
-    hipLaunchKernelGGL(gemm_nt_kernel, dim3((n + 3) / 4), dim3(256), 0, stream, m, k, n, a, w, bias, out, vec);
     ONHIP_CHECK_HIP(hipGetLastError());
     return ONHIP_OK;
 }

@@ -371,6 +371,7 @@ int rows_to_h16_launch(int dt, const float *x, long long rows, int k, int kp, vo
 int rows_from_h16_launch(int dt, const void *x, long long rows, int k, int kp, float *y, hipStream_t stream);
 int pack_w8_launch(const int8_t *w8, int cout, int cin, int kh, int kw, int cp, int k_units, int8_t *packed,
                    hipStream_t stream);
+bool gemm_nt_mfma_ok(int m, int k, int n, const float *a, const float *w);
 int gemm_nt_launch(int m, int k, int n, const float *a, const float *w, const float *bias, float *out,
                    hipStream_t stream);
 int copy_f32_launch(const float *src, float *dst, long long n, hipStream_t stream);
