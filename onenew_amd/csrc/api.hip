@@ -1609,6 +1609,18 @@ static int conv2d_w8a32_impl(const onhip_conv_desc_t *d, const float *x, const i
     } else if (reinterpret_cast<uintptr_t>(w8) % 16) {
         return set_error(ONHIP_ERR_ARG, "conv w8a32: packed weights must be 16-byte aligned");
     }
+    // tuning hooks: ONHIP_NO_PATCH keeps to the implicit-GEMM kernels, and so does a forced tile of theirs; ONHIP_PATCH_ALL
+    // sends every shape the LDS-patch kernel can take to it, not only those it is measured to win
+    const bool no_patch = getenv("ONHIP_NO_PATCH") != nullptr || getenv("ONHIP_TILE") != nullptr;
+    // few output pixels, fp32 in and out: quantised, multiplied and finished in one launch.  (It needs no workspace; a caller that gives less
+    // than onhip_conv2d_w8a32_workspace asks for has the layer in one piece of the staged form, as it always had.)
+    I8SmallPlan small;
+    if (!xq && !d->out_s8 && !acc32 && !addend && !no_patch && !tl_hint_bm && workspace_bytes >= packed_bytes + q_bytes + w8a32_slices_bytes(d, k_units) &&
+        i8small_ok(*d, OH, OW, &small)) {
+        const int ran[7] = {32 * small.wm, 32 * small.nb, 8 / small.wm, 0, 4, 0, 0};   // tile, wavefronts along K, which kernel
+        memcpy(tl_last_choice, ran, sizeof(ran));
+        return i8small_launch(*d, OH, OW, small, x, packed, bias32, weight_aux, ep, reinterpret_cast<float *>(y), st);
+    }
     if (xq) {
         q = const_cast<int8_t *>(xq);
     } else {
@@ -1680,9 +1692,6 @@ static int conv2d_w8a32_impl(const onhip_conv_desc_t *d, const float *x, const i
         p.twin_inv_scale = twin ? 1.0f / d->output_scale : 0.0f;
     }
     // 3x3, stride 1, few channels, int8 in and out: the kernel that keeps the band's input in LDS and the weights in registers
-    // tuning hooks: ONHIP_NO_PATCH keeps to the implicit-GEMM kernels, and so does a forced tile of theirs; ONHIP_PATCH_ALL
-    // sends every shape the LDS-patch kernel can take to it, not only those it is measured to win
-    const bool no_patch = getenv("ONHIP_NO_PATCH") != nullptr || getenv("ONHIP_TILE") != nullptr;
     if (nhwc_out && !no_patch && i8patch_ok(p, getenv("ONHIP_PATCH_ALL") != nullptr)) return i8patch_launch(p, st);
     if (nhwc_out && !no_patch && i8direct_ok(p)) return i8direct_launch(p, st);
     return plan_and_launch(cfg, p, st);
