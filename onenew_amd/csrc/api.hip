@@ -480,7 +480,12 @@ static bool tile_exists(const Choice &c) {
 static bool f3_ok(const IgemmLaunch &cfg, const IgemmProblem &p) {
     static const bool off = getenv("ONHIP_NO_F3") != nullptr;   // tuning hook: fp32 matrix instructions only
     if (off || cfg.dtype != DT_F32 || cfg.batch != 1 || !p.w_src) return false;
-    if (cfg.bl != BL_PLAIN && cfg.bl != BL_ROWS && !((cfg.bl == BL_TAPC || cfg.bl == BL_GATHER) && p.use_tapmask)) return false;
+    // filters of at most 64 taps, or larger ones where every window lies inside the image (a patch layer: 16 x 16, stride 16) and the
+    // multiply-high divisions by the taps are exact
+    const bool taps = cfg.bl == BL_TAPC || cfg.bl == BL_GATHER;
+    const bool large = cfg.bl == BL_GATHER && !p.use_tapmask && p.pt == 0 && p.pl == 0 && (p.OHW / p.OW - 1) * p.sh + p.kh <= p.H &&
+                       (p.OW - 1) * p.sw + p.kw <= p.W && (p.K + 64LL) * p.khkw < (1LL << 32) && (long long) p.khkw * p.kw < (1LL << 32);
+    if (cfg.bl != BL_PLAIN && cfg.bl != BL_ROWS && !(taps && p.use_tapmask) && !large) return false;
     const long long bytes = split_weights_bytes(p.M, p.K);
     return bytes < (1LL << 31) && (p.keeper || bytes <= kSplitWsBytes);
 }
@@ -1837,7 +1842,9 @@ static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float
         if (form.p.M > 32 && form.p.K >= 48 && p.b_slice_bytes < (1LL << 31) && form.p.b_slice_bytes < (1LL << 31) &&
             form.p.c_slice_bytes < (1LL << 31) && f3_choice(form.cfg, form.p, &form.rows, &us)) {
             form.plain = model_choice(cfg, p);
-            form.faster = !tl_hint_bm && us < f32_us(cfg, p, form.plain);   // a hint is for the plain form's tile
+            // (a product's residual operand costs the plain form more than a convolution's: 0.15 us a MB, 192 x 12544 x 192 with one 16.1 us)
+            const double plain_us = f32_us(cfg, p, form.plain) + (p.res ? 0.084e-6 * 4.0 * p.M * p.N : 0.0);
+            form.faster = !tl_hint_bm && us < plain_us;   // a hint is for the plain form's tile
             form.p.keeper = keeper;
             return plan_and_launch(cfg, p, st, &form);
         }

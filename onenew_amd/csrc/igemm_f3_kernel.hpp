@@ -87,10 +87,15 @@ __device__ constexpr int f3_pb(int i) { constexpr int t[F3_PRODUCTS] = {0, 1, 0,
 template <int BL>
 __device__ __forceinline__ ColState f3_col(const IgemmProblem &p, int n) {
     if constexpr (BL == BL_ROWS) return {n < p.N ? (unsigned) (n * p.ldb) * 4u : OOB, 0, 0, 0u, 0u};
-    else return make_col<BL>(p, n);
+    else {
+        ColState c = make_col<BL>(p, n);
+        if constexpr (BL == BL_GATHER)
+            if (!p.use_tapmask) c.mask_lo = c.mask_hi = ~0u;   // every window lies inside the image (f3_ok)
+        return c;
+    }
 }
 
-// prep_b and b_voff for the K loop: filters of at most 64 taps (f3_ok) and no test of the reduction index, so nothing that a
+// prep_b and b_voff for the K loop: filters of at most 64 taps, or windows inside the image (f3_ok), and no test of the reduction index, so nothing that a
 // branch could come of (those stood between the MFMAs of every K tile).  Beyond K the tap's bit is clear, or another tap's:
 // what is read there meets zero weights.
 struct F3Prep { unsigned soff, tap; };
