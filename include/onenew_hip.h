@@ -543,6 +543,19 @@ int onhip_matmul_bias_gelu_eval(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BU
  * result, in one call (onhip_matmul_add).  Slots as for `eval_bias`; the second addend travels in inputs[3] (it has the
  * result's operand, so no params slot of its own), as the addend of the Conv plugin's `eval_add` does. */
 int onhip_matmul_bias_add_eval(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_INFO_S *outputs);
+/* `eval_bias_group` of libMatMul_hip.so: up to four products with a bias on one left operand (the q, k and v projections of an attention
+ * block), in one launch where that is expected to be faster, one after the other where not; the values of `eval_bias` for each either way.
+ * Slots as for `eval_bias` of the first product, whose weight, bias and result all of them share the shapes of; inputs[4] = the address of an
+ * onhip_product_group_t in host memory.  Device memory throughout, weights and biases held (onhip_plugin_hold); the results lie out_step
+ * bytes apart, a multiple of 16.  w_all, bias_all: the weights [k][parts * n] and the biases side by side. */
+#define ONHIP_GROUP_MAX 4
+typedef struct {
+    int32_t parts;
+    const float *w[ONHIP_GROUP_MAX], *bias[ONHIP_GROUP_MAX];
+    const float *w_all, *bias_all;
+    int64_t out_step;
+} onhip_product_group_t;
+int onhip_matmul_bias_group_eval(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_INFO_S *outputs);
 /*
  * No counterpart in the reference, whose operators always finish before eval returns (device/cuda/MaxPool/
  * maxpool.cu:76).  on != 0: an eval whose output is device memory returns as soon as its kernels are queued on

@@ -1776,8 +1776,23 @@ static void matmul_rows_problem(const onhip_matmul_desc_t *d, const float *a, co
     p->res = addend;
 }
 
-static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias,
-                       const float *gelu_lut, const float *addend, float *out, void *stream, const SplitKeeper *keeper = nullptr) {
+// How a product whose rows form is `form` runs; false where it has no such form.  Rule as in model_choice; the pass that splits the weights
+// is priced in even where the caller keeps them split, so that a product runs the same way, with the same bits, whether its right operand is
+// a model's weight or not.
+static bool rows_form(const IgemmLaunch &cfg, const IgemmProblem &p, RowsForm *form, double *us) {
+    if (form->p.M <= 32 || form->p.K < 48 || p.b_slice_bytes >= (1LL << 31) || form->p.b_slice_bytes >= (1LL << 31) ||
+        form->p.c_slice_bytes >= (1LL << 31) || !f3_choice(form->cfg, form->p, &form->rows, us))
+        return false;
+    form->plain = model_choice(cfg, p);
+    // (a product's residual operand costs the plain form more than a convolution's: 0.15 us a MB, 192 x 12544 x 192 with one 16.1 us)
+    const double plain_us = f32_us(cfg, p, form->plain) + (p.res ? 0.084e-6 * 4.0 * p.M * p.N : 0.0);
+    form->faster = !tl_hint_bm && *us < plain_us;   // a hint is for the plain form's tile
+    return true;
+}
+
+// rows_us: nothing is launched; what the rows form takes where the product would run in it, else 0
+static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias, const float *gelu_lut, const float *addend,
+                       float *out, void *stream, const SplitKeeper *keeper = nullptr, double *rows_us = nullptr) {
     if (!d || d->batch < 1 || d->m < 1 || d->k < 1 || d->n < 1) return set_error(ONHIP_ERR_ARG, "matmul: bad shape");
     if (!a || !b || !out) return set_error(ONHIP_ERR_ARG, "matmul: null tensor pointer");
     int batch = d->batch, M = d->m;
@@ -1837,19 +1852,46 @@ static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float
         RowsForm form;
         matmul_rows_problem(d, a, b, bias, gelu_lut, addend, out, &form.cfg, &form.p);
         double us;
-        // rule as in model_choice; the pass that splits the weights is priced in even where the caller keeps them split, so that
-        // a product runs the same way, with the same bits, whether its right operand is a model's weight or not
-        if (form.p.M > 32 && form.p.K >= 48 && p.b_slice_bytes < (1LL << 31) && form.p.b_slice_bytes < (1LL << 31) &&
-            form.p.c_slice_bytes < (1LL << 31) && f3_choice(form.cfg, form.p, &form.rows, &us)) {
-            form.plain = model_choice(cfg, p);
-            // (a product's residual operand costs the plain form more than a convolution's: 0.15 us a MB, 192 x 12544 x 192 with one 16.1 us)
-            const double plain_us = f32_us(cfg, p, form.plain) + (p.res ? 0.084e-6 * 4.0 * p.M * p.N : 0.0);
-            form.faster = !tl_hint_bm && us < plain_us;   // a hint is for the plain form's tile
+        if (rows_form(cfg, p, &form, &us)) {
+            if (rows_us) { *rows_us = form.faster ? us : 0.0; return ONHIP_OK; }
             form.p.keeper = keeper;
             return plan_and_launch(cfg, p, st, &form);
         }
     }
+    if (rows_us) { *rows_us = 0.0; return ONHIP_OK; }
     return plan_and_launch(cfg, p, st);
+}
+
+// Why: three products of 192 columns over 12544 rows are 12 us each, half of it first loads and stores; as one of 576 columns a tile of 128
+// columns is a workgroup's.  Only where a product on its own runs on the 16-bit matrix cores as well: the arithmetic is the same, so are the bits.
+static int matmul_group_impl(const onhip_matmul_desc_t *d, int parts, const float *a, const float *w_all, const float *bias_all, float *out,
+                             long long out_step, const SplitKeeper *keeper, void *stream, bool *ran) {
+    *ran = false;
+    if (!d || !a || !w_all || !bias_all || !out) return set_error(ONHIP_ERR_ARG, "matmul group: null pointer");
+    if (parts < 2 || parts > ONHIP_GROUP_MAX) return set_error(ONHIP_ERR_ARG, "matmul group: %d products", parts);
+    if (d->compute != ONHIP_COMPUTE_F32 || d->n % 32 || out_step % 16 || tune_mode() || tl_noalloc || tl_hint_bm || getenv("ONHIP_TILE")) return ONHIP_OK;
+    double each;
+    const int rc = matmul_impl(d, a, w_all, bias_all, nullptr, nullptr, out, stream, nullptr, &each);   // a plan: the weights are not read
+    if (rc || each == 0.0) return rc;
+    onhip_matmul_desc_t all = *d;
+    all.n = parts * d->n;
+    IgemmLaunch cfg;
+    IgemmProblem p;
+    const long long rows = (long long) d->batch * d->m, extent = (parts - 1) * out_step + rows * d->n * 4;
+    if ((long long) d->k * all.n >= (1LL << 31) || rows * all.n >= (1LL << 31) || out_step < rows * d->n * 4 || extent >= (1LL << 31)) return ONHIP_OK;
+    matmul_rows_problem(&all, a, w_all, bias_all, nullptr, nullptr, out, &cfg, &p);
+    p.c_stride_n = d->n;
+    p.c_slice_bytes = extent;
+    p.c_part = d->n;
+    p.c_part_step = (unsigned) out_step;
+    Choice c;
+    double us;
+    if (!f3_choice(cfg, p, &c, &us) || us >= parts * each) return ONHIP_OK;
+    p.keeper = keeper;
+    const int launched = launch_choice(cfg, p, c, reinterpret_cast<hipStream_t>(stream));
+    if (launched == kNoSplitSlot) return ONHIP_OK;
+    *ran = launched == ONHIP_OK;
+    return launched;
 }
 
 int onhip_matmul(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias,
@@ -2228,5 +2270,9 @@ int conv2d_f32_kept(const onhip_conv_desc_t *d, const float *x, const float *w, 
 int matmul_f32_kept(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias, const float *gelu_lut, const float *addend,
                     float *out, const SplitKeeper *keeper, void *stream) {
     return matmul_impl(d, a, b, bias, gelu_lut, addend, out, stream, keeper);
+}
+int matmul_group_f32_kept(const onhip_matmul_desc_t *d, int parts, const float *a, const float *w_all, const float *bias_all, float *out, long long out_step,
+                          const SplitKeeper *keeper, void *stream, bool *ran) {
+    return matmul_group_impl(d, parts, a, w_all, bias_all, out, out_step, keeper, stream, ran);
 }
 }  // namespace onhip

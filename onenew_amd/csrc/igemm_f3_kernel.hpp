@@ -216,7 +216,11 @@ __device__ __forceinline__ void write_tile_rows(const IgemmProblem &p, f32x16 (&
 #pragma unroll
         for (int a = 0; a < TM; ++a) {
             const int m4 = m_wave + a * 32 + 4 * lh;
-            const unsigned base = n < p.N ? (unsigned) (n * (int) p.c_stride_n + m4) * 4u : OOB;
+            unsigned base = n < p.N ? (unsigned) (n * (int) p.c_stride_n + m4) * 4u : OOB;
+            if (p.c_part) {   // several products: a block of 32 rows lies inside one of them
+                const int row = m_wave + a * 32, part = (row >= p.c_part) + (row >= 2 * p.c_part) + (row >= 3 * p.c_part);
+                base = n < p.N ? base + (unsigned) part * (p.c_part_step - (unsigned) p.c_part * 4u) : OOB;
+            }
             u32x4 rv[4];
             if constexpr (RES)
 #pragma unroll

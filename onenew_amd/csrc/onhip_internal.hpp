@@ -265,6 +265,10 @@ struct IgemmProblem : IgemmParams {
     float *slices;
     long long slices_bytes;
     int ldb;                   // B given as rows (BL_ROWS): elements between them
+    // BL_ROWS, several products on one left operand: 0, or the columns of C of each (a multiple of 32); product i's result starts
+    // i * c_part_step bytes after the first one's
+    int c_part;
+    unsigned c_part_step;
 };
 
 enum { DT_F32 = 0, DT_BF16 = 1, DT_F16 = 2, DT_I8 = 3 };
@@ -305,6 +309,10 @@ int conv2d_f32_kept(const onhip_conv_desc_t *d, const float *x, const float *w, 
                     const float *addend, int relu_after, float *y, const SplitKeeper *keeper, void *stream);
 int matmul_f32_kept(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias, const float *gelu_lut, const float *addend,
                     float *out, const SplitKeeper *keeper, void *stream);
+// `parts` products of the shape d on one left operand, weights [k][parts * n] and biases side by side, results out_step bytes apart: as one
+// launch if that is expected to be faster than each on its own, which then has the same bits (*ran says whether)
+int matmul_group_f32_kept(const onhip_matmul_desc_t *d, int parts, const float *a, const float *w_all, const float *bias_all, float *out, long long out_step,
+                          const SplitKeeper *keeper, void *stream, bool *ran);
 // st is being captured; true as well for the legacy stream while another thread's capture keeps it from being asked
 bool under_capture(hipStream_t st);
 // hipMalloc that is no part of what is captured, by this thread or by another

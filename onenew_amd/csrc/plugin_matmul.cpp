@@ -36,3 +36,9 @@ extern "C" __attribute__((visibility("default"))) int eval_bias_add(BUFFER_INFO_
                                                                     BUFFER_INFO_S *outputs) {
     return onhip_matmul_bias_add_eval(params, inputs, outputs);
 }
+// Several products with a bias on one left operand (the q, k and v projections of an attention block): as one launch where that is faster.
+// inputs[4] = an onhip_product_group_t.
+extern "C" __attribute__((visibility("default"))) int eval_bias_group(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs,
+                                                                      BUFFER_INFO_S *outputs) {
+    return onhip_matmul_bias_group_eval(params, inputs, outputs);
+}

@@ -28,6 +28,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include "../../include/onenew_abi.h"
+#include "../../include/onenew_hip.h"
 #include "../../include/onenew_rt.h"
 
 namespace {
@@ -120,6 +121,7 @@ struct Tensor {
     std::string alias;       // an operand folded away with its producer reads as this one (fuse_residual_blocks)
     bool never_written = false;   // an operand inside a fused attention block: it has no buffer and no value
     bool as_s8 = false;           // written and read as int8 NHWC, channels padded to 16 (link_int8_convs)
+    std::vector<char> made;       // an initialiser that is not in the file: its data until uploaded (group_products)
     bool has_twin = false;        // fp32, and stored once more as int8 NHWC for the int8 convolutions among its readers
     void *twin_dev = nullptr;
 };
@@ -138,6 +140,11 @@ struct Node {
     // inputs[4] ({in_s8, out_s8, out_scale}) and inputs[5] (the fold code, when an Add is folded in)
     struct { int32_t in_s8, out_s8; float out_scale; int32_t twin; } link = {0, 0, 0.0f, 0};
     int32_t link_fuse = 0;
+    // products on one left operand that run in one call (group_products): the nodes, this one first; and on the others that they do not run
+    std::vector<int> group;
+    bool in_group = false;
+    std::string group_w, group_b;            // their weights and biases side by side
+    onhip_product_group_t group_args = {};
     bool reads_twin = false;   // its input is the int8 copy of an fp32 operand
     BUFFER_INFO_S params[BUF_MAXNUM], inputs[BUF_MAXNUM], outputs[BUF_MAXNUM];
     const BASE_CONFIG_S *base() const { return reinterpret_cast<const BASE_CONFIG_S *>(cfg.data()); }
@@ -177,7 +184,7 @@ struct onrt_net {
     onenew_eval_fn conv_block = nullptr, conv_block_takes = nullptr, conv_link = nullptr, conv_link_takes = nullptr;
     onenew_eval_fn conv_pair = nullptr, conv_pair_relu = nullptr, conv_pair_takes = nullptr;
     onenew_eval_fn maxpool_s8 = nullptr;   // optional entry point of the MaxPool plugin
-    onenew_eval_fn matmul_attention = nullptr, matmul_bias = nullptr, matmul_bias_gelu = nullptr, matmul_bias_add = nullptr;   // optional entry points of the MatMul plugin
+    onenew_eval_fn matmul_attention = nullptr, matmul_bias = nullptr, matmul_bias_gelu = nullptr, matmul_bias_add = nullptr, matmul_bias_group = nullptr;   // optional entry points of the MatMul plugin
     int fused_blocks = 0, folded_relus = 0, folded_acts = 0, fused_attentions = 0, fused_linears = 0, fused_skips = 0, fused_ir_blocks = 0, fused_pairs = 0, int8_links = 0;
     void *init_arena = nullptr, *act_arena = nullptr, *tables = nullptr;
     std::vector<float> silu_lut, gelu_lut;
@@ -428,8 +435,10 @@ int allocate(onrt_net &net) {
             Tensor &t = kv.second;
             if (!t.is_init) continue;
             t.dev = static_cast<char *>(net.init_arena) + off;
-            if (t.bytes) ONRT_HIP(hipMemcpy(t.dev, net.file.data() + (size_t) t.desc.p_data, t.bytes, hipMemcpyHostToDevice));
+            const char *data = t.made.empty() ? net.file.data() + (size_t) t.desc.p_data : t.made.data();
+            if (t.bytes) ONRT_HIP(hipMemcpy(t.dev, data, t.bytes, hipMemcpyHostToDevice));
             t.desc.p_data = 0;
+            t.made = std::vector<char>();
             off += (t.bytes + 255) & ~(size_t) 255;
         }
         // they stay as they are until the net is freed (and the plugins told to forget them)
@@ -451,9 +460,15 @@ int allocate(onrt_net &net) {
     if (act_total) {
         ONRT_HIP(hipMalloc(&net.act_arena, act_total));
         size_t off = 0;
+        for (const Node &nd : net.nodes)   // the results of a group of products one behind the other
+            for (int g : nd.group) {
+                Tensor &t = net.tensors[net.nodes[g].fused_out];
+                t.dev = static_cast<char *>(net.act_arena) + off;
+                off += (t.bytes + 255) & ~(size_t) 255;
+            }
         for (auto &kv : net.tensors) {
             Tensor &t = kv.second;
-            if (t.is_init || t.desc.not_need_buf || !t.alias.empty() || t.never_written) continue;
+            if (t.is_init || t.desc.not_need_buf || !t.alias.empty() || t.never_written || t.dev) continue;
             t.dev = static_cast<char *>(net.act_arena) + off;
             off += (t.bytes + 255) & ~(size_t) 255;
             if (t.has_twin) {
@@ -560,6 +575,7 @@ int bind_plugins(onrt_net &net) {
             net.matmul_bias = reinterpret_cast<onenew_eval_fn>(dlsym(it->second, "eval_bias"));
             net.matmul_bias_gelu = reinterpret_cast<onenew_eval_fn>(dlsym(it->second, "eval_bias_gelu"));
             net.matmul_bias_add = reinterpret_cast<onenew_eval_fn>(dlsym(it->second, "eval_bias_add"));
+            net.matmul_bias_group = reinterpret_cast<onenew_eval_fn>(dlsym(it->second, "eval_bias_group"));
         }
     }
     return ONRT_OK;
@@ -1209,6 +1225,59 @@ int fuse_linear(onrt_net &net) {
     return ONRT_OK;
 }
 
+// Linear layers of one shape on one input (the q, k and v projections of an attention block): the first of them in the order makes all their
+// results, in one call of the MatMul plugin's `eval_bias_group`; the others stay in the order and have nothing to do.  Their weights lie side
+// by side in a copy of their own, for the call to run as one product; the operands are the same as without.
+int group_products(onrt_net &net) {
+    if (!fusing_enabled() || !net.matmul_bias_group) return ONRT_OK;
+    for (size_t at = 0; at < net.order.size(); ++at) {
+        Node &first = net.nodes[net.order[at]];
+        if (strcmp(first.kind->type, "MatMul") || first.fuse != 4 || first.in_group || first.in.size() != 3) continue;
+        const Tensor &x = net.tensors[first.in[0]], &w = net.tensors[first.in[1]], &b = net.tensors[first.in[2]], &y = net.tensors[first.fused_out];
+        const int rank = y.desc.dim_num_of_shapes, n = y.desc.shapes[rank - 1], k = x.desc.shapes[x.desc.dim_num_of_shapes - 1];
+        if (x.is_init || !w.is_init || w.desc.dim_num_of_shapes != 2 || w.desc.shapes[0] != k || w.desc.shapes[1] != n || w.bytes != (size_t) k * n * 4 ||
+            b.bytes != (size_t) n * 4 || n % 32 || !y.alias.empty() || y.never_written || y.as_s8 || y.has_twin)
+            continue;
+        std::vector<int> group = {net.order[at]};
+        for (size_t j = at + 1; j < net.order.size() && group.size() < ONHIP_GROUP_MAX; ++j) {
+            const Node &nd = net.nodes[net.order[j]];
+            if (strcmp(nd.kind->type, "MatMul") || nd.fuse != 4 || nd.in_group || nd.in.size() != 3 || nd.in[0] != first.in[0]) continue;
+            const Tensor &w2 = net.tensors[nd.in[1]], &b2 = net.tensors[nd.in[2]], &y2 = net.tensors[nd.fused_out];
+            if (!w2.is_init || w2.bytes != w.bytes || b2.bytes != b.bytes || w2.desc.data_type != w.desc.data_type || b2.desc.data_type != b.desc.data_type ||
+                memcmp(w2.desc.shapes, w.desc.shapes, sizeof(w.desc.shapes)) || w2.desc.dim_num_of_shapes != 2 || !y2.alias.empty() || y2.never_written ||
+                y2.as_s8 || y2.has_twin || memcmp(y2.desc.shapes, y.desc.shapes, sizeof(y.desc.shapes)))
+                continue;
+            group.push_back(net.order[j]);
+        }
+        if (group.size() < 2) continue;
+        const size_t parts = group.size();
+        Tensor w_all, b_all;
+        w_all.desc = w.desc;
+        w_all.desc.shapes[1] = (int32_t) parts * n;
+        w_all.bytes = parts * w.bytes;
+        b_all.desc = b.desc;
+        b_all.desc.shapes[b.desc.dim_num_of_shapes - 1] = (int32_t) parts * n;
+        b_all.bytes = parts * b.bytes;
+        w_all.is_init = b_all.is_init = w_all.produced = b_all.produced = true;
+        w_all.made.resize(w_all.bytes);
+        b_all.made.resize(b_all.bytes);
+        const size_t row = (size_t) n * 4;
+        for (size_t i = 0; i < parts; ++i) {
+            const char *from = net.file.data() + net.tensors[net.nodes[group[i]].in[1]].desc.p_data;
+            for (int r = 0; r < k; ++r) memcpy(w_all.made.data() + (r * parts + i) * row, from + r * row, row);
+            memcpy(b_all.made.data() + i * row, net.file.data() + net.tensors[net.nodes[group[i]].in[2]].desc.p_data, row);
+            net.nodes[group[i]].in_group = i > 0;
+        }
+        first.group = group;
+        first.group_w = first.fused_out + "/weights side by side";   // no operand's name: those have at most OPERAND_NAME_LEN - 1 letters and come from the file
+        first.group_b = first.fused_out + "/biases side by side";
+        first.eval = net.matmul_bias_group;
+        net.tensors[first.group_w] = w_all;
+        net.tensors[first.group_b] = b_all;
+    }
+    return ONRT_OK;
+}
+
 // ---- slot arrays (op::rt_prepare, host/op.h:109-168, and prepare_init_operand_data of each operator) ----
 int fill_slots(onrt_net &net) {
     const size_t lut_len = net.silu_lut.size();
@@ -1227,6 +1296,19 @@ int fill_slots(onrt_net &net) {
             nd.inputs[slot].addr = (int64_t) t.dev;
         }
         if (nd.fuse == 3) nd.inputs[4].addr = (int64_t) nd.token_major;
+        if (!nd.group.empty()) {
+            onhip_product_group_t &g = nd.group_args;
+            g.parts = (int32_t) nd.group.size();
+            for (int i = 0; i < g.parts; ++i) {
+                const Node &part = net.nodes[nd.group[i]];
+                g.w[i] = static_cast<const float *>(net.tensors[part.in[1]].dev);
+                g.bias[i] = static_cast<const float *>(net.tensors[part.in[2]].dev);
+            }
+            g.w_all = static_cast<const float *>(net.tensors[nd.group_w].dev);
+            g.bias_all = static_cast<const float *>(net.tensors[nd.group_b].dev);
+            g.out_step = (int64_t) ((net.tensors[nd.fused_out].bytes + 255) & ~(size_t) 255);
+            nd.inputs[4].addr = (int64_t) &g;
+        }
         if (nd.fuse == 7) {
             const Node &b = net.nodes[nd.block_dw], &c = net.nodes[nd.block_pw];
             block_slots(net, nd, b, c, net.tensors[nd.fused_out]);
@@ -1289,6 +1371,7 @@ int prepare(onrt_net &net, const char *op_lib_dir) {
     if (!rc) rc = fuse_attention(net);
     if (!rc) rc = fuse_linear(net);
     if (!rc) rc = link_int8_convs(net);
+    if (!rc) rc = group_products(net);
     if (!rc) rc = allocate(net);
     if (!rc) rc = build_tables(net);
     if (!rc) rc = fill_slots(net);
@@ -1346,7 +1429,7 @@ void set_stream(onrt_net &net, hipStream_t s) {
 int run_operators(onrt_net &net) {
     for (int idx : net.order) {
         Node &nd = net.nodes[idx];
-        if (nd.kind->view) continue;
+        if (nd.kind->view || nd.in_group) continue;
         const int r = nd.eval(nd.params, nd.inputs, nd.outputs);
         if (r) return fail(ONRT_ERR_PLUGIN, "%s %s: eval returned %d", nd.kind->type, nd.base()->op_name, r);
     }

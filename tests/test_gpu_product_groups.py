@@ -1,0 +1,65 @@
+"""Linear layers of one shape on one input, which the runtime runs as one call (and the library as one launch where that is faster): the bits of
+the net run operator by operator."""
+import numpy as np
+import pytest
+
+from onenew_amd import hip, onefile, rt
+
+pytestmark = pytest.mark.gpu
+
+
+# (rows, k, n, products): one launch with tiles that cover two products and end inside the last one, K off sixteen, rows off every tile, more
+# products than a group takes; few rows, where each runs on its own
+CASES = [(2099, 192, 192, 3), (5000, 64, 96, 2), (1500, 201, 224, 4), (3000, 192, 160, 5), (50, 96, 64, 3), (12544, 192, 192, 3)]
+
+
+@pytest.mark.parametrize("rows,k,n,products", CASES)
+def test_group(rows, k, n, products, monkeypatch):
+    hip.init(0)
+    print("product group", rows, k, n, products, flush=True)
+    m, rng = onefile.OneModel(), np.random.default_rng(rows + n)
+    w = lambda *s: (rng.normal(size=s) / s[0] ** 0.5).astype(np.float32)   # noqa: E731
+    m.input("x", (2, rows // 2, k))
+    for i in range(products):
+        m.matmul(f"p{i}", "x", w(k, n), f"p{i}_mm")
+        m.add(f"p{i}_bias", f"p{i}_mm", w(n), f"y{i}")
+        if i == 0:   # another shape between them
+            m.matmul("odd", "x", w(k, 33), "odd_mm")
+            m.add("odd_bias", "odd_mm", w(33), "odd_y")
+        m.output(f"y{i}", (2, rows // 2, n))
+    m.output("odd_y", (2, rows // 2, 33))
+    data = m.tobytes()
+    fused = rt.Net(data)
+    monkeypatch.setenv("ONENEW_RT_FUSE", "0")
+    plain = rt.Net(data)
+    assert fused.fused_linears() == products + 1
+    for scale in (1.0, -0.3):
+        x = (rng.normal(size=(2, rows // 2, k)) * scale).astype(np.float32)
+        if scale < 0:
+            x[1, 3, 5] = np.inf
+        got, ref = fused.run(x), plain.run(x)
+        for i, (a, b) in enumerate(zip(got, ref)):
+            assert np.array_equal(a, b, equal_nan=True), i
+        assert np.isfinite(got[0][0]).all()
+        for i in range(products):
+            assert np.array_equal(fused.fetch(f"y{i}"), ref[i], equal_nan=True)
+    fused.close()
+    plain.close()
+
+
+def test_one_launch():
+    """three products of 192 columns run as one of 576, in tiles that a product of 192 is not cut into"""
+    hip.init(0)
+    ran = []
+    for products in (1, 3):
+        m, rng = onefile.OneModel(), np.random.default_rng(3)
+        m.input("x", (64, 196, 192))
+        for i in range(products):
+            m.matmul(f"p{i}", "x", (rng.normal(size=(192, 192)) * 0.07).astype(np.float32), f"p{i}_mm")
+            m.add(f"p{i}_bias", f"p{i}_mm", rng.normal(size=192).astype(np.float32), f"y{i}")
+            m.output(f"y{i}", (64, 196, 192))
+        net = rt.Net(m.tobytes())
+        net.run(rng.normal(size=(64, 196, 192)).astype(np.float32))
+        ran.append(tuple(hip.last_launch_choice()))
+        net.close()
+    assert ran[0][4] == ran[1][4] == 2 and ran[0][:2] != ran[1][:2], ran
