@@ -30,16 +30,18 @@ struct AttnParams {
 };
 
 template <int NKT, int HD>
-__global__ __launch_bounds__(256, 2) void attention_f32_kernel(const AttnParams p) {
-    static_assert(HD % 16 == 0 && HD <= 64 && NKT >= 1 && NKT <= 16, "head dimension in 16s, at most 256 keys");
+__global__ __launch_bounds__(256, NKT <= 13 ? 3 : 2) void attention_f32_kernel(const AttnParams p) {
+    static_assert((HD == 32 || HD == 64) && NKT >= 1 && NKT <= 16, "head dimension of 32 or 64, at most 256 keys");
     constexpr int KEYS = NKT * 16;
-    // floats per key row: 16-byte reads of 16 consecutive rows spread over 64 banks, and rows four apart (the lane
-    // quarters of a step of the second product) start 16 banks apart
-    constexpr int LD = HD + 4;
     constexpr int DT = HD / 16, QF = HD / 16;
     constexpr int PARTS = HD / 4, NV = (KEYS * PARTS + 255) / 256;
-    // one buffer, first k, then v (fetched into registers while the scores are computed): two workgroups fit a compute unit
-    __shared__ __attribute__((aligned(16))) float lds[KEYS * LD];
+    // where 16-byte unit u of a key's row lies: rows back to back, units exchanged by the row, so that the 16 rows of a
+    // first product's read and the row of a second one's each spread over all banks
+    auto place = [](int key, int u) { return key * HD + (u ^ ((key * HD / 64) & (PARTS - 1))) * 4; };
+    // One buffer, first k, then v (fetched into registers during the Softmax).  Up to 208 keys three workgroups fit a compute unit, in LDS (rows
+    // without padding) and in registers (v not in flight next to the first product's operands): 64 x 3 heads of 196 tokens are 768
+    // workgroups, all of them resident at once where two a unit were a round and a half: 35.1 -> 32.0 us a launch.
+    __shared__ __attribute__((aligned(16))) float lds[KEYS * HD];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
@@ -68,7 +70,7 @@ __global__ __launch_bounds__(256, 2) void attention_f32_kernel(const AttnParams 
         // buffer loads, rows past the last key at the out-of-range offset (zeros): no branch around a load, so the
         // compiler can count the loads in flight and wait for exactly the ones it needs
         const uint4 kk = buf_load_b128(rk, key < T ? (unsigned) key * kstride + part * 16 : OOB, 0);
-        if ((i + 1) * 256 <= KEYS * PARTS || f < KEYS * PARTS) *reinterpret_cast<uint4 *>(lds + key * LD + part * 4) = kk;
+        if ((i + 1) * 256 <= KEYS * PARTS || f < KEYS * PARTS) *reinterpret_cast<uint4 *>(lds + place(key, part)) = kk;
     }
     // this lane's query row, the channels it feeds to the first product
     const int q0 = (qblock * 4 + wave) * 16;
@@ -79,14 +81,6 @@ __global__ __launch_bounds__(256, 2) void attention_f32_kernel(const AttnParams 
         const float *qb = p.q + b * p.qs[0] + h * p.qs[1] + (long long) (query < T ? query : T - 1) * p.qs[2];
 #pragma unroll
         for (int j = 0; j < QF; ++j) qf[j] = *reinterpret_cast<const float4 *>(qb + 16 * j + 4 * lg);   // rows past the last: unused
-    }
-    // v on its way into registers
-    uint4 vreg[NV];
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        const int f = tid + i * 256;
-        const int key = f / PARTS, part = f % PARTS;
-        vreg[i] = buf_load_b128(rv, key < T ? (unsigned) key * vstride + part * 16 : OOB, 0);
     }
     __syncthreads();
 
@@ -101,7 +95,7 @@ __global__ __launch_bounds__(256, 2) void attention_f32_kernel(const AttnParams 
         for (int j = 0; j < QF; ++j) {
             float4 kf[NKT];
 #pragma unroll
-            for (int t = 0; t < NKT; ++t) kf[t] = *reinterpret_cast<const float4 *>(lds + (16 * t + li) * LD + 16 * j + 4 * lg);
+            for (int t = 0; t < NKT; ++t) kf[t] = *reinterpret_cast<const float4 *>(lds + place(16 * t + li, 4 * j + lg));
             // consecutive MFMAs go to different accumulators
 #pragma unroll
             for (int t = 0; t < NKT; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t].x, qf[j].x, s[t], 0, 0, 0);
@@ -113,6 +107,17 @@ __global__ __launch_bounds__(256, 2) void attention_f32_kernel(const AttnParams 
             for (int t = 0; t < NKT; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t].w, qf[j].w, s[t], 0, 0, 0);
         }
 
+    }
+    // v on its way into registers while the Softmax runs (no earlier: the first product needs the registers)
+    __builtin_amdgcn_sched_barrier(0);
+    uint4 vreg[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int f = tid + i * 256;
+        const int key = f / PARTS, part = f % PARTS;
+        vreg[i] = buf_load_b128(rv, key < T ? (unsigned) key * vstride + part * 16 : OOB, 0);
+    }
+    if (active) {
         // Softmax over the keys (softmax.c:26-59: subtract the row maximum, exponential, divide by the sum); keys past the
         // last count as minus infinity.  exp(x) as exp2(x log2 e) with the hardware's exp2: within 1e-5 of expf here
         float mx = -INFINITY;
@@ -151,7 +156,7 @@ __global__ __launch_bounds__(256, 2) void attention_f32_kernel(const AttnParams 
     for (int i = 0; i < NV; ++i) {
         const int f = tid + i * 256;
         const int key = f / PARTS, part = f % PARTS;
-        if ((i + 1) * 256 <= KEYS * PARTS || f < KEYS * PARTS) *reinterpret_cast<uint4 *>(lds + key * LD + part * 4) = vreg[i];
+        if ((i + 1) * 256 <= KEYS * PARTS || f < KEYS * PARTS) *reinterpret_cast<uint4 *>(lds + place(key, part)) = vreg[i];
     }
     __syncthreads();
     if (!active) return;
@@ -167,15 +172,16 @@ __global__ __launch_bounds__(256, 2) void attention_f32_kernel(const AttnParams 
     for (int d = 0; d < DT; ++d)
 #pragma unroll
         for (int r = 0; r < 4; ++r) o[d][r] = 0.0f;
+    auto row_of_v = [&](int key) __attribute__((always_inline)) { return *reinterpret_cast<const vrow_t *>(lds + place(key, DT * li / 4) + DT * li % 4); };
     vrow_t va[2][4];   // the operands of the next tile are read while this tile's products run
 #pragma unroll
-    for (int r = 0; r < 4; ++r) va[0][r] = *reinterpret_cast<const vrow_t *>(lds + (4 * lg + r) * LD + DT * li);
+    for (int r = 0; r < 4; ++r) va[0][r] = row_of_v(4 * lg + r);
 #pragma unroll
     for (int t = 0; t < NKT; ++t) {
         if (t + 1 < NKT) {
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                va[(t + 1) & 1][r] = *reinterpret_cast<const vrow_t *>(lds + (16 * (t + 1) + 4 * lg + r) * LD + DT * li);
+                va[(t + 1) & 1][r] = row_of_v(16 * (t + 1) + 4 * lg + r);
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r)
