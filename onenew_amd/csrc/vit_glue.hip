@@ -5,6 +5,8 @@
 // reference by the last bits of expf and is held to the fp32 tolerance.
 #include <string.h>
 
+#include <type_traits>
+
 #include "onhip_internal.hpp"
 
 namespace onhip {
@@ -135,15 +137,38 @@ __global__ __launch_bounds__(256) void layernorm_rows4_kernel(const float *__res
             tile[at[i]] = v[i].x; tile[at[i] + 1] = v[i].y; tile[at[i] + 2] = v[i].z; tile[at[i] + 3] = v[i].w;
         }
     __syncthreads();
-    if ((int) threadIdx.x < nr) {
-        const float *t = tile + threadIdx.x * pitch;
-        float psum = 0.0f, psq = 0.0f;
-        for (int i = 0; i < reduce; ++i) {
-            psum = __fadd_rn(psum, t[i]);
-            psq = __fadd_rn(psq, __fmul_rn(t[i], t[i]));
-        }
-        ln_stats(psum, psq, inv_n, &s_mean[threadIdx.x], &s_inv[threadIdx.x]);
+    // A wavefront adds up the rows, another one their squares: the additions of a row are one chain, which sets the pace (in a graph 12544 rows of
+    // 192 8.0 -> 7.2 us, 4000 of 768 18.2 -> 14.5; with both sums in a lane, reading ahead alone 7.8 and 18.1)
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (wave < 2 && lane < nr) {
+        const float *t = tile + lane * pitch;
+        auto chain = [&](auto squares) {
+            constexpr bool SQ = decltype(squares)::value;
+            constexpr int AHEAD = 16;   // elements read ahead of the additions
+            float sum = 0.0f, next[AHEAD];
+            auto add = [&](float v) { sum = __fadd_rn(sum, SQ ? __fmul_rn(v, v) : v); };
+#pragma unroll
+            for (int j = 0; j < AHEAD; ++j) next[j] = t[j];
+            int i = AHEAD;
+            for (; i + AHEAD <= reduce; i += AHEAD) {
+                float now[AHEAD];
+#pragma unroll
+                for (int j = 0; j < AHEAD; ++j) now[j] = next[j];
+#pragma unroll
+                for (int j = 0; j < AHEAD; ++j) next[j] = t[i + j];
+#pragma unroll
+                for (int j = 0; j < AHEAD; ++j) add(now[j]);
+            }
+#pragma unroll
+            for (int j = 0; j < AHEAD; ++j) add(next[j]);
+            for (; i < reduce; ++i) add(t[i]);
+            return sum;
+        };
+        if (wave == 0) s_mean[lane] = chain(std::false_type{});
+        else s_inv[lane] = chain(std::true_type{});
     }
+    __syncthreads();
+    if ((int) threadIdx.x < nr) ln_stats(s_mean[threadIdx.x], s_inv[threadIdx.x], inv_n, &s_mean[threadIdx.x], &s_inv[threadIdx.x]);
     __syncthreads();
     float4 *dst = reinterpret_cast<float4 *>(y + (long long) row0 * reduce);
 #pragma unroll
