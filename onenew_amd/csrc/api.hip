@@ -1617,14 +1617,17 @@ static int conv2d_w8a32_impl(const onhip_conv_desc_t *d, const float *x, const i
     // tuning hooks: ONHIP_NO_PATCH keeps to the implicit-GEMM kernels, and so does a forced tile of theirs; ONHIP_PATCH_ALL
     // sends every shape the LDS-patch kernel can take to it, not only those it is measured to win
     const bool no_patch = getenv("ONHIP_NO_PATCH") != nullptr || getenv("ONHIP_TILE") != nullptr;
-    // few output pixels, fp32 in and out: quantised, multiplied and finished in one launch.  (It needs no workspace; a caller that gives less
+    // Few output pixels: (quantised,) multiplied and finished in one launch.  (From fp32 it needs no workspace; a caller that gives less
     // than onhip_conv2d_w8a32_workspace asks for has the layer in one piece of the staged form, as it always had.)
+    const long long n_out = (long long) d->n * d->cout * OH * OW;
+    const unsigned res_body = (unsigned) (n_out - n_out % 32);   // relu.c:27-52
+    const I8SmallIO io = {x, xq, y, nhwc_out != 0, addend, relu_after ? 1 : 0, res_body, twin};
     I8SmallPlan small;
-    if (!xq && !d->out_s8 && !acc32 && !addend && !no_patch && !tl_hint_bm && workspace_bytes >= packed_bytes + q_bytes + w8a32_slices_bytes(d, k_units) &&
-        i8small_ok(*d, OH, OW, &small)) {
+    const bool small_form = (nhwc_out || !d->out_s8) && (xq || (!addend && workspace_bytes >= packed_bytes + q_bytes + w8a32_slices_bytes(d, k_units)));
+    if (small_form && !acc32 && !no_patch && !tl_hint_bm && i8small_ok(*d, OH, OW, io, &small)) {
         const int ran[7] = {32 * small.wm, 32 * small.nb, 8 / small.wm, 0, 4, 0, 0};   // tile, wavefronts along K, which kernel
         memcpy(tl_last_choice, ran, sizeof(ran));
-        return i8small_launch(*d, OH, OW, small, x, packed, bias32, weight_aux, ep, reinterpret_cast<float *>(y), st);
+        return i8small_launch(*d, OH, OW, small, io, packed, bias32, weight_aux, ep, st);
     }
     if (xq) {
         q = const_cast<int8_t *>(xq);
@@ -1688,10 +1691,9 @@ static int conv2d_w8a32_impl(const onhip_conv_desc_t *d, const float *x, const i
         if (rc) return rc;
     }
     if (addend) {   // the Add (and Relu) after the convolution, in its store
-        const long long n_out = (long long) d->n * d->cout * OH * OW;
         p.res = addend;
         p.res_relu = relu_after ? 1 : 0;
-        p.res_body = (unsigned) (n_out - n_out % 32);   // relu.c:27-52
+        p.res_body = res_body;
         p.twin = twin;
         p.twin_pitch = d->cout;
         p.twin_inv_scale = twin ? 1.0f / d->output_scale : 0.0f;

@@ -335,9 +335,19 @@ int depthwise_w8a32_launch(const onhip_conv_desc_t &d, int OH, int OW, const flo
 // W8A32 convolution with few output pixels, quantised, multiplied and finished in one launch (i8small.hip).  A plan: blocks of 32 pixels and
 // of 32 rows of a workgroup, its rectangle of output pixels, and what it comes to.
 struct I8SmallPlan { int nb, wm, tr, tw; long long wgs; size_t lds; double us; };
-bool i8small_ok(const onhip_conv_desc_t &d, int OH, int OW, I8SmallPlan *plan);
-int i8small_launch(const onhip_conv_desc_t &d, int OH, int OW, const I8SmallPlan &plan, const float *x, const int8_t *packed, const int32_t *bias32,
-                   const float *weight_aux, const Epilogue &ep, float *y, hipStream_t stream);
+struct I8SmallIO {   // the tensors on either side
+    const float *x;          // fp32 NCHW in, or
+    const int8_t *xq;        // int8 NHWC, channels padded to 16
+    void *y;                 // fp32 NCHW out, or int8 NHWC
+    bool out_s8;
+    const float *res;        // fp32 results from int8 activations: the Add of a residual block, its Relu, and the int8 form of what comes out
+    int res_relu;
+    unsigned res_body;
+    int8_t *twin;
+};
+bool i8small_ok(const onhip_conv_desc_t &d, int OH, int OW, const I8SmallIO &io, I8SmallPlan *plan);
+int i8small_launch(const onhip_conv_desc_t &d, int OH, int OW, const I8SmallPlan &plan, const I8SmallIO &io, const int8_t *packed, const int32_t *bias32,
+                   const float *weight_aux, const Epilogue &ep, hipStream_t stream);
 // dw_s8.hip: depthwise convolution on int8 NHWC activations (the chain form's twin of depthwise_w8a32_launch)
 bool dw_s8_ok(const onhip_conv_desc_t &d, int OH, int OW);
 int dw_s8_launch(const onhip_conv_desc_t &d, int OH, int OW, const int8_t *xq, const int8_t *w8, const int32_t *bias32,

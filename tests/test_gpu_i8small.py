@@ -62,6 +62,54 @@ def test_every_workgroup_shape_ran():
     assert SHAPES_SEEN >= {(32, 32), (64, 32), (128, 32), (64, 64)}
 
 
+# the forms either side: int8 or fp32 in; int8, fp32, or fp32 after an Add (and Relu) with its int8 twin out
+FORMS = ["s8 to s8", "f32 to s8", "s8 to f32", "s8 add", "s8 add relu"]
+LINKS = [(1, 16, 7, 7, 33, 1, 1, 0, N), (2, 40, 13, 9, 64, 3, 2, 1, R), (1, 72, 20, 20, 128, 3, 1, 1, S), (1, 576, 7, 7, 160, 1, 1, 0, N), (8, 960, 7, 7, 176, 1, 1, 0, C),
+         (1, 512, 20, 20, 80, 3, 1, 1, S), (8, 256, 14, 14, 256, 3, 1, 1, R), (1, 48, 14, 14, 70, 7, 2, 3, S), (5, 24, 3, 3, 20, 3, 1, 0, C), (3, 2048, 7, 7, 272, 1, 1, 0, N)]
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("case", LINKS, ids=[str(c) for c in LINKS])
+def test_link(case, form, monkeypatch):
+    import torch
+    hip.init(0)
+    print("i8small", form, case, flush=True)
+    d, x, wp, b32, aux, lut = layer(torch, *case)
+    d.output_scale, d.out_s8 = 0.031, int(form.endswith("to s8"))
+    add = "add" in form
+    if add and (d.cout % 16 or d.act_type == S):
+        pytest.skip("a twin has channels in sixteens, an Add follows no table activation here")
+    src = dict(x=x) if form.startswith("f32") else dict(xq=hip.quantize_nhwc_s8(x, d.input_scale))
+    oh, ow = d.out_hw()
+    g = torch.Generator(device="cuda").manual_seed(5)
+    addend = torch.randn((d.n, d.cout, oh, ow), generator=g, device="cuda") if add else None
+    results, before = [], hip.set_tuning(0)
+    try:
+        for other in (False, True):
+            if other:
+                monkeypatch.setenv("ONHIP_NO_PATCH", "1")
+            twin = torch.full((d.n, oh, ow, d.cout), 55, dtype=torch.int8, device="cuda") if add else None
+            out = torch.full((d.n, oh, ow, (d.cout + 15) // 16 * 16), 55, dtype=torch.int8, device="cuda") if d.out_s8 else torch.full((d.n, d.cout, oh, ow), 55.0, device="cuda")
+            hip.conv2d_w8_link(d, wp, b32, aux, lut, addend=addend, relu_after="relu" in form, out=out, twin=twin, **src)
+            results.append((out, twin, hip.last_launch_choice()[4]))
+    finally:
+        monkeypatch.delenv("ONHIP_NO_PATCH", raising=False)
+        hip.set_tuning(before)
+    LINKS_SEEN.append((form, results[0][2]))
+    assert results[1][2] == 0 and torch.equal(results[0][0], results[1][0]) and bool((results[0][0] != 0).any())
+    assert not add or torch.equal(results[0][1], results[1][1])
+
+
+LINKS_SEEN = []
+
+
+def test_every_form_ran():
+    if not LINKS_SEEN:
+        pytest.skip("the layers above did not run")
+    for form in FORMS:
+        assert sum(ran == 4 for f, ran in LINKS_SEEN if f == form) >= 2, (form, LINKS_SEEN)
+
+
 def test_no_bias_leaves_the_activation_out(monkeypatch):
     import torch
     hip.init(0)
