@@ -1388,9 +1388,10 @@ int onhip_conv2d_pw_pack_weights(const onhip_conv_desc_t *b, const float *wb, fl
     return pack_pw2_launch(wb, b->cout, b->cin, packed, reinterpret_cast<hipStream_t>(stream));
 }
 
-int onhip_conv2d_pw_f32(const onhip_conv_desc_t *a, const onhip_conv_desc_t *b, const float *x, const float *wa_packed,
-                        const float *bias_a, const float *wb_packed, const float *bias_b, const float *addend, int32_t relu_after,
-                        float *y, void *stream) {
+// wb: the second convolution's weights as given, with the two keepers, or none of the three
+static int conv2d_pw_impl(const onhip_conv_desc_t *a, const onhip_conv_desc_t *b, const float *x, const float *wa_packed,
+                          const float *bias_a, const float *wb, const float *wb_packed, const float *bias_b, const float *addend, int32_t relu_after,
+                          float *y, const SplitKeeper *keep_a, const SplitKeeper *keep_b, void *stream) {
     int32_t OH, OW, OH2, OW2;
     int rc = check_conv(a, &OH, &OW);
     if (!rc) rc = check_conv(b, &OH2, &OW2);
@@ -1440,7 +1441,27 @@ int onhip_conv2d_pw_f32(const onhip_conv_desc_t *a, const onhip_conv_desc_t *b, 
         p.res_relu = relu_after ? 1 : 0;
         p.res_body = (unsigned) (n_out - n_out % 32);   // relu.c:27-52
     }
+    // on the 16-bit matrix cores where both weights are kept split (first stage of a ResNet-50 at batch 32, 3x3 64 -> 64 and 1x1 64 -> 256
+    // on 56 x 56 with the Add: 95 us instead of 130)
+    static const bool off = getenv("ONHIP_NO_F3") != nullptr;   // tuning hook: fp32 matrix instructions only
+    if (!off && keep_a && keep_b) {
+        const void *sa = nullptr, *sb = nullptr;
+        rc = keep_a->get(keep_a->key, wa_packed, {p.M, p.K, p.K, 1}, &sa);
+        if (!rc && sa) rc = keep_b->get(keep_b->key, wb, {b->cout, b->cin, b->cin, 1}, &sb);
+        if (rc) return rc;
+        if (sa && sb) {
+            p.a_split = sa;
+            p.a_split_bytes = split_weights_bytes(p.M, p.K);
+            p.w2 = static_cast<const float *>(sb);
+        }
+    }
     return igemm_launch_f32_pw(p, reinterpret_cast<hipStream_t>(stream));
+}
+
+int onhip_conv2d_pw_f32(const onhip_conv_desc_t *a, const onhip_conv_desc_t *b, const float *x, const float *wa_packed,
+                        const float *bias_a, const float *wb_packed, const float *bias_b, const float *addend, int32_t relu_after,
+                        float *y, void *stream) {
+    return conv2d_pw_impl(a, b, x, wa_packed, bias_a, nullptr, wb_packed, bias_b, addend, relu_after, y, nullptr, nullptr, stream);
 }
 
 static void w8a32_layout(const onhip_conv_desc_t *d, int *cp, int *k_units, size_t *packed_bytes, size_t *q_bytes) {
@@ -2268,6 +2289,11 @@ namespace onhip {
 int conv2d_f32_kept(const onhip_conv_desc_t *d, const float *x, const float *w, int packed, const float *bias, const float *silu_lut,
                     const float *addend, int relu_after, float *y, const SplitKeeper *keeper, void *stream) {
     return conv2d_f32_impl(d, x, w, packed, bias, silu_lut, y, stream, addend, relu_after, keeper);
+}
+int conv2d_pw_f32_kept(const onhip_conv_desc_t *a, const onhip_conv_desc_t *b, const float *x, const float *wa_packed, const float *bias_a,
+                       const float *wb, const float *wb_packed, const float *bias_b, const float *addend, int relu_after, float *y,
+                       const SplitKeeper *keep_a, const SplitKeeper *keep_b, void *stream) {
+    return conv2d_pw_impl(a, b, x, wa_packed, bias_a, wb, wb_packed, bias_b, addend, relu_after, y, keep_a, keep_b, stream);
 }
 int matmul_f32_kept(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias, const float *gelu_lut, const float *addend,
                     float *out, const SplitKeeper *keeper, void *stream) {

@@ -5,9 +5,11 @@
 
 namespace onhip {
 
-int igemm_launch_f32_pw(const IgemmParams &p_in, hipStream_t stream) {
+int f3_launch_pw(const IgemmProblem &p, dim3 grid, hipStream_t stream);   // igemm_f3_pw.hip
+
+int igemm_launch_f32_pw(const IgemmProblem &p_in, hipStream_t stream) {
     constexpr int BM = 64, BN = 64;
-    IgemmParams p = p_in;
+    IgemmProblem p = p_in;
     if (p.M < 1 || p.M > BM || p.N < 1 || p.k_units < 1 || p.m2 < 1 || !p.w2 || reinterpret_cast<uintptr_t>(p.w2) % 16)
         return set_error(ONHIP_ERR_ARG, "conv + 1x1: %d rows of the first product (1 to 64), %d of the second", p.M, p.m2);
     if (p.partial || p.dp_tiles || p.out_mode != OUT_CONV)
@@ -23,10 +25,12 @@ int igemm_launch_f32_pw(const IgemmParams &p_in, hipStream_t stream) {
     p.div_tiles_n = make_div31((unsigned) tiles);
     p.n_fast = 0;
     const dim3 grid(tiles, 1, 1);
+    if (p.a_split) return f3_launch_pw(p, grid, stream);
+    const IgemmParams &plain = p;
     if (p.res)
-        hipLaunchKernelGGL((igemm_kernel<DT_F32, BL_TAPC, BM, BN, 2, 2, 1, true, true>), grid, dim3(THREADS), 0, stream, p);
+        hipLaunchKernelGGL((igemm_kernel<DT_F32, BL_TAPC, BM, BN, 2, 2, 1, true, true>), grid, dim3(THREADS), 0, stream, plain);
     else
-        hipLaunchKernelGGL((igemm_kernel<DT_F32, BL_TAPC, BM, BN, 2, 2, 1, false, true>), grid, dim3(THREADS), 0, stream, p);
+        hipLaunchKernelGGL((igemm_kernel<DT_F32, BL_TAPC, BM, BN, 2, 2, 1, false, true>), grid, dim3(THREADS), 0, stream, plain);
     ONHIP_CHECK_HIP(hipGetLastError());
     return ONHIP_OK;
 }

@@ -131,6 +131,18 @@ __device__ __forceinline__ unsigned f3_element(const IgemmProblem &p, const ColS
     return at == OOB ? OOB : at + q.soff + (BL == BL_TAPC ? (k % 4) * (unsigned) p.HW * 4u : 0u);
 }
 
+// Element j of eight split values: its parts add up to the scaled value exactly, or are a marker and the value's two halves
+// (split_weights_kernel).
+__device__ __forceinline__ float f3_whole(const uint4 (&part)[3], int j) {
+    auto up = [&](const uint4 &q) __attribute__((always_inline)) {
+        const unsigned w = j / 2 == 0 ? q.x : j / 2 == 1 ? q.y : j / 2 == 2 ? q.z : q.w;
+        return __uint_as_float(j % 2 ? w & 0xffff0000u : w << 16);
+    };
+    const float hi = up(part[0]), mid = up(part[1]), low = up(part[2]);
+    const float whole = __uint_as_float(__float_as_uint(mid) | __float_as_uint(low) >> 16);
+    return hi - hi == 0.0f ? ((hi + mid) + low) * (1.0f / F3_SCALE) : whole;
+}
+
 // Sums with the operands' scale taken out, and those that are not finite computed again in fp32 (see the head of the file): a wavefront that holds one multiplies its whole tile
 // again with v_mfma_f32_32x32x2_f32, operands straight from memory, and takes the elements that were not finite from there.
 // Sixteen of K a step, 8 (lane / 32) + j in MFMA j.  Units u_begin .. of the reduction up to klim elements.
@@ -184,14 +196,7 @@ __device__ __forceinline__ void unscale_fix_nonfinite(const IgemmProblem &p, f32
                 }
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                auto up = [&](const uint4 &q) __attribute__((always_inline)) {
-                    const unsigned w = j / 2 == 0 ? q.x : j / 2 == 1 ? q.y : j / 2 == 2 ? q.z : q.w;
-                    return __uint_as_float(j % 2 ? w & 0xffff0000u : w << 16);
-                };
-                // the parts add up to the scaled weight exactly, or are a marker and the weight's two halves (split_weights_kernel)
-                const float hi = up(part[0]), mid = up(part[1]), low = up(part[2]);
-                const float whole = __uint_as_float(__float_as_uint(mid) | __float_as_uint(low) >> 16);
-                const float av = hi - hi == 0.0f ? ((hi + mid) + low) * (1.0f / F3_SCALE) : whole;
+                const float av = f3_whole(part, j);
 #pragma unroll
                 for (int b = 0; b < TN; ++b) s[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv[b][j], s[b], 0, 0, 0);
             }
@@ -252,7 +257,167 @@ __device__ __forceinline__ void write_tile_rows(const IgemmProblem &p, f32x16 (&
     }
 }
 
-template <int BL, int BM, int BN, int WM, int WN, bool RES>
+// ---- a second, 1x1 product over the finished tile (the PW2 variant of the kernel, tile 64 x 64) --------------------------------
+// As pw2_stage of igemm_kernel.hpp, on the 16-bit matrix cores: the workgroup's tile, with bias and activation applied in fp32, is
+// split into its three parts and goes to LDS as the B operand of out[m2][64] = w2[m2][M] * tile ([part][row / 8][column][8 bf16]; a lane's
+// accumulator registers 4 q .. 4 q + 3 are half of such a slot).  Every wavefront then walks w2, split ahead of time like the first weights,
+// 32 rows at a time, four steps of 16 rows of the tile each: six matrix instructions a step, A two steps ahead from memory, B a step ahead
+// from LDS, no barrier.  A value that is not finite when scaled is kept as split_weights_kernel keeps one, so sums that are not finite
+// are computed again in fp32 from the same operands.
+// Bound by HBM in the first stage of a ResNet (the addend and the result): 3x3 64 -> 64 and 1x1 64 -> 256 with the Add on 56 x 56 at batch 32 take 95 us (231 MB;
+// 130 on fp32 matrix instructions), without it 87 (124).
+// tl: LDS of at least 3 * 8 * 64 * 16 bytes that no wavefront reads any more (the caller has synchronised).
+template <bool RES>
+__device__ __forceinline__ void pw2_split_stage(const IgemmProblem &p, const f32x16 &acc1, uint4 *tl, const float *sbias, int n0, int wm, int wn,
+                                                int li, int lh) {
+    const int cmid = p.M;
+    constexpr int STEPS = 4;   // 64 rows of the tile; those beyond cmid are zero
+    const int ksteps = (cmid + 15) / 16, lane = lh * 32 + li;
+    const rsrc_t rw2 = make_rsrc(p.w2, (unsigned) ((p.m2 + 31) / 32 * ksteps) * 3072u);
+    const unsigned pitch = (unsigned) ksteps * 3072u, lane16 = (unsigned) lane * 16u;
+    const int mblocks = (p.m2 + 63) / 64;
+    struct Step { uint4 part[3]; };
+    // nothing is read of steps beyond ksteps (their rows of the tile are zero as well) and of blocks of rows beyond m2
+    auto load_a = [&](Step &o, int mb, int s, int z) __attribute__((always_inline)) {
+        const bool on = s < ksteps && (mb * 2 + wm) * 32 < p.m2;   // uniform
+        o.part[z] = buf_load_b128(rw2, on ? lane16 : OOB, on ? (unsigned) (mb * 2 + wm) * pitch + (unsigned) s * 3072u + (unsigned) z * 1024u : 0u);
+    };
+    Step wa[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int z = 0; z < 3; ++z) load_a(wa[s], 0, s, z);
+    // none, Relu or Clip (the launcher refuses others): apply_act's comparisons as selects under two uniform flags
+    const bool lo_on = p.ep.act == RELU || p.ep.act == CLIP, hi_on = p.ep.act == CLIP;
+    const float lo = p.ep.act == CLIP ? p.ep.clip_min : 0.0f, hi = p.ep.clip_max;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const float4 t = *reinterpret_cast<const float4 *>(sbias + wm * 32 + 8 * q + 4 * lh);
+        const float b1[4] = {t.x, t.y, t.z, t.w};
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float x = __fadd_rn(acc1[4 * q + j], b1[j]);
+            x = (lo_on & !(x > lo)) ? lo : x;
+            x = (hi_on & !(x < hi)) ? hi : x;
+            v[j] = wm * 32 + 8 * q + 4 * lh + j < cmid ? x : 0.0f;
+        }
+        SplitUnit u;
+        u.phase<0>(v[0], v[1], v[2], v[3]);
+        const float probe = __builtin_fmaf(u.u0, 0.0f, __builtin_fmaf(u.u1, 0.0f, __builtin_fmaf(u.u2, 0.0f, u.u3 * 0.0f)));
+        const float first[4] = {u.u0, u.u1, u.u2, u.u3};
+        u.phase<1>(v[0], v[1], v[2], v[3]);
+        u.phase<2>(v[0], v[1], v[2], v[3]);
+        u.phase<3>(v[0], v[1], v[2], v[3]);
+        if (probe != probe) {
+            unsigned *h[2] = {&u.h0, &u.h1}, *m[2] = {&u.m0, &u.m1}, *l[2] = {&u.l0, &u.l1};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (first[j] - first[j] == 0.0f) continue;
+                const unsigned raw = __float_as_uint(v[j]), keep = j % 2 ? 0xffffu : 0xffff0000u, at = j % 2 * 16;
+                *h[j / 2] = (*h[j / 2] & keep) | 0x7f80u << at;
+                *m[j / 2] = (*m[j / 2] & keep) | (raw >> 16) << at;
+                *l[j / 2] = (*l[j / 2] & keep) | (raw & 0xffffu) << at;
+            }
+        }
+        uint2 *base = reinterpret_cast<uint2 *>(&tl[(wm * 4 + q) * 64 + wn * 32 + li]) + lh;
+        base[0] = make_uint2(u.h0, u.h1);
+        base[2 * 8 * 64] = make_uint2(u.m0, u.m1);
+        base[4 * 8 * 64] = make_uint2(u.l0, u.l1);
+    }
+    __syncthreads();
+    const uint4 *tbp = tl + lh * 64 + wn * 32 + li;
+    auto read_b = [&](Step &o, int s, int z) __attribute__((always_inline)) { o.part[z] = tbp[(z * 8 + 2 * s) * 64]; };
+    Step tb;
+#pragma unroll
+    for (int z = 0; z < 3; ++z) read_b(tb, 0, z);
+
+    const rsrc_t rc = make_rsrc(p.C, RSRC_RANGE);
+    const rsrc_t rres = make_rsrc(RES ? p.res : nullptr, RES ? RSRC_RANGE : 0u);
+    const rsrc_t rb2 = make_rsrc(p.bias2, p.bias2 ? (unsigned) (p.m2 * 4) : 0u);
+    const bool bias2_on = p.bias2 != nullptr, lo2_on = p.ep2.act == RELU || p.ep2.act == CLIP, hi2_on = p.ep2.act == CLIP;
+    const float lo2 = p.ep2.act == CLIP ? p.ep2.clip_min : 0.0f, hi2 = p.ep2.clip_max;
+    const unsigned row_bytes = (unsigned) p.c_stride_m * 4u, lh16 = (unsigned) lh * 16u;
+    const int n = n0 + wn * 32 + li, lh4 = 4 * lh;
+    const unsigned col_voff = n < p.N ? out_col_offset(p, n, 4) + (unsigned) lh4 * row_bytes : OOB;
+    // rows in groups of four: a lane's are inside or beyond m2 by group and remainder, asked again for the store
+    auto row_voff = [&](int m_uni) __attribute__((always_inline)) { return lh4 < p.m2 - m_uni ? col_voff : OOB; };
+    // relu.c's rule by element index: row offsets of this lane's column that lie in its body (one register, not sixteen sums)
+    const unsigned body = p.res_body * 4u > col_voff ? p.res_body * 4u - col_voff : 0u;
+    auto finish = [&](float v, float bias, float addend, int m_uni) __attribute__((always_inline)) {
+        v = bias2_on ? __fadd_rn(v, bias) : v;
+        v = (lo2_on & !(v > lo2)) ? lo2 : v;
+        v = (hi2_on & !(v < hi2)) ? hi2 : v;
+        if constexpr (RES) v = add_res(v, addend, p.res_relu, (unsigned) m_uni * row_bytes, body);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rc, row_voff(m_uni), (unsigned) m_uni * row_bytes, 0);
+    };
+    bool fine = true;   // every sum of the wavefront so far is finite (uniform)
+    for (int mb = 0; mb < mblocks; ++mb) {
+        const int m_wave = mb * 64 + wm * 32;   // uniform
+        float b2[16], rv[RES ? 16 : 1];
+        if constexpr (RES) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m_uni = m_wave + 8 * (r / 4) + (r % 4);
+                rv[r] = buf_load_f32(rres, row_voff(m_uni), (unsigned) m_uni * row_bytes);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        f32x16 acc2;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc2[r] = 0.0f;
+        static_for<STEPS>([&](auto step) __attribute__((always_inline)) {
+            constexpr int s = decltype(step)::value;
+            static_for<F3_PRODUCTS>([&](auto product) __attribute__((always_inline)) {
+                constexpr int pr = decltype(product)::value;
+                mma_bf16(acc2, wa[s & 1].part[f3_pa(pr)], tb.part[f3_pb(pr)]);
+                // two steps on, into the registers whose products are done
+                if constexpr (pr == 0 || pr == 2 || pr == 5) load_a(wa[s & 1], s + 2 < STEPS ? mb : mb + 1, (s + 2) % STEPS, f3_pa(pr));
+                if constexpr (pr >= 3) read_b(tb, (s + 1) % STEPS, f3_pb(pr));
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            if constexpr (s == STEPS - 2) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) b2[r] = buf_load_f32(rb2, lh16, (unsigned) (m_wave + 8 * (r / 4) + (r % 4)) * 4u);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        });
+        float probe = 0.0f;   // as in unscale_fix_nonfinite
+#pragma unroll
+        for (int r = 0; r < 16; ++r) probe = __builtin_fmaf(acc2[r], 0.0f, probe);
+        fine &= __builtin_amdgcn_ballot_w64(probe != probe) == 0ull;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) finish(acc2[r] * F3_UNSCALE, b2[r], RES ? rv[r] : 0.0f, m_wave + 8 * (r / 4) + (r % 4));
+    }
+    if (fine) return;
+    // All blocks once more, sums that are not finite from fp32 matrix instructions: a pass of its own, so that the one above
+    // keeps no registers for it.  Behind the stores that it writes over.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll 1
+    for (int mb = 0; mb < mblocks; ++mb) {
+        f32x16 acc2, again;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc2[r] = again[r] = 0.0f;
+#pragma unroll 1
+        for (int s = 0; s < STEPS; ++s) {
+            Step a;
+#pragma unroll
+            for (int z = 0; z < 3; ++z) { load_a(a, mb, s, z); read_b(tb, s, z); }
+            static_for<F3_PRODUCTS>([&](auto pr) __attribute__((always_inline)) { mma_bf16(acc2, a.part[f3_pa(pr)], tb.part[f3_pb(pr)]); });
+#pragma unroll
+            for (int j = 0; j < 8; ++j) again = __builtin_amdgcn_mfma_f32_32x32x2f32(f3_whole(a.part, j), f3_whole(tb.part, j), again, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int m_uni = mb * 64 + wm * 32 + 8 * (r / 4) + (r % 4);
+            const float bias = buf_load_f32(rb2, lh16, (unsigned) m_uni * 4u);
+            const float addend = RES ? buf_load_f32(rres, row_voff(m_uni), (unsigned) m_uni * row_bytes) : 0.0f;
+            finish(acc2[r] * 0.0f != 0.0f ? again[r] : acc2[r] * F3_UNSCALE, bias, addend, m_uni);
+        }
+    }
+}
+
+template <int BL, int BM, int BN, int WM, int WN, bool RES, bool PW2 = false>
 __global__ __launch_bounds__(64 * WM * WN, (BM / WM) * (BN / WN) >= 32 * 128 ? 2 : (BM / WM) * (BN / WN) >= 32 * 64 ? 3 : 4)
 void igemm_f3_kernel(const IgemmProblem p) {
     static_assert(BM % (WM * 32) == 0 && BN % (WN * 32) == 0, "wavefronts of 32 x 32 blocks");
@@ -261,7 +426,9 @@ void igemm_f3_kernel(const IgemmProblem p) {
     static_assert(BN * UPT == NT, "a thread stages one unit of B per K tile");
     constexpr int LD = BL == BL_ROWS ? BN + 1 : BN;   // 16-byte slots per 8 elements of K; rows arrive from neighbouring lanes
     constexpr int PLANE = 2 * LD, SLOTS = 3 * PLANE;
-    __shared__ uint4 lds[2 * SLOTS];   // two K tiles
+    static_assert(!PW2 || (BM == 64 && BN == 64 && WM == 2 && WN == 2), "the second product exists for tiles of 64 x 64");
+    __shared__ uint4 lds[PW2 ? 3 * 8 * 64 : 2 * SLOTS];   // two K tiles; with PW2 then the first product as three parts
+    static_assert(sizeof(lds) >= 2 * SLOTS * sizeof(uint4));
     __shared__ __attribute__((aligned(16))) float s_bias[BM];
 
     warm_params<sizeof(IgemmProblem)>();
@@ -271,7 +438,7 @@ void igemm_f3_kernel(const IgemmProblem p) {
     const int wm = wave / WN, wn = wave % WN;
 
     extern __shared__ __attribute__((aligned(1024))) float s_table[];   // TABLE_BYTES where table_in_lds says so
-    if (table_in_lds(p)) request_table(p.ep.lut, s_table, wave, lane, NT);
+    if (!PW2 && table_in_lds(p)) request_table(p.ep.lut, s_table, wave, lane, NT);
 
     const TilePlace tp = place_tile<BM, BN>(p);
     const int m0 = tp.m0, n0 = tp.n0, slice = tp.slice;
@@ -427,6 +594,10 @@ void igemm_f3_kernel(const IgemmProblem p) {
 
     const int m_wave = m0 + wm * (BM / WM), n_wave = n0 + wn * (BN / WN);
     unscale_fix_nonfinite<BL, TM, TN>(p, acc, ra, make_rsrc(b_base, b_bytes), m_wave, n_wave, lane, u_begin, klim);
+    if constexpr (PW2) {   // the launcher gives this variant one row tile and all of K
+        pw2_split_stage<RES>(p, acc[0][0], lds, s_bias, n0, wm, wn, li, lh);
+        return;
+    }
     if (p.partial) {   // a finishing launch adds the slices up
         write_partial<TM, TN, false>(p, acc, slice, m_wave, n_wave, li, lh);
         return;

@@ -241,7 +241,8 @@ struct IgemmParams {
     int n_fast;
     Div31 div_tiles_n;
     // a second, 1x1 product over the finished tile (igemm_kernel's PW2 variant, one row tile: M <= 64): the M rows of the
-    // first product, with `bias` and `ep` applied, are the reduction of w2 ([m2][M], in pack_pw2_launch's order).  C, the
+    // first product, with `bias` and `ep` applied, are the reduction of w2 ([m2][M], in pack_pw2_launch's order, or split where the
+    // problem's a_split is given).  C, the
     // c_* strides and res then describe the m2-row result, bias2 and ep2 its epilogue; the M-row tensor between the two
     // never exists
     const float *w2;
@@ -284,8 +285,8 @@ struct IgemmLaunch {
 
 int igemm_launch(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t stream);
 // fp32 convolution followed by a 1x1 convolution over its result in one launch (igemm_f32_pw.hip): p as for the tap-major
-// packed loader with M <= 64 rows, plus w2 / bias2 / m2 / ep2
-int igemm_launch_f32_pw(const IgemmParams &p, hipStream_t stream);
+// packed loader with M <= 64 rows, plus w2 / bias2 / m2 / ep2; with a_split, w2 is split as well (igemm_f3_pw.hip)
+int igemm_launch_f32_pw(const IgemmProblem &p, hipStream_t stream);
 // fp32 kernel for plain problems with B rows contiguous along N (igemm_rowb.hip): tiles 64x128, 128x128, 64x256
 bool rowb_f32_ok(const IgemmLaunch &cfg, const IgemmParams &p);
 int rowb_f32_launch(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t stream);
@@ -307,6 +308,10 @@ struct SplitKeeper {
 // api.hip: fp32 convolution and product whose caller keeps the weights split
 int conv2d_f32_kept(const onhip_conv_desc_t *d, const float *x, const float *w, int packed, const float *bias, const float *silu_lut,
                     const float *addend, int relu_after, float *y, const SplitKeeper *keeper, void *stream);
+// a convolution and the 1x1 convolution after it (onhip_conv2d_pw_f32); wb: the second one's weights as given, wb_packed in the plain kernel's order
+int conv2d_pw_f32_kept(const onhip_conv_desc_t *a, const onhip_conv_desc_t *b, const float *x, const float *wa_packed, const float *bias_a,
+                       const float *wb, const float *wb_packed, const float *bias_b, const float *addend, int relu_after, float *y,
+                       const SplitKeeper *keep_a, const SplitKeeper *keep_b, void *stream);
 int matmul_f32_kept(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias, const float *gelu_lut, const float *addend,
                     float *out, const SplitKeeper *keeper, void *stream);
 // `parts` products of the shape d on one left operand, weights [k][parts * n] and biases side by side, results out_step bytes apart: as one

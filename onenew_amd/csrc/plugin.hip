@@ -669,8 +669,11 @@ static int conv_pair_eval_mode(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUF
     if (!rc && !wa_packed) rc = set_error(ONHIP_ERR_ARG, "Conv pair eval: the first convolution has no packed weight form");
     if (!rc) rc = packed_pair_weights(&d[1], (const float *) wb, &wb_packed);
     if (rc) return rc;
-    rc = onhip_conv2d_pw_f32(&d[0], &d[1], (const float *) x, wa_packed, (const float *) ba, wb_packed, (const float *) bb,
-                             (const float *) addend, relu ? 1 : 0, (float *) y, g_stream);
+    // weights that stay as they are, as in conv_eval_fused
+    const bool stay = (wa != reinterpret_cast<const void *>(inputs[1].addr) || is_held(wa)) && (wb != reinterpret_cast<const void *>(inputs[5].addr) || is_held(wb));
+    const SplitKeeper keep_a = {wa, split_of}, keep_b = {wb, split_of};
+    rc = conv2d_pw_f32_kept(&d[0], &d[1], (const float *) x, wa_packed, (const float *) ba, (const float *) wb, wb_packed, (const float *) bb,
+                            (const float *) addend, relu ? 1 : 0, (float *) y, stay ? &keep_a : nullptr, stay ? &keep_b : nullptr, g_stream);
     if (rc) return rc;
     return out_on_dev ? wait_for_output() : copy_out(host_out, y, out_bytes);
 }
