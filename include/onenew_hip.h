@@ -543,6 +543,10 @@ int onhip_matmul_bias_gelu_eval(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BU
  * result, in one call (onhip_matmul_add).  Slots as for `eval_bias`; the second addend travels in inputs[3] (it has the
  * result's operand, so no params slot of its own), as the addend of the Conv plugin's `eval_add` does. */
 int onhip_matmul_bias_add_eval(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_INFO_S *outputs);
+/* `eval_bias_add_norm` of libMatMul_hip.so: `eval_bias_add`, and the LayerNormalization of the result over its last axis as a second result
+ * (in the same launch where a tile of the product holds whole rows, else as onhip_layernorm_f32; the same bits either way).  Slots as for
+ * `eval_bias_add`; inputs[5] / inputs[6] = the normalisation's weight and bias, outputs[1] = the normalised tensor, all in device memory. */
+int onhip_matmul_bias_add_norm_eval(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_INFO_S *outputs);
 /* `eval_bias_group` of libMatMul_hip.so: up to four products with a bias on one left operand (the q, k and v projections of an attention
  * block), in one launch where that is expected to be faster, one after the other where not; the values of `eval_bias` for each either way.
  * Slots as for `eval_bias` of the first product, whose weight, bias and result all of them share the shapes of; inputs[4] = the address of an

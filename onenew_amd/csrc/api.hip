@@ -1815,7 +1815,7 @@ static bool rows_form(const IgemmLaunch &cfg, const IgemmProblem &p, RowsForm *f
 
 // rows_us: nothing is launched; what the rows form takes where the product would run in it, else 0
 static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias, const float *gelu_lut, const float *addend,
-                       float *out, void *stream, const SplitKeeper *keeper = nullptr, double *rows_us = nullptr) {
+                       float *out, void *stream, const SplitKeeper *keeper = nullptr, double *rows_us = nullptr, RowNorm *norm = nullptr) {
     if (!d || d->batch < 1 || d->m < 1 || d->k < 1 || d->n < 1) return set_error(ONHIP_ERR_ARG, "matmul: bad shape");
     if (!a || !b || !out) return set_error(ONHIP_ERR_ARG, "matmul: null tensor pointer");
     int batch = d->batch, M = d->m;
@@ -1878,6 +1878,7 @@ static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float
         if (rows_form(cfg, p, &form, &us)) {
             if (rows_us) { *rows_us = form.faster ? us : 0.0; return ONHIP_OK; }
             form.p.keeper = keeper;
+            form.p.norm = tune_mode() ? nullptr : norm;   // measuring launches the product many times
             return plan_and_launch(cfg, p, st, &form);
         }
     }
@@ -2296,8 +2297,8 @@ int conv2d_pw_f32_kept(const onhip_conv_desc_t *a, const onhip_conv_desc_t *b, c
     return conv2d_pw_impl(a, b, x, wa_packed, bias_a, wb, wb_packed, bias_b, addend, relu_after, y, keep_a, keep_b, stream);
 }
 int matmul_f32_kept(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias, const float *gelu_lut, const float *addend,
-                    float *out, const SplitKeeper *keeper, void *stream) {
-    return matmul_impl(d, a, b, bias, gelu_lut, addend, out, stream, keeper);
+                    float *out, const SplitKeeper *keeper, void *stream, RowNorm *norm) {
+    return matmul_impl(d, a, b, bias, gelu_lut, addend, out, stream, keeper, nullptr, norm);
 }
 int matmul_group_f32_kept(const onhip_matmul_desc_t *d, int parts, const float *a, const float *w_all, const float *bias_all, float *out, long long out_step,
                           const SplitKeeper *keeper, void *stream, bool *ran) {

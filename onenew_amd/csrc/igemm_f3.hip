@@ -16,6 +16,7 @@ int f3_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t stream)
         case BL_TAPC: return f3_launch_tapc(cfg, p, stream);
         case BL_ROWS:
             if (p.partial) return set_error(ONHIP_ERR_ARG, "igemm f3: no split along K for rows");
+            if (f3_norm_ok(cfg, p)) return f3_launch_norm(cfg, p, stream);
             return p.res ? f3_launch_tile<BL_ROWS, true>(cfg, p, stream) : f3_launch_tile<BL_ROWS, false>(cfg, p, stream);
         default: return set_error(ONHIP_ERR_ARG, "igemm f3: unsupported loader %d", cfg.bl);
     }

@@ -34,6 +34,7 @@
 // opt_gemm.h SGEMM (:17) + bias sweep (:405) + do_act (:1216); device/x86/MatMul/mat_mul.c:10.
 #pragma once
 #include "igemm_kernel.hpp"
+#include "row_norm.hpp"
 
 namespace onhip {
 
@@ -211,9 +212,10 @@ __device__ __forceinline__ void unscale_fix_nonfinite(const IgemmProblem &p, f32
 // The store for B given as rows (a product's left operand): C is row-major with the tile's columns as its rows, so the four
 // consecutive rows of the tile that a lane holds in registers 4 q .. 4 q + 3 are 16 contiguous bytes of C.  Residual and bias
 // as in write_tile.
-template <int EPI, int TM, int TN, bool RES>
+// norm_row: LDS for the lane's row of C as well, at its first column (the variant that normalises the rows), or nullptr.
+template <int EPI, int TM, int TN, bool RES, bool NORM = false>
 __device__ __forceinline__ void write_tile_rows(const IgemmProblem &p, f32x16 (&acc)[TM][TN], int m_wave, int n_wave, int li, int lh,
-                                                const float *sbias, lds_f32_t table) {
+                                                const float *sbias, lds_f32_t table, float *norm_row = nullptr) {
     const rsrc_t rc = make_rsrc(p.C, (unsigned) p.c_slice_bytes), rr = make_rsrc(RES ? p.res : nullptr, RES ? (unsigned) p.c_slice_bytes : 0u);
 #pragma unroll
     for (int b = 0; b < TN; ++b) {
@@ -245,6 +247,10 @@ __device__ __forceinline__ void write_tile_rows(const IgemmProblem &p, f32x16 (&
                     o[j] = __float_as_uint(v[j]);
                 }
                 const int left = p.M - (m4 + 8 * q);   // columns of C from this group on
+                if constexpr (NORM)
+                    if (left > 0)   // rows of a multiple of four
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) norm_row[m4 + 8 * q + j] = v[j];
                 if (left >= 4) {
                     __builtin_amdgcn_raw_buffer_store_b128(o, rc, base + 32u * q, 0, 0);
                 } else {
@@ -254,6 +260,36 @@ __device__ __forceinline__ void write_tile_rows(const IgemmProblem &p, f32x16 (&
                 }
             }
         }
+    }
+}
+
+// A problem whose rows of C are normalised as well (RowNorm): what the kernel takes of it.
+struct IgemmNormProblem : IgemmProblem {
+    const float *norm_w, *norm_b;
+    float *norm_y, inv_n;
+};
+
+// ---- LayerNormalization of the finished tile's rows (the NORM variant, rows of B, one tile over all columns of C) ------------------------
+// The tile holds whole rows of C, so their LayerNormalization needs no launch of its own and no trip to memory in between: the store leaves
+// a copy in LDS (odd pitch), a wavefront adds up the 64 rows, another one their squares, all of them normalise.  Same operations in the same
+// order as layernorm_rows4_kernel: the same bits.  A chain of M additions and a pass over LDS are 3 to 4 us more on the product (12544 rows of
+// 192 columns from K = 192 15.8 -> 19.0, from K = 768 34.4 -> 38.6) instead of a launch of 6.8; ViT-Tiny at batch 64 1866 -> 1756 us.
+__device__ __forceinline__ void normalise_rows(const IgemmNormProblem &p, const float *tile, float *stats, int n0, int tid) {
+    const int pitch = p.M + 1, rows = min(64, p.N - n0), groups = p.M / 4, lane = tid & 63, wave = tid >> 6;
+    // a thread keeps its four columns and walks down the rows
+    const int per_pass = 256 / groups, r0 = tid / groups, c = tid - r0 * groups;
+    const float4 w = reinterpret_cast<const float4 *>(p.norm_w)[c], b = reinterpret_cast<const float4 *>(p.norm_b)[c];
+    __syncthreads();
+    if (wave < 2 && lane < rows) stats[wave * 64 + lane] = wave == 0 ? ln_chain<false>(tile + lane * pitch, p.M) : ln_chain<true>(tile + lane * pitch, p.M);
+    __syncthreads();
+    if (tid < rows) ln_stats(stats[tid], stats[64 + tid], p.inv_n, &stats[tid], &stats[64 + tid]);
+    __syncthreads();
+    if (r0 >= per_pass) return;
+    for (int r = r0; r < rows; r += per_pass) {
+        const float *t = tile + r * pitch + 4 * c;
+        const float m = stats[r], s = stats[64 + r];
+        const float4 o = make_float4(ln_one(t[0], m, s, w.x, b.x), ln_one(t[1], m, s, w.y, b.y), ln_one(t[2], m, s, w.z, b.z), ln_one(t[3], m, s, w.w, b.w));
+        reinterpret_cast<float4 *>(p.norm_y + (size_t) (n0 + r) * p.M)[c] = o;
     }
 }
 
@@ -417,9 +453,10 @@ __device__ __forceinline__ void pw2_split_stage(const IgemmProblem &p, const f32
     }
 }
 
-template <int BL, int BM, int BN, int WM, int WN, bool RES, bool PW2 = false>
+template <int BL, int BM, int BN, int WM, int WN, bool RES, bool PW2 = false, bool NORM = false>
 __global__ __launch_bounds__(64 * WM * WN, (BM / WM) * (BN / WN) >= 32 * 128 ? 2 : (BM / WM) * (BN / WN) >= 32 * 64 ? 3 : 4)
-void igemm_f3_kernel(const IgemmProblem p) {
+void igemm_f3_kernel(const std::conditional_t<NORM, IgemmNormProblem, IgemmProblem> p) {
+    static_assert(!NORM || (BL == BL_ROWS && WM * WN == 4 && BN == 64 && RES), "rows are normalised behind a residual operand, four wavefronts, 64 rows a tile");
     static_assert(BM % (WM * 32) == 0 && BN % (WN * 32) == 0, "wavefronts of 32 x 32 blocks");
     constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
     constexpr int UPT = 4, NT = 64 * WM * WN;
@@ -431,14 +468,14 @@ void igemm_f3_kernel(const IgemmProblem p) {
     static_assert(sizeof(lds) >= 2 * SLOTS * sizeof(uint4));
     __shared__ __attribute__((aligned(16))) float s_bias[BM];
 
-    warm_params<sizeof(IgemmProblem)>();
+    warm_params<(sizeof(p) < 640 ? sizeof(p) : 640)>();
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 31, lh = lane >> 5;
     const int wm = wave / WN, wn = wave % WN;
 
     extern __shared__ __attribute__((aligned(1024))) float s_table[];   // TABLE_BYTES where table_in_lds says so
-    if (!PW2 && table_in_lds(p)) request_table(p.ep.lut, s_table, wave, lane, NT);
+    if (!PW2 && !NORM && table_in_lds(p)) request_table(p.ep.lut, s_table, wave, lane, NT);   // NORM: s_table is the rows' copy
 
     const TilePlace tp = place_tile<BM, BN>(p);
     const int m0 = tp.m0, n0 = tp.n0, slice = tp.slice;
@@ -603,6 +640,12 @@ void igemm_f3_kernel(const IgemmProblem p) {
         return;
     }
     const float *sb = s_bias + wm * (BM / WM);
+    if constexpr (NORM) {   // the launcher gives this variant no activation and a tile over all of M
+        write_tile_rows<EPI_NONE, TM, TN, RES, true>(p, acc, m_wave, n_wave, li, lh, sb, (lds_f32_t) nullptr, s_table + (wn * (BN / WN) + li) * (p.M + 1));
+        static_assert(TN == 1 && BM >= 128, "a lane holds one row; the bias's LDS takes the statistics");
+        normalise_rows(p, s_table, s_bias, n0, tid);
+        return;
+    }
     auto store = [&](auto epi) __attribute__((always_inline)) {
         constexpr int EPI = decltype(epi)::value;
         if constexpr (BL == BL_ROWS) write_tile_rows<EPI, TM, TN, RES>(p, acc, m_wave, n_wave, li, lh, sb, (lds_f32_t) s_table);
@@ -629,6 +672,26 @@ static int f3_launch_one(const IgemmLaunch &cfg, const IgemmProblem &p_in, hipSt
     hipLaunchKernelGGL((igemm_f3_kernel<BL, BM, BN, WM, WN, RES>), grid, dim3(64 * WM * WN), table_lds_bytes(p), stream, p);
     ONHIP_CHECK_HIP(hipGetLastError());
     return finish_launch<false>(cfg, p, stream);
+}
+
+// The rows of C normalised in the product's launch: the tile covers all columns, results and parameters are whole 16-byte pieces.
+inline bool f3_norm_ok(const IgemmLaunch &cfg, const IgemmProblem &p) {
+    const RowNorm *r = p.norm;
+    return r && cfg.bl == BL_ROWS && cfg.bm == 192 && cfg.bn == 64 && p.res && !p.partial && !p.c_part && p.M <= 192 && p.M >= 32 && p.M % 4 == 0 &&
+           p.c_stride_n == p.M && p.ep.act == NOT_ACT &&
+           ((reinterpret_cast<uintptr_t>(r->w) | reinterpret_cast<uintptr_t>(r->b) | reinterpret_cast<uintptr_t>(r->y)) & 15) == 0;
+}
+inline int f3_launch_norm(const IgemmLaunch &cfg, const IgemmProblem &p_in, hipStream_t stream) {
+    IgemmNormProblem p;
+    static_cast<IgemmProblem &>(p) = p_in;
+    dim3 grid;
+    const int rc = tile_grid<192, 64>(cfg, p, &grid);
+    if (rc) return rc;
+    p.norm_w = p_in.norm->w; p.norm_b = p_in.norm->b; p.norm_y = p_in.norm->y; p.inv_n = 1.0f / p.M;
+    hipLaunchKernelGGL((igemm_f3_kernel<BL_ROWS, 192, 64, 2, 2, true, false, true>), grid, dim3(256), 64 * (p.M + 1) * 4, stream, p);
+    ONHIP_CHECK_HIP(hipGetLastError());
+    p_in.norm->done = true;
+    return ONHIP_OK;
 }
 
 template <int BL, bool RES>

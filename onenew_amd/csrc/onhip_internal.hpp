@@ -270,6 +270,15 @@ struct IgemmProblem : IgemmParams {
     // i * c_part_step bytes after the first one's
     int c_part;
     unsigned c_part_step;
+    struct RowNorm *norm;      // the caller would have the rows of C normalised as well, or nullptr
+};
+
+// LayerNormalization of a product's rows, in the product's launch where its kernel can (done says whether it did): y = the rows of the
+// result, laid out like it, normalised with w and b.
+struct RowNorm {
+    const float *w, *b;
+    float *y;
+    bool done;
 };
 
 enum { DT_F32 = 0, DT_BF16 = 1, DT_F16 = 2, DT_I8 = 3 };
@@ -313,7 +322,7 @@ int conv2d_pw_f32_kept(const onhip_conv_desc_t *a, const onhip_conv_desc_t *b, c
                        const float *wb, const float *wb_packed, const float *bias_b, const float *addend, int relu_after, float *y,
                        const SplitKeeper *keep_a, const SplitKeeper *keep_b, void *stream);
 int matmul_f32_kept(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias, const float *gelu_lut, const float *addend,
-                    float *out, const SplitKeeper *keeper, void *stream);
+                    float *out, const SplitKeeper *keeper, void *stream, struct RowNorm *norm = nullptr);
 // `parts` products of the shape d on one left operand, weights [k][parts * n] and biases side by side, results out_step bytes apart: as one
 // launch if that is expected to be faster than each on its own, which then has the same bits (*ran says whether)
 int matmul_group_f32_kept(const onhip_matmul_desc_t *d, int parts, const float *a, const float *w_all, const float *bias_all, float *out, long long out_step,

@@ -710,7 +710,8 @@ static int conv_link_eval_locked(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, B
 
 // mode 0: MatMul.  mode 1: MatMul -> Add of a bias over the last axis (params[3] / inputs[2], n elements; the result's
 // operand moves to params[4]).  mode 2: -> Gelu as well, through the table in inputs[11] like the Gelu operator.
-// mode 3: mode 1 -> Add of the tensor in inputs[3], which has the result's shape.
+// mode 3: mode 1 -> Add of the tensor in inputs[3], which has the result's shape.  mode 4: mode 3, and the LayerNormalization of the
+// result's rows into outputs[1] (weight and bias in inputs[5], inputs[6]).
 static int matmul_eval_mode(int mode, BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_INFO_S *outputs) {
     const OPERAND_S *a_t = reinterpret_cast<const OPERAND_S *>(params[1].addr);
     const OPERAND_S *b_t = reinterpret_cast<const OPERAND_S *>(params[2].addr);
@@ -762,12 +763,16 @@ static int matmul_eval_mode(int mode, BUFFER_INFO_S *params, BUFFER_INFO_S *inpu
         rc = const_on_device(reinterpret_cast<const void *>(inputs[BUF_MAXNUM - 1].addr), 8192 * 4, &lut);
         if (rc) return rc;
     }
-    if (mode == 3) {
+    if (mode >= 3) {
         if (!inputs[3].addr) return set_error(ONHIP_ERR_ARG, "MatMul eval: no addend in inputs[3]");
         const void *addend;
         rc = input_on_device(5, reinterpret_cast<const void *>(inputs[3].addr), o_bytes, &addend);
         if (rc) return rc;
-        rc = matmul_f32_kept(&d, (const float *) a, (const float *) b, (const float *) bias, nullptr, (const float *) addend, (float *) y, keeper, g_stream);
+        RowNorm norm = {reinterpret_cast<const float *>(inputs[5].addr), reinterpret_cast<const float *>(inputs[6].addr), reinterpret_cast<float *>(outputs[1].addr), false};
+        if (mode == 4 && (!norm.w || !norm.b || !norm.y || !out_on_dev || !is_device_ptr(norm.w) || !is_device_ptr(norm.b) || !is_device_ptr(norm.y)))
+            return set_error(ONHIP_ERR_ARG, "MatMul eval: LayerNormalization on tensors in device memory only");
+        rc = matmul_f32_kept(&d, (const float *) a, (const float *) b, (const float *) bias, nullptr, (const float *) addend, (float *) y, keeper, g_stream, mode == 4 ? &norm : nullptr);
+        if (!rc && mode == 4 && !norm.done) rc = onhip_layernorm_f32((int32_t) (o_bytes / 4 / d.n), d.n, 0, (const float *) y, norm.w, norm.b, norm.y, g_stream);
     } else {
         rc = matmul_f32_kept(&d, (const float *) a, (const float *) b, (const float *) bias, (const float *) lut, nullptr, (float *) y, keeper, g_stream);
     }
@@ -803,6 +808,10 @@ static int matmul_bias_gelu_eval_locked(BUFFER_INFO_S *params, BUFFER_INFO_S *in
 }
 static int matmul_bias_add_eval_locked(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_INFO_S *outputs) {
     return matmul_eval_mode(3, params, inputs, outputs);
+}
+
+static int matmul_bias_add_norm_eval_locked(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_INFO_S *outputs) {
+    return matmul_eval_mode(4, params, inputs, outputs);
 }
 
 static int matmul_bias_group_eval_locked(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_INFO_S *outputs) {
@@ -1259,6 +1268,9 @@ int onhip_matmul_bias_eval(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_
 }
 int onhip_matmul_bias_gelu_eval(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_INFO_S *outputs) {
     return guarded("MatMul (+ bias + Gelu)", matmul_bias_gelu_eval_locked, params, inputs, outputs);
+}
+int onhip_matmul_bias_add_norm_eval(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_INFO_S *outputs) {
+    return guarded("MatMul (+ bias + Add + LayerNormalization)", matmul_bias_add_norm_eval_locked, params, inputs, outputs);
 }
 int onhip_matmul_bias_add_eval(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_INFO_S *outputs) {
     return guarded("MatMul (+ bias + Add)", matmul_bias_add_eval_locked, params, inputs, outputs);

@@ -36,6 +36,12 @@ extern "C" __attribute__((visibility("default"))) int eval_bias_add(BUFFER_INFO_
                                                                     BUFFER_INFO_S *outputs) {
     return onhip_matmul_bias_add_eval(params, inputs, outputs);
 }
+// eval_bias_add -> LayerNormalization of the result over its last axis, both results kept: weight and bias in inputs[5] and inputs[6], the
+// normalised tensor in outputs[1]; device memory throughout.
+extern "C" __attribute__((visibility("default"))) int eval_bias_add_norm(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs,
+                                                                         BUFFER_INFO_S *outputs) {
+    return onhip_matmul_bias_add_norm_eval(params, inputs, outputs);
+}
 // Several products with a bias on one left operand (the q, k and v projections of an attention block): as one launch where that is faster.
 // inputs[4] = an onhip_product_group_t.
 extern "C" __attribute__((visibility("default"))) int eval_bias_group(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs,

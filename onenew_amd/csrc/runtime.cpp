@@ -142,7 +142,8 @@ struct Node {
     int32_t link_fuse = 0;
     // products on one left operand that run in one call (group_products): the nodes, this one first; and on the others that they do not run
     std::vector<int> group;
-    bool in_group = false;
+    bool in_group = false;                   // also a LayerNormalization that its product's call does (normalise_in_products)
+    int norm = -1;                           // that LayerNormalization, on the product
     std::string group_w, group_b;            // their weights and biases side by side
     onhip_product_group_t group_args = {};
     bool reads_twin = false;   // its input is the int8 copy of an fp32 operand
@@ -184,7 +185,7 @@ struct onrt_net {
     onenew_eval_fn conv_block = nullptr, conv_block_takes = nullptr, conv_link = nullptr, conv_link_takes = nullptr;
     onenew_eval_fn conv_pair = nullptr, conv_pair_relu = nullptr, conv_pair_takes = nullptr;
     onenew_eval_fn maxpool_s8 = nullptr;   // optional entry point of the MaxPool plugin
-    onenew_eval_fn matmul_attention = nullptr, matmul_bias = nullptr, matmul_bias_gelu = nullptr, matmul_bias_add = nullptr, matmul_bias_group = nullptr;   // optional entry points of the MatMul plugin
+    onenew_eval_fn matmul_attention = nullptr, matmul_bias = nullptr, matmul_bias_gelu = nullptr, matmul_bias_add = nullptr, matmul_bias_group = nullptr, matmul_bias_add_norm = nullptr;   // optional entry points of the MatMul plugin
     int fused_blocks = 0, folded_relus = 0, folded_acts = 0, fused_attentions = 0, fused_linears = 0, fused_skips = 0, fused_ir_blocks = 0, fused_pairs = 0, int8_links = 0;
     void *init_arena = nullptr, *act_arena = nullptr, *tables = nullptr;
     std::vector<float> silu_lut, gelu_lut;
@@ -576,6 +577,7 @@ int bind_plugins(onrt_net &net) {
             net.matmul_bias_gelu = reinterpret_cast<onenew_eval_fn>(dlsym(it->second, "eval_bias_gelu"));
             net.matmul_bias_add = reinterpret_cast<onenew_eval_fn>(dlsym(it->second, "eval_bias_add"));
             net.matmul_bias_group = reinterpret_cast<onenew_eval_fn>(dlsym(it->second, "eval_bias_group"));
+            net.matmul_bias_add_norm = reinterpret_cast<onenew_eval_fn>(dlsym(it->second, "eval_bias_add_norm"));
         }
     }
     return ONRT_OK;
@@ -1278,6 +1280,33 @@ int group_products(onrt_net &net) {
     return ONRT_OK;
 }
 
+// The LayerNormalization of a product's result behind a skip connection (fuse 6): the product's call makes both tensors, in one launch where
+// a tile of it holds whole rows.  It stays in the order with nothing to do, like the followers of a group.
+int normalise_in_products(onrt_net &net) {
+    if (!fusing_enabled() || !net.matmul_bias_add_norm) return ONRT_OK;
+    for (int idx : net.order) {
+        Node &mm = net.nodes[idx];
+        if (strcmp(mm.kind->type, "MatMul") || mm.fuse != 6) continue;
+        const Tensor &y = net.tensors[mm.fused_out];
+        const int rank = y.desc.dim_num_of_shapes, n = y.desc.shapes[rank - 1];
+        if (n < 2 || !y.alias.empty() || y.never_written || y.as_s8 || y.has_twin) continue;
+        for (int r : readers_of(net, mm.fused_out)) {
+            Node &ln = net.nodes[r];
+            if (strcmp(ln.kind->type, "LayerNormalization") || ln.in.size() != 3 || ln.out.size() != 1 || ln.in[0] != mm.fused_out || ln.in_group) continue;
+            if (reinterpret_cast<const LAYERNORMALIZATION_CONFIG_S *>(ln.cfg.data())->axes[0] == 1) continue;   // over axis 1 (layer_normalization.c:28)
+            const Tensor &w = net.tensors[ln.in[1]], &b = net.tensors[ln.in[2]], &out = net.tensors[ln.out[0]];
+            if (!w.is_init || !b.is_init || w.bytes != (size_t) n * 4 || b.bytes != (size_t) n * 4 || !out.alias.empty() || out.never_written ||
+                out.as_s8 || out.has_twin || numel(out.desc) != numel(y.desc) || !ln.fused_out.empty())
+                continue;
+            mm.norm = r;
+            mm.eval = net.matmul_bias_add_norm;
+            ln.in_group = true;
+            break;
+        }
+    }
+    return ONRT_OK;
+}
+
 // ---- slot arrays (op::rt_prepare, host/op.h:109-168, and prepare_init_operand_data of each operator) ----
 int fill_slots(onrt_net &net) {
     const size_t lut_len = net.silu_lut.size();
@@ -1345,6 +1374,12 @@ int fill_slots(onrt_net &net) {
             nd.params[out_slot].addr = (int64_t) &t.desc;
             nd.outputs[k].addr = (int64_t) t.dev;
         }
+        if (nd.norm >= 0) {
+            const Node &ln = net.nodes[nd.norm];
+            nd.inputs[5].addr = (int64_t) net.tensors[ln.in[1]].dev;
+            nd.inputs[6].addr = (int64_t) net.tensors[ln.in[2]].dev;
+            nd.outputs[1].addr = (int64_t) net.tensors[ln.out[0]].dev;
+        }
         if (nd.link.twin) nd.outputs[1].addr = (int64_t) net.tensors[nd.fused_out.empty() ? nd.out[0] : nd.fused_out].twin_dev;
         // per-model tunables in the last params slot (host/ops/conv.h:66-69, host/ops/maxpool.h:57-62); the
         // HIP operators bring their own workspace, so the shared scratch buffer stays unallocated
@@ -1372,6 +1407,7 @@ int prepare(onrt_net &net, const char *op_lib_dir) {
     if (!rc) rc = fuse_linear(net);
     if (!rc) rc = link_int8_convs(net);
     if (!rc) rc = group_products(net);
+    if (!rc) rc = normalise_in_products(net);
     if (!rc) rc = allocate(net);
     if (!rc) rc = build_tables(net);
     if (!rc) rc = fill_slots(net);

@@ -7,7 +7,7 @@
 
 #include <type_traits>
 
-#include "onhip_internal.hpp"
+#include "row_norm.hpp"
 
 namespace onhip {
 
@@ -43,22 +43,6 @@ __global__ __launch_bounds__(256) void gelu_lut_kernel(const float *__restrict__
 }
 
 // ---- LayerNormalization ---------------------------------------------------------------------------------
-// layer_normalization.c:62-97: per row, psum and psum of squares added up element by element in float, then
-// mean = psum / n (as a product with 1/n), var = (1/n) * psq - mean * mean, + 1e-20 (a double constant),
-// 1 / sqrtf(var), and out = (x - mean) * inv_std * weight + bias with every operation rounded.
-__device__ __forceinline__ void ln_stats(float psum, float psq, float inv_n, float *mean, float *inv_std) {
-    const float m = __fmul_rn(psum, inv_n);
-    float var = __fsub_rn(__fmul_rn(inv_n, psq), __fmul_rn(m, m));
-    var = (float) ((double) var + 1e-20);
-    *mean = m;
-    // sqrtf, then 1 / std, each correctly rounded as on the CPU.  The single-precision square root of this
-    // toolchain is the bare v_sqrt_f32 (a last bit off on some inputs); the double-precision one rounded to float
-    // is exact (53 >= 2 * 24 + 2 bits).  The two steps are kept apart so that they cannot merge into v_rsq_f32.
-    float sd = (float) sqrt((double) var);
-    asm volatile("" : "+v"(sd));
-    *inv_std = __fdiv_rn(1.0f, sd);
-}
-
 constexpr int LN_LDS_FLOATS = 8192;
 
 // rows contiguous in memory: a workgroup stages `rpw` rows in LDS (pitch reduce + 1, so the threads that
@@ -142,30 +126,8 @@ __global__ __launch_bounds__(256) void layernorm_rows4_kernel(const float *__res
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (wave < 2 && lane < nr) {
         const float *t = tile + lane * pitch;
-        auto chain = [&](auto squares) {
-            constexpr bool SQ = decltype(squares)::value;
-            constexpr int AHEAD = 16;   // elements read ahead of the additions
-            float sum = 0.0f, next[AHEAD];
-            auto add = [&](float v) { sum = __fadd_rn(sum, SQ ? __fmul_rn(v, v) : v); };
-#pragma unroll
-            for (int j = 0; j < AHEAD; ++j) next[j] = t[j];
-            int i = AHEAD;
-            for (; i + AHEAD <= reduce; i += AHEAD) {
-                float now[AHEAD];
-#pragma unroll
-                for (int j = 0; j < AHEAD; ++j) now[j] = next[j];
-#pragma unroll
-                for (int j = 0; j < AHEAD; ++j) next[j] = t[i + j];
-#pragma unroll
-                for (int j = 0; j < AHEAD; ++j) add(now[j]);
-            }
-#pragma unroll
-            for (int j = 0; j < AHEAD; ++j) add(next[j]);
-            for (; i < reduce; ++i) add(t[i]);
-            return sum;
-        };
-        if (wave == 0) s_mean[lane] = chain(std::false_type{});
-        else s_inv[lane] = chain(std::true_type{});
+        if (wave == 0) s_mean[lane] = ln_chain<false>(t, reduce);
+        else s_inv[lane] = ln_chain<true>(t, reduce);
     }
     __syncthreads();
     if ((int) threadIdx.x < nr) ln_stats(s_mean[threadIdx.x], s_inv[threadIdx.x], inv_n, &s_mean[threadIdx.x], &s_inv[threadIdx.x]);
@@ -176,10 +138,10 @@ __global__ __launch_bounds__(256) void layernorm_rows4_kernel(const float *__res
         if (at[i] < 0) continue;
         const float m = s_mean[row[i]], s = s_inv[row[i]];
         float4 o;
-        o.x = __fadd_rn(__fmul_rn(__fmul_rn(__fsub_rn(v[i].x, m), s), wv[i].x), bv[i].x);
-        o.y = __fadd_rn(__fmul_rn(__fmul_rn(__fsub_rn(v[i].y, m), s), wv[i].y), bv[i].y);
-        o.z = __fadd_rn(__fmul_rn(__fmul_rn(__fsub_rn(v[i].z, m), s), wv[i].z), bv[i].z);
-        o.w = __fadd_rn(__fmul_rn(__fmul_rn(__fsub_rn(v[i].w, m), s), wv[i].w), bv[i].w);
+        o.x = ln_one(v[i].x, m, s, wv[i].x, bv[i].x);
+        o.y = ln_one(v[i].y, m, s, wv[i].y, bv[i].y);
+        o.z = ln_one(v[i].z, m, s, wv[i].z, bv[i].z);
+        o.w = ln_one(v[i].w, m, s, wv[i].w, bv[i].w);
         dst[threadIdx.x + i * 256] = o;
     }
 }

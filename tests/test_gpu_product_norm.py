@@ -1,0 +1,43 @@
+"""A product with a bias and a skip connection whose result goes into a LayerNormalization: the runtime has the product's call make both tensors,
+in one launch where a tile of the product holds whole rows.  The bits of the net run operator by operator."""
+import numpy as np
+import pytest
+
+from onenew_amd import hip, onefile, rt
+
+pytestmark = pytest.mark.gpu
+
+# (rows, k, n): rows that end inside a tile of 64, alone in one, and full; the widest row a tile holds and narrower ones, off 32 and off 16 columns;
+# rows the tile does not hold (196, 256), of three columns more than a multiple of four, and few rows, where the normalisation is a launch of its own
+CASES = [(12544, 192, 192), (12544, 768, 192), (12481, 192, 192), (9999, 201, 180), (12544, 64, 164), (20001, 96, 132), (9999, 96, 100),
+         (12544, 64, 196), (9999, 192, 256), (9999, 64, 163), (50, 192, 192), (65, 64, 64)]
+
+
+@pytest.mark.parametrize("rows,k,n", CASES)
+def test_product_norm(rows, k, n, monkeypatch):
+    hip.init(0)
+    print("product + LayerNormalization", rows, k, n, flush=True)
+    m, rng = onefile.OneModel(), np.random.default_rng(rows + k + n)
+    w = lambda *s: (rng.normal(size=s) / s[0] ** 0.5).astype(np.float32)   # noqa: E731
+    m.input("x", (1, rows, k))
+    m.matmul("skip", "x", w(k, n), "skip_out")
+    m.matmul("p", "x", w(k, n), "p_mm")
+    m.add("p_bias", "p_mm", w(n), "p_out")
+    m.add("res", "p_out", "skip_out", "y")
+    m.layernorm("ln", "y", 1 + w(n), w(n), "z")
+    m.matmul("after", "z", w(n, 32), "u")
+    for name, cols in (("y", n), ("z", n), ("u", 32)):
+        m.output(name, (1, rows, cols))
+    data = m.tobytes()
+    fused = rt.Net(data)
+    monkeypatch.setenv("ONENEW_RT_FUSE", "0")
+    plain = rt.Net(data)
+    for special in (False, True):
+        x = rng.normal(size=(1, rows, k)).astype(np.float32)
+        if special:
+            x[0, rows - 1, 3], x[0, rows // 2, 5] = np.inf, np.nan
+        for a, b in zip(fused.run(x), plain.run(x)):
+            assert np.array_equal(a, b, equal_nan=True)
+            assert special or np.isfinite(a).all()
+    fused.close()
+    plain.close()
