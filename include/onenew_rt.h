@@ -147,7 +147,8 @@ int onrt_net_fused_attentions(const onrt_net_t *net, int32_t *n);
 int onrt_net_fused_linears(const onrt_net_t *net, int32_t *n);
 /* Of those layers, the ones (without Gelu) whose result goes, with no other reader, into an Add with an activation of the
  * same shape (the skip connection around a transformer block's projection): that Add joins the call (`eval_bias_add`,
- * the addend in inputs[3]), which then runs where the second Add stood.  n: how many. */
+ * the addend in inputs[3]), which then runs where the second Add stood.  A LayerNormalization that reads the sum joins it as well
+ * (`eval_bias_add_norm`); it keeps its buffer and its place, where nothing is left to do.  n: how many. */
 int onrt_net_fused_skips(const onrt_net_t *net, int32_t *n);
 
 /*

@@ -38,8 +38,8 @@ LEGEND = ("Kernel names: `onhip::igemm_kernel<dtype, loader, BM, BN, WM, WN, PF,
           "RES the variant whose store adds a residual operand; PW2 the variant that multiplies its finished tile by a second, 1x1 weight "
           "matrix before storing: a convolution and the 1x1 convolution after it in one launch), `onhip::igemm_dma_kernel<dtype, BM, BN, WM, WN, KS, NST>` (int8 and "
           "16-bit storage: operand tiles loaded straight into LDS, KS bytes of K per stage, ring of NST stages), `onhip::rowb_f32_kernel<WM, WN>` (fp32, B "
-          "straight from memory, tile 32 WM x 128 WN), `onhip::igemm_f3_kernel<loader, BM, BN, WM, WN, RES>` (fp32 on the 16-bit matrix cores; loader 5 "
-          "the rows of a product) and `onhip::split_weights_kernel` in front of it where the weights are split on the call, `onhip::splitk_finish_kernel`, `onhip::depthwise_tiled_kernel<int8, stride, "
+          "straight from memory, tile 32 WM x 128 WN), `onhip::igemm_f3_kernel<loader, BM, BN, WM, WN, RES, PW2, NORM>` (fp32 on the 16-bit matrix cores; loader 5 "
+          "the rows of a product; NORM the variant that normalises the rows of its result as well) and `onhip::split_weights_kernel` in front of it where the weights are split on the call, `onhip::splitk_finish_kernel`, `onhip::depthwise_tiled_kernel<int8, stride, "
           "act>`, `onhip::quantize_nhwc_kernel<CBW>`, `onhip::stem_f32_kernel<filter size, act, two row tiles>` (first-layer "
           "convolutions from an LDS patch), `onhip::i8patch_kernel<bytes per pixel, WM, pixel tiles>` and `onhip::i8direct_kernel<bytes per pixel, taps, WM, TM, pixel "
           "tiles, workgroups per CU>` (int8 chain form, 3x3 with few channels: input rows in LDS / windows loaded per tap), `onhip::attention_f32_kernel<16-key tiles, head dim>`, `onhip::dw_s8_nhwc_kernel<3x3 stride, epilogue, fp32 out>` (depthwise on int8 NHWC), `onhip::irblock_f32_kernel<act, input channels / 4, row tiles, "
