@@ -1271,8 +1271,8 @@ int group_products(onrt_net &net) {
             net.nodes[group[i]].in_group = i > 0;
         }
         first.group = group;
-        first.group_w = first.fused_out + "/weights side by side";   // no operand's name: those have at most OPERAND_NAME_LEN - 1 letters and come from the file
-        first.group_b = first.fused_out + "/biases side by side";
+        first.group_w = first.fused_out + std::string("\0weights", 8);   // no operand's name: the file's end at the first zero byte
+        first.group_b = first.fused_out + std::string("\0biases", 7);
         first.eval = net.matmul_bias_group;
         net.tensors[first.group_w] = w_all;
         net.tensors[first.group_b] = b_all;

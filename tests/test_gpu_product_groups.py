@@ -63,3 +63,28 @@ def test_one_launch():
         ran.append(tuple(hip.last_launch_choice()))
         net.close()
     assert ran[0][4] == ran[1][4] == 2 and ran[0][:2] != ran[1][:2], ran
+
+
+def test_an_operand_with_the_name_of_the_weights_side_by_side(monkeypatch):
+    """the copy that a group's weights and biases have is no operand: one of the model's that is called like it stays what it is"""
+    hip.init(0)
+    m, rng = onefile.OneModel(), np.random.default_rng(8)
+    w = lambda *s: (rng.normal(size=s) / s[0] ** 0.5).astype(np.float32)   # noqa: E731
+    rows, k, n = 2099, 192, 192
+    m.input("x", (1, rows, k))
+    for i in range(2):
+        m.matmul(f"p{i}", "x", w(k, n), f"p{i}_mm")
+        m.add(f"p{i}_bias", f"p{i}_mm", w(n), f"y{i}")
+        m.output(f"y{i}", (1, rows, n))
+    m.matmul("q", "x", m.init("y0/weights side by side", w(k, 2 * n)), "q_mm")
+    m.add("q_bias", "q_mm", m.init("y0/biases side by side", w(2 * n)), "z")
+    m.output("z", (1, rows, 2 * n))
+    data, x = m.tobytes(), rng.normal(size=(1, rows, k)).astype(np.float32)
+    fused = rt.Net(data)
+    monkeypatch.setenv("ONENEW_RT_FUSE", "0")
+    plain = rt.Net(data)
+    for a, b in zip(fused.run(x), plain.run(x)):
+        assert np.array_equal(a, b)
+    assert np.array_equal(fused.fetch("y0/weights side by side"), plain.fetch("y0/weights side by side"))
+    fused.close()
+    plain.close()
