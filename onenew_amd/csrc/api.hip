@@ -1444,7 +1444,9 @@ static int conv2d_pw_impl(const onhip_conv_desc_t *a, const onhip_conv_desc_t *b
     // on the 16-bit matrix cores where both weights are kept split (first stage of a ResNet-50 at batch 32, 3x3 64 -> 64 and 1x1 64 -> 256
     // on 56 x 56 with the Add: 95 us instead of 130)
     static const bool off = getenv("ONHIP_NO_F3") != nullptr;   // tuning hook: fp32 matrix instructions only
-    if (!off && keep_a && keep_b && !getenv("ONHIP_TILE")) {   // a tile asked for is the plain kernel's
+    // (split weights are 6 bytes an element, reductions in sixteens: more than the 32-bit offsets reach before the fp32 ones are)
+    const bool reach = split_weights_bytes(p.M, p.K) < (1LL << 31) && split_weights_bytes(p.m2, p.M) < (1LL << 30);
+    if (!off && reach && keep_a && keep_b && !getenv("ONHIP_TILE")) {   // a tile asked for is the plain kernel's
         const void *sa = nullptr, *sb = nullptr;
         rc = keep_a->get(keep_a->key, wa_packed, {p.M, p.K, p.K, 1}, &sa);
         if (!rc && sa) rc = keep_b->get(keep_b->key, wb, {b->cout, b->cin, b->cin, 1}, &sb);

@@ -82,3 +82,22 @@ def test_operands_without_finite_parts(what, torch_dev):
     # both sum at most 72 and 40 products in fp32: 112 roundings of the sum of magnitudes
     scale = plain[ok].abs().max().double()
     assert float((y[ok].double() - plain[ok].double()).abs().max()) <= 112 * 2.0 ** -24 * float(scale) * 8
+
+
+def test_split_weights_out_of_reach(torch_dev):
+    """more rows of the second product than the split form's 32-bit offsets reach, fewer than the fp32 one's: the fp32 kernel runs"""
+    torch = torch_dev
+    rows, mid = 2_800_001, 64
+    print(f"conv + 1x1, {rows} rows of the second product", flush=True)
+    a, b = descs(1, 4, mid, 1, 2, rows, 3, 1, 1, R, N)
+    x, wa, ba, _, _ = operands("convpw_split_rows", a, descs(1, 4, mid, 1, 2, 1, 3, 1, 1, R, N)[1])
+    g = torch.Generator(device="cuda").manual_seed(3)
+    wb, bb = torch.randn((rows, mid, 1, 1), generator=g, device="cuda"), torch.randn(rows, generator=g, device="cuda")
+    y = plugin_pair(a, b, wa, ba, wb.cpu().numpy(), bb.cpu().numpy())(x)
+    t = lambda v: torch.from_numpy(v).double()   # noqa: E731
+    conv = lambda f: torch.nn.functional.conv2d(f(t(x)), f(t(wa)), f(t(ba)), padding=1).view(mid, 2).cuda()   # noqa: E731
+    product = lambda f, m: f(wb.view(rows, mid).double()) @ m + f(bb.double())[:, None]   # noqa: E731
+    ref, magnitude = product(lambda v: v, torch.relu(conv(lambda v: v))), product(torch.abs, conv(torch.abs))
+    got = torch.from_numpy(y).cuda().view(rows, 2).double()
+    # 36 and 64 products and a bias each: at most 102 roundings to fp32 of what the magnitudes add up to
+    assert bool(((got - ref).abs() <= 102 * 2.0 ** -24 * magnitude).all())
