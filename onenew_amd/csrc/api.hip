@@ -1446,7 +1446,11 @@ static int conv2d_pw_impl(const onhip_conv_desc_t *a, const onhip_conv_desc_t *b
     static const bool off = getenv("ONHIP_NO_F3") != nullptr;   // tuning hook: fp32 matrix instructions only
     // (split weights are 6 bytes an element, reductions in sixteens: more than the 32-bit offsets reach before the fp32 ones are)
     const bool reach = split_weights_bytes(p.M, p.K) < (1LL << 31) && split_weights_bytes(p.m2, p.M) < (1LL << 30);
-    if (!off && reach && keep_a && keep_b && !getenv("ONHIP_TILE")) {   // a tile asked for is the plain kernel's
+    // A first reduction below 48 (3x3 over 4 channels) in one round of workgroups has nothing for them to save: 7.2-7.8 us on fp32 matrix
+    // instructions, 7.5-8.2 here.  In more rounds it does (a batch of 32 on 56 x 56 23.2 -> 19.2), and longer ones do at once, narrow middle
+    // results included (16 -> 8 -> 16 channels at batch 32 0.71 of the time, 64 -> 8 -> 64 0.64).
+    const bool pays = p.K >= 48 || p.N > 256 * 64;
+    if (!off && reach && pays && keep_a && keep_b && !getenv("ONHIP_TILE")) {   // a tile asked for is the plain kernel's
         const void *sa = nullptr, *sb = nullptr;
         rc = keep_a->get(keep_a->key, wa_packed, {p.M, p.K, p.K, 1}, &sa);
         if (!rc && sa) rc = keep_b->get(keep_b->key, wb, {b->cout, b->cin, b->cin, 1}, &sb);

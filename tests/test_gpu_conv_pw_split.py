@@ -101,3 +101,15 @@ def test_split_weights_out_of_reach(torch_dev):
     got = torch.from_numpy(y).cuda().view(rows, 2).double()
     # 36 and 64 products and a bias each: at most 102 roundings to fp32 of what the magnitudes add up to
     assert bool(((got - ref).abs() <= 102 * 2.0 ** -24 * magnitude).all())
+
+
+@pytest.mark.parametrize("n,cin,cmid,hw,split", [(1, 4, 24, 40, False), (1, 4, 24, 128, False), (2, 4, 24, 93, True), (1, 8, 8, 40, True)])
+def test_choice(n, cin, cmid, hw, split, torch_dev):
+    """a short first reduction in one round of workgroups stays with fp32 matrix instructions: the bits of the fp32 kernel"""
+    torch = torch_dev
+    a, b = descs(n, cin, cmid, hw, hw, 16, 3, 1, 1, R, N)
+    x, wa, ba, wb, bb = operands("convpw_split_choice", a, b)
+    y = torch.from_numpy(plugin_pair(a, b, wa, ba, wb, bb)(x).copy())
+    plain = hip.conv2d_pw_f32(a, b, dev(torch, x), hip.pack_conv_weights(a, dev(torch, wa)), dev(torch, ba), hip.conv2d_pw_pack_weights(b, dev(torch, wb)),
+                              dev(torch, bb)).cpu()
+    assert torch.equal(y, plain) != split
