@@ -668,22 +668,32 @@ static bool f3_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out
     return true;
 }
 // Best shape of the kernel whose wavefronts share K, and its microseconds.  From the layers of ResNet-50 at batch 1 (80 layers, 4
-// shapes and both forms of the weights, weights beyond the L2; error 10 %): a compute unit does its workgroups' steps one after the
+// shapes and both forms of the weights, weights beyond the L2; error 10 %) and 950 launches of random layers, small planes and batches of
+// one-pixel images among them: a compute unit does its workgroups' steps one after the
 // other, whoever's they are, and a workgroup costs its start.  A stride along the columns takes twice the cache lines.  Two wavefronts per
 // SIMD pay from 32 steps a tile on where a workgroup has its unit to itself (128 x 784 x 1152 12.0 -> 9.7 us).  Only for operands that
 // fit the L2s: with more the other kernels, which load a tile once, are ahead anyway.
+// Columns of different images are apart by a whole image, and a load of 64 lanes touches a cache line for each: with one-pixel images the
+// lines set the pace (29 of them, 848 -> 299 channels, 16.6 us, 7.7 on the other kernels; 96 of them, 1280 -> 1000, 26.6 and 12.4), and rows
+// that straddle lines cost on other small planes (12 images of 3 x 3, 592 -> 267, 9.3 and 8.1).
+// Fewer steps of 16 than wavefronts leave some of them idle, and the launch costs what it costs: 16 -> 618 channels on 15 x 15 at batch 2 in
+// tiles of 64 x 32 5.0 us, 4.2 on the other kernels; in more than one round of 32 x 32 8 -> 47 on 24 x 24 at batch 8 4.4 and 4.0, 64 -> 182 on
+// 39 x 39 5.4 and 4.9.
 static bool kw_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out, double *us) {
     static const double step[2][3] = {{0.122, 0.105, 0.21}, {0.087, 0.086, 0.13}};   // fp32 / split weights; tiles of 16, 32, 64 rows
-    static const double base[2][3] = {{2.8, 3.6, 4.0}, {3.4, 3.6, 3.9}}, start[3] = {0.0016, 0.003, 0.003};
+    static const double base[2][3] = {{2.8, 3.6, 4.4}, {3.4, 3.6, 4.4}}, start[3] = {0.0016, 0.003, 0.003};
     *us = 1e300;
     if (cfg.dtype != DT_F32 || p.b_slice_bytes > (8LL << 20)) return false;
     const int split = kw_split(cfg, p);
     for (int t = 0; t < 3; ++t) {
         const int bm = 16 << t, bn = t ? 32 : 16, ks = t ? 16 : 32;
         const long long tiles = (long long) ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
-        if (tiles > 2048 || (bm > p.M + 15) || !kw_ok(cfg, p, bm, split != 0)) continue;
         const int steps = (p.K + ks - 1) / ks;
-        const double t_us = base[split][t] + ((tiles + 255) / 256) * steps * step[split][t] * (p.sw > 1 ? 1.4 : 1.0) + tiles * start[t];
+        if (tiles > 2048 || (bm > p.M + 15) || (t == 2 && steps < 6) || (t == 1 && tiles > 256 && steps < 5) || !kw_ok(cfg, p, bm, split != 0)) continue;
+        const double lines = 64.0 / bn * std::min(bn, p.N) / p.OHW;   // of a load of B, where images are smaller than the tile
+        const double apart = p.OHW == 1 ? (t == 0 ? 0.0032 * std::max(0.0, lines - 12.0) : (t == 1 ? 0.0028 : 0.002) * lines) : p.OHW < 16 && p.HW % 4 && cfg.bl == BL_PLAIN ? 0.05 : 0.0;
+        const double a_step = step[split][t] * (p.sw > 1 && p.OW > 1 ? 1.4 : 1.0) + apart;
+        const double t_us = base[split][t] + ((tiles + 255) / 256) * steps * a_step + tiles * start[t];
         if (t_us < *us) { *us = t_us; *out = Choice{bm, bn, t == 1 && tiles <= 256 && steps >= 32 ? 8 : 4, 0, 3, 0, 0}; }
     }
     return *us < 1e299;
@@ -744,7 +754,14 @@ static Choice model_choice(const IgemmLaunch &cfg, const IgemmProblem &p) {
     if (cfg.dtype == DT_I8 && !p.out_s8 && room <= 1 && best.split == 1) cheapest(1, true);
     double kw_us = 1e300;
     Choice kw;
-    if (cfg.dtype == DT_F32 && !tl_hint_bm && kw_choice(cfg, p, &kw, &kw_us) && kw_us > 0.95 * f32_us(cfg, p, best)) kw_us = 1e300;
+    // (the loads of one-pixel images cost the other kernels lines as well, 0.15 us a K tile of 64 columns, which f32_us does not know; on small
+    // odd planes it is 15 % over)
+    auto others = [&]() {
+        const double slices = std::max(1, best.split), rounds = std::ceil(((p.M + best.bm - 1) / best.bm) * ((p.N + best.bn - 1) / best.bn) * slices / 256.0);
+        const double apart = p.OHW == 1 ? 0.15 * std::min(1.0, p.N / 64.0) * std::ceil((p.K + 15) / 16 / slices) * rounds : 0.0;
+        return (p.OHW < 16 && p.OHW > 1 && p.HW % 4 && cfg.bl == BL_PLAIN ? 0.85 : 0.95) * (f32_us(cfg, p, best) + apart);
+    };
+    if (cfg.dtype == DT_F32 && !tl_hint_bm && kw_choice(cfg, p, &kw, &kw_us) && kw_us > others()) kw_us = 1e300;
     // fp32 with a weight matrix for A: the 16-bit matrix cores where that is expected to be faster.  Not for up to 32 rows
     // (the smallest of those tiles has 64: 0.74-0.98 of these kernels' speed on MobileNetV2's projections) nor for reductions
     // below 48 (bound by memory: 0.69 on its 16 -> 96 expansion, where the kernel that reads B straight from memory runs).
