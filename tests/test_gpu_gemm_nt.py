@@ -48,3 +48,18 @@ def test_gemm_operands_off_sixteen_bytes(m, torch_dev):
     y = hip.gemm_f32(a, w, b).double()
     bound = 65 * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T + b.double().abs())
     assert bool(((y - (a.double() @ w.double().T + b.double())).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("m,k,n,tiled", [(16, 25088, 512, True), (64, 4096, 512, True), (16, 8192, 2048, True), (17, 1028, 5000, True), (16, 4096, 4096, False),
+                                         (48, 2048, 1000, False), (9, 2048, 1000, False), (64, 192, 1000, False)])
+def test_gemm_hand_over(m, k, n, tiled, torch_dev):
+    """a K that the tiled kernels are faster on, cut into slices, goes there (they leave a launch choice, the kernels of a batch's rows do not)"""
+    torch = torch_dev
+    x, filt = torch.randn(1, 8, 4, 4, device="cuda"), torch.randn(4, 8, 1, 1, device="cuda")
+    hip.conv2d_f32(hip.ConvDesc(n=1, cin=8, h=4, w=4, cout=4, kh=1, kw=1, stride_h=1, stride_w=1, group=1), x, filt)
+    before = hip.last_launch_choice()
+    a, w, b = torch.randn(m, k, device="cuda"), torch.randn(n, k, device="cuda"), torch.randn(n, device="cuda")
+    y = hip.gemm_f32(a, w, b).double()
+    bound = (k + 1) * 2.0 ** -24 * (a.abs().double() @ w.abs().double().T + b.abs().double())
+    assert bool(((y - (a.double() @ w.double().T + b.double())).abs() <= bound).all())
+    assert (hip.last_launch_choice() != before) == tiled
