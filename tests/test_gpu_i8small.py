@@ -136,3 +136,17 @@ def test_many_tiles_stay_staged():
     d, x, wp, b32, aux, lut = layer(torch, 4, 64, 112, 112, 64, 3, 1, 1, R)
     hip.conv2d_w8a32(d, x, wp, b32, aux, lut, packed=True)
     assert hip.last_launch_choice()[4] != 4
+
+
+@pytest.mark.parametrize("case,ours", [((4, 1198, 5, 5, 248, 7, 3, 3, N), False), ((1, 832, 11, 11, 35, 7, 1, 3, R), False), ((2, 1844, 5, 5, 147, 5, 3, 2, S), False),
+                                       ((1, 512, 7, 7, 96, 3, 1, 1, R), True), ((1, 800, 7, 7, 64, 3, 1, 1, N), True), ((2, 1366, 13, 13, 172, 3, 1, 1, R), True)])
+def test_long_reductions_are_cut_into_slices(case, ours):
+    """from int8 activations: where the other kernels cut K, one launch is the slower form of a long one"""
+    import torch
+    hip.init(0)
+    print("i8small, long K", case, flush=True)
+    d, x, wp, b32, aux, lut = layer(torch, *case)
+    xq = hip.quantize_nhwc_s8(x, d.input_scale)
+    y = hip.conv2d_w8_link(d, wp, b32, aux, lut, xq=xq)
+    assert (hip.last_launch_choice()[4] == 4) == ours, hip.last_launch_choice()
+    assert torch.equal(y, hip.conv2d_w8a32(d, x, wp, b32, aux, lut, packed=True))
