@@ -596,15 +596,19 @@ static bool dma_model_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choi
         if (cost < best_cost) { best_cost = cost; best = t; }
     }
     if (best < 0) return false;
-    // The ring by how many workgroups a compute unit gets.  Up to two wait for their loads (an L2 trip a stage with the short ring,
-    // which leaves room for three): in bf16 128 x 25088 x 1152 19.4 -> 16.0 us, 256 x 6272 x 2304 17.8 -> 16.4, in int8 128 x 25600 x
-    // 1152 13.7 -> 12.8.  A lone one takes all the LDS: 512 x 1568 x 4608 in bf16 27.0 -> 19.8 (21.3 with the ring in between), in int8
-    // 16.0 -> 12.3.  With more workgroups than that the third resident one is worth more (100352 columns: 20.1 against 22.8), and so it is
-    // with stages of 64 bytes.
-    const int bm = order[best][0], bn = order[best][1];
+    // The ring by how many workgroups a compute unit gets and how many stages there are to have in flight.  Up to two workgroups wait for their
+    // loads (an L2 trip a stage with the short ring, which leaves room for three): in bf16 128 x 25088 x 1152 19.4 -> 16.0 us, 256 x 6272 x 2304
+    // 17.8 -> 16.4, in int8 128 x 25600 x 1152 13.7 -> 12.8.  A lone one of many stages takes as long a ring as there is (five stages of 64 x 64, half
+    // of the LDS): 512 x 1568 x 4608 in bf16 27.0 -> 19.8 (21.3 with the ring in between), in int8 16.0 -> 12.3.  With more workgroups than that the
+    // third resident one is worth more (100352 columns: 20.1 against 22.8), and so it is with stages of 64 bytes.
+    // Few stages gain nothing from a ring that holds more of them, and a workgroup with more LDS starts later: 64 x 64 tiles of one stage
+    // 3.73 / 3.88 / 4.00 us with the short ring, the one in between and the long one (3.30 / 3.45 / 3.58 on weights from beyond the L2), of nine
+    // 5.67 / 5.84 / 6.03 (5.42 / 5.56 / 5.70); of 16 6.53 / 6.72 / 6.72 (6.61 / 6.39 / 6.47), of 36 10.7 / 11.0 / 10.9 (11.2 / 10.8 / 10.6).  The wider
+    // tiles' short ring has one stage in flight: of one 4.35 / 4.46 (3.93 / 4.06), of four 5.21 / 5.26 (5.52 / 4.99).
+    const int bm = order[best][0], bn = order[best][1], stages = p.k_units / 8;
     const long long tiles = (long long) ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
     int dma = 1;
-    if (tiles <= 512 && dma_ring_ok(cfg, p, bm, bn, 2)) dma = tiles <= 256 && best == 3 ? 2 : 3;
+    if (tiles <= 512 && stages >= (best == 3 ? 12 : 3) && dma_ring_ok(cfg, p, bm, bn, 2)) dma = tiles <= 256 && best == 3 && stages >= 32 ? 2 : 3;
     *out = Choice{bm, bn, 1, 0, 0, 0, dma};
     return true;
 }

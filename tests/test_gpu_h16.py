@@ -302,3 +302,26 @@ def test_h16_argument_errors(torch_dev):
     with pytest.raises(hip.OnhipError, match="64 taps"):
         hip.conv2d_h16(big, torch.zeros((1, 12, 12, 32), dtype=torch.bfloat16, device="cuda"),
                        torch.zeros((32, 81, 32), dtype=torch.bfloat16, device="cuda"), b)
+
+
+# 1x1 and 3x3 layers of few stages of 64 channels, of the middle and of many; in 64 x 64 tiles, then in wider ones
+RING_CHOICES = [(1, 64, 16, 64, 1, 1), (1, 512, 28, 128, 1, 1), (1, 64, 28, 256, 3, 1), (1, 1024, 28, 128, 1, 3), (1, 512, 20, 128, 3, 2),
+                (8, 64, 56, 128, 1, 1), (8, 256, 56, 128, 1, 3), (64, 64, 56, 128, 1, 1)]
+
+
+@pytest.mark.parametrize("n,cin,hw,cout,k,ring", RING_CHOICES)
+def test_ring_by_the_count_of_stages(n, cin, hw, cout, k, ring, torch_dev, monkeypatch):
+    """the ring of stage buffers that the cost model takes, and the same bits as with the short one"""
+    torch = torch_dev
+    print("ring", n, cin, hw, cout, k, flush=True)
+    monkeypatch.delenv("ONHIP_TILE", raising=False)
+    d = with_compute(cases.cd(cin, cout, k, 1, k // 2, hw, n=n, act=abi.RELU), abi.COMPUTE_BF16)
+    g = torch.Generator(device="cuda").manual_seed(cin + cout)
+    x = hip.h16_from_nchw(torch.randn((n, cin, hw, hw), generator=g, device="cuda"), d.compute)
+    w = hip.h16_pack_conv_weights(d, torch.randn((cout, cin, k, k), generator=g, device="cuda") / (cin * k * k) ** 0.5)
+    b = torch.randn(cout, generator=g, device="cuda")
+    y = hip.conv2d_h16(d, x, w, b)
+    ran = hip.last_launch_choice()
+    assert ran[6] == ring, ran
+    monkeypatch.setenv("ONHIP_TILE", f"{ran[0]}x{ran[1]}x1x0x0x0x1")
+    assert torch.equal(hip.conv2d_h16(d, x, w, b), y) and hip.last_launch_choice()[6] == 1
