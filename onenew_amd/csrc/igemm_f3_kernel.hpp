@@ -627,6 +627,7 @@ void igemm_f3_kernel(const std::conditional_t<NORM, IgemmNormProblem, IgemmProbl
 #pragma unroll
     for (int i = 0; i < (BM + NT - 1) / NT; ++i)
         if (tid + i * NT < BM) s_bias[tid + i * NT] = bias_row[i];
+    if (!PW2 && !NORM && table_in_lds(p)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's part of the table
     __syncthreads();
 
     const int m_wave = m0 + wm * (BM / WM), n_wave = n0 + wn * (BN / WN);

@@ -307,7 +307,8 @@ __host__ __device__ inline bool table_in_lds(const IgemmParams &p) {
     return (p.ep.act == SILU || p.ep.act == ONHIP_ACT_GELU_LUT) && !int8_rows && !p.out_h16 && !slices_only;
 }
 inline unsigned table_lds_bytes(const IgemmParams &p) { return table_in_lds(p) ? TABLE_BYTES : 0u; }
-// every wavefront of the workgroup (nt threads) takes its share; complete once its loads are (vmcnt) and a barrier has passed
+// every wavefront of the workgroup (nt threads) takes its share; complete once each has waited for its loads (vmcnt, in so many words: no
+// register tells the compiler) and a barrier has passed
 __device__ __forceinline__ void request_table(const float *lut, float *table, int wave, int lane, int nt) {
 #if defined(__HIP_DEVICE_COMPILE__)
     const rsrc_t rt = make_rsrc(lut, TABLE_BYTES);
@@ -1467,6 +1468,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(PW2 ? 4
             s_bias[tid] = bias_row;
         }
     }
+    if (!PW2 && table_in_lds(p)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's part of the table
     if constexpr (!PW2) __syncthreads();
 
     if constexpr (PW2) {
