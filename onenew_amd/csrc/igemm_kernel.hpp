@@ -306,6 +306,12 @@ __host__ __device__ inline bool table_in_lds(const IgemmParams &p) {
     const bool slices_only = p.partial && !p.arrive && p.dp_tiles == 0;
     return (p.ep.act == SILU || p.ep.act == ONHIP_ACT_GELU_LUT) && !int8_rows && !p.out_h16 && !slices_only;
 }
+// igemm_kernel's tiles of 4096 results (16 KiB, half the table) have it there only where a launch's workgroups are all resident with it, three a
+// compute unit (two in 32 x 128): five or six are without, and where there is a second round that is worth more (fp32 33 -> 668 channels on 58 x 58 at batch 8, 4431
+// workgroups, 58 -> 44 us, 16 -> 52 under 3x3 at 113 x 113 and batch 16, 3193, 54 -> 50; 14 -> 21 on 36 x 36 at batch 16, 162, 5.7 and 6.8).  In int8
+// 64 x 64 it is not (88 -> 292 on 50 x 50 at batch 16, 3125, 22.9 with it and 25.1).
+__host__ __device__ constexpr bool table_unless_many(int dt, int bm, int bn) { return bm * bn <= 4096 && (dt != DT_I8 || bm == 32); }
+__host__ __device__ inline bool table_few(int bm, unsigned workgroups) { return workgroups <= (bm == 32 ? 512u : 768u); }
 inline unsigned table_lds_bytes(const IgemmParams &p) { return table_in_lds(p) ? TABLE_BYTES : 0u; }
 // every wavefront of the workgroup (nt threads) takes its share; complete once each has waited for its loads (vmcnt, in so many words: no
 // register tells the compiler) and a barrier has passed
@@ -1199,7 +1205,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(PW2 ? 4
     const int wm = wave / WN, wn = wave % WN;
 
     extern __shared__ __attribute__((aligned(1024))) float s_table[];   // TABLE_BYTES where table_in_lds says so
-    if (!PW2 && table_in_lds(p)) request_table(p.ep.lut, s_table, wave, lane, THREADS);
+    const bool table = !PW2 && table_in_lds(p) && (!table_unless_many(DT, BM, BN) || table_few(BM, gridDim.x * gridDim.y * gridDim.z));   // uniform
+    if (table) request_table(p.ep.lut, s_table, wave, lane, THREADS);
 
     const TilePlace tp = place_tile<BM, BN>(p);
     const int m0 = tp.m0, n0 = tp.n0, slice = tp.slice, lid = tp.lid;
@@ -1468,7 +1475,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(PW2 ? 4
             s_bias[tid] = bias_row;
         }
     }
-    if (!PW2 && table_in_lds(p)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's part of the table
+    if (table) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's part of the table
     if constexpr (!PW2) __syncthreads();
 
     if constexpr (PW2) {
@@ -1525,7 +1532,10 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(PW2 ? 4
         case RELU: write_tile<DT, EPI_RELU, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM), twin_at, BM + 16); break;
         case CLIP: write_tile<DT, EPI_CLIP, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM), twin_at, BM + 16); break;
         case SILU:
-        case ONHIP_ACT_GELU_LUT: write_tile<DT, EPI_LUT, TM, TN, RES, BIAS_LDS, true>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM), twin_at, BM + 16, (lds_f32_t) s_table); break;
+        case ONHIP_ACT_GELU_LUT:
+            if (!table_unless_many(DT, BM, BN) || table) write_tile<DT, EPI_LUT, TM, TN, RES, BIAS_LDS, true>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM), twin_at, BM + 16, (lds_f32_t) s_table);
+            else write_tile<DT, EPI_LUT, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM), twin_at, BM + 16);
+            break;
         default: write_tile<DT, EPI_GENERIC, TM, TN, RES, BIAS_LDS>(p, acc, batch, m_wave, n_wave, li, lh, s_bias + wm * (BM / WM), s_bias + BM + wm * (BM / WM), twin_at, BM + 16); break;
     }
     if constexpr (DT == DT_I8 && RES)
@@ -1646,7 +1656,7 @@ static int launch_one(const IgemmLaunch &cfg, const IgemmParams &p_in, hipStream
     const int rc = tile_grid<BM, BN>(cfg, p, &grid);
     if (rc) return rc;
     if (RES != (p.res != nullptr)) return set_error(ONHIP_ERR_ARG, "igemm: residual operand and kernel variant do not match");
-    hipLaunchKernelGGL((igemm_kernel<DT, BL, BM, BN, WM, WN, PF, RES>), grid, dim3(THREADS), table_lds_bytes(p), stream, p);
+    hipLaunchKernelGGL((igemm_kernel<DT, BL, BM, BN, WM, WN, PF, RES>), grid, dim3(THREADS), !table_unless_many(DT, BM, BN) || table_few(BM, grid.x * grid.y * grid.z) ? table_lds_bytes(p) : 0u, stream, p);
     ONHIP_CHECK_HIP(hipGetLastError());
     return finish_launch<DT == DT_I8>(cfg, p, stream);
 }
