@@ -560,6 +560,9 @@ typedef struct {
     int64_t out_step;
 } onhip_product_group_t;
 int onhip_matmul_bias_group_eval(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_INFO_S *outputs);
+/* `eval_bias_group_takes` of libMatMul_hip.so: same slots, of which params[1], params[2], params[4] and the structure's parts and out_step are
+ * read; 1 when one launch is expected to be faster (whatever measured choices and tile hints say at the time), else 0. */
+int onhip_matmul_bias_group_takes(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_INFO_S *outputs);
 /*
  * No counterpart in the reference, whose operators always finish before eval returns (device/cuda/MaxPool/
  * maxpool.cu:76).  on != 0: an eval whose output is device memory returns as soon as its kernels are queued on

@@ -150,6 +150,10 @@ int onrt_net_fused_linears(const onrt_net_t *net, int32_t *n);
  * the addend in inputs[3]), which then runs where the second Add stood.  A LayerNormalization that reads the sum joins it as well
  * (`eval_bias_add_norm`); it keeps its buffer and its place, where nothing is left to do.  n: how many. */
 int onrt_net_fused_skips(const onrt_net_t *net, int32_t *n);
+/* Layers of that kind (a bias, no Gelu, no skip) of one shape on one input, the q, k and v projections of an attention block: one call of the
+ * MatMul plugin's `eval_bias_group` where its `eval_bias_group_takes` expects one product to be faster at the net's row count; such a group's
+ * weights lie side by side in a copy of their own.  n: how many groups. */
+int onrt_net_product_groups(const onrt_net_t *net, int32_t *n);
 
 /*
  * One inference as a HIP graph, on request: with ONENEW_RT_GRAPH=1 in the environment at load time.  The operators

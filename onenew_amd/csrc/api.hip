@@ -1915,29 +1915,38 @@ static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float
 
 // Why: three products of 192 columns over 12544 rows are 12 us each, half of it first loads and stores; as one of 576 columns a tile of 128
 // columns is a workgroup's.  Only where a product on its own runs on the 16-bit matrix cores as well: the arithmetic is the same, so are the bits.
+// plan: the one product, how it runs, and whether that is expected to be faster.  Weights and tensors are not read.
+static int matmul_group_plan(const onhip_matmul_desc_t *d, int parts, const float *a, const float *w_all, const float *bias_all, float *out, long long out_step,
+                             void *stream, IgemmLaunch *cfg, IgemmProblem *p, Choice *c, bool *pays) {
+    *pays = false;
+    if (d->compute != ONHIP_COMPUTE_F32 || d->n % 32 || out_step % 16) return ONHIP_OK;
+    double each, us;
+    const int rc = matmul_impl(d, a, w_all, bias_all, nullptr, nullptr, out, stream, nullptr, &each);   // a plan as well
+    if (rc || each == 0.0) return rc;
+    onhip_matmul_desc_t all = *d;
+    all.n = parts * d->n;
+    const long long rows = (long long) d->batch * d->m, extent = (parts - 1) * out_step + rows * d->n * 4;
+    if ((long long) d->k * all.n >= (1LL << 31) || rows * all.n >= (1LL << 31) || out_step < rows * d->n * 4 || extent >= (1LL << 31)) return ONHIP_OK;
+    matmul_rows_problem(&all, a, w_all, bias_all, nullptr, nullptr, out, cfg, p);
+    p->c_stride_n = d->n;
+    p->c_slice_bytes = extent;
+    p->c_part = d->n;
+    p->c_part_step = (unsigned) out_step;
+    *pays = f3_choice(*cfg, *p, c, &us) && us < parts * each;
+    return ONHIP_OK;
+}
 static int matmul_group_impl(const onhip_matmul_desc_t *d, int parts, const float *a, const float *w_all, const float *bias_all, float *out,
                              long long out_step, const SplitKeeper *keeper, void *stream, bool *ran) {
     *ran = false;
     if (!d || !a || !w_all || !bias_all || !out) return set_error(ONHIP_ERR_ARG, "matmul group: null pointer");
     if (parts < 2 || parts > ONHIP_GROUP_MAX) return set_error(ONHIP_ERR_ARG, "matmul group: %d products", parts);
-    if (d->compute != ONHIP_COMPUTE_F32 || d->n % 32 || out_step % 16 || tune_mode() || tl_noalloc || tl_hint_bm || getenv("ONHIP_TILE")) return ONHIP_OK;
-    double each;
-    const int rc = matmul_impl(d, a, w_all, bias_all, nullptr, nullptr, out, stream, nullptr, &each);   // a plan: the weights are not read
-    if (rc || each == 0.0) return rc;
-    onhip_matmul_desc_t all = *d;
-    all.n = parts * d->n;
+    if (tune_mode() || tl_noalloc || tl_hint_bm || getenv("ONHIP_TILE")) return ONHIP_OK;
     IgemmLaunch cfg;
     IgemmProblem p;
-    const long long rows = (long long) d->batch * d->m, extent = (parts - 1) * out_step + rows * d->n * 4;
-    if ((long long) d->k * all.n >= (1LL << 31) || rows * all.n >= (1LL << 31) || out_step < rows * d->n * 4 || extent >= (1LL << 31)) return ONHIP_OK;
-    matmul_rows_problem(&all, a, w_all, bias_all, nullptr, nullptr, out, &cfg, &p);
-    p.c_stride_n = d->n;
-    p.c_slice_bytes = extent;
-    p.c_part = d->n;
-    p.c_part_step = (unsigned) out_step;
     Choice c;
-    double us;
-    if (!f3_choice(cfg, p, &c, &us) || us >= parts * each) return ONHIP_OK;
+    bool pays;
+    const int rc = matmul_group_plan(d, parts, a, w_all, bias_all, out, out_step, stream, &cfg, &p, &c, &pays);
+    if (rc || !pays) return rc;
     p.keeper = keeper;
     const int launched = launch_choice(cfg, p, c, reinterpret_cast<hipStream_t>(stream));
     if (launched == kNoSplitSlot) return ONHIP_OK;
@@ -2326,6 +2335,18 @@ int conv2d_pw_f32_kept(const onhip_conv_desc_t *a, const onhip_conv_desc_t *b, c
 int matmul_f32_kept(const onhip_matmul_desc_t *d, const float *a, const float *b, const float *bias, const float *gelu_lut, const float *addend,
                     float *out, const SplitKeeper *keeper, void *stream, RowNorm *norm) {
     return matmul_impl(d, a, b, bias, gelu_lut, addend, out, stream, keeper, nullptr, norm);
+}
+bool matmul_group_takes(const onhip_matmul_desc_t *d, int parts, long long out_step) {
+    float *some = reinterpret_cast<float *>(4096);   // an aligned address that is not read
+    const int bm = tl_hint_bm;
+    tl_hint_bm = 0;
+    IgemmLaunch cfg;
+    IgemmProblem p;
+    Choice c;
+    bool pays;
+    const int rc = matmul_group_plan(d, parts, some, some, some, some, out_step, nullptr, &cfg, &p, &c, &pays);
+    tl_hint_bm = bm;
+    return !rc && pays;
 }
 int matmul_group_f32_kept(const onhip_matmul_desc_t *d, int parts, const float *a, const float *w_all, const float *bias_all, float *out, long long out_step,
                           const SplitKeeper *keeper, void *stream, bool *ran) {

@@ -325,6 +325,7 @@ int matmul_f32_kept(const onhip_matmul_desc_t *d, const float *a, const float *b
                     float *out, const SplitKeeper *keeper, void *stream, struct RowNorm *norm = nullptr);
 // `parts` products of the shape d on one left operand, weights [k][parts * n] and biases side by side, results out_step bytes apart: as one
 // launch if that is expected to be faster than each on its own, which then has the same bits (*ran says whether)
+bool matmul_group_takes(const onhip_matmul_desc_t *d, int parts, long long out_step);   // it is expected to be (no tensor is read)
 int matmul_group_f32_kept(const onhip_matmul_desc_t *d, int parts, const float *a, const float *w_all, const float *bias_all, float *out, long long out_step,
                           const SplitKeeper *keeper, void *stream, bool *ran);
 // st is being captured; true as well for the legacy stream while another thread's capture keeps it from being asked

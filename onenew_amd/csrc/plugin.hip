@@ -814,29 +814,34 @@ static int matmul_bias_add_norm_eval_locked(BUFFER_INFO_S *params, BUFFER_INFO_S
     return matmul_eval_mode(4, params, inputs, outputs);
 }
 
-static int matmul_bias_group_eval_locked(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_INFO_S *outputs) {
+// the products of a group as the library describes one of them; false where a slot is empty or the shapes do not fit
+static bool group_desc(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, onhip_matmul_desc_t *d, const onhip_product_group_t **group) {
     const OPERAND_S *a_t = reinterpret_cast<const OPERAND_S *>(params[1].addr), *b_t = reinterpret_cast<const OPERAND_S *>(params[2].addr);
     const OPERAND_S *o_t = reinterpret_cast<const OPERAND_S *>(params[4].addr);
-    const onhip_product_group_t *g = reinterpret_cast<const onhip_product_group_t *>(inputs[4].addr);
+    const onhip_product_group_t *g = *group = reinterpret_cast<const onhip_product_group_t *>(inputs[4].addr);
+    if (!a_t || !b_t || !o_t || !g) return false;
+    const int nd = a_t->dim_num_of_shapes;
+    if (nd < 2 || nd > SHAPE_LEN || o_t->dim_num_of_shapes < 1 || o_t->dim_num_of_shapes > SHAPE_LEN || g->parts < 2 || g->parts > ONHIP_GROUP_MAX) return false;
+    memset(d, 0, sizeof(*d));
+    d->batch = 1;
+    for (int i = 0; i < nd - 2; ++i) d->batch *= a_t->shapes[i];
+    d->m = a_t->shapes[nd - 2];
+    d->k = a_t->shapes[nd - 1];
+    d->n = o_t->shapes[o_t->dim_num_of_shapes - 1];
+    d->b_shared = 1;
+    return numel(b_t) == (long long) d->k * d->n;
+}
+
+static int matmul_bias_group_eval_locked(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_INFO_S *outputs) {
+    const onhip_product_group_t *g;
+    onhip_matmul_desc_t d;
     const float *a = reinterpret_cast<const float *>(inputs[0].addr);
     char *y = reinterpret_cast<char *>(outputs[0].addr);
-    if (!a_t || !b_t || !o_t || !g || !a || !y) return set_error(ONHIP_ERR_ARG, "MatMul group eval: empty slot");
-    const int nd = a_t->dim_num_of_shapes;
-    if (nd < 2 || nd > SHAPE_LEN || o_t->dim_num_of_shapes < 1 || o_t->dim_num_of_shapes > SHAPE_LEN) return set_error(ONHIP_ERR_ARG, "MatMul group eval: rank %d", nd);
-    if (g->parts < 2 || g->parts > ONHIP_GROUP_MAX) return set_error(ONHIP_ERR_ARG, "MatMul group eval: %d products", g->parts);
+    if (!group_desc(params, inputs, &d, &g) || !a || !y) return set_error(ONHIP_ERR_ARG, "MatMul group eval: an empty slot, or shapes that do not fit together");
     if (!is_device_ptr(a) || !is_device_ptr(y)) return set_error(ONHIP_ERR_ARG, "MatMul group eval: tensors in device memory only");
     for (int i = 0; i < g->parts; ++i)
         if (!g->w[i] || !g->bias[i] || !is_held(g->w[i])) return set_error(ONHIP_ERR_ARG, "MatMul group eval: weights that are not held");
     if (!g->w_all || !g->bias_all || !is_held(g->w_all)) return set_error(ONHIP_ERR_ARG, "MatMul group eval: weights that are not held");
-    onhip_matmul_desc_t d;
-    memset(&d, 0, sizeof(d));
-    d.batch = 1;
-    for (int i = 0; i < nd - 2; ++i) d.batch *= a_t->shapes[i];
-    d.m = a_t->shapes[nd - 2];
-    d.k = a_t->shapes[nd - 1];
-    d.n = o_t->shapes[o_t->dim_num_of_shapes - 1];
-    d.b_shared = 1;
-    if (numel(b_t) != (long long) d.k * d.n) return set_error(ONHIP_ERR_ARG, "MatMul group eval: weights of %lld elements for %d x %d", numel(b_t), d.k, d.n);
     bool ran = false;
     const SplitKeeper all = {g->w_all, split_of};
     int rc = matmul_group_f32_kept(&d, g->parts, a, g->w_all, g->bias_all, reinterpret_cast<float *>(y), g->out_step, &all, g_stream, &ran);
@@ -1277,6 +1282,13 @@ int onhip_matmul_bias_add_eval(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUF
 }
 int onhip_matmul_bias_group_eval(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_INFO_S *outputs) {
     return guarded("MatMul (+ bias), a group", matmul_bias_group_eval_locked, params, inputs, outputs);
+}
+int onhip_matmul_bias_group_takes(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_INFO_S *outputs) {
+    (void) outputs;
+    const onhip_product_group_t *g;
+    onhip_matmul_desc_t d;
+    if (!params || !inputs || !group_desc(params, inputs, &d, &g)) return 0;
+    return matmul_group_takes(&d, g->parts, g->out_step) ? 1 : 0;
 }
 int onhip_matmul_attention_eval(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs, BUFFER_INFO_S *outputs) {
     return guarded("MatMul (attention)", matmul_attention_eval_locked, params, inputs, outputs);

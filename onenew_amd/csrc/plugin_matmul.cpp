@@ -48,3 +48,8 @@ extern "C" __attribute__((visibility("default"))) int eval_bias_group(BUFFER_INF
                                                                       BUFFER_INFO_S *outputs) {
     return onhip_matmul_bias_group_eval(params, inputs, outputs);
 }
+// Same slots, no tensor touched: 1 when the library expects one launch to be faster.
+extern "C" __attribute__((visibility("default"))) int eval_bias_group_takes(BUFFER_INFO_S *params, BUFFER_INFO_S *inputs,
+                                                                            BUFFER_INFO_S *outputs) {
+    return onhip_matmul_bias_group_takes(params, inputs, outputs);
+}

@@ -121,7 +121,7 @@ struct Tensor {
     std::string alias;       // an operand folded away with its producer reads as this one (fuse_residual_blocks)
     bool never_written = false;   // an operand inside a fused attention block: it has no buffer and no value
     bool as_s8 = false;           // written and read as int8 NHWC, channels padded to 16 (link_int8_convs)
-    std::vector<char> made;       // an initialiser that is not in the file: its data until uploaded (group_products)
+    std::vector<std::string> parts;   // an initialiser that is not in the file: these, whose rows lie side by side in it (group_products)
     bool has_twin = false;        // fp32, and stored once more as int8 NHWC for the int8 convolutions among its readers
     void *twin_dev = nullptr;
 };
@@ -185,8 +185,8 @@ struct onrt_net {
     onenew_eval_fn conv_block = nullptr, conv_block_takes = nullptr, conv_link = nullptr, conv_link_takes = nullptr;
     onenew_eval_fn conv_pair = nullptr, conv_pair_relu = nullptr, conv_pair_takes = nullptr;
     onenew_eval_fn maxpool_s8 = nullptr;   // optional entry point of the MaxPool plugin
-    onenew_eval_fn matmul_attention = nullptr, matmul_bias = nullptr, matmul_bias_gelu = nullptr, matmul_bias_add = nullptr, matmul_bias_group = nullptr, matmul_bias_add_norm = nullptr;   // optional entry points of the MatMul plugin
-    int fused_blocks = 0, folded_relus = 0, folded_acts = 0, fused_attentions = 0, fused_linears = 0, fused_skips = 0, fused_ir_blocks = 0, fused_pairs = 0, int8_links = 0;
+    onenew_eval_fn matmul_attention = nullptr, matmul_bias = nullptr, matmul_bias_gelu = nullptr, matmul_bias_add = nullptr, matmul_bias_group = nullptr, matmul_bias_group_takes = nullptr, matmul_bias_add_norm = nullptr;   // optional entry points of the MatMul plugin
+    int fused_blocks = 0, folded_relus = 0, folded_acts = 0, fused_attentions = 0, fused_linears = 0, fused_skips = 0, fused_ir_blocks = 0, fused_pairs = 0, product_groups = 0, int8_links = 0;
     void *init_arena = nullptr, *act_arena = nullptr, *tables = nullptr;
     std::vector<float> silu_lut, gelu_lut;
 };
@@ -436,12 +436,22 @@ int allocate(onrt_net &net) {
             Tensor &t = kv.second;
             if (!t.is_init) continue;
             t.dev = static_cast<char *>(net.init_arena) + off;
-            const char *data = t.made.empty() ? net.file.data() + (size_t) t.desc.p_data : t.made.data();
-            if (t.bytes) ONRT_HIP(hipMemcpy(t.dev, data, t.bytes, hipMemcpyHostToDevice));
+            if (t.bytes && t.parts.empty()) ONRT_HIP(hipMemcpy(t.dev, net.file.data() + (size_t) t.desc.p_data, t.bytes, hipMemcpyHostToDevice));
             t.desc.p_data = 0;
-            t.made = std::vector<char>();
             off += (t.bytes + 255) & ~(size_t) 255;
         }
+        bool copied = false;
+        for (auto &kv : net.tensors) {
+            const Tensor &t = kv.second;
+            const size_t n = t.parts.size();
+            if (!n) continue;
+            const size_t row = (size_t) t.desc.shapes[t.desc.dim_num_of_shapes - 1] * 4, share = row / n;
+            for (size_t i = 0; i < n; ++i)
+                ONRT_HIP(hipMemcpy2DAsync(static_cast<char *>(t.dev) + i * share, row, net.tensors[t.parts[i]].dev, share, share, t.bytes / row,
+                                          hipMemcpyDeviceToDevice, nullptr));
+            copied = true;
+        }
+        if (copied) ONRT_HIP(hipStreamSynchronize(nullptr));
         // they stay as they are until the net is freed (and the plugins told to forget them)
         for (forget_fn f : net.holders)
             if (f(net.init_arena, init_total)) return fail(ONRT_ERR_PLUGIN, "onhip_plugin_hold failed");
@@ -577,6 +587,7 @@ int bind_plugins(onrt_net &net) {
             net.matmul_bias_gelu = reinterpret_cast<onenew_eval_fn>(dlsym(it->second, "eval_bias_gelu"));
             net.matmul_bias_add = reinterpret_cast<onenew_eval_fn>(dlsym(it->second, "eval_bias_add"));
             net.matmul_bias_group = reinterpret_cast<onenew_eval_fn>(dlsym(it->second, "eval_bias_group"));
+            net.matmul_bias_group_takes = reinterpret_cast<onenew_eval_fn>(dlsym(it->second, "eval_bias_group_takes"));
             net.matmul_bias_add_norm = reinterpret_cast<onenew_eval_fn>(dlsym(it->second, "eval_bias_add_norm"));
         }
     }
@@ -1227,11 +1238,15 @@ int fuse_linear(onrt_net &net) {
     return ONRT_OK;
 }
 
+// bytes from a product's result to that of the next one in its group (allocate places them one behind the other)
+int64_t result_step(const Tensor &t) { return ((int64_t) numel(t.desc) * 4 + 255) & ~(int64_t) 255; }
+
 // Linear layers of one shape on one input (the q, k and v projections of an attention block): the first of them in the order makes all their
 // results, in one call of the MatMul plugin's `eval_bias_group`; the others stay in the order and have nothing to do.  Their weights lie side
-// by side in a copy of their own, for the call to run as one product; the operands are the same as without.
+// by side in a copy of their own, for the call to run as one product; the operands are the same as without.  Only where the plugin's
+// `eval_bias_group_takes` expects one product to be faster at the net's own row count: elsewhere the copy would be made for nothing.
 int group_products(onrt_net &net) {
-    if (!fusing_enabled() || !net.matmul_bias_group) return ONRT_OK;
+    if (!fusing_enabled() || !net.matmul_bias_group || !net.matmul_bias_group_takes) return ONRT_OK;
     for (size_t at = 0; at < net.order.size(); ++at) {
         Node &first = net.nodes[net.order[at]];
         if (strcmp(first.kind->type, "MatMul") || first.fuse != 4 || first.in_group || first.in.size() != 3) continue;
@@ -1253,6 +1268,17 @@ int group_products(onrt_net &net) {
         }
         if (group.size() < 2) continue;
         const size_t parts = group.size();
+        onhip_product_group_t asked = {};
+        asked.parts = (int32_t) parts;
+        asked.out_step = result_step(y);
+        first.params[1].addr = (int64_t) &x.desc;
+        first.params[2].addr = (int64_t) &w.desc;
+        first.params[4].addr = (int64_t) &y.desc;
+        first.inputs[4].addr = (int64_t) &asked;
+        const bool takes = net.matmul_bias_group_takes(first.params, first.inputs, first.outputs) == 1;
+        for (BUFFER_INFO_S &slot : first.params) slot.addr = 0;
+        first.inputs[4].addr = 0;
+        if (!takes) continue;
         Tensor w_all, b_all;
         w_all.desc = w.desc;
         w_all.desc.shapes[1] = (int32_t) parts * n;
@@ -1261,13 +1287,9 @@ int group_products(onrt_net &net) {
         b_all.desc.shapes[b.desc.dim_num_of_shapes - 1] = (int32_t) parts * n;
         b_all.bytes = parts * b.bytes;
         w_all.is_init = b_all.is_init = w_all.produced = b_all.produced = true;
-        w_all.made.resize(w_all.bytes);
-        b_all.made.resize(b_all.bytes);
-        const size_t row = (size_t) n * 4;
         for (size_t i = 0; i < parts; ++i) {
-            const char *from = net.file.data() + net.tensors[net.nodes[group[i]].in[1]].desc.p_data;
-            for (int r = 0; r < k; ++r) memcpy(w_all.made.data() + (r * parts + i) * row, from + r * row, row);
-            memcpy(b_all.made.data() + i * row, net.file.data() + net.tensors[net.nodes[group[i]].in[2]].desc.p_data, row);
+            w_all.parts.push_back(net.nodes[group[i]].in[1]);
+            b_all.parts.push_back(net.nodes[group[i]].in[2]);
             net.nodes[group[i]].in_group = i > 0;
         }
         first.group = group;
@@ -1276,6 +1298,7 @@ int group_products(onrt_net &net) {
         first.eval = net.matmul_bias_group;
         net.tensors[first.group_w] = w_all;
         net.tensors[first.group_b] = b_all;
+        ++net.product_groups;
     }
     return ONRT_OK;
 }
@@ -1335,7 +1358,7 @@ int fill_slots(onrt_net &net) {
             }
             g.w_all = static_cast<const float *>(net.tensors[nd.group_w].dev);
             g.bias_all = static_cast<const float *>(net.tensors[nd.group_b].dev);
-            g.out_step = (int64_t) ((net.tensors[nd.fused_out].bytes + 255) & ~(size_t) 255);
+            g.out_step = result_step(net.tensors[nd.fused_out]);
             nd.inputs[4].addr = (int64_t) &g;
         }
         if (nd.fuse == 7) {
@@ -1665,6 +1688,12 @@ ONRT_API int onrt_net_fused_ir_blocks(const onrt_net_t *net, int32_t *n) {
 ONRT_API int onrt_net_fused_pairs(const onrt_net_t *net, int32_t *n) {
     if (!net || !n) return fail(ONRT_ERR_ARG, "fused convolution pairs: null argument");
     *n = (int32_t) net->fused_pairs;
+    return ONRT_OK;
+}
+
+ONRT_API int onrt_net_product_groups(const onrt_net_t *net, int32_t *n) {
+    if (!net || !n) return fail(ONRT_ERR_ARG, "groups of products: null argument");
+    *n = (int32_t) net->product_groups;
     return ONRT_OK;
 }
 

@@ -44,7 +44,7 @@ EXPORTS = ["onhip_init", "onhip_last_error", "onhip_set_tuning", "onhip_split_ta
            "onhip_conv2d_pw_supported", "onhip_conv2d_pw_packed_weight_bytes", "onhip_conv2d_pw_pack_weights", "onhip_conv2d_pw_f32",
            "onhip_add_f32", "onhip_relu_f32", "onhip_maxpool_out_shape", "onhip_maxpool_f32", "onhip_maxpool_s8_nhwc", "onhip_maxpool_s8_eval", "onhip_global_avgpool_f32",
            "onhip_gelu_lut_f32", "onhip_layernorm_f32", "onhip_softmax_f32", "onhip_transpose_f32",
-           "onhip_conv_eval", "onhip_matmul_eval", "onhip_matmul_attention_eval", "onhip_matmul_bias_eval", "onhip_matmul_bias_gelu_eval", "onhip_matmul_bias_add_eval", "onhip_matmul_bias_add_norm_eval", "onhip_matmul_bias_group_eval", "onhip_gemm_eval", "onhip_add_eval", "onhip_relu_eval",
+           "onhip_conv_eval", "onhip_matmul_eval", "onhip_matmul_attention_eval", "onhip_matmul_bias_eval", "onhip_matmul_bias_gelu_eval", "onhip_matmul_bias_add_eval", "onhip_matmul_bias_add_norm_eval", "onhip_matmul_bias_group_eval", "onhip_matmul_bias_group_takes", "onhip_gemm_eval", "onhip_add_eval", "onhip_relu_eval",
            "onhip_maxpool_eval", "onhip_global_avgpool_eval", "onhip_gelu_eval", "onhip_layernorm_eval",
            "onhip_softmax_eval", "onhip_transpose_eval", "onhip_plugin_set_async", "onhip_plugin_set_stream", "onhip_plugin_forget", "onhip_plugin_hold", "onhip_plugin_trust_weights", "onhip_plugin_release"]
 
@@ -137,7 +137,7 @@ def load():
     L.onhip_conv2d_pw_pack_weights.argtypes = [C.POINTER(ConvDesc), vp, vp, vp]
     L.onhip_conv2d_pw_f32.argtypes = [C.POINTER(ConvDesc)] * 2 + [vp] * 6 + [i32, vp, vp]
     L.onhip_linear_h16.argtypes = [C.c_longlong, i32, i32, i32, vp, vp, vp, vp, vp, vp, i32, vp]
-    for name in ("onhip_conv_eval", "onhip_matmul_eval", "onhip_matmul_attention_eval", "onhip_matmul_bias_eval", "onhip_matmul_bias_gelu_eval", "onhip_matmul_bias_add_eval", "onhip_matmul_bias_group_eval", "onhip_gemm_eval"):
+    for name in ("onhip_conv_eval", "onhip_matmul_eval", "onhip_matmul_attention_eval", "onhip_matmul_bias_eval", "onhip_matmul_bias_gelu_eval", "onhip_matmul_bias_add_eval", "onhip_matmul_bias_add_norm_eval", "onhip_matmul_bias_group_eval", "onhip_matmul_bias_group_takes", "onhip_gemm_eval"):
         getattr(L, name).argtypes = [C.POINTER(BUFFER_INFO_S)] * 3
     _lib = L
     return L

@@ -8,7 +8,7 @@ from . import hip
 
 EXPORTS = ["onrt_last_error", "onrt_net_load_file", "onrt_net_load_buf", "onrt_net_free", "onrt_net_io_count",
            "onrt_net_io_info", "onrt_net_op_count", "onrt_net_op_info", "onrt_net_operand", "onrt_net_run", "onrt_net_enqueue", "onrt_net_fused_count", "onrt_net_graph_launches", "onrt_net_plan_buf",
-           "onrt_net_folded_activations", "onrt_net_fused_attentions", "onrt_net_fused_linears", "onrt_net_fused_skips", "onrt_net_fused_ir_blocks", "onrt_net_fused_pairs", "onrt_net_quantised_links", "onrt_net_tune_tiles", "onrt_net_get_tiles", "onrt_net_set_tiles", "onrt_one_set_tiles", "onrt_one_quantise"]
+           "onrt_net_folded_activations", "onrt_net_fused_attentions", "onrt_net_fused_linears", "onrt_net_fused_skips", "onrt_net_product_groups", "onrt_net_fused_ir_blocks", "onrt_net_fused_pairs", "onrt_net_quantised_links", "onrt_net_tune_tiles", "onrt_net_get_tiles", "onrt_net_set_tiles", "onrt_one_set_tiles", "onrt_one_quantise"]
 
 _lib = None
 
@@ -48,6 +48,7 @@ def load():
     L.onrt_net_fused_skips.argtypes = [vp, i32p]
     L.onrt_net_fused_ir_blocks.argtypes = [vp, i32p]
     L.onrt_net_fused_pairs.argtypes = [vp, i32p]
+    L.onrt_net_product_groups.argtypes = [vp, i32p]
     L.onrt_net_quantised_links.argtypes = [vp, i32p]
     L.onrt_net_operand.argtypes = [vp, C.c_char_p, i32p, i32p, C.POINTER(vp)]
     L.onrt_net_run.argtypes = [vp, C.POINTER(vp), C.POINTER(vp)]
@@ -178,6 +179,12 @@ class Net:
         """number of those groups that also take in the Add of a skip connection after them"""
         n = C.c_int32()
         _check(load().onrt_net_fused_skips(self._h, C.byref(n)), "onrt_net_fused_skips")
+        return n.value
+
+    def product_groups(self):
+        """number of groups of such layers on one input that run as one call (their weights lie side by side in a copy)"""
+        n = C.c_int32()
+        _check(load().onrt_net_product_groups(self._h, C.byref(n)), "onrt_net_product_groups")
         return n.value
 
     def fused_ir_blocks(self):

@@ -8,13 +8,14 @@ from onenew_amd import hip, onefile, rt
 pytestmark = pytest.mark.gpu
 
 
-# (rows, k, n, products): one launch with tiles that cover two products and end inside the last one, K off sixteen, rows off every tile, more
-# products than a group takes; few rows, where each runs on its own
-CASES = [(2099, 192, 192, 3), (5000, 64, 96, 2), (1500, 201, 224, 4), (3000, 192, 160, 5), (50, 96, 64, 3), (12544, 192, 192, 3)]
+# (rows, k, n, products, groups): rows and products for which each runs on its own and no copy of the weights is made; then one launch, with tiles that
+# cover two products and end inside the last one, K off sixteen, rows off every tile, more products than a group takes
+CASES = [(2099, 192, 192, 3, 0), (5000, 64, 96, 2, 0), (1500, 201, 224, 4, 0), (3000, 192, 160, 5, 0), (50, 96, 64, 3, 0),
+         (12544, 192, 192, 3, 1), (12546, 192, 192, 2, 1), (9002, 201, 224, 4, 1), (12622, 192, 160, 5, 1), (3154, 384, 384, 3, 1)]
 
 
-@pytest.mark.parametrize("rows,k,n,products", CASES)
-def test_group(rows, k, n, products, monkeypatch):
+@pytest.mark.parametrize("rows,k,n,products,groups", CASES)
+def test_group(rows, k, n, products, groups, monkeypatch):
     hip.init(0)
     print("product group", rows, k, n, products, flush=True)
     m, rng = onefile.OneModel(), np.random.default_rng(rows + n)
@@ -33,6 +34,7 @@ def test_group(rows, k, n, products, monkeypatch):
     monkeypatch.setenv("ONENEW_RT_FUSE", "0")
     plain = rt.Net(data)
     assert fused.fused_linears() == products + 1
+    assert fused.product_groups() == groups and plain.product_groups() == 0
     for scale in (1.0, -0.3):
         x = (rng.normal(size=(2, rows // 2, k)) * scale).astype(np.float32)
         if scale < 0:
@@ -70,7 +72,7 @@ def test_an_operand_with_the_name_of_the_weights_side_by_side(monkeypatch):
     hip.init(0)
     m, rng = onefile.OneModel(), np.random.default_rng(8)
     w = lambda *s: (rng.normal(size=s) / s[0] ** 0.5).astype(np.float32)   # noqa: E731
-    rows, k, n = 2099, 192, 192
+    rows, k, n = 12544, 192, 192
     m.input("x", (1, rows, k))
     for i in range(2):
         m.matmul(f"p{i}", "x", w(k, n), f"p{i}_mm")
@@ -83,6 +85,7 @@ def test_an_operand_with_the_name_of_the_weights_side_by_side(monkeypatch):
     fused = rt.Net(data)
     monkeypatch.setenv("ONENEW_RT_FUSE", "0")
     plain = rt.Net(data)
+    assert fused.product_groups() == 1
     for a, b in zip(fused.run(x), plain.run(x)):
         assert np.array_equal(a, b)
     assert np.array_equal(fused.fetch("y0/weights side by side"), plain.fetch("y0/weights side by side"))
