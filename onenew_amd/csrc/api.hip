@@ -807,6 +807,7 @@ static Choice model_choice(const IgemmLaunch &cfg, const IgemmProblem &p) {
 
 static std::atomic<long long> g_tail_launches{0};
 static std::atomic<long long> g_dma_launches{0};
+static std::atomic<long long> g_norm_launches{0};   // products that normalised their rows themselves
 
 // what the calling thread's last implicit-GEMM launch ran as (onhip_last_launch_choice): tile, K slices as launched,
 // slices of the leftover tiles, and which kernel
@@ -1186,6 +1187,8 @@ long long onhip_scratch_bytes(void) {
 }
 
 long long onhip_direct_lds_launches(void) { return g_dma_launches.load(std::memory_order_relaxed); }
+
+long long onhip_product_norm_launches(void) { return g_norm_launches.load(std::memory_order_relaxed); }
 
 long long onhip_split_tail_launches(void) { return g_tail_launches.load(std::memory_order_relaxed); }
 
@@ -1906,7 +1909,9 @@ static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float
             if (rows_us) { *rows_us = form.faster ? us : 0.0; return ONHIP_OK; }
             form.p.keeper = keeper;
             form.p.norm = tune_mode() ? nullptr : norm;   // measuring launches the product many times
-            return plan_and_launch(cfg, p, st, &form);
+            const int rc = plan_and_launch(cfg, p, st, &form);
+            if (!rc && norm && norm->done) g_norm_launches.fetch_add(1, std::memory_order_relaxed);
+            return rc;
         }
     }
     if (rows_us) { *rows_us = 0.0; return ONHIP_OK; }

@@ -7,14 +7,16 @@ from onenew_amd import hip, onefile, rt
 
 pytestmark = pytest.mark.gpu
 
-# (rows, k, n): rows that end inside a tile of 64, alone in one, and full; the widest row a tile holds and narrower ones, off 32 and off 16 columns;
-# rows the tile does not hold (196, 256), of three columns more than a multiple of four, and few rows, where the normalisation is a launch of its own
-CASES = [(12544, 192, 192), (12544, 768, 192), (12481, 192, 192), (9999, 201, 180), (12544, 64, 164), (20001, 96, 132), (9999, 96, 100),
-         (12544, 64, 196), (9999, 192, 256), (9999, 64, 163), (50, 192, 192), (65, 64, 64)]
+# (rows, k, n, in one launch): rows that end inside a tile of 64, alone in one, and full; the widest row a tile holds and narrower ones, off 32 and off 16
+# columns; then products that run in another tile, rows that no tile holds (196, 256), of three columns more than a multiple of four, and few rows, where
+# the normalisation is a launch of its own
+CASES = [(12544, 192, 192, 1), (12544, 768, 192, 1), (12481, 192, 192, 1), (12481, 201, 180, 1), (12544, 192, 164, 1), (16001, 201, 132, 1), (14001, 200, 148, 1),
+         (9999, 201, 180, 0), (12544, 64, 164, 0), (20001, 96, 132, 0), (9999, 96, 100, 0), (12544, 64, 196, 0), (9999, 192, 256, 0), (9999, 64, 163, 0),
+         (12544, 192, 163, 0), (50, 192, 192, 0), (65, 64, 64, 0)]
 
 
-@pytest.mark.parametrize("rows,k,n", CASES)
-def test_product_norm(rows, k, n, monkeypatch):
+@pytest.mark.parametrize("rows,k,n,one_launch", CASES)
+def test_product_norm(rows, k, n, one_launch, monkeypatch):
     hip.init(0)
     print("product + LayerNormalization", rows, k, n, flush=True)
     m, rng = onefile.OneModel(), np.random.default_rng(rows + k + n)
@@ -36,7 +38,10 @@ def test_product_norm(rows, k, n, monkeypatch):
         x = rng.normal(size=(1, rows, k)).astype(np.float32)
         if special:
             x[0, rows - 1, 3], x[0, rows // 2, 5] = np.inf, np.nan
-        for a, b in zip(fused.run(x), plain.run(x)):
+        before = hip.load().onhip_product_norm_launches()
+        got = fused.run(x)
+        assert hip.load().onhip_product_norm_launches() - before == one_launch
+        for a, b in zip(got, plain.run(x)):
             assert np.array_equal(a, b, equal_nan=True)
             assert special or np.isfinite(a).all()
     fused.close()
