@@ -968,11 +968,14 @@ struct RowsForm {
 
 // Chooses tile, split and tail handling for the problem and launches it.
 static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t st, const RowsForm *other = nullptr) {
-    auto launch = [&](const Choice &c) {
+    auto launch = [&](const Choice &c, bool measuring = false) {
         if (!other || c.rowb != 2) return launch_choice(cfg, p, c, st);
-        const int rc = launch_choice(other->cfg, other->p, c, st);
+        IgemmProblem rows = other->p;
+        if (measuring) rows.norm = nullptr;   // the product alone, like its other kernels, which do not normalise
+        const int rc = launch_choice(other->cfg, rows, c, st);
         return rc == kNoSplitSlot ? launch_choice(cfg, p, slotless_choice(cfg, p, st), st) : rc;
     };
+    auto timed = [&](const Choice &c) { return launch(c, true); };
     auto ok = [&](const Choice &c) { return other && c.rowb == 2 ? candidate_ok(other->cfg, other->p, c) : candidate_ok(cfg, p, c); };
     auto by_model = [&]() { return !other ? model_choice(cfg, p) : other->faster ? other->rows : other->plain; };
     // the entry point that allocates nothing: the cost model's choice (never the in-launch reduction, whose uncached
@@ -1036,7 +1039,7 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
     // The model's own choice is measured first (it need not be among the candidates below), and another one takes its
     // place only by beating it by 2 %: the measurements repeat within about 3 %, and without the margin a launch that is
     // no faster replaces the model's on a coin toss (seen as a tuned stack slower than the untuned one).
-    rc = time_choice(launch, guess, st, e0, e1, &guess_ms);
+    rc = time_choice(timed, guess, st, e0, e1, &guess_ms);
     best_ms = guess_ms;
     auto same = [](const Choice &a, const Choice &b) {
         return a.bm == b.bm && a.bn == b.bn && a.split == b.split && a.tail == b.tail && a.rowb == b.rowb && a.fin == b.fin && a.dma == b.dma;
@@ -1044,7 +1047,7 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
     auto try_choice = [&](const Choice &c) {
         if (same(c, guess)) return;
         float ms = 0.f;
-        rc = time_choice(launch, c, st, e0, e1, &ms);
+        rc = time_choice(timed, c, st, e0, e1, &ms);
         if (!rc && ms < best_ms && ms < 0.98f * guess_ms) { best_ms = ms; best = c; }
     };
     for (int t = 0; t < kNumTiles && !rc; ++t) {
@@ -1908,7 +1911,7 @@ static int matmul_impl(const onhip_matmul_desc_t *d, const float *a, const float
         if (rows_form(cfg, p, &form, &us)) {
             if (rows_us) { *rows_us = form.faster ? us : 0.0; return ONHIP_OK; }
             form.p.keeper = keeper;
-            form.p.norm = tune_mode() ? nullptr : norm;   // measuring launches the product many times
+            form.p.norm = norm;
             const int rc = plan_and_launch(cfg, p, st, &form);
             if (!rc && norm && norm->done) g_norm_launches.fetch_add(1, std::memory_order_relaxed);
             return rc;

@@ -46,3 +46,34 @@ def test_product_norm(rows, k, n, one_launch, monkeypatch):
             assert special or np.isfinite(a).all()
     fused.close()
     plain.close()
+
+
+def test_measured_choices(monkeypatch):
+    """the product alone is measured; what is chosen then normalises its rows where its tile holds them: the bits of the separate launches"""
+    hip.init(0)
+    rows, k, n = 12544, 192, 192
+    m, rng = onefile.OneModel(), np.random.default_rng(5)
+    w = lambda *s: (rng.normal(size=s) / s[0] ** 0.5).astype(np.float32)   # noqa: E731
+    m.input("x", (1, rows, k))
+    m.input("s", (1, rows, n))
+    m.matmul("p", "x", w(k, n), "p_mm")
+    m.add("p_bias", "p_mm", w(n), "p_out")
+    m.add("res", "p_out", "s", "y")
+    m.layernorm("ln", "y", 1 + w(n), w(n), "z")
+    m.output("y", (1, rows, n))
+    m.output("z", (1, rows, n))
+    x, skip = rng.normal(size=(1, rows, k)).astype(np.float32), rng.normal(size=(1, rows, n)).astype(np.float32)
+    net = rt.Net(m.tobytes())
+    before = hip.set_tuning(1)
+    try:
+        for _ in range(2):   # measured, and chosen from what was
+            launches = hip.load().onhip_product_norm_launches()
+            y, z = net.run(x, skip)
+            ran = hip.last_launch_choice()
+            assert hip.load().onhip_product_norm_launches() - launches == (1 if ran[4] == 2 and ran[:2] == (192, 64) else 0), ran
+    finally:
+        hip.set_tuning(before)
+    import torch
+    t = lambda name: torch.from_numpy(net.fetch(name)).cuda()   # noqa: E731
+    assert np.array_equal(hip.layernorm_f32(torch.from_numpy(y).cuda(), t("ln.weight"), t("ln.bias")).cpu().numpy(), z)
+    net.close()
