@@ -1948,7 +1948,7 @@ static int matmul_group_impl(const onhip_matmul_desc_t *d, int parts, const floa
     *ran = false;
     if (!d || !a || !w_all || !bias_all || !out) return set_error(ONHIP_ERR_ARG, "matmul group: null pointer");
     if (parts < 2 || parts > ONHIP_GROUP_MAX) return set_error(ONHIP_ERR_ARG, "matmul group: %d products", parts);
-    if (tune_mode() || tl_noalloc || tl_hint_bm || getenv("ONHIP_TILE")) return ONHIP_OK;
+    if (tl_noalloc || tl_hint_bm || getenv("ONHIP_TILE")) return ONHIP_OK;
     IgemmLaunch cfg;
     IgemmProblem p;
     Choice c;

@@ -49,11 +49,12 @@ def test_group(rows, k, n, products, groups, monkeypatch):
     plain.close()
 
 
-def test_one_launch():
-    """three products of 192 columns run as one of 576, in tiles that a product of 192 is not cut into"""
+@pytest.mark.parametrize("measured", [0, 1], ids=["by the model", "measured choices"])
+def test_one_launch(measured):
+    """three products of 192 columns run as one of 576, in tiles that a product of 192 is not cut into; under measured choices as well"""
     hip.init(0)
     ran = []
-    for products in (1, 3):
+    for products, tuning in ((1, 0), (3, measured)):
         m, rng = onefile.OneModel(), np.random.default_rng(3)
         m.input("x", (64, 196, 192))
         for i in range(products):
@@ -61,7 +62,11 @@ def test_one_launch():
             m.add(f"p{i}_bias", f"p{i}_mm", rng.normal(size=192).astype(np.float32), f"y{i}")
             m.output(f"y{i}", (64, 196, 192))
         net = rt.Net(m.tobytes())
-        net.run(rng.normal(size=(64, 196, 192)).astype(np.float32))
+        before = hip.set_tuning(tuning)
+        try:
+            net.run(rng.normal(size=(64, 196, 192)).astype(np.float32))
+        finally:
+            hip.set_tuning(before)
         ran.append(tuple(hip.last_launch_choice()))
         net.close()
     assert ran[0][4] == ran[1][4] == 2 and ran[0][:2] != ran[1][:2], ran
