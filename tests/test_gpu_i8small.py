@@ -14,7 +14,6 @@ N, R, C, S = abi.NOT_ACT, abi.RELU, abi.CLIP, abi.SILU
 LAYERS = [(1, 3, 9, 11, 5, 3, 1, 1, R), (1, 16, 7, 7, 33, 1, 1, 0, N), (2, 40, 13, 9, 64, 3, 2, 1, S), (1, 72, 20, 20, 128, 3, 1, 1, S), (1, 31, 17, 23, 30, 5, 1, 2, C),
           (1, 48, 14, 14, 70, 7, 2, 3, S), (3, 20, 5, 6, 17, 2, 1, 0, R), (1, 33, 12, 10, 40, 3, 3, 4, S), (1, 592, 6, 6, 40, 3, 1, 1, S), (5, 24, 3, 3, 20, 3, 1, 0, S),
           (1, 64, 80, 80, 64, 3, 1, 1, S), (1, 128, 80, 80, 128, 1, 1, 0, S), (4, 128, 40, 40, 128, 3, 1, 1, S), (1, 512, 20, 20, 70, 3, 1, 1, S), (2, 144, 52, 51, 100, 1, 1, 0, S)]
-SHAPES_SEEN = set()
 
 
 def layer(torch, n, cin, h, w, cout, k, stride, pad, act, bias=1):
@@ -52,14 +51,20 @@ def test_layer(case, monkeypatch):
     print("i8small", case, flush=True)
     y, staged, ran = both(torch, monkeypatch, *layer(torch, *case))
     assert ran[4] == 4
-    SHAPES_SEEN.add(tuple(ran[:2]))
     assert torch.equal(y, staged) and bool((y != 0).any())
 
 
-def test_every_workgroup_shape_ran():
-    if len(LAYERS) and not SHAPES_SEEN:
-        pytest.skip("the layers above did not run")
-    assert SHAPES_SEEN >= {(32, 32), (64, 32), (128, 32), (64, 64)}
+def test_the_layers_take_every_workgroup_shape():
+    import torch
+    hip.init(0)
+    seen, before = set(), hip.set_tuning(0)
+    try:
+        for case in LAYERS:
+            hip.conv2d_w8a32(*layer(torch, *case), packed=True)
+            seen.add(tuple(hip.last_launch_choice()[:2]))
+    finally:
+        hip.set_tuning(before)
+    assert seen >= {(32, 32), (64, 32), (128, 32), (64, 64)}
 
 
 # the forms either side: int8 or fp32 in; int8, fp32, or fp32 after an Add (and Relu) with its int8 twin out
@@ -68,46 +73,47 @@ LINKS = [(1, 16, 7, 7, 33, 1, 1, 0, N), (2, 40, 13, 9, 64, 3, 2, 1, R), (1, 72, 
          (1, 512, 20, 20, 80, 3, 1, 1, S), (8, 256, 14, 14, 256, 3, 1, 1, R), (1, 48, 14, 14, 70, 7, 2, 3, S), (5, 24, 3, 3, 20, 3, 1, 0, C), (3, 2048, 7, 7, 272, 1, 1, 0, N)]
 
 
-@pytest.mark.parametrize("form", FORMS)
-@pytest.mark.parametrize("case", LINKS, ids=[str(c) for c in LINKS])
-def test_link(case, form, monkeypatch):
-    import torch
-    hip.init(0)
-    print("i8small", form, case, flush=True)
+def link_fits(case, form):
+    """a twin has channels in sixteens, an Add follows no table activation here"""
+    return "add" not in form or (case[4] % 16 == 0 and case[8] != S)
+
+
+def run_link(torch, case, form):
+    """-> result, its int8 twin (of an Add) or None, the kernel that ran"""
     d, x, wp, b32, aux, lut = layer(torch, *case)
     d.output_scale, d.out_s8 = 0.031, int(form.endswith("to s8"))
     add = "add" in form
-    if add and (d.cout % 16 or d.act_type == S):
-        pytest.skip("a twin has channels in sixteens, an Add follows no table activation here")
     src = dict(x=x) if form.startswith("f32") else dict(xq=hip.quantize_nhwc_s8(x, d.input_scale))
     oh, ow = d.out_hw()
     g = torch.Generator(device="cuda").manual_seed(5)
     addend = torch.randn((d.n, d.cout, oh, ow), generator=g, device="cuda") if add else None
-    results, before = [], hip.set_tuning(0)
+    twin = torch.full((d.n, oh, ow, d.cout), 55, dtype=torch.int8, device="cuda") if add else None
+    out = torch.full((d.n, oh, ow, (d.cout + 15) // 16 * 16), 55, dtype=torch.int8, device="cuda") if d.out_s8 else torch.full((d.n, d.cout, oh, ow), 55.0, device="cuda")
+    before = hip.set_tuning(0)
     try:
-        for other in (False, True):
-            if other:
-                monkeypatch.setenv("ONHIP_NO_PATCH", "1")
-            twin = torch.full((d.n, oh, ow, d.cout), 55, dtype=torch.int8, device="cuda") if add else None
-            out = torch.full((d.n, oh, ow, (d.cout + 15) // 16 * 16), 55, dtype=torch.int8, device="cuda") if d.out_s8 else torch.full((d.n, d.cout, oh, ow), 55.0, device="cuda")
-            hip.conv2d_w8_link(d, wp, b32, aux, lut, addend=addend, relu_after="relu" in form, out=out, twin=twin, **src)
-            results.append((out, twin, hip.last_launch_choice()[4]))
+        hip.conv2d_w8_link(d, wp, b32, aux, lut, addend=addend, relu_after="relu" in form, out=out, twin=twin, **src)
     finally:
-        monkeypatch.delenv("ONHIP_NO_PATCH", raising=False)
         hip.set_tuning(before)
-    LINKS_SEEN.append((form, results[0][2]))
-    assert results[1][2] == 0 and torch.equal(results[0][0], results[1][0]) and bool((results[0][0] != 0).any())
-    assert not add or torch.equal(results[0][1], results[1][1])
+    return out, twin, hip.last_launch_choice()[4]
 
 
-LINKS_SEEN = []
+@pytest.mark.parametrize("case,form", [(c, f) for c in LINKS for f in FORMS if link_fits(c, f)], ids=str)
+def test_link(case, form, monkeypatch):
+    import torch
+    hip.init(0)
+    print("i8small", form, case, flush=True)
+    out, twin, _ = run_link(torch, case, form)
+    monkeypatch.setenv("ONHIP_NO_PATCH", "1")
+    staged, staged_twin, ran = run_link(torch, case, form)
+    assert ran == 0 and torch.equal(out, staged) and bool((out != 0).any())
+    assert twin is None or torch.equal(twin, staged_twin)
 
 
-def test_every_form_ran():
-    if not LINKS_SEEN:
-        pytest.skip("the layers above did not run")
-    for form in FORMS:
-        assert sum(ran == 4 for f, ran in LINKS_SEEN if f == form) >= 2, (form, LINKS_SEEN)
+@pytest.mark.parametrize("form", FORMS)
+def test_two_layers_or_more_take_each_form(form):
+    import torch
+    hip.init(0)
+    assert sum(run_link(torch, case, form)[2] == 4 for case in LINKS if link_fits(case, form)) >= 2
 
 
 def test_no_bias_leaves_the_activation_out(monkeypatch):
