@@ -113,12 +113,15 @@ def run_conv_h16(torch, oracle, d, name, tile, monkeypatch, lut=None):
     return x, w, b, rnd, y_nhwc.cpu().numpy(), y_nchw.cpu().numpy(), out16
 
 
+# ring of stage buffers: 1 = within 64 KiB of LDS, 2 = the long one (up to 144 KiB), 3 = the one in between (64 to 72 KiB), which stages of
+# 128 bytes have (channels a multiple of 64) and the largest tile does not
+TILES = ["128x128", "128x64", "64x128", "64x64"]
+RINGS = [(ring, tile, shape) for shape in CONV_SHAPES for tile in TILES for ring in (1, 2, 3) if ring < 3 or (shape[1] % 64 == 0 and tile != "128x128")]
+
+
 @pytest.mark.parametrize("compute", TYPES)
-@pytest.mark.parametrize("ring", [1, 2])
-@pytest.mark.parametrize("tile", ["128x128", "128x64", "64x128", "64x64"])
-@pytest.mark.parametrize("shape", CONV_SHAPES)
+@pytest.mark.parametrize("ring,tile,shape", RINGS)
 def test_conv_h16_every_tile(compute, ring, tile, shape, torch_dev, oracle, monkeypatch):
-    """ring: 1 = stage buffers within 64 KiB of LDS, 2 = the long ring (up to 144 KiB)"""
     torch = torch_dev
     tile = f"{tile}x1x0x0x0x{ring}"
     n, cin, hw, cout, k, stride, pad = shape
@@ -126,6 +129,7 @@ def test_conv_h16_every_tile(compute, ring, tile, shape, torch_dev, oracle, monk
     name = f"h16_{cin}_{cout}_{k}_{stride}"
     print(f"case {name} tile {tile} compute {compute}", flush=True)
     x, w, b, rnd, y_nhwc, y_nchw, out16 = run_conv_h16(torch, oracle, d, name, tile, monkeypatch)
+    assert hip.last_launch_choice()[6] == ring
     ref = oracle.conv2d_f32(d, rnd(x), rnd(w), b)
     assert np.array_equal(y_nhwc, np.transpose(y_nchw, (0, 2, 3, 1))), "the two fp32 layouts hold different values"
     assert norm_diff(y_nchw, ref) <= 1e-4, f"vs oracle on rounded operands: {norm_diff(y_nchw, ref):.3e}"
@@ -222,7 +226,7 @@ def test_conv_h16_activations(compute, act, torch_dev, oracle, monkeypatch):
 
 @pytest.mark.parametrize("compute", TYPES)
 @pytest.mark.parametrize("relu", [False, True])
-@pytest.mark.parametrize("tile", ["128x128", "64x64"])
+@pytest.mark.parametrize("tile", ["128x128", "64x64", "64x128x1x0x0x0x3", "64x64x1x0x0x0x3"])
 def test_conv_h16_residual_operand(compute, relu, tile, torch_dev, oracle, monkeypatch):
     torch = torch_dev
     monkeypatch.setenv("ONHIP_TILE", tile)

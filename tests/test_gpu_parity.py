@@ -1279,6 +1279,50 @@ def test_conv_int8_direct_to_lds_kernel_every_tile(ring, tile, shape, act, torch
     assert hip.load().onhip_direct_lds_launches() == launches + 2, "the forced tile did not run the direct-to-LDS kernel"
 
 
+# layers whose stages are 128 bytes: one stage and many, ragged rows and columns, one tap and many; the last two with fewer and with more than
+# 256 workgroups in every tile (a lone workgroup has the activation's table in LDS of its own, others behind the K loop, in the ring's)
+RING_SHAPES = [(3, 128, 9, 130, 1, 1, 0), (1, 128, 23, 200, 3, 2, 1), (1, 256, 7, 33, 3, 1, 1), (2, 128, 12, 64, 5, 1, 2), (1, 256, 30, 136, 1, 1, 0),
+               (6, 128, 59, 140, 1, 1, 0)]
+
+
+@pytest.mark.parametrize("tile", ["128x64", "64x128", "64x64"])
+@pytest.mark.parametrize("shape", RING_SHAPES)
+@pytest.mark.parametrize("act", [abi.SILU, abi.RELU])
+def test_conv_int8_direct_to_lds_kernel_ring_in_between(tile, shape, act, torch_dev, oracle, monkeypatch):
+    """the ring of 64 to 72 KiB (two resident workgroups, two or three stages in flight each): fp32 results without and with the raw accumulators
+    and int8 results, all equal to the oracle"""
+    torch = torch_dev
+    n, cin, hw, cout, k, stride, pad = shape
+    print("ring in between", tile, shape, act, flush=True)
+    d = cases.cd(cin, cout, k, stride, pad, hw, n=n, act=act, input_scale=0.037)
+    x, w8, b32, aux = cases.conv_inputs(f"ring3_{cin}_{cout}_{k}_{stride}", d, quant=True)
+    lut = cases.silu_lut()
+    ref, ref_acc = oracle.conv2d_w8a32(d, x, w8, b32, aux, lut, want_acc=True)
+    oh, ow = d.out_hw()
+    operands = (dev(torch, b32), dev(torch, aux), dev(torch, lut))
+    monkeypatch.setenv("ONHIP_TILE", tile + "x1x0x0x0x3")
+
+    def ran():
+        bm, bn = map(int, tile.split("x"))
+        assert tuple(hip.last_launch_choice()) == (bm, bn, 1, 0, 0, 0, 3)
+
+    y = hip.conv2d_w8a32(d, dev(torch, x), dev(torch, w8), *operands)
+    ran()
+    assert np.array_equal(y.cpu().numpy(), ref)
+    acc = torch.empty((d.n, d.cout, oh, ow), dtype=torch.int32, device="cuda")
+    y = hip.conv2d_w8a32(d, dev(torch, x), dev(torch, w8), *operands, acc32=acc)
+    ran()
+    assert np.array_equal(acc.cpu().numpy(), ref_acc) and np.array_equal(y.cpu().numpy(), ref)
+    dq = ConvDesc.from_buffer_copy(d)
+    dq.out_s8, dq.output_scale = 1, 0.045
+    refq = oracle.conv2d_w8a32(dq, x, w8, b32, aux, lut)
+    out = torch.full((d.n, oh, ow, (d.cout + 15) // 16 * 16), 77, dtype=torch.int8, device="cuda")
+    hip.conv2d_w8a8_nhwc(dq, hip.quantize_nhwc_s8(dev(torch, x), d.input_scale), hip.pack_conv_weights_w8(d, dev(torch, w8)), *operands, out=out)
+    ran()
+    got = out.cpu().numpy()
+    assert np.array_equal(got[..., :d.cout], np.transpose(refq, (0, 2, 3, 1))) and not got[..., d.cout:].any()
+
+
 _TUNE_CHILD = r"""
 import sys, numpy as np, torch
 sys.path.insert(0, sys.argv[1]); sys.path.insert(0, sys.argv[1] + "/tests/golden")
