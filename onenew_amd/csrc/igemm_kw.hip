@@ -1,6 +1,6 @@
 // fp32 implicit GEMM for launches with few tiles (gfx950): K cut over the wavefronts of a workgroup.
 //
-// A tile of 32 x 32, 64 x 32 or 16 x 16 belongs to one workgroup of 4, 8 or 16 wavefronts; wavefront w takes the K steps w,
+// A tile of 32 x 32, 64 x 32 or 16 x 16 belongs to one workgroup of four wavefronts (32 x 32: or eight); wavefront w takes the K steps w,
 // w + NW, w + 2 NW ... of it, with both operands straight from memory in registers: no LDS, no barrier and no neighbour to wait
 // for in the K loop.  The wavefronts' sums meet in LDS once, and every thread finishes one to eight outputs.
 //

@@ -5,8 +5,6 @@
 // reference by the last bits of expf and is held to the fp32 tolerance.
 #include <string.h>
 
-#include <type_traits>
-
 #include "row_norm.hpp"
 
 namespace onhip {
