@@ -53,8 +53,19 @@ __host__ __device__ inline bool dma_lone(unsigned workgroups) { return workgroup
 
 template <int KS> __device__ __forceinline__ int dma_swz(int row) { return KS == 128 ? ((row >> 1) & 7) : ((row >> 2) & 3); }
 
+// LDS of a workgroup: the ring, then in the same memory what the store needs: its staging area, the quantised or 16-bit activation table and
+// the per-row constants; or, for fp32 results through an activation table, that table (TABLE; not for the kernels of short taps, which
+// would lose a resident workgroup to it)
+__host__ __device__ constexpr int dma_rows_at(int dt, int bm, int bn) { return dt == DT_I8 ? bn * (bm + 16) + 8192 : bn * (2 * bm + 16) + 16384; }
+__host__ __device__ constexpr int dma_lds_bytes(int dt, int bm, int bn, int ks, int nst, bool multi) {
+    const int ring = nst * (bm + bn) * ks, out = dma_rows_at(dt, bm, bn) + 2 * bm * 4, store = !multi && out < TABLE_BYTES ? TABLE_BYTES : out;
+    return ring > store ? ring : store;
+}
+
+// (the second bound: as many wavefronts a SIMD as LDS has room for workgroups.  A register more than that, 169 in the int8 128 x 128 tile of
+// 64-byte stages, is a resident workgroup less: 57 -> 206 channels on 123 x 123 at batch 4 13.7 and 15.0 us)
 template <int DT, int BM, int BN, int WM, int WN, int KS, int NST, bool MULTI = false>
-__global__ __launch_bounds__(THREADS) void igemm_dma_kernel(const IgemmParams p) {
+__global__ __launch_bounds__(THREADS, 160 * 1024 / dma_lds_bytes(DT, BM, BN, KS, NST, MULTI)) void igemm_dma_kernel(const IgemmParams p) {
     // device pass only: the host pass cannot parse the inline assembly's register constraints, and a kernel whose body it
     // rejects gets no launch stub
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -73,15 +84,9 @@ __global__ __launch_bounds__(THREADS) void igemm_dma_kernel(const IgemmParams p)
     // 64 KiB window, and a stage's offset inside its window is the instruction's immediate
     static_assert(NST >= 2 && NST * STAGE <= 160 * 1024, "the ring must fit the 160 KiB of LDS of a compute unit");
     constexpr int NSETS = (NST * STAGE + 65535) / 65536;
-    // after the K loop the same memory holds the store's staging area, the quantised activation table and the per-row constants
-    constexpr int OUT_STAGE = DT == DT_I8 ? BN * (BM + 16) : BN * (2 * BM + 16), ROWS_AT = OUT_STAGE + (DT == DT_I8 ? 8192 : 16384), OUT_BYTES = ROWS_AT + 2 * BM * 4;
+    constexpr int ROWS_AT = dma_rows_at(DT, BM, BN), LDS_BYTES = dma_lds_bytes(DT, BM, BN, KS, NST, MULTI);
     static_assert(ROWS_AT % 16 == 0, "the per-row constants are read 16 bytes at a time");
-    // stores of fp32 results through an activation table: the table, and the per-row constants behind it (not for the kernels of
-    // short taps, which would lose a resident workgroup to it)
     constexpr bool TABLE = !MULTI;
-    constexpr int TABLE_ROWS = TABLE_BYTES + 2 * BM * 4;
-    constexpr int STORE_BYTES = TABLE && TABLE_ROWS > OUT_BYTES ? TABLE_ROWS : OUT_BYTES;
-    constexpr int LDS_BYTES = NST * STAGE > STORE_BYTES ? NST * STAGE : STORE_BYTES;
     __shared__ __attribute__((aligned(1024))) unsigned char lds[LDS_BYTES];
 
     warm_params<sizeof(IgemmParams)>();
@@ -297,7 +302,9 @@ __global__ __launch_bounds__(THREADS) void igemm_dma_kernel(const IgemmParams p)
     // every wavefront done with the operand buffers, before the store reuses that memory
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    float *rows = reinterpret_cast<float *>(lds + (table ? TABLE_BYTES : ROWS_AT));
+    // where the ring's memory holds the table, the per-row constants are in LDS that the launcher adds: the kernel would otherwise keep it for
+    // them in every launch, and 64 x 64 tiles of 64-byte stages one workgroup less
+    float *rows = table && !table_first ? s_table : reinterpret_cast<float *>(lds + ROWS_AT);
     if (table && !table_first) request_table(p.ep.lut, reinterpret_cast<float *>(lds), wave, lane, THREADS);
     if (tid < BM) {
         if constexpr (DT == DT_I8) {
@@ -379,7 +386,7 @@ int dma_launch_one(const IgemmParams &p_in, hipStream_t stream) {
     p.div_ow = make_div31((unsigned) (p.OW > 0 ? p.OW : 1));
     p.div_tiles_m = make_div31((unsigned) tiles_m);
     hipLaunchKernelGGL((igemm_dma_kernel<DT, BM, BN, 2, 2, KS, NST, MULTI>), dim3((unsigned) tiles), dim3(THREADS),
-                       !MULTI && dma_lone((unsigned) tiles) ? table_lds_bytes(p) : 0u, stream, p);
+                       MULTI || !table_in_lds(p) ? 0u : dma_lone((unsigned) tiles) ? (unsigned) TABLE_BYTES : 2u * BM * 4u, stream, p);
     ONHIP_CHECK_HIP(hipGetLastError());
     return ONHIP_OK;
 }

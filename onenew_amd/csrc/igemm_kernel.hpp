@@ -302,9 +302,10 @@ __device__ __forceinline__ unsigned b_voff(const IgemmParams &p, const ColState 
 constexpr int TABLE_BYTES = 8192 * 4;
 typedef const __attribute__((address_space(3))) float *lds_f32_t;
 __host__ __device__ inline bool table_in_lds(const IgemmParams &p) {
+    if (p.ep.act != SILU && p.ep.act != ONHIP_ACT_GELU_LUT) return false;   // first: most launches have nothing more to ask
     const bool int8_rows = p.out_s8 && p.out_mode == OUT_PLAIN && p.c_stride_m == 1 && !p.acc_out;   // has the quantised table
     const bool slices_only = p.partial && !p.arrive && p.dp_tiles == 0;
-    return (p.ep.act == SILU || p.ep.act == ONHIP_ACT_GELU_LUT) && !int8_rows && !p.out_h16 && !slices_only;
+    return !int8_rows && !p.out_h16 && !slices_only;
 }
 // igemm_kernel's tiles of 4096 results (16 KiB, half the table) have it there only where a launch's workgroups are all resident with it, three a
 // compute unit (two in 32 x 128): five or six are without, and where there is a second round that is worth more (fp32 33 -> 668 channels on 58 x 58 at batch 8, 4431

@@ -48,3 +48,34 @@ def test_table(tile, rows, cols, kind, monkeypatch):
     assert torch.equal(run(), ref + r if kind == "add" else ref)
     ran = hip.last_launch_choice()
     assert f"{ran[0]}x{ran[1]}" == tile.removesuffix("x2") and (ran[2] == 2) == tile.endswith("x2"), ran
+
+
+@pytest.mark.parametrize("tiles", [40, 257], ids=["alone", "several a unit"])
+@pytest.mark.parametrize("tile", ["128x128", "128x64", "64x128", "64x64"])
+@pytest.mark.parametrize("kind,cin", [("w8a32", 64), ("w8a32", 128), ("bf16", 32), ("bf16", 64)])
+def test_table_of_the_direct_to_lds_kernel(kind, cin, tile, tiles, monkeypatch):
+    """stages of 64 and of 128 bytes; the table in LDS of its own with up to 256 workgroups, in the ring's memory with more, where the per-row
+    constants move out of it"""
+    import torch
+    hip.init(0)
+    print("table, direct to LDS", kind, cin, tile, tiles, flush=True)
+    monkeypatch.setenv("ONHIP_TILE", tile + "x1x0x0x0x1")
+    bm, bn = map(int, tile.split("x"))
+    d = ConvDesc(n=1, cin=cin, h=1, w=(tiles - 1) * bn + 5, cout=bm - 3, kh=1, kw=1, stride_h=1, stride_w=1, group=1, has_bias=1, act_type=abi.NOT_ACT,
+                 compute=abi.COMPUTE_F32)
+    g = torch.Generator(device="cuda").manual_seed(cin + tiles)
+    x, table = torch.randn((1, cin, 1, d.w), generator=g, device="cuda"), torch.randn(8192, generator=g, device="cuda")
+    if kind == "w8a32":
+        d.input_scale = 0.02
+        w = hip.pack_conv_weights_w8(d, torch.randint(-127, 128, (d.cout, cin, 1, 1), generator=g, device="cuda", dtype=torch.int8))
+        b, aux = torch.randint(-999, 999, (d.cout,), generator=g, device="cuda", dtype=torch.int32), torch.rand(d.cout, generator=g, device="cuda")
+        run = lambda: hip.conv2d_w8a32(d, x, w, b, aux, table, packed=True)   # noqa: E731
+    else:
+        d.compute = abi.COMPUTE_BF16
+        xh, w = hip.h16_from_nchw(x, d.compute), hip.h16_pack_conv_weights(d, torch.randn((d.cout, cin, 1, 1), generator=g, device="cuda"))
+        b = torch.randn(d.cout, generator=g, device="cuda")
+        run = lambda: hip.conv2d_h16(d, xh, w, b, table, y_kind=hip.H16_OUT_F32_NCHW)   # noqa: E731
+    y = run()
+    d.act_type = abi.SILU
+    assert torch.equal(run(), through_table(torch, y, table)) and bool((y < -8.0).any()) and bool((y > 8.0).any())
+    assert tuple(hip.last_launch_choice()) == (bm, bn, 1, 0, 0, 0, 1)
