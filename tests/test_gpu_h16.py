@@ -329,3 +329,26 @@ def test_ring_by_the_count_of_stages(n, cin, hw, cout, k, ring, torch_dev, monke
     assert ran[6] == ring, ran
     monkeypatch.setenv("ONHIP_TILE", f"{ran[0]}x{ran[1]}x1x0x0x0x1")
     assert torch.equal(hip.conv2d_h16(d, x, w, b), y) and hip.last_launch_choice()[6] == 1
+
+
+# (n, cin, hw, cout, residual operand, tile): one and two stages, where the store is most of the launch
+TILE_CHOICES = [(16, 21, 145, 83, False, (128, 128)), (16, 74, 71, 384, False, (128, 128)), (4, 49, 135, 93, False, (128, 64)), (4, 50, 92, 134, False, (64, 128)),
+                (16, 74, 71, 384, True, (64, 128))]
+
+
+@pytest.mark.parametrize("n,cin,hw,cout,add,tile", TILE_CHOICES)
+def test_tile_of_few_stages(n, cin, hw, cout, add, tile, torch_dev, monkeypatch):
+    """the tile that the cost model takes, and the same bits as with another one"""
+    torch = torch_dev
+    print("few stages", n, cin, hw, cout, add, flush=True)
+    monkeypatch.delenv("ONHIP_TILE", raising=False)
+    d = with_compute(cases.cd(cin, cout, 1, 1, 0, hw, n=n, act=abi.RELU), abi.COMPUTE_BF16)
+    g = torch.Generator(device="cuda").manual_seed(cin + cout)
+    x = hip.h16_from_nchw(torch.randn((n, cin, hw, hw), generator=g, device="cuda"), d.compute)
+    w = hip.h16_pack_conv_weights(d, torch.randn((cout, cin, 1, 1), generator=g, device="cuda") / cin ** 0.5)
+    b = torch.randn(cout, generator=g, device="cuda")
+    r = hip.h16_from_nchw(torch.randn((n, cout, hw, hw), generator=g, device="cuda"), d.compute) if add else None
+    y = hip.conv2d_h16(d, x, w, b, residual=r)
+    assert tuple(hip.last_launch_choice()[:2]) == tile
+    monkeypatch.setenv("ONHIP_TILE", "64x64x1x0x0x0x1")
+    assert torch.equal(hip.conv2d_h16(d, x, w, b, residual=r), y) and tuple(hip.last_launch_choice()[:2]) == (64, 64)
