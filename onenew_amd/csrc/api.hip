@@ -682,7 +682,8 @@ static bool f3_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out
 // fit the L2s: with more the other kernels, which load a tile once, are ahead anyway.
 // Columns of different images are apart by a whole image, and a load of 64 lanes touches a cache line for each: with one-pixel images the
 // lines set the pace (29 of them, 848 -> 299 channels, 16.6 us, 7.7 on the other kernels; 96 of them, 1280 -> 1000, 26.6 and 12.4), and rows
-// that straddle lines cost on other small planes (12 images of 3 x 3, 592 -> 267, 9.3 and 8.1).
+// that straddle lines cost on other small planes (12 images of 3 x 3, 592 -> 267, 9.3 and 8.1; with a stride, so that a load's columns are in more
+// than a dozen images, 16 of 4 x 4, 432 -> 176, 11.0 and 7.8).
 // Fewer steps of 16 than wavefronts leave some of them idle, and the launch costs what it costs: 16 -> 618 channels on 15 x 15 at batch 2 in
 // tiles of 64 x 32 5.0 us, 4.2 on the other kernels; in more than one round of 32 x 32 8 -> 47 on 24 x 24 at batch 8 4.4 and 4.0, 64 -> 182 on
 // 39 x 39 5.4 and 4.9.
@@ -698,7 +699,8 @@ static bool kw_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out
         const int steps = (p.K + ks - 1) / ks;
         if (tiles > 2048 || (bm > p.M + 15) || (t == 2 && steps < 6) || (t == 1 && tiles > 256 && steps < 5) || !kw_ok(cfg, p, bm, split != 0)) continue;
         const double lines = 64.0 / bn * std::min(bn, p.N) / p.OHW;   // of a load of B, where images are smaller than the tile
-        const double apart = p.OHW == 1 ? (t == 0 ? 0.0032 * std::max(0.0, lines - 12.0) : (t == 1 ? 0.0028 : 0.002) * lines) : p.OHW < 16 && p.HW % 4 && cfg.bl == BL_PLAIN ? 0.05 : 0.0;
+        const double apart = p.OHW == 1 ? (t == 0 ? 0.0032 * std::max(0.0, lines - 12.0) : (t == 1 ? 0.0028 : 0.002) * lines)
+                             : p.OHW <= 4 && p.sw > 1 && lines > 12.0 ? 0.11 : p.OHW < 16 && p.HW % 4 && cfg.bl == BL_PLAIN ? 0.05 : 0.0;
         const double a_step = step[split][t] * (p.sw > 1 && p.OW > 1 ? 1.4 : 1.0) + apart;
         const double t_us = base[split][t] + ((tiles + 255) / 256) * steps * a_step + tiles * start[t];
         if (t_us < *us) { *us = t_us; *out = Choice{bm, bn, t == 1 && tiles <= 256 && steps >= 32 ? 8 : 4, 0, 3, 0, 0}; }

@@ -127,7 +127,7 @@ def test_choice(torch_dev, monkeypatch):
 
 
 @pytest.mark.parametrize("layer,ours", [((29, 848, 1, 1, 299, 1, 1, 0), False), ((96, 1280, 1, 1, 1000, 1, 1, 0), False), ((2, 16, 15, 15, 618, 1, 1, 0), False),
-                                        ((8, 8, 24, 24, 47, 1, 1, 0), False), ((4, 64, 1, 1, 746, 1, 1, 0), (16, 16)), ((4, 1376, 2, 2, 110, 1, 1, 0), (16, 16))])
+                                        ((8, 8, 24, 24, 47, 1, 1, 0), False), ((16, 432, 4, 4, 176, 1, 2, 0), False), ((4, 64, 1, 1, 746, 1, 1, 0), (16, 16)), ((4, 1376, 2, 2, 110, 1, 1, 0), (16, 16))])
 def test_choice_where_loads_or_steps_do_not_fit_it(layer, ours, torch_dev, monkeypatch):
     """one-pixel images (a cache line for each column of a load) and reductions of fewer steps than wavefronts"""
     torch = torch_dev
