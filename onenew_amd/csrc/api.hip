@@ -576,7 +576,7 @@ static bool dma_model_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choi
     // stages of K are mostly the tile's store.  One of 16 bits with a residual operand, or of fp32 results, takes as long per output in 64 x 128
     // (256 x 100352 x 64 in bf16 with an Add 25.0 -> 23.2 us, 512 x 25088 x 128 17.8 -> 16.0, 17.0 in 128 x 64); one of 16 bits alone or of int8 does
     // not, and costs more where a tile is small (83 x 336400 x 32 with SiLU in bf16 39 us, 32 in 128 x 128; 249 x 150152 x 144 in int8 37.8 and
-    // 33.0).  Fitted to four tiles of 650 such layers of 3 to 40 million results: the choices 1.2-1.7 % above the fastest (2.1-3.5 before).
+    // 33.0).  Fitted to the four tiles of 600 such layers of 3 to 40 million results: the choices 1.2-1.7 % above the fastest (the last sort 2.0-3.7 before).
     const bool only = cfg.dtype != DT_I8;   // the 16-bit types have no other kernel for these operands
     static const double kEff[3][4] = {{1.0, 1.10, 1.08, 1.20}, {1.0, 1.10, 1.0, 1.20}, {1.0, 1.12, 1.12, 1.40}};
     const double *eff = kEff[p.k_units > 16 ? 0 : only && (p.res16 || !p.out_h16) ? 1 : 2];

@@ -312,7 +312,12 @@ __host__ __device__ inline bool table_in_lds(const IgemmParams &p) {
 // workgroups, 58 -> 44 us, 16 -> 52 under 3x3 at 113 x 113 and batch 16, 3193, 54 -> 50; 14 -> 21 on 36 x 36 at batch 16, 162, 5.7 and 6.8).  In int8
 // 64 x 64 it is not (88 -> 292 on 50 x 50 at batch 16, 3125, 22.9 with it and 25.1).
 __host__ __device__ constexpr bool table_unless_many(int dt, int bm, int bn) { return bm * bn <= 4096 && (dt != DT_I8 || bm == 32); }
-__host__ __device__ inline bool table_few(int bm, unsigned workgroups) { return workgroups <= (bm == 32 ? 512u : 768u); }
+// With more workgroups than that the table stays worth it in 64 x 64 while K is short and the store most of the launch (150 layers with SiLU, 769 to
+// 12348 workgroups: up to a K of 24 0.90-0.97 of the time, from 45 on 1.0-1.13; with a residual operand, whose registers leave no sixth
+// workgroup, 0.79-0.97 up to 64 of a 1x1 filter and 36 of others; 32 x 128, three workgroups fewer, 1.06-1.39 whatever K).
+__host__ __device__ inline bool table_few(int bl, int bm, bool res, int k, unsigned workgroups) {
+    return workgroups <= (bm == 32 ? 512u : 768u) || (bm == 64 && k <= (!res ? 24 : bl == BL_PLAIN ? 64 : 36));
+}
 inline unsigned table_lds_bytes(const IgemmParams &p) { return table_in_lds(p) ? TABLE_BYTES : 0u; }
 // every wavefront of the workgroup (nt threads) takes its share; complete once each has waited for its loads (vmcnt, in so many words: no
 // register tells the compiler) and a barrier has passed
@@ -1210,7 +1215,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(igemm_w
     const int wm = wave / WN, wn = wave % WN;
 
     extern __shared__ __attribute__((aligned(1024))) float s_table[];   // TABLE_BYTES where table_in_lds says so
-    const bool table = !PW2 && table_in_lds(p) && (!table_unless_many(DT, BM, BN) || table_few(BM, gridDim.x * gridDim.y * gridDim.z));   // uniform
+    const bool table = !PW2 && table_in_lds(p) && (!table_unless_many(DT, BM, BN) || table_few(BL, BM, RES, p.K, gridDim.x * gridDim.y * gridDim.z));   // uniform
     if (table) request_table(p.ep.lut, s_table, wave, lane, THREADS);
 
     const TilePlace tp = place_tile<BM, BN>(p);
@@ -1661,7 +1666,7 @@ static int launch_one(const IgemmLaunch &cfg, const IgemmParams &p_in, hipStream
     const int rc = tile_grid<BM, BN>(cfg, p, &grid);
     if (rc) return rc;
     if (RES != (p.res != nullptr)) return set_error(ONHIP_ERR_ARG, "igemm: residual operand and kernel variant do not match");
-    hipLaunchKernelGGL((igemm_kernel<DT, BL, BM, BN, WM, WN, PF, RES>), grid, dim3(THREADS), !table_unless_many(DT, BM, BN) || table_few(BM, grid.x * grid.y * grid.z) ? table_lds_bytes(p) : 0u, stream, p);
+    hipLaunchKernelGGL((igemm_kernel<DT, BL, BM, BN, WM, WN, PF, RES>), grid, dim3(THREADS), !table_unless_many(DT, BM, BN) || table_few(BL, BM, RES, p.K, grid.x * grid.y * grid.z) ? table_lds_bytes(p) : 0u, stream, p);
     ONHIP_CHECK_HIP(hipGetLastError());
     return finish_launch<DT == DT_I8>(cfg, p, stream);
 }

@@ -14,21 +14,23 @@ def through_table(torch, y, table):
     return torch.where(y < -8.0, torch.zeros_like(y), torch.where(y >= 8.0, y, z))
 
 
-# (tile, rows, columns): 512 and 513 workgroups of 32 x 128, 768 and 769 of 64 x 64, one, and more than a round of a tile that always has it in LDS
-SIZES = [("32x128", 32, 512 * 128), ("32x128", 29, 512 * 128 + 1), ("32x128", 7, 40), ("64x64", 64, 768 * 64), ("64x64", 61, 768 * 64 + 3), ("64x64", 200, 50),
-         ("64x64x2", 130, 385 * 64), ("64x128", 64, 1025 * 128), ("128x128", 100, 300 * 128)]
+# (tile, rows, columns, K): 512 and 513 workgroups of 32 x 128, 768 and 769 of 64 x 64 (with more, a K on either side of the one up to which the table
+# is in LDS: 24, and 64 with a residual operand), one, and more than a round of a tile that always has it in LDS
+SIZES = [("32x128", 32, 512 * 128, 20), ("32x128", 29, 512 * 128 + 1, 20), ("32x128", 7, 40, 20), ("64x64", 64, 768 * 64, 20), ("64x64", 61, 768 * 64 + 3, 20),
+         ("64x64", 64, 768 * 64, 65), ("64x64", 61, 768 * 64 + 3, 25), ("64x64", 61, 768 * 64 + 3, 64), ("64x64", 61, 768 * 64 + 3, 65), ("64x64", 200, 50, 20),
+         ("64x64x2", 130, 385 * 64, 20), ("64x128", 64, 1025 * 128, 20), ("128x128", 100, 300 * 128, 20)]
 
 
 @pytest.mark.parametrize("kind", ["f32", "w8a32", "add"])
-@pytest.mark.parametrize("tile,rows,cols", SIZES)
-def test_table(tile, rows, cols, kind, monkeypatch):
+@pytest.mark.parametrize("tile,rows,cols,k", SIZES)
+def test_table(tile, rows, cols, k, kind, monkeypatch):
     import torch
     hip.init(0)
     if kind == "w8a32" and tile.endswith("x2"):
         pytest.skip("one K tile: nothing to cut")
-    print("table store", tile, rows, cols, kind, flush=True)
+    print("table store", tile, rows, cols, k, kind, flush=True)
     monkeypatch.setenv("ONHIP_TILE", tile)
-    d = ConvDesc(n=1, cin=20, h=1, w=cols, cout=rows, kh=1, kw=1, stride_h=1, stride_w=1, group=1, has_bias=1, act_type=abi.NOT_ACT, compute=abi.COMPUTE_F32)
+    d = ConvDesc(n=1, cin=k, h=1, w=cols, cout=rows, kh=1, kw=1, stride_h=1, stride_w=1, group=1, has_bias=1, act_type=abi.NOT_ACT, compute=abi.COMPUTE_F32)
     g = torch.Generator(device="cuda").manual_seed(rows + cols)
     x = torch.randn((1, d.cin, 1, cols), generator=g, device="cuda")
     table = torch.randn(8192, generator=g, device="cuda")
