@@ -1171,12 +1171,8 @@ __device__ __forceinline__ bool reduce_in_launch(const IgemmParams &p, f32x16 (&
 }
 
 // ---- the kernel --------------------------------------------------------------------------------
-// wavefronts a SIMD that the registers have to leave room for, where the compiler's own choice is a few registers past it
-__host__ __device__ constexpr int igemm_waves(int dt, int bm, int bn, bool res, bool pw2) {
-    return pw2 ? 4 : dt == DT_I8 && res && bm * bn <= 4096 ? 5 : 1;
-}
 template <int DT, int BL, int BM, int BN, int WM, int WN, int PF = 1, bool RES = false, bool PW2 = false>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(igemm_waves(DT, BM, BN, RES, PW2)))) void igemm_kernel(const IgemmParams p) {
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(PW2 ? 4 : 1))) void igemm_kernel(const IgemmParams p) {
     static_assert(!PW2 || (DT == DT_F32 && BM == 64 && BN == 64 && WM == 2 && WN == 2), "the second product exists for fp32 tiles of 64 x 64");
     static_assert(!RES || DT == DT_F32 || DT == DT_I8, "the residual store exists for fp32 and int8 operands (fp32 results)");
     static_assert(WM * WN == 4, "four wavefronts per workgroup");
