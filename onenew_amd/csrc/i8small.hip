@@ -338,14 +338,14 @@ bool i8small_ok(const onhip_conv_desc_t &d, int OH, int OW, const I8SmallIO &io,
     if (!io.xq) return plan->us < 0.9 * (5.9 + std::min(0.002 * k, 5.0) + 4e-6 * d.n * (in + out) / 4.4 - (table ? 0.0 : 1.0));
     const long long tiles = (d.cout + 63LL) / 64 * (((long long) d.n * OH * OW + 63) / 64);
     const double other = io.res ? 4.3 + 0.0027 * k : 3.4 + (table ? 0.5 : 0.0) + (tiles < 96 && units >= 128 ? 0.0029 * k : std::min(0.002 * k, 6.6));
-    // From a K of some 7000 on the other kernels cut it into slices, which a launch more adds up (not with a residual operand).  What that takes is
-    // fitted to 180 launches of up to 90 tiles and a K of 58800 (5 % off), and this kernel's own time there, where more than 3 MB of weights go past
-    // every workgroup, to 176; the choices within 8 % of the faster one.  1198 channels under a 7x7 filter, stride 3, on 5 x 5 at batch 4 48 us, 15 in
-    // slices; 832 -> 35, 7x7 on 11 x 11, 24 and 12; 1372 -> 73, 5x5 and stride 3 on 8 x 8 at batch 4, 20 and 12; 1366 -> 172, 3x3 on 13 x 13 at batch
-    // 2, 11.0 and 13.4.
-    if (k > 7000.0 && !io.res) {
-        const double sliced = 8.38 + 1e-4 * k + 1.44e-5 * k * (double) (tiles - 1) - 0.06 * (double) tiles + 1.28e-5 * d.cout * ((double) d.n * OH * OW);
-        if (plan->us / 0.95 + 0.9 * std::max(0.0, 1e-6 * d.cout * k - 3.0) > 0.98 * sliced) return false;
+    // From a K of some 7000 on, the longer the more tiles there are (130 tiles from 26000), the other kernels cut it into slices, which a launch more
+    // adds up (not with a residual operand).  What that takes is fitted to 605 launches (4 % off), and this kernel's own time there, where more than
+    // 3 MB of weights go past every workgroup, to 532 (7 %); the choices within 20 % of the faster one and 0.2 % on average (16 % without the rule).
+    // 1198 channels under a 7x7 filter, stride 3, on 5 x 5 at batch 4 48 us, 15 in slices; 832 -> 35, 7x7 on 11 x 11, 24 and 12; 154 -> 1146, 7x7
+    // and stride 2 on 11 x 11, K 7840 and not cut, 8.0 and 31.6.
+    if (k > 7000.0 + 90.0 * (double) tiles && !io.res) {
+        const double sliced = 8.55 + 7.7e-5 * k + 1.3e-5 * k * (double) tiles - 0.0836 * (double) tiles + 3.6e-5 * d.cout * ((double) d.n * OH * OW);
+        if (1.193 * plan->us - 1.02 + 0.183 * std::max(0.0, 1e-6 * d.cout * k - 3.0) > 0.98 * sliced) return false;
     }
     return plan->us < 0.92 * other;
 }

@@ -145,6 +145,7 @@ def test_many_tiles_stay_staged():
 
 
 @pytest.mark.parametrize("case,ours", [((4, 1198, 5, 5, 248, 7, 3, 3, N), False), ((1, 832, 11, 11, 35, 7, 1, 3, R), False), ((2, 1844, 5, 5, 147, 5, 3, 2, S), False),
+                                       ((1, 154, 11, 11, 1146, 7, 2, 3, R), True), ((4, 784, 6, 6, 948, 3, 3, 1, N), True), ((2, 811, 7, 7, 795, 3, 3, 1, S), True),
                                        ((1, 512, 7, 7, 96, 3, 1, 1, R), True), ((1, 800, 7, 7, 64, 3, 1, 1, N), True), ((2, 1366, 13, 13, 172, 3, 1, 1, R), True)])
 def test_long_reductions_are_cut_into_slices(case, ours):
     """from int8 activations: where the other kernels cut K, one launch is the slower form of a long one"""
