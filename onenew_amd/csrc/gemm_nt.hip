@@ -164,19 +164,19 @@ static void gemm_nt_few(int m, int k, int n, const float *a, const float *w, con
 // second round of workgroups the other kernels, which share operands among more columns, are ahead: 2048 -> 1000 at 96 rows (378
 // workgroups) 16.6 against 14.7 us, 4096 -> 4096 at 16 rows (256) 17.4 against 38, at 24 rows (512) 31 against 24.5.  Up to 8 rows it
 // takes 6.3 to 7.6 us where the vector kernel takes 2.7 to 4.1.
-// A workgroup walks all of K, 3.3 ns an element whatever the other workgroups do; the convolution kernels cut a long K into slices
-// and are then bound by the weights: 25088 -> 512 at 16 rows 88 against 25 us, 8192 -> 2048 31 against 25, 4096 -> 512 at 64 rows 16.5 against
-// 12.4.  Both are fitted to 500 launches of 9 to 128 rows, 10 to 4096 columns and K of 128 to 25088, the choices within 7 % of the
-// faster one.
+// A workgroup walks all of K, 1.4 to 3 ns an element, slowest with rows that start at the same place of a cache line; the convolution kernels
+// cut a long K into slices and are then bound by the weights: 25088 -> 512 at 16 rows 88 against 25 us, 8192 -> 2048 31 against 25, 4096 -> 512 at
+// 64 rows 16.9 against 12.4, but 4096 -> 4096 at 16 rows 19.3 and 25.1, 2544 -> 1641 at 21 rows 10.0 and 13.2, 3992 -> 706 at 65 12.7 and 23.3.
+// Both are fitted to 1121 launches of 9 to 160 rows, 10 to 5000 columns and K of 1025 to 26000, on weights in the L2s and beyond them; the
+// choices are 0.4 % above the faster one.
 bool gemm_nt_mfma_ok(int m, int k, int n, const float *a, const float *w) {
     const long long lim = 1LL << 29;
     if (k % 4 || ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w)) & 15) || (long long) m * k >= lim || (long long) n * k >= lim ||
         (long long) m * n >= lim || (long long) ((m + 15) / 16) * ((n + 15) / 16) > 256)
         return false;
-    const double mb = 4e-6 * n * k, us = 2.5 + (k > 2048 ? 1.0 : 0.0) + (m > 16 ? 0.3 : 0.0) + 0.0033 * k * (0.6 + 0.025 * std::min(m, 16)) * (n < 64 ? 0.8 : 1.0);
-    const double other = 6.4 + 0.00055 * k + (0.25 * std::min(mb, 20.0) + 0.23 * std::max(0.0, mb - 20.0)) * std::min(1.0, n / 1000.0) +
-                         std::max(0, m - 16) * (0.015 + 0.0057 * std::min(mb, 20.0));
-    return k <= 1024 || us < 0.97 * other;
+    const double mb = 4e-6 * n * k, lines = k % 32 ? 1.0 : k <= 2048 ? 1.15 : 1.25;
+    const double us = lines * (3.0 + k * (0.00141 + 6.3e-5 * std::min(m, 16)) + 0.088 * mb), other = 6.85 + 0.00054 * k + mb * (0.17 + 0.0058 * m) + 0.0123 * m;
+    return k <= 1024 || us < other;
 }
 
 int gemm_nt_launch(int m, int k, int n, const float *a, const float *w, const float *bias, float *out, hipStream_t stream) {

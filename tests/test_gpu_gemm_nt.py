@@ -50,7 +50,7 @@ def test_gemm_operands_off_sixteen_bytes(m, torch_dev):
     assert bool(((y - (a.double() @ w.double().T + b.double())).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("m,k,n,tiled", [(16, 25088, 512, True), (64, 4096, 512, True), (16, 8192, 2048, True), (17, 1028, 5000, True), (16, 4096, 4096, False),
+@pytest.mark.parametrize("m,k,n,tiled", [(16, 25088, 512, True), (64, 4096, 512, True), (16, 8192, 2048, True), (17, 1028, 5000, True), (16, 4096, 4096, False), (21, 2544, 1641, False), (46, 1796, 311, False), (130, 2100, 28, False), (68, 3752, 642, False),
                                          (48, 2048, 1000, False), (9, 2048, 1000, False), (64, 192, 1000, False)])
 def test_gemm_hand_over(m, k, n, tiled, torch_dev):
     """a K that the tiled kernels are faster on, cut into slices, goes there (they leave a launch choice, the kernels of a batch's rows do not)"""
