@@ -674,6 +674,8 @@ static bool f3_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out
     }
     return true;
 }
+// the part of a one-pixel result's taps that lie inside the image: the others are not loaded
+static double one_pixel_share(const IgemmProblem &p) { return std::min(1.0, (double) p.H * p.W / p.khkw); }
 // Best shape of the kernel whose wavefronts share K, and its microseconds.  From the layers of ResNet-50 at batch 1 (80 layers, 4
 // shapes and both forms of the weights, weights beyond the L2; error 10 %) and 950 launches of random layers, small planes and batches of
 // one-pixel images among them: a compute unit does its workgroups' steps one after the
@@ -686,20 +688,21 @@ static bool f3_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out
 // than a dozen images, 16 of 4 x 4, 432 -> 176, 11.0 and 7.8).
 // Fewer steps of 16 than wavefronts leave some of them idle, and the launch costs what it costs: 16 -> 618 channels on 15 x 15 at batch 2 in
 // tiles of 64 x 32 5.0 us, 4.2 on the other kernels; in more than one round of 32 x 32 8 -> 47 on 24 x 24 at batch 8 4.4 and 4.0, 64 -> 182 on
-// 39 x 39 5.4 and 4.9.
+// 39 x 39 5.4 and 4.9; but with a table activation, for which the others fetch the table, 16 -> 144 under stride 2 on 30 x 30 at batch 8 4.9 and 5.8.
 static bool kw_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out, double *us) {
     static const double step[2][3] = {{0.122, 0.105, 0.21}, {0.087, 0.086, 0.13}};   // fp32 / split weights; tiles of 16, 32, 64 rows
     static const double base[2][3] = {{2.8, 3.6, 4.4}, {3.4, 3.6, 4.4}}, start[3] = {0.0016, 0.003, 0.003};
     *us = 1e300;
     if (cfg.dtype != DT_F32 || p.b_slice_bytes > (8LL << 20)) return false;
     const int split = kw_split(cfg, p);
+    const bool table = p.ep.act == SILU || p.ep.act == ONHIP_ACT_GELU_LUT;
     for (int t = 0; t < 3; ++t) {
         const int bm = 16 << t, bn = t ? 32 : 16, ks = t ? 16 : 32;
         const long long tiles = (long long) ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
         const int steps = (p.K + ks - 1) / ks;
-        if (tiles > 2048 || (bm > p.M + 15) || (t == 2 && steps < 6) || (t == 1 && tiles > 256 && steps < 5) || !kw_ok(cfg, p, bm, split != 0)) continue;
+        if (tiles > 2048 || (bm > p.M + 15) || (t == 2 && steps < 6) || (t == 1 && tiles > 256 && steps < 5 && !table) || !kw_ok(cfg, p, bm, split != 0)) continue;
         const double lines = 64.0 / bn * std::min(bn, p.N) / p.OHW;   // of a load of B, where images are smaller than the tile
-        const double apart = p.OHW == 1 ? (t == 0 ? 0.0032 * std::max(0.0, lines - 12.0) : (t == 1 ? 0.0028 : 0.002) * lines)
+        const double apart = p.OHW == 1 ? one_pixel_share(p) * (t == 0 ? 0.0032 * std::max(0.0, lines - 12.0) : (t == 1 ? 0.0028 : 0.002) * lines)
                              : p.OHW <= 4 && p.sw > 1 && lines > 12.0 ? 0.11 : p.OHW < 16 && p.HW % 4 && cfg.bl == BL_PLAIN ? 0.05 : 0.0;
         const double a_step = step[split][t] * (p.sw > 1 && p.OW > 1 ? 1.4 : 1.0) + apart;
         const double t_us = base[split][t] + ((tiles + 255) / 256) * steps * a_step + tiles * start[t];
@@ -767,7 +770,7 @@ static Choice model_choice(const IgemmLaunch &cfg, const IgemmProblem &p) {
     // odd planes it is 15 % over)
     auto others = [&]() {
         const double slices = std::max(1, best.split), rounds = std::ceil(((p.M + best.bm - 1) / best.bm) * ((p.N + best.bn - 1) / best.bn) * slices / 256.0);
-        const double apart = p.OHW == 1 ? 0.15 * std::min(1.0, p.N / 64.0) * std::ceil((p.K + 15) / 16 / slices) * rounds : 0.0;
+        const double apart = p.OHW == 1 ? one_pixel_share(p) * 0.15 * std::min(1.0, p.N / 64.0) * std::ceil((p.K + 15) / 16 / slices) * rounds : 0.0;
         return (p.OHW < 16 && p.OHW > 1 && p.HW % 4 && cfg.bl == BL_PLAIN ? 0.85 : 0.95) * (f32_us(cfg, p, best) + apart);
     };
     if (cfg.dtype == DT_F32 && !tl_hint_bm && kw_choice(cfg, p, &kw, &kw_us) && kw_us > others()) kw_us = 1e300;

@@ -127,14 +127,14 @@ def test_choice(torch_dev, monkeypatch):
 
 
 @pytest.mark.parametrize("layer,ours", [((29, 848, 1, 1, 299, 1, 1, 0), False), ((96, 1280, 1, 1, 1000, 1, 1, 0), False), ((2, 16, 15, 15, 618, 1, 1, 0), False),
-                                        ((8, 8, 24, 24, 47, 1, 1, 0), False), ((16, 432, 4, 4, 176, 1, 2, 0), False), ((4, 64, 1, 1, 746, 1, 1, 0), (16, 16)), ((4, 1376, 2, 2, 110, 1, 1, 0), (16, 16))])
+                                        ((8, 8, 24, 24, 47, 1, 1, 0), False), ((16, 432, 4, 4, 176, 1, 2, 0), False), ((64, 48, 1, 1, 1760, 3, 1, 1), (32, 32)), ((4, 64, 1, 1, 746, 1, 1, 0), (16, 16)), ((4, 1376, 2, 2, 110, 1, 1, 0), (16, 16))])
 def test_choice_where_loads_or_steps_do_not_fit_it(layer, ours, torch_dev, monkeypatch):
     """one-pixel images (a cache line for each column of a load) and reductions of fewer steps than wavefronts"""
     torch = torch_dev
     monkeypatch.delenv("ONHIP_TILE", raising=False)
     d = conv_desc(*layer)
     x, w, b = (t.cuda() for t in operands(torch, d, 3, False))
-    y = hip.conv2d_f32(d, x, w, b)
+    y = hip.conv2d_f32(d, x, hip.pack_conv_weights(d, w) if d.kh > 1 else w, b, packed=d.kh > 1)
     ran = hip.last_launch_choice()
     compare(torch, d, y, x.cpu(), w.cpu(), b.cpu())
     assert (ran[4] == 3 and ran[:2] == ours) if ours else ran[4] != 3, ran
