@@ -574,12 +574,14 @@ static bool dma_model_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choi
     static const int order[4][2] = {{128, 128}, {128, 64}, {64, 128}, {64, 64}};
     // What a tile's steady state costs per output against the largest one's (measured on the YOLOv8s and, in bf16, the ResNet-50 layers).  Up to two
     // stages of K are mostly the tile's store.  One of 16 bits with a residual operand, or of fp32 results, takes as long per output in 64 x 128
-    // (256 x 100352 x 64 in bf16 with an Add 25.0 -> 23.2 us, 512 x 25088 x 128 17.8 -> 16.0, 17.0 in 128 x 64); one of 16 bits alone or of int8 does
-    // not, and costs more where a tile is small (83 x 336400 x 32 with SiLU in bf16 39 us, 32 in 128 x 128; 249 x 150152 x 144 in int8 37.8 and
-    // 33.0).  Fitted to the four tiles of 600 such layers of 3 to 40 million results: the choices 1.2-1.7 % above the fastest (the last sort 2.0-3.7 before).
+    // (256 x 100352 x 64 in bf16 with an Add 25.0 -> 23.2 us, 512 x 25088 x 128 17.8 -> 16.0, 17.0 in 128 x 64), and so does any 16-bit one behind stages of
+    // 128 bytes, of which 128 x 128 has two workgroups resident and 64 x 128 three (91 x 147456 x 128 21.2 us in the former, 18.6 in the latter); one of 16 bits
+    // alone behind stages of 64 bytes, or of int8, does not, and costs more where a tile is small (83 x 336400 x 32 with SiLU in bf16 39 us, 32 in
+    // 128 x 128; 249 x 150152 x 144 in int8 37.8 and 33.0).  Fitted to the four tiles of 600 such layers of 3 to 40 million results: the choices
+    // 1.0-1.6 % above the fastest.
     const bool only = cfg.dtype != DT_I8;   // the 16-bit types have no other kernel for these operands
     static const double kEff[3][4] = {{1.0, 1.10, 1.08, 1.20}, {1.0, 1.10, 1.0, 1.20}, {1.0, 1.12, 1.12, 1.40}};
-    const double *eff = kEff[p.k_units > 16 ? 0 : only && (p.res16 || !p.out_h16) ? 1 : 2];
+    const double *eff = kEff[p.k_units > 16 ? 0 : only && (p.res16 || !p.out_h16 || p.units_per_tap % 8 == 0) ? 1 : 2];
     // int8 with a large fp32 result (the reference's W8A32 form on big planes): the register-staged kernel's store of
     // fp32 rows is the faster one from about 6.5 million outputs up (every such YOLOv8s layer at batch 16, 5-35 %)
     if (!only && !p.out_s8 && (long long) p.M * p.N >= (long long) 256 * 25600) return false;

@@ -332,7 +332,7 @@ def test_ring_by_the_count_of_stages(n, cin, hw, cout, k, ring, torch_dev, monke
 
 
 # (n, cin, hw, cout, residual operand, tile): one and two stages, where the store is most of the launch
-TILE_CHOICES = [(16, 21, 145, 83, False, (128, 128)), (16, 74, 71, 384, False, (128, 128)), (4, 49, 135, 93, False, (128, 64)), (4, 50, 92, 134, False, (64, 128)),
+TILE_CHOICES = [(16, 21, 145, 83, False, (128, 128)), (16, 74, 71, 384, False, (128, 128)), (4, 49, 135, 93, False, (64, 128)), (4, 50, 92, 134, False, (64, 128)), (16, 99, 96, 91, False, (64, 128)),
                 (16, 74, 71, 384, True, (64, 128))]
 
 
