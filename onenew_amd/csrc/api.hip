@@ -580,7 +580,7 @@ static bool dma_model_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choi
     // 128 x 128; 249 x 150152 x 144 in int8 37.8 and 33.0).  Fitted to the four tiles of 600 such layers of 3 to 40 million results: the choices
     // 1.0-1.6 % above the fastest.
     const bool only = cfg.dtype != DT_I8;   // the 16-bit types have no other kernel for these operands
-    static const double kEff[3][4] = {{1.0, 1.10, 1.08, 1.20}, {1.0, 1.10, 1.0, 1.20}, {1.0, 1.12, 1.12, 1.40}};
+    static const double kEff[3][4] = {{1.0, 1.10, 1.08, 1.20}, {1.0, 1.10, 1.0, 1.20}, {1.0, 1.12, 1.119, 1.40}};   // (of 128 x 64 and 64 x 128 in as many rounds the latter)
     const double *eff = kEff[p.k_units > 16 ? 0 : only && (p.res16 || !p.out_h16 || p.units_per_tap % 8 == 0) ? 1 : 2];
     // int8 with a large fp32 result (the reference's W8A32 form on big planes): the register-staged kernel's store of
     // fp32 rows is the faster one from about 6.5 million outputs up (every such YOLOv8s layer at batch 16, 5-35 %)
