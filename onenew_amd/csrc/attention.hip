@@ -14,9 +14,10 @@
 // The first product's reduction index (the head dimension) may be enumerated in any order as long as both operands
 // agree: a lane reads four consecutive channels 16 j + 4 (lane / 16) .. + 3 of its row with one 16-byte access and
 // feeds them to four MFMA steps.
-// 16-query wavefronts rather than 32-query ones: 197 tokens are 13 such units per head, 2496 for 64 images of 3 heads,
-// which spread over the 1024 SIMDs in three rounds of a quarter of the 32-query unit's work each; 32-query units (7 per
-// head, 1344) need two rounds of the full unit.
+// 16-query wavefronts rather than 32-query ones, which reach twice the SIMDs.  Head dimension 64 with more workgroups than compute units runs on the
+// 16-bit matrix cores instead (attention_f3.hip).
+#include <stdlib.h>
+
 #include "igemm_kernel.hpp"
 
 namespace onhip {
@@ -235,6 +236,8 @@ int attention_f32_launch(const onhip_attention_desc_t &d, const float *q, const 
     // k and v are read through 32-bit byte offsets from the head's first row
     if (d.tokens * d.k_strides[2] * 4 >= (1LL << 31) || d.tokens * d.v_strides[2] * 4 >= (1LL << 31))
         return set_error(ONHIP_ERR_ARG, "attention: tokens x token stride of k or v reaches 2 GiB");
+    static const bool off = getenv("ONHIP_NO_F3") != nullptr;   // tuning hook: fp32 matrix instructions only
+    if (!off && attention_f3_ok(d)) return attention_f3_launch(d, q, k, v, out, stream);
     if (d.head_dim == 64) return attention_launch_hd<64>(p, d.batch, stream);
     return attention_launch_hd<32>(p, d.batch, stream);
 }

@@ -61,9 +61,10 @@ struct SplitUnit {
         u0 = __uint_as_float(a << 16); u1 = __uint_as_float(a & 0xffff0000u);
         u2 = __uint_as_float(b << 16); u3 = __uint_as_float(b & 0xffff0000u);
     }
-    template <int Q> __device__ __forceinline__ void phase(float x0, float x1, float x2, float x3) {
+    template <int Q, bool SCALED = true> __device__ __forceinline__ void phase(float x0, float x1, float x2, float x3) {
         if constexpr (Q == 0) {
-            r0 = x0 * F3_SCALE; r1 = x1 * F3_SCALE; r2 = x2 * F3_SCALE; r3 = x3 * F3_SCALE;
+            constexpr float scale = SCALED ? F3_SCALE : 1.0f;
+            r0 = x0 * scale; r1 = x1 * scale; r2 = x2 * scale; r3 = x3 * scale;
             h0 = cvt_pk_bf16(r0, r1); h1 = cvt_pk_bf16(r2, r3);
             unpack(h0, h1);
         } else if constexpr (Q == 1) {

@@ -394,6 +394,9 @@ bool stem_f32_ok(const onhip_conv_desc_t &d, int OH, int OW);
 int stem_pack_launch(const onhip_conv_desc_t &d, const float *w, float *packed, hipStream_t stream);
 int stem_f32_launch(const onhip_conv_desc_t &d, int OH, int OW, const float *x, const float *w, int packed, const float *bias,
                     const Epilogue &ep, float *y, hipStream_t stream);
+// attention_f3.hip
+bool attention_f3_ok(const onhip_attention_desc_t &d);
+int attention_f3_launch(const onhip_attention_desc_t &d, const float *q, const float *k, const float *v, float *out, hipStream_t stream);
 // attention.hip
 int attention_f32_launch(const onhip_attention_desc_t &d, const float *q, const float *k, const float *v, float *out,
                          hipStream_t stream);
