@@ -575,6 +575,29 @@ void igemm_f3_kernel(const std::conditional_t<NORM, IgemmNormProblem, IgemmProbl
     issue_b(1, S1);
 #pragma unroll
     for (int z = 2; z >= 0; --z) load_a(op1, 1, z);
+    // One workgroup a compute unit and a long K: nothing but this workgroup's own loads, two K tiles ahead, covers the trip its part of A
+    // makes to the L2, and all workgroups of an XCD ask for the same K tile at the same time, so each of them is that trip again.  A touch of
+    // every cache line of A up front, shared out among the XCD's workgroups with the same rows, makes them one trip (rows 192 x 768, 196
+    // workgroups: 39.0 -> 34.7 us a launch; 64 x 384 and 96 x 576, 196 of 128 x 64: 16.4 -> 14.0 and 24.2 -> 20.3).  Not for a short K (one trip as
+    // well), not for several workgroups a unit (4099 x 1031 x 2053 106 -> 115), nor for more of A than leaves the L2 room (512 x 1024 43.6 -> 47.4).
+    constexpr int TOUCH = BM > 64 ? 2 : 0;   // (64 x 64 tiles would lose a wavefront a SIMD to the registers)
+    unsigned touch[TOUCH + 1];
+    if constexpr (TOUCH) {
+        constexpr int ROW = BM / 32 * 24;   // cache lines of a K tile
+        unsigned at[TOUCH];
+#pragma unroll
+        for (int i = 0; i < TOUCH; ++i) at[i] = OOB;
+        if (gridDim.x <= 256 && gridDim.y == 1 && !p.n_fast && k_tiles >= 24 && p.a_split_bytes <= (2 << 20)) {   // uniform
+            const int share = max(1, (int) div31(gridDim.x >> 3, p.div_tiles_m)), turn = (int) div31(blockIdx.x >> 3, p.div_tiles_m);
+#pragma unroll
+            for (int i = 0; i < TOUCH; ++i) {
+                const int l = (i * share + turn) * NT + tid, kt = l / ROW, r = l - kt * ROW;
+                if (kt < k_tiles) at[i] = (unsigned) (r / 24) * a_pitch + (unsigned) kt * 3072u + (unsigned) (r % 24) * 128u;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < TOUCH; ++i) touch[i] = __builtin_amdgcn_raw_buffer_load_b32(ra, at[i], (unsigned) (m0 / 32) * a_pitch, 0);
+    }
     float bias_row[(BM + NT - 1) / NT];   // the tile's rows of the bias, for LDS when the K loop is over; -0.0f changes nothing
 #pragma unroll
     for (int i = 0; i < (BM + NT - 1) / NT; ++i) {
@@ -627,6 +650,8 @@ void igemm_f3_kernel(const std::conditional_t<NORM, IgemmNormProblem, IgemmProbl
         body(op0, op1, kt, S1);
         body(op1, op0, kt + 1, S0);
     }
+#pragma unroll
+    for (int i = 0; i < TOUCH; ++i) asm volatile("" :: "v"(touch[i]));   // kept until here
 #pragma unroll
     for (int i = 0; i < (BM + NT - 1) / NT; ++i)
         if (tid + i * NT < BM) s_bias[tid + i * NT] = bias_row[i];
