@@ -271,12 +271,7 @@ static int rowb_launch_one(const IgemmLaunch &cfg, const IgemmParams &p_in, hipS
     }
     hipLaunchKernelGGL((rowb_f32_kernel<WM, WN>), dim3(grid_x, 1, cfg.batch), dim3(64 * WM * WN), 0, stream, p);
     ONHIP_CHECK_HIP(hipGetLastError());
-    if (p.dp_tiles > 0) {
-        const dim3 fgrid((p.N - p.part_begin + 63) / 64, (p.M + 3) / 4, 1);
-        hipLaunchKernelGGL((splitk_finish_kernel<false>), fgrid, dim3(64, 4), 0, stream, p, cfg.split, 1);
-        ONHIP_CHECK_HIP(hipGetLastError());
-    }
-    return ONHIP_OK;
+    return p.dp_tiles > 0 ? finish_launch<false>(cfg, p, stream) : ONHIP_OK;
 }
 
 // cfg.bm x cfg.bn names the workgroup tile: 64x128 (2 wavefronts), 128x128 (4, stacked along M), 64x256 (2 x 2),
