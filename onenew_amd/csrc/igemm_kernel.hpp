@@ -817,6 +817,40 @@ template <int DT> __device__ __forceinline__ float unpack_h16(unsigned w, int ha
     }
 }
 
+// Table activations whose results are stored in 16 bits: N values to N / 2 packed pairs of table entries, by act_fast<EPI_LUT>'s rules.  tab:
+// the 8192 entries in LDS, rounded to the type, with a zero in front of them, which is the entry of values below the table (floor(512 v + 4096),
+// and 512 v + 4096 rounded is 512 times v + 8 rounded).  Values of 8 and more are themselves, a NaN takes entry 0: rare, so the
+// wavefront asks once for all of them.  Six vector instructions a value; with the two ends compared and selected value by value, unpacked and packed
+// again they were thirteen and a half.
+typedef const volatile __attribute__((address_space(3))) unsigned short *lds_u16_t;
+template <int DT, int N>
+__device__ __forceinline__ void table_h16(const float (&v)[N], unsigned (&w)[N / 2], lds_u16_t tab) {
+    unsigned short l[N];
+    float top = v[0];
+#pragma unroll
+    for (int i = 1; i < N; ++i) top = __builtin_elementwise_maximum(top, v[i]);   // NaN if any is
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        int idx;
+        asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(idx) : "v"(__builtin_fmaf(v[i], 512.0f, 4096.0f)));
+        idx = idx < -1 ? -1 : idx > 8191 ? 8191 : idx;
+        l[i] = tab[idx];
+    }
+    __builtin_amdgcn_sched_barrier(0);   // all on their way before the first is used
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) w[i] = (unsigned) l[2 * i + 1] << 16 | l[2 * i];
+    if (__builtin_amdgcn_ballot_w64(!(top < 8.0f)) != 0ull) {   // uniform
+        const unsigned zero = tab[0];
+#pragma unroll
+        for (int i = 0; i < N / 2; ++i) {
+            const unsigned own = pack_h16<DT>(v[2 * i], v[2 * i + 1]);
+            const unsigned lo = v[2 * i] != v[2 * i] ? zero : v[2 * i] >= 8.0f ? own & 0xffffu : w[i] & 0xffffu;
+            const unsigned hi = v[2 * i + 1] != v[2 * i + 1] ? zero << 16 : v[2 * i + 1] >= 8.0f ? own & 0xffff0000u : w[i] & 0xffff0000u;
+            w[i] = lo | hi;
+        }
+    }
+}
+
 // 16-bit NHWC output (bf16 or fp16; element (pixel n, channel m) at (n * pitch + m) * 2 bytes, pitch = p.c_stride_n a
 // multiple of 8): bias and activation in fp32 on the accumulators, rounding to the 16-bit type, then the tile is
 // transposed through LDS so that a thread stores 8 consecutive channels of one pixel with a single 128-bit access.  A
@@ -853,7 +887,6 @@ __device__ __forceinline__ void write_tile_nhwc_h16(const IgemmParams &p, f32x16
     // Table activations: the 8192 fp32 entries rounded to the output type, 16 KiB of LDS behind the staging area (the
     // caller leaves them free).  The value stored is round(table[i]) either way; the gathers then hit LDS instead of
     // sending 64 addresses per instruction to memory.
-    typedef const __attribute__((address_space(3))) unsigned short *lds_u16_t;
     lds_u16_t tab = nullptr;
     if constexpr (EPI == EPI_LUT) {
         unsigned char *tl = stage + BN * PITCH;
@@ -864,9 +897,11 @@ __device__ __forceinline__ void write_tile_nhwc_h16(const IgemmParams &p, f32x16
 #pragma unroll
         for (int i = 0; i < 8192 / 4 / THREADS; ++i)
             reinterpret_cast<uint2 *>(tl)[tid + i * THREADS] = make_uint2(pack_h16<DT>(t[i].x, t[i].y), pack_h16<DT>(t[i].z, t[i].w));
+        if (tid == 0) reinterpret_cast<unsigned short *>(tl)[-1] = 0;   // in the padding behind the last staged row
         __syncthreads();
-        tab = (lds_u16_t) tl;
+        tab = (lds_u16_t) reinterpret_cast<unsigned short *>(tl);
     }
+    const bool edge = m0 + BM > p.M;   // uniform: only the last row tile has channels beyond M
 #pragma unroll
     for (int a = 0; a < TM; ++a)
 #pragma unroll
@@ -875,40 +910,34 @@ __device__ __forceinline__ void write_tile_nhwc_h16(const IgemmParams &p, f32x16
             const float4 bias = *reinterpret_cast<const float4 *>(rows + ml);
             const float bv[4] = {bias.x, bias.y, bias.z, bias.w};
             float y[TN][4];
+            unsigned w[TN * 2];
             if constexpr (EPI == EPI_LUT) {
-                // act_fast<EPI_LUT>'s rules; the table reads of the row group all in flight together
-                float v[TN][4];
-                unsigned short l[TN][4];
+                float v[TN * 4];
 #pragma unroll
                 for (int b = 0; b < TN; ++b)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        v[b][j] = __fadd_rn(acc[a][b][4 * q + j], bv[j]);
-                        int idx = (int) __fmul_rn(__fadd_rn(v[b][j], 8.0f), 512.0f);
-                        idx = idx < 0 ? 0 : idx > 8191 ? 8191 : idx;
-                        l[b][j] = tab[idx];
-                    }
-#pragma unroll
-                for (int b = 0; b < TN; ++b)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const float lv = unpack_h16<DT>((unsigned) l[b][j], 0);
-                        const float r = v[b][j] < -8.0f ? 0.0f : v[b][j] >= 8.0f ? v[b][j] : lv;
-                        y[b][j] = (m0 + ml + j < p.M) ? r : 0.0f;
-                    }
+                    for (int j = 0; j < 4; ++j) v[4 * b + j] = __fadd_rn(acc[a][b][4 * q + j], bv[j]);
+                table_h16<DT>(v, w, tab);
             } else {
 #pragma unroll
-                for (int b = 0; b < TN; ++b)
+                for (int b = 0; b < TN; ++b) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const float v = act_fast<EPI>(__fadd_rn(acc[a][b][4 * q + j], bv[j]), p.ep);
-                        y[b][j] = (m0 + ml + j < p.M) ? v : 0.0f;
-                    }
+                    for (int j = 0; j < 4; ++j) y[b][j] = act_fast<EPI>(__fadd_rn(acc[a][b][4 * q + j], bv[j]), p.ep);
+                    w[2 * b] = pack_h16<DT>(y[b][0], y[b][1]);
+                    w[2 * b + 1] = pack_h16<DT>(y[b][2], y[b][3]);
+                }
+            }
+            if (edge) {   // uniform
+#pragma unroll
+                for (int i = 0; i < TN * 2; ++i) {
+                    const int m = m0 + ml + i % 2 * 2;
+                    w[i] = (m < p.M ? w[i] & 0xffffu : 0u) | (m + 1 < p.M ? w[i] & 0xffff0000u : 0u);
+                }
             }
 #pragma unroll
             for (int b = 0; b < TN; ++b) {
                 const int nl = n_wave - n0 + b * 32 + li;
-                *reinterpret_cast<uint2 *>(stage + nl * PITCH + ml * 2) = make_uint2(pack_h16<DT>(y[b][0], y[b][1]), pack_h16<DT>(y[b][2], y[b][3]));
+                *reinterpret_cast<uint2 *>(stage + nl * PITCH + ml * 2) = make_uint2(w[2 * b], w[2 * b + 1]);
             }
         }
     __syncthreads();
