@@ -19,13 +19,13 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++20", "-fPIC", "-Wall", "-Wno-unused-function", "-Wno-c++20-extensions",
              "-ffp-contract=off",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
-KERNEL_SOURCES = ["depthwise.hip", "dw_s8.hip", "igemm_f32.hip", "igemm_f32_res.hip", "igemm_f32_pw.hip", "igemm_bf16.hip", "igemm_f16.hip", "igemm_i8.hip", "igemm_i8_res.hip", "igemm_f3.hip", "igemm_f3_conv.hip", "igemm_f3_pw.hip", "igemm_kw.hip", "igemm_rowb.hip", "igemm_dma.hip", "igemm_dma_bf16.hip", "igemm_dma_f16.hip", "igemm.hip", "direct.hip", "gemm_nt.hip", "h16.hip", "attention.hip", "attention_f3.hip", "attention_h16.hip", "stem.hip", "irblock.hip", "i8patch.hip", "i8small.hip", "calib.hip", "elementwise.hip", "vit_glue.hip", "api.hip",
+KERNEL_SOURCES = ["depthwise.hip", "dw_s8.hip", "igemm_f32.hip", "igemm_f32_res.hip", "igemm_f32_pw.hip", "igemm_bf16.hip", "igemm_f16.hip", "igemm_i8.hip", "igemm_i8_res.hip", "igemm_f3.hip", "igemm_f3_conv.hip", "igemm_f3_pw.hip", "igemm_kw.hip", "igemm_rowb.hip", "igemm_dma.hip", "igemm_dma_bf16.hip", "igemm_dma_f16.hip", "igemm.hip", "direct.hip", "gemm_nt.hip", "h16.hip", "h16_rows.hip", "attention.hip", "attention_f3.hip", "attention_h16.hip", "stem.hip", "irblock.hip", "i8patch.hip", "i8small.hip", "calib.hip", "elementwise.hip", "vit_glue.hip", "api.hip",
                   "plugin.hip"]
 # per-file compiler options.  The implicit-GEMM kernels keep their accumulators in ordinary vector registers (the
 # compiler's default puts them into the accumulation half of the register file and copies them out, one instruction per
 # register, for the store): the same kernels fit one more wavefront per SIMD (fp32 64 x 64: 75 registers instead of
 # 75 + 16, six instead of five; with a residual operand five instead of four; int8 128 x 128 three instead of two)
-EXTRA_FLAGS = {src: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for src in KERNEL_SOURCES if src.startswith("igemm") or src == "attention_f3.hip"}
+EXTRA_FLAGS = {src: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for src in KERNEL_SOURCES if src.startswith("igemm") or src in ("attention_f3.hip", "h16_rows.hip")}
 PLUGINS = {"Conv": "plugin_conv.cpp", "MatMul": "plugin_matmul.cpp", "Gemm": "plugin_gemm.cpp",
            "Add": "plugin_add.cpp", "Relu": "plugin_relu.cpp", "MaxPool": "plugin_maxpool.cpp",
            "GlobalAveragePool": "plugin_global_avgpool.cpp", "Gelu": "plugin_gelu.cpp",

@@ -329,7 +329,8 @@ static const int kNumSplits = 13;
 // tail > 1: the tiles left over after whole rounds of 256 are cut `tail` ways along K (launch_choice)
 // rowb == 1: the kernel that feeds B from global memory straight into the MFMAs (igemm_rowb.hip), tile bm x bn; rowb == 2: the
 // fp32 kernel on the 16-bit matrix cores (igemm_f3.hip), tile bm x bn; rowb == 3: the fp32 kernel whose wavefronts share K
-// (igemm_kw.hip), tile bm x bn, `split` wavefronts a workgroup
+// (igemm_kw.hip), tile bm x bn, `split` wavefronts a workgroup; 4 (onhip_last_launch_choice alone): a 16-bit product with its rows in registers
+// (h16_rows.hip)
 // fin != 0 (with split > 1 or tail > 1): the slices of a tile are added up by the last of them to arrive, inside the
 // launch, instead of by a finishing launch (igemm_kernel, `arrive`)
 // dma != 0: the kernel that loads its operand tiles straight into LDS (igemm_dma_kernel.hpp), tile bm x bn, never split;
@@ -1014,6 +1015,11 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
             if (c.tail > 1 && !candidate_ok(cfg, p, c)) c.tail = 0;   // no leftover to split on this shape
             return launch_choice(cfg, p, c, st);
         }
+    }
+    if (rows_h16_ok(cfg, p)) {   // measured choices as well: it is not one of the kernels that they choose among
+        static const int as[7] = {256, 64, 1, 0, 4, 0, 0};
+        std::copy(as, as + 7, tl_last_choice);
+        return rows_h16_launch(cfg, p, st);
     }
     if (!tune_mode()) return launch(by_model());
     std::vector<long long> key = {cfg.dtype, cfg.bl, cfg.batch, p.M, p.N, p.K, p.k_units, p.khkw, p.sh, p.sw,

@@ -1,0 +1,71 @@
+"""16-bit products with a short K whose rows stay in registers (h16_rows.hip): the bits of the direct-to-LDS kernel's smallest tile, at rows off its
+blocks of 256 and 32, columns off its panels of 64 and off the 32 channels a row is padded to, each depth it has, one panel a workgroup and several, with
+table activations, an addend, an addend and a Relu, without a bias; values beyond both ends of the table, infinities and NaN."""
+import pytest
+
+from onenew_amd import abi, hip
+from onenew_amd.abi import ConvDesc
+
+pytestmark = pytest.mark.gpu
+
+# rows, K, columns: more than a workgroup a compute unit; runs of several panels; of one
+SHAPES = [(66000, 64, 96), (65536, 256, 40), (30011, 192, 200), (12608, 192, 768), (25088, 128, 513), (4100, 256, 520), (40001, 50, 129), (8193, 120, 300)]
+
+
+def table(torch, gelu):
+    x = torch.arange(8192, dtype=torch.float64) / 512 - 8
+    return (x * 0.5 * (1 + torch.erf(x / 2 ** 0.5)) if gelu else x * torch.sigmoid(x)).float().cuda()
+
+
+@pytest.mark.parametrize("compute", [abi.COMPUTE_BF16, abi.COMPUTE_F16])
+@pytest.mark.parametrize("rows,k,cols", SHAPES)
+def test_linear(rows, k, cols, compute, monkeypatch):
+    import torch
+    hip.init(0)
+    print(f"{rows} rows, {k} -> {cols}, {compute}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(rows + cols)
+    x = torch.randn((rows, k), generator=g, device="cuda")
+    x[::701] *= 12.0   # beyond both ends of the table
+    x[5, 3], x[6, 0], x[7, 1] = float("inf"), float("-inf"), float("nan")
+    x = hip.h16_from_rows(x, compute)
+    w = hip.h16_pack_matmul_weights(torch.randn((k, cols), generator=g, device="cuda") / k ** 0.5, compute)
+    b = torch.randn(cols, generator=g, device="cuda") * 0.1
+    r = hip.h16_from_rows(torch.randn((rows, cols), generator=g, device="cuda"), compute)
+    for bias, gelu, addend in [(b, False, None), (None, False, None), (b, True, None), (b, False, r), (b, True, r)]:
+        args = dict(bias=bias, gelu_lut=table(torch, True) if gelu else None, residual=addend)
+        monkeypatch.delenv("ONHIP_TILE", raising=False)
+        y = hip.linear_h16(x, w, k, cols, compute, **args)
+        assert hip.last_launch_choice()[4] == 4
+        monkeypatch.setenv("ONHIP_TILE", "64x64x1x0x0x0x1")
+        ref = hip.linear_h16(x, w, k, cols, compute, **args)
+        assert hip.last_launch_choice()[4] == 0
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int16), ref.view(torch.int16)), (gelu, addend is not None)
+        if gelu and addend is None:   # the table as fp32 results have it, on its other code: one rounding apart
+            whole = hip.linear_h16(x, w, k, cols, compute, y_kind=hip.H16_OUT_F32_NHWC, **args)
+            assert torch.equal(y[:, :cols].view(torch.int16), whole.to(y.dtype).view(torch.int16)) and not y[:, cols:].view(torch.int16).any()
+
+
+@pytest.mark.parametrize("n,cin,hw,cout,act,relu", [(32, 64, 56, 256, abi.NOT_ACT, True), (12, 60, 31, 130, abi.SILU, False), (20, 256, 29, 100, abi.SILU, True),
+                                                    (16, 180, 23, 300, abi.NOT_ACT, True)])
+def test_convolution(n, cin, hw, cout, act, relu, monkeypatch):
+    import torch
+    hip.init(0)
+    print(f"{n} x {cin} x {hw}^2 -> {cout}, activation {act}", flush=True)
+    d = ConvDesc(n=n, cin=cin, h=hw, w=hw, cout=cout, kh=1, kw=1, stride_h=1, stride_w=1, pad_t=0, pad_l=0, pad_b=0, pad_r=0, group=1, has_bias=1, act_type=act,
+                 compute=abi.COMPUTE_BF16)
+    g = torch.Generator(device="cuda").manual_seed(cin + cout)
+    x = hip.h16_from_nchw(torch.randn((n, cin, hw, hw), generator=g, device="cuda"), d.compute)
+    w = hip.h16_pack_conv_weights(d, torch.randn((cout, cin, 1, 1), generator=g, device="cuda") * (3.0 / cin ** 0.5))
+    b = torch.randn(cout, generator=g, device="cuda")
+    r = hip.h16_from_nchw(torch.randn((n, cout, hw, hw), generator=g, device="cuda"), d.compute)
+    lut = table(torch, False) if act == abi.SILU else None
+    for addend in (None, r):
+        run = lambda: hip.conv2d_h16(d, x, w, b, lut, residual=addend, residual_relu=relu and addend is not None)  # noqa: E731
+        monkeypatch.delenv("ONHIP_TILE", raising=False)
+        y = run()
+        assert hip.last_launch_choice()[4] == 4
+        monkeypatch.setenv("ONHIP_TILE", "64x64x1x0x0x0x1")
+        ref = run()
+        torch.cuda.synchronize()
+        assert hip.last_launch_choice()[4] == 0 and torch.equal(y.view(torch.int16), ref.view(torch.int16))
