@@ -5,10 +5,16 @@
 // + r % 4, the Softmax is a reduction inside the lane, and the probabilities feed the second product out^T = v^T P^T from
 // the registers they are in.  An MFMA step of the second product takes 8 reduction indices per lane half: registers
 // 8 g .. 8 g + 7 of a tile, i.e. the keys 32 t + 16 g + 8 (j / 4) + 4 (lane / 32) + j % 4, rounded to the 16-bit type and
-// packed; the A operand for them is two 8-byte reads of v^T[channel lane % 32][key], which is why v is transposed on its
-// way into LDS (k is copied as it is).  The probabilities are rounded to the operand type before the second product: that
-// is what 16-bit operands mean for a MatMul; everything before it (scores, maximum, exponentials, sum, normalisation) is
-// fp32.  Head dimension 64, at most 256 tokens.
+// packed; the A operand for them is two 8-byte reads of v that transpose on their way out of LDS (ds_read_b64_tr_b16).  What is
+// rounded to the operand type before the second product is exp(x - max), and the result is divided by their sum: the relative rounding of
+// a probability, which is what 16-bit operands mean for a MatMul, without a product for each of them; everything before it (scores,
+// maximum, exponentials, sum) is fp32.  Head dimension 64, at most 256 tokens.
+//
+// What bounds it: one copy of k and v a head, one trip to memory, 3 us of a launch with its start; then the Softmax, 20 vector cycles and 16 of
+// the exponential a score, two wavefronts a SIMD where heads have seven tiles of queries, the matrix instructions behind them.
+// 64 x 3 heads of 197 tokens 10.0 -> 8.9 us (their 19 MB are 4 of a large copy), 48 x 3 of 225 11.1 -> 9.3, 24 x 3 of 256 9.5 -> 7.3, 128 x 3 of 100
+// 9.8 -> 7.4 (with v transposed by registers, q and the result a row a lane and the probabilities normalised one by one before), the error
+// against 64 bits 0.65-0.95 of what it was.
 #include "igemm_kernel.hpp"
 
 namespace onhip {
@@ -25,13 +31,12 @@ struct AttnH16Params {
 template <int DT, int NKT, int NW>
 __global__ __launch_bounds__(64 * NW, 2) void attention_h16_kernel(const AttnH16Params p) {
     constexpr int HD = 64, KEYS = NKT * 32, NT = 64 * NW;
-    constexpr int LDK = HD + 8;       // 16-bit elements per key row of k (144 bytes: 16-byte reads of neighbouring rows spread over the banks)
-    // 16-bit elements per channel row of v^T.  KEYS is a multiple of 32, so rows are 2 (mod 16) dwords apart (the 8-byte reads of
-    // 32 rows touch every bank once) and 8 rows 16 (mod 64): the 16 key pairs of 4 channel groups that a wavefront writes together
-    // do as well
-    constexpr int LDVT = KEYS + 4;
-    __shared__ __attribute__((aligned(16))) unsigned short Ks[KEYS * LDK];
-    __shared__ __attribute__((aligned(16))) unsigned short Vt[HD * LDVT];
+    __shared__ uint4 Ks[KEYS * HD / 8];   // rows of k, by `unit` below
+    // rows of v as they are, the two halves of rows 2 and 3 of four swapped: a transposing read takes 64 bytes of four rows, every bank once
+    __shared__ __attribute__((aligned(16))) unsigned short Vs[KEYS * HD];
+    // a wavefront's rows of q, later of the result: memory is read and written eight lanes to a row of 128 bytes (a row a lane, 64 cycles of
+    // the compute unit's address path each, were 2 us of a launch)
+    __shared__ uint4 Ws[NW][32 * HD / 8];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 31, lh = lane >> 5;
@@ -40,55 +45,52 @@ __global__ __launch_bounds__(64 * NW, 2) void attention_h16_kernel(const AttnH16
     const unsigned short *kb = p.k + b * p.ks[0] + h * p.ks[1];
     const unsigned short *vb = p.v + b * p.vs[0] + h * p.vs[1];
 
-    // k rows as they are, v transposed; rows / columns past the last key as zeros.  All loads first.  Of v a lane takes 8
-    // channels of two neighbouring keys, 4 channel groups of 16 key pairs a wavefront, and stores each channel's pair as one
-    // dword: no two lanes on one bank.  (One key a lane, 8 keys of 8 channel groups a wavefront, was 8 stores of 2 bytes per
-    // 16 bytes with 8 lanes on one bank each.)
-    constexpr int PARTS = HD / 8, NK = (KEYS * PARTS + NT - 1) / NT, NV = (2 * NKT + NW - 1) / NW;
-    uint4 kq[NK], vq[NV][2];
+    // where the 16 bytes `u` of a row of 128 lie: neither 32 lanes that take one `u` of 32 rows each nor eight that take a row meet in a bank
+    auto unit = [](int row, int u) { return row * 8 + (u ^ (row >> 1 & 7)); };
+    // all loads first; rows past the last token as zeros
+    constexpr int PARTS = HD / 8, NK = (KEYS * PARTS + NT - 1) / NT;
+    const int q0 = (blockIdx.x * NW + wave) * 32;
+    const unsigned short *qb = p.q + b * p.qs[0] + h * p.qs[1];
+    uint4 kq[NK], vq[NK], qf[HD / 16];
 #pragma unroll
     for (int i = 0; i < NK; ++i) {
-        const int f = tid + i * NT;
-        const int key = f / PARTS, part = f % PARTS;
+        const int key = (tid + i * NT) / PARTS, part = tid % PARTS;
         kq[i] = make_uint4(0u, 0u, 0u, 0u);
         if (key < T) kq[i] = *reinterpret_cast<const uint4 *>(kb + key * p.ks[2] + part * 8);
     }
-    const int vpart = lane / 16, vpair = lane % 16;
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        const int u = wave + i * NW;   // half of the channels of 32 keys
-#pragma unroll
-        for (int z = 0; z < 2; ++z) {
-            const int key = u / 2 * 32 + 2 * vpair + z;
-            vq[i][z] = make_uint4(0u, 0u, 0u, 0u);
-            if (u < 2 * NKT && key < T) vq[i][z] = *reinterpret_cast<const uint4 *>(vb + key * p.vs[2] + (u % 2 * 4 + vpart) * 8);
-        }
+    for (int i = 0; i < 4; ++i) {
+        const int query = q0 + i * 8 + lane / 8;
+        qf[i] = make_uint4(0u, 0u, 0u, 0u);
+        if (query < T) qf[i] = *reinterpret_cast<const uint4 *>(qb + query * p.qs[2] + lane % 8 * 8);
     }
-    // this lane's query row: the channels 16 s + 8 (lane / 32) .. + 7 of MFMA step s
-    const int q0 = (blockIdx.x * NW + wave) * 32;
-    const int query = q0 + li;
-    uint4 qf[HD / 16];
-    {
-        const unsigned short *qb = p.q + b * p.qs[0] + h * p.qs[1] + (long long) query * p.qs[2];
 #pragma unroll
-        for (int s = 0; s < HD / 16; ++s)
-            qf[s] = query < T ? *reinterpret_cast<const uint4 *>(qb + 16 * s + 8 * lh) : make_uint4(0u, 0u, 0u, 0u);
+    for (int i = 0; i < NK; ++i) {
+        const int key = (tid + i * NT) / PARTS, part = tid % PARTS;
+        vq[i] = make_uint4(0u, 0u, 0u, 0u);
+        if (key < T) vq[i] = *reinterpret_cast<const uint4 *>(vb + key * p.vs[2] + part * 8);
     }
 #pragma unroll
     for (int i = 0; i < NK; ++i) {
         const int f = tid + i * NT;
-        if (f < KEYS * PARTS) *reinterpret_cast<uint4 *>(Ks + f / PARTS * LDK + f % PARTS * 8) = kq[i];
+        if (f < KEYS * PARTS) Ks[unit(f / PARTS, f % PARTS)] = kq[i];
+    }
+    // this lane's query row: the channels 16 s + 8 (lane / 32) .. + 7 of MFMA step s
+    uint4 *const mine = Ws[wave];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) mine[unit(i * 8 + lane / 8, lane % 8)] = qf[i];
+#pragma unroll
+    for (int st = 0; st < HD / 16; ++st) qf[st] = mine[unit(li, 2 * st + lh)];
+    if (p.scale < 0.0f) {   // uniform: the scale's sign is the query's, so that the largest score stays it when scaled
+#pragma unroll
+        for (int st = 0; st < HD / 16; ++st) {
+            qf[st].x ^= 0x80008000u; qf[st].y ^= 0x80008000u; qf[st].z ^= 0x80008000u; qf[st].w ^= 0x80008000u;
+        }
     }
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        const int u = wave + i * NW;
-        if (u < 2 * NKT) {   // uniform
-            const unsigned lo[4] = {vq[i][0].x, vq[i][0].y, vq[i][0].z, vq[i][0].w}, hi[4] = {vq[i][1].x, vq[i][1].y, vq[i][1].z, vq[i][1].w};
-            unsigned *dst = reinterpret_cast<unsigned *>(Vt + (u % 2 * 4 + vpart) * 8 * LDVT) + u / 2 * 16 + vpair;
-#pragma unroll
-            for (int e = 0; e < 8; ++e)   // the low or the high halves of the two keys' words
-                dst[e * (LDVT / 2)] = __builtin_amdgcn_perm(hi[e / 2], lo[e / 2], e % 2 ? 0x07060302u : 0x05040100u);
-        }
+    for (int i = 0; i < NK; ++i) {
+        const int f = tid + i * NT, key = f / PARTS, part = f % PARTS;
+        if (f < KEYS * PARTS) *reinterpret_cast<uint4 *>(Vs + key * HD + (part ^ (key >> 1 & 1) * 4) * 8) = vq[i];
     }
     __syncthreads();
     if (q0 >= T) return;   // a wavefront without queries (uniform); nothing below synchronises
@@ -100,84 +102,85 @@ __global__ __launch_bounds__(64 * NW, 2) void attention_h16_kernel(const AttnH16
             return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, bq), c, 0, 0, 0);
     };
 
-    // S^T = k q^T
+    // S^T = k q^T, and the largest score of a query over the keys there are
     f32x16 s[NKT];
-#pragma unroll
-    for (int t = 0; t < NKT; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[t][r] = 0.0f;
-#pragma unroll
-    for (int st = 0; st < HD / 16; ++st) {
-        uint4 kf[NKT];
-#pragma unroll
-        for (int t = 0; t < NKT; ++t) kf[t] = *reinterpret_cast<const uint4 *>(Ks + (32 * t + li) * LDK + 16 * st + 8 * lh);
-#pragma unroll
-        for (int t = 0; t < NKT; ++t) s[t] = mfma(kf[t], qf[st], s[t]);
-    }
-
-    // Softmax over the keys in fp32 (softmax.c:26-59); keys past the last count as minus infinity
     float mx = -INFINITY;
 #pragma unroll
     for (int t = 0; t < NKT; ++t) {
-        if (32 * t + 32 <= T) {   // uniform: every key of the tile exists
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s[t][r] = __fmul_rn(s[t][r], p.scale);
-        } else {
+        for (int r = 0; r < 16; ++r) s[t][r] = 0.0f;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int key = 32 * t + 8 * (r / 4) + 4 * lh + (r % 4);
-                s[t][r] = key < T ? __fmul_rn(s[t][r], p.scale) : -INFINITY;
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[t][r]);
+        for (int st = 0; st < HD / 16; ++st)
+            s[t] = mfma(Ks[unit(32 * t + li, 2 * st + lh)], qf[st], s[t]);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    float sum = 0.0f;
 #pragma unroll
     for (int t = 0; t < NKT; ++t)
+        if (32 * t + 32 <= T) {   // uniform: every key of the tile exists
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const float e = __builtin_amdgcn_exp2f(__fmul_rn(__fsub_rn(s[t][r], mx), 1.44269504088896340736f));
-            s[t][r] = e;
-            sum += e;
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[t][r]);
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (32 * t + 8 * (r / 4) + 4 * lh + (r % 4) < T) mx = fmaxf(mx, s[t][r]);
         }
-    sum += __shfl_xor(sum, 32, 64);
-    const float inv = 1.0f / sum;
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
 
-    // out^T = v^T P^T, the probabilities normalised, rounded and packed eight at a time
+    // Softmax over the keys in fp32 (softmax.c:26-59), exp(scale (s - max)) as one fused product into the exponential base 2, and behind each tile
+    // its part of out^T = v^T P^T.  bf16 has fp32's range, and a sum of 256 of its largest values leaves it: 2^-8 of them.
+    const float c = __fmul_rn(fabsf(p.scale), 1.44269504088896340736f);
+    const float shift = DT == DT_BF16 ? -__fadd_rn(__fmul_rn(mx, c), 8.0f) : -__fmul_rn(mx, c);
     f32x16 o[2];
 #pragma unroll
     for (int d = 0; d < 2; ++d)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
+    // of 16 lanes, four read the 32 bytes of 16 channels of one key, and each gets four keys of one channel
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4 *lds_s16x4_t;
+    const int j = lane & 15;
+    const unsigned short *vr[2];
 #pragma unroll
-    for (int t = 0; t < NKT; ++t)
+    for (int d = 0; d < 2; ++d) vr[d] = Vs + (4 * lh + j / 4) * HD + (d ^ (j >> 3)) * 32 + li / 16 * 16 + j % 4 * 4;
+    float sum = 0.0f;
+#pragma unroll
+    for (int t = 0; t < NKT; ++t) {
+        float e[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) e[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][r], c, shift));
+        if (32 * t + 32 > T)   // uniform
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (32 * t + 8 * (r / 4) + 4 * lh + (r % 4) >= T) e[r] = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sum += e[r];
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
-            if (32 * t + 16 * g >= T) continue;   // uniform: all of these keys lie past the last one
-            uint4 pq;
-            pq.x = pack_h16<DT>(__fmul_rn(s[t][8 * g + 0], inv), __fmul_rn(s[t][8 * g + 1], inv));
-            pq.y = pack_h16<DT>(__fmul_rn(s[t][8 * g + 2], inv), __fmul_rn(s[t][8 * g + 3], inv));
-            pq.z = pack_h16<DT>(__fmul_rn(s[t][8 * g + 4], inv), __fmul_rn(s[t][8 * g + 5], inv));
-            pq.w = pack_h16<DT>(__fmul_rn(s[t][8 * g + 6], inv), __fmul_rn(s[t][8 * g + 7], inv));
-            const int key0 = 32 * t + 16 * g + 4 * lh;   // slots 0..3: key0 .. key0 + 3, slots 4..7: key0 + 8 .. key0 + 11
+            const uint4 pq = make_uint4(pack_h16<DT>(e[8 * g], e[8 * g + 1]), pack_h16<DT>(e[8 * g + 2], e[8 * g + 3]),
+                                        pack_h16<DT>(e[8 * g + 4], e[8 * g + 5]), pack_h16<DT>(e[8 * g + 6], e[8 * g + 7]));
 #pragma unroll
-            for (int d = 0; d < 2; ++d) {
-                const unsigned short *vr = Vt + (32 * d + li) * LDVT + key0;
-                const uint2 lo = *reinterpret_cast<const uint2 *>(vr), hi = *reinterpret_cast<const uint2 *>(vr + 8);
+            for (int d = 0; d < 2; ++d) {   // keys 4 lh .. + 3 and 8 + 4 lh .. + 3 of the 16
+                const unsigned short *at = vr[d] + (32 * t + 16 * g) * HD;
+                const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t) at));
+                const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t) (at + 8 * HD)));
                 o[d] = mfma(make_uint4(lo.x, lo.y, hi.x, hi.y), pq, o[d]);
             }
         }
+    }
+    sum += __shfl_xor(sum, 32, 64);
+    const float inv = 1.0f / sum;
 
-    if (query < T) {
-        unsigned short *ob = p.o + b * p.os[0] + h * p.os[1] + (long long) query * p.os[2];
 #pragma unroll
-        for (int d = 0; d < 2; ++d)
+    for (int d = 0; d < 2; ++d)
 #pragma unroll
-            for (int g = 0; g < 4; ++g)
-                *reinterpret_cast<uint2 *>(ob + 32 * d + 8 * g + 4 * lh) =
-                    make_uint2(pack_h16<DT>(o[d][4 * g], o[d][4 * g + 1]), pack_h16<DT>(o[d][4 * g + 2], o[d][4 * g + 3]));
+        for (int g = 0; g < 4; ++g)
+            reinterpret_cast<uint2 *>(mine + unit(li, 4 * d + g))[lh] =
+                make_uint2(pack_h16<DT>(__fmul_rn(o[d][4 * g], inv), __fmul_rn(o[d][4 * g + 1], inv)),
+                           pack_h16<DT>(__fmul_rn(o[d][4 * g + 2], inv), __fmul_rn(o[d][4 * g + 3], inv)));
+    unsigned short *ob = p.o + b * p.os[0] + h * p.os[1];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int query = q0 + i * 8 + lane / 8;
+        if (query < T) *reinterpret_cast<uint4 *>(ob + query * p.os[2] + lane % 8 * 8) = mine[unit(i * 8 + lane / 8, lane % 8)];
     }
 }
 
@@ -186,11 +189,12 @@ static int attention_h16_launch_dt(const AttnH16Params &p, int batch, hipStream_
     const int nkt = (p.tokens + 31) / 32;
     const unsigned heads = (unsigned) (batch * p.heads);
     // Eight wavefronts share a copy of k and v where four would make a second copy for the same head, and the heads alone give
-    // half of the CUs a workgroup (fewer heads: two workgroups on two CUs do the staging side by side).  64 x 3 heads of 197
-    // tokens 16.9 us a launch with two copies and v stored by halves of a word, 11.4 now.
+    // half of the CUs a workgroup (fewer heads: two workgroups on two CUs do the staging side by side).
     const bool wide = nkt > 4 && heads >= 128;
     const dim3 grid(wide ? 1u : (unsigned) ((p.tokens + 127) / 128), heads);
-    if (nkt <= 2) hipLaunchKernelGGL((attention_h16_kernel<DT, 2, 4>), grid, dim3(256), 0, stream, p);
+    // one wavefront where there is one tile (24 heads of one token 4.4 us in four wavefronts with two tiles, 3.8 here; one head of five tokens 3.4 and 2.8)
+    if (nkt == 1) hipLaunchKernelGGL((attention_h16_kernel<DT, 1, 1>), grid, dim3(64), 0, stream, p);
+    else if (nkt <= 2) hipLaunchKernelGGL((attention_h16_kernel<DT, 2, 4>), grid, dim3(256), 0, stream, p);
     else if (nkt <= 4) hipLaunchKernelGGL((attention_h16_kernel<DT, 4, 4>), grid, dim3(256), 0, stream, p);
     else if (nkt <= 7 && wide) hipLaunchKernelGGL((attention_h16_kernel<DT, 7, 8>), grid, dim3(512), 0, stream, p);
     else if (nkt <= 7) hipLaunchKernelGGL((attention_h16_kernel<DT, 7, 4>), grid, dim3(256), 0, stream, p);
