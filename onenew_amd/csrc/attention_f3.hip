@@ -15,8 +15,8 @@
 // the next k and v behind the former, the exponentials of tile t + 1 and the loads behind the latter; one barrier.  It is a loop, not unrolled
 // over the tiles with all scores in registers, whose 40 KB of code run once and are not there in time.
 // What bounds it: two wavefronts a SIMD, whose 21500 cycles of matrix instructions (196 keys) take 29000 because the barrier keeps them
-// in step, and 10000 before the first of them: loads, the split of the queries and the first tile.  64 x 3 heads of 196 tokens 23.5 us, on fp32
-// matrix instructions (attention.hip) 30.2.  Error against 64 bits (relative, 2-norm; normal operands, 5 to 256 tokens) 0.8e-7 ... 6.9e-7, there 1.2e-7 ... 9.3e-7.
+// in step, and some 8000 before the first of them: loads, the split of the queries and the first tile.  64 x 3 heads of 196 tokens 22.0 us (23.5
+// with q and the result a row a lane), on fp32 matrix instructions (attention.hip) 30.2.  Error against 64 bits (relative, 2-norm; normal operands, 5 to 256 tokens) 0.8e-7 ... 6.9e-7, there 1.2e-7 ... 9.3e-7.
 //
 // Results that are not finite (an operand that is not, or of 2^104 and more, sums of 2^80 and more) are made again from the tensors in
 // memory with fp32 matrix instructions, as in igemm_f3_kernel.hpp: a score that is not finite makes its query's results NaN.
@@ -38,6 +38,9 @@ __global__ __launch_bounds__(64 * NW, 2) void attention_f3_kernel(const AttnF3Pa
     constexpr int NT = 64 * NW, HD = 64, STEPS = HD / 16, UNITS = 8 / NW;
     constexpr int PART = 32 * HD / 8, TILE = 3 * PART;   // 16-byte slots of one part of a tile of k or v, and of a tile
     __shared__ uint4 lds[4 * TILE];                      // two tiles of k, two of v
+    // a wavefront's rows of q, later of the result: memory is read and written sixteen lanes to a row of 256 bytes (a row a lane, 64 cycles of
+    // the compute unit's address path each, were 2 us of a launch)
+    __shared__ uint4 rows[NW][32 * HD / 4];
 
     // k: [part][key][8 slots of 8 channels], slots exchanged by the row so that 16 rows' reads of one slot cover the banks
     auto k_slot = [](int key, int u) { return key * 8 + (u ^ (key >> 1 & 7)); };
@@ -118,9 +121,14 @@ __global__ __launch_bounds__(64 * NW, 2) void attention_f3_kernel(const AttnF3Pa
     const int q0 = (qblock * NW + wave) * 32, query = q0 + li;
     const bool active = q0 < T;   // uniform: a wavefront without queries only helps with the operands
     const float *qb = p.q + b * p.qs[0] + h * p.qs[1] + (long long) (query < T ? query : T - 1) * p.qs[2];   // rows past the last: unused
-    float4 qf[2 * STEPS];
+    uint4 *const mine = rows[wave];
+    auto row_slot = [](int row, int u) { return row * 16 + (u ^ (row & 15)); };   // 16 bytes `u` of a row
+    uint4 qf[2 * STEPS];
 #pragma unroll
-    for (int i = 0; i < 2 * STEPS; ++i) qf[i] = *reinterpret_cast<const float4 *>(qb + i / 2 * 16 + 8 * lh + i % 2 * 4);
+    for (int i = 0; i < 2 * STEPS; ++i) {
+        const int row = q0 + 4 * i + lane / 16;
+        qf[i] = *reinterpret_cast<const uint4 *>(p.q + b * p.qs[0] + h * p.qs[1] + (long long) (row < T ? row : T - 1) * p.qs[2] + lane % 16 * 4);
+    }
     __builtin_amdgcn_sched_barrier(0);
     load_k(1, ODD);
     load_v(0, EVEN);
@@ -129,13 +137,18 @@ __global__ __launch_bounds__(64 * NW, 2) void attention_f3_kernel(const AttnF3Pa
     stage_all(stage_k, EVEN);
     load_k(2, EVEN);
     __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 2 * STEPS; ++i) mine[row_slot(4 * i + lane / 16, lane % 16)] = qf[i];
+#pragma unroll
+    for (int i = 0; i < 2 * STEPS; ++i) qf[i] = mine[row_slot(li, i / 2 * 4 + 2 * lh + i % 2)];
     uint4 qp[STEPS][3];
 #pragma unroll
     for (int s = 0; s < STEPS; ++s) {
         SplitUnit u, w;
+        const float4 lo = __builtin_bit_cast(float4, qf[2 * s]), hi = __builtin_bit_cast(float4, qf[2 * s + 1]);
         static_for<4>([&](auto ph) __attribute__((always_inline)) {
-            u.phase<decltype(ph)::value>(qf[2 * s].x, qf[2 * s].y, qf[2 * s].z, qf[2 * s].w);
-            w.phase<decltype(ph)::value>(qf[2 * s + 1].x, qf[2 * s + 1].y, qf[2 * s + 1].z, qf[2 * s + 1].w);
+            u.phase<decltype(ph)::value>(lo.x, lo.y, lo.z, lo.w);
+            w.phase<decltype(ph)::value>(hi.x, hi.y, hi.z, hi.w);
         });
         qp[s][0] = make_uint4(u.h0, u.h1, w.h0, w.h1);
         qp[s][1] = make_uint4(u.m0, u.m1, w.m0, w.m1);
@@ -361,13 +374,17 @@ __global__ __launch_bounds__(64 * NW, 2) void attention_f3_kernel(const AttnF3Pa
 #pragma unroll
             for (int r = 0; r < 16; ++r) o[d][r] = o[d][r] * 0.0f != 0.0f ? again[d][r] : o[d][r];
     }
-    if (query < T) {
-        float *ob = p.o + b * p.os[0] + h * p.os[1] + (long long) query * p.os[2] + 32 * lh;
 #pragma unroll
-        for (int d = 0; d < 2; ++d)
+    for (int d = 0; d < 2; ++d)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                *reinterpret_cast<float4 *>(ob + 16 * d + 4 * i) = make_float4(o[d][4 * i], o[d][4 * i + 1], o[d][4 * i + 2], o[d][4 * i + 3]);
+        for (int i = 0; i < 4; ++i)
+            mine[row_slot(li, 8 * lh + 4 * d + i)] = make_uint4(__float_as_uint(o[d][4 * i]), __float_as_uint(o[d][4 * i + 1]),
+                                                                __float_as_uint(o[d][4 * i + 2]), __float_as_uint(o[d][4 * i + 3]));
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int row = q0 + 4 * i + lane / 16;
+        if (row < T)
+            *reinterpret_cast<uint4 *>(p.o + b * p.os[0] + h * p.os[1] + (long long) row * p.os[2] + lane % 16 * 4) = mine[row_slot(4 * i + lane / 16, lane % 16)];
     }
 }
 
@@ -381,8 +398,8 @@ static int attention_f3_launch_one(AttnF3Params &p, int batch, hipStream_t strea
 
 // Head dimension 64; a scale for which neither it nor its product with the sums' unscaling leaves the normal numbers; and more 64-query
 // workgroups of attention.hip than compute units.  Up to one each, that kernel's 16 queries a wavefront reach four times the SIMDs: 16 x 3
-// heads of 129 tokens 9.9 us there and 12.7 here, 3 heads of 196 11.7 and 14.5; 48 x 3 of 100 12.3 and 11.0, 64 x 3 of 196 30.2 and 23.5,
-// 48 x 3 of 225 36.2 and 24.9.
+// heads of 129 tokens 9.9 us there and 12.7 here, 3 heads of 196 11.7 and 14.5; 48 x 3 of 100 12.3 and 10.5, 64 x 3 of 196 30.2 and 22.0,
+// 48 x 3 of 225 36.2 and 22.9.
 bool attention_f3_ok(const onhip_attention_desc_t &d) {
     return d.head_dim == 64 && d.scale >= 0x1p-60f && d.scale <= 0x1p60f && (long long) d.batch * d.heads * ((d.tokens + 63) / 64) > 256;
 }
@@ -396,8 +413,8 @@ int attention_f3_launch(const onhip_attention_desc_t &d, const float *q, const f
     p.heads = d.heads;
     p.tokens = d.tokens;
     p.scale = d.scale;
-    // Eight wavefronts share the tiles where the heads alone give half of the compute units a workgroup (64 x 3 heads of 196 tokens 23.5 us, with
-    // four 25.3); fewer heads take four, for twice the workgroups (24 x 3 of 256 tokens 19.0 and 22.6).
+    // Eight wavefronts share the tiles where the heads alone give half of the compute units a workgroup (64 x 3 heads of 196 tokens 23.5 us before the
+    // rows went through LDS, with four 25.3); fewer heads take four, for twice the workgroups (24 x 3 of 256 tokens 19.0 and 22.6).
     const bool wide = d.tokens > 128 && d.batch * d.heads >= 128;
     return wide ? attention_f3_launch_one<8>(p, d.batch, stream) : attention_f3_launch_one<4>(p, d.batch, stream);
 }
