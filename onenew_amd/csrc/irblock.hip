@@ -17,8 +17,12 @@
 //   * depthwise and projection as in dwproj.hip: taps added in ascending (i, j) order to a zero sum, multiply and add
 //     rounded separately, bias last (conv.c:757-899), so the depthwise stage is bit-identical to the operator on the same
 //     input; the projection accumulates in v_mfma_f32_32x32x2_f32 with its weights k-major in registers;
-//   * per chunk: [projection of the previous chunk, expansion of this one] -> barrier -> depthwise -> barrier.  Two
-//     workgroups share a compute unit, one in its MFMA phase while the other does depthwise arithmetic.
+//   * per chunk: expansion of the next one (into a second patch where LDS has room for it), depthwise and projection of this one, barrier.  Two
+//     workgroups of eight wavefronts share a compute unit (with four each, waiting for each other and for weights was half of the time: MobileNetV2
+//     batch 64, its six blocks 104, 92, 76, 40, 39 and 55 us; eight with 16-byte weight loads 83, 87, 52, 35, 34, and 48 with four).
+// What bounds it: the vector instructions' issue.  fp32 matrix instructions take it as long as they run (measured: one of 32 x 32 is 65 cycles, and n vector
+// instructions behind it, of any wavefront, make 65 + 4 n), and 75 thousand cycles of them and 85 thousand of the rest are most of the 183
+// thousand that 24 -> 144 -> 24 channels on 56 x 56 take a SIMD.
 // The expansion sums in another order than the library's separate 1x1 kernel (k in steps of 4 instead of 2), so the block
 // equals the chain of three operators within fp32 summation error, not bit for bit.
 #include <stdlib.h>
@@ -32,8 +36,8 @@ namespace onhip {
 
 constexpr int IR_BN = 128;        // output pixels of a band, at most
 constexpr int IR_KC = 16;         // expanded channels per chunk
-constexpr int IR_XSLOTS = 12;
-constexpr int IR_TPW = 9;         // pixel tiles of the expansion per wavefront, at most     // 16-byte input loads per thread, at most
+constexpr int IR_LOADS = 12 * 256; // 16-byte input loads of a workgroup, at most
+constexpr int IR_TILES = 36;      // pixel tiles of the expansion, at most
 constexpr int IR_LDS_HALF = 80 * 1024;   // bytes of LDS a workgroup may take: two workgroups per compute unit
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -42,11 +46,11 @@ typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
 struct IrParams {
     const float *x;        // [n][cin][h][w]
-    const float *exp_w;    // [ce / 16][cin / 4][64]: A fragments of the expansion
+    const float *exp_w;    // [ce / 16][steps of k, up to four together][64][those steps]: A fragments of the expansion
     const float *exp_b;    // [ce]
     const float *dw_w;     // [ce][9]
     const float *dw_b;     // [ce]
-    const float *pw_t;     // [ce][cop]: projection weights k-major, output channels padded to cop with zeros
+    const float *pw_t;     // [ce / 4][cop][4]: projection weights, output channels padded to cop with zeros
     const float *pw_b;     // [co] or nullptr
     const float *res;      // [n][co][oh][ow] or nullptr
     float *y;              // [n][co][oh][ow]
@@ -57,7 +61,7 @@ struct IrParams {
     int tiles;             // ceil(P / 16)
     int vec;               // floats per load of the block input: 4 (rows a multiple of 4 floats) or 2
     int groups;            // loads per channel: P / vec
-    int slots;             // loads per thread: ceil(cin * groups / 256)
+    int slots;             // loads per thread: ceil(cin * groups / threads)
     unsigned x_bytes;
     int xs_floats, patch_floats;   // LDS: Xs, then one or two patches
     Div31 div_ow, div_w, div_groups;
@@ -72,18 +76,23 @@ __device__ __forceinline__ float ir_act(float v, const Epilogue &e) {
     else return apply_act(v, e);
 }
 
+// wavefronts of a workgroup: eight (two workgroups make four a SIMD), four where 64 output channels' sums would not leave them registers
+constexpr int ir_waves(int mt) { return mt == 1 ? 8 : 4; }
+
 extern __shared__ __attribute__((aligned(16))) float ir_lds[];
 
 // NBUF = 2: two patches, the next chunk's expansion overlaps this chunk's depthwise stage (one barrier per chunk)
 template <int EPI, int KS, int MT, int NBUF>
-__global__ __launch_bounds__(256, 2) void irblock_f32_kernel(const IrParams p) {
+__global__ __launch_bounds__(64 * ir_waves(MT), ir_waves(MT) / 2) void irblock_f32_kernel(const IrParams p) {
+    constexpr int NW = ir_waves(MT), NT = 64 * NW, PARTS = NW / 2, CH = IR_KC / PARTS;   // parts of a chunk, channels of a part
+    constexpr int XSLOTS = IR_LOADS / NT, TPW = (IR_TILES + NW - 1) / NW;                // input loads of a thread, tiles of a wavefront, at most
     float *const Xs = ir_lds;
     float *const patch0 = ir_lds + p.xs_floats;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 31, lh = lane >> 5;
     const int l16 = lane & 15, lq = lane >> 4;
-    const int pxh = wave & 1, kh = wave >> 1;   // which 64 pixels of the band, which 8 channels of a chunk
+    const int pxh = wave & 1, kh = wave >> 1;   // which 64 pixels of the band, which part of a chunk's channels
     const int pitch = p.w + 2, plane = p.in_rows * pitch;
     const int OHW = p.oh * p.ow;
     const int img = blockIdx.x / p.bands, band = blockIdx.x - img * p.bands;
@@ -92,19 +101,52 @@ __global__ __launch_bounds__(256, 2) void irblock_f32_kernel(const IrParams p) {
     const int chunks = p.ce / IR_KC;
 
     // the whole patch to zero once: padding columns and the rows outside the image stay that way
-    for (int f = tid; f < NBUF * p.patch_floats / 4; f += 256) reinterpret_cast<float4 *>(patch0)[f] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int f = tid; f < NBUF * p.patch_floats / 4; f += NT) reinterpret_cast<float4 *>(patch0)[f] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+
+    const rsrc_t rew = make_rsrc(p.exp_w, (unsigned) (p.ce * p.cin * 4));
+    const rsrc_t reb = make_rsrc(p.exp_b, (unsigned) (p.ce * 4));
+    const rsrc_t rpw = make_rsrc(p.pw_t, (unsigned) (p.ce * p.cop * 4));
+    float aexp[KS];       // expansion weights of the chunk about to be expanded
+    float eb[4];          // and its biases for this lane's four rows
+    float pa[CH][MT];     // projection weights of this wavefront's channels of the chunk about to be projected
+    // 16 bytes a lane: all wavefronts read them, a column a lane they kept the address path busy for longer than the matrix cores
+    auto load_exp = [&](int chunk) __attribute__((always_inline)) {
+        const unsigned soff = (unsigned) (chunk * KS * 64) * 4u;
+#pragma unroll
+        for (int s = 0; s + 4 <= KS; s += 4) {
+            const uint4 t = buf_load_b128(rew, (unsigned) lane * 16u + (unsigned) s * 256u, soff);
+            aexp[s] = __uint_as_float(t.x); aexp[s + 1] = __uint_as_float(t.y); aexp[s + 2] = __uint_as_float(t.z); aexp[s + 3] = __uint_as_float(t.w);
+        }
+        if constexpr (KS % 4 == 2) {
+            const u32x2 t = __builtin_amdgcn_raw_buffer_load_b64(rew, (unsigned) lane * 8u + (unsigned) (KS - 2) * 256u, soff, 0);
+            aexp[KS - 2] = __uint_as_float(t.x); aexp[KS - 1] = __uint_as_float(t.y);
+        }
+        const uint4 t = buf_load_b128(reb, (unsigned) lq * 16u, (unsigned) (chunk * IR_KC) * 4u);
+        eb[0] = __uint_as_float(t.x); eb[1] = __uint_as_float(t.y); eb[2] = __uint_as_float(t.z); eb[3] = __uint_as_float(t.w);
+    };
+    auto load_proj = [&](int chunk) __attribute__((always_inline)) {
+#pragma unroll
+        for (int g = 0; g < CH / 4; ++g)
+#pragma unroll
+            for (int a = 0; a < MT; ++a) {
+                const uint4 t = buf_load_b128(rpw, (unsigned) (a * 32 + li) * 16u, (unsigned) ((chunk * (IR_KC / 4) + kh * (CH / 4) + g) * p.cop) * 16u);
+                pa[4 * g][a] = __uint_as_float(t.x); pa[4 * g + 1][a] = __uint_as_float(t.y);
+                pa[4 * g + 2][a] = __uint_as_float(t.z); pa[4 * g + 3][a] = __uint_as_float(t.w);
+            }
+    };
+    load_exp(0);
 
     // block input: channel c, floats [0, P) of the rows ih_first .. (contiguous in memory), rows outside the image zero
     {
         const rsrc_t rx = make_rsrc(p.x, p.x_bytes);
-        uint4 xr[IR_XSLOTS];
-        int l_off[IR_XSLOTS];
+        uint4 xr[XSLOTS];
+        int l_off[XSLOTS];
 #pragma unroll
-        for (int i = 0; i < IR_XSLOTS; ++i) {
+        for (int i = 0; i < XSLOTS; ++i) {
             xr[i] = make_uint4(0u, 0u, 0u, 0u);
             l_off[i] = -1;
             if (i >= p.slots) continue;   // uniform
-            const int f = tid + i * 256;
+            const int f = tid + i * NT;
             const bool live = f < p.cin * p.groups;
             const int ff = live ? f : 0;
             const int c = (int) div31((unsigned) ff, p.div_groups), g = ff - c * p.groups;
@@ -122,7 +164,7 @@ __global__ __launch_bounds__(256, 2) void irblock_f32_kernel(const IrParams p) {
             l_off[i] = live ? c * p.xs_pitch + p.vec * g : -1;
         }
 #pragma unroll
-        for (int i = 0; i < IR_XSLOTS; ++i)
+        for (int i = 0; i < XSLOTS; ++i)
             if (l_off[i] >= 0) {
                 if (p.vec == 4) *reinterpret_cast<uint4 *>(Xs + l_off[i]) = xr[i];
                 else *reinterpret_cast<uint2 *>(Xs + l_off[i]) = make_uint2(xr[i].x, xr[i].y);
@@ -140,34 +182,14 @@ __global__ __launch_bounds__(256, 2) void irblock_f32_kernel(const IrParams p) {
         win = r * p.stride * pitch + c * p.stride;
     }
 
-    const rsrc_t rew = make_rsrc(p.exp_w, (unsigned) (p.ce * p.cin * 4));
-    const rsrc_t reb = make_rsrc(p.exp_b, (unsigned) (p.ce * 4));
-    const rsrc_t rpw = make_rsrc(p.pw_t, (unsigned) (p.ce * p.cop * 4));
-    float aexp[KS];       // expansion weights of the chunk about to be expanded
-    float eb[4];          // and its biases for this lane's four rows
-    float pa[8][MT];      // projection weights of this wavefront's 8 channels of the chunk about to be projected
-    auto load_exp = [&](int chunk) __attribute__((always_inline)) {
-        const unsigned soff = (unsigned) (chunk * KS * 64) * 4u;
-#pragma unroll
-        for (int s = 0; s < KS; ++s) aexp[s] = buf_load_f32(rew, (unsigned) lane * 4u + (unsigned) s * 256u, soff);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) eb[r] = buf_load_f32(reb, (unsigned) (4 * lq + r) * 4u, (unsigned) (chunk * IR_KC) * 4u);
-    };
-    auto load_proj = [&](int chunk) __attribute__((always_inline)) {
-        const unsigned soff = (unsigned) ((chunk * IR_KC + kh * 8) * p.cop) * 4u;
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-#pragma unroll
-            for (int a = 0; a < MT; ++a) pa[c][a] = buf_load_f32(rpw, (unsigned) (c * p.cop + a * 32 + li) * 4u, soff);
-    };
-    // chunk's expansion into the patch: wavefront w takes the pixel tiles w, w + 4, ..., two at a time (two independent
+    // chunk's expansion into the patch: wavefront w takes the pixel tiles w, w + NW, ..., two at a time (two independent
     // chains of MFMAs).  Where a lane's four values of tile j (one pixel, the four channels 4 (lane / 16) .. + 3, which are
     // one channel group of the patch) go is the same for every chunk: eo[j], in floats, or -1 for a pixel past the band's
     // input or in a row outside the image.
-    int eo[IR_TPW];
+    int eo[TPW];
 #pragma unroll
-    for (int j = 0; j < IR_TPW; ++j) {
-        const int px = 16 * (wave + 4 * j) + l16;
+    for (int j = 0; j < TPW; ++j) {
+        const int px = 16 * (wave + NW * j) + l16;
         const int ir = (int) div31((unsigned) px, p.div_w), col = px - ir * p.w;
         const bool ok = px < p.P && (unsigned) (ih_first + ir) < (unsigned) p.h;
         eo[j] = ok ? ((lq * p.in_rows + ir) * pitch + 1 + col) * 4 : -1;
@@ -179,7 +201,7 @@ __global__ __launch_bounds__(256, 2) void irblock_f32_kernel(const IrParams p) {
 #pragma unroll
         for (int u = 0; u < NT; ++u) {
             e[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            const float *xb = Xs + lq * p.xs_pitch + 16 * (wave + 4 * (J0 + u)) + l16;
+            const float *xb = Xs + lq * p.xs_pitch + 16 * (wave + NW * (J0 + u)) + l16;
 #pragma unroll
             for (int s = 0; s < KS; ++s) xv[u][s] = xb[4 * s * p.xs_pitch];
         }
@@ -201,8 +223,8 @@ __global__ __launch_bounds__(256, 2) void irblock_f32_kernel(const IrParams p) {
     };
     auto expand_from = [&](float *patch, auto j0) __attribute__((always_inline)) {
         constexpr int J0 = decltype(j0)::value;
-        if (wave + 4 * J0 < p.tiles) {   // uniform
-            if (J0 + 1 < IR_TPW && wave + 4 * (J0 + 1) < p.tiles) expand_tiles(patch, j0, std::integral_constant<int, (J0 + 1 < IR_TPW ? 2 : 1)>());
+        if (wave + NW * J0 < p.tiles) {   // uniform
+            if (J0 + 1 < TPW && wave + NW * (J0 + 1) < p.tiles) expand_tiles(patch, j0, std::integral_constant<int, (J0 + 1 < TPW ? 2 : 1)>());
             else expand_tiles(patch, j0, std::integral_constant<int, 1>());
         }
     };
@@ -210,8 +232,10 @@ __global__ __launch_bounds__(256, 2) void irblock_f32_kernel(const IrParams p) {
         expand_from(patch, std::integral_constant<int, 0>());
         expand_from(patch, std::integral_constant<int, 2>());
         expand_from(patch, std::integral_constant<int, 4>());
-        expand_from(patch, std::integral_constant<int, 6>());
-        expand_from(patch, std::integral_constant<int, 8>());
+        if constexpr (TPW > 6) {
+            expand_from(patch, std::integral_constant<int, 6>());
+            expand_from(patch, std::integral_constant<int, 8>());
+        }
     };
 
     // v_mfma_f32_32x32x1_2b_f32: two 32x32 blocks (pixels 0..31 and 32..63 of the wavefront's 64), one reduction index per
@@ -223,15 +247,15 @@ __global__ __launch_bounds__(256, 2) void irblock_f32_kernel(const IrParams p) {
     for (int a = 0; a < MT; ++a)
 #pragma unroll
         for (int r = 0; r < 32; ++r) acc[a][r] = 0.0f;
-    // depthwise values of this wavefront's 8 channels for the lane's pixel, each straight into the projection's MFMAs
+    // depthwise values of this wavefront's channels for the lane's pixel, each straight into the projection's MFMAs
     auto depthwise_project = [&](int chunk, const float *patch) __attribute__((always_inline)) {
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
+        for (int h = 0; h < CH / 4; ++h) {
             // one channel group (four channels side by side in the patch): nine 16-byte reads give the lane its window in
             // all four
             float wd[4][9], bd[4];
             float4 tv[9];
-            const int g = kh * 2 + half;
+            const int g = kh * (CH / 4) + h;
 #pragma unroll
             for (int cc = 0; cc < 4; ++cc) {
                 const int c = chunk * IR_KC + g * 4 + cc;   // uniform: scalar loads
@@ -256,16 +280,15 @@ __global__ __launch_bounds__(256, 2) void irblock_f32_kernel(const IrParams p) {
                 float v = ir_act<EPI>(__fadd_rn(sum, bd[cc]), p.dw_ep);
                 v = q_ok ? v : 0.0f;
 #pragma unroll
-                for (int a = 0; a < MT; ++a) acc[a] = __builtin_amdgcn_mfma_f32_32x32x1f32(pa[half * 4 + cc][a], v, acc[a], 0, 0, 0);
+                for (int a = 0; a < MT; ++a) acc[a] = __builtin_amdgcn_mfma_f32_32x32x1f32(pa[h * 4 + cc][a], v, acc[a], 0, 0, 0);
             }
         }
     };
 
-    load_exp(0);
+    load_proj(0);
     __syncthreads();   // Xs and the zeroed patches are in place
     expand(patch0);
     if (chunks > 1) load_exp(1);
-    load_proj(0);
     __syncthreads();
     for (int chunk = 0; chunk < chunks; ++chunk) {
         if constexpr (NBUF == 2) {
@@ -289,20 +312,12 @@ __global__ __launch_bounds__(256, 2) void irblock_f32_kernel(const IrParams p) {
         }
     }
 
-    // the two halves of every chunk were summed by different wavefronts: those of the upper half hand their sums over
-    // through LDS (Xs and the patches are free now), the others add them and store
-    float *xchg = ir_lds + (size_t) (pxh * 64 + lane) * (32 * MT + 1);   // odd pitch: no two lanes of a wavefront in one bank
-    if (kh == 1) {
-#pragma unroll
-        for (int a = 0; a < MT; ++a)
-#pragma unroll
-            for (int r = 0; r < 32; ++r) xchg[a * 32 + r] = acc[a][r];
-    }
-    __syncthreads();
-    if (kh == 1) return;
-
-    // store: D register r of lane l is pixel 32 (r / 16) + l % 32 of the wavefront's 64 (rows of a band are contiguous in
-    // NCHW) and output channel 8 ((r % 16) / 4) + 4 (l / 32) + r % 4 of row tile a
+    // The parts of every chunk were summed by different wavefronts.  Through LDS (Xs and the patches are free now), 32 output channels at a time,
+    // the wavefront that had part kh gets all sums of its share of the 32 registers, adds them and stores: register r of lane l is pixel
+    // 32 (r / 16) + l % 32 of the 64 (rows of a band are contiguous in NCHW) and output channel 8 ((r % 16) / 4) + 4 (l / 32) + r % 4
+    // of row tile a
+    constexpr int SHARE = 32 / PARTS;
+    float *const xchg = ir_lds + pxh * 64 + lane;   // [part][register][pixel]
     const rsrc_t ry = make_rsrc(p.y, RSRC_RANGE);
     const rsrc_t rr = make_rsrc(p.res, p.res ? RSRC_RANGE : 0u);
     const rsrc_t rb = make_rsrc(p.pw_b, p.pw_b ? (unsigned) (p.co * 4) : 0u);
@@ -310,47 +325,53 @@ __global__ __launch_bounds__(256, 2) void irblock_f32_kernel(const IrParams p) {
     const int band_px = min(p.band_rows, p.oh - oh0) * p.ow;
     const bool plain = !has_bias || p.pw_ep.act == NOT_ACT;   // conv.c:18-27: without a bias the activation is skipped too
     // every bias and residual value is requested before the first one is used: one memory round trip for the store
-    float bias[MT][16], resv[MT][32];
-    unsigned off[MT][32];
-#pragma unroll
-    for (int a = 0; a < MT; ++a) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) bias[a][r] = buf_load_f32(rb, (unsigned) (a * 32 + 8 * (r / 4) + 4 * lh + (r % 4)) * 4u, 0);
-#pragma unroll
-        for (int r = 0; r < 32; ++r) {
-            const int m = a * 32 + 8 * ((r % 16) / 4) + 4 * lh + (r % 4);
-            const int px = pxh * 64 + 32 * (r / 16) + li;
-            const bool ok = px < band_px && m < p.co;
-            off[a][r] = ok ? (unsigned) ((img * p.co + m) * OHW + oh0 * p.ow + px) * 4u : OOB;
-            resv[a][r] = buf_load_f32(rr, off[a][r], 0);   // no residual: an empty buffer, zeros
-        }
-    }
+    float bias[MT][SHARE], resv[MT][SHARE];
+    unsigned off[MT][SHARE];
+    const int px = pxh * 64 + kh * SHARE / 16 * 32 + li;
 #pragma unroll
     for (int a = 0; a < MT; ++a)
 #pragma unroll
-        for (int r = 0; r < 32; ++r) {
-            float v = __fadd_rn(acc[a][r], xchg[a * 32 + r]);
-            const float vb = __fadd_rn(v, bias[a][r % 16]);
+        for (int i = 0; i < SHARE; ++i) {
+            const int m = a * 32 + 2 * (kh * SHARE % 16) + 8 * (i / 4) + 4 * lh + i % 4;
+            const bool ok = px < band_px && m < p.co;
+            bias[a][i] = buf_load_f32(rb, (unsigned) m * 4u, 0);
+            off[a][i] = ok ? (unsigned) ((img * p.co + m) * OHW + oh0 * p.ow + px) * 4u : OOB;
+            resv[a][i] = buf_load_f32(rr, off[a][i], 0);   // no residual: an empty buffer, zeros
+        }
+#pragma unroll
+    for (int a = 0; a < MT; ++a) {
+        if (a) __syncthreads();   // the sums before these are read
+#pragma unroll
+        for (int r = 0; r < 32; ++r) xchg[(kh * 32 + r) * IR_BN] = acc[a][r];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < SHARE; ++i) {
+            float v = xchg[(kh * SHARE + i) * IR_BN];
+#pragma unroll
+            for (int part = 1; part < PARTS; ++part) v = __fadd_rn(v, xchg[(part * 32 + kh * SHARE + i) * IR_BN]);
+            const float vb = __fadd_rn(v, bias[a][i]);
             v = has_bias ? vb : v;
             if (!plain) v = apply_act(v, p.pw_ep);
-            const float vr = __fadd_rn(v, resv[a][r]);
+            const float vr = __fadd_rn(v, resv[a][i]);
             v = has_res ? vr : v;
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), ry, off[a][r], 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), ry, off[a][i], 0, 0);
         }
+    }
 }
 
-// expansion weights [ce][cin] -> [ce / 16][cin / 4][64] (lane l of step s: row 16 chunk + l % 16, column 4 s + l / 16),
-// then the projection weights [co][ce] -> [ce][cop] k-major, zeros in the padding columns
+// expansion weights [ce][cin] -> fragments (lane l of step s: row 16 chunk + l % 16, column 4 s + l / 16; up to four steps of a lane together),
+// then the projection weights [co][ce] -> [ce / 4][cop][4], zeros in the padding columns
 __global__ __launch_bounds__(256) void irblock_pack_kernel(const float *w_exp, const float *w_proj, int cin, int ce, int co, int cop,
                                                            float *packed) {
     const int idx = blockIdx.x * 256 + threadIdx.x;
     const int n_exp = ce * cin;
     if (idx < n_exp) {
-        const int l = idx & 63, s = (idx >> 6) % (cin / 4), chunk = (idx >> 6) / (cin / 4);
+        const int steps = cin / 4, chunk = idx / (steps * 64), r = idx - chunk * steps * 64;
+        const int s0 = r / 256 * 4, side = min(4, steps - s0), l = (r - s0 * 64) / side, s = s0 + (r - s0 * 64) % side;
         packed[idx] = w_exp[(size_t) (chunk * 16 + (l & 15)) * cin + 4 * s + (l >> 4)];
     } else if (idx < n_exp + ce * cop) {
         const int j = idx - n_exp;
-        const int k = j / cop, m = j - k * cop;
+        const int k = j / (4 * cop) * 4 + j % 4, m = j / 4 % cop;
         packed[idx] = m < co ? w_proj[(size_t) m * ce + k] : 0.0f;
     }
 }
@@ -384,9 +405,9 @@ int irblock_band_rows(const onhip_conv_desc_t &dw, int OH, int OW, int cin) {
     for (; rows >= 1; --rows) {
         const int in_rows = (rows - 1) * dw.stride_h + 3;
         const int P = in_rows * dw.w;
-        const long long slots = ((long long) cin * (P / vec) + 255) / 256;
+        const long long loads = (long long) cin * (P / vec);
         const long long lds = ((long long) cin * ir_xs_pitch(P) + 4 + (long long) IR_KC * in_rows * (dw.w + 2) + 4) * 4;
-        if (lds > IR_LDS_HALF || slots > IR_XSLOTS || (P + 15) / 16 > 4 * IR_TPW) continue;
+        if (lds > IR_LDS_HALF || loads > IR_LOADS || (P + 15) / 16 > IR_TILES) continue;
         if (!tallest) tallest = rows;
         if ((long long) dw.n * ((OH + rows - 1) / rows) >= 256) return rows;
     }
@@ -402,7 +423,7 @@ static int irblock_launch_one(const IrParams &p, size_t lds_bytes, hipStream_t s
                                             hipFuncAttributeMaxDynamicSharedMemorySize, IR_LDS_HALF));
         allowed.store(IR_LDS_HALF);
     }
-    hipLaunchKernelGGL((irblock_f32_kernel<EPI, KS, MT, NBUF>), dim3((unsigned) (p.n * p.bands)), dim3(256), lds_bytes, stream, p);
+    hipLaunchKernelGGL((irblock_f32_kernel<EPI, KS, MT, NBUF>), dim3((unsigned) (p.n * p.bands)), dim3(64 * ir_waves(MT)), lds_bytes, stream, p);
     ONHIP_CHECK_HIP(hipGetLastError());
     return ONHIP_OK;
 }
@@ -412,7 +433,7 @@ static int irblock_launch_ks(const IrParams &p, hipStream_t stream) {
     const int mt = p.cop / 32;
     if (mt > 2) return set_error(ONHIP_ERR_ARG, "inverted-residual block: more than 64 output channels");
     // LDS: Xs, the patch(es), and at least room for the exchange of partial sums at the end of a band
-    const size_t xchg = (size_t) 128 * (32 * mt + 1);
+    const size_t xchg = (size_t) (ir_waves(mt) / 2) * 32 * IR_BN;
     const size_t two = (size_t) p.xs_floats + 2 * (size_t) p.patch_floats, one = (size_t) p.xs_floats + p.patch_floats;
     const bool dbl = two * 4 <= (size_t) IR_LDS_HALF;
     size_t floats = dbl ? two : one;
@@ -457,7 +478,8 @@ int irblock_f32_launch(const onhip_conv_desc_t &ex, const onhip_conv_desc_t &dw,
     p.tiles = (p.P + 15) / 16;
     p.vec = p.w % 4 ? 2 : 4;
     p.groups = p.P / p.vec;
-    p.slots = (p.cin * p.groups + 255) / 256;
+    const int threads = 64 * ir_waves(p.cop / 32);
+    p.slots = (p.cin * p.groups + threads - 1) / threads;
     p.x_bytes = (unsigned) ((size_t) ex.n * ex.cin * ex.h * ex.w * 4);
     p.div_ow = make_div31((unsigned) OW);
     p.div_w = make_div31((unsigned) p.w);
