@@ -211,28 +211,39 @@ __device__ __forceinline__ void unscale_fix_nonfinite(const IgemmProblem &p, f32
 }
 
 // The store for B given as rows (a product's left operand): C is row-major with the tile's columns as its rows, so the four
-// consecutive rows of the tile that a lane holds in registers 4 q .. 4 q + 3 are 16 contiguous bytes of C.  Residual and bias
-// as in write_tile.
-// norm_row: LDS for the lane's row of C as well, at its first column (the variant that normalises the rows), or nullptr.
+// consecutive rows of the tile that a lane holds in registers 4 q .. 4 q + 3 are 16 contiguous bytes of C.  A block of 32 x 32 at a time goes
+// through 4 KB of LDS of the wavefront's own to eight lanes a row of 128 bytes, as which the residual operand arrives too: a row a lane was
+// 64 cycles of the compute unit's address path for each of the four stores and loads, 16 now.  Residual and bias as in write_tile.
+// norm: LDS for the rows of C as well, M + 1 floats apart, at row n_wave (the variant that normalises the rows), or nullptr.
 template <int EPI, int TM, int TN, bool RES, bool NORM = false>
 __device__ __forceinline__ void write_tile_rows(const IgemmProblem &p, f32x16 (&acc)[TM][TN], int m_wave, int n_wave, int li, int lh,
-                                                const float *sbias, lds_f32_t table, float *norm_row = nullptr) {
+                                                const float *sbias, lds_f32_t table, uint4 *turn, float *norm = nullptr) {
     const rsrc_t rc = make_rsrc(p.C, (unsigned) p.c_slice_bytes), rr = make_rsrc(RES ? p.res : nullptr, RES ? (unsigned) p.c_slice_bytes : 0u);
+    const int lane = lh * 32 + li, row8 = lane / 8, u8 = lane % 8;
+    auto unit = [](int row, int u) { return row * 8 + (u ^ (row >> 1 & 7)); };
+    // this lane's piece i of block (a, b): row 8 i + lane / 8, columns 4 (lane % 8) .. + 3
+    auto place = [&](int a, int b, int i) __attribute__((always_inline)) {
+        const int n = n_wave + b * 32 + 8 * i + row8;
+        unsigned base = (unsigned) (n * (int) p.c_stride_n + m_wave + a * 32 + 4 * u8) * 4u;
+        if (p.c_part) {   // several products: a block of 32 rows lies inside one of them
+            const int row = m_wave + a * 32, part = (row >= p.c_part) + (row >= 2 * p.c_part) + (row >= 3 * p.c_part);
+            base += (unsigned) part * (p.c_part_step - (unsigned) p.c_part * 4u);
+        }
+        return n < p.N ? base : OOB;
+    };
+    u32x4 rv[2][4];   // a block ahead
+    auto load_res = [&](int blk) __attribute__((always_inline)) {
+        if constexpr (RES)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) rv[blk & 1][i] = __builtin_amdgcn_raw_buffer_load_b128(rr, place(blk % TM, blk / TM, i), 0, 0);
+    };
+    load_res(0);
 #pragma unroll
     for (int b = 0; b < TN; ++b) {
-        const int n = n_wave + b * 32 + li;
 #pragma unroll
         for (int a = 0; a < TM; ++a) {
-            const int m4 = m_wave + a * 32 + 4 * lh;
-            unsigned base = n < p.N ? (unsigned) (n * (int) p.c_stride_n + m4) * 4u : OOB;
-            if (p.c_part) {   // several products: a block of 32 rows lies inside one of them
-                const int row = m_wave + a * 32, part = (row >= p.c_part) + (row >= 2 * p.c_part) + (row >= 3 * p.c_part);
-                base = n < p.N ? base + (unsigned) part * (p.c_part_step - (unsigned) p.c_part * 4u) : OOB;
-            }
-            u32x4 rv[4];
-            if constexpr (RES)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) rv[q] = __builtin_amdgcn_raw_buffer_load_b128(rr, base + 32u * q, 0, 0);
+            const int blk = b * TM + a;
+            if (blk + 1 < TM * TN) load_res(blk + 1);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const float4 bias = *reinterpret_cast<const float4 *>(sbias + a * 32 + 8 * q + 4 * lh);
@@ -241,23 +252,27 @@ __device__ __forceinline__ void write_tile_rows(const IgemmProblem &p, f32x16 (&
 #pragma unroll
                 for (int j = 0; j < 4; ++j) v[j] = __fadd_rn(acc[a][b][4 * q + j], bv[j]);
                 act_store<EPI, true>(v, p.ep, table);
-                u32x4 o;
+                turn[unit(li, 2 * q + lh)] = make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3]));
+            }
+            const int m = m_wave + a * 32 + 4 * u8, left = p.M - m;   // columns of C from this lane's on
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if constexpr (RES) v[j] = __fadd_rn(v[j], __uint_as_float(rv[q][j]));
-                    o[j] = __float_as_uint(v[j]);
-                }
-                const int left = p.M - (m4 + 8 * q);   // columns of C from this group on
+            for (int i = 0; i < 4; ++i) {
+                const uint4 t = turn[unit(8 * i + row8, u8)];
+                u32x4 o = {t.x, t.y, t.z, t.w};
+                if constexpr (RES)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) o[j] = __float_as_uint(__fadd_rn(__uint_as_float(o[j]), __uint_as_float(rv[blk & 1][i][j])));
                 if constexpr (NORM)
                     if (left > 0)   // rows of a multiple of four
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) norm_row[m4 + 8 * q + j] = v[j];
+                        for (int j = 0; j < 4; ++j) norm[(b * 32 + 8 * i + row8) * (p.M + 1) + m + j] = __uint_as_float(o[j]);
+                const unsigned at = place(a, b, i);
                 if (left >= 4) {
-                    __builtin_amdgcn_raw_buffer_store_b128(o, rc, base + 32u * q, 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b128(o, rc, at, 0, 0);
                 } else {
 #pragma unroll
                     for (int j = 0; j < 3; ++j)
-                        if (j < left) __builtin_amdgcn_raw_buffer_store_b32(o[j], rc, base + 32u * q + 4u * j, 0, 0);
+                        if (j < left) __builtin_amdgcn_raw_buffer_store_b32(o[j], rc, at + 4u * j, 0, 0);
                 }
             }
         }
@@ -467,7 +482,9 @@ void igemm_f3_kernel(const std::conditional_t<NORM, IgemmNormProblem, IgemmProbl
     constexpr int LD = BL == BL_ROWS ? BN + 1 : BN;   // 16-byte slots per 8 elements of K; rows arrive from neighbouring lanes
     constexpr int PLANE = 2 * LD, SLOTS = 3 * PLANE;
     static_assert(!PW2 || (BM == 64 && BN == 64 && WM == 2 && WN == 2), "the second product exists for tiles of 64 x 64");
-    __shared__ uint4 lds[PW2 ? 3 * 8 * 64 : 2 * SLOTS];   // two K tiles; with PW2 then the first product as three parts
+    // two K tiles; with PW2 then the first product as three parts, for rows 4 KB a wavefront for their store
+    constexpr int AFTER = PW2 ? 3 * 8 * 64 : BL == BL_ROWS ? WM * WN * 256 : 0;
+    __shared__ uint4 lds[AFTER > 2 * SLOTS ? AFTER : 2 * SLOTS];
     static_assert(sizeof(lds) >= 2 * SLOTS * sizeof(uint4));
     __shared__ __attribute__((aligned(16))) float s_bias[BM];
 
@@ -670,14 +687,14 @@ void igemm_f3_kernel(const std::conditional_t<NORM, IgemmNormProblem, IgemmProbl
     }
     const float *sb = s_bias + wm * (BM / WM);
     if constexpr (NORM) {   // the launcher gives this variant no activation and a tile over all of M
-        write_tile_rows<EPI_NONE, TM, TN, RES, true>(p, acc, m_wave, n_wave, li, lh, sb, (lds_f32_t) nullptr, s_table + (wn * (BN / WN) + li) * (p.M + 1));
+        write_tile_rows<EPI_NONE, TM, TN, RES, true>(p, acc, m_wave, n_wave, li, lh, sb, (lds_f32_t) nullptr, lds + wave * 256, s_table + wn * (BN / WN) * (p.M + 1));
         static_assert(TN == 1 && BM >= 128, "a lane holds one row; the bias's LDS takes the statistics");
         normalise_rows(p, s_table, s_bias, n0, tid);
         return;
     }
     auto store = [&](auto epi) __attribute__((always_inline)) {
         constexpr int EPI = decltype(epi)::value;
-        if constexpr (BL == BL_ROWS) write_tile_rows<EPI, TM, TN, RES>(p, acc, m_wave, n_wave, li, lh, sb, (lds_f32_t) s_table);
+        if constexpr (BL == BL_ROWS) write_tile_rows<EPI, TM, TN, RES>(p, acc, m_wave, n_wave, li, lh, sb, (lds_f32_t) s_table, lds + wave * 256);
         else write_tile<DT_F32, EPI, TM, TN, RES, true, true>(p, acc, 0, m_wave, n_wave, li, lh, sb, nullptr, nullptr, 0, (lds_f32_t) s_table);
     };
     switch (p.ep.act) {
