@@ -290,10 +290,11 @@ struct IgemmNormProblem : IgemmProblem {
 // a copy in LDS (odd pitch), a wavefront adds up the 64 rows, another one their squares, all of them normalise.  Same operations in the same
 // order as layernorm_rows4_kernel: the same bits.  A chain of M additions and a pass over LDS are 3 to 4 us more on the product (12544 rows of
 // 192 columns from K = 192 15.8 -> 19.0, from K = 768 34.4 -> 38.6) instead of a launch of 6.8; ViT-Tiny at batch 64 1866 -> 1756 us.
+template <int NT>
 __device__ __forceinline__ void normalise_rows(const IgemmNormProblem &p, const float *tile, float *stats, int n0, int tid) {
     const int pitch = p.M + 1, rows = min(64, p.N - n0), groups = p.M / 4, lane = tid & 63, wave = tid >> 6;
     // a thread keeps its four columns and walks down the rows
-    const int per_pass = 256 / groups, r0 = tid / groups, c = tid - r0 * groups;
+    const int per_pass = NT / groups, r0 = tid / groups, c = tid - r0 * groups;
     const float4 w = reinterpret_cast<const float4 *>(p.norm_w)[c], b = reinterpret_cast<const float4 *>(p.norm_b)[c];
     __syncthreads();
     if (wave < 2 && lane < rows) stats[wave * 64 + lane] = wave == 0 ? ln_chain<false>(tile + lane * pitch, p.M) : ln_chain<true>(tile + lane * pitch, p.M);
@@ -474,11 +475,12 @@ __device__ __forceinline__ void pw2_split_stage(const IgemmProblem &p, const f32
 template <int BL, int BM, int BN, int WM, int WN, bool RES, bool PW2 = false, bool NORM = false>
 __global__ __launch_bounds__(64 * WM * WN, (BM / WM) * (BN / WN) >= 32 * 128 ? 2 : (BM / WM) * (BN / WN) > 32 * 64 ? 3 : 4)
 void igemm_f3_kernel(const std::conditional_t<NORM, IgemmNormProblem, IgemmProblem> p) {
-    static_assert(!NORM || (BL == BL_ROWS && WM * WN == 4 && BN == 64 && RES), "rows are normalised behind a residual operand, four wavefronts, 64 rows a tile");
+    static_assert(!NORM || (BL == BL_ROWS && WM * WN >= 4 && BN == 64 && RES), "rows are normalised behind a residual operand, 64 rows a tile");
     static_assert(BM % (WM * 32) == 0 && BN % (WN * 32) == 0, "wavefronts of 32 x 32 blocks");
     constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
     constexpr int UPT = 4, NT = 64 * WM * WN;
-    static_assert(BN * UPT == NT, "a thread stages one unit of B per K tile");
+    constexpr bool ALL = BN * UPT == NT;   // a thread stages one unit of B per K tile, or the first wavefronts' do
+    static_assert(ALL || (BN * UPT < NT && BN * UPT % 64 == 0));
     constexpr int LD = BL == BL_ROWS ? BN + 1 : BN;   // 16-byte slots per 8 elements of K; rows arrive from neighbouring lanes
     constexpr int PLANE = 2 * LD, SLOTS = 3 * PLANE;
     static_assert(!PW2 || (BM == 64 && BN == 64 && WM == 2 && WN == 2), "the second product exists for tiles of 64 x 64");
@@ -517,6 +519,7 @@ void igemm_f3_kernel(const std::conditional_t<NORM, IgemmNormProblem, IgemmProbl
     const int bcol = BL == BL_ROWS ? tid / UPT : tid % BN;
     const int bunit = BL == BL_ROWS ? tid % UPT : __builtin_amdgcn_readfirstlane(tid / BN);
     const ColState col = f3_col<BL>(p, n0 + bcol);
+    const bool stages = ALL || wave < BN * UPT / 64;   // uniform
 
     f32x16 acc[TM][TN];
 #pragma unroll
@@ -585,11 +588,11 @@ void igemm_f3_kernel(const std::conditional_t<NORM, IgemmNormProblem, IgemmProbl
     constexpr std::integral_constant<int, 0> S0{};
     constexpr std::integral_constant<int, 1> S1{};
     prep_unit(0);
-    issue_b(0, S0);
+    if (stages) issue_b(0, S0);
 #pragma unroll
     for (int z = 2; z >= 0; --z) load_a(op0, 0, z);
     prep_unit(1);
-    issue_b(1, S1);
+    if (stages) issue_b(1, S1);
 #pragma unroll
     for (int z = 2; z >= 0; --z) load_a(op1, 1, z);
     // One workgroup a compute unit and a long K: nothing but this workgroup's own loads, two K tiles ahead, covers the trip its part of A
@@ -623,9 +626,9 @@ void igemm_f3_kernel(const std::conditional_t<NORM, IgemmNormProblem, IgemmProbl
         const float bv = buf_load_f32(make_rsrc(p.bias, on ? (unsigned) (p.M * 4) : 0u), row < BM ? (unsigned) (m0 + row) * 4u : OOB, 0);
         bias_row[i] = on ? bv : -0.0f;
     }
-    static_for<4>([&](auto ph) __attribute__((always_inline)) { stage_b(0, ph, S0); });
+    if (stages) static_for<4>([&](auto ph) __attribute__((always_inline)) { stage_b(0, ph, S0); });
     prep_unit(2);
-    issue_b(2, S0);
+    if (stages) issue_b(2, S0);
     prep_unit(3);
     __syncthreads();
     static_for<READS>([&](auto i) __attribute__((always_inline)) { read_operand(op0, 0, i); });
@@ -634,7 +637,7 @@ void igemm_f3_kernel(const std::conditional_t<NORM, IgemmNormProblem, IgemmProbl
     // barrier, B of tile kt + 1 goes through the split to LDS, with the loads of tile kt + 3 into the registers that frees;
     // after the barrier the LDS reads of tile kt + 1.  A of tile kt + 2 is loaded into the operand registers of tile kt as
     // its products retire them (l first, h last).
-    auto body = [&](Operands &cur, Operands &nxt, int kt, auto wr) __attribute__((always_inline)) {
+    auto body = [&](Operands &cur, Operands &nxt, int kt, auto wr, auto stager) __attribute__((always_inline)) {
         constexpr int WR = decltype(wr)::value * SLOTS;
         __builtin_amdgcn_sched_barrier(0);
         static_for<STEPS>([&](auto step) __attribute__((always_inline)) {
@@ -642,7 +645,7 @@ void igemm_f3_kernel(const std::conditional_t<NORM, IgemmNormProblem, IgemmProbl
             mma_bf16(acc[a][b], cur.a[f3_pa(pr)][a], cur.b[f3_pb(pr)][b]);
             static_for<4>([&](auto phase) __attribute__((always_inline)) {
                 constexpr int ph = decltype(phase)::value;
-                if constexpr (ph * (BAR - 1) / 4 == st) {
+                if constexpr (decltype(stager)::value && ph * (BAR - 1) / 4 == st) {
                     stage_b(WR, phase, wr);
                     if constexpr (ph == 1) {   // the unit's floats are used up
                         issue_b(kt + 3, wr);
@@ -663,10 +666,14 @@ void igemm_f3_kernel(const std::conditional_t<NORM, IgemmNormProblem, IgemmProbl
     // Two tiles a trip; behind an odd last tile runs one more, whose B is zero.  No test of reduction indices anywhere: beyond
     // K the split weights are zero, and what B brings in there (the next row or image, zeros behind the tensor) is multiplied
     // by that; should it not be finite, unscale_fix_nonfinite sums the elements over K alone.
-    for (int kt = 0; kt < k_tiles; kt += 2) {
-        body(op0, op1, kt, S1);
-        body(op1, op0, kt + 1, S0);
-    }
+    auto loop = [&](auto stager) __attribute__((always_inline)) {
+        for (int kt = 0; kt < k_tiles; kt += 2) {
+            body(op0, op1, kt, S1, stager);
+            body(op1, op0, kt + 1, S0, stager);
+        }
+    };
+    if (ALL || stages) loop(std::true_type{});
+    else loop(std::false_type{});   // as many barriers
 #pragma unroll
     for (int i = 0; i < TOUCH; ++i) asm volatile("" :: "v"(touch[i]));   // kept until here
 #pragma unroll
@@ -689,7 +696,7 @@ void igemm_f3_kernel(const std::conditional_t<NORM, IgemmNormProblem, IgemmProbl
     if constexpr (NORM) {   // the launcher gives this variant no activation and a tile over all of M
         write_tile_rows<EPI_NONE, TM, TN, RES, true>(p, acc, m_wave, n_wave, li, lh, sb, (lds_f32_t) nullptr, lds + wave * 256, s_table + wn * (BN / WN) * (p.M + 1));
         static_assert(TN == 1 && BM >= 128, "a lane holds one row; the bias's LDS takes the statistics");
-        normalise_rows(p, s_table, s_bias, n0, tid);
+        normalise_rows<NT>(p, s_table, s_bias, n0, tid);
         return;
     }
     auto store = [&](auto epi) __attribute__((always_inline)) {
@@ -720,6 +727,18 @@ static int f3_launch_one(const IgemmLaunch &cfg, const IgemmProblem &p_in, hipSt
     return finish_launch<false>(cfg, p, stream);
 }
 
+// Up to one workgroup a compute unit: a tile of 192 x 64 in twelve wavefronts of one 32 x 32 block each instead of four of three, three a SIMD where
+// there was one to wait for each barrier and each trip of A (196 workgroups, 192 x 12544 x 768 with rows normalised 36.4 -> 32.2 us, from K = 192 15.8 ->
+// 12.8, 192 x 12544 x 768 from 16 x 16 pixels 50.1 -> 46.3; in slices, 160 x 3136 x 960 13.7 -> 12.9); with more of them they stand in for each
+// other.  128 x 64 in eight of one instead of four of two from 32 K tiles on (256 x 6272 x 1024 30.0 -> 28.2, 96 x 12544 x 576 with
+// an Add 20.4 -> 19.2; from 24, without one, 13.8 -> 14.6).  128 x 128 in sixteen was slower (128 x 25088 x 576 56 -> 66).  Same products in the
+// same order: same bits.
+inline int f3_slice_tiles(const IgemmProblem &p) { return (p.k_split_units ? (p.k_split_units < p.k_units ? p.k_split_units : p.k_units) : p.k_units) / 4; }
+inline bool f3_alone(const IgemmLaunch &cfg, const IgemmProblem &p) {
+    const long long slices = p.k_split_units ? (p.k_units + p.k_split_units - 1) / p.k_split_units : 1;
+    return (long long) ((p.M + cfg.bm - 1) / cfg.bm) * ((p.N + cfg.bn - 1) / cfg.bn) * slices <= 256;
+}
+
 // The rows of C normalised in the product's launch: the tile covers all columns, results and parameters are whole 16-byte pieces.
 inline bool f3_norm_ok(const IgemmLaunch &cfg, const IgemmProblem &p) {
     const RowNorm *r = p.norm;
@@ -734,7 +753,8 @@ inline int f3_launch_norm(const IgemmLaunch &cfg, const IgemmProblem &p_in, hipS
     const int rc = tile_grid<192, 64>(cfg, p, &grid);
     if (rc) return rc;
     p.norm_w = p_in.norm->w; p.norm_b = p_in.norm->b; p.norm_y = p_in.norm->y; p.inv_n = 1.0f / p.M;
-    hipLaunchKernelGGL((igemm_f3_kernel<BL_ROWS, 192, 64, 2, 2, true, false, true>), grid, dim3(256), 64 * (p.M + 1) * 4, stream, p);
+    if (f3_alone(cfg, p)) hipLaunchKernelGGL((igemm_f3_kernel<BL_ROWS, 192, 64, 6, 2, true, false, true>), grid, dim3(768), 64 * (p.M + 1) * 4, stream, p);
+    else hipLaunchKernelGGL((igemm_f3_kernel<BL_ROWS, 192, 64, 2, 2, true, false, true>), grid, dim3(256), 64 * (p.M + 1) * 4, stream, p);
     ONHIP_CHECK_HIP(hipGetLastError());
     p_in.norm->done = true;
     return ONHIP_OK;
@@ -745,9 +765,9 @@ int f3_launch_tile(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t st
     switch (cfg.bm * 1000 + cfg.bn) {
         case 256128: return f3_launch_one<BL, 256, 128, 8, 1, RES>(cfg, p, stream);
         case 256064: return f3_launch_one<BL, 256, 64, 4, 1, RES>(cfg, p, stream);
-        case 192064: return f3_launch_one<BL, 192, 64, 2, 2, RES>(cfg, p, stream);
+        case 192064: return f3_alone(cfg, p) ? f3_launch_one<BL, 192, 64, 6, 2, RES>(cfg, p, stream) : f3_launch_one<BL, 192, 64, 2, 2, RES>(cfg, p, stream);
         case 128128: return f3_launch_one<BL, 128, 128, 4, 2, RES>(cfg, p, stream);
-        case 128064: return f3_launch_one<BL, 128, 64, 4, 1, RES>(cfg, p, stream);
+        case 128064: return f3_alone(cfg, p) && f3_slice_tiles(p) >= 32 ? f3_launch_one<BL, 128, 64, 4, 2, RES>(cfg, p, stream) : f3_launch_one<BL, 128, 64, 4, 1, RES>(cfg, p, stream);
         case 64064: return f3_launch_one<BL, 64, 64, 2, 2, RES>(cfg, p, stream);
         default: return set_error(ONHIP_ERR_ARG, "igemm f32: no kernel for tile %dx%d", cfg.bm, cfg.bn);
     }
