@@ -730,10 +730,10 @@ static int f3_launch_one(const IgemmLaunch &cfg, const IgemmProblem &p_in, hipSt
 // Up to one workgroup a compute unit: a tile of 192 x 64 in twelve wavefronts of one 32 x 32 block each instead of four of three, three a SIMD where
 // there was one to wait for each barrier and each trip of A (196 workgroups, 192 x 12544 x 768 with rows normalised 36.4 -> 32.2 us, from K = 192 15.8 ->
 // 12.8, 192 x 12544 x 768 from 16 x 16 pixels 50.1 -> 46.3; in slices, 160 x 3136 x 960 13.7 -> 12.9); with more of them they stand in for each
-// other.  128 x 64 in eight of one instead of four of two from 32 K tiles on (256 x 6272 x 1024 30.0 -> 28.2, 96 x 12544 x 576 with
-// an Add 20.4 -> 19.2; from 24, without one, 13.8 -> 14.6).  128 x 128 in sixteen was slower (128 x 25088 x 576 56 -> 66).  Same products in the
+// other.  The other tiles stay as they are: 128 x 64 in eight and 256 x 64 in eight took 6 % and 14 % less a launch (256 x 6272 x 1024 30.0 -> 28.2, 512 x
+// 1568 x 4608 in slices 46.5 -> 39.6) and ResNet-50 at batch 32 as long as before, its clock lower by as much; 128 x 128 in sixteen was slower
+// (128 x 25088 x 576 56 -> 66).  Same products in the
 // same order: same bits.
-inline int f3_slice_tiles(const IgemmProblem &p) { return (p.k_split_units ? (p.k_split_units < p.k_units ? p.k_split_units : p.k_units) : p.k_units) / 4; }
 inline bool f3_alone(const IgemmLaunch &cfg, const IgemmProblem &p) {
     const long long slices = p.k_split_units ? (p.k_units + p.k_split_units - 1) / p.k_split_units : 1;
     return (long long) ((p.M + cfg.bm - 1) / cfg.bm) * ((p.N + cfg.bn - 1) / cfg.bn) * slices <= 256;
@@ -767,7 +767,7 @@ int f3_launch_tile(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t st
         case 256064: return f3_launch_one<BL, 256, 64, 4, 1, RES>(cfg, p, stream);
         case 192064: return f3_alone(cfg, p) ? f3_launch_one<BL, 192, 64, 6, 2, RES>(cfg, p, stream) : f3_launch_one<BL, 192, 64, 2, 2, RES>(cfg, p, stream);
         case 128128: return f3_launch_one<BL, 128, 128, 4, 2, RES>(cfg, p, stream);
-        case 128064: return f3_alone(cfg, p) && f3_slice_tiles(p) >= 32 ? f3_launch_one<BL, 128, 64, 4, 2, RES>(cfg, p, stream) : f3_launch_one<BL, 128, 64, 4, 1, RES>(cfg, p, stream);
+        case 128064: return f3_launch_one<BL, 128, 64, 4, 1, RES>(cfg, p, stream);
         case 64064: return f3_launch_one<BL, 64, 64, 2, 2, RES>(cfg, p, stream);
         default: return set_error(ONHIP_ERR_ARG, "igemm f32: no kernel for tile %dx%d", cfg.bm, cfg.bn);
     }
