@@ -683,8 +683,12 @@ static double one_pixel_share(const IgemmProblem &p) { return std::min(1.0, (dou
 // shapes and both forms of the weights, weights beyond the L2; error 10 %) and 950 launches of random layers, small planes and batches of
 // one-pixel images among them: a compute unit does its workgroups' steps one after the
 // other, whoever's they are, and a workgroup costs its start.  A stride along the columns takes twice the cache lines.  Two wavefronts per
-// SIMD pay from 32 steps a tile on where a workgroup has its unit to itself (128 x 784 x 1152 12.0 -> 9.7 us).  Only for operands that
-// fit the L2s: with more the other kernels, which load a tile once, are ahead anyway.
+// SIMD pay from 32 steps a tile on where a workgroup has its unit to itself (128 x 784 x 1152 12.0 -> 9.7 us).  For operands that
+// fit the L2s, and up to 64 MB for 1x1 convolutions whose weights are kept split: there several workgroups a unit load while one multiplies, so that a step
+// costs less (`many`), and few rows read a column once or twice.  Of 296 such layers (24 to 384 channels from 96 to 1500 on 3136 to 31360 pixels) it
+// is taken for 70 and those are 22 % faster on average (64 x 12544 x 384 with an Add 17.6 -> 12.4 us, 160 x 3136 x 960 20.9 -> 16.1, 130 x 6272 x 960
+// 31.7 -> 20.8), at most 2 % slower: not for more than 96 rows with a longer K (130 x 6272 x 1500 28.5 and 33.2) nor in 64 rows from a short one
+// (64 x 12544 x 192 8.2 and 9.1).  MobileNetV2 at batch 64 958 -> 934.
 // Columns of different images are apart by a whole image, and a load of 64 lanes touches a cache line for each: with one-pixel images the
 // lines set the pace (29 of them, 848 -> 299 channels, 16.6 us, 7.7 on the other kernels; 96 of them, 1280 -> 1000, 26.6 and 12.4), and rows
 // that straddle lines cost on other small planes (12 images of 3 x 3, 592 -> 267, 9.3 and 8.1; with a stride, so that a load's columns are in more
@@ -695,20 +699,24 @@ static double one_pixel_share(const IgemmProblem &p) { return std::min(1.0, (dou
 static bool kw_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choice *out, double *us) {
     static const double step[2][3] = {{0.122, 0.105, 0.21}, {0.087, 0.086, 0.13}};   // fp32 / split weights; tiles of 16, 32, 64 rows
     static const double base[2][3] = {{2.8, 3.6, 4.4}, {3.4, 3.6, 4.4}}, start[3] = {0.0016, 0.003, 0.003};
+    static const double many[3][2] = {{0.087, 0.087}, {0.080, 0.068}, {0.105, 0.105}};   // split weights, two workgroups a unit and more, above 8 MB
     *us = 1e300;
-    if (cfg.dtype != DT_F32 || p.b_slice_bytes > (8LL << 20)) return false;
+    if (cfg.dtype != DT_F32) return false;
     const int split = kw_split(cfg, p);
+    const bool large = p.b_slice_bytes > (8LL << 20);
+    if (large && (!split || cfg.bl != BL_PLAIN || p.sw != 1 || p.sh != 1 || p.b_slice_bytes > (64LL << 20) || (p.M > 96 && p.K > 1024))) return false;
     const bool table = p.ep.act == SILU || p.ep.act == ONHIP_ACT_GELU_LUT;
     for (int t = 0; t < 3; ++t) {
         const int bm = 16 << t, bn = t ? 32 : 16, ks = t ? 16 : 32;
         const long long tiles = (long long) ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
         const int steps = (p.K + ks - 1) / ks;
-        if (tiles > 2048 || (bm > p.M + 15) || (t == 2 && steps < 6) || (t == 1 && tiles > 256 && steps < 5 && !table) || !kw_ok(cfg, p, bm, split != 0)) continue;
+        if (tiles > 2048 || (bm > p.M + 15) || (t == 2 && steps < (large ? 20 : 6)) || (t == 1 && tiles > 256 && steps < 5 && !table) || !kw_ok(cfg, p, bm, split != 0)) continue;
         const double lines = 64.0 / bn * std::min(bn, p.N) / p.OHW;   // of a load of B, where images are smaller than the tile
         const double apart = p.OHW == 1 ? one_pixel_share(p) * (t == 0 ? 0.0032 * std::max(0.0, lines - 12.0) : (t == 1 ? 0.0028 : 0.002) * lines)
                              : p.OHW <= 4 && p.sw > 1 && lines > 12.0 ? 0.11 : p.OHW < 16 && p.HW % 4 && cfg.bl == BL_PLAIN ? 0.05 : 0.0;
-        const double a_step = step[split][t] * (p.sw > 1 && p.OW > 1 ? 1.4 : 1.0) + apart;
-        const double t_us = base[split][t] + ((tiles + 255) / 256) * steps * a_step + tiles * start[t];
+        const long long rounds = (tiles + 255) / 256;
+        const double a_step = (large && rounds > 1 ? many[t][rounds > 2] : step[split][t]) * (p.sw > 1 && p.OW > 1 ? 1.4 : 1.0) + apart;
+        const double t_us = base[split][t] + (large ? 0.5 : 0.0) + rounds * steps * a_step + tiles * start[t];
         if (t_us < *us) { *us = t_us; *out = Choice{bm, bn, t == 1 && tiles <= 256 && steps >= 32 ? 8 : 4, 0, 3, 0, 0}; }
     }
     return *us < 1e299;
