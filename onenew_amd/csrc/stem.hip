@@ -98,23 +98,28 @@ __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
     // [0, pw): a thread takes column tid (and tid + 256 where the row is that long) of every row
     constexpr int PCH = (127 * 2 + KS + 255) / 256;   // column chunks of 256 per row, at most
     float pv[ROWS][PCH];
-    auto issue = [&](int item) __attribute__((always_inline)) {
+    // where an item's patch lies; past the last item an empty buffer
+    struct Place { rsrc_t rx; int ih0; unsigned voff[PCH]; };
+    auto place = [&](int item) __attribute__((always_inline)) {
         int b = item;
         const int seg = b % p.segs; b /= p.segs;
         const int oh = b % p.oh, img = b / p.oh;
-        const int ih0 = oh * p.stride - p.pt, iw0 = seg * ST_TW * p.stride - p.pl;
-        const rsrc_t rx = make_rsrc(p.x + (size_t) img * CIN * p.h * p.w_in, (unsigned) (CIN * p.h * p.w_in * 4));
+        const int iw0 = seg * ST_TW * p.stride - p.pl;
+        Place q;
+        q.ih0 = oh * p.stride - p.pt;
+        q.rx = make_rsrc(p.x + (size_t) img * CIN * p.h * p.w_in, item < item_end ? (unsigned) (CIN * p.h * p.w_in * 4) : 0u);
 #pragma unroll
         for (int ch = 0; ch < PCH; ++ch) {
             const int col = tid + ch * 256, iw = iw0 + col;
-            const bool col_in = col < pw && (unsigned) iw < (unsigned) p.w_in;
-#pragma unroll
-            for (int r = 0; r < ROWS; ++r) {
-                const int ih = ih0 + r % KS;                                        // uniform
-                const bool in = col_in && (unsigned) ih < (unsigned) p.h;
-                pv[r][ch] = buf_load_f32(rx, in ? (unsigned) iw * 4u : OOB, (unsigned) (((r / KS) * p.h + ih) * p.w_in) * 4u);
-            }
+            q.voff[ch] = col < pw && (unsigned) iw < (unsigned) p.w_in ? (unsigned) iw * 4u : OOB;
         }
+        return q;
+    };
+    constexpr int LOADS = PCH * ROWS;
+    auto load = [&](const Place &q, int which) __attribute__((always_inline)) {
+        const int ch = which / ROWS, r = which % ROWS;
+        const int ih = q.ih0 + r % KS;   // uniform
+        pv[r][ch] = buf_load_f32(q.rx, (unsigned) ih < (unsigned) p.h ? q.voff[ch] : OOB, (unsigned) (((r / KS) * p.h + ih) * p.w_in) * 4u);
     };
     const rsrc_t ry = make_rsrc(p.y, RSRC_RANGE);
     const rsrc_t rb = make_rsrc(p.bias, p.bias ? (unsigned) (p.cout * 4) : 0u);
@@ -132,7 +137,11 @@ __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
             bias_r[a][r] = buf_load_f32(rb, m < p.cout ? (unsigned) m * 4u : OOB, 0);
         }
 
-    issue(item_begin);
+    {
+        const Place q = place(item_begin);
+#pragma unroll
+        for (int l = 0; l < LOADS; ++l) load(q, l);
+    }
     for (int item = item_begin; item < item_end; ++item) {
         __syncthreads();   // everybody has read the previous patch (and, the first time, written the weights)
 #pragma unroll
@@ -144,7 +153,13 @@ __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
             }
         }
         __syncthreads();
-        if (item + 1 < item_end) issue(item + 1);   // uniform
+        // The next patch's loads spread over the steps of a 7x7 filter: all in front, they keep the address path, and with it every wavefront, for as
+        // long as a quarter of the product (64 channels under 7x7 and stride 2 on 32 x 224 x 224 97.9 -> 90.8 us).  Under 3x3 there is seldom a next one.
+        constexpr bool SPREAD = KS == 7;
+        const Place next = place(item + 1);
+        if (!SPREAD && item + 1 < item_end)   // uniform
+#pragma unroll
+            for (int l = 0; l < LOADS; ++l) load(next, l);
 
         f32x16 acc[2];
 #pragma unroll
@@ -153,6 +168,8 @@ __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
             for (int r = 0; r < 16; ++r) acc[a][r] = 0.0f;
 #pragma unroll
         for (int s = 0; s < STEPS; ++s) {
+#pragma unroll
+            for (int l = SPREAD ? s * LOADS / STEPS : LOADS; l < (SPREAD ? (s + 1) * LOADS / STEPS : LOADS); ++l) load(next, l);
             // the two reduction indices of this step, one per lane half: positions in the patch known at compile time
             const int k0 = 2 * s, k1 = 2 * s + 1;
             const int t0 = k0 / CIN, c0 = k0 % CIN, t1 = (k1 < K ? k1 : 0) / CIN, c1 = (k1 < K ? k1 : 0) % CIN;
@@ -160,6 +177,7 @@ __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
             const float bv = pb[lh ? o1 : o0];   // index K (the pad) multiplies a zero weight
             acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(ab[s * 128], bv, acc[0], 0, 0, 0);
             if constexpr (TWO) acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(ab[s * 128 + 64], bv, acc[1], 0, 0, 0);
+            if (SPREAD) __builtin_amdgcn_sched_barrier(0x386);   // matrix instructions and loads stay in this order; arithmetic and LDS may cross
         }
 
         // store: lane = pixel, rows 8 (r / 4) + 4 lh + r % 4 of each 32-channel tile
@@ -167,19 +185,21 @@ __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
         const int seg = b % p.segs; b /= p.segs;
         const int oh = b % p.oh, img = b / p.oh;
         const int ow = seg * ST_TW + wave * 32 + li;
-        const bool col_ok = ow < p.ow;
+        // the row of a register in the scalar offset: one address a lane (one for each register was as long as a 3x3 filter's whole product)
+        const unsigned ohw4 = (unsigned) (p.oh * p.ow) * 4u;
+        const unsigned voff = ow < p.ow ? (unsigned) ((img * p.cout + 4 * lh) * p.oh + oh) * (unsigned) p.ow * 4u + (unsigned) ow * 4u : OOB;
 #pragma unroll
         for (int a = 0; a < (TWO ? 2 : 1); ++a) {
+            const bool whole = p.cout >= a * 32 + 32;   // uniform
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int m = a * 32 + 8 * (r / 4) + 4 * lh + (r % 4);
-                const bool ok = col_ok && m < p.cout;
-                const unsigned off = ok ? (unsigned) (((img * p.cout + m) * p.oh + oh) * p.ow + ow) * 4u : OOB;
+                const int m = a * 32 + 8 * (r / 4) + (r % 4);   // uniform; the lane's row is 4 lh further
                 const float v = acc[a][r];
                 // bias after the full sum; without a bias the value is left alone (the sign of a zero sum) and, like the
                 // reference (conv.c:18-27), so is the activation: p.ep says NOT_ACT then
                 const float vb = __fadd_rn(v, bias_r[a][r]);
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(act_fast<EPI>(has_bias ? vb : v, p.ep)), ry, off, 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(act_fast<EPI>(has_bias ? vb : v, p.ep)), ry,
+                                                      whole || 4 * lh < p.cout - m ? voff : OOB, (unsigned) m * ohw4, 0);
             }
         }
     }
@@ -247,9 +267,9 @@ int stem_f32_launch(const onhip_conv_desc_t &d, int OH, int OW, const float *x, 
     p.div_pw = make_div31((unsigned) p.pw);
     p.ep = ep;
     // 7x7: persistent workgroups, two per compute unit (what its LDS allows), each a run of consecutive row segments
-    // (measured on 64 x 3 x 7 x 7 stride 2 at 32 x 224 x 224: 123 us against 136 us with one segment per workgroup).
+    // (measured on 64 x 3 x 7 x 7 stride 2 at 32 x 224 x 224, when it took 123 us: 136 us with one segment per workgroup; 90 us now).
     // 3x3: one segment per workgroup; eight fit a compute unit and hide each other's loads (32 x 3 x 3 x 3 stride 2 at
-    // 64 x 224 x 224: 42 us against 50 us with 2048 persistent workgroups).
+    // 64 x 224 x 224: 50 us with 2048 persistent workgroups, 45 with one each, 42 since a lane has one store address; 29 at a large copy's rate).
     const long long items = (long long) d.n * OH * p.segs;
     const long long resident = d.kh == 7 ? 512 : items;
     const unsigned grid = (unsigned) (items < resident ? items : resident);
