@@ -155,9 +155,9 @@ __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
         __syncthreads();
         // The next patch's loads spread over the steps of a 7x7 filter: all in front, they keep the address path, and with it every wavefront, for as
         // long as a quarter of the product (64 channels under 7x7 and stride 2 on 32 x 224 x 224 97.9 -> 90.8 us).  Under 3x3 there is seldom a next one.
-        constexpr bool SPREAD = KS == 7;
         const Place next = place(item + 1);
-        if (!SPREAD && item + 1 < item_end)   // uniform
+        const bool more = item + 1 < item_end;   // uniform
+        if (KS != 7 && more)
 #pragma unroll
             for (int l = 0; l < LOADS; ++l) load(next, l);
 
@@ -166,19 +166,24 @@ __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
         for (int a = 0; a < 2; ++a)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[a][r] = 0.0f;
+        auto product = [&](auto spread) __attribute__((always_inline)) {
+            constexpr bool SPREAD = decltype(spread)::value;
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) {
+            for (int s = 0; s < STEPS; ++s) {
 #pragma unroll
-            for (int l = SPREAD ? s * LOADS / STEPS : LOADS; l < (SPREAD ? (s + 1) * LOADS / STEPS : LOADS); ++l) load(next, l);
-            // the two reduction indices of this step, one per lane half: positions in the patch known at compile time
-            const int k0 = 2 * s, k1 = 2 * s + 1;
-            const int t0 = k0 / CIN, c0 = k0 % CIN, t1 = (k1 < K ? k1 : 0) / CIN, c1 = (k1 < K ? k1 : 0) % CIN;
-            const int o0 = (c0 * KS + t0 / KS) * pw + t0 % KS, o1 = (c1 * KS + t1 / KS) * pw + t1 % KS;
-            const float bv = pb[lh ? o1 : o0];   // index K (the pad) multiplies a zero weight
-            acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(ab[s * 128], bv, acc[0], 0, 0, 0);
-            if constexpr (TWO) acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(ab[s * 128 + 64], bv, acc[1], 0, 0, 0);
-            if (SPREAD) __builtin_amdgcn_sched_barrier(0x386);   // matrix instructions and loads stay in this order; arithmetic and LDS may cross
-        }
+                for (int l = SPREAD ? s * LOADS / STEPS : LOADS; l < (SPREAD ? (s + 1) * LOADS / STEPS : LOADS); ++l) load(next, l);
+                // the two reduction indices of this step, one per lane half: positions in the patch known at compile time
+                const int k0 = 2 * s, k1 = 2 * s + 1;
+                const int t0 = k0 / CIN, c0 = k0 % CIN, t1 = (k1 < K ? k1 : 0) / CIN, c1 = (k1 < K ? k1 : 0) % CIN;
+                const int o0 = (c0 * KS + t0 / KS) * pw + t0 % KS, o1 = (c1 * KS + t1 / KS) * pw + t1 % KS;
+                const float bv = pb[lh ? o1 : o0];   // index K (the pad) multiplies a zero weight
+                acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(ab[s * 128], bv, acc[0], 0, 0, 0);
+                if constexpr (TWO) acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(ab[s * 128 + 64], bv, acc[1], 0, 0, 0);
+                if (SPREAD) __builtin_amdgcn_sched_barrier(0x386);   // matrix instructions and loads stay in this order; arithmetic and LDS may cross
+            }
+        };
+        if (KS == 7 && more) product(std::true_type{});
+        else product(std::false_type{});
 
         // store: lane = pixel, rows 8 (r / 4) + 4 lh + r % 4 of each 32-channel tile
         int b = item;
