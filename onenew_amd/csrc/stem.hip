@@ -32,11 +32,14 @@ struct StemParams {
     Epilogue ep;
 };
 
-template <int KS, int EPI, bool TWO>
+// HALF: 64 pixels a workgroup, a wavefront one of the two row tiles
+template <int KS, int EPI, bool TWO, bool HALF = false>
 __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
+    static_assert(!HALF || TWO, "two row tiles to share out");
+    constexpr int TW = HALF ? 64 : ST_TW, TM = TWO && !HALF ? 2 : 1;   // pixels of a segment, row tiles of a wavefront
     constexpr int CIN = 3, TAPS = KS * KS, K = TAPS * CIN, KP = (K + 1) / 2 * 2, STEPS = KP / 2;
     constexpr int ROWS = CIN * KS;                       // patch rows: (channel, filter row)
-    constexpr int PATCH_MAX = ROWS * (127 * 2 + KS) + 8;   // strides up to 2 fit; larger strides are refused by the host
+    constexpr int PATCH_MAX = ROWS * ((TW - 1) * 2 + KS) + 8;   // strides up to 2 fit; larger strides are refused by the host
     __shared__ __attribute__((aligned(16))) float patch[PATCH_MAX];
     // weights in the order the matrix cores read them: [step][row tile][lane half][32 rows] (one conflict-free read per
     // operand: the 64 lanes of a wavefront hit 64 different banks)
@@ -96,7 +99,7 @@ __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
 
     // input patch of an item: row (c, i) holds input row oh * stride - pt + i of channel c, columns ow0 * stride - pl +
     // [0, pw): a thread takes column tid (and tid + 256 where the row is that long) of every row
-    constexpr int PCH = (127 * 2 + KS + 255) / 256;   // column chunks of 256 per row, at most
+    constexpr int PCH = ((TW - 1) * 2 + KS + 255) / 256;   // column chunks of 256 per row, at most
     float pv[ROWS][PCH];
     // where an item's patch lies; past the last item an empty buffer
     struct Place { rsrc_t rx; int ih0; unsigned voff[PCH]; };
@@ -104,7 +107,7 @@ __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
         int b = item;
         const int seg = b % p.segs; b /= p.segs;
         const int oh = b % p.oh, img = b / p.oh;
-        const int iw0 = seg * ST_TW * p.stride - p.pl;
+        const int iw0 = seg * TW * p.stride - p.pl;
         Place q;
         q.ih0 = oh * p.stride - p.pt;
         q.rx = make_rsrc(p.x + (size_t) img * CIN * p.h * p.w_in, item < item_end ? (unsigned) (CIN * p.h * p.w_in * 4) : 0u);
@@ -124,16 +127,17 @@ __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
     const rsrc_t ry = make_rsrc(p.y, RSRC_RANGE);
     const rsrc_t rb = make_rsrc(p.bias, p.bias ? (unsigned) (p.cout * 4) : 0u);
     const bool has_bias = p.bias != nullptr;
-    const float *pb = patch + (wave * 32 + li) * p.stride;
-    const float *ab = At + lh * 32 + li;
+    const int px = HALF ? (wave & 1) * 32 : wave * 32, m_wave = HALF ? (wave >> 1) * 32 : 0;   // uniform
+    const float *pb = patch + (px + li) * p.stride;
+    const float *ab = At + 2 * m_wave + lh * 32 + li;
 
     // the biases of this lane's rows: the same for every item
-    float bias_r[TWO ? 2 : 1][16];
+    float bias_r[TM][16];
 #pragma unroll
-    for (int a = 0; a < (TWO ? 2 : 1); ++a)
+    for (int a = 0; a < TM; ++a)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const int m = a * 32 + 8 * (r / 4) + 4 * lh + (r % 4);
+            const int m = m_wave + a * 32 + 8 * (r / 4) + 4 * lh + (r % 4);
             bias_r[a][r] = buf_load_f32(rb, m < p.cout ? (unsigned) m * 4u : OOB, 0);
         }
 
@@ -161,9 +165,9 @@ __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
 #pragma unroll
             for (int l = 0; l < LOADS; ++l) load(next, l);
 
-        f32x16 acc[2];
+        f32x16 acc[TM];
 #pragma unroll
-        for (int a = 0; a < 2; ++a)
+        for (int a = 0; a < TM; ++a)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[a][r] = 0.0f;
         auto product = [&](auto spread) __attribute__((always_inline)) {
@@ -178,7 +182,7 @@ __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
                 const int o0 = (c0 * KS + t0 / KS) * pw + t0 % KS, o1 = (c1 * KS + t1 / KS) * pw + t1 % KS;
                 const float bv = pb[lh ? o1 : o0];   // index K (the pad) multiplies a zero weight
                 acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(ab[s * 128], bv, acc[0], 0, 0, 0);
-                if constexpr (TWO) acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(ab[s * 128 + 64], bv, acc[1], 0, 0, 0);
+                if constexpr (TM == 2) acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(ab[s * 128 + 64], bv, acc[1], 0, 0, 0);
                 if (SPREAD) __builtin_amdgcn_sched_barrier(0x386);   // matrix instructions and loads stay in this order; arithmetic and LDS may cross
             }
         };
@@ -189,16 +193,16 @@ __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
         int b = item;
         const int seg = b % p.segs; b /= p.segs;
         const int oh = b % p.oh, img = b / p.oh;
-        const int ow = seg * ST_TW + wave * 32 + li;
+        const int ow = seg * TW + px + li;
         // the row of a register in the scalar offset: one address a lane (one for each register was as long as a 3x3 filter's whole product)
         const unsigned ohw4 = (unsigned) (p.oh * p.ow) * 4u;
         const unsigned voff = ow < p.ow ? (unsigned) ((img * p.cout + 4 * lh) * p.oh + oh) * (unsigned) p.ow * 4u + (unsigned) ow * 4u : OOB;
 #pragma unroll
-        for (int a = 0; a < (TWO ? 2 : 1); ++a) {
-            const bool whole = p.cout >= a * 32 + 32;   // uniform
+        for (int a = 0; a < TM; ++a) {
+            const bool whole = p.cout >= m_wave + a * 32 + 32;   // uniform
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int m = a * 32 + 8 * (r / 4) + (r % 4);   // uniform; the lane's row is 4 lh further
+                const int m = m_wave + a * 32 + 8 * (r / 4) + (r % 4);   // uniform; the lane's row is 4 lh further
                 const float v = acc[a][r];
                 // bias after the full sum; without a bias the value is left alone (the sign of a zero sum) and, like the
                 // reference (conv.c:18-27), so is the activation: p.ep says NOT_ACT then
@@ -241,12 +245,17 @@ bool stem_f32_ok(const onhip_conv_desc_t &d, int OH, int OW) {
     return true;
 }
 
+// Segments of 64 pixels where those of 128 would leave half of the compute units without one: each is a wavefront's 148 steps of one row tile instead of
+// two, and half of the loads in front of them (64 channels under 7x7 and stride 2 on one image of 224 x 224 13.1 us in 112 workgroups, 8.8 in 224).
+static int stem_tw(int cout, int ks, long long rows, int ow) { return ks == 7 && cout > 32 && rows * ((ow + ST_TW - 1) / ST_TW) <= 128 ? 64 : ST_TW; }
+
 template <int KS>
 static int stem_launch_ks(const StemParams &p, unsigned grid, hipStream_t stream) {
-    const bool two = p.cout > 32;
+    const bool two = p.cout > 32, half = stem_tw(p.cout, KS, (long long) p.n * p.oh, p.ow) != ST_TW;
 #define ONHIP_STEM_LAUNCH(EPI)                                                                                              \
     do {                                                                                                                    \
-        if (two) hipLaunchKernelGGL((stem_f32_kernel<KS, EPI, true>), dim3(grid), dim3(256), 0, stream, p);                 \
+        if (KS == 7 && half) hipLaunchKernelGGL((stem_f32_kernel<KS, EPI, true, KS == 7>), dim3(grid), dim3(256), 0, stream, p); \
+        else if (two) hipLaunchKernelGGL((stem_f32_kernel<KS, EPI, true>), dim3(grid), dim3(256), 0, stream, p);                 \
         else hipLaunchKernelGGL((stem_f32_kernel<KS, EPI, false>), dim3(grid), dim3(256), 0, stream, p);                    \
     } while (0)
     switch (epi_of_act(p.ep.act)) {
@@ -267,8 +276,9 @@ int stem_f32_launch(const onhip_conv_desc_t &d, int OH, int OW, const float *x, 
     p.x = x; p.w = w; p.bias = d.has_bias ? bias : nullptr; p.y = y;
     p.n = d.n; p.h = d.h; p.w_in = d.w; p.oh = OH; p.ow = OW; p.cout = d.cout; p.stride = d.stride_h; p.pt = d.pad_t; p.pl = d.pad_l;
     p.packed = packed;
-    p.segs = (OW + ST_TW - 1) / ST_TW;
-    p.pw = (ST_TW - 1) * d.stride_h + d.kh;
+    const int tw = stem_tw(d.cout, d.kh, (long long) d.n * OH, OW);
+    p.segs = (OW + tw - 1) / tw;
+    p.pw = (tw - 1) * d.stride_h + d.kh;
     p.div_pw = make_div31((unsigned) p.pw);
     p.ep = ep;
     // 7x7: persistent workgroups, two per compute unit (what its LDS allows), each a run of consecutive row segments

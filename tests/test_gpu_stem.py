@@ -1,5 +1,6 @@
 """First-layer convolutions (stem.hip): output channels off a row tile of 32, one and two of them, widths off a segment of 128 pixels, one and several segments
-a row, fewer items than workgroups and several a workgroup, both weight layouts; against 64-bit sums, within what a chain of fp32 multiply-adds can be off."""
+a row, fewer items than workgroups and several a workgroup, either side of where segments of 64 pixels
+take over, both weight layouts; against 64-bit sums, within what a chain of fp32 multiply-adds can be off."""
 import pytest
 
 from onenew_amd import abi, hip
@@ -10,6 +11,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("packed", [False, True])
 @pytest.mark.parametrize("n,h,w,cout,k,stride,pad,act", [(1, 20, 33, 13, 7, 2, 3, abi.RELU), (5, 230, 224, 64, 7, 2, 3, abi.RELU), (3, 190, 257, 40, 7, 1, 3, abi.NOT_ACT), (9, 125, 300, 32, 7, 2, 0, abi.NOT_ACT),
+                                                         (1, 224, 224, 64, 7, 2, 3, abi.RELU), (1, 20, 261, 50, 7, 1, 3, abi.NOT_ACT), (4, 63, 99, 33, 7, 2, 3, abi.RELU), (3, 85, 99, 33, 7, 2, 3, abi.RELU),
                                                          (1, 9, 7, 5, 3, 1, 1, abi.NOT_ACT), (2, 64, 260, 33, 3, 2, 1, abi.RELU), (2, 40, 129, 64, 3, 1, 1, abi.NOT_ACT), (1, 300, 128, 24, 3, 2, 1, abi.RELU)])
 def test_stem(n, h, w, cout, k, stride, pad, act, packed):
     import torch
