@@ -31,7 +31,7 @@ PLUGINS = {"Conv": "plugin_conv.cpp", "MatMul": "plugin_matmul.cpp", "Gemm": "pl
            "GlobalAveragePool": "plugin_global_avgpool.cpp", "Gelu": "plugin_gelu.cpp",
            "LayerNormalization": "plugin_layernorm.cpp", "Softmax": "plugin_softmax.cpp",
            "Transpose": "plugin_transpose.cpp"}
-HEADERS = [os.path.join(CSRC, "onhip_internal.hpp"), os.path.join(CSRC, "igemm_kernel.hpp"), os.path.join(CSRC, "igemm_f3_kernel.hpp"), os.path.join(CSRC, "igemm_dma_kernel.hpp"), os.path.join(CSRC, "row_norm.hpp"), os.path.join(HERE, "..", "include", "onenew_hip.h"),
+HEADERS = [os.path.join(CSRC, "onhip_internal.hpp"), os.path.join(CSRC, "igemm_kernel.hpp"), os.path.join(CSRC, "igemm_f3_kernel.hpp"), os.path.join(CSRC, "igemm_dma_kernel.hpp"), os.path.join(CSRC, "row_norm.hpp"), os.path.join(CSRC, "row_offset.hpp"), os.path.join(HERE, "..", "include", "onenew_hip.h"),
            os.path.join(HERE, "..", "include", "onenew_abi.h"), os.path.abspath(__file__)]
 
 

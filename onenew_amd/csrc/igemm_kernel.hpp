@@ -34,6 +34,7 @@
 // device/x86/MatMul/mat_mul.c:10.
 #pragma once
 #include "onhip_internal.hpp"
+#include "row_offset.hpp"
 #include <type_traits>
 #include <utility>
 
@@ -50,8 +51,6 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int THREADS = 256;
-constexpr unsigned OOB = 0x80000000u;       // vector offset outside every buffer: loads give 0, stores vanish
-constexpr unsigned RSRC_RANGE = 0x80000000u; // num_records of the data buffers (all offsets stay below 2 GiB)
 constexpr unsigned RSRC_FLAGS = 0x00020000u; // 32-bit data format, raw buffer
 
 typedef __amdgpu_buffer_rsrc_t rsrc_t;

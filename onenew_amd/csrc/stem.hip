@@ -208,7 +208,7 @@ __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
                 // reference (conv.c:18-27), so is the activation: p.ep says NOT_ACT then
                 const float vb = __fadd_rn(v, bias_r[a][r]);
                 __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(act_fast<EPI>(has_bias ? vb : v, p.ep)), ry,
-                                                      whole || 4 * lh < p.cout - m ? voff : OOB, (unsigned) m * ohw4, 0);
+                                                      whole || 4 * lh < p.cout - m ? voff : OOB, row_offset(m, p.cout, ohw4), 0);
             }
         }
     }
