@@ -402,7 +402,7 @@ __device__ __forceinline__ void pw2_split_stage(const IgemmProblem &p, const f32
         v = (lo2_on & !(v > lo2)) ? lo2 : v;
         v = (hi2_on & !(v < hi2)) ? hi2 : v;
         if constexpr (RES) v = add_res(v, addend, p.res_relu, (unsigned) m_uni * row_bytes, body);
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rc, row_voff(m_uni), (unsigned) m_uni * row_bytes, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rc, row_voff(m_uni), row_offset(m_uni, p.m2, row_bytes), 0);
     };
     bool fine = true;   // every sum of the wavefront so far is finite (uniform)
     for (int mb = 0; mb < mblocks; ++mb) {
@@ -412,7 +412,7 @@ __device__ __forceinline__ void pw2_split_stage(const IgemmProblem &p, const f32
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int m_uni = m_wave + 8 * (r / 4) + (r % 4);
-                rv[r] = buf_load_f32(rres, row_voff(m_uni), (unsigned) m_uni * row_bytes);
+                rv[r] = buf_load_f32(rres, row_voff(m_uni), row_offset(m_uni, p.m2, row_bytes));
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -464,7 +464,7 @@ __device__ __forceinline__ void pw2_split_stage(const IgemmProblem &p, const f32
         for (int r = 0; r < 16; ++r) {
             const int m_uni = mb * 64 + wm * 32 + 8 * (r / 4) + (r % 4);
             const float bias = buf_load_f32(rb2, lh16, (unsigned) m_uni * 4u);
-            const float addend = RES ? buf_load_f32(rres, row_voff(m_uni), (unsigned) m_uni * row_bytes) : 0.0f;
+            const float addend = RES ? buf_load_f32(rres, row_voff(m_uni), row_offset(m_uni, p.m2, row_bytes)) : 0.0f;
             finish(acc2[r] * 0.0f != 0.0f ? again[r] : acc2[r] * F3_UNSCALE, bias, addend, m_uni);
         }
     }

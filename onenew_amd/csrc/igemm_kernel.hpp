@@ -461,7 +461,7 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
                         const int m_uni = m_wave + a * 32 + 8 * (r / 4) + (r % 4);
                         const bool row_ok = !EDGE || m_uni + 4 * lh < p.M;
 #pragma unroll
-                        for (int b = 0; b < TN; ++b) rv[r][b] = buf_load_f32(rres, row_ok ? col_voff[b] : OOB, (unsigned) m_uni * row_bytes);
+                        for (int b = 0; b < TN; ++b) rv[r][b] = buf_load_f32(rres, row_ok ? col_voff[b] : OOB, EDGE ? row_offset(m_uni, p.M, row_bytes) : (unsigned) m_uni * row_bytes);
                     }
                 }
 #pragma unroll
@@ -485,7 +485,7 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
                             if constexpr (!FP32)
                                 if (p.acc_out)
                                     __builtin_amdgcn_raw_buffer_store_b32((unsigned) acc[a][b][4 * q + j], racc, row_ok ? col_voff4[b] : OOB,
-                                                                          (unsigned) (m_uni + j) * row_bytes4, 0);
+                                                                          row_offset(m_uni + j, p.M, row_bytes4), 0);
                             float v = y[j * TN + b];
                             if constexpr (RES) {
                                 v = add_res(v, rv[4 * q + j][b], p.res_relu, (col_voff[b] + (unsigned) (m_uni + j) * row_bytes) >> 2, p.res_body);
@@ -505,11 +505,11 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
                                 }
                             }
                             const unsigned voff = row_ok ? col_voff[b] : OOB;
+                            const unsigned soff = EDGE ? row_offset(m_uni + j, p.M, row_bytes) : (unsigned) (m_uni + j) * row_bytes;
                             if (!FP32 && p.out_s8)
-                                __builtin_amdgcn_raw_buffer_store_b8((unsigned char) requant_s8(v, p.out_inv_scale), rc, voff,
-                                                                     (unsigned) (m_uni + j) * row_bytes, 0);
+                                __builtin_amdgcn_raw_buffer_store_b8((unsigned char) requant_s8(v, p.out_inv_scale), rc, voff, soff, 0);
                             else
-                                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rc, voff, (unsigned) (m_uni + j) * row_bytes, 0);
+                                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rc, voff, soff, 0);
                         }
                     }
                 }
@@ -534,7 +534,7 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
                     const bool row_ok = !m_edge || m_uni + 4 * lh < p.M;
 #pragma unroll
                     for (int b = 0; b < TN; ++b)
-                        rv[a][r][b] = buf_load_f32(rres, row_ok ? col_voff[b] : OOB, (unsigned) m_uni * row_bytes);
+                        rv[a][r][b] = buf_load_f32(rres, row_ok ? col_voff[b] : OOB, row_offset(m_uni, p.M, row_bytes));
                 }
         }
         float bias_m[TM][16];
@@ -581,7 +581,7 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
                             if constexpr (RES)
                                 v = add_res(v, rv[a][r][b], p.res_relu, (col_voff[b] + (unsigned) m_uni * row_bytes) >> 2, p.res_body);
                             __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rc, row_ok ? col_voff[b] : OOB,
-                                                                  (unsigned) m_uni * row_bytes, 0);
+                                                                  EDGE ? row_offset(m_uni, p.M, row_bytes) : (unsigned) m_uni * row_bytes, 0);
                         }
                     }
                 }
@@ -987,7 +987,7 @@ __device__ __forceinline__ void write_partial(const IgemmParams &p, ACC (&acc)[T
                 const bool row_ok = !m_edge || m_uni + 4 * lh < p.M;
                 const auto val = acc[a][b][r];   // element copy first: bit-casting the vector element in place miscompiles
                 __builtin_amdgcn_raw_buffer_store_b32(to_bits(val), rp, row_ok ? cv : OOB,
-                                                      (unsigned) m_uni * (unsigned) width * 4u, PUBLISH ? AUX_SYSTEM_SCOPE : 0);
+                                                      row_offset(m_uni, p.M, (unsigned) width * 4u), PUBLISH ? AUX_SYSTEM_SCOPE : 0);
             }
     }
 }
@@ -1067,7 +1067,7 @@ __device__ __forceinline__ void pw2_stage(const IgemmParams &p, const f32x16 &ac
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int m_uni = m_wave + 8 * (r / 4) + (r % 4);
-                rv[r] = buf_load_f32(rres, (!m_edge || m_uni + 4 * lh < p.m2) ? col_voff : OOB, (unsigned) m_uni * row_bytes);
+                rv[r] = buf_load_f32(rres, (!m_edge || m_uni + 4 * lh < p.m2) ? col_voff : OOB, row_offset(m_uni, p.m2, row_bytes));
             }
         }
         f32x16 acc2;
@@ -1092,7 +1092,7 @@ __device__ __forceinline__ void pw2_stage(const IgemmParams &p, const f32x16 &ac
             v = bias2_on ? __fadd_rn(v, b2[r]) : v;
             v = act_fast<EPI>(v, p.ep2);
             if constexpr (RES) v = add_res(v, rv[r], p.res_relu, (col_voff + (unsigned) m_uni * row_bytes) >> 2, p.res_body);
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rc, row_ok ? col_voff : OOB, (unsigned) m_uni * row_bytes, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rc, row_ok ? col_voff : OOB, row_offset(m_uni, p.m2, row_bytes), 0);
         }
     }
 }
@@ -1187,7 +1187,7 @@ __device__ __forceinline__ bool reduce_in_launch(const IgemmParams &p, f32x16 (&
                         const int m_uni = m_wave + a * 32 + 8 * (r / 4) + (r % 4);
                         const bool row_ok = !m_edge || m_uni + 4 * lh < p.M;
                         v[q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                            rp, row_ok ? cv : OOB, (unsigned) m_uni * (unsigned) width * 4u, AUX_SYSTEM_SCOPE));
+                            rp, row_ok ? cv : OOB, row_offset(m_uni, p.M, (unsigned) width * 4u), AUX_SYSTEM_SCOPE));
                     }
 #pragma unroll
                     for (int q = 0; q < 8; ++q) acc[a][b][8 * h + q] = __fadd_rn(acc[a][b][8 * h + q], v[q]);

@@ -52,7 +52,7 @@ def scalar_offsets(text):
         yield m.group(1), args[3 if "store" in m.group(1) else 2]
 
 
-@pytest.mark.parametrize("name", ["stem.hip"])
+@pytest.mark.parametrize("name", ["stem.hip", "igemm_kernel.hpp", "igemm_f3_kernel.hpp"])
 def test_kernels_bound_the_rows_they_mask(name):
     """no buffer access takes a product of a result's row and the bytes of one as its scalar offset"""
     offsets = list(scalar_offsets(open(os.path.join(CSRC, name)).read()))
