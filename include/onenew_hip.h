@@ -103,8 +103,8 @@ long long onhip_product_norm_launches(void);
 /* Diagnostic, no counterpart in the reference: how the calling thread's last dense convolution / MatMul launch ran:
  * out = {tile rows, tile columns, K slices of every tile (1 = none), K slices of the leftover tiles only (0 = none),
  * 1 if the fp32 kernel that reads B straight from memory ran, 2 if the fp32 kernel on the 16-bit matrix cores did (its
- * rows are then the columns of a MatMul), 3 if the fp32 kernel whose wavefronts share K did, 4 if the W8A32 kernel of one launch did (the
- * slices are then wavefronts), 1 if the slices were added up inside the launch,
+ * rows are then the columns of a MatMul), 3 if the fp32 kernel whose wavefronts share K did, 4 if the W8A32 kernel of one launch (the
+ * slices are then wavefronts) or the 16-bit kernel with its rows in registers did, 1 if the slices were added up inside the launch,
  * 1 / 2 / 3 if the kernel that loads operand tiles straight into LDS ran (short ring, long ring, the one in between)}; zeros before the first such
  * launch; launches of the other kernel families (depthwise, first-layer, few-channel int8) leave it as it is. */
 void onhip_last_launch_choice(int32_t out[7]);

@@ -329,8 +329,7 @@ static const int kNumSplits = 13;
 // tail > 1: the tiles left over after whole rounds of 256 are cut `tail` ways along K (launch_choice)
 // rowb == 1: the kernel that feeds B from global memory straight into the MFMAs (igemm_rowb.hip), tile bm x bn; rowb == 2: the
 // fp32 kernel on the 16-bit matrix cores (igemm_f3.hip), tile bm x bn; rowb == 3: the fp32 kernel whose wavefronts share K
-// (igemm_kw.hip), tile bm x bn, `split` wavefronts a workgroup; 4 (onhip_last_launch_choice alone): a 16-bit product with its rows in registers
-// (h16_rows.hip)
+// (igemm_kw.hip), tile bm x bn, `split` wavefronts a workgroup; rowb == 4: the 16-bit kernel with its rows in registers (h16_rows.hip), 256 x 64
 // fin != 0 (with split > 1 or tail > 1): the slices of a tile are added up by the last of them to arrive, inside the
 // launch, instead of by a finishing launch (igemm_kernel, `arrive`)
 // dma != 0: the kernel that loads its operand tiles straight into LDS (igemm_dma_kernel.hpp), tile bm x bn, never split;
@@ -348,6 +347,8 @@ static int tune_mode() {
     }
     return g_tune_mode;
 }
+
+static const long long kKeyRowsH16 = 64;   // in a signature's out_mode: a product that h16_rows.hip has a form for
 
 // Optional persistence of measured choices: ONHIP_TUNE_CACHE names a text file, one line per problem
 // signature ("v0 v1 ... v13 : bm bn split"), read once and appended to after every measurement.
@@ -373,8 +374,14 @@ static void load_tune_cache_locked() {
         }
         Choice c = {0, 0, 1, 0, 0, 0, 0};
         if (*s == ':' && key.size() == 14 && sscanf(s + 1, "%d %d %d %d %d %d %d", &c.bm, &c.bn, &c.split, &c.tail, &c.rowb, &c.fin, &c.dma) >= 3 &&
-            c.bm > 0 && c.bn > 0 && c.split >= 1 && c.split <= 64 && c.tail >= 0 && c.tail <= 64)
+            c.bm > 0 && c.bn > 0 && c.split >= 1 && c.split <= 64 && c.tail >= 0 && c.tail <= 64) {
             g_tuned[key] = c;
+            // 16-bit layers: a line of before they had two kernels holds for the layers that have, until one of theirs follows
+            if ((key[0] == DT_BF16 || key[0] == DT_F16) && key[12] < kKeyRowsH16) {
+                key[12] += kKeyRowsH16;
+                g_tuned.emplace(key, c);
+            }
+        }
     }
     fclose(f);
 }
@@ -465,6 +472,7 @@ static const int kKwShapes[][3] = {{16, 16, 4}, {32, 32, 4}, {32, 32, 8}, {64, 3
 // (bm, bn) is a tile this build has a kernel for
 static bool tile_exists(const Choice &c) {
     if (c.dma) return c.dma <= 3 && dma_tile_ok(c.bm, c.bn);
+    if (c.rowb == 4) return c.bm == 256 && c.bn == 64;
     if (c.rowb == 3) {
         for (const auto &k : kKwShapes)
             if (k[0] == c.bm && k[1] == c.bn && k[2] == c.split) return true;
@@ -504,6 +512,7 @@ static bool candidate_ok(const IgemmLaunch &cfg, const IgemmProblem &p, const Ch
         static const bool off = getenv("ONHIP_NO_DMA") != nullptr;   // tuning hook: the register-staged kernel only
         return (!off || h16) && c.split == 1 && c.tail <= 1 && !c.rowb && !c.fin && dma_ok(cfg, p) && dma_ring_ok(cfg, p, c.bm, c.bn, c.dma - 1);
     }
+    if (c.rowb == 4) return c.split == 1 && c.tail <= 1 && !c.fin && rows_h16_ok(cfg, p);
     if (h16) return false;
     if (c.rowb == 3) return c.tail <= 1 && !c.fin && kw_ok(cfg, p, c.bm, kw_split(cfg, p));
     if (c.rowb == 2 && (c.tail > 1 || c.fin || (c.split > 1 && cfg.bl == BL_ROWS) || !f3_ok(cfg, p))) return false;   // whole tiles, or slices and a finishing launch
@@ -617,6 +626,14 @@ static bool dma_model_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choi
     if (tiles <= 512 && stages >= (best == 3 ? 12 : 3) && dma_ring_ok(cfg, p, bm, bn, 2)) dma = tiles <= 256 && best == 3 && stages >= 32 ? 2 : 3;
     *out = Choice{bm, bn, 1, 0, 0, 0, dma};
     return true;
+}
+
+// A 16-bit product with a short K: the kernel with its rows in registers (h16_rows.hip) from 128 workgroups on; below, the direct-to-LDS kernel's
+// smaller ones reach more of the chip (1000 rows, 192 -> 768 with GELU 5.3 us there and 6.2 in 48 workgroups, 3000 rows, 192 -> 576 5.2 and 5.6 in 108;
+// 4000 rows, 192 -> 768 with GELU 8.0 and 7.2 in 192).
+static const Choice kRowsH16 = {256, 64, 1, 0, 4, 0, 0};
+static bool rows_h16_faster(const IgemmLaunch &cfg, const IgemmProblem &p) {
+    return rows_h16_ok(cfg, p) && (p.N + 255LL) / 256 * rows_h16_subs(p) >= 128;
 }
 
 // a 1x1 convolution whose activations come from beyond the L2s
@@ -740,7 +757,7 @@ static bool f3_wins(const IgemmLaunch &cfg, const IgemmProblem &p, double f3, do
 static Choice model_choice(const IgemmLaunch &cfg, const IgemmProblem &p) {
     Choice best = {64, 64, 1, 0, 0, 0};
     const bool vec = cfg.bl == BL_KVEC || cfg.bl == BL_KVEC_TAP;
-    if (vec && (cfg.dtype != DT_I8 || !tl_hint_bm) && dma_model_choice(cfg, p, &best)) return best;
+    if (vec && (cfg.dtype != DT_I8 || !tl_hint_bm) && dma_model_choice(cfg, p, &best)) return rows_h16_faster(cfg, p) ? kRowsH16 : best;
     // int8 with a large fp32 result (see dma_model_choice): 64 x 64 on the register-staged kernel (measured 1-5 % ahead of
     // 64 x 128 on every such layer of YOLOv8s at batch 16), 32 x 128 where there are no more than 32 rows
     if (vec && cfg.dtype == DT_I8 && !tl_hint_bm && !p.out_s8 && (long long) p.M * p.N >= (long long) 256 * 25600) {
@@ -911,6 +928,11 @@ static int launch_choice(IgemmLaunch cfg, IgemmProblem p, const Choice &c, hipSt
             for (int i = 0; i < 7; ++i) tl_last_choice[i] = v[i];
         }
     } note{cfg, p, c};
+    if (c.rowb == 4) {
+        cfg.split = 1;
+        p.arrive = nullptr;
+        return rows_h16_launch(cfg, p, st);
+    }
     if (c.dma) {
         cfg.bm = c.bm; cfg.bn = c.bn; cfg.split = 1;
         cfg.ring = c.dma - 1;
@@ -1004,7 +1026,7 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
         Choice c = {0, 0, 1, 0, 0, 0, 0};
         if (sscanf(env, "%dx%dx%dx%dx%dx%dx%d", &c.bm, &c.bn, &c.split, &c.tail, &c.rowb, &c.fin, &c.dma) >= 2) {
             if (cfg.dtype != DT_I8 && (cfg.bl == BL_KVEC || cfg.bl == BL_KVEC_TAP)) {   // 16-bit storage: one kernel, its tiles
-                c = {c.bm, c.bn, 1, 0, 0, 0, c.dma > 1 ? c.dma : 1};
+                c = c.rowb == 4 ? kRowsH16 : Choice{c.bm, c.bn, 1, 0, 0, 0, c.dma > 1 ? c.dma : 1};
                 if (!candidate_ok(cfg, p, c)) c = model_choice(cfg, p);
             }
             if (c.dma && !candidate_ok(cfg, p, c)) {   // not a problem (or a tile) for that kernel: the register-staged one
@@ -1024,16 +1046,12 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
             return launch_choice(cfg, p, c, st);
         }
     }
-    if (rows_h16_ok(cfg, p)) {   // measured choices as well: it is not one of the kernels that they choose among
-        static const int as[7] = {256, 64, 1, 0, 4, 0, 0};
-        std::copy(as, as + 7, tl_last_choice);
-        return rows_h16_launch(cfg, p, st);
-    }
     if (!tune_mode()) return launch(by_model());
     std::vector<long long> key = {cfg.dtype, cfg.bl, cfg.batch, p.M, p.N, p.K, p.k_units, p.khkw, p.sh, p.sw,
                                   p.H, p.W, p.out_mode, p.lda};
     if (p.res) key[12] += 16;   // a residual operand narrows the kernels
     if (other ? other->p.keeper : p.keeper) key[12] += 32;   // weights kept split: no pass to pay for, and none too large
+    if (rows_h16_ok(cfg, p)) key[12] += kKeyRowsH16;         // an activation or a result of another type narrows them
     {
         std::unique_lock<std::mutex> lock(g_tune_mu);
         load_tune_cache_locked();
@@ -1134,6 +1152,7 @@ static int plan_and_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStr
             const Choice whole = {c.bm, c.bn, 1, 0, 2, 0, 0};
             if (!rc && f3.split > 1 && candidate_ok(cfg, p, whole)) try_choice(whole);
         }
+    if (!rc && candidate_ok(cfg, p, kRowsH16)) try_choice(kRowsH16);
     // the int8 kernel that loads its tiles straight into LDS
     static const int kDmaTiles[][2] = {{128, 128}, {128, 64}, {64, 128}, {64, 64}};
     for (int t = 0; t < 12 && !rc; ++t) {

@@ -227,20 +227,19 @@ static int rows_h16_launch_dt(const RowsH16Params &p, int ks, bool table, hipStr
 }
 
 // runs of panels that the 64-row panels of A (the channels that pad a row of C as well) are cut into: a workgroup a compute unit
-static int rows_h16_subs(const IgemmParams &p) {
+int rows_h16_subs(const IgemmParams &p) {
     const int blocks = (p.N + 255) / 256, panels = ((int) p.c_stride_n + 63) / 64;
     return blocks >= 256 ? 1 : 256 / blocks < panels ? 256 / blocks : panels;
 }
 
-// Which problems.  From 128 workgroups on: below, igemm_dma_kernel's smaller ones reach more of the chip (1000 rows, 192 -> 768 with GELU 5.3 us there and
-// 6.2 in 48 workgroups here, 3000 rows, 192 -> 576 5.2 and 5.6 in 108; 4000 rows, 192 -> 768 with GELU 8.0 and 7.2 in 192).  Not with a Relu or a Clip
-// alone, the narrow layers in front of a filter, where neither is ahead (100352 rows, 256 -> 64 15.2 and 15.6).
+// Which problems there is a form for (which of them it is faster for: rows_h16_faster).  Not with a Relu or a Clip alone, the narrow layers in front of a
+// filter, where neither is ahead (100352 rows, 256 -> 64 15.2 and 15.6).
 bool rows_h16_ok(const IgemmLaunch &cfg, const IgemmParams &p) {
     if ((cfg.dtype != DT_BF16 && cfg.dtype != DT_F16) || cfg.bl != BL_KVEC || cfg.batch != 1 || !p.out_h16 || p.out_mode != OUT_PLAIN || p.c_stride_m != 1) return false;
     // rows of B as they lie: one tap, no stride, no padding
     if (p.khkw != 1 || p.tap_spans_pixels || p.sh != 1 || p.sw != 1 || p.pt || p.pl || p.OHW != p.HW || p.pix_stride != p.k_units * 16 || p.lda != p.k_units * 16) return false;
     if (p.ep.act != NOT_ACT && p.ep.act != SILU && p.ep.act != ONHIP_ACT_GELU_LUT) return false;
-    return (p.k_units == 8 || p.k_units == 16 || p.k_units == 24 || p.k_units == 32) && (long long) ((p.N + 255) / 256) * rows_h16_subs(p) >= 128;
+    return p.k_units == 8 || p.k_units == 16 || p.k_units == 24 || p.k_units == 32;
 }
 
 int rows_h16_launch(const IgemmLaunch &cfg, const IgemmParams &q, hipStream_t stream) {

@@ -295,6 +295,7 @@ struct IgemmLaunch {
 int igemm_launch(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t stream);
 // 16-bit products with a short K, rows of the left operand in registers (h16_rows.hip)
 bool rows_h16_ok(const IgemmLaunch &cfg, const IgemmParams &p);
+int rows_h16_subs(const IgemmParams &p);
 int rows_h16_launch(const IgemmLaunch &cfg, const IgemmParams &p, hipStream_t stream);
 // fp32 convolution followed by a 1x1 convolution over its result in one launch (igemm_f32_pw.hip): p as for the tap-major
 // packed loader with M <= 64 rows, plus w2 / bias2 / m2 / ep2; with a_split, w2 is split as well (igemm_f3_pw.hip)

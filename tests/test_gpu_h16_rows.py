@@ -9,7 +9,8 @@ from onenew_amd.abi import ConvDesc
 pytestmark = pytest.mark.gpu
 
 # rows, K, columns: more than a workgroup a compute unit; runs of several panels; of one
-SHAPES = [(66000, 64, 96), (65536, 256, 40), (30011, 192, 200), (12608, 192, 768), (25088, 128, 513), (4100, 256, 520), (40001, 50, 129), (8193, 120, 300)]
+OURS = "256x64x1x0x4"
+SHAPES = [(66000, 64, 96), (65536, 256, 40), (30011, 192, 200), (12608, 192, 768), (25088, 128, 513), (4100, 256, 520), (40001, 50, 129), (8193, 120, 300), (300, 192, 70)]
 
 
 def table(torch, gelu):
@@ -33,7 +34,7 @@ def test_linear(rows, k, cols, compute, monkeypatch):
     r = hip.h16_from_rows(torch.randn((rows, cols), generator=g, device="cuda"), compute)
     for bias, gelu, addend in [(b, False, None), (None, False, None), (b, True, None), (b, False, r), (b, True, r)]:
         args = dict(bias=bias, gelu_lut=table(torch, True) if gelu else None, residual=addend)
-        monkeypatch.delenv("ONHIP_TILE", raising=False)
+        monkeypatch.setenv("ONHIP_TILE", OURS)
         y = hip.linear_h16(x, w, k, cols, compute, **args)
         assert hip.last_launch_choice()[4] == 4
         monkeypatch.setenv("ONHIP_TILE", "64x64x1x0x0x0x1")
@@ -62,10 +63,50 @@ def test_convolution(n, cin, hw, cout, act, relu, monkeypatch):
     lut = table(torch, False) if act == abi.SILU else None
     for addend in (None, r):
         run = lambda: hip.conv2d_h16(d, x, w, b, lut, residual=addend, residual_relu=relu and addend is not None)  # noqa: E731
-        monkeypatch.delenv("ONHIP_TILE", raising=False)
+        monkeypatch.setenv("ONHIP_TILE", OURS)
         y = run()
         assert hip.last_launch_choice()[4] == 4
         monkeypatch.setenv("ONHIP_TILE", "64x64x1x0x0x0x1")
         ref = run()
         torch.cuda.synchronize()
         assert hip.last_launch_choice()[4] == 0 and torch.equal(y.view(torch.int16), ref.view(torch.int16))
+
+
+_CHILD = """
+import sys
+sys.path.insert(0, sys.argv[1])
+import torch
+from onenew_amd import abi, hip
+hip.init(0)
+g = torch.Generator(device="cuda").manual_seed(3)
+x = torch.randn((5000, 192), generator=g, device="cuda").to(torch.bfloat16)
+w = hip.h16_pack_matmul_weights(torch.randn((192, 576), generator=g, device="cuda"), abi.COMPUTE_BF16)
+y = hip.linear_h16(x, w, 192, 576, abi.COMPUTE_BF16)
+torch.cuda.synchronize()
+print(*hip.last_launch_choice(), int(y.view(torch.int16).to(torch.int64).sum()))
+"""
+
+
+def test_measured_choices(tmp_path):
+    """measuring asks this kernel and the other one, writes down which it was, and a line of either, or of before there were two, is followed"""
+    import os, subprocess, sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    cache = tmp_path / "choices"
+
+    def run():
+        env = dict(os.environ, ONHIP_TUNE="1", ONHIP_TUNE_CACHE=str(cache))
+        env.pop("ONHIP_TILE", None)
+        res = subprocess.run([sys.executable, "-c", _CHILD, root], env=env, capture_output=True, text=True, timeout=100)
+        assert res.returncode == 0, res.stderr[-2000:]
+        v = [int(t) for t in res.stdout.split()]
+        return v[:7], v[7]
+
+    measured, bits = run()
+    line = cache.read_text().strip().split("\n")[-1].split(" : ")[0].split()
+    assert len(line) == 14 and (measured[4] == 4 or measured[6] > 0)
+    before = [str(int(v) - 64 * (i == 12)) for i, v in enumerate(line)]
+    for key in (line, before):
+        for choice, ran in (([128, 64, 1, 0, 0, 0, 1], [128, 64, 1, 0, 0, 0, 1]), ([256, 64, 1, 0, 4, 0, 0], [256, 64, 1, 0, 4, 0, 0])):
+            cache.write_text(" ".join(key) + " : " + " ".join(map(str, choice)) + "\n")
+            got, same = run()
+            assert got == ran and same == bits
