@@ -628,12 +628,35 @@ static bool dma_model_choice(const IgemmLaunch &cfg, const IgemmProblem &p, Choi
     return true;
 }
 
-// A 16-bit product with a short K: the kernel with its rows in registers (h16_rows.hip) from 128 workgroups on; below, the direct-to-LDS kernel's
-// smaller ones reach more of the chip (1000 rows, 192 -> 768 with GELU 5.3 us there and 6.2 in 48 workgroups, 3000 rows, 192 -> 576 5.2 and 5.6 in 108;
-// 4000 rows, 192 -> 768 with GELU 8.0 and 7.2 in 192).
+// A 16-bit product with a short K: the kernel with its rows in registers (h16_rows.hip) where it is expected to be faster than the direct-to-LDS
+// kernel's choice.  It is a question of how its workgroups, 256 rows and a run of panels each, fill the chip: on 256 rows more than a round of compute units
+// half of them idle through a second (128 -> 512 with an addend 35.0 us at 65436 rows, where the other takes 41.4, and 52.4 at 65692, 43.3 there), a
+// run of all panels for 129 to 255 blocks of rows leaves the other units without any (20.7 and 18.3 at 132 blocks less 100 rows), and a deep K with
+// few columns is start and nothing to spread it over (256 -> 64 13.6 and 10.7 at 65692 rows).  Times in us, fitted to 9190 layers of both kernels (K of 64 to 256, 16 to
+// 1200 columns, 128 to 900 blocks of rows, each with and without a table and an addend; either fit 5 % off): of those it is taken for two thirds, which are 11 %
+// faster on average, 2 % of them more than 3 % slower; all of them were 5 % faster on average, 24 % of them more than 3 % slower, the worst 41 %.
 static const Choice kRowsH16 = {256, 64, 1, 0, 4, 0, 0};
-static bool rows_h16_faster(const IgemmLaunch &cfg, const IgemmProblem &p) {
-    return rows_h16_ok(cfg, p) && (p.N + 255LL) / 256 * rows_h16_subs(p) >= 128;
+static bool rows_h16_faster(const IgemmLaunch &cfg, const IgemmProblem &p, const Choice &dma) {
+    if (!rows_h16_ok(cfg, p)) return false;
+    // without and with an addend, the same with a table: a workgroup's start and a panel, each and for every 64 of K, and the time of a MB; a 64 x 64 tile of the
+    // other kernel, each and for every 64 of K, and the time of a MB
+    static const double rows[4][5] = {{1.69, 0.35, 0.81, 0.38, 0.25}, {0.93, 0.60, 2.22, 0.16, 0.22}, {1.64, 0.33, 1.69, 0.34, 0.29}, {0.96, 0.57, 3.15, 0.13, 0.24}};
+    static const double tile[4][3] = {{0.62, 0.17, 0.23}, {0.77, 0.19, 0.20}, {0.98, 0.16, 0.26}, {1.28, 0.17, 0.23}};
+    const bool table = p.ep.act == SILU || p.ep.act == ONHIP_ACT_GELU_LUT;
+    const int kind = 2 * table + (p.res16 != nullptr);
+    const long long subs = rows_h16_subs(p), panels = ((long long) p.c_stride_n + 63) / 64, blocks = (p.N + 255LL) / 256 * subs;
+    if (blocks < 128) return false;   // the other kernel's smaller workgroups reach more of the chip
+    const double z = p.k_units / 8.0, mb = 1e-6 * 2.0 * p.N * (8.0 * p.k_units + (double) p.c_stride_n * (p.res16 ? 2 : 1));
+    auto either = [](double a, double b) { return sqrt(sqrt(a * a * a * a + b * b * b * b)); };   // the larger, more where they are level
+    // two workgroups a unit with a K of 64 and no table: their starts overlap, of their panels a fifth of the time
+    const bool two = p.k_units == 8 && !table;
+    const double *r = rows[kind], *t = tile[kind];
+    const double starts = two ? (blocks + 511) / 512 : (blocks + 255) / 256, rounds = (blocks + 255) / 256;
+    const double ours = either(1.37 + starts * (r[0] + r[1] * z) + rounds * ((panels + subs - 1) / subs) * (r[2] + r[3] * z) * (two && blocks > 256 ? 0.82 : 1.0), 0.25 + mb * r[4]);
+    const double tiles = (double) ((p.M + dma.bm - 1) / dma.bm) * ((p.N + dma.bn - 1) / dma.bn) / 256.0;
+    const double area = dma.bm * dma.bn == 64 * 64 ? 1.0 : dma.bm * dma.bn == 128 * 128 ? 3.02 : 1.6;
+    const double other = either(3.01 + (0.75 * ceil(tiles) + 0.25 * std::max(tiles, 1.0)) * area * (t[0] + t[1] * z), 0.85 + mb * t[2]);
+    return ours < 0.99 * other;
 }
 
 // a 1x1 convolution whose activations come from beyond the L2s
@@ -757,7 +780,7 @@ static bool f3_wins(const IgemmLaunch &cfg, const IgemmProblem &p, double f3, do
 static Choice model_choice(const IgemmLaunch &cfg, const IgemmProblem &p) {
     Choice best = {64, 64, 1, 0, 0, 0};
     const bool vec = cfg.bl == BL_KVEC || cfg.bl == BL_KVEC_TAP;
-    if (vec && (cfg.dtype != DT_I8 || !tl_hint_bm) && dma_model_choice(cfg, p, &best)) return rows_h16_faster(cfg, p) ? kRowsH16 : best;
+    if (vec && (cfg.dtype != DT_I8 || !tl_hint_bm) && dma_model_choice(cfg, p, &best)) return rows_h16_faster(cfg, p, best) ? kRowsH16 : best;
     // int8 with a large fp32 result (see dma_model_choice): 64 x 64 on the register-staged kernel (measured 1-5 % ahead of
     // 64 x 128 on every such layer of YOLOv8s at batch 16), 32 x 128 where there are no more than 32 rows
     if (vec && cfg.dtype == DT_I8 && !tl_hint_bm && !p.out_s8 && (long long) p.M * p.N >= (long long) 256 * 25600) {

@@ -72,6 +72,30 @@ def test_convolution(n, cin, hw, cout, act, relu, monkeypatch):
         assert hip.last_launch_choice()[4] == 0 and torch.equal(y.view(torch.int16), ref.view(torch.int16))
 
 
+# K, columns, blocks of 256 rows less 100, table, addend: which kernel, by 8 % and more in the times it was fitted to
+CHOICES = [(192, 768, 50, True, False, True), (192, 576, 50, False, False, True), (128, 512, 128, False, True, True), (64, 256, 256, True, False, True), (128, 512, 256, False, True, True),
+           (64, 64, 513, False, False, True), (192, 768, 192, True, False, True), (128, 512, 257, False, True, False), (128, 512, 129, False, True, False), (192, 192, 257, False, True, False),
+           (256, 64, 272, False, False, False), (256, 64, 128, False, False, False), (128, 128, 300, True, False, False), (64, 256, 257, True, False, False), (192, 768, 257, True, False, False),
+           (192, 768, 4, True, False, False)]
+
+
+@pytest.mark.parametrize("k,cols,blocks,gelu,addend,ours", CHOICES)
+def test_choice(k, cols, blocks, gelu, addend, ours, monkeypatch):
+    """whole rounds of workgroups here, a second round of a few of them and a deep K with few columns on the direct-to-LDS kernel"""
+    import torch
+    hip.init(0)
+    monkeypatch.delenv("ONHIP_TILE", raising=False)
+    rows, compute = 256 * blocks - 100, abi.COMPUTE_BF16
+    print(f"{rows} rows, {k} -> {cols}, table {gelu}, addend {addend}", flush=True)
+    x = torch.zeros((rows, k), dtype=torch.bfloat16, device="cuda")
+    w = hip.h16_pack_matmul_weights(torch.zeros((k, cols), device="cuda"), compute)
+    r = torch.ones((rows, cols), dtype=torch.bfloat16, device="cuda") if addend else None
+    y = hip.linear_h16(x, w, k, cols, compute, gelu_lut=table(torch, True) if gelu else None, residual=r)
+    assert (hip.last_launch_choice()[4] == 4) == ours, hip.last_launch_choice()
+    torch.cuda.synchronize()
+    assert bool((y == (1.0 if addend else 0.0)).all())
+
+
 _CHILD = """
 import sys
 sys.path.insert(0, sys.argv[1])
