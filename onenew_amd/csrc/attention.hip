@@ -14,8 +14,8 @@
 // The first product's reduction index (the head dimension) may be enumerated in any order as long as both operands
 // agree: a lane reads four consecutive channels 16 j + 4 (lane / 16) .. + 3 of its row with one 16-byte access and
 // feeds them to four MFMA steps.
-// 16-query wavefronts rather than 32-query ones, which reach twice the SIMDs.  Head dimension 64 with more workgroups than compute units runs on the
-// 16-bit matrix cores instead (attention_f3.hip).
+// 16-query wavefronts rather than 32-query ones, which reach twice the SIMDs.  Head dimension 64 and more than 64 tokens with more workgroups
+// than compute units run on the 16-bit matrix cores instead (attention_f3.hip).
 #include <stdlib.h>
 
 #include "igemm_kernel.hpp"

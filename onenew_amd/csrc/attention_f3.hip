@@ -1,4 +1,4 @@
-// Attention of one (batch, head) on the 16-bit matrix cores, operands and result fp32, head dimension 64, at most 256 tokens: the
+// Attention of one (batch, head) on the 16-bit matrix cores, operands and result fp32, head dimension 64, 65 to 256 tokens: the
 // chain of attention.hip (scores = q k^T * scale, Softmax over the keys, context = scores v) with every product as the six partial
 // products of three bf16 parts (igemm_f3_kernel.hpp: same parts, same order).
 //
@@ -16,7 +16,9 @@
 // over the tiles with all scores in registers, whose 40 KB of code run once and are not there in time.
 // What bounds it: two wavefronts a SIMD, whose 21500 cycles of matrix instructions (196 keys) take 29000 because the barrier keeps them
 // in step, and some 8000 before the first of them: loads, the split of the queries and the first tile.  64 x 3 heads of 196 tokens 22.0 us (23.5
-// with q and the result a row a lane), on fp32 matrix instructions (attention.hip) 30.2.  Error against 64 bits (relative, 2-norm; normal operands, 5 to 256 tokens) 0.8e-7 ... 6.9e-7, there 1.2e-7 ... 9.3e-7.
+// with q and the result a row a lane), on fp32 matrix instructions (attention.hip) 30.2.  Error against 64 bits (relative, 2-norm; normal operands of a spread of 1 to 3,
+// 100 to 256 tokens) 2.5e-7 ... 7.2e-7, there 3.1e-7 ... 9.5e-7; on operands spread over 2^+-4 0.71-0.80 of there, on operands of one sign 0.99-1.03;
+// where one key has all the weight, 5e-8 (v as its three parts' sum, rounded on the way) instead of v itself.
 //
 // Results that are not finite (an operand that is not, or of 2^104 and more, sums of 2^80 and more) are made again from the tensors in
 // memory with fp32 matrix instructions, as in igemm_f3_kernel.hpp: a score that is not finite makes its query's results NaN.
@@ -396,12 +398,14 @@ static int attention_f3_launch_one(AttnF3Params &p, int batch, hipStream_t strea
     return ONHIP_OK;
 }
 
-// Head dimension 64; a scale for which neither it nor its product with the sums' unscaling leaves the normal numbers; and more 64-query
-// workgroups of attention.hip than compute units.  Up to one each, that kernel's 16 queries a wavefront reach four times the SIMDs: 16 x 3
+// Head dimension 64; a scale for which neither it nor its product with the sums' unscaling leaves the normal numbers; more than 64 tokens; and more
+// 64-query workgroups of attention.hip than compute units.  Up to one each, that kernel's 16 queries a wavefront reach four times the SIMDs: 16 x 3
 // heads of 129 tokens 9.9 us there and 12.7 here, 3 heads of 196 11.7 and 14.5; 48 x 3 of 100 12.3 and 10.5, 64 x 3 of 196 30.2 and 22.0,
-// 48 x 3 of 225 36.2 and 22.9.
+// 48 x 3 of 225 36.2 and 22.9.  Up to 64 tokens half of the wavefronts here and more have no queries, and two tiles of keys do not pay for the start: 260
+// heads of 64 tokens 9.0 us there and 10.7 here, 768 of 64 14.1 and 17.1, of 33 11.4 and 15.4, of 16 7.4 and 11.1, 1536 of one 9.1 and 17.1 (17 to 32
+// tokens of 260 to 512 heads are level); of more than 64, 130 to 2048 heads take 0.55-0.99 of the time here.
 bool attention_f3_ok(const onhip_attention_desc_t &d) {
-    return d.head_dim == 64 && d.scale >= 0x1p-60f && d.scale <= 0x1p60f && (long long) d.batch * d.heads * ((d.tokens + 63) / 64) > 256;
+    return d.head_dim == 64 && d.tokens > 64 && d.scale >= 0x1p-60f && d.scale <= 0x1p60f && (long long) d.batch * d.heads * ((d.tokens + 63) / 64) > 256;
 }
 
 int attention_f3_launch(const onhip_attention_desc_t &d, const float *q, const float *k, const float *v, float *out, hipStream_t stream) {
