@@ -6,6 +6,28 @@ namespace onhip {
 int f3_launch_tapc(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t stream);     // igemm_f3_conv.hip
 int f3_launch_gather(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t stream);
 
+// The rows of C normalised in the product's launch: the tile covers all columns, results and parameters are whole 16-byte pieces.
+static bool f3_norm_ok(const IgemmLaunch &cfg, const IgemmProblem &p) {
+    const RowNorm *r = p.norm;
+    return r && cfg.bl == BL_ROWS && cfg.bm == 192 && cfg.bn == 64 && p.res && !p.partial && !p.c_part && p.M <= 192 && p.M >= 32 && p.M % 4 == 0 &&
+           p.c_stride_n == p.M && p.ep.act == NOT_ACT &&
+           ((reinterpret_cast<uintptr_t>(r->w) | reinterpret_cast<uintptr_t>(r->b) | reinterpret_cast<uintptr_t>(r->y)) & 15) == 0;
+}
+// (here and not in the header: what launches a kernel there puts a copy of it into every file that includes it)
+static int f3_launch_norm(const IgemmLaunch &cfg, const IgemmProblem &p_in, hipStream_t stream) {
+    IgemmNormProblem p;
+    static_cast<IgemmProblem &>(p) = p_in;
+    dim3 grid;
+    const int rc = tile_grid<192, 64>(cfg, p, &grid);
+    if (rc) return rc;
+    p.norm_w = p_in.norm->w; p.norm_b = p_in.norm->b; p.norm_y = p_in.norm->y; p.inv_n = 1.0f / p.M;
+    if (f3_alone(cfg, p)) hipLaunchKernelGGL((igemm_f3_kernel<BL_ROWS, 192, 64, 6, 2, true, false, true>), grid, dim3(768), 64 * (p.M + 1) * 4, stream, p);
+    else hipLaunchKernelGGL((igemm_f3_kernel<BL_ROWS, 192, 64, 2, 2, true, false, true>), grid, dim3(256), 64 * (p.M + 1) * 4, stream, p);
+    ONHIP_CHECK_HIP(hipGetLastError());
+    p_in.norm->done = true;
+    return ONHIP_OK;
+}
+
 int f3_launch(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t stream) {
     if (p.M < 1 || p.N < 1 || p.K < 1 || cfg.batch != 1 || cfg.split < 1 || p.dp_tiles || p.arrive || !p.a_split || p.a_split_bytes >= (1LL << 31) ||
         p.b_slice_bytes + 2 * p.b_shift_bytes >= (1LL << 31) || p.c_slice_bytes >= (1LL << 31))

@@ -739,27 +739,6 @@ inline bool f3_alone(const IgemmLaunch &cfg, const IgemmProblem &p) {
     return (long long) ((p.M + cfg.bm - 1) / cfg.bm) * ((p.N + cfg.bn - 1) / cfg.bn) * slices <= 256;
 }
 
-// The rows of C normalised in the product's launch: the tile covers all columns, results and parameters are whole 16-byte pieces.
-inline bool f3_norm_ok(const IgemmLaunch &cfg, const IgemmProblem &p) {
-    const RowNorm *r = p.norm;
-    return r && cfg.bl == BL_ROWS && cfg.bm == 192 && cfg.bn == 64 && p.res && !p.partial && !p.c_part && p.M <= 192 && p.M >= 32 && p.M % 4 == 0 &&
-           p.c_stride_n == p.M && p.ep.act == NOT_ACT &&
-           ((reinterpret_cast<uintptr_t>(r->w) | reinterpret_cast<uintptr_t>(r->b) | reinterpret_cast<uintptr_t>(r->y)) & 15) == 0;
-}
-inline int f3_launch_norm(const IgemmLaunch &cfg, const IgemmProblem &p_in, hipStream_t stream) {
-    IgemmNormProblem p;
-    static_cast<IgemmProblem &>(p) = p_in;
-    dim3 grid;
-    const int rc = tile_grid<192, 64>(cfg, p, &grid);
-    if (rc) return rc;
-    p.norm_w = p_in.norm->w; p.norm_b = p_in.norm->b; p.norm_y = p_in.norm->y; p.inv_n = 1.0f / p.M;
-    if (f3_alone(cfg, p)) hipLaunchKernelGGL((igemm_f3_kernel<BL_ROWS, 192, 64, 6, 2, true, false, true>), grid, dim3(768), 64 * (p.M + 1) * 4, stream, p);
-    else hipLaunchKernelGGL((igemm_f3_kernel<BL_ROWS, 192, 64, 2, 2, true, false, true>), grid, dim3(256), 64 * (p.M + 1) * 4, stream, p);
-    ONHIP_CHECK_HIP(hipGetLastError());
-    p_in.norm->done = true;
-    return ONHIP_OK;
-}
-
 template <int BL, bool RES>
 int f3_launch_tile(const IgemmLaunch &cfg, const IgemmProblem &p, hipStream_t stream) {
     switch (cfg.bm * 1000 + cfg.bn) {
