@@ -16,7 +16,8 @@
 //     memory traffic;
 //   * depthwise and projection as in dwproj.hip: taps added in ascending (i, j) order to a zero sum, multiply and add
 //     rounded separately, bias last (conv.c:757-899), so the depthwise stage is bit-identical to the operator on the same
-//     input; the projection accumulates in v_mfma_f32_32x32x2_f32 with its weights k-major in registers;
+//     input; the projection accumulates in v_mfma_f32_32x32x1_2b_f32 (a lane's pixel of the wavefront's 64, one channel an
+//     instruction), its weights [channel / 4][output channel][channel % 4] in memory: four channels a 16-byte load, kept in registers;
 //   * per chunk: expansion of the next one (into a second patch where LDS has room for it), depthwise and projection of this one, barrier.  Two
 //     workgroups of eight wavefronts share a compute unit (with four each, waiting for each other and for weights was half of the time: MobileNetV2
 //     batch 64, its six blocks 104, 92, 76, 40, 39 and 55 us; eight with 16-byte weight loads 83, 87, 52, 35, 34, and 48 with four).

@@ -1,15 +1,15 @@
 // First-layer convolutions: three input channels, k x k filter (7x7 or 3x3), any stride and padding, at most 64 output
 // channels, fp32 NCHW.  The implicit-GEMM kernels spend this layer gathering: with three channels there is no run of the
 // reduction index that is contiguous in memory, so every operand element is its own load, and the many short tiles pay
-// the per-tile set-up over and over.  Here a workgroup takes 128 consecutive output pixels of one output row:
+// the per-tile set-up over and over.  Here a workgroup takes 128 consecutive output pixels of one output row (64 where a 7x7 layer has few rows: stem_tw):
 //
 //   * the input patch those pixels read (3 channels x k rows x (127 stride + k) columns) is copied into LDS once with
 //     coalesced loads, zeros where it hangs over the image's edge;
-//   * the weights go to LDS transposed ([reduction index][output channel]);
+//   * the weights go to LDS as the matrix instructions read them ([step][row tile][lane half][32 output channels]);
 //   * the B operand of v_mfma_f32_32x32x2_f32 is read straight from the patch: reduction index (tap, channel) is a
 //     compile-time position in the patch, the pixel a stride between lanes; the reduction runs over 3 k k (+ 1 zero)
 //     indices, none wasted on channel padding;
-//   * wavefront w owns pixels 32 w .. 32 w + 31 and both 32-row tiles of output channels.
+//   * wavefront w owns pixels 32 w .. 32 w + 31 and both 32-row tiles of output channels; of 64 pixels, 32 (w % 2) .. + 31 and tile w / 2.
 //
 // Same arithmetic as the other fp32 convolutions of this library (fp32 products summed in fp32 by the matrix cores, bias
 // after the sum, then the activation): device/x86/Conv/conv.c:1024-1056 (im2col + GEMM) with its epilogue :1216-1304.
@@ -19,15 +19,15 @@
 
 namespace onhip {
 
-constexpr int ST_TW = 128;   // output pixels per workgroup
+constexpr int ST_TW = 128;   // output pixels per workgroup and segment
 
 struct StemParams {
     const float *x, *w, *bias;
     float *y;
     int n, h, w_in, oh, ow, cout, stride, pt, pl;
     int packed;        // weights as stem_pack_kernel lays them out (the LDS image) instead of [cout][3][k][k]
-    int segs;          // row segments of 128 pixels per output row
-    int pw;            // patch columns: 127 * stride + k
+    int segs;          // row segments (of 128 or 64 pixels) per output row
+    int pw;            // patch columns: (pixels of a segment - 1) * stride + k
     Div31 div_pw;
     Epilogue ep;
 };
@@ -245,8 +245,8 @@ bool stem_f32_ok(const onhip_conv_desc_t &d, int OH, int OW) {
     return true;
 }
 
-// Segments of 64 pixels where those of 128 would leave half of the compute units without one: each is a wavefront's 148 steps of one row tile instead of
-// two, and half of the loads in front of them (64 channels under 7x7 and stride 2 on one image of 224 x 224 13.1 us in 112 workgroups, 8.8 in 224).
+// Segments of 64 pixels where those of 128 would leave half of the compute units without one: each is a wavefront's 74 steps of one row tile instead of
+// two (74 matrix instructions instead of 148), and half of the loads in front of them (64 channels under 7x7 and stride 2 on one image of 224 x 224 13.1 us in 112 workgroups, 8.8 in 224).
 static int stem_tw(int cout, int ks, long long rows, int ow) { return ks == 7 && cout > 32 && rows * ((ow + ST_TW - 1) / ST_TW) <= 128 ? 64 : ST_TW; }
 
 template <int KS>

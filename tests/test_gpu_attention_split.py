@@ -64,7 +64,7 @@ def test_attention_against_64_bits(b, h, t, std, torch_dev):
     assert error(out) <= error(other), (error(out), error(other))
 
 
-@pytest.mark.parametrize("b,h,t", [(260, 1, 64), (768, 1, 64), (300, 2, 33), (520, 1, 16), (600, 1, 1), (64, 4, 33), (64, 2, 65), (32, 2, 200), (60, 1, 196), (64, 1, 256)])
+@pytest.mark.parametrize("b,h,t", [(260, 1, 64), (768, 1, 64), (300, 2, 33), (520, 1, 16), (600, 1, 1), (130, 2, 5), (260, 1, 31), (90, 3, 32), (260, 1, 33), (90, 3, 63), (64, 4, 33), (64, 2, 65), (32, 2, 200), (60, 1, 196), (64, 1, 256)])
 def test_calls_for_fp32_instructions(b, h, t, torch_dev):
     """up to 64 tokens, and up to one workgroup a compute unit"""
     torch = torch_dev

@@ -1,6 +1,6 @@
 """fp32 on the 16-bit matrix cores, the tile of 192 x 64 on either side of one workgroup a compute unit, where it takes twelve wavefronts instead of four:
-the bits of the 64 x 64 tile, whose wavefronts are the same everywhere.  Rows, 1x1 and 3x3 convolutions, with an addend, a table activation, ragged rows and
-columns, slices of K."""
+the bits of the 64 x 64 tile, whose wavefronts are the same everywhere, and of each other.  Rows, 1x1 and 3x3 convolutions, with an addend, a table
+activation, ragged rows and columns, slices of K."""
 import pytest
 
 from onenew_amd import abi, hip
@@ -24,9 +24,10 @@ def both(tile, other, run, monkeypatch, torch):
     assert torch.equal(got[0].view(torch.int32), got[1].view(torch.int32))
 
 
-# (tiles of a product cannot be asked for; the model takes it for the first three and others for the rest)
-@pytest.mark.parametrize("rows,k,n", [(12544, 192, 192), (12481, 767, 187), (16384, 200, 190), (6272, 1024, 250), (17000, 520, 187), (33000, 192, 192)])
-def test_product(rows, k, n):
+# Tiles of a product cannot be asked for: with the one that the model takes.  192 x 64 in twelve wavefronts up to 16384 rows and in four above, then others.
+@pytest.mark.parametrize("rows,k,n,tile", [(12544, 192, 192, (192, 64)), (12481, 767, 187, (192, 64)), (16384, 200, 190, (192, 64)), (33000, 520, 187, (192, 64)),
+                                           (32961, 768, 192, (192, 64)), (6272, 1024, 250, None), (17000, 520, 187, (64, 64)), (33000, 192, 192, (64, 64))])
+def test_product(rows, k, n, tile):
     import torch
     hip.init(0)
     g = torch.Generator(device="cuda").manual_seed(rows + k)
@@ -38,8 +39,14 @@ def test_product(rows, k, n):
     y = hip.matmul(a, b, bias=bias)
     plain = list(hip.last_launch_choice())
     print(rows, k, n, plain, flush=True)
+    assert plain[4] == 2 and (tile is None or tuple(plain[:2]) == tile)
     assert bool(((y.double() - ref).abs() <= bound).all())
+    if rows > 16384:   # the first rows alone, in twelve wavefronts: the same products in the same order
+        part = hip.matmul(a[:12481], b, bias=bias)
+        assert tuple(hip.last_launch_choice()[:2]) == (192, 64) and hip.last_launch_choice()[4] == 2
+        assert torch.equal(y[:12481].view(torch.int32), part.view(torch.int32))
     z = hip.matmul(a, b, bias=bias, addend=add)
+    assert tile != (192, 64) or list(hip.last_launch_choice()) == plain
     if list(hip.last_launch_choice()) == plain:   # a choice of its own, so perhaps other sums
         assert torch.equal(z, y + add)
     else:

@@ -8,9 +8,10 @@ from onenew_amd import hip, onefile, rt
 pytestmark = pytest.mark.gpu
 
 # (rows, k, n, in one launch): rows that end inside a tile of 64, alone in one, and full; the widest row a tile holds and narrower ones, off 32 and off 16
-# columns; then products that run in another tile, rows that no tile holds (196, 256), of three columns more than a multiple of four, and few rows, where
+# columns, in twelve wavefronts up to 16384 rows and in four above; then products that run in another tile, rows that no tile holds (196, 256), of three columns more than a multiple of four, and few rows, where
 # the normalisation is a launch of its own
 CASES = [(12544, 192, 192, 1), (12544, 768, 192, 1), (12481, 192, 192, 1), (12481, 201, 180, 1), (12544, 192, 164, 1), (16001, 201, 132, 1), (14001, 200, 148, 1),
+         (33001, 768, 192, 1), (32961, 520, 180, 1), (33024, 600, 164, 1),
          (9999, 201, 180, 0), (12544, 64, 164, 0), (20001, 96, 132, 0), (9999, 96, 100, 0), (12544, 64, 196, 0), (9999, 192, 256, 0), (9999, 64, 163, 0),
          (12544, 192, 163, 0), (50, 192, 192, 0), (65, 64, 64, 0)]
 
