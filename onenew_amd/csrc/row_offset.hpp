@@ -19,4 +19,11 @@ ONHIP_BOTH constexpr unsigned row_offset(int row, int rows, unsigned row_bytes) 
     return (unsigned) (row < rows ? row : rows - 1) * row_bytes;
 }
 
+// The same for a patch's row `ih` of channel c, which may lie above or below an image of h rows (its lanes are masked then, and the padding may be of any
+// height): the nearest row of the channel, below the image's size.  (3 x 10 x 30000 with 20000 rows of padding below: row 17900 was asked for at 2 GiB and
+// 500 KB, which is byte 500000 of the image if the sum with OOB wraps; so was a row above an image of nearly 2 GiB.)
+ONHIP_BOTH constexpr unsigned patch_row_offset(int c, int ih, int h, unsigned row_bytes) {
+    return (unsigned) (c * h + (ih < 0 ? 0 : ih < h ? ih : h - 1)) * row_bytes;
+}
+
 }  // namespace onhip

@@ -122,7 +122,7 @@ __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
     auto load = [&](const Place &q, int which) __attribute__((always_inline)) {
         const int ch = which / ROWS, r = which % ROWS;
         const int ih = q.ih0 + r % KS;   // uniform
-        pv[r][ch] = buf_load_f32(q.rx, (unsigned) ih < (unsigned) p.h ? q.voff[ch] : OOB, (unsigned) (((r / KS) * p.h + ih) * p.w_in) * 4u);
+        pv[r][ch] = buf_load_f32(q.rx, (unsigned) ih < (unsigned) p.h ? q.voff[ch] : OOB, patch_row_offset(r / KS, ih, p.h, (unsigned) p.w_in * 4u));
     };
     const rsrc_t ry = make_rsrc(p.y, RSRC_RANGE);
     const rsrc_t rb = make_rsrc(p.bias, p.bias ? (unsigned) (p.cout * 4) : 0u);

@@ -10,6 +10,7 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 
 PROGRAM = r"""
 #include <cstdio>
+#include <initializer_list>
 #include "row_offset.hpp"
 using namespace onhip;
 int main() {
@@ -23,6 +24,17 @@ int main() {
                 const unsigned long long sum = (unsigned long long) OOB + at;
                 if (sum < RSRC_RANGE || sum >= 1ull << 32) return printf("row %d of %d, %u bytes each: %llu\n", row, rows, row_bytes, sum), 1;
             }
+        }
+    // images of three channels up to just below 2 GiB, rows far above and below
+    for (int h : {1, 2, 10, 224, 4700, 13000})
+        for (long long bytes : {4ll, 896ll, 120000ll, (long long) (((1ll << 31) - 1) / 3 / h / 4 * 4)}) {
+            if (3 * h * bytes >= 1ll << 31) continue;
+            for (int c = 0; c < 3; ++c)
+                for (int ih = -300; ih < h + 30000; ++ih) {
+                    const unsigned at = patch_row_offset(c, ih, h, (unsigned) bytes);
+                    if (ih >= 0 && ih < h && at != (unsigned) ((c * h + ih) * bytes)) return printf("row %d of %d is at %u\n", ih, h, at), 1;
+                    if ((unsigned long long) OOB + at >= 1ull << 32 || at >= 3ull * h * bytes) return printf("row %d of %d, %lld bytes each: %u\n", ih, h, bytes, at), 1;
+                }
         }
     return 0;
 }
@@ -57,5 +69,6 @@ def test_kernels_bound_the_rows_they_mask(name):
     """no buffer access takes a product of a result's row and the bytes of one as its scalar offset"""
     offsets = list(scalar_offsets(open(os.path.join(CSRC, name)).read()))
     assert any("row_offset(" in at for _, at in offsets)
-    bare = [(call, at) for call, at in offsets if re.search(r"\bm(_uni)?\b", at) and "row_offset(" not in at and not at.endswith("* 4u")]
+    assert name != "stem.hip" or any("patch_row_offset(" in at for _, at in offsets)
+    bare = [(call, at) for call, at in offsets if re.search(r"\b(m(_uni)?|ih)\b", at) and "row_offset(" not in at and not at.endswith("* 4u")]
     assert not bare, bare
