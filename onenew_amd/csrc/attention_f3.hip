@@ -14,8 +14,9 @@
 // behind them a piece at a time, up to six vector instructions a matrix instruction being free: the split of tile t's exponentials and of
 // the next k and v behind the former, the exponentials of tile t + 1 and the loads behind the latter; one barrier.  It is a loop, not unrolled
 // over the tiles with all scores in registers, whose 40 KB of code run once and are not there in time.
-// What bounds it: two wavefronts a SIMD, whose 21500 cycles of matrix instructions (196 keys) take 29000 because the barrier keeps them
-// in step, and some 8000 before the first of them: loads, the split of the queries and the first tile.  64 x 3 heads of 196 tokens 22.0 us (23.5
+// What bounds it: two wavefronts a SIMD, whose 21500 cycles of matrix instructions (196 keys) are half of a launch's 45000, because the barrier keeps
+// them in step (0.39 of their time is waiting) and nothing covers what lies before the first of them: loads, the split of the queries and the first tile.
+// 64 x 3 heads of 196 tokens 22.0 us (23.5
 // with q and the result a row a lane), on fp32 matrix instructions (attention.hip) 30.2.  Error against 64 bits (relative, 2-norm; normal operands of a spread of 1 to 3,
 // 100 to 256 tokens) 2.5e-7 ... 7.2e-7, there 3.1e-7 ... 9.5e-7; on operands spread over 2^+-4 0.71-0.80 of there, on operands of one sign 0.99-1.03;
 // where one key has all the weight, 5e-8 (v as its three parts' sum, rounded on the way) instead of v itself.

@@ -22,7 +22,7 @@
 //     workgroups of eight wavefronts share a compute unit (with four each, waiting for each other and for weights was half of the time: MobileNetV2
 //     batch 64, its six blocks 104, 92, 76, 40, 39 and 55 us; eight with 16-byte weight loads 83, 87, 52, 35, 34, and 48 with four).
 // What bounds it: the vector instructions' issue.  fp32 matrix instructions take it as long as they run (measured: one of 32 x 32 is 65 cycles, and n vector
-// instructions behind it, of any wavefront, make 65 + 4 n), and 75 thousand cycles of them and 85 thousand of the rest are most of the 183
+// instructions behind it, of any wavefront, make 65 + 4 n), and 75 thousand cycles of them and 86 thousand of the rest are most of the 186
 // thousand that 24 -> 144 -> 24 channels on 56 x 56 take a SIMD.
 // The expansion sums in another order than the library's separate 1x1 kernel (k in steps of 4 instead of 2), so the block
 // equals the chain of three operators within fp32 summation error, not bit for bit.

@@ -31,6 +31,7 @@ import sys
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SIMDS = 256 * 4            # MI355X: 256 compute units of 4 SIMDs
+ENGINES = 8 * 4            # shader engines, over which SQ_BUSY_CYCLES is summed
 CLOCK_HZ = 2.4e9           # peak engine clock the MFMA peak is quoted at
 GLUE = ("add_kernel", "relu_kernel", "maxpool", "gap_kernel", "layernorm", "softmax", "transpose_kernel", "gelu_lut")
 LEGEND = ("Kernel names: `onhip::igemm_kernel<dtype, loader, BM, BN, WM, WN, PF, RES, PW2>` (dtype 0 fp32, 1 bf16, 2 f16, 3 int8; loader 0 "
@@ -40,9 +41,11 @@ LEGEND = ("Kernel names: `onhip::igemm_kernel<dtype, loader, BM, BN, WM, WN, PF,
           "16-bit storage: operand tiles loaded straight into LDS, KS bytes of K per stage, ring of NST stages), `onhip::rowb_f32_kernel<WM, WN>` (fp32, B "
           "straight from memory, tile 32 WM x 128 WN), `onhip::igemm_f3_kernel<loader, BM, BN, WM, WN, RES, PW2, NORM>` (fp32 on the 16-bit matrix cores; loader 5 "
           "the rows of a product; NORM the variant that normalises the rows of its result as well) and `onhip::split_weights_kernel` in front of it where the weights are split on the call, `onhip::splitk_finish_kernel`, `onhip::depthwise_tiled_kernel<int8, stride, "
-          "act>`, `onhip::quantize_nhwc_kernel<CBW>`, `onhip::stem_f32_kernel<filter size, act, two row tiles>` (first-layer "
+          "act>`, `onhip::quantize_nhwc_kernel<CBW>`, `onhip::stem_f32_kernel<filter size, act, two row tiles, segments of 64 pixels>` (first-layer "
           "convolutions from an LDS patch), `onhip::i8patch_kernel<bytes per pixel, WM, pixel tiles>` and `onhip::i8direct_kernel<bytes per pixel, taps, WM, TM, pixel "
-          "tiles, workgroups per CU>` (int8 chain form, 3x3 with few channels: input rows in LDS / windows loaded per tap), `onhip::attention_f32_kernel<16-key tiles, head dim>`, `onhip::dw_s8_nhwc_kernel<3x3 stride, epilogue, fp32 out>` (depthwise on int8 NHWC), `onhip::irblock_f32_kernel<act, input channels / 4, row tiles, "
+          "tiles, workgroups per CU>` (int8 chain form, 3x3 with few channels: input rows in LDS / windows loaded per tap), `onhip::attention_f32_kernel<16-key tiles, head dim>`, "
+          "`onhip::attention_f3_kernel<wavefronts>` (fp32 on the 16-bit matrix cores), `onhip::attention_h16_kernel<dtype, 32-key tiles, wavefronts>`, "
+          "`onhip::rows_h16_kernel<dtype, K / 16, table activation>` (16-bit products with a short K), `onhip::igemm_kw_kernel` (fp32, wavefronts that share K), `onhip::dw_s8_nhwc_kernel<3x3 stride, epilogue, fp32 out>` (depthwise on int8 NHWC), `onhip::irblock_f32_kernel<act, input channels / 4, row tiles, "
           "patches>` (1x1 expansion + depthwise 3x3 + 1x1 projection in one launch), and the element-wise kernels.")
 
 
@@ -62,7 +65,7 @@ def short(name):
 def family(name):
     if "_pack_kernel" in name:   # weight re-layouts: once per model, not part of a pass
         return None
-    if "igemm" in name or helper(name) or "rowb_f32" in name or "attention" in name or "stem_f32" in name or "i8patch" in name or "i8direct" in name:
+    if "igemm" in name or helper(name) or "rowb_f32" in name or "rows_h16" in name or "i8small" in name or "attention" in name or "stem_f32" in name or "i8patch" in name or "i8direct" in name:
         return "igemm"
     if "depthwise" in name or "irblock" in name or "dw_s8" in name:
         return "depthwise"
@@ -174,10 +177,10 @@ def summarise(workload, raw, out_dir):
         L.append("## Matrix-core and LDS counters (`--pmc SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CYCLES SQ_INSTS_LDS SQ_LDS_BANK_CONFLICT SQ_WAVE_CYCLES "
                  "SQ_INSTS_VALU SQ_WAIT_ANY`, means per dispatch)\n")
         L.append("MFMA utilisation = SQ_VALU_MFMA_BUSY_CYCLES (summed over the SIMDs) / (kernel duration from the trace x "
-                 f"{CLOCK_HZ / 1e9:.1f} GHz x {SIMDS} SIMDs); wait share = SQ_WAIT_ANY / SQ_WAVE_CYCLES; conflict share = "
+                 f"{CLOCK_HZ / 1e9:.1f} GHz x {SIMDS} SIMDs); cycles a launch = SQ_BUSY_CYCLES / {ENGINES} shader engines; wait share = SQ_WAIT_ANY / SQ_WAVE_CYCLES; conflict share = "
                  "SQ_LDS_BANK_CONFLICT cycles / (4 x SQ_WAVE_CYCLES) is left out where no LDS instruction ran.\n")
-        L.append("| kernel | dispatches | MFMA busy cycles | MFMA utilisation | LDS instructions | LDS bank-conflict cycles | VALU instructions | wait share |\n"
-                 "|---|---:|---:|---:|---:|---:|---:|---:|")
+        L.append("| kernel | dispatches | cycles a launch | MFMA busy cycles | MFMA utilisation | LDS instructions | LDS bank-conflict cycles | VALU instructions | wait share |\n"
+                 "|---|---:|---:|---:|---:|---:|---:|---:|---:|")
         for k in sorted(sq):
             if family(k) is None:
                 continue
@@ -186,7 +189,7 @@ def summarise(workload, raw, out_dir):
             d = dur_us.get(k)
             util = busy / (d * 1e-6 * CLOCK_HZ * SIMDS) if d else float("nan")
             wave = mean(c["SQ_WAVE_CYCLES"])
-            L.append(f"| `{k}` | {len(c['SQ_BUSY_CYCLES'])} | {busy:.4g} | {util:.3f} | {mean(c['SQ_INSTS_LDS']):.4g} | "
+            L.append(f"| `{k}` | {len(c['SQ_BUSY_CYCLES'])} | {mean(c['SQ_BUSY_CYCLES']) / ENGINES:.4g} | {busy:.4g} | {util:.3f} | {mean(c['SQ_INSTS_LDS']):.4g} | "
                      f"{mean(c['SQ_LDS_BANK_CONFLICT']):.4g} | {mean(c['SQ_INSTS_VALU']):.4g} | "
                      f"{(mean(c['SQ_WAIT_ANY']) / wave if wave else 0):.2f} |")
         L.append("")
