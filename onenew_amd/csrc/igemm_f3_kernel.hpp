@@ -394,26 +394,33 @@ __device__ __forceinline__ void pw2_split_stage(const IgemmProblem &p, const f32
     const int n = n0 + wn * 32 + li, lh4 = 4 * lh;
     const unsigned col_voff = n < p.N ? out_col_offset(p, n, 4) + (unsigned) lh4 * row_bytes : OOB;
     // rows in groups of four: a lane's are inside or beyond m2 by group and remainder, asked again for the store
-    auto row_voff = [&](int m_uni) __attribute__((always_inline)) { return lh4 < p.m2 - m_uni ? col_voff : OOB; };
+    auto row_voff = [&](int m_uni, auto edge) __attribute__((always_inline)) { return !decltype(edge)::value || lh4 < p.m2 - m_uni ? col_voff : OOB; };
     // relu.c's rule by element index: row offsets of this lane's column that lie in its body (one register, not sixteen sums)
     const unsigned body = p.res_body * 4u > col_voff ? p.res_body * 4u - col_voff : 0u;
-    auto finish = [&](float v, float bias, float addend, int m_uni) __attribute__((always_inline)) {
+    auto finish = [&](float v, float bias, float addend, int m_uni, auto edge) __attribute__((always_inline)) {
+        if (!row_there<decltype(edge)::value>(m_uni, p.m2)) return;   // uniform
         v = bias2_on ? __fadd_rn(v, bias) : v;
         v = (lo2_on & !(v > lo2)) ? lo2 : v;
         v = (hi2_on & !(v < hi2)) ? hi2 : v;
         if constexpr (RES) v = add_res(v, addend, p.res_relu, (unsigned) m_uni * row_bytes, body);
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rc, row_voff(m_uni), row_offset(m_uni, p.m2, row_bytes), 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rc, row_voff(m_uni, edge), (unsigned) m_uni * row_bytes, 0);
     };
     bool fine = true;   // every sum of the wavefront so far is finite (uniform)
     for (int mb = 0; mb < mblocks; ++mb) {
         const int m_wave = mb * 64 + wm * 32;   // uniform
+        const bool m_edge = m_wave + 32 > p.m2;
         float b2[16], rv[RES ? 16 : 1];
-        if constexpr (RES) {
+        auto addends = [&](auto edge) __attribute__((always_inline)) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int m_uni = m_wave + 8 * (r / 4) + (r % 4);
-                rv[r] = buf_load_f32(rres, row_voff(m_uni), row_offset(m_uni, p.m2, row_bytes));
+                rv[r] = 0.0f;
+                if (row_there<decltype(edge)::value>(m_uni, p.m2)) rv[r] = buf_load_f32(rres, row_voff(m_uni, edge), (unsigned) m_uni * row_bytes);
             }
+        };
+        if constexpr (RES) {
+            if (m_edge) addends(std::true_type{});
+            else addends(std::false_type{});
         }
         __builtin_amdgcn_sched_barrier(0);
         f32x16 acc2;
@@ -439,8 +446,12 @@ __device__ __forceinline__ void pw2_split_stage(const IgemmProblem &p, const f32
 #pragma unroll
         for (int r = 0; r < 16; ++r) probe = __builtin_fmaf(acc2[r], 0.0f, probe);
         fine &= __builtin_amdgcn_ballot_w64(probe != probe) == 0ull;
+        auto store = [&](auto edge) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) finish(acc2[r] * F3_UNSCALE, b2[r], RES ? rv[r] : 0.0f, m_wave + 8 * (r / 4) + (r % 4));
+            for (int r = 0; r < 16; ++r) finish(acc2[r] * F3_UNSCALE, b2[r], RES ? rv[r] : 0.0f, m_wave + 8 * (r / 4) + (r % 4), edge);
+        };
+        if (m_edge) store(std::true_type{});
+        else store(std::false_type{});
     }
     if (fine) return;
     // All blocks once more, sums that are not finite from fp32 matrix instructions: a pass of its own, so that the one above
@@ -464,8 +475,9 @@ __device__ __forceinline__ void pw2_split_stage(const IgemmProblem &p, const f32
         for (int r = 0; r < 16; ++r) {
             const int m_uni = mb * 64 + wm * 32 + 8 * (r / 4) + (r % 4);
             const float bias = buf_load_f32(rb2, lh16, (unsigned) m_uni * 4u);
-            const float addend = RES ? buf_load_f32(rres, row_voff(m_uni), row_offset(m_uni, p.m2, row_bytes)) : 0.0f;
-            finish(acc2[r] * 0.0f != 0.0f ? again[r] : acc2[r] * F3_UNSCALE, bias, addend, m_uni);
+            if (!row_there<true>(m_uni, p.m2)) continue;   // uniform
+            const float addend = RES ? buf_load_f32(rres, row_voff(m_uni, std::true_type{}), (unsigned) m_uni * row_bytes) : 0.0f;
+            finish(acc2[r] * 0.0f != 0.0f ? again[r] : acc2[r] * F3_UNSCALE, bias, addend, m_uni, std::true_type{});
         }
     }
 }

@@ -461,7 +461,10 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
                         const int m_uni = m_wave + a * 32 + 8 * (r / 4) + (r % 4);
                         const bool row_ok = !EDGE || m_uni + 4 * lh < p.M;
 #pragma unroll
-                        for (int b = 0; b < TN; ++b) rv[r][b] = buf_load_f32(rres, row_ok ? col_voff[b] : OOB, EDGE ? row_offset(m_uni, p.M, row_bytes) : (unsigned) m_uni * row_bytes);
+                        for (int b = 0; b < TN; ++b) rv[r][b] = 0.0f;
+                        if (row_there<EDGE>(m_uni, p.M))   // uniform
+#pragma unroll
+                            for (int b = 0; b < TN; ++b) rv[r][b] = buf_load_f32(rres, row_ok ? col_voff[b] : OOB, (unsigned) m_uni * row_bytes);
                     }
                 }
 #pragma unroll
@@ -480,12 +483,13 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         const bool row_ok = !EDGE || m_uni + j + 4 * lh < p.M;
+                        const bool there = row_there<EDGE>(m_uni + j, p.M);   // uniform
 #pragma unroll
                         for (int b = 0; b < TN; ++b) {
                             if constexpr (!FP32)
-                                if (p.acc_out)
+                                if (p.acc_out && there)
                                     __builtin_amdgcn_raw_buffer_store_b32((unsigned) acc[a][b][4 * q + j], racc, row_ok ? col_voff4[b] : OOB,
-                                                                          row_offset(m_uni + j, p.M, row_bytes4), 0);
+                                                                          (unsigned) (m_uni + j) * row_bytes4, 0);
                             float v = y[j * TN + b];
                             if constexpr (RES) {
                                 v = add_res(v, rv[4 * q + j][b], p.res_relu, (col_voff[b] + (unsigned) (m_uni + j) * row_bytes) >> 2, p.res_body);
@@ -504,8 +508,8 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
                                     }
                                 }
                             }
-                            const unsigned voff = row_ok ? col_voff[b] : OOB;
-                            const unsigned soff = EDGE ? row_offset(m_uni + j, p.M, row_bytes) : (unsigned) (m_uni + j) * row_bytes;
+                            if (!there) continue;
+                            const unsigned voff = row_ok ? col_voff[b] : OOB, soff = (unsigned) (m_uni + j) * row_bytes;
                             if (!FP32 && p.out_s8)
                                 __builtin_amdgcn_raw_buffer_store_b8((unsigned char) requant_s8(v, p.out_inv_scale), rc, voff, soff, 0);
                             else
@@ -523,43 +527,46 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
         if (RES && p.twin) kind(std::bool_constant<RES>{});
         else kind(std::false_type{});
     } else {
-        float rv[RES ? TM : 1][RES ? 16 : 1][RES ? TN : 1];
-        if constexpr (RES) {
-            const rsrc_t rres = make_rsrc(reinterpret_cast<const char *>(p.res) + (size_t) batch * p.c_batch_stride * 4, RSRC_RANGE);
-#pragma unroll
-            for (int a = 0; a < TM; ++a)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m_uni = m_wave + a * 32 + 8 * (r / 4) + (r % 4);
-                    const bool row_ok = !m_edge || m_uni + 4 * lh < p.M;
-#pragma unroll
-                    for (int b = 0; b < TN; ++b)
-                        rv[a][r][b] = buf_load_f32(rres, row_ok ? col_voff[b] : OOB, row_offset(m_uni, p.M, row_bytes));
-                }
-        }
-        float bias_m[TM][16];
-        if constexpr (BIAS_LDS) {
-#pragma unroll
-            for (int a = 0; a < TM; ++a)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float4 t = *reinterpret_cast<const float4 *>(sbias + a * 32 + 8 * q + 4 * lh);
-                    bias_m[a][4 * q + 0] = t.x; bias_m[a][4 * q + 1] = t.y; bias_m[a][4 * q + 2] = t.z; bias_m[a][4 * q + 3] = t.w;
-                }
-        } else {
-#pragma unroll
-            for (int a = 0; a < TM; ++a)
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    bias_m[a][r] = buf_load_f32(rbias_m, lh16, (unsigned) (m_wave + a * 32 + 8 * (r / 4) + (r % 4)) * 4u);
-        }
-        // One add per value whatever the bias: the addend is the row's or the column's bias, or -0.0f, which leaves every
-        // value as it is (the sign of a zero sum included).  Rows are tested against M in the last row tile only.
-        float bias_sel[TN];
-#pragma unroll
-        for (int b = 0; b < TN; ++b) bias_sel[b] = bias_n_on ? bias_n[b] : -0.0f;
-        auto store_rows = [&](auto edge) __attribute__((always_inline)) {
+        // the tile at the edge of M, where rows are tested, is a variant of its own
+        auto store = [&](auto edge) __attribute__((always_inline)) {
             constexpr bool EDGE = decltype(edge)::value;
+            float rv[RES ? TM : 1][RES ? 16 : 1][RES ? TN : 1];
+            if constexpr (RES) {
+                const rsrc_t rres = make_rsrc(reinterpret_cast<const char *>(p.res) + (size_t) batch * p.c_batch_stride * 4, RSRC_RANGE);
+#pragma unroll
+                for (int a = 0; a < TM; ++a)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int m_uni = m_wave + a * 32 + 8 * (r / 4) + (r % 4);
+                        const bool row_ok = !EDGE || m_uni + 4 * lh < p.M;
+#pragma unroll
+                        for (int b = 0; b < TN; ++b) rv[a][r][b] = 0.0f;
+                        if (row_there<EDGE>(m_uni, p.M))   // uniform
+#pragma unroll
+                            for (int b = 0; b < TN; ++b) rv[a][r][b] = buf_load_f32(rres, row_ok ? col_voff[b] : OOB, (unsigned) m_uni * row_bytes);
+                    }
+            }
+            float bias_m[TM][16];
+            if constexpr (BIAS_LDS) {
+#pragma unroll
+                for (int a = 0; a < TM; ++a)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const float4 t = *reinterpret_cast<const float4 *>(sbias + a * 32 + 8 * q + 4 * lh);
+                        bias_m[a][4 * q + 0] = t.x; bias_m[a][4 * q + 1] = t.y; bias_m[a][4 * q + 2] = t.z; bias_m[a][4 * q + 3] = t.w;
+                    }
+            } else {
+#pragma unroll
+                for (int a = 0; a < TM; ++a)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        bias_m[a][r] = buf_load_f32(rbias_m, lh16, (unsigned) (m_wave + a * 32 + 8 * (r / 4) + (r % 4)) * 4u);
+            }
+            // One add per value whatever the bias: the addend is the row's or the column's bias, or -0.0f, which leaves every
+            // value as it is (the sign of a zero sum included).
+            float bias_sel[TN];
+#pragma unroll
+            for (int b = 0; b < TN; ++b) bias_sel[b] = bias_n_on ? bias_n[b] : -0.0f;
 #pragma unroll
             for (int a = 0; a < TM; ++a)
 #pragma unroll
@@ -575,19 +582,19 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
                     for (int j = 0; j < 4; ++j) {
                         const int r = 4 * q + j, m_uni = m_wave + a * 32 + 8 * q + j;   // row of lanes with lh == 0
                         const bool row_ok = !EDGE || m_uni + 4 * lh < p.M;
+                        if (row_there<EDGE>(m_uni, p.M))   // uniform
 #pragma unroll
-                        for (int b = 0; b < TN; ++b) {
-                            float v = y[j * TN + b];
-                            if constexpr (RES)
-                                v = add_res(v, rv[a][r][b], p.res_relu, (col_voff[b] + (unsigned) m_uni * row_bytes) >> 2, p.res_body);
-                            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rc, row_ok ? col_voff[b] : OOB,
-                                                                  EDGE ? row_offset(m_uni, p.M, row_bytes) : (unsigned) m_uni * row_bytes, 0);
-                        }
+                            for (int b = 0; b < TN; ++b) {
+                                float v = y[j * TN + b];
+                                if constexpr (RES)
+                                    v = add_res(v, rv[a][r][b], p.res_relu, (col_voff[b] + (unsigned) m_uni * row_bytes) >> 2, p.res_body);
+                                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rc, row_ok ? col_voff[b] : OOB, (unsigned) m_uni * row_bytes, 0);
+                            }
                     }
                 }
         };
-        if (m_edge) store_rows(std::true_type{});
-        else store_rows(std::false_type{});
+        if (m_edge) store(std::true_type{});
+        else store(std::false_type{});
     }
 }
 
@@ -974,22 +981,27 @@ __device__ __forceinline__ void write_partial(const IgemmParams &p, ACC (&acc)[T
                                               int n_wave, int li, int lh) {
     const int width = p.N - p.part_begin;   // partial sums cover the columns from part_begin on
     const rsrc_t rp = make_rsrc(reinterpret_cast<const char *>(p.partial) + (size_t) slice * p.M * width * 4, RSRC_RANGE);
-    const bool m_edge = m_wave + TM * 32 > p.M;
+    auto store = [&](auto edge) __attribute__((always_inline)) {
+        constexpr bool EDGE = decltype(edge)::value;
 #pragma unroll
-    for (int b = 0; b < TN; ++b) {
-        const int n = n_wave + b * 32 + li;
-        const unsigned cv = n < p.N ? (unsigned) (n - p.part_begin + 4 * lh * width) * 4u : OOB;
+        for (int b = 0; b < TN; ++b) {
+            const int n = n_wave + b * 32 + li;
+            const unsigned cv = n < p.N ? (unsigned) (n - p.part_begin + 4 * lh * width) * 4u : OOB;
 #pragma unroll
-        for (int a = 0; a < TM; ++a)
+            for (int a = 0; a < TM; ++a)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m_uni = m_wave + a * 32 + 8 * (r / 4) + (r % 4);
-                const bool row_ok = !m_edge || m_uni + 4 * lh < p.M;
-                const auto val = acc[a][b][r];   // element copy first: bit-casting the vector element in place miscompiles
-                __builtin_amdgcn_raw_buffer_store_b32(to_bits(val), rp, row_ok ? cv : OOB,
-                                                      row_offset(m_uni, p.M, (unsigned) width * 4u), PUBLISH ? AUX_SYSTEM_SCOPE : 0);
-            }
-    }
+                for (int r = 0; r < 16; ++r) {
+                    const int m_uni = m_wave + a * 32 + 8 * (r / 4) + (r % 4);
+                    const bool row_ok = !EDGE || m_uni + 4 * lh < p.M;
+                    const auto val = acc[a][b][r];   // element copy first: bit-casting the vector element in place miscompiles
+                    if (row_there<EDGE>(m_uni, p.M))   // uniform
+                        __builtin_amdgcn_raw_buffer_store_b32(to_bits(val), rp, row_ok ? cv : OOB,
+                                                              (unsigned) m_uni * (unsigned) width * 4u, PUBLISH ? AUX_SYSTEM_SCOPE : 0);
+                }
+        }
+    };
+    if (m_wave + TM * 32 > p.M) store(std::true_type{});   // uniform
+    else store(std::false_type{});
 }
 
 // ---- a second, 1x1 product over the finished tile (the PW2 variant of the kernel, fp32, tile 64 x 64) ---------------------
@@ -1063,12 +1075,18 @@ __device__ __forceinline__ void pw2_stage(const IgemmParams &p, const f32x16 &ac
         float b2[16], rv[RES ? 16 : 1];
 #pragma unroll
         for (int r = 0; r < 16; ++r) b2[r] = buf_load_f32(rb2, lh16, (unsigned) (m_wave + 8 * (r / 4) + (r % 4)) * 4u);
-        if constexpr (RES) {
+        auto addends = [&](auto edge) __attribute__((always_inline)) {
+            constexpr bool EDGE = decltype(edge)::value;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int m_uni = m_wave + 8 * (r / 4) + (r % 4);
-                rv[r] = buf_load_f32(rres, (!m_edge || m_uni + 4 * lh < p.m2) ? col_voff : OOB, row_offset(m_uni, p.m2, row_bytes));
+                rv[r] = 0.0f;
+                if (row_there<EDGE>(m_uni, p.m2)) rv[r] = buf_load_f32(rres, (!EDGE || m_uni + 4 * lh < p.m2) ? col_voff : OOB, (unsigned) m_uni * row_bytes);
             }
+        };
+        if constexpr (RES) {
+            if (m_edge) addends(std::true_type{});
+            else addends(std::false_type{});
         }
         f32x16 acc2;
 #pragma unroll
@@ -1084,16 +1102,22 @@ __device__ __forceinline__ void pw2_stage(const IgemmParams &p, const f32x16 &ac
             wa[s] = buf_load_b128(rw2, next_voff, next_soff + 1024u * s);
             __builtin_amdgcn_sched_barrier(0);
         }
+        auto store = [&](auto edge) __attribute__((always_inline)) {
+            constexpr bool EDGE = decltype(edge)::value;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int m_uni = m_wave + 8 * (r / 4) + (r % 4);
-            const bool row_ok = !m_edge || m_uni + 4 * lh < p.m2;
-            float v = acc2[r];
-            v = bias2_on ? __fadd_rn(v, b2[r]) : v;
-            v = act_fast<EPI>(v, p.ep2);
-            if constexpr (RES) v = add_res(v, rv[r], p.res_relu, (col_voff + (unsigned) m_uni * row_bytes) >> 2, p.res_body);
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rc, row_ok ? col_voff : OOB, row_offset(m_uni, p.m2, row_bytes), 0);
-        }
+            for (int r = 0; r < 16; ++r) {
+                const int m_uni = m_wave + 8 * (r / 4) + (r % 4);
+                const bool row_ok = !EDGE || m_uni + 4 * lh < p.m2;
+                if (!row_there<EDGE>(m_uni, p.m2)) continue;
+                float v = acc2[r];
+                v = bias2_on ? __fadd_rn(v, b2[r]) : v;
+                v = act_fast<EPI>(v, p.ep2);
+                if constexpr (RES) v = add_res(v, rv[r], p.res_relu, (col_voff + (unsigned) m_uni * row_bytes) >> 2, p.res_body);
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rc, row_ok ? col_voff : OOB, (unsigned) m_uni * row_bytes, 0);
+            }
+        };
+        if (m_edge) store(std::true_type{});
+        else store(std::false_type{});
     }
 }
 
@@ -1160,18 +1184,18 @@ __device__ __forceinline__ bool reduce_in_launch(const IgemmParams &p, f32x16 (&
     __syncthreads();
     if (!s_last) return false;
     const int width = p.N - p.part_begin;
-    const bool m_edge = m_wave + TM * 32 > p.M;
 #pragma unroll
     for (int a = 0; a < TM; ++a)
 #pragma unroll
         for (int b = 0; b < TN; ++b)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[a][b][r] = 0;
+    const bool m_edge = m_wave + TM * 32 > p.M;
     for (int s = 0; s < p.n_slices; ++s) {
         const rsrc_t rp = make_rsrc(reinterpret_cast<const char *>(p.partial) +
                                     (size_t) (s * gridDim.z + batch) * p.M * width * 4, RSRC_RANGE);
         // half a 32x32 block at a time: eight loads in flight, not sixteen per block of the tile, which would
-        // cost the kernels registers and with them occupancy
+        // cost the kernels registers and with them occupancy (as a variant of this loop for the last row tile would)
 #pragma unroll
         for (int a = 0; a < TM; ++a)
 #pragma unroll

@@ -32,8 +32,9 @@ struct StemParams {
     Epilogue ep;
 };
 
-// HALF: 64 pixels a workgroup, a wavefront one of the two row tiles
-template <int KS, int EPI, bool TWO, bool HALF = false>
+// HALF: 64 pixels a workgroup, a wavefront one of the two row tiles.  FAR: planes so large that a masked row's place has to be bounded (far_rows); a variant of its
+// own, since the bounds are 7 % of a 3x3 layer (32 channels on 50 x 145 x 145 65.4 and 71.4 us)
+template <int KS, int EPI, bool TWO, bool HALF = false, bool FAR = false>
 __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
     static_assert(!HALF || TWO, "two row tiles to share out");
     constexpr int TW = HALF ? 64 : ST_TW, TM = TWO && !HALF ? 2 : 1;   // pixels of a segment, row tiles of a wavefront
@@ -122,7 +123,8 @@ __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
     auto load = [&](const Place &q, int which) __attribute__((always_inline)) {
         const int ch = which / ROWS, r = which % ROWS;
         const int ih = q.ih0 + r % KS;   // uniform
-        pv[r][ch] = buf_load_f32(q.rx, (unsigned) ih < (unsigned) p.h ? q.voff[ch] : OOB, patch_row_offset(r / KS, ih, p.h, (unsigned) p.w_in * 4u));
+        pv[r][ch] = buf_load_f32(q.rx, (unsigned) ih < (unsigned) p.h ? q.voff[ch] : OOB,
+                                 FAR ? patch_row_offset(r / KS, ih, p.h, (unsigned) p.w_in * 4u) : (unsigned) (((r / KS) * p.h + ih) * p.w_in) * 4u);
     };
     const rsrc_t ry = make_rsrc(p.y, RSRC_RANGE);
     const rsrc_t rb = make_rsrc(p.bias, p.bias ? (unsigned) (p.cout * 4) : 0u);
@@ -208,7 +210,7 @@ __global__ __launch_bounds__(256, 2) void stem_f32_kernel(const StemParams p) {
                 // reference (conv.c:18-27), so is the activation: p.ep says NOT_ACT then
                 const float vb = __fadd_rn(v, bias_r[a][r]);
                 __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(act_fast<EPI>(has_bias ? vb : v, p.ep)), ry,
-                                                      whole || 4 * lh < p.cout - m ? voff : OOB, row_offset(m, p.cout, ohw4), 0);
+                                                      whole || 4 * lh < p.cout - m ? voff : OOB, FAR ? row_offset(m, p.cout, ohw4) : (unsigned) m * ohw4, 0);
             }
         }
     }
@@ -249,12 +251,19 @@ bool stem_f32_ok(const onhip_conv_desc_t &d, int OH, int OW) {
 // two (74 matrix instructions instead of 148), and half of the loads in front of them (64 channels under 7x7 and stride 2 on one image of 224 x 224 13.1 us in 112 workgroups, 8.8 in 224).
 static int stem_tw(int cout, int ks, long long rows, int ow) { return ks == 7 && cout > 32 && rows * ((ow + ST_TW - 1) / ST_TW) <= 128 ? 64 : ST_TW; }
 
+// (never with segments of 64 pixels, whose results are up to 128 x 128)
+static bool stem_far(const StemParams &p, int ks) {
+    return far_rows(p.h, p.w_in, p.pt, (long long) (p.oh - 1) * p.stride - p.pt + ks - 1, p.cout > 32 ? 64 : 32, (long long) p.oh * p.ow);
+}
+
 template <int KS>
 static int stem_launch_ks(const StemParams &p, unsigned grid, hipStream_t stream) {
-    const bool two = p.cout > 32, half = stem_tw(p.cout, KS, (long long) p.n * p.oh, p.ow) != ST_TW;
+    const bool two = p.cout > 32, half = stem_tw(p.cout, KS, (long long) p.n * p.oh, p.ow) != ST_TW, far = !half && stem_far(p, KS);
 #define ONHIP_STEM_LAUNCH(EPI)                                                                                              \
     do {                                                                                                                    \
         if (KS == 7 && half) hipLaunchKernelGGL((stem_f32_kernel<KS, EPI, true, KS == 7>), dim3(grid), dim3(256), 0, stream, p); \
+        else if (far && two) hipLaunchKernelGGL((stem_f32_kernel<KS, EPI, true, false, true>), dim3(grid), dim3(256), 0, stream, p); \
+        else if (far) hipLaunchKernelGGL((stem_f32_kernel<KS, EPI, false, false, true>), dim3(grid), dim3(256), 0, stream, p);  \
         else if (two) hipLaunchKernelGGL((stem_f32_kernel<KS, EPI, true>), dim3(grid), dim3(256), 0, stream, p);                 \
         else hipLaunchKernelGGL((stem_f32_kernel<KS, EPI, false>), dim3(grid), dim3(256), 0, stream, p);                    \
     } while (0)
