@@ -41,7 +41,7 @@ LEGEND = ("Kernel names: `onhip::igemm_kernel<dtype, loader, BM, BN, WM, WN, PF,
           "16-bit storage: operand tiles loaded straight into LDS, KS bytes of K per stage, ring of NST stages), `onhip::rowb_f32_kernel<WM, WN>` (fp32, B "
           "straight from memory, tile 32 WM x 128 WN), `onhip::igemm_f3_kernel<loader, BM, BN, WM, WN, RES, PW2, NORM>` (fp32 on the 16-bit matrix cores; loader 5 "
           "the rows of a product; NORM the variant that normalises the rows of its result as well) and `onhip::split_weights_kernel` in front of it where the weights are split on the call, `onhip::splitk_finish_kernel`, `onhip::depthwise_tiled_kernel<int8, stride, "
-          "act>`, `onhip::quantize_nhwc_kernel<CBW>`, `onhip::stem_f32_kernel<filter size, act, two row tiles, segments of 64 pixels>` (first-layer "
+          "act>`, `onhip::quantize_nhwc_kernel<CBW>`, `onhip::stem_f32_kernel<filter size, act, two row tiles, segments of 64 pixels, large planes>` (first-layer "
           "convolutions from an LDS patch), `onhip::i8patch_kernel<bytes per pixel, WM, pixel tiles>` and `onhip::i8direct_kernel<bytes per pixel, taps, WM, TM, pixel "
           "tiles, workgroups per CU>` (int8 chain form, 3x3 with few channels: input rows in LDS / windows loaded per tap), `onhip::attention_f32_kernel<16-key tiles, head dim>`, "
           "`onhip::attention_f3_kernel<wavefronts>` (fp32 on the 16-bit matrix cores), `onhip::attention_h16_kernel<dtype, 32-key tiles, wavefronts>`, "
