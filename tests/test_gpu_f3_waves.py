@@ -24,10 +24,36 @@ def both(tile, other, run, monkeypatch, torch):
     assert torch.equal(got[0].view(torch.int32), got[1].view(torch.int32))
 
 
+# (tiles of a product cannot be asked for; the model takes it for the first three and others for the rest)
+@pytest.mark.parametrize("rows,k,n", [(12544, 192, 192), (12481, 767, 187), (16384, 200, 190), (6272, 1024, 250), (17000, 520, 187), (33000, 192, 192)])
+def test_product(rows, k, n):
+    import torch
+    hip.init(0)
+    g = torch.Generator(device="cuda").manual_seed(rows + k)
+    a, b, bias = torch.randn((rows, k), generator=g, device="cuda"), torch.randn((k, n), generator=g, device="cuda") / k ** 0.5, torch.randn(n, generator=g, device="cuda")
+    add = torch.randn((rows, n), generator=g, device="cuda")
+    ref, mass = torch.matmul(a.double(), b.double()) + bias, torch.matmul(a.abs().double(), b.abs().double()) + bias.abs()
+    # a chain of fp32 multiply-adds, what the left-out partial products can reach, the roundings of the bias and the result (and of the addend's sum)
+    bound = mass * ((k + 4) * 2.0 ** -24 + 2.0 ** -23)
+    y = hip.matmul(a, b, bias=bias)
+    plain = list(hip.last_launch_choice())
+    print(rows, k, n, plain, flush=True)
+    assert bool(((y.double() - ref).abs() <= bound).all())
+    z = hip.matmul(a, b, bias=bias, addend=add)
+    if list(hip.last_launch_choice()) == plain:   # a choice of its own, so perhaps other sums
+        assert torch.equal(z, y + add)
+    else:
+        assert bool(((z.double() - ref - add).abs() <= bound + 2.0 ** -23 * add.abs()).all())
+    t = table(torch)
+    i = ((y + 8.0) * 512.0).to(torch.int32).clamp(0, 8191)
+    z = hip.matmul(a, b, bias=bias, gelu_lut=t)
+    assert list(hip.last_launch_choice()) == plain and torch.equal(z, torch.where(y < -8.0, 0.0, torch.where(y >= 8.0, y, t[i.long()])))
+
+
 # Tiles of a product cannot be asked for: with the one that the model takes.  192 x 64 in twelve wavefronts up to 16384 rows and in four above, then others.
 @pytest.mark.parametrize("rows,k,n,tile", [(12544, 192, 192, (192, 64)), (12481, 767, 187, (192, 64)), (16384, 200, 190, (192, 64)), (33000, 520, 187, (192, 64)),
                                            (32961, 768, 192, (192, 64)), (6272, 1024, 250, None), (17000, 520, 187, (64, 64)), (33000, 192, 192, (64, 64))])
-def test_product(rows, k, n, tile):
+def test_product_tiles(rows, k, n, tile):
     import torch
     hip.init(0)
     g = torch.Generator(device="cuda").manual_seed(rows + k)
