@@ -444,6 +444,9 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
             col_voff4[b] = n < p.N ? out_col_offset(p, n, 4) + (unsigned) (4 * lh) * row_bytes4 : OOB;
         }
         // RES: the residual operand of a folded Add (fp32 results): a row tile's addends are requested together
+        // and, in the last row tile, where a row past the last may be 2 GiB away (row_offset.hpp), have their row in the vector offset, as the results have:
+        // with a branch a row (the form without an addend) each value waits for the stores before it (24 channels of 8 x 56 x 56 with an Add 8.8 us
+        // a launch, 7.1 like this)
         const rsrc_t rres = make_rsrc(RES ? reinterpret_cast<const char *>(p.res) + (size_t) batch * p.c_batch_stride * 4 : nullptr,
                                       RES ? RSRC_RANGE : 0u);
         // What is the same for all values of a launch is decided once, out here: the tile at the edge of M (rows are tested), whether
@@ -460,11 +463,9 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
                     for (int r = 0; r < 16; ++r) {
                         const int m_uni = m_wave + a * 32 + 8 * (r / 4) + (r % 4);
                         const bool row_ok = !EDGE || m_uni + 4 * lh < p.M;
+                        const unsigned at = (unsigned) m_uni * row_bytes;
 #pragma unroll
-                        for (int b = 0; b < TN; ++b) rv[r][b] = 0.0f;
-                        if (row_there<EDGE>(m_uni, p.M))   // uniform
-#pragma unroll
-                            for (int b = 0; b < TN; ++b) rv[r][b] = buf_load_f32(rres, row_ok ? col_voff[b] : OOB, (unsigned) m_uni * row_bytes);
+                        for (int b = 0; b < TN; ++b) rv[r][b] = buf_load_f32(rres, row_ok ? col_voff[b] + (EDGE ? at : 0u) : OOB, EDGE ? 0u : at);
                     }
                 }
 #pragma unroll
@@ -508,8 +509,9 @@ __device__ __forceinline__ void write_tile(const IgemmParams &p, ACC (&acc)[TM][
                                     }
                                 }
                             }
-                            if (!there) continue;
-                            const unsigned voff = row_ok ? col_voff[b] : OOB, soff = (unsigned) (m_uni + j) * row_bytes;
+                            if (!RES && !there) continue;
+                            const unsigned at = (unsigned) (m_uni + j) * row_bytes;
+                            const unsigned voff = row_ok ? col_voff[b] + (RES && EDGE ? at : 0u) : OOB, soff = RES && EDGE ? 0u : at;
                             if (!FP32 && p.out_s8)
                                 __builtin_amdgcn_raw_buffer_store_b8((unsigned char) requant_s8(v, p.out_inv_scale), rc, voff, soff, 0);
                             else

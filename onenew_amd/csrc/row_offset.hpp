@@ -15,7 +15,7 @@ constexpr unsigned RSRC_RANGE = 0x80000000u; // num_records of the data buffers 
 // `rows` rows reach less than 2 GiB; a tile's rows past the last may reach more.  A masked lane (OOB) of one of those would ask for OOB plus that, and
 // from 2 GiB on the sum is no longer outside by itself: 20 channels of 4700 x 4700 are 1.8 GB, and channel 27 would be at 2.4 GB.  So nothing
 // is asked for a row that no lane has; OOB and the place of a row that is there stay at 2 GiB or more, and below 4.  EDGE: the variant for tiles with rows
-// past the last, the others have none.  (A branch a row in the last row tile, which also saves it those rows' accesses.  The place bounded
+// past the last, the others have none.  (A branch a row in the last row tile, which also saves it those rows' accesses; the W8A32 store with a residual operand has the row in the vector offset there.  The place bounded
 // by the last row's instead was a minimum and a product a row, for which the compiler kept scalars in vector registers: fp32 64 x 64 tiles
 // with a residual operand 3-5 % slower.)
 template <bool EDGE> ONHIP_BOTH constexpr bool row_there(int row, int rows) { return !EDGE || row < rows; }
